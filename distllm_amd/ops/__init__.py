@@ -371,9 +371,15 @@ def attn_varlen(Q, K, V, cu_seqlens, block_map=None, scale=None):
                 torch.nn.functional.pad(V, (0, pad)).contiguous(),
                 cu_seqlens.int(), blk_seq, blk_qb, scale)
             return O[..., :D].contiguous()
-        return _hip_ops.attn_varlen(Q.contiguous(), K.contiguous(),
-                                    V.contiguous(), cu_seqlens.int(),
-                                    blk_seq, blk_qb, scale)
+        if not all(t.stride(2) == 1 and t.stride(1) == D
+                   and t.stride(0) == s and s % 8 == 0
+                   and t.data_ptr() % 16 == 0
+                   for t, s in ((Q, Q.stride(0)), (K, K.stride(0)),
+                                (V, K.stride(0)))):
+            Q, K, V = (t.clone(memory_format=torch.contiguous_format)
+                       for t in (Q, K, V))
+        return _hip_ops.attn_varlen(Q, K, V, cu_seqlens.int(), blk_seq,
+                                    blk_qb, scale)
     return torch_ref.attn_varlen(Q, K, V, cu_seqlens, scale)
 
 

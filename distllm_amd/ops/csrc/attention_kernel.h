@@ -6,7 +6,6 @@
 // The reference delegated all of this to HF transformers / faesm /
 // flash-attn (reference: distllm/embed/encoders/*.py).
 //
-// v2 structure (guide Appendix B "fused attention prefill" + §5.5):
 //  - workgroup = 256 threads = 4 waves; each wave owns 32 q rows
 //    (128 q rows per workgroup); KV tiles of 64 keys, double-buffered,
 //    ONE barrier per tile.
@@ -14,57 +13,96 @@
 //    lane holds 32 of the 64 scores of ONE q row -> online softmax is
 //    lane-local + one shfl_xor(32) combine.
 //  - PV is swapped too: accO^T = mfma(A=V^T, B=P): the O accumulator
-//    keeps q on lanes, so the alpha rescale is lane-local.
-//  - P(f32) -> bf16 B-fragments via hardware cvt + permlane32_swap.
-//  - T14 async-STAGE split: next tile's V goes global->regs right at
-//    the top of the iteration (HBM latency hides under QK/softmax/PV),
-//    the ds_write lands after PV; K tiles stream by global_load_lds
-//    (lane-linear dest, T2 XOR swizzle on the SOURCE address, rule 21).
-//  - s_setprio(1) around the MFMA clusters (T5).
-//  - epilogue transposes O through padded LDS for coalesced stores.
+//    keeps q on lanes, so the alpha rescale is lane-local. The order of
+//    the 16 keys of a product is free, so P goes in as the score product
+//    left it on the lanes: keys 4h..4h+3 and 8+4h..8+4h+3 of lane half h.
+//  - K and V tiles stream by global_load_lds, row by row, their 16-byte
+//    (V: 32-byte) pieces XOR-swizzled by the row on the SOURCE address; V is
+//    transposed on its way out of LDS (ds_read_b64_tr_b16, 4 keys x 16
+//    columns per 16 lanes).
+//  - a tile in which no key is masked for any row of the wave takes the
+//    scores as they are: max over the raw products, then one fused multiply
+//    and add per exponential.
+//  - O leaves by 16-byte stores straight from the accumulators (one lane
+//    swap per 8 columns), so that LDS holds the tiles only.
+//
+// Bound by the vector units (per tile and wave at D = 64: 512 cycles of
+// MFMA, about 700 of exponentials, max, sum and conversion) and, at D = 128,
+// by LDS reads (32 KB per wave and tile). Measured, before (V transposed
+// through registers at D = 64, read element by element from memory at 128,
+// every score scaled and masked by itself) and now: 512 x 512 tokens, 12
+// heads of 64, masked 1341 -> 640 us (640 TFLOP/s); packed proteins of 64 to
+// 1024, 20 heads of 64, 248 -> 111 us; causal, 32 heads of 128 on 8,
+// 16 x 1024 536 -> 260 us and 4 x 4096 2354 -> 621 us (885 TFLOP/s); window
+// 1024 of 6 x 2048, 32 heads of 128, 370 -> 289 us. Four waves a SIMD at
+// D = 64 unless the causal compares need more registers (3), two at 128.
+// Wave priorities around the products and reading all K or V fragments
+// ahead of them measured 0 to 5% slower than leaving the order to the
+// compiler.
 //
 // Layouts: Q [B, SQ, H, D] (token stride parametric), K/V
 // [B, SKV, HKV, D] (shared strides), O contiguous BSHD; mask f32
-// [B, SKV] additive (0 / -inf) or nullptr.
+// [B, SKV] additive (0 / -inf) or nullptr. K, V and their strides are
+// multiples of 16 bytes.
 #pragma once
 #include "common.h"
 #include <cstdlib>
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
 
 #define KVBLK 64
 #define QWAVE 32
 #define LOG2E 1.4426950408889634f
-#define VROW 68   // padded V^T row length in bf16 elems (136 B)
 
 extern __shared__ __attribute__((aligned(16))) char smem[];
 
 union frag_u {
   bf16x8 v;
+  s16x4 h[2];
   unsigned int d[4];
 };
+
+__device__ __forceinline__ unsigned int pack_bf16(float a, float b) {
+  const bf16x2 v = __builtin_convertvector(f32x2{a, b}, bf16x2);
+  return __builtin_bit_cast(unsigned int, v);
+}
+
+__device__ __forceinline__ void copy_to_lds(const unsigned short* src,
+                                            char* dst) {
+  __builtin_amdgcn_global_load_lds(
+      (const __attribute__((address_space(1))) unsigned int*)src,
+      (__attribute__((address_space(3))) unsigned int*)dst, 16, 0, 0);
+}
+
+// LDS of a workgroup: two buffers of keys (and their shared part), values
+// and mask numbers.
+constexpr int attn_lds(int D, int DV, int ROT, bool mask) {
+  return 2 * KVBLK * ((D + DV + ROT) * 2 + (mask ? 4 : 0));
+}
 
 // VARLEN: Q/K/V are PACKED [total_tokens, H(KV), D] (cu_seqlens int32
 // [B+1]); one workgroup per (sequence, q-block, head) via the
 // host-built blk_seq/blk_qb map — the protein/fasta path with zero
 // padded FLOPs (reference: the faesm flash-attn varlen role,
-// distllm/embed/encoders/esm2.py:41-55).
+// distllm/embed/encoders/esm2.py:41-55). Without WINDOW, workgroups past
+// nblk * H (nblk = SQa here) zero the rows from cu[Bsz] to SKVa, which no
+// sequence holds.
 //
 // WINDOW (with VARLEN and CAUSAL): the packed queries of a sequence are the
 // last ones of its packed keys (cu for queries, cu_k for keys), as when a
 // prompt is continued from a cache, and a query sees only the `window`
 // latest keys up to its own position. Keys and values may have different
-// head sizes (DV) and interleave in one row (tstr_k counts both). V is
-// staged in units of 4 keys x 8 columns, transposed in registers, so that
-// the V^T image is written 8 bytes at a time; its 16-byte pieces are swizzled
-// by the row, for both the writes and the reads.
+// head sizes (DV) and interleave in one row (tstr_k counts both).
 // With ROT, queries have ROT more numbers per head, against ROT numbers of
 // each key that all heads share (Kr [Tk, ROT]). sink (a number per head, part
 // of the softmax's denominator) and gate (sigmoid of a number per query and
 // head on the output) may be null.
-template <int D, bool CAUSAL, bool HAS_MASK, bool VDIRECT,
-          bool VARLEN = false, int DV = D, bool WINDOW = false, int ROT = 0>
-__global__ void __launch_bounds__(256, WINDOW && D + DV <= 256 ? 2 : 1)
+template <int D, bool CAUSAL, bool HAS_MASK, bool VARLEN = false, int DV = D,
+          bool WINDOW = false, int ROT = 0>
+__global__ void __launch_bounds__(256, D + DV <= 128   ? (CAUSAL ? 3 : 4)
+                                       : D + DV <= 256 ? 2
+                                                       : 1)
 attn_fwd_kernel(const unsigned short* __restrict__ Q,
                 const unsigned short* __restrict__ Kt,
                 const unsigned short* __restrict__ Vt,
@@ -81,19 +119,13 @@ attn_fwd_kernel(const unsigned short* __restrict__ Q,
                 const unsigned short* __restrict__ gate = nullptr,
                 int ld_gate = 0) {
   constexpr int NWAVE = 4;  // waves per workgroup (8 measured slower)
-  constexpr int NTHR = NWAVE * 64;
   constexpr int QBLK = NWAVE * QWAVE;       // q rows per workgroup
   constexpr int NCH = D / 8;             // 16B chunks per K row
   constexpr int NCHV = DV / 8;           // 16B chunks per V row
   constexpr int DBLK = DV / 32;          // 32-wide d blocks of V
   constexpr int KTILE_B = KVBLK * D * 2; // K tile bytes
   constexpr int RTILE_B = KVBLK * ROT * 2; // shared key part of a tile
-  constexpr int VR = WINDOW ? KVBLK : VROW; // V^T row length
-  constexpr int VTILE_B = DV * VR * 2;   // V^T tile bytes
-  // V chunks per thread; 4-key units with WINDOW
-  constexpr int VUNITS = KVBLK / 4 * NCHV;
-  constexpr int VCH =
-      WINDOW ? (VUNITS + NTHR - 1) / NTHR * 4 : KVBLK * NCHV / NTHR;
+  constexpr int VTILE_B = KVBLK * DV * 2;  // V tile bytes
 
   const int lane = threadIdx.x & 63;
   const int wid = threadIdx.x >> 6;
@@ -101,36 +133,32 @@ attn_fwd_kernel(const unsigned short* __restrict__ Q,
   const int qcol = lane & 31;
 
   int qb, b, head;
-  if (VARLEN && WINDOW) {
+  if (VARLEN) {
+    const int nblk = WINDOW ? gridDim.x / H : SQa;
+    if (!WINDOW && (int)blockIdx.x >= nblk * H) {
+      const long n8 = (long)H * DV / 8;
+      const long first = (long)cu[Bsz] * n8, end = (long)SKVa * n8;
+      const long step = (gridDim.x - nblk * H) * blockDim.x;
+      for (long i = first + (long)(blockIdx.x - nblk * H) * blockDim.x +
+                    threadIdx.x;
+           i < end; i += step)
+        reinterpret_cast<i32x4*>(O)[i] = i32x4{0, 0, 0, 0};
+      return;
+    }
     // neighbouring q-blocks of one head share most of their keys: give
     // each XCD a contiguous run of them
-    const int nwg = gridDim.x, nblk = nwg / H;
-    const int per = nwg / 8, rem = nwg % 8;
-    const int xcd = blockIdx.x % 8, j = blockIdx.x / 8;
-    const int bid =
-        (xcd < rem ? xcd * (per + 1) : rem * (per + 1) + (xcd - rem) * per) +
-        j;
+    const int bid = xcd_run(blockIdx.x, nblk * H);
     head = bid / nblk;
     const int i = bid % nblk;
     b = blk_seq[i];
     qb = blk_qb[i];
-  } else if (VARLEN) {
-    const int i = blockIdx.x / H;
-    head = blockIdx.x % H;
-    b = blk_seq[i];
-    qb = blk_qb[i];
   } else {
     const int nqb0 = (SQa + QBLK - 1) / QBLK;
-    // T1 bijective XCD swizzle: keep the q-blocks sharing one
-    // (b, head)'s K/V on one XCD's L2 (+12% at D=128/GQA).
-    int bid = blockIdx.x;
-    {
-      const int nwg = Bsz * H * nqb0;
-      const int q = nwg / 8, r = nwg % 8;
-      const int xcd = bid % 8, j = bid / 8;
-      bid = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + j;
-    }
-    qb = bid % nqb0;
+    // keep the q-blocks sharing one (b, head)'s K/V on one XCD's L2
+    // (+12% at D=128/GQA).
+    const int bid = xcd_run(blockIdx.x, Bsz * H * nqb0);
+    // causal: the blocks with most keys first, they would be the tail
+    qb = CAUSAL ? nqb0 - 1 - bid % nqb0 : bid % nqb0;
     const int bh = bid / nqb0;
     head = bh % H;
     b = bh / H;
@@ -160,17 +188,25 @@ attn_fwd_kernel(const unsigned short* __restrict__ Q,
   const int offK[2] = {0, KTILE_B};
   constexpr int offR = 2 * KTILE_B;
   const int offV[2] = {offR + 2 * RTILE_B, offR + 2 * RTILE_B + VTILE_B};
-  const int offM[2] = {2 * KTILE_B + 2 * VTILE_B,
-                       2 * KTILE_B + 2 * VTILE_B + KVBLK * 4};
+  constexpr int offM = offR + 2 * RTILE_B + 2 * VTILE_B;
+  const float* mask_lds = reinterpret_cast<const float*>(smem + offM);
 
-  const float scale2 = scale * LOG2E;
+  // the maximum is taken before scaling: with a negative scale, of the
+  // negated scores
+  const float scale2 = fabsf(scale) * LOG2E;
+  const unsigned int flip = scale < 0.f ? 0x80008000u : 0u;
 
   // ---- Q fragments in registers ---------------------------------------
   bf16x8 qf[(D + ROT) / 16];
 #pragma unroll
-  for (int s = 0; s < (D + ROT) / 16; ++s)
-    qf[s] = *reinterpret_cast<const bf16x8*>(Qb + (long)qload * tstr_q +
-                                             s * 16 + h * 8);
+  for (int s = 0; s < (D + ROT) / 16; ++s) {
+    frag_u f;
+    f.v = *reinterpret_cast<const bf16x8*>(Qb + (long)qload * tstr_q +
+                                           s * 16 + h * 8);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) f.d[i] ^= flip;
+    qf[s] = f.v;
+  }
 
   float m = -1e30f, l = 0.f;
   f32x16 accO[DBLK];
@@ -179,129 +215,42 @@ attn_fwd_kernel(const unsigned short* __restrict__ Q,
 #pragma unroll
     for (int i = 0; i < 16; ++i) accO[d][i] = 0.f;
 
-  // ---- staging helpers --------------------------------------------------
-  auto stage_k = [&](int k0, int buf) {   // glds, swizzled source
-    constexpr int ROWS_PER = 1024 / (2 * D);   // 8 (D=64) / 4 (D=128)
-    constexpr int NPIECE = KVBLK / ROWS_PER;   // 8 / 16
-    const int r_in = lane / NCH;
-    const int c_dst = lane % NCH;
-    for (int p = wid; p < NPIECE; p += NWAVE) {
-      const int row = p * ROWS_PER + r_in;
-      const int c_src = c_dst ^ (row & (NCH - 1));
-      int krow = k0 + row;
-      if (krow >= SKV) krow = SKV - 1;
-      const unsigned short* src = Kb + (long)krow * tstr_k + c_src * 8;
-      auto dst = (__attribute__((address_space(3))) unsigned int*)(
-          smem + offK[buf] + p * ROWS_PER * (2 * D) + lane * 16);
+  // ---- staging: 1 KiB pieces of whole rows, swizzled source -------------
+  auto stage = [&](int k0, int buf) {
+    if (HAS_MASK && wid == 0)
       __builtin_amdgcn_global_load_lds(
-          (const __attribute__((address_space(1))) unsigned int*)src, dst,
-          16, 0, 0);
+          (const __attribute__((address_space(1))) unsigned int*)(
+              maskp + (long)b * SKV + min(k0 + lane, SKV - 1)),
+          (__attribute__((address_space(3))) unsigned int*)(
+              smem + offM + buf * KVBLK * 4 + lane * 4),
+          4, 0, 0);
+    constexpr int KROWS = 1024 / (2 * D), VROWS = 1024 / (2 * DV);
+#pragma unroll
+    for (int p = 0; p < KVBLK / KROWS / NWAVE; ++p) {
+      const int row = (p * NWAVE + wid) * KROWS + lane / NCH;
+      const int c = (lane % NCH) ^ (row & (NCH - 1));
+      copy_to_lds(Kb + (long)min(k0 + row, SKV - 1) * tstr_k + c * 8,
+                  smem + offK[buf] + (p * NWAVE + wid) * 1024 + lane * 16);
     }
     if constexpr (ROT > 0) {
       static_assert(ROT == 64, "eight 16-byte pieces per row");
-      for (int p = wid; p < KVBLK / 8; p += NWAVE) {
-        const int row = p * 8 + (lane >> 3);
-        const int krow = min(k0 + row, SKV - 1);
-        const unsigned short* src =
-            Kr + (long)(cu_k[b] + krow) * ROT + ((lane & 7) ^ (row & 7)) * 8;
-        auto dst = (__attribute__((address_space(3))) unsigned int*)(
-            smem + offR + buf * RTILE_B + p * 1024 + lane * 16);
-        __builtin_amdgcn_global_load_lds(
-            (const __attribute__((address_space(1))) unsigned int*)src, dst,
-            16, 0, 0);
+#pragma unroll
+      for (int p = 0; p < KVBLK / 8 / NWAVE; ++p) {
+        const int row = (p * NWAVE + wid) * 8 + (lane >> 3);
+        copy_to_lds(Kr + (long)(cu_k[b] + min(k0 + row, SKV - 1)) * ROT +
+                        ((lane & 7) ^ (row & 7)) * 8,
+                    smem + offR + buf * RTILE_B + (p * NWAVE + wid) * 1024 +
+                        lane * 16);
       }
     }
-  };
-  // per-thread V staging geometry, hoisted out of the tile loop
-  int v_k[VCH < 1 ? 1 : VCH];                       // key index within tile
-  const unsigned short* v_src[VCH];   // &V[v_k][d0] (tile k0 = 0)
-  int v_woff[VCH];                    // LDS elem offset d0*VROW + k
 #pragma unroll
-  for (int c = 0; c < VCH; ++c) {
-    const int ci = threadIdx.x + c * NTHR;
-    v_k[c] = ci / NCHV;
-    const int d0 = (ci % NCHV) * 8;
-    v_src[c] = Vb + (long)v_k[c] * tstr_k + d0;
-    v_woff[c] = d0 * VROW + v_k[c];
-  }
-  const unsigned short* v_src_last = Vb + (long)(SKV - 1) * tstr_k;
-
-  // T14 split: issue V loads into regs (no wait) ...
-  auto v_issue = [&](int k0, s16x8* vreg) {
-    if constexpr (WINDOW) {
-#pragma unroll
-      for (int c = 0; c < VCH / 4; ++c) {
-        const int u = threadIdx.x + c * NTHR;
-        if (VUNITS % NTHR == 0 || u < VUNITS) {
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const int key = min(k0 + u / NCHV * 4 + j, SKV - 1);
-            vreg[c * 4 + j] = *reinterpret_cast<const s16x8*>(
-                Vb + (long)key * tstr_k + u % NCHV * 8);
-          }
-        }
-      }
-      return;
-    }
-    const long koff = (long)k0 * tstr_k;
-#pragma unroll
-    for (int c = 0; c < VCH; ++c) {
-      const unsigned short* src =
-          (k0 + v_k[c] < SKV)
-              ? v_src[c] + koff
-              : v_src_last + ((v_src[c] - Vb) - (long)v_k[c] * tstr_k);
-      vreg[c] = *reinterpret_cast<const s16x8*>(src);
+    for (int p = 0; p < KVBLK / VROWS / NWAVE; ++p) {
+      const int row = (p * NWAVE + wid) * VROWS + lane / NCHV;
+      const int c = (lane % NCHV) ^ ((row & 3) << 1);
+      copy_to_lds(Vb + (long)min(k0 + row, SKV - 1) * tstr_k + c * 8,
+                  smem + offV[buf] + (p * NWAVE + wid) * 1024 + lane * 16);
     }
   };
-  // ... and transpose-write them into the padded V^T image later.
-  auto v_write = [&](int buf, const s16x8* vreg) {
-    unsigned short* vt = reinterpret_cast<unsigned short*>(smem + offV[buf]);
-    if constexpr (WINDOW) {
-#pragma unroll
-      for (int c = 0; c < VCH / 4; ++c) {
-        const int u = threadIdx.x + c * NTHR;
-        if (VUNITS % NTHR == 0 || u < VUNITS) {
-          i32x4 k[4];
-#pragma unroll
-          for (int j = 0; j < 4; ++j)
-            k[j] = __builtin_bit_cast(i32x4, vreg[c * 4 + j]);
-          const int d8 = u % NCHV, kq = u / NCHV;
-          unsigned short* dst = vt + d8 * 8 * VR + (kq & 1) * 4;
-          const int piece = (kq >> 1) ^ (d8 & 7);
-#pragma unroll
-          for (int w = 0; w < 4; ++w) {
-            i32x2 even, odd;
-            even[0] = __builtin_amdgcn_perm(k[1][w], k[0][w], 0x05040100);
-            even[1] = __builtin_amdgcn_perm(k[3][w], k[2][w], 0x05040100);
-            odd[0] = __builtin_amdgcn_perm(k[1][w], k[0][w], 0x07060302);
-            odd[1] = __builtin_amdgcn_perm(k[3][w], k[2][w], 0x07060302);
-            *reinterpret_cast<i32x2*>(dst + w * 2 * VR +
-                                      (piece ^ (w * 2)) * 8) = even;
-            *reinterpret_cast<i32x2*>(dst + (w * 2 + 1) * VR +
-                                      (piece ^ (w * 2 + 1)) * 8) = odd;
-          }
-        }
-      }
-      return;
-    }
-#pragma unroll
-    for (int c = 0; c < VCH; ++c) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i)
-        vt[v_woff[c] + i * VROW] = (unsigned short)vreg[c][i];
-    }
-  };
-  auto stage_m = [&](int k0, int buf) {
-    if (!WINDOW && threadIdx.x < KVBLK) {
-      const int krow = k0 + threadIdx.x;
-      float mv;
-      if (krow >= SKV) mv = -INFINITY;
-      else if (HAS_MASK) mv = maskp[(long)b * SKV + krow] * LOG2E;
-      else mv = 0.f;
-      reinterpret_cast<float*>(smem + offM[buf])[threadIdx.x] = mv;
-    }
-  };
-
   int ntile = (SKV + KVBLK - 1) / KVBLK;
   if (CAUSAL) {
     const int qmax_blk = min(qb * QBLK + QBLK - 1, SQ - 1);
@@ -313,14 +262,16 @@ attn_fwd_kernel(const unsigned short* __restrict__ Q,
     tile0 = first > 0 ? first / KVBLK : 0;
   }
 
-  // prologue: stage the first tile synchronously
-  s16x8 vreg[VCH];
-  stage_k(tile0 * KVBLK, 0);
-  if (!VDIRECT) {
-    v_issue(tile0 * KVBLK, vreg);
-    v_write(0, vreg);
-  }
-  stage_m(tile0 * KVBLK, 0);
+  // V^T fragments: 16 lanes take 4 keys x 16 columns; a lane's address is
+  // key (lane & 15) / 4 of them, columns 4 * (lane & 3)
+  const int vi = lane & 15;
+  int v_off[2];  // of column blocks 0 and 1 (of 32); others 128 bytes on
+#pragma unroll
+  for (int d = 0; d < 2; ++d)
+    v_off[d] = (4 * h + (vi >> 2)) * (2 * DV) +
+               ((d * 2 + ((lane >> 4) & 1)) ^ (vi >> 2)) * 32 + (vi & 3) * 8;
+
+  if (tile0 < ntile) stage(tile0 * KVBLK, 0);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
 
@@ -328,162 +279,144 @@ attn_fwd_kernel(const unsigned short* __restrict__ Q,
   for (int t = tile0; t < ntile; ++t) {
     const int k0 = t * KVBLK;
     const bool have_next = t + 1 < ntile;
-    if (have_next) {
-      stage_k(k0 + KVBLK, cur ^ 1);   // async glds into the other buffer
-      if (!VDIRECT) v_issue(k0 + KVBLK, vreg);  // V -> regs (T14)
-    }
+    if (have_next) stage(k0 + KVBLK, cur ^ 1);  // into the other buffer
 
     const bool wave_active =
         q0w < SQ && (!CAUSAL || k0 <= q0w + shift + QWAVE - 1) &&
         (!WINDOW || k0 + KVBLK - 1 > q0w + shift - window);
-    // mask values are only needed when a real mask exists or the tile
-    // hangs over the end of the sequence (padded keys); skipping the 32
-    // LDS reads otherwise removes a large per-tile VALU cost.
-    // (WINDOW needs neither: padded keys are past every query.)
-    const bool tile_masked = HAS_MASK || (!WINDOW && k0 + KVBLK > SKV);
-    // WINDOW: key k is visible when 0 <= k - qlo <= qpos - qlo, one
-    // unsigned compare; kept free of branches, which cost the unrolled
-    // score loop far more than the compares
-    const unsigned int wspan = WINDOW ? qpos - qlo : 0;
-    const int woff = WINDOW ? k0 + 4 * h - qlo : 0;
 
     if (wave_active) {
-      // ---- QK^T: two 32-key blocks, ONE live accumulator ----------
-      // (sequential kb keeps a single f32x16 accP: -16 VGPR, which is
-      // what lifts the D=128 variant from 1 to 2 waves/SIMD)
-      const float* mrow = reinterpret_cast<const float*>(smem + offM[cur]);
-      float p[32];
-      float pmax = -1e30f;
+      // ---- QK^T: two 32-key blocks, side by side ------------------------
+      f32x16 sc[2];
+      const f32x16 zero = {};
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb) {
-        f32x16 accP;
+      for (int s = 0; s < D / 16; ++s)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) accP[i] = 0.f;
-        __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-        for (int s = 0; s < D / 16; ++s) {
+        for (int kb = 0; kb < 2; ++kb) {
           const int key = kb * 32 + (lane & 31);
-          const int chunk = (s * 16 + h * 8) / 8;
-          const int swz = chunk ^ (key & (NCH - 1));
-          bf16x8 kf = *reinterpret_cast<const bf16x8*>(
+          const int swz = (s * 2 + h) ^ (key & (NCH - 1));
+          const bf16x8 kf = *reinterpret_cast<const bf16x8*>(
               smem + offK[cur] + key * (2 * D) + swz * 16);
-          accP = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-              kf, qf[s], accP, 0, 0, 0);
+          sc[kb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+              kf, qf[s], s == 0 ? zero : sc[kb], 0, 0, 0);
         }
 #pragma unroll
-        for (int s = 0; s < ROT / 16; ++s) {
+      for (int s = 0; s < ROT / 16; ++s)
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) {
           const int key = kb * 32 + (lane & 31);
-          bf16x8 kf = *reinterpret_cast<const bf16x8*>(
+          const bf16x8 kf = *reinterpret_cast<const bf16x8*>(
               smem + offR + cur * RTILE_B + key * (2 * ROT) +
               (((s * 2 + h) ^ (key & 7)) * 16));
-          accP = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-              kf, qf[D / 16 + s], accP, 0, 0, 0);
+          sc[kb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+              kf, qf[D / 16 + s], sc[kb], 0, 0, 0);
         }
-        __builtin_amdgcn_s_setprio(0);
+      // ---- scores in log2 units; r of a block is key
+      // (r & 3) + 8 (r >> 2) + 4 h ---------------------------------------
+      bool masked;  // whether a row of the wave does not see a key
+      if (WINDOW)
+        masked = k0 + KVBLK - 1 > q0w + shift ||
+                 k0 <= q0w + QWAVE - 1 + shift - window;
+      else
+        masked = k0 + KVBLK > SKV || (CAUSAL && k0 + KVBLK - 1 > q0w) ||
+                 (HAS_MASK && __any(mask_lds[cur * KVBLK + lane] != 0.f));
+      float pmax = -INFINITY, off, mul;
+      if (masked) {
+        const unsigned int wspan = WINDOW ? qpos - qlo : 0;
+        const int woff = k0 + 4 * h - qlo;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int key_loc = kb * 32 + (r & 3) + 8 * (r >> 2) + 4 * h;
-          float s2 = accP[r] * scale2;
-          if (tile_masked) s2 += mrow[key_loc];
-          if (WINDOW) {
-            const int e = woff + kb * 32 + (r & 3) + 8 * (r >> 2);
-            s2 = (unsigned int)e <= wspan ? s2 : -INFINITY;
-          } else if (CAUSAL && (k0 + key_loc > qrow_abs)) {
-            s2 = -INFINITY;
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            f32x4 mv = {0.f, 0.f, 0.f, 0.f};
+            if (HAS_MASK)
+              mv = *reinterpret_cast<const f32x4*>(
+                  mask_lds + cur * KVBLK + kb * 32 + g * 8 + 4 * h);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              const int e = kb * 32 + g * 8 + j;  // key - k0 - 4h
+              float s2 = sc[kb][g * 4 + j] * scale2;
+              if (HAS_MASK) s2 += mv[j] * LOG2E;
+              // WINDOW: key k is visible when 0 <= k - qlo <= qpos - qlo,
+              // one unsigned compare
+              if (WINDOW)
+                s2 = (unsigned int)(woff + e) <= wspan ? s2 : -INFINITY;
+              else {
+                if (CAUSAL && k0 + 4 * h + e > qrow_abs) s2 = -INFINITY;
+                if (k0 + 4 * h + e >= SKV) s2 = -INFINITY;
+              }
+              sc[kb][g * 4 + j] = s2;
+              pmax = fmaxf(pmax, s2);
+            }
           }
-          p[kb * 16 + r] = s2;
-          pmax = fmaxf(pmax, s2);
-        }
+        mul = 1.f;
+      } else {
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) pmax = fmaxf(pmax, sc[kb][r]);
+        pmax *= scale2;
+        mul = scale2;
       }
       pmax = fmaxf(pmax, __shfl_xor(pmax, 32, 64));
-      // defer-max (guide T13, THR=8 in log2 units): skip the O rescale
-      // while the running max has not grown by more than THR — P is then
-      // bounded by 2^THR, which the fp32 l/O accumulation absorbs. The
-      // decision covers THIS tile's P entirely (textbook-safe order:
-      // nothing of this tile is exponentiated before the decision).
-      float mn = m, alpha = 1.f;
+      // defer-max (THR=8 in log2 units): skip the O rescale while the
+      // running max has not grown by more than THR — P is then bounded by
+      // 2^THR, which the fp32 l/O accumulation absorbs. The decision covers
+      // THIS tile's P entirely (nothing of this tile is exponentiated
+      // before the decision).
+      float alpha = 1.f;
       if (!__all(pmax - m <= 8.f)) {
-        mn = fmaxf(fmaxf(m, pmax), -1e30f);
+        const float mn = fmaxf(fmaxf(m, pmax), -1e30f);
         alpha = __builtin_amdgcn_exp2f(m - mn);
+        m = mn;
 #pragma unroll
         for (int d = 0; d < DBLK; ++d)
 #pragma unroll
           for (int i = 0; i < 16; ++i) accO[d][i] *= alpha;
       }
-      float rs = 0.f;
+      off = -m;
+      float rs[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int r = 0; r < 32; ++r) {
-        p[r] = __builtin_amdgcn_exp2f(p[r] - mn);
-        rs += p[r];
-      }
-      rs += __shfl_xor(rs, 32, 64);
-      l = l * alpha + rs;
-      m = mn;
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          sc[kb][r] = __builtin_amdgcn_exp2f(fmaf(sc[kb][r], mul, off));
+          rs[r & 3] += sc[kb][r];
+        }
+      float rsum = (rs[0] + rs[1]) + (rs[2] + rs[3]);
+      rsum += __shfl_xor(rsum, 32, 64);
+      l = l * alpha + rsum;
 
-      // ---- P -> bf16 fragments + PV, per kh (one pa live at a time:
-      // -12 VGPR vs materializing all four fragments) ----------------
-      const unsigned short* vimg =
-          reinterpret_cast<const unsigned short*>(smem + offV[cur]);
+      // ---- PV, 16 keys at a time --------------------------------------
 #pragma unroll
       for (int kh = 0; kh < 4; ++kh) {
-        const float* pp = p + (kh >> 1) * 16 + (kh & 1) * 8;
-        unsigned int a0 = ((unsigned int)f2bf(pp[0])) |
-                          ((unsigned int)f2bf(pp[1]) << 16);
-        unsigned int b0 = ((unsigned int)f2bf(pp[4])) |
-                          ((unsigned int)f2bf(pp[5]) << 16);
-        unsigned int a1 = ((unsigned int)f2bf(pp[2])) |
-                          ((unsigned int)f2bf(pp[3]) << 16);
-        unsigned int b1 = ((unsigned int)f2bf(pp[6])) |
-                          ((unsigned int)f2bf(pp[7]) << 16);
-        i32x2 s0 = __builtin_amdgcn_permlane32_swap((int)a0, (int)b0,
-                                                    false, false);
-        i32x2 s1 = __builtin_amdgcn_permlane32_swap((int)a1, (int)b1,
-                                                    false, false);
         frag_u pa;
-        pa.d[0] = (unsigned int)s0[0];
-        pa.d[1] = (unsigned int)s1[0];
-        pa.d[2] = (unsigned int)s0[1];
-        pa.d[3] = (unsigned int)s1[1];
-        __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          pa.d[i] = pack_bf16(sc[kh >> 1][(kh & 1) * 8 + i * 2],
+                              sc[kh >> 1][(kh & 1) * 8 + i * 2 + 1]);
 #pragma unroll
         for (int d = 0; d < DBLK; ++d) {
-          bf16x8 vf;
-          if (VDIRECT) {
-            // strided-but-coalesced global reads (per i: 64 lanes hit
-            // 2 key rows of consecutive d) served from L1/L2
+          frag_u vf;
+          const char* src = smem + offV[cur] + v_off[d & 1] + (d >> 1) * 128 +
+                            kh * 16 * (2 * DV);
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-              int key = k0 + kh * 16 + h * 8 + i;
-              if (key >= SKV) key = SKV - 1;
-              vf[i] = *reinterpret_cast<const __bf16*>(
-                  Vb + (long)key * tstr_k + d * 32 + (lane & 31));
-            }
-          } else if (WINDOW) {
-            const int row = d * 32 + (lane & 31);
-            vf = *reinterpret_cast<const bf16x8*>(
-                vimg + row * VR +
-                ((kh * 2 + h) ^ ((row ^ (row >> 3)) & 7)) * 8);
-          } else {
-            vf = *reinterpret_cast<const bf16x8*>(
-                vimg + (d * 32 + (lane & 31)) * VR + kh * 16 + h * 8);
-          }
+          for (int j = 0; j < 2; ++j)
+            vf.h[j] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                (__attribute__((address_space(3))) s16x4*)(
+                    src + j * 8 * (2 * DV)));
           accO[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-              vf, pa.v, accO[d], 0, 0, 0);
+              vf.v, pa.v, accO[d], 0, 0, 0);
         }
-        __builtin_amdgcn_s_setprio(0);
       }
     }
 
-    if (have_next) {
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // V regs + glds
-      if (!VDIRECT) v_write(cur ^ 1, vreg);
-      stage_m(k0 + KVBLK, cur ^ 1);
-    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();  // ONE barrier per tile
     cur ^= 1;
   }
 
-  // ---- epilogue: O^T regs -> padded LDS -> coalesced bf16 stores ------
+  // ---- epilogue: a swap of lane halves leaves 8 columns on each ---------
   float inv_l = (l > 0.f) ? 1.f / l : 0.f;
   if (WINDOW && sink != nullptr && l > 0.f) {
     const float s = sink[head] * LOG2E, top = fmaxf(m, s);
@@ -492,44 +425,26 @@ attn_fwd_kernel(const unsigned short* __restrict__ Q,
   }
   if (WINDOW && gate != nullptr)
     inv_l *= sigmoid_exact(bf2f(gate[(cu[b] + (long)qload) * ld_gate + head]));
-  float* oimg = reinterpret_cast<float*>(smem) + wid * QWAVE * (DV + 1);
 #pragma unroll
   for (int d = 0; d < DBLK; ++d)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int drow = d * 32 + (r & 3) + 8 * (r >> 2) + 4 * h;
-      oimg[qcol * (DV + 1) + drow] = accO[d][r] * inv_l;
-    }
-  __syncthreads();
-
-  if (q0w < SQ) {
-    if (DV >= 128) {
-      for (int q = 0; q < QWAVE; ++q) {
-        const int qa = q0w + q;
-        if (qa >= SQ) break;
+    for (int g = 0; g < 4; g += 2) {
+      unsigned int w[2][2];
 #pragma unroll
-        for (int c = 0; c < DV; c += 128) {
-          float v0 = oimg[q * (DV + 1) + c + lane * 2];
-          float v1 = oimg[q * (DV + 1) + c + lane * 2 + 1];
-          unsigned int pk = ((unsigned int)f2bf(v0)) |
-                            ((unsigned int)f2bf(v1) << 16);
-          *reinterpret_cast<unsigned int*>(Ob + (long)qa * ostride + c +
-                                           lane * 2) = pk;
-        }
-      }
-    } else {
-      for (int q = 0; q < QWAVE; q += 2) {
-        const int qa = q0w + q + h;
-        if (qa < SQ) {
-          const int col = (lane & 31) * 2;
-          float v0 = oimg[(q + h) * (DV + 1) + col];
-          float v1 = oimg[(q + h) * (DV + 1) + col + 1];
-          unsigned int pk = ((unsigned int)f2bf(v0)) |
-                            ((unsigned int)f2bf(v1) << 16);
-          *reinterpret_cast<unsigned int*>(Ob + (long)qa * ostride + col) =
-              pk;
-        }
-      }
+      for (int e = 0; e < 2; ++e)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+          w[e][i] = pack_bf16(accO[d][(g + e) * 4 + i * 2] * inv_l,
+                              accO[d][(g + e) * 4 + i * 2 + 1] * inv_l);
+      const i32x2 s0 = __builtin_amdgcn_permlane32_swap((int)w[0][0],
+                                                        (int)w[1][0], false,
+                                                        false);
+      const i32x2 s1 = __builtin_amdgcn_permlane32_swap((int)w[0][1],
+                                                        (int)w[1][1], false,
+                                                        false);
+      if (qrow_abs < SQ)
+        *reinterpret_cast<i32x4*>(Ob + (long)qrow_abs * ostride + d * 32 +
+                                  g * 8 + h * 8) =
+            i32x4{s0[0], s1[0], s0[1], s1[1]};
     }
-  }
 }

@@ -25,7 +25,7 @@ void launch_attn_fwd(const void*, const void*, const void*, const float*,
                      long, long, long, hipStream_t);
 void launch_attn_varlen(const void*, const void*, const void*, void*,
                         const int*, const int*, const int*, int, int, int,
-                        int, int, float, hipStream_t);
+                        int, int, int, long, long, float, hipStream_t);
 void launch_rope(const void*, void*, const float*, const float*, const int*,
                  long, int, int, int, hipStream_t);
 void launch_topk_chunk(const float*, const int*, float*, int*, int, long, int,
@@ -149,6 +149,11 @@ torch::Tensor adjacent_cosine(torch::Tensor emb) {
 }
 
 // ---- attention -------------------------------------------------------------
+static bool in_16s(const torch::Tensor& t) {
+  return (uintptr_t)t.data_ptr() % 16 == 0 && t.stride(0) % 8 == 0 &&
+         t.stride(1) % 8 == 0;
+}
+
 torch::Tensor attn_fwd(torch::Tensor Q, torch::Tensor K, torch::Tensor V,
                        c10::optional<torch::Tensor> mask, bool causal,
                        double scale) {
@@ -175,6 +180,11 @@ torch::Tensor attn_fwd(torch::Tensor Q, torch::Tensor K, torch::Tensor V,
     mp = mask->data_ptr<float>();
   }
   auto O = torch::empty({B, SQ, H, D}, Q.options());
+  // keys and values are copied 16 bytes at a time
+  if (!in_16s(K) || !in_16s(V)) {
+    K = K.clone(at::MemoryFormat::Contiguous);
+    V = V.clone(at::MemoryFormat::Contiguous);
+  }
   launch_attn_fwd(Q.data_ptr(), K.data_ptr(), V.data_ptr(), mp, O.data_ptr(),
                   B, SQ, SKV, H, HKV, D, causal, (float)scale,
                   (long)Q.stride(0), (long)Q.stride(1), (long)K.stride(0),
@@ -185,10 +195,12 @@ torch::Tensor attn_fwd(torch::Tensor Q, torch::Tensor K, torch::Tensor V,
 torch::Tensor attn_varlen(torch::Tensor Q, torch::Tensor K, torch::Tensor V,
                           torch::Tensor cu, torch::Tensor blk_seq,
                           torch::Tensor blk_qb, double scale) {
-  // packed [T, H(KV), D] bf16; cu int32 [B+1]; blk_* int32 [nblocks]
-  CHECK_DEV(Q); CHECK_CONT(Q); CHECK_BF16(Q);
-  CHECK_DEV(K); CHECK_CONT(K); CHECK_BF16(K);
-  CHECK_DEV(V); CHECK_CONT(V); CHECK_BF16(V);
+  // packed [T, H(KV), D] bf16, heads side by side in a row, rows of any
+  // stride that is a multiple of 16 bytes (K's and V's the same); cu int32
+  // [B+1]; blk_* int32 [nblocks]
+  CHECK_DEV(Q); CHECK_BF16(Q);
+  CHECK_DEV(K); CHECK_BF16(K);
+  CHECK_DEV(V); CHECK_BF16(V);
   CHECK_DEV(cu); CHECK_CONT(cu);
   CHECK_DEV(blk_seq); CHECK_CONT(blk_seq);
   CHECK_DEV(blk_qb); CHECK_CONT(blk_qb);
@@ -196,17 +208,23 @@ torch::Tensor attn_varlen(torch::Tensor Q, torch::Tensor K, torch::Tensor V,
               blk_seq.scalar_type() == torch::kInt32 &&
               blk_qb.scalar_type() == torch::kInt32,
               "cu/blk maps must be int32");
-  const int H = Q.size(1), D = Q.size(2), HKV = K.size(1);
+  const int T = Q.size(0), H = Q.size(1), D = Q.size(2), HKV = K.size(1);
   const int B = cu.size(0) - 1, nblocks = blk_seq.size(0);
   TORCH_CHECK(D == 64 || D == 128, "head_dim must be 64 or 128");
   TORCH_CHECK(H % HKV == 0, "GQA requires H % HKV == 0");
-  // zeros: rows past cu[B] (padding added to keep GEMM shapes 256-
-  // aligned) are not covered by the block map and must stay inert
-  auto O = torch::zeros_like(Q);
+  for (const auto& t : {Q, K, V})
+    TORCH_CHECK(t.stride(2) == 1 && t.stride(1) == D &&
+                    t.stride(0) % 8 == 0 &&
+                    (uintptr_t)t.data_ptr() % 16 == 0,
+                "heads must be neighbours, rows aligned to 16 bytes");
+  TORCH_CHECK(K.stride(0) == V.stride(0), "K/V must share layout");
+  // rows past cu[B] (padding added to keep GEMM shapes 256-aligned) are not
+  // covered by the block map and are zeroed
+  auto O = torch::empty({T, H, D}, Q.options());
   launch_attn_varlen(Q.data_ptr(), K.data_ptr(), V.data_ptr(), O.data_ptr(),
                      cu.data_ptr<int>(), blk_seq.data_ptr<int>(),
-                     blk_qb.data_ptr<int>(), nblocks, B, H, HKV, D,
-                     (float)scale, cur_stream());
+                     blk_qb.data_ptr<int>(), nblocks, B, T, H, HKV, D,
+                     Q.stride(0), K.stride(0), (float)scale, cur_stream());
   return O;
 }
 

@@ -10,16 +10,11 @@ extern "C" void launch_attn_window(
     int nblocks, int B, int H, int DK, int DV, long tstr_q, long tstr_kv,
     int window, float scale, const float* sink, const void* gate, int ld_gate,
     hipStream_t stream) {
-  const int nwave = 4;
   const int rot = Kr != nullptr ? 64 : 0;
-  const int ktile = KVBLK * (DK + rot) * 2, vtile = DV * KVBLK * 2;
-  const int stage_b = 2 * ktile + 2 * vtile;
-  const int epi_b = nwave * QWAVE * (DV + 1) * 4;
-  const int lds = stage_b > epi_b ? stage_b : epi_b;
 #define AWN(KK, VV, RO)                                                       \
   hipLaunchKernelGGL(                                                         \
-      (attn_fwd_kernel<KK, true, false, false, true, VV, true, RO>),          \
-      dim3(nblocks * H), dim3(nwave * 64), lds, stream,                       \
+      (attn_fwd_kernel<KK, true, false, true, VV, true, RO>),                 \
+      dim3(nblocks * H), dim3(256), attn_lds(KK, VV, RO, false), stream,      \
       (const unsigned short*)Q, (const unsigned short*)K,                     \
       (const unsigned short*)V, (const float*)nullptr, (unsigned short*)O, B, \
       0, 0, H, H, scale, 0L, tstr_q, 0L, tstr_kv, cu_q, blk_seq, blk_qb,      \
