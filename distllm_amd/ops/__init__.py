@@ -173,21 +173,31 @@ def _autotune_gemm(x2, weight, bias, act):
     return min(times, key=times.get)
 
 
-def _decode_splitk(M, N, K):
-    """SPLITK so (N/64)*SPLITK lands near the CU count (256-512):
-    narrow projections (k/v heads) need deep K splits to fill the chip."""
-    ncb = N // 64
-    for sk in (16, 8, 4, 2, 1):
-        if ncb * sk <= 512 and K % (64 * sk) == 0:
-            return sk
-    return 1
+# activation codes of decode_gemm for those of linear
+_DECODE_ACT = {ACT_NONE: 0, ACT_GELU_TANH: 6, ACT_GELU_ERF: 7, ACT_SILU: 8}
+
+
+def _few_rows(x2, N, columns=64):
+    """Whether a product of x2 with N columns and an activation in the same
+    launch takes decode_gemm (csrc/decode_gemm.hip): up to 64 rows it is
+    faster than the library's product at every size measured (64 rows of
+    28672 x 4096, gated: 51 against 57 us; 768 x 768: 3.8 against 7), up to 256
+    where the product is narrow enough for the launch that it saves to count
+    (128 rows of 16384 x 2048, gated: 20 against 23 us, of 28672 x 4096: 64
+    against 59). K of a single 64-wide chunk, which would leave three of a
+    workgroup's four waves idle, keeps its general path."""
+    M, K = x2.shape
+    return (x2.dtype == torch.bfloat16 and x2.is_contiguous()
+            and K % 64 == 0 and K >= 128 and N % columns == 0
+            and (M <= 64 or (M <= 256 and N <= 16384)))
 
 
 def linear(x, weight, bias=None, act=ACT_NONE):
     """Linear layer entry used by models. GPU path: autotuned choice
-    between hipBLASLt (plain and fused-epilogue), the hand-written
-    MFMA GEMMs (gemm8.hip, 8-phase gemm16.hip) and the skinny-M
-    split-K decode GEMM (decode_gemm.hip) for M <= 256. Override with
+    between hipBLASLt (plain and fused-epilogue) and the hand-written
+    MFMA GEMMs (gemm8.hip, 8-phase gemm16.hip); the products of few rows
+    (decode_gemm.hip, with the activation) for M <= 64 and among the
+    choices for M <= 256. Override with
     DISTLLM_GEMM=blaslt|gemm8|gemm16|decode."""
     import os
 
@@ -200,18 +210,19 @@ def linear(x, weight, bias=None, act=ACT_NONE):
         mode = os.environ.get("DISTLLM_GEMM", "auto")
         if x2.dtype == torch.float32:  # true 32-bit products
             mode = "blaslt"
+        if mode != "blaslt" and M <= 64 and _few_rows(x2, N):
+            out = _hip_ops.decode_gemm(x2, weight, bias, 0, _DECODE_ACT[act])
+            return out.reshape(*orig_shape[:-1], N)
         if (mode != "blaslt" and act == ACT_NONE and M <= 256
                 and N % 64 == 0 and K % 64 == 0 and x2.is_contiguous()):
             if mode == "decode":  # forced in-chain A/B (profiling)
-                sk = _decode_splitk(M, N, K)
-                out = _hip_ops.decode_gemm(x2, weight, bias, sk)
+                out = _hip_ops.decode_gemm(x2, weight, bias, 0)
                 return out.reshape(*orig_shape[:-1], N)
             # bucket by padded M so varying decode/prefill
             # batch sizes reuse one tuning decision
             key = ("dec", 128 if M <= 128 else 256, N, K,
                    bias is not None)
             choice = _GEMM_CHOICE.get(key)
-            sk = _decode_splitk(M, N, K)
             if choice is None:
                 import time as _t
 
@@ -228,7 +239,7 @@ def linear(x, weight, bias=None, act=ACT_NONE):
                     "blaslt": timeit(lambda: torch.nn.functional.linear(
                         x2, weight, bias)),
                     "decode": timeit(lambda: _hip_ops.decode_gemm(
-                        x2, weight, bias, sk)),
+                        x2, weight, bias, 0)),
                 }
                 try:  # hipBLASLt with measured algo search (blt_gemm.cpp)
                     times["blt_fused"] = timeit(
@@ -238,7 +249,7 @@ def linear(x, weight, bias=None, act=ACT_NONE):
                 choice = min(times, key=times.get)
                 _GEMM_CHOICE[key] = choice
             if choice == "decode":
-                out = _hip_ops.decode_gemm(x2, weight, bias, sk)
+                out = _hip_ops.decode_gemm(x2, weight, bias, 0)
             elif choice == "blt_fused":
                 out = _blt_fused_path(x2, weight, bias, act)
             else:
@@ -395,19 +406,17 @@ def rope_apply(x, cs, sn, pos, rope_heads: int = -1):
 
 def gateup_swiglu(x, wgup, bias=None):
     """silu(x @ Wg^T) * (x @ Wu^T) with Wg|Wu packed as wgup [2I, K].
-    Decode path (M <= 256): ONE split-K GEMM with the swiglu fused into
-    its reduce; otherwise one big GEMM + packed swiglu."""
+    Few rows: ONE product with the swiglu in the same launch; otherwise one
+    big GEMM + packed swiglu."""
     orig_shape = x.shape
     x2 = x.reshape(-1, orig_shape[-1])
     M, K = x2.shape
     I = wgup.shape[0] // 2
     if x.is_cuda:
         _require_hip("_hip_gemm")
-        if M <= 256 and wgup.shape[0] % 128 == 0 and x2.is_contiguous():
-            sk = _decode_splitk(M, wgup.shape[0], K)
-            if sk > 1:
-                out = _hip_ops.decode_gemm(x2, wgup, bias, sk, 1)
-                return out.reshape(*orig_shape[:-1], I)
+        if _few_rows(x2, wgup.shape[0], 128):
+            out = _hip_ops.decode_gemm(x2, wgup, bias, 0, 1)
+            return out.reshape(*orig_shape[:-1], I)
     gu = linear(x2, wgup, bias)
     if gu.is_cuda:
         out = _hip_ops.swiglu_packed(gu.contiguous())
@@ -419,17 +428,12 @@ def gateup_swiglu(x, wgup, bias=None):
 def gateup_clamped_glu(x, wgup, limit, alpha, shift):
     """Clamped gated unit of x @ Wg^T and x @ Wu^T, Wg|Wu packed as wgup
     [2I, K]: min(g, limit) * sigmoid(alpha * g) * (clamp(u) + shift), all
-    with the clamped g. Decode-sized inputs fuse it into the split-K
-    reduce of ONE GEMM, as gateup_swiglu does."""
-    M, K = x.shape
+    with the clamped g. For few rows ONE launch, as gateup_swiglu."""
     if x.is_cuda:
         _require_hip("_hip_gemm")
-        if (M <= 256 and x.dtype == torch.bfloat16 and K % 64 == 0
-                and wgup.shape[0] % 128 == 0):
-            sk = _decode_splitk(M, wgup.shape[0], K)
-            if sk > 1:
-                return _hip_ops.decode_gemm(x, wgup, None, sk, 2, limit,
-                                            alpha, shift)
+        if _few_rows(x, wgup.shape[0], 128):
+            return _hip_ops.decode_gemm(x, wgup, None, 0, 2, limit, alpha,
+                                        shift)
         return _hip_ops.clamped_glu(linear(x, wgup), limit, alpha, shift)
     return torch_ref.clamped_glu(linear(x, wgup), limit, alpha, shift)
 
@@ -743,16 +747,11 @@ def gated_delta(ab, heads, kv_heads, dp, vp, dim, vdim, conv_w, decay,
 
 def up_xielu(x, wup, act):
     """xielu(x @ wup^T); act: the activation's two raw numbers."""
-    M, K = x.shape
     if x.is_cuda:
         _require_hip("_hip_gemm")
         _require_hip("_hip_experts")
-        if (M <= 256 and x.dtype == torch.bfloat16 and K % 64 == 0
-                and wup.shape[0] % 64 == 0):
-            sk = _decode_splitk(M, wup.shape[0], K)
-            if sk > 1:
-                return _hip_ops.decode_gemm(x, wup, None, sk, 3,
-                                            act_nums=act)
+        if _few_rows(x, wup.shape[0]):
+            return _hip_ops.decode_gemm(x, wup, None, 0, 3, act_nums=act)
         return _hip_ops.xielu(linear(x, wup), act)
     return torch_ref.xielu(linear(x, wup), act)
 
@@ -801,14 +800,10 @@ def route_sigmoid(h, router, correction, ctx, top, scale, shards=0):
 
 def up_relu2(x, wup):
     """The square of relu(x @ wup^T)."""
-    M, K = x.shape
     if x.is_cuda:
         _require_hip("_hip_gemm")
-        if (M <= 256 and x.dtype == torch.bfloat16 and K % 64 == 0
-                and wup.shape[0] % 64 == 0):
-            sk = _decode_splitk(M, wup.shape[0], K)
-            if sk > 1:
-                return _hip_ops.decode_gemm(x, wup, None, sk, 5)
+        if _few_rows(x, wup.shape[0]):
+            return _hip_ops.decode_gemm(x, wup, None, 0, 5)
         return _hip_ops.relu2(linear(x, wup))
     return torch_ref.relu2(linear(x, wup))
 
@@ -846,12 +841,9 @@ def gated_rows(x, wgate, tokens, table, col0, n):
     columns of wgate behind n."""
     if x.is_cuda:
         _require_hip("_hip_gemm")
-        M, K = x.shape
-        if (M <= 256 and x.dtype == torch.bfloat16 and K % 64 == 0):
-            sk = _decode_splitk(M, wgate.shape[0], K)
-            if sk > 1:
-                return _hip_ops.decode_gemm_rows(x, wgate, sk, tokens, table,
-                                                 col0, n)
+        if _few_rows(x, wgate.shape[0]):
+            return _hip_ops.decode_gemm_rows(x, wgate, 0, tokens, table,
+                                             col0, n)
         return _hip_ops.gelu_rows(linear(x, wgate), tokens, table, col0, n)
     return torch_ref.gelu_rows(linear(x, wgate), tokens, table, col0, n)
 

@@ -12,8 +12,9 @@ void launch_gemm8_bf16(const void*, const void*, const void*, void*, int, int,
 void launch_gemm16_bf16(const void*, const void*, const void*, void*, int,
                         int, int, int, hipStream_t);
 void launch_decode_gemm(const void*, const void*, const void*, void*, void*,
-                        int, int, int, int, int, float, float, float,
+                        int, int, int, int, bool, int, float, float, float,
                         const float*, const RowsArgs*, hipStream_t);
+int decode_gemm_shares(int, int, int);
 void launch_clamped_glu(const void*, void*, long, int, float, float, float,
                         bool, hipStream_t);
 void launch_relu2(const void*, void*, long, bool, hipStream_t);
@@ -74,19 +75,24 @@ static torch::Tensor decode_gemm_act(torch::Tensor X, torch::Tensor W,
                                      double shift,
                                      c10::optional<torch::Tensor> act_nums,
                                      const RowsArgs* rows) {
-  // act 1, 2 = packed gated unit in the reduce (swiglu, clamped with the
-  // given constants): W is [2I, K] (gate rows then up rows), output is
-  // [M, I]. act 3 = xIELU with the raw numbers act_nums [2]. act 4 = GELU
-  // times a part of a table's row. act 5 = relu(.)^2. All require splitk > 1.
+  // act 1, 2 = packed gated unit (swiglu, clamped with the given constants):
+  // W is [2I, K] (gate rows then up rows), output is [M, I]. act 3 = xIELU
+  // with the raw numbers act_nums [2]. act 4 = GELU times a part of a table's
+  // row. act 5 = relu(.)^2. act 6, 7, 8 = GELU (tanh, erf), SiLU. splitk
+  // workgroups share K (activations: not 1); 0: form and split follow from
+  // the sizes.
   CHECK_DEV(X); CHECK_CONT(X); CHECK_BF16(X);
   CHECK_DEV(W); CHECK_CONT(W); CHECK_BF16(W);
   const int M = X.size(0), K = X.size(1), N = W.size(0);
   TORCH_CHECK(W.size(1) == K, "K mismatch");
   TORCH_CHECK(M <= 256, "decode_gemm is for M <= 256");
   TORCH_CHECK(N % 64 == 0, "N % 64");
-  TORCH_CHECK(K % (64 * splitk) == 0, "K % (64*splitk)");
+  const bool tile = splitk != 0;
+  if (!tile) splitk = decode_gemm_shares(M, N, K);
+  TORCH_CHECK(splitk > 0 && K % (64 * splitk) == 0, "K % (64*splitk)");
   const bool glu = act == 1 || act == 2;
-  TORCH_CHECK(act == 0 || splitk > 1, "a fused activation needs splitk > 1");
+  TORCH_CHECK(act == 0 || !tile || splitk > 1,
+              "a fused activation needs splitk > 1");
   TORCH_CHECK(!glu || N % 128 == 0, "gated-unit fusion needs N % 128 == 0");
   const float* nums = nullptr;
   if (act == 3) {
@@ -94,19 +100,20 @@ static torch::Tensor decode_gemm_act(torch::Tensor X, torch::Tensor W,
     CHECK_DEV(act_nums.value()); CHECK_F32(act_nums.value());
     nums = act_nums->data_ptr<float>();
   }
-  const int MP = M <= 128 ? 128 : 256;
   auto out = torch::empty({M, glu ? N / 2 : N}, X.options());
+  if (M == 0) return out;
   torch::Tensor slabs;
   void* slabp = nullptr;
   if (splitk > 1) {
-    slabs = torch::empty({splitk, (long)MP, (long)N},
+    slabs = torch::empty({splitk, (long)M, (long)N},
                          X.options().dtype(at::kFloat));
     slabp = slabs.data_ptr();
   }
   launch_decode_gemm(X.data_ptr(), W.data_ptr(),
                      bias ? bias->data_ptr() : nullptr, out.data_ptr(),
-                     slabp, M, N, K, (int)splitk, (int)act, (float)limit,
-                     (float)alpha, (float)shift, nums, rows, cur_stream());
+                     slabp, M, N, K, (int)splitk, tile, (int)act,
+                     (float)limit, (float)alpha, (float)shift, nums, rows,
+                     cur_stream());
   return out;
 }
 
@@ -116,7 +123,7 @@ torch::Tensor decode_gemm(torch::Tensor X, torch::Tensor W,
                           double limit = 0.0, double alpha = 0.0,
                           double shift = 0.0,
                           c10::optional<torch::Tensor> act_nums = {}) {
-  TORCH_CHECK((act >= 0 && act <= 3) || act == 5, "activation");
+  TORCH_CHECK(act >= 0 && act <= 8 && act != 4, "activation");
   return decode_gemm_act(X, W, bias, splitk, act, limit, alpha, shift,
                          act_nums, nullptr);
 }

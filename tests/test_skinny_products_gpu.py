@@ -1,0 +1,91 @@
+"""Products of few rows in every form (direct, ring, tile, shared K) at the
+edges of their ranges, with every activation."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from distllm_amd import ops
+from distllm_amd.ops import torch_ref
+
+pytestmark = pytest.mark.gpu
+
+ROWS = [1, 2, 3, 15, 16, 17, 32, 33, 64, 65, 128, 129, 256]
+# least sizes; K of one, of fewer chunks than waves or buffers, of odd
+# chunk counts; columns that change the form at 17 to 32 rows
+SIZES = [(64, 64), (64, 192), (192, 320), (768, 768), (128, 3072),
+         (8192, 256), (8320, 448)]
+
+
+def _inputs(M, N, K, device, seed):
+    g = torch.Generator(device=device).manual_seed(seed)
+
+    def some(*s):
+        return torch.randn(*s, device=device, generator=g).to(torch.bfloat16)
+
+    return some(M, K), some(N, K) * K ** -0.5, some(N)
+
+
+def _close(out, ref):
+    # both sides sum in fp32; what is left is the rounding of the result
+    # (2^-9 of it) and of sums that cancel
+    torch.testing.assert_close(out.float(), ref, atol=4e-3, rtol=8e-3)
+
+
+@pytest.mark.parametrize("N,K", SIZES)
+@pytest.mark.parametrize("M", ROWS)
+def test_forms(device, M, N, K):
+    x, w, b = _inputs(M, N, K, device, M * N + K)
+    ref = x.float() @ w.float().T
+    _close(ops._hip_ops.decode_gemm(x, w, None, 0), ref)
+    _close(ops._hip_ops.decode_gemm(x, w, b, 0), ref + b.float())
+    for share in (1, 2, 5):
+        if K % (64 * share) == 0:
+            _close(ops._hip_ops.decode_gemm(x, w, b, share), ref + b.float())
+
+
+@pytest.mark.parametrize("M", [1, 2, 9, 24, 48, 100, 200])
+@pytest.mark.parametrize("share", [0, 2])
+def test_activations(device, M, share):
+    N, K = 256, 512
+    x, w, b = _inputs(M, N, K, device, M)
+    z = x.float() @ w.float().T
+    zb = z + b.float()
+    gate, up = zb[:, : N // 2], zb[:, N // 2:]
+    act = torch.tensor([0.3, -0.2], device=device)
+    F = torch.nn.functional
+    run = ops._hip_ops.decode_gemm
+    _close(run(x, w, b, share, 1), F.silu(gate) * up)
+    _close(run(x, w, b, share, 2, 1.1, 1.702, 1.0),
+           torch_ref.clamped_glu(zb, 1.1, 1.702, 1.0).float())
+    _close(run(x, w, b, share, 3, act_nums=act), torch_ref.xielu(zb, act))
+    _close(run(x, w, b, share, 5), F.relu(zb) ** 2)
+    _close(run(x, w, b, share, 6), F.gelu(zb, approximate="tanh"))
+    _close(run(x, w, b, share, 7), F.gelu(zb))
+    _close(run(x, w, b, share, 8), F.silu(zb))
+    table = torch.randn(11, 300, device=device).to(torch.bfloat16)
+    tokens = torch.arange(M, device=device) % 11
+    rows = torch.zeros(M, N, device=device)
+    rows[:, :200] = (F.gelu(z, approximate="tanh")[:, :200]
+                     * table.float()[tokens, 30:230])
+    _close(ops._hip_ops.decode_gemm_rows(x, w, share, tokens, table, 30, 200),
+           rows)
+
+
+def test_refusals(device):
+    x, w, _ = _inputs(4, 128, 128, device, 1)
+    for args in ((x, w, None, 1, 1), (x, w, None, 3), (x, w, None, 0, 4),
+                 (x, w[:96], None, 0), (x[:, :96].contiguous(),
+                                        w[:, :96].contiguous(), None, 0)):
+        with pytest.raises(RuntimeError):
+            ops._hip_ops.decode_gemm(*args)
+
+
+@pytest.mark.parametrize("act", [ops.ACT_NONE, ops.ACT_GELU_TANH,
+                                 ops.ACT_GELU_ERF, ops.ACT_SILU])
+@pytest.mark.parametrize("M", [1, 24, 128, 130])
+def test_linear(device, M, act):
+    x, w, b = _inputs(M, 192, 256, device, M)
+    _close(ops.linear(x[None], w, b, act)[0],
+           torch_ref.gemm(x.float(), w.float(), b.float(), act).float())
