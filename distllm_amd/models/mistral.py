@@ -293,31 +293,23 @@ class DecoderModel(nn.Module):
         nh, kvh, hd = self.local_heads, self.local_kv_heads, d.head_dim
         cs, sn = self._rope(tokens.device)
         x = self.tok_emb[tokens.long()].unsqueeze(1)  # [B,1,H]
-        pos = (ctx_lens - 1).int()
-        slot = pos
+        ctx_lens, block_tables = ctx_lens.int(), block_tables.int()
         # W8A16 small-batch path: fp8 weight GEMV (enable_fp8_decode)
         fp8 = (self._fp8w if self._fp8w is not None and B <= 8
                and x.is_cuda else None)
         h = ops.rms_norm(x, self.layers[0].in_norm, eps=d.rms_norm_eps)
         for li, layer in enumerate(self.layers):
-            # ONE fused qkv GEMM + ONE rope (q|k roped, v copied):
-            # 5 launches -> 2 on the per-token critical path
+            # ONE fused qkv GEMM + ONE launch that rotates q and k and
+            # writes k and v to their pages
             if fp8 is not None:
                 f = fp8[li]
                 qkv = ops.gemv_fp8(h[:, 0], *f["wqkv"], layer.bqkv)
-                qkv = qkv.view(B, 1, nh + 2 * kvh, hd)
             else:
-                qkv = ops.linear(h, layer.wqkv,
-                                 layer.bqkv).view(B, 1, nh + 2 * kvh, hd)
-            qkv = ops.rope_apply(qkv, cs, sn, pos, rope_heads=nh + kvh)
-            q = qkv[:, 0, :nh]
-            k = qkv[:, 0, nh: nh + kvh].contiguous()
-            v = qkv[:, 0, nh + kvh:].contiguous()
-            ops.cache_put(k, v, kcaches[li], vcaches[li],
-                          block_tables, slot)
-            ctx = ops.paged_attn(q.contiguous(), kcaches[li],
-                                 vcaches[li], block_tables, ctx_lens,
-                                 scale=1.0 / math.sqrt(hd))
+                qkv = ops.linear(h, layer.wqkv, layer.bqkv)
+            q = ops.rope_put(qkv.view(B, nh + 2 * kvh, hd), cs, sn, ctx_lens,
+                             kcaches[li], vcaches[li], block_tables)
+            ctx = ops.paged_attn(q, kcaches[li], vcaches[li], block_tables,
+                                 ctx_lens, scale=1.0 / math.sqrt(hd))
             if fp8 is not None:
                 attn = self._allreduce(ops.gemv_fp8(
                     ctx.reshape(B, nh * hd), *f["wo"])).unsqueeze(1)

@@ -532,6 +532,23 @@ def cache_put(knew, vnew, kcache, vcache, block_table, slot):
         vcache[blk, :, pos % BLK] = vnew[b]
 
 
+def rope_put(qkv, cs, sn, ctx, kcache, vcache, block_table):
+    """A decode step's projections [B, H + 2 HKV, D]: queries and keys are
+    rotated by position ctx - 1; queries are returned [B, H, D], keys and
+    values go to that position of the cache, in one launch."""
+    H = qkv.shape[1] - 2 * kcache.shape[1]
+    if qkv.is_cuda and qkv.shape[2] in (64, 128):
+        _require_hip()
+        return _hip_ops.rope_put(qkv.contiguous(), cs, sn, ctx.int(), kcache,
+                                 vcache, block_table.int())
+    slot = (ctx - 1).int()
+    qkv = rope_apply(qkv, cs, sn, slot, rope_heads=H + kcache.shape[1])
+    cache_put(qkv[:, H: H + kcache.shape[1]].contiguous(),
+              qkv[:, H + kcache.shape[1]:].contiguous(), kcache, vcache,
+              block_table, slot)
+    return qkv[:, :H].contiguous()
+
+
 # ---- sandwich-norm / latent-attention decoder -----------------------------
 
 def embed_norm(tokens, table, w_next, n, eps):

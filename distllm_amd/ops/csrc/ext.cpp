@@ -38,13 +38,12 @@ void launch_gemv_fp8(const void*, const void*, const float*, const void*,
                      void*, int, int, long, hipStream_t);
 void launch_sample(const float*, const float*, int*, int, int, float, float,
                    hipStream_t);
-void launch_paged_attn_split(const void*, const void*, const void*,
-                             const int*, const int*, void*, void*, void*,
-                             int, int, int, int, int, int, float, bool,
-                             hipStream_t);
-void launch_paged_attn(const void*, const void*, const void*, const int*,
-                       const int*, void*, int, int, int, int, int, float,
-                       bool, hipStream_t);
+void launch_paged_attn(const void*, long, const void*, const void*,
+                       const int*, const int*, void*, void*, void*, int, int,
+                       int, int, int, int, float, bool, hipStream_t);
+void launch_rope_put(const void*, const float*, const float*, const int*,
+                     void*, void*, void*, const int*, int, int, int, int, int,
+                     bool, hipStream_t);
 void launch_cache_put(const void*, const void*, void*, void*, const int*,
                       const int*, int, int, int, int, bool, hipStream_t);
 }
@@ -286,6 +285,26 @@ torch::Tensor sample_tokens(torch::Tensor logits, torch::Tensor rand,
   return out;
 }
 
+static void check_kv_pages(const torch::Tensor& kcache,
+                           const torch::Tensor& vcache,
+                           const torch::Tensor& block_table,
+                           const torch::Tensor& ctx, long B, long D) {
+  CHECK_DEV(kcache); CHECK_CONT(kcache);
+  CHECK_DEV(vcache); CHECK_CONT(vcache);
+  CHECK_SAME(kcache, vcache);
+  TORCH_CHECK(kcache.scalar_type() == at::kByte ||
+                  kcache.scalar_type() == at::kBFloat16,
+              "pages are bf16 or fp8 (uint8)");
+  TORCH_CHECK(kcache.dim() == 4 && kcache.sizes() == vcache.sizes() &&
+                  kcache.size(2) == 16 && kcache.size(3) == D,
+              "pages must be [blocks, HKV, 16, D]");
+  CHECK_INTS(block_table);
+  CHECK_INTS(ctx);
+  TORCH_CHECK(block_table.dim() == 2 && block_table.size(0) == B &&
+                  ctx.numel() == B,
+              "one block-table row and context length per sequence");
+}
+
 torch::Tensor paged_attn(torch::Tensor q, torch::Tensor kcache,
                          torch::Tensor vcache, torch::Tensor block_table,
                          torch::Tensor ctx_len, double scale) {
@@ -293,43 +312,58 @@ torch::Tensor paged_attn(torch::Tensor q, torch::Tensor kcache,
   const int B = q.size(0), H = q.size(1), D = q.size(2);
   const int HKV = kcache.size(1);
   const int max_blocks = block_table.size(1);
+  TORCH_CHECK(D == 64 || D == 128, "head_dim must be 64 or 128");
+  TORCH_CHECK(H % HKV == 0, "GQA requires H % HKV == 0");
+  check_kv_pages(kcache, vcache, block_table, ctx_len, B, D);
   const bool fp8 = kcache.scalar_type() == at::kByte;
   auto out = torch::empty_like(q);
-  // Flash-decoding context split when B*HKV alone underfills the chip
-  // (small batches): parallelize over context chunks + combine pass.
-  const int GR = (HKV > 0 && H % HKV == 0) ? H / HKV : 0;
-  const bool gr_ok = (GR == 1 || GR == 2 || GR == 4 || GR == 8);
-  // Measured policy (profiles/RESULTS.md): split pays when B*HKV <= 128
-  // AND the context is long (max_blocks >= 64 i.e. >= 1k tokens) —
-  // B=1 ctx8192: 322 -> 50 us; B=32 ctx2048 regressed with split, so
-  // larger batches keep the one-pass kernel.
-  int NS = 1;
-  if (gr_ok && B * HKV <= 128 && max_blocks >= 64)
-    NS = (int)std::min<long>(std::min(512L / (B * HKV) + 1, 16L),
-                             max_blocks);
-  static const int ns_env = [] {  // probe override: 0=auto, 1=off, N
-    const char* e = getenv("DISTLLM_PA_NSPLIT");
-    return e ? atoi(e) : 0;
-  }();
-  if (ns_env > 0 && gr_ok)
-    NS = std::min(ns_env, max_blocks);
+  if (B == 0) return out;
+  // Workgroups that share a sequence: as many as make two for every CU, each
+  // with at least 256 of the positions that the block table has room for. In
+  // us, 1, 2, 4, 8, 16 shares: B = 1 of 2048 25, 18, 13, 11.2, 11.9; B = 8 of
+  // 1000 19, 16, 15, 18; B = 16 of 100 to 4000 55, 39, 38, 41, 55; B = 64 of
+  // 1124 59, 68, 82.
+  const long groups = (long)B * HKV * ((H / HKV + 15) / 16);
+  const int NS = (int)std::max<long>(
+      std::min<long>({512 / groups, max_blocks / 16, 32}), 1);
+  torch::Tensor pacc, pml;
   if (NS > 1) {
     auto f32 = q.options().dtype(at::kFloat);
-    auto pacc = torch::empty({(long)B * HKV * NS * GR, D}, f32);
-    auto pml = torch::empty({(long)B * HKV * NS * GR, 2}, f32);
-    launch_paged_attn_split(q.data_ptr(), kcache.data_ptr(),
-                            vcache.data_ptr(), block_table.data_ptr<int>(),
-                            ctx_len.data_ptr<int>(), pacc.data_ptr(),
-                            pml.data_ptr(), out.data_ptr(), B, H, HKV, D,
-                            max_blocks, NS, (float)scale, fp8,
-                            cur_stream());
-    return out;
+    pacc = torch::empty({(long)B * H * NS, D}, f32);
+    pml = torch::empty({(long)B * H * NS, 2}, f32);
   }
-  launch_paged_attn(q.data_ptr(), kcache.data_ptr(), vcache.data_ptr(),
-                    block_table.data_ptr<int>(), ctx_len.data_ptr<int>(),
-                    out.data_ptr(), B, H, HKV, D, max_blocks, (float)scale,
-                    fp8, cur_stream());
+  launch_paged_attn(q.data_ptr(), q.stride(0), kcache.data_ptr(),
+                    vcache.data_ptr(), block_table.data_ptr<int>(),
+                    ctx_len.data_ptr<int>(), out.data_ptr(),
+                    NS > 1 ? pacc.data_ptr() : nullptr,
+                    NS > 1 ? pml.data_ptr() : nullptr, B, H, HKV, D,
+                    max_blocks, NS, (float)scale, fp8, cur_stream());
   return out;
+}
+
+// qkv [B, H + 2 HKV, D] of a decode step -> rotated q [B, H, D]; rotated keys
+// and the values to their places (position ctx - 1) in the cache
+torch::Tensor rope_put(torch::Tensor qkv, torch::Tensor cs, torch::Tensor sn,
+                       torch::Tensor ctx, torch::Tensor kcache,
+                       torch::Tensor vcache, torch::Tensor block_table) {
+  CHECK_DEV(qkv); CHECK_CONT(qkv); CHECK_BF16(qkv);
+  CHECK_FLOATS(cs); CHECK_FLOATS(sn);
+  const int B = qkv.size(0), D = qkv.size(2), HKV = kcache.size(1);
+  const int H = (int)qkv.size(1) - 2 * HKV;
+  TORCH_CHECK(D == 64 || D == 128, "head_dim must be 64 or 128");
+  TORCH_CHECK(qkv.dim() == 3 && H > 0, "qkv must be [B, H + 2 HKV, D]");
+  TORCH_CHECK(cs.size(-1) == D / 2 && cs.sizes() == sn.sizes(),
+              "rotation tables must be [positions, D / 2]");
+  check_kv_pages(kcache, vcache, block_table, ctx, B, D);
+  auto q = torch::empty({B, H, D}, qkv.options());
+  if (B > 0)
+    launch_rope_put(qkv.data_ptr(), cs.data_ptr<float>(),
+                    sn.data_ptr<float>(), ctx.data_ptr<int>(), q.data_ptr(),
+                    kcache.data_ptr(), vcache.data_ptr(),
+                    block_table.data_ptr<int>(), B, H, HKV, D,
+                    block_table.size(1), kcache.scalar_type() == at::kByte,
+                    cur_stream());
+  return q;
 }
 
 void cache_put(torch::Tensor knew, torch::Tensor vnew, torch::Tensor kcache,
@@ -412,4 +446,5 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("sample_tokens", &sample_tokens);
   m.def("paged_attn", &paged_attn);
   m.def("cache_put", &cache_put);
+  m.def("rope_put", &rope_put);
 }

@@ -1,631 +1,430 @@
-// Paged-KV decode attention (single new token per sequence), bf16.
+// Paged-KV decode attention (single new token per sequence).
 // Replaces vLLM's paged attention (reference delegated generation to
 // vLLM, generate/generators/vllm_backend.py).
 //
-// Cache layout: kcache/vcache [nblocks, HKV, BLK, D] bf16, BLK=16.
+// Cache layout: kcache/vcache [nblocks, HKV, BLK, D], BLK=16, bf16 or OCP
+// fp8 e4m3 (CDNA4-native; halves decode KV bandwidth, doubles capacity;
+// values are stored unscaled, |k|,|v| << 448 in practice).
 // block_table [B, max_blocks] int32 ; ctx_len [B] int32.
-// q: [B, H, D] bf16 ; out: [B, H, D] bf16.
+// q: [B, H, D] bf16, rows of any stride ; out: [B, H, D] bf16.
 //
-// Decode is latency-bound at small contexts: the v2 kernel stages the
-// block table in LDS once, keeps the QK dot lane-per-key (independent
-// vector loads), and runs the PV accumulation branch-free with an
-// 8-deep unroll so the per-key V reads pipeline instead of serializing
-// on L2 latency. Cross-wave combine via LDS.
+// Bound by reading the cache. A workgroup has the query heads of one key
+// head (up to 16 of them: the columns of the products) and a share of the
+// sequence; its 4 waves take tiles of 32 keys (two pages) in turn and work
+// alone until their softmax states meet in LDS.
+//  - bf16 pages go to the wave's own ring of LDS buffers as they lie in the
+//    cache, whole lines by global_load_lds; fp8 pages pass through registers,
+//    the next tile's loads in flight, and are widened on the way.
+//  - scores are mfma(K, Q^T), keys on rows and heads on lanes, the output is
+//    mfma(V^T, P), columns on rows and heads on lanes, V transposed on its
+//    way out of LDS. Softmax state and rescaling are lane-local but for the
+//    maximum over the four groups of lanes that share a head.
+//  - probabilities stay fp32: each goes in as the sum of two bf16 numbers,
+//    which leaves 2^-17 of it, against the 2^-9 of the bf16 result.
+//  - NS workgroups share a sequence where B * HKV is small; a second launch
+//    joins them.
+// Measured, us, with kernels that read a key row per lane and a value element
+// per lane, and now (32 heads on 8 of 128, bf16; fp8): B = 1, 2048 cached
+// tokens 32 -> 11.2 (31 -> 11.1); B = 16 of 100 to 4000 115 -> 39 (104 -> 24);
+// B = 64 of 200 to 2048 137 -> 65, 4.5 TB/s (117 -> 38); B = 128 of 1000 150 ->
+// 100, 5.2 TB/s (96 -> 56). The 128 KiB of buffers leave one workgroup per CU.
 #include "common.h"
 #include <hip/hip_fp8.h>
 
 #define PBLK 16  // tokens per KV block
+#define KT 32    // keys of a tile
 
-__device__ __forceinline__ float fp8_to_f32(unsigned char u) {
-  __hip_fp8_e4m3 v;
-  v.__x = u;
-  return float(v);
+typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
+
+extern __shared__ __attribute__((aligned(16))) char smem[];
+
+union pa_frag {
+  bf16x8 v;
+  s16x4 h[2];
+  unsigned int d[4];
+};
+
+__device__ __forceinline__ unsigned int pa_pack(float a, float b) {
+  return __builtin_bit_cast(
+      unsigned int, __builtin_convertvector(f32x2{a, b}, bf16x2));
 }
 
-// CT: cache element type (unsigned short = bf16, unsigned char = OCP
-// fp8 e4m3 — CDNA4-native; halves decode KV bandwidth, doubles
-// capacity; values are stored unscaled, |k|,|v| << 448 in practice).
-template <int D, typename CT>
+// 16 fp8 numbers as 16 bf16 (exact)
+__device__ __forceinline__ void pa_widen(const i32x4 v, i32x4 (&out)[2]) {
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    const f32x2 lo = __builtin_amdgcn_cvt_pk_f32_fp8(v[w], false);
+    const f32x2 hi = __builtin_amdgcn_cvt_pk_f32_fp8(v[w], true);
+    out[w >> 1][(w & 1) * 2] = (int)pa_pack(lo[0], lo[1]);
+    out[w >> 1][(w & 1) * 2 + 1] = (int)pa_pack(hi[0], hi[1]);
+  }
+}
+
+constexpr int pa_ring(int D, bool fp8) { return fp8 ? 1 : D == 64 ? 4 : 2; }
+constexpr int pa_lds(int D, bool fp8) {
+  return 4 * pa_ring(D, fp8) * 2 * KT * D * 2;
+}
+
+template <int D, bool FP8>
 __global__ void __launch_bounds__(256)
-paged_attn_kernel(const unsigned short* __restrict__ q,
-                  const CT* __restrict__ kcache,
-                  const CT* __restrict__ vcache,
+paged_attn_kernel(const unsigned short* __restrict__ q, long q_stride,
+                  const char* __restrict__ kcache,
+                  const char* __restrict__ vcache,
                   const int* __restrict__ block_table,
                   const int* __restrict__ ctx_len,
-                  unsigned short* __restrict__ out, int B, int H, int HKV,
-                  int max_blocks, float scale) {
-  const int b = blockIdx.x / H;
-  const int h = blockIdx.x % H;
-  const int kvh = h / (H / HKV);
-  const int lane = threadIdx.x & 63;
-  const int wid = threadIdx.x >> 6;
-  const int L = ctx_len[b];
+                  unsigned short* __restrict__ out,
+                  float* __restrict__ pacc, float* __restrict__ pml, int H,
+                  int HKV, int max_blocks, int NS, float scale) {
+  constexpr int NCH = D / 8;            // 16-byte pieces of a bf16 row
+  constexpr int ROWS = 1024 / (2 * D);  // rows of a 1 KiB piece of a tile
+  constexpr int PIECES = KT / ROWS;     // pieces of K or V of a tile
+  constexpr int TILE = KT * D * 2;      // bytes of K or V of a tile
+  constexpr int R = pa_ring(D, FP8);
+  constexpr int DB = D / 16;
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  const int c16 = lane & 15, g = lane >> 4;
+  const int GR = H / HKV, NG = (GR + 15) / 16;
+  const int split = blockIdx.x % NS;
+  const int hg = blockIdx.x / NS % NG;
+  const int kvh = blockIdx.x / NS / NG % HKV;
+  const int b = blockIdx.x / NS / NG / HKV;
+  const int head0 = kvh * GR + hg * 16, nh = min(GR - hg * 16, 16);
 
-  extern __shared__ __attribute__((aligned(16))) char smem[];
-  float* p_lds = reinterpret_cast<float*>(smem);                 // 4*64
-  float* q_lds = p_lds + 4 * 64;                                 // D
-  float* wstate = q_lds + D;                                     // 8
-  float* wacc = wstate + 8;                                      // 4*D
-  int* bt_lds = reinterpret_cast<int*>(wacc + 4 * D);            // nblk
+  const int L = min(ctx_len[b], max_blocks * PBLK);
+  const int T = (L + KT - 1) / KT, per = (T + NS - 1) / NS;
+  const int t0 = split * per + wid, t1 = min(T, split * per + per);
+  const int mine = t1 > t0 ? (t1 - t0 + 3) / 4 : 0;  // tiles t0, t0 + 4, ...
+  const int last_page = max(L - 1, 0) / PBLK;
+  const int* bt = block_table + (long)b * max_blocks;
+  const long page_bytes = (long)HKV * PBLK * D * (FP8 ? 1 : 2);
+  const long head_bytes = (long)kvh * PBLK * D * (FP8 ? 1 : 2);
 
-  const int nblk = (L + PBLK - 1) / PBLK;
-  for (int i = threadIdx.x; i < nblk; i += 256)
-    bt_lds[i] = block_table[(long)b * max_blocks + i];
-  for (int d = threadIdx.x; d < D; d += 256)
-    q_lds[d] = bf2f(q[((long)b * H + h) * D + d]) * scale;
-  __syncthreads();
-
-  float m = -1e30f, l = 0.f;
-  float acc[2] = {0.f, 0.f};
-  constexpr int DPL = D / 64;  // d-cols per lane (1 or 2)
-  const long blk_stride = (long)HKV * PBLK * D;
-  const long head_off = (long)kvh * PBLK * D;
-
-  for (int t0 = wid * 64; t0 < L; t0 += 256) {
-    const int key = t0 + lane;
-    float s = -INFINITY;
-    if (key < L) {
-      const CT* krow = kcache +
-          (long)bt_lds[key / PBLK] * blk_stride + head_off +
-          (key % PBLK) * D;
-      float dot = 0.f;
+  bf16x8 qf[D / 32];
 #pragma unroll
-      for (int c = 0; c < D / 8; ++c) {
-        float kf[8];
-        if constexpr (sizeof(CT) == 2) {
-          s16x8 kv8 = *reinterpret_cast<const s16x8*>(krow + c * 8);
-          bf8_to_f32(kv8, kf);
-        } else {
-          i32x2 kv8 = *reinterpret_cast<const i32x2*>(krow + c * 8);
-          const unsigned char* b =
-              reinterpret_cast<const unsigned char*>(&kv8);
+  for (int s = 0; s < D / 32; ++s) {
+    pa_frag f;
 #pragma unroll
-          for (int i = 0; i < 8; ++i) kf[i] = fp8_to_f32(b[i]);
-        }
+    for (int i = 0; i < 4; ++i) f.d[i] = 0;
+    if (c16 < nh)
+      f.v = *reinterpret_cast<const bf16x8*>(
+          q + b * q_stride + (long)(head0 + c16) * D + s * 32 + g * 8);
+    qf[s] = f.v;
+  }
+
+  // page numbers of the wave's next 32 tiles, two a tile, on the lanes
+  int pages = 0;
+  auto fetch_pages = [&](int i) {
+    const int p = (t0 + (i + (lane >> 1)) * 4) * 2 + (lane & 1);
+    pages = mine > 0 ? bt[min(p, last_page)] : 0;
+  };
+  auto page = [&](int i, int half) {
+    return __builtin_amdgcn_readlane(pages, (i & 31) * 2 + half);
+  };
+  char* ring = smem + wid * R * 2 * TILE;
+
+  // bf16: pieces of K and V of tile i, pieces of 16 bytes XOR-ed with the
+  // row in K, of 32 bytes in V
+  auto issue = [&](int i) {
+    char* dst = ring + (i % R) * 2 * TILE + lane * 16;
+    const int r = lane / NCH, c = lane % NCH;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) dot += kf[i] * q_lds[c * 8 + i];
-      }
-      s = dot;
+    for (int p = 0; p < PIECES; ++p) {
+      const int row = p * ROWS + r;
+      const long at = page(i, p * ROWS / PBLK) * page_bytes + head_bytes +
+                      (row % PBLK) * (D * 2);
+      auto go = [&](const char* src, char* to) {
+        __builtin_amdgcn_global_load_lds(
+            (const __attribute__((address_space(1))) unsigned int*)src,
+            (__attribute__((address_space(3))) unsigned int*)to, 16, 0, 0);
+      };
+      go(kcache + at + ((c ^ (row & (NCH - 1))) * 16), dst + p * 1024);
+      go(vcache + at + ((c ^ ((row & 3) << 1)) * 16),
+         dst + TILE + p * 1024);
     }
-    const float pmax = wave_reduce_max(s);
-    const float mn = fmaxf(fmaxf(m, pmax), -1e30f);
-    const float alpha = exp2f((m - mn) * 1.4426950408889634f);
-    const float p = (key < L)
-        ? exp2f((s - mn) * 1.4426950408889634f) : 0.f;
-    l = l * alpha + wave_reduce_sum(p);
-    m = mn;
-    p_lds[wid * 64 + lane] = p;
+  };
+  // fp8: the same rows through registers, 16 numbers a load
+  constexpr int LOADS = FP8 ? KT * D / 1024 : 1;
+  i32x4 kreg[LOADS], vreg[LOADS];
+  auto issue8 = [&](int i) {
 #pragma unroll
-    for (int i = 0; i < DPL; ++i) acc[i] *= alpha;
-    // branch-free 8-deep PV: independent loads pipeline over L2 latency
-    const int kmax = min(64, L - t0);
-    int kk = 0;
-    for (; kk + 8 <= kmax; kk += 8) {
-      float pv[8];
-      float vv[8][DPL];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int key2 = t0 + kk + j;
-        pv[j] = p_lds[wid * 64 + kk + j];
-        const CT* vrow = vcache +
-            (long)bt_lds[key2 / PBLK] * blk_stride + head_off +
-            (key2 % PBLK) * D + lane * DPL;
-#pragma unroll
-        for (int i = 0; i < DPL; ++i)
-          vv[j][i] = (sizeof(CT) == 2)
-              ? bf2f((unsigned short)vrow[i])
-              : fp8_to_f32((unsigned char)vrow[i]);
-      }
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-#pragma unroll
-        for (int i = 0; i < DPL; ++i) acc[i] += pv[j] * vv[j][i];
+    for (int j = 0; j < LOADS; ++j) {
+      const int at = (j * 64 + lane) * 16, row = at / D, col = at % D;
+      const int pg = row < PBLK ? page(i, 0) : page(i, 1);
+      const long off = pg * page_bytes + head_bytes + (row % PBLK) * D + col;
+      kreg[j] = *reinterpret_cast<const i32x4*>(kcache + off);
+      vreg[j] = *reinterpret_cast<const i32x4*>(vcache + off);
     }
-    for (; kk < kmax; ++kk) {
-      const int key2 = t0 + kk;
-      const float pv = p_lds[wid * 64 + kk];
-      const CT* vrow = vcache +
-          (long)bt_lds[key2 / PBLK] * blk_stride + head_off +
-          (key2 % PBLK) * D + lane * DPL;
+  };
+  auto store8 = [&]() {
 #pragma unroll
-      for (int i = 0; i < DPL; ++i)
-        acc[i] += pv * ((sizeof(CT) == 2)
-                        ? bf2f((unsigned short)vrow[i])
-                        : fp8_to_f32((unsigned char)vrow[i]));
+    for (int j = 0; j < LOADS; ++j) {
+      const int at = (j * 64 + lane) * 16, row = at / D, c = at % D / 8;
+      i32x4 w[2];
+      pa_widen(kreg[j], w);
+#pragma unroll
+      for (int e = 0; e < 2; ++e)
+        *reinterpret_cast<i32x4*>(
+            ring + row * (2 * D) + ((c + e) ^ (row & (NCH - 1))) * 16) = w[e];
+      pa_widen(vreg[j], w);
+#pragma unroll
+      for (int e = 0; e < 2; ++e)
+        *reinterpret_cast<i32x4*>(
+            ring + TILE + row * (2 * D) + ((c + e) ^ ((row & 3) << 1)) * 16) =
+            w[e];
+    }
+  };
+
+  const float scale2 = scale * 1.4426950408889634f;
+  float m = -1e30f, l = 0.f;  // l: of the keys of this lane group
+  f32x4 acc[DB];
+#pragma unroll
+  for (int d = 0; d < DB; ++d) acc[d] = {0.f, 0.f, 0.f, 0.f};
+
+  auto compute = [&](int i) {
+    char* kt = ring + (i % R) * 2 * TILE;
+    char* vt = kt + TILE;
+    const int left = L - (t0 + i * 4) * KT;  // keys of the tile, if < 32
+    if (left < KT) {
+      // what lies behind the last key must not meet its zero probability
+      for (int k = left * (2 * D) + lane * 16; k < TILE; k += 1024)
+        *reinterpret_cast<i32x4*>(vt + k) = i32x4{0, 0, 0, 0};
+    }
+    f32x4 sc[2];
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) {
+      sc[kb] = {0.f, 0.f, 0.f, 0.f};
+      const int key = kb * 16 + c16;
+#pragma unroll
+      for (int s = 0; s < D / 32; ++s) {
+        const bf16x8 kf = *reinterpret_cast<const bf16x8*>(
+            kt + key * (2 * D) + (((s * 4 + g) ^ (key & (NCH - 1))) * 16));
+        sc[kb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[s], sc[kb], 0,
+                                                         0, 0);
+      }
+    }
+    float top = -INFINITY;
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float s =
+            kb * 16 + g * 4 + r < left ? sc[kb][r] * scale2 : -INFINITY;
+        sc[kb][r] = s;
+        top = fmaxf(top, s);
+      }
+    top = fmaxf(top, __shfl_xor(top, 16, 64));
+    top = fmaxf(top, __shfl_xor(top, 32, 64));
+    if (!__all(top <= m)) {
+      const float mn = fmaxf(m, top);
+      const float alpha = __builtin_amdgcn_exp2f(m - mn);
+      m = mn;
+      l *= alpha;
+#pragma unroll
+      for (int d = 0; d < DB; ++d)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[d][r] *= alpha;
+    }
+    pa_frag hi, lo;
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int r = 0; r < 4; r += 2) {
+        const float p0 = __builtin_amdgcn_exp2f(sc[kb][r] - m);
+        const float p1 = __builtin_amdgcn_exp2f(sc[kb][r + 1] - m);
+        l += p0 + p1;
+        const unsigned int h = pa_pack(p0, p1);
+        hi.d[kb * 2 + r / 2] = h;
+        lo.d[kb * 2 + r / 2] =
+            pa_pack(p0 - __builtin_bit_cast(float, h << 16),
+                    p1 - __builtin_bit_cast(float, h & 0xffff0000u));
+      }
+    // columns 16 d .. of V, keys 4 g .. 4 g + 3 of both halves: the order in
+    // which a lane holds its probabilities
+    const int row = g * 4 + (c16 >> 2);
+#pragma unroll
+    for (int d = 0; d < DB; ++d) {
+      pa_frag vf;
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+        vf.h[kb] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (__attribute__((address_space(3))) s16x4*)(
+                vt + (kb * 16 + row) * (2 * D) +
+                ((d ^ (row & 3)) * 32) + (c16 & 3) * 8));
+      acc[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf.v, hi.v, acc[d], 0,
+                                                       0, 0);
+      acc[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf.v, lo.v, acc[d], 0,
+                                                       0, 0);
+    }
+    // the buffer is read before the wave fills it again
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  };
+
+  if constexpr (FP8) {
+    if (mine > 0) {
+      fetch_pages(0);
+      issue8(0);
+    }
+    for (int i = 0; i < mine; ++i) {
+      store8();
+      if (i + 1 < mine) {
+        if (((i + 1) & 31) == 0) fetch_pages(i + 1);
+        issue8(i + 1);
+      }
+      wave_sync();
+      compute(i);
+    }
+  } else {
+    int at = 0;  // tiles issued
+    auto next = [&]() {
+      if ((at & 31) == 0) fetch_pages(at);
+      issue(at++);
+    };
+    while (at < R - 1 && at < mine) next();
+    for (int i = 0; i < mine; ++i) {
+      if (at < mine) {
+        next();
+        asm volatile("s_waitcnt vmcnt(%0)" ::"i"((R - 1) * 2 * PIECES)
+                     : "memory");
+      } else {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      }
+      compute(i);
     }
   }
 
-  if (lane == 0) {
-    wstate[wid * 2] = m;
-    wstate[wid * 2 + 1] = l;
+  // ---- the waves' states meet ---------------------------------------------
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  __syncthreads();
+  float* ml = reinterpret_cast<float*>(smem);  // [4][16][2]
+  float* wacc = ml + 4 * 16 * 2;               // [4][16][D]
+  if (g == 0) {
+    ml[(wid * 16 + c16) * 2] = m;
+    ml[(wid * 16 + c16) * 2 + 1] = l;
   }
 #pragma unroll
-  for (int i = 0; i < DPL; ++i) wacc[wid * D + lane * DPL + i] = acc[i];
+  for (int d = 0; d < DB; ++d)
+    *reinterpret_cast<f32x4*>(wacc + (wid * 16 + c16) * D + d * 16 + g * 4) =
+        acc[d];
   __syncthreads();
-
-  if (wid == 0) {
+  const long part = ((long)(b * HKV + kvh) * NS + split) * GR + hg * 16;
+  for (int i = threadIdx.x; i < nh * (D / 4); i += 256) {
+    const int head = i / (D / 4), col = i % (D / 4) * 4;
     float M = -1e30f;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) M = fmaxf(M, wstate[w * 2]);
-    float Ltot = 0.f;
-    float o[2] = {0.f, 0.f};
+    for (int w = 0; w < 4; ++w) M = fmaxf(M, ml[(w * 16 + head) * 2]);
+    float sum = 0.f;
+    f32x4 o = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
-      const float a = exp2f((wstate[w * 2] - M) * 1.4426950408889634f);
-      Ltot += wstate[w * 2 + 1] * a;
+      const float a = __builtin_amdgcn_exp2f(ml[(w * 16 + head) * 2] - M);
+      sum += ml[(w * 16 + head) * 2 + 1] * a;
+      const f32x4 v =
+          *reinterpret_cast<const f32x4*>(wacc + (w * 16 + head) * D + col);
 #pragma unroll
-      for (int i = 0; i < DPL; ++i) o[i] += a * wacc[w * D + lane * DPL + i];
+      for (int r = 0; r < 4; ++r) o[r] += a * v[r];
     }
-    const float inv = (Ltot > 0.f) ? 1.f / Ltot : 0.f;
-#pragma unroll
-    for (int i = 0; i < DPL; ++i)
-      out[((long)b * H + h) * D + lane * DPL + i] = f2bf(o[i] * inv);
-  }
-}
-
-// GQA-grouped variant: ONE workgroup per (b, kv-head) computes all
-// GR = H/HKV query heads that share that KV head, so each K/V row is
-// read ONCE instead of GR times. At llama3-8b shapes (GR=4) this cuts
-// decode-attention HBM traffic 4x; at bs128 ctx2048 the step is
-// KV-bandwidth-bound, so it shows up ~1:1 end-to-end.
-template <int D, int GR, typename CT>
-__global__ void __launch_bounds__(256)
-paged_attn_gqa_kernel(const unsigned short* __restrict__ q,
-                      const CT* __restrict__ kcache,
-                      const CT* __restrict__ vcache,
-                      const int* __restrict__ block_table,
-                      const int* __restrict__ ctx_len,
-                      unsigned short* __restrict__ out, int B, int H,
-                      int HKV, int max_blocks, float scale) {
-  const int b = blockIdx.x / HKV;
-  const int kvh = blockIdx.x % HKV;
-  const int lane = threadIdx.x & 63;
-  const int wid = threadIdx.x >> 6;
-  const int L = ctx_len[b];
-
-  extern __shared__ __attribute__((aligned(16))) char smem[];
-  float* p_lds = reinterpret_cast<float*>(smem);        // 4*GR*64
-  float* q_lds = p_lds + 4 * GR * 64;                   // GR*D
-  float* wstate = q_lds + GR * D;                       // 4*GR*2
-  float* wacc = wstate + 8 * GR;                        // 4*GR*D
-  int* bt_lds = reinterpret_cast<int*>(wacc + 4 * GR * D);
-
-  const int nblk = (L + PBLK - 1) / PBLK;
-  for (int i = threadIdx.x; i < nblk; i += 256)
-    bt_lds[i] = block_table[(long)b * max_blocks + i];
-  for (int i = threadIdx.x; i < GR * D; i += 256) {
-    const int g = i / D, d = i % D;
-    q_lds[i] = bf2f(q[((long)b * H + kvh * GR + g) * D + d]) * scale;
-  }
-  __syncthreads();
-
-  constexpr int DPL = D / 64;
-  float m[GR], l[GR], acc[GR][DPL];
-#pragma unroll
-  for (int g = 0; g < GR; ++g) {
-    m[g] = -1e30f;
-    l[g] = 0.f;
-#pragma unroll
-    for (int i = 0; i < DPL; ++i) acc[g][i] = 0.f;
-  }
-  const long blk_stride = (long)HKV * PBLK * D;
-  const long head_off = (long)kvh * PBLK * D;
-
-  for (int t0 = wid * 64; t0 < L; t0 += 256) {
-    const int key = t0 + lane;
-    float dot[GR];
-#pragma unroll
-    for (int g = 0; g < GR; ++g) dot[g] = 0.f;
-    if (key < L) {
-      const CT* krow = kcache +
-          (long)bt_lds[key / PBLK] * blk_stride + head_off +
-          (key % PBLK) * D;
-#pragma unroll
-      for (int c = 0; c < D / 8; ++c) {
-        float kf[8];
-        if constexpr (sizeof(CT) == 2) {
-          s16x8 kv8 = *reinterpret_cast<const s16x8*>(krow + c * 8);
-          bf8_to_f32(kv8, kf);
-        } else {
-          i32x2 kv8 = *reinterpret_cast<const i32x2*>(krow + c * 8);
-          const unsigned char* bb =
-              reinterpret_cast<const unsigned char*>(&kv8);
-#pragma unroll
-          for (int i = 0; i < 8; ++i) kf[i] = fp8_to_f32(bb[i]);
-        }
-#pragma unroll
-        for (int g = 0; g < GR; ++g)
-#pragma unroll
-          for (int i = 0; i < 8; ++i)
-            dot[g] += kf[i] * q_lds[g * D + c * 8 + i];
-      }
-    }
-#pragma unroll
-    for (int g = 0; g < GR; ++g) {
-      const float s = (key < L) ? dot[g] : -INFINITY;
-      const float pmax = wave_reduce_max(s);
-      const float mn = fmaxf(fmaxf(m[g], pmax), -1e30f);
-      const float alpha = exp2f((m[g] - mn) * 1.4426950408889634f);
-      const float p = (key < L)
-          ? exp2f((s - mn) * 1.4426950408889634f) : 0.f;
-      l[g] = l[g] * alpha + wave_reduce_sum(p);
-      m[g] = mn;
-      p_lds[(wid * GR + g) * 64 + lane] = p;
-#pragma unroll
-      for (int i = 0; i < DPL; ++i) acc[g][i] *= alpha;
-    }
-    const int kmax = min(64, L - t0);
-    int kk = 0;
-    for (; kk + 4 <= kmax; kk += 4) {
-      float vv[4][DPL];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int key2 = t0 + kk + j;
-        const CT* vrow = vcache +
-            (long)bt_lds[key2 / PBLK] * blk_stride + head_off +
-            (key2 % PBLK) * D + lane * DPL;
-#pragma unroll
-        for (int i = 0; i < DPL; ++i)
-          vv[j][i] = (sizeof(CT) == 2)
-              ? bf2f((unsigned short)vrow[i])
-              : fp8_to_f32((unsigned char)vrow[i]);
-      }
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int g = 0; g < GR; ++g) {
-          const float pv = p_lds[(wid * GR + g) * 64 + kk + j];
-#pragma unroll
-          for (int i = 0; i < DPL; ++i) acc[g][i] += pv * vv[j][i];
-        }
-    }
-    for (; kk < kmax; ++kk) {
-      const int key2 = t0 + kk;
-      const CT* vrow = vcache +
-          (long)bt_lds[key2 / PBLK] * blk_stride + head_off +
-          (key2 % PBLK) * D + lane * DPL;
-      float vv[DPL];
-#pragma unroll
-      for (int i = 0; i < DPL; ++i)
-        vv[i] = (sizeof(CT) == 2)
-            ? bf2f((unsigned short)vrow[i])
-            : fp8_to_f32((unsigned char)vrow[i]);
-#pragma unroll
-      for (int g = 0; g < GR; ++g) {
-        const float pv = p_lds[(wid * GR + g) * 64 + kk];
-#pragma unroll
-        for (int i = 0; i < DPL; ++i) acc[g][i] += pv * vv[i];
-      }
-    }
-  }
-
-#pragma unroll
-  for (int g = 0; g < GR; ++g) {
-    if (lane == 0) {
-      wstate[(wid * GR + g) * 2] = m[g];
-      wstate[(wid * GR + g) * 2 + 1] = l[g];
-    }
-#pragma unroll
-    for (int i = 0; i < DPL; ++i)
-      wacc[(wid * GR + g) * D + lane * DPL + i] = acc[g][i];
-  }
-  __syncthreads();
-
-  if (wid == 0) {
-#pragma unroll
-    for (int g = 0; g < GR; ++g) {
-      float M = -1e30f;
-#pragma unroll
-      for (int w = 0; w < 4; ++w)
-        M = fmaxf(M, wstate[(w * GR + g) * 2]);
-      float Ltot = 0.f;
-      float o[DPL];
-#pragma unroll
-      for (int i = 0; i < DPL; ++i) o[i] = 0.f;
-#pragma unroll
-      for (int w = 0; w < 4; ++w) {
-        const float a =
-            exp2f((wstate[(w * GR + g) * 2] - M) * 1.4426950408889634f);
-        Ltot += wstate[(w * GR + g) * 2 + 1] * a;
-#pragma unroll
-        for (int i = 0; i < DPL; ++i)
-          o[i] += a * wacc[(w * GR + g) * D + lane * DPL + i];
-      }
-      const float inv = (Ltot > 0.f) ? 1.f / Ltot : 0.f;
-#pragma unroll
-      for (int i = 0; i < DPL; ++i)
-        out[((long)b * H + kvh * GR + g) * D + lane * DPL + i] =
-            f2bf(o[i] * inv);
-    }
-  }
-}
-
-// Context-split ("flash-decoding") variant for SMALL batches: B*HKV
-// workgroups underfill 256 CUs (B=1, HKV=8 -> 8 WGs = 3% of the chip),
-// so split each sequence's context into NS chunks, compute partial
-// (m, l, acc) per chunk in parallel, and combine in a second kernel.
-// Scratch: pacc [B*HKV*NS, GR, D] f32 ; pml [B*HKV*NS, GR, 2] f32.
-template <int D, int GR, typename CT>
-__global__ void __launch_bounds__(256)
-paged_attn_split_kernel(const unsigned short* __restrict__ q,
-                        const CT* __restrict__ kcache,
-                        const CT* __restrict__ vcache,
-                        const int* __restrict__ block_table,
-                        const int* __restrict__ ctx_len,
-                        float* __restrict__ pacc, float* __restrict__ pml,
-                        int B, int H, int HKV, int max_blocks, int NS,
-                        float scale) {
-  const int split = blockIdx.x % NS;
-  const int bg = blockIdx.x / NS;         // (b * HKV + kvh)
-  const int b = bg / HKV;
-  const int kvh = bg % HKV;
-  const int lane = threadIdx.x & 63;
-  const int wid = threadIdx.x >> 6;
-  const int L = ctx_len[b];
-  const int chunk = ((L + NS * PBLK - 1) / (NS * PBLK)) * PBLK;
-  const int s0 = split * chunk;
-  const int s1 = min(L, s0 + chunk);
-
-  extern __shared__ __attribute__((aligned(16))) char smem[];
-  float* p_lds = reinterpret_cast<float*>(smem);        // 4*GR*64
-  float* q_lds = p_lds + 4 * GR * 64;                   // GR*D
-  float* wstate = q_lds + GR * D;                       // 4*GR*2
-  float* wacc = wstate + 8 * GR;                        // 4*GR*D
-  int* bt_lds = reinterpret_cast<int*>(wacc + 4 * GR * D);
-
-  const int nblk = (L + PBLK - 1) / PBLK;
-  for (int i = threadIdx.x; i < nblk; i += 256)
-    bt_lds[i] = block_table[(long)b * max_blocks + i];
-  for (int i = threadIdx.x; i < GR * D; i += 256) {
-    const int g = i / D, d = i % D;
-    q_lds[i] = bf2f(q[((long)b * H + kvh * GR + g) * D + d]) * scale;
-  }
-  __syncthreads();
-
-  constexpr int DPL = D / 64;
-  float m[GR], l[GR], acc[GR][DPL];
-#pragma unroll
-  for (int g = 0; g < GR; ++g) {
-    m[g] = -1e30f;
-    l[g] = 0.f;
-#pragma unroll
-    for (int i = 0; i < DPL; ++i) acc[g][i] = 0.f;
-  }
-  const long blk_stride = (long)HKV * PBLK * D;
-  const long head_off = (long)kvh * PBLK * D;
-
-  for (int t0 = s0 + wid * 64; t0 < s1; t0 += 256) {
-    const int key = t0 + lane;
-    float dot[GR];
-#pragma unroll
-    for (int g = 0; g < GR; ++g) dot[g] = 0.f;
-    if (key < s1) {
-      const CT* krow = kcache +
-          (long)bt_lds[key / PBLK] * blk_stride + head_off +
-          (key % PBLK) * D;
-#pragma unroll
-      for (int c = 0; c < D / 8; ++c) {
-        float kf[8];
-        if constexpr (sizeof(CT) == 2) {
-          s16x8 kv8 = *reinterpret_cast<const s16x8*>(krow + c * 8);
-          bf8_to_f32(kv8, kf);
-        } else {
-          i32x2 kv8 = *reinterpret_cast<const i32x2*>(krow + c * 8);
-          const unsigned char* bb =
-              reinterpret_cast<const unsigned char*>(&kv8);
-#pragma unroll
-          for (int i = 0; i < 8; ++i) kf[i] = fp8_to_f32(bb[i]);
-        }
-#pragma unroll
-        for (int g = 0; g < GR; ++g)
-#pragma unroll
-          for (int i = 0; i < 8; ++i)
-            dot[g] += kf[i] * q_lds[g * D + c * 8 + i];
-      }
-    }
-#pragma unroll
-    for (int g = 0; g < GR; ++g) {
-      const float s = (key < s1) ? dot[g] : -INFINITY;
-      const float pmax = wave_reduce_max(s);
-      const float mn = fmaxf(fmaxf(m[g], pmax), -1e30f);
-      const float alpha = exp2f((m[g] - mn) * 1.4426950408889634f);
-      const float p = (key < s1)
-          ? exp2f((s - mn) * 1.4426950408889634f) : 0.f;
-      l[g] = l[g] * alpha + wave_reduce_sum(p);
-      m[g] = mn;
-      p_lds[(wid * GR + g) * 64 + lane] = p;
-#pragma unroll
-      for (int i = 0; i < DPL; ++i) acc[g][i] *= alpha;
-    }
-    const int kmax = min(64, s1 - t0);
-    for (int kk = 0; kk < kmax; ++kk) {
-      const int key2 = t0 + kk;
-      const CT* vrow = vcache +
-          (long)bt_lds[key2 / PBLK] * blk_stride + head_off +
-          (key2 % PBLK) * D + lane * DPL;
-      float vv[DPL];
-#pragma unroll
-      for (int i = 0; i < DPL; ++i)
-        vv[i] = (sizeof(CT) == 2)
-            ? bf2f((unsigned short)vrow[i])
-            : fp8_to_f32((unsigned char)vrow[i]);
-#pragma unroll
-      for (int g = 0; g < GR; ++g) {
-        const float pv = p_lds[(wid * GR + g) * 64 + kk];
-#pragma unroll
-        for (int i = 0; i < DPL; ++i) acc[g][i] += pv * vv[i];
-      }
-    }
-  }
-
-#pragma unroll
-  for (int g = 0; g < GR; ++g) {
-    if (lane == 0) {
-      wstate[(wid * GR + g) * 2] = m[g];
-      wstate[(wid * GR + g) * 2 + 1] = l[g];
-    }
-#pragma unroll
-    for (int i = 0; i < DPL; ++i)
-      wacc[(wid * GR + g) * D + lane * DPL + i] = acc[g][i];
-  }
-  __syncthreads();
-
-  if (wid == 0) {
-    const long po = ((long)bg * NS + split) * GR;
-#pragma unroll
-    for (int g = 0; g < GR; ++g) {
-      float M = -1e30f;
-#pragma unroll
-      for (int w = 0; w < 4; ++w)
-        M = fmaxf(M, wstate[(w * GR + g) * 2]);
-      float Ltot = 0.f;
-      float o[DPL];
-#pragma unroll
-      for (int i = 0; i < DPL; ++i) o[i] = 0.f;
-#pragma unroll
-      for (int w = 0; w < 4; ++w) {
-        const float a =
-            exp2f((wstate[(w * GR + g) * 2] - M) * 1.4426950408889634f);
-        Ltot += wstate[(w * GR + g) * 2 + 1] * a;
-#pragma unroll
-        for (int i = 0; i < DPL; ++i)
-          o[i] += a * wacc[(w * GR + g) * D + lane * DPL + i];
-      }
-#pragma unroll
-      for (int i = 0; i < DPL; ++i)
-        pacc[(po + g) * D + lane * DPL + i] = o[i];
-      if (lane == 0) {
-        pml[(po + g) * 2] = M;
-        pml[(po + g) * 2 + 1] = Ltot;
+    if (NS == 1) {
+      const float inv = sum > 0.f ? 1.f / sum : 0.f;
+      const i32x2 two = {(int)pa_pack(o[0] * inv, o[1] * inv),
+                         (int)pa_pack(o[2] * inv, o[3] * inv)};
+      *reinterpret_cast<i32x2*>(out + ((long)b * H + head0 + head) * D + col) =
+          two;
+    } else {
+      *reinterpret_cast<f32x4*>(pacc + (part + head) * D + col) = o;
+      if (col == 0) {
+        pml[(part + head) * 2] = M;
+        pml[(part + head) * 2 + 1] = sum;
       }
     }
   }
 }
 
-// Combine NS partials -> normalized bf16 out. Grid: B*HKV, 256 thr.
-template <int D, int GR>
+// Join NS partial results; a wave per (sequence, head), the shares' states on
+// its lanes. NS <= 64.
+template <int D>
 __global__ void __launch_bounds__(256)
 paged_attn_combine_kernel(const float* __restrict__ pacc,
                           const float* __restrict__ pml,
-                          unsigned short* __restrict__ out, int B, int H,
+                          unsigned short* __restrict__ out, int rows, int H,
                           int HKV, int NS) {
-  const int bg = blockIdx.x;
-  const int b = bg / HKV;
-  const int kvh = bg % HKV;
   constexpr int DPL = D / 64;
   const int lane = threadIdx.x & 63;
-  const int wid = threadIdx.x >> 6;
-  // wave w handles head group g = wid (GR <= 4 per wave pass)
-  for (int g = wid; g < GR; g += 4) {
-    const long po = ((long)bg * NS) * GR;
-    float M = -1e30f;
-    for (int s = 0; s < NS; ++s)
-      M = fmaxf(M, pml[(po + (long)s * GR + g) * 2]);
-    float Ltot = 0.f;
-    float o[DPL];
+  const int row = blockIdx.x * 4 + (threadIdx.x >> 6);  // b * H + head
+  if (row >= rows) return;
+  const int GR = H / HKV, b = row / H, h = row % H;
+  const long part = (long)(b * HKV + h / GR) * NS * GR + h % GR;
+  float m = -1e30f, l = 0.f;
+  if (lane < NS) {
+    m = pml[(part + (long)lane * GR) * 2];
+    l = pml[(part + (long)lane * GR) * 2 + 1];
+  }
+  const float M = wave_reduce_max(m);
+  const float a = lane < NS ? __builtin_amdgcn_exp2f(m - M) : 0.f;
+  const float sum = wave_reduce_sum(l * a);
+  float o[DPL];
 #pragma unroll
-    for (int i = 0; i < DPL; ++i) o[i] = 0.f;
-    for (int s = 0; s < NS; ++s) {
-      const long pi = po + (long)s * GR + g;
-      const float a = exp2f((pml[pi * 2] - M) * 1.4426950408889634f);
-      Ltot += pml[pi * 2 + 1] * a;
-#pragma unroll
-      for (int i = 0; i < DPL; ++i)
-        o[i] += a * pacc[pi * D + lane * DPL + i];
-    }
-    const float inv = (Ltot > 0.f) ? 1.f / Ltot : 0.f;
+  for (int i = 0; i < DPL; ++i) o[i] = 0.f;
+#pragma unroll 8
+  for (int s = 0; s < NS; ++s) {
+    const float w = __builtin_bit_cast(
+        float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, a), s));
 #pragma unroll
     for (int i = 0; i < DPL; ++i)
-      out[((long)b * H + kvh * GR + g) * D + lane * DPL + i] =
-          f2bf(o[i] * inv);
+      o[i] += w * pacc[(part + (long)s * GR) * D + lane * DPL + i];
   }
+  const float inv = sum > 0.f ? 1.f / sum : 0.f;
+#pragma unroll
+  for (int i = 0; i < DPL; ++i)
+    out[(long)row * D + lane * DPL + i] = f2bf(o[i] * inv);
 }
 
-extern "C" void launch_paged_attn_split(
-    const void* q, const void* kcache, const void* vcache,
-    const int* block_table, const int* ctx_len, void* pacc, void* pml,
-    void* out, int B, int H, int HKV, int D, int max_blocks, int NS,
-    float scale, bool fp8, hipStream_t stream) {
-  const int GR = H / HKV;
-#define PS(DD, GG, CT)                                                         \
-  do {                                                                         \
-    const int lds_g =                                                          \
-        (4 * GG * 64 + GG * DD + 8 * GG + 4 * GG * DD) * 4 + max_blocks * 4;   \
-    hipLaunchKernelGGL((paged_attn_split_kernel<DD, GG, CT>),                  \
-                       dim3(B * HKV * NS), dim3(256), lds_g, stream,           \
-                       (const unsigned short*)q, (const CT*)kcache,            \
-                       (const CT*)vcache, block_table, ctx_len,                \
-                       (float*)pacc, (float*)pml, B, H, HKV, max_blocks, NS,   \
-                       scale);                                                 \
-    hipLaunchKernelGGL((paged_attn_combine_kernel<DD, GG>),                    \
-                       dim3(B * HKV), dim3(256), 0, stream,                    \
-                       (const float*)pacc, (const float*)pml,                  \
-                       (unsigned short*)out, B, H, HKV, NS);                   \
-  } while (0)
-#define PS_D(DD, CT)                                                           \
-  do {                                                                         \
-    if (GR == 1) PS(DD, 1, CT);                                                \
-    else if (GR == 2) PS(DD, 2, CT);                                           \
-    else if (GR == 4) PS(DD, 4, CT);                                           \
-    else PS(DD, 8, CT);                                                        \
-  } while (0)
+extern "C" void launch_paged_attn(const void* q, long q_stride,
+                                  const void* kcache, const void* vcache,
+                                  const int* block_table, const int* ctx_len,
+                                  void* out, void* pacc, void* pml, int B,
+                                  int H, int HKV, int D, int max_blocks,
+                                  int NS, float scale, bool fp8,
+                                  hipStream_t stream) {
+  const int GR = H / HKV, NG = (GR + 15) / 16;
+  const int grid = B * HKV * NG * NS;
+#define PA(DD, F8)                                                            \
+  hipLaunchKernelGGL((paged_attn_kernel<DD, F8>), dim3(grid), dim3(256),      \
+                     pa_lds(DD, F8) > 4 * 16 * (DD + 2) * 4                   \
+                         ? pa_lds(DD, F8)                                     \
+                         : 4 * 16 * (DD + 2) * 4,                             \
+                     stream, (const unsigned short*)q, q_stride,              \
+                     (const char*)kcache, (const char*)vcache, block_table,   \
+                     ctx_len, (unsigned short*)out, (float*)pacc,             \
+                     (float*)pml, H, HKV, max_blocks, NS, scale)
   if (D == 64) {
-    if (fp8) PS_D(64, unsigned char); else PS_D(64, unsigned short);
-  } else if (D == 128) {
-    if (fp8) PS_D(128, unsigned char); else PS_D(128, unsigned short);
-  }
-#undef PS_D
-#undef PS
-}
-
-extern "C" void launch_paged_attn(const void* q, const void* kcache,
-                                  const void* vcache, const int* block_table,
-                                  const int* ctx_len, void* out, int B, int H,
-                                  int HKV, int D, int max_blocks, float scale,
-                                  bool fp8, hipStream_t stream) {
-  const int GR = (HKV > 0 && H % HKV == 0) ? H / HKV : 1;
-  if (GR == 2 || GR == 4 || GR == 8) {
-    // grouped launch: each workgroup serves one (b, kv-head), K/V read
-    // once for all GR query heads
-    dim3 grid(B * HKV);
-#define PG(DD, GG, CT)                                                         \
-  do {                                                                         \
-    const int lds_g =                                                          \
-        (4 * GG * 64 + GG * DD + 8 * GG + 4 * GG * DD) * 4 + max_blocks * 4;   \
-    hipLaunchKernelGGL((paged_attn_gqa_kernel<DD, GG, CT>), grid, dim3(256),   \
-                       lds_g, stream, (const unsigned short*)q,                \
-                       (const CT*)kcache, (const CT*)vcache, block_table,      \
-                       ctx_len, (unsigned short*)out, B, H, HKV, max_blocks,   \
-                       scale);                                                 \
-  } while (0)
-#define PG_D(DD, CT)                                                           \
-  do {                                                                         \
-    if (GR == 2) PG(DD, 2, CT);                                                \
-    else if (GR == 4) PG(DD, 4, CT);                                           \
-    else PG(DD, 8, CT);                                                        \
-  } while (0)
-    if (D == 64) {
-      if (fp8) PG_D(64, unsigned char); else PG_D(64, unsigned short);
-    } else if (D == 128) {
-      if (fp8) PG_D(128, unsigned char); else PG_D(128, unsigned short);
-    }
-#undef PG_D
-#undef PG
-    return;
-  }
-  const int lds = (4 * 64 + D + 8 + 4 * D) * 4 + max_blocks * 4;
-  dim3 grid(B * H);
-#define PA(DD, CT)                                                             \
-  hipLaunchKernelGGL((paged_attn_kernel<DD, CT>), grid, dim3(256), lds,        \
-                     stream, (const unsigned short*)q, (const CT*)kcache,      \
-                     (const CT*)vcache, block_table, ctx_len,                  \
-                     (unsigned short*)out, B, H, HKV, max_blocks, scale)
-  if (D == 64) {
-    if (fp8) PA(64, unsigned char); else PA(64, unsigned short);
-  } else if (D == 128) {
-    if (fp8) PA(128, unsigned char); else PA(128, unsigned short);
+    if (fp8) PA(64, true); else PA(64, false);
+  } else {
+    if (fp8) PA(128, true); else PA(128, false);
   }
 #undef PA
+  if (NS > 1) {
+    const int rows = B * H;
+#define PC(DD)                                                                \
+  hipLaunchKernelGGL(paged_attn_combine_kernel<DD>, dim3((rows + 3) / 4),     \
+                     dim3(256), 0, stream, (const float*)pacc,                \
+                     (const float*)pml, (unsigned short*)out, rows, H, HKV,   \
+                     NS)
+    if (D == 64) PC(64);
+    else PC(128);
+#undef PC
+  }
+}
+
+// Cache element of a bf16 number.
+__device__ __forceinline__ void cache_store(unsigned short* p,
+                                            unsigned short v) {
+  *p = v;
+}
+__device__ __forceinline__ void cache_store(unsigned char* p,
+                                            unsigned short v) {
+  *p = __hip_fp8_e4m3(bf2f(v)).__x;
 }
 
 // Write one new token's K/V into the paged cache (decode step).
@@ -651,13 +450,8 @@ cache_put_kernel(const unsigned short* __restrict__ knew,
     const int blk = block_table[(long)b * max_blocks + pos / PBLK];
     const long off =
         (long)blk * blk_stride + ((long)kvh * PBLK + pos % PBLK) * D + d;
-    if constexpr (sizeof(CT) == 2) {
-      kcache[off] = knew[i];
-      vcache[off] = vnew[i];
-    } else {
-      kcache[off] = __hip_fp8_e4m3(bf2f(knew[i])).__x;
-      vcache[off] = __hip_fp8_e4m3(bf2f(vnew[i])).__x;
-    }
+    cache_store(kcache + off, knew[i]);
+    cache_store(vcache + off, vnew[i]);
   }
 }
 
@@ -679,4 +473,76 @@ extern "C" void launch_cache_put(const void* knew, const void* vnew,
     if (fp8) CP(128, unsigned char); else CP(128, unsigned short);
   }
 #undef CP
+}
+
+// A decode step's projections qkv [B, H + 2 HKV, D] on their way: queries and
+// keys are rotated by the position ctx - 1 of the new token (half-split, fp32,
+// tables [positions, D / 2]); queries go to q [B, H, D], keys and values to
+// their place in the cache. One launch for what a rotation, three copies and
+// a cache write took (5 launches of 4 us each, in a graph). A thread has
+// columns c .. c + 3 of either half of a head.
+template <int D, typename CT>
+__global__ void __launch_bounds__(256)
+rope_put_kernel(const unsigned short* __restrict__ qkv,
+                const float* __restrict__ cs, const float* __restrict__ sn,
+                const int* __restrict__ ctx, unsigned short* __restrict__ q,
+                CT* __restrict__ kcache, CT* __restrict__ vcache,
+                const int* __restrict__ block_table, int B, int H, int HKV,
+                int max_blocks) {
+  constexpr int PER = D / 8;  // threads of a head
+  const int heads = H + 2 * HKV;
+  const long i = (long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= (long)B * heads * PER) return;
+  const int c = (int)(i % PER) * 4;
+  const int h = (int)(i / PER % heads), b = (int)(i / PER / heads);
+  const int pos = ctx[b] - 1;
+  const unsigned short* x = qkv + ((long)b * heads + h) * D + c;
+  unsigned short a[4], e[4];
+  *reinterpret_cast<i32x2*>(a) = *reinterpret_cast<const i32x2*>(x);
+  *reinterpret_cast<i32x2*>(e) = *reinterpret_cast<const i32x2*>(x + D / 2);
+  if (h < H + HKV) {
+    const f32x4 co = *reinterpret_cast<const f32x4*>(cs + (long)pos * (D / 2) + c);
+    const f32x4 si = *reinterpret_cast<const f32x4*>(sn + (long)pos * (D / 2) + c);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float x1 = bf2f(a[j]), x2 = bf2f(e[j]);
+      a[j] = f2bf(x1 * co[j] - x2 * si[j]);
+      e[j] = f2bf(x2 * co[j] + x1 * si[j]);
+    }
+  }
+  if (h < H) {
+    unsigned short* o = q + ((long)b * H + h) * D + c;
+    *reinterpret_cast<i32x2*>(o) = *reinterpret_cast<const i32x2*>(a);
+    *reinterpret_cast<i32x2*>(o + D / 2) = *reinterpret_cast<const i32x2*>(e);
+    return;
+  }
+  const int kvh = (h - H) % HKV;
+  CT* o = (h < H + HKV ? kcache : vcache) +
+          (((long)block_table[(long)b * max_blocks + pos / PBLK] * HKV + kvh) *
+               PBLK + pos % PBLK) * D + c;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    cache_store(o + j, a[j]);
+    cache_store(o + D / 2 + j, e[j]);
+  }
+}
+
+extern "C" void launch_rope_put(const void* qkv, const float* cs,
+                                const float* sn, const int* ctx, void* q,
+                                void* kcache, void* vcache,
+                                const int* block_table, int B, int H, int HKV,
+                                int D, int max_blocks, bool fp8,
+                                hipStream_t stream) {
+  const long total = (long)B * (H + 2 * HKV) * (D / 8);
+#define RP(DD, CT)                                                            \
+  hipLaunchKernelGGL((rope_put_kernel<DD, CT>), dim3((total + 255) / 256),    \
+                     dim3(256), 0, stream, (const unsigned short*)qkv, cs,    \
+                     sn, ctx, (unsigned short*)q, (CT*)kcache, (CT*)vcache,   \
+                     block_table, B, H, HKV, max_blocks)
+  if (D == 64) {
+    if (fp8) RP(64, unsigned char); else RP(64, unsigned short);
+  } else {
+    if (fp8) RP(128, unsigned char); else RP(128, unsigned short);
+  }
+#undef RP
 }
