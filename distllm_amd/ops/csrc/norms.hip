@@ -102,10 +102,9 @@ norm_fwd_kernel(const unsigned short* __restrict__ x,
 
 
 // Small-batch variant: ONE 256-thread block per row (4 waves split the
-// chunks, LDS cross-wave combine). At decode B<=8 the wave-per-row
-// kernel is a single wave doing NCL dependent 16-B load rounds
-// (~9.5us/call measured at B=1 H=4096); spreading the row across the
-// block quarters the rounds on the per-token critical path.
+// chunks, LDS cross-wave combine). With few rows the wave-per-row kernel is
+// a few waves doing NCL dependent 16-B load rounds; spreading the row across
+// the block quarters the rounds on the per-token critical path.
 template <int NCL, bool HAS_RES, bool WRITE_SUM, bool RMS>
 __global__ void __launch_bounds__(256)
 norm_fwd_small_kernel(const unsigned short* __restrict__ x,
@@ -194,6 +193,13 @@ norm_fwd_small_kernel(const unsigned short* __restrict__ x,
   }
 }
 
+// Up to how many rows each takes a workgroup. Measured in a graph with
+// residual and sum, us, workgroup and wave per row: 64 rows of 768 2.6 and
+// 3.3, of 4096 3.4 and 6.6, of 8192 4.6 and 11.1; 1024 rows 3.2 and 3.7, 6.0
+// and 8.2, 9.4 and 17.0; 2048 rows 4.2 and 4.3, 9.2 and 11.5, 15.7 and 20.4;
+// 4096 rows 6.4 and 5.5, 16.1 and 20.7, 30.3 and 37.9.
+#define NORM_ROWS_BLOCK 2048
+
 extern "C" void launch_norm_fwd(const void* x, const void* res, const void* w,
                                 const void* b, void* out, void* sum_out,
                                 int n_rows, int H, float eps, bool rms,
@@ -210,7 +216,7 @@ extern "C" void launch_norm_fwd(const void* x, const void* res, const void* w,
   int blocks = min((n_rows + 3) / 4, cap);
   bool has_res = res != nullptr;
   bool write_sum = sum_out != nullptr;
-  const bool small = n_rows <= 8;
+  const bool small = n_rows <= NORM_ROWS_BLOCK;
   int ncl = small ? (H / 8 + 255) / 256 : (H / 8 + WAVE - 1) / WAVE;
 
 #define DISPATCH3(NCL, HR, WS, RM)                                             \

@@ -1,0 +1,26 @@
+"""Residual norms on both sides of the row count where a row gets a wave
+instead of a workgroup, at sizes of one and of many loads a thread."""
+
+import pytest
+import torch
+
+from distllm_amd import ops
+from distllm_amd.ops import torch_ref
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("rms", [False, True])
+@pytest.mark.parametrize("H", [8, 768, 2056, 4096, 8192])
+@pytest.mark.parametrize("rows", [9, 2048, 2049])
+def test_rows(device, rows, H, rms):
+    g = torch.Generator(device=device).manual_seed(rows + H)
+    x, r = (torch.randn(rows, H, device=device, generator=g)
+            .to(torch.bfloat16) for _ in range(2))
+    w, b = (torch.randn(H, device=device, generator=g).to(torch.bfloat16)
+            for _ in range(2))
+    b = None if rms else b
+    got = ops.norm_fwd_sum(x, r, w, b, eps=1e-5, rms=rms)
+    want = torch_ref.norm_fwd(x, r, w, b, 1e-5, rms, return_sum=True)
+    for a, e in zip(got, want):  # a bf16 step of results of a few units
+        torch.testing.assert_close(a.float(), e.float(), atol=1e-2, rtol=8e-3)
