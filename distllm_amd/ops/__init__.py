@@ -464,20 +464,23 @@ rope_tables = torch_ref.rope_tables
 def topk(scores, k, chunk=1 << 15):
     """Row-wise top-k over a [Q, N] f32 score matrix.
 
-    GPU: chunked radix-select kernel + candidate-merge round. The
-    32k default chunk keeps the grid >= 1024 workgroups even for a few
-    queries (the chip needs >> 256 workgroups to fill).
+    GPU: chunks of scores by workgroups, then rounds over the candidates.
+    Up to k = 256 a workgroup holds its chunk of 8192 in registers; beyond, a
+    radix select reads chunks of `chunk` (the 32k default keeps the grid >=
+    1024 workgroups even for a few queries).
     Returns (values [Q,k] f32 desc-sorted, indices [Q,k] int32).
     """
     if scores.is_cuda:
         _require_hip()
         Q, N = scores.shape
         k_eff = min(k, N)
+        few = 0 < k_eff <= 256
+        if few:
+            chunk = min(chunk, 8192)
         v, i = _hip_ops.topk_chunked(scores.contiguous(), None, k_eff, chunk)
-        if v.shape[1] > k_eff:  # merge candidates from multiple chunks
-            v2, i2 = _hip_ops.topk_chunked(v.contiguous(), i.contiguous(),
-                                           k_eff, v.shape[1])
-            v, i = v2, i2
+        while v.shape[1] > k_eff:  # candidates of several chunks
+            v, i = _hip_ops.topk_chunked(
+                v, i, k_eff, 8192 if few else v.shape[1])
         if k_eff < k:
             pad_v = torch.full((Q, k - k_eff), float("-inf"),
                                device=v.device)

@@ -1,0 +1,58 @@
+"""Top-k at the edges of its chunks, with piled-up and equal scores."""
+
+import pytest
+import torch
+
+from distllm_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(scores, k):
+    v, i = ops.topk(scores, k)
+    n = min(k, scores.shape[1])
+    want = scores.sort(dim=1, descending=True).values[:, :n]
+    assert v.shape == i.shape == (scores.shape[0], k)
+    assert torch.equal(v[:, :n], want)
+    # every index once, and of the score it stands beside
+    assert torch.equal(scores.gather(1, i[:, :n].long()), want)
+    assert all(len(set(r)) == n for r in i[:, :n].tolist())
+    assert (i[:, n:] == -1).all() and torch.isinf(v[:, n:]).all()
+
+
+@pytest.mark.parametrize("k", [1, 5, 256, 257, 1000])
+@pytest.mark.parametrize("N", [1, 4, 255, 257, 8191, 8192, 8193, 70001])
+def test_sizes(device, N, k):
+    g = torch.Generator(device=device).manual_seed(N + k)
+    _check(torch.randn(3, N, device=device, generator=g), k)
+
+
+@pytest.mark.parametrize("k", [1, 10, 256])
+def test_few_threads_have_the_large_scores(device, k):
+    """All large scores at places of one residue mod 256: far more than the
+    buffer of candidates reach the first bound."""
+    s = torch.rand(2, 20000, device=device)
+    s[:, 3::256] += 10
+    s[:, :8192] = torch.linspace(1, 2, 8192, device=device)
+    _check(s, k)
+    _check(s.flip(1).contiguous(), k)
+
+
+@pytest.mark.parametrize("k", [1, 7, 200])
+def test_equal_scores(device, k):
+    s = torch.zeros(2, 30000, device=device)
+    _check(s, k)
+    s[:, 12345:12350] = 1.0
+    _check(s, k)
+    s[1] = float("-inf")
+    s[1, 17] = torch.finfo(torch.float32).min
+    v, i = ops.topk(s, k)
+    assert i[1, 0] == 17 and torch.isinf(v[1, 1:]).all()
+
+
+def test_equal_scores_by_place(device):
+    """Among a moderate number of equals the first places win."""
+    s = torch.randn(1, 8000, device=device)
+    s[0, 100::500] = 9.0
+    _, i = ops.topk(s, 5)
+    assert i[0].tolist() == [100, 600, 1100, 1600, 2100]
