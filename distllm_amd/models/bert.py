@@ -125,26 +125,24 @@ class BertEncoder(nn.Module):
                 and token_type_ids is None
                 and os.environ.get("DISTLLM_FORCE_VARLEN")):
             return self._forward_packed(ids, attention_mask)
+        pos2d = None
         if self.dims.position_style == "roberta":
             pad = self.dims.pad_token_id
             nz = (ids != pad).int()
             pos2d = (nz.cumsum(1) * nz + pad).long()
-            x = self.word_emb[ids] + self.pos_emb[pos2d]
+        if token_type_ids is None:
+            x = ops.embed_layer_norm(ids, pos2d, self.word_emb, self.pos_emb,
+                                     self.type_emb[0], self.emb_ln_w,
+                                     self.emb_ln_b,
+                                     self.dims.layer_norm_eps)
         else:
-            pos = torch.arange(S, device=ids.device)
-            x = self.word_emb[ids] + self.pos_emb[pos][None, :, :]
-        if token_type_ids is not None:
-            x = x + self.type_emb[token_type_ids.long()]
-        else:
-            x = x + self.type_emb[0]
-        x = ops.layer_norm(x, self.emb_ln_w, self.emb_ln_b,
-                           eps=self.dims.layer_norm_eps)
-        mask_f = torch.where(
-            attention_mask.bool(),
-            torch.zeros((), device=ids.device, dtype=torch.float32),
-            torch.full((), float("-inf"), device=ids.device,
-                       dtype=torch.float32),
-        )
+            if pos2d is None:
+                pos2d = torch.arange(S, device=ids.device)[None, :]
+            x = (self.word_emb[ids] + self.pos_emb[pos2d]
+                 + self.type_emb[token_type_ids.long()])
+            x = ops.layer_norm(x, self.emb_ln_w, self.emb_ln_b,
+                               eps=self.dims.layer_norm_eps)
+        mask_f = ops.key_bias(attention_mask)
         for layer in self.layers:
             x = layer(x, mask_f)
         return x

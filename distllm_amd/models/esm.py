@@ -127,12 +127,7 @@ class Esm2Encoder(nn.Module, _RotaryMixin):
             )
             scale = (1 - mask_ratio_train) / (1 - ratio_obs).clamp(min=1e-6)
             x = (x.float() * scale.unsqueeze(-1)).to(x.dtype)
-        mask_f = torch.where(
-            attention_mask.bool(),
-            torch.zeros((), device=ids.device, dtype=torch.float32),
-            torch.full((), float("-inf"), device=ids.device,
-                       dtype=torch.float32),
-        )
+        mask_f = ops.key_bias(attention_mask)
         pos = (
             torch.arange(S, device=ids.device, dtype=torch.int32)
             .repeat(B, 1)
@@ -141,25 +136,38 @@ class Esm2Encoder(nn.Module, _RotaryMixin):
         cs, sn = self._rope(x.device)
         nh, hd = d.num_heads, d.head_dim
         H = d.hidden_size
-        for layer in self.layers:
-            h = ops.layer_norm(x, layer.ln1_w, layer.ln1_b,
-                               eps=d.layer_norm_eps)
-            qkv = ops.linear(h, layer.wqkv, layer.bqkv)
-            q = qkv[..., :H].view(B, S, nh, hd)
-            k = qkv[..., H : 2 * H].view(B, S, nh, hd)
-            v = qkv[..., 2 * H :].view(B, S, nh, hd)
-            q = ops.rope_apply(q, cs, sn, pos)
-            k = ops.rope_apply(k, cs, sn, pos)
-            ctx = ops.attn_fwd(q, k, v, mask=mask_f, causal=False,
+        h = self._norm(x, self.layers[0].ln1_w, self.layers[0].ln1_b)
+        for li, layer in enumerate(self.layers):
+            qkv = ops.linear(h, layer.wqkv, layer.bqkv).view(B, S, 3 * nh, hd)
+            qkv = ops.rope_qk_(qkv, cs, sn, pos, 2 * nh)
+            ctx = ops.attn_fwd(qkv[:, :, :nh], qkv[:, :, nh: 2 * nh],
+                               qkv[:, :, 2 * nh:], mask=mask_f, causal=False,
                                scale=1.0 / math.sqrt(hd))
-            x = x + ops.linear(ctx.reshape(B, S, H), layer.wo, layer.bo)
-            h = ops.layer_norm(x, layer.ln2_w, layer.ln2_b,
-                               eps=d.layer_norm_eps)
-            act = ops.ACT_GELU_ERF
-            ff = ops.linear(h, layer.w1, layer.b1, act=act)
-            x = x + ops.linear(ff, layer.w2, layer.b2)
-        return ops.layer_norm(x, self.final_ln_w, self.final_ln_b,
-                              eps=d.layer_norm_eps)
+            h, x = self._rest(li, layer, ctx.reshape(B, S, H), x)
+        return h
+
+    def _norm(self, x, w, b):
+        return ops.layer_norm(x, w, b, eps=self.dims.layer_norm_eps)
+
+    def _add_norm(self, y, x, w, b):
+        """(norm(x + y), x + y)"""
+        return ops.norm_fwd_sum(y, x, w, b, eps=self.dims.layer_norm_eps)
+
+    def _next_norm(self, li: int):
+        """Weights of the norm that follows layer li."""
+        if li + 1 < len(self.layers):
+            n = self.layers[li + 1]
+            return n.ln1_w, n.ln1_b
+        return self.final_ln_w, self.final_ln_b
+
+    def _rest(self, li: int, layer, ctx, x):
+        """A layer behind its attention: (normed input of what follows,
+        residual)."""
+        h, x = self._add_norm(ops.linear(ctx, layer.wo, layer.bo), x,
+                              layer.ln2_w, layer.ln2_b)
+        ff = ops.linear(h, layer.w1, layer.b1, act=ops.ACT_GELU_ERF)
+        return self._add_norm(ops.linear(ff, layer.w2, layer.b2), x,
+                              *self._next_norm(li))
 
     @torch.no_grad()
     def _forward_packed(self, ids, attention_mask, x):
@@ -199,26 +207,16 @@ class Esm2Encoder(nn.Module, _RotaryMixin):
             xp = torch.nn.functional.pad(xp, (0, 0, 0, Tp - T0))
             pos = torch.nn.functional.pad(pos, (0, Tp - T0))
         T = xp.shape[0]
-        for layer in self.layers:
-            h = ops.layer_norm(xp, layer.ln1_w, layer.ln1_b,
-                               eps=d.layer_norm_eps)
-            qkv = ops.linear(h, layer.wqkv, layer.bqkv)
-            q = qkv[..., :H].view(T, nh, hd)
-            k = qkv[..., H: 2 * H].view(T, nh, hd)
-            v = qkv[..., 2 * H:].view(T, nh, hd).contiguous()
-            q = ops.rope_apply(q.contiguous(), cs, sn, pos)
-            k = ops.rope_apply(k.contiguous(), cs, sn, pos)
-            ctx = ops.attn_varlen(q, k, v, cu, bmap,
+        h = self._norm(xp, self.layers[0].ln1_w, self.layers[0].ln1_b)
+        for li, layer in enumerate(self.layers):
+            qkv = ops.linear(h, layer.wqkv, layer.bqkv).view(T, 3 * nh, hd)
+            qkv = ops.rope_qk_(qkv, cs, sn, pos, 2 * nh)
+            ctx = ops.attn_varlen(qkv[:, :nh], qkv[:, nh: 2 * nh],
+                                  qkv[:, 2 * nh:], cu, bmap,
                                   scale=1.0 / math.sqrt(hd))
-            xp = xp + ops.linear(ctx.reshape(T, H), layer.wo, layer.bo)
-            h = ops.layer_norm(xp, layer.ln2_w, layer.ln2_b,
-                               eps=d.layer_norm_eps)
-            ff = ops.linear(h, layer.w1, layer.b1, act=ops.ACT_GELU_ERF)
-            xp = xp + ops.linear(ff, layer.w2, layer.b2)
-        xp = ops.layer_norm(xp, self.final_ln_w, self.final_ln_b,
-                            eps=d.layer_norm_eps)
+            h, xp = self._rest(li, layer, ctx.reshape(T, H), xp)
         out = torch.zeros(B, S, H, dtype=xp.dtype, device=xp.device)
-        out[maskb] = xp[:T0]
+        out[maskb] = h[:T0]
         return out
 
 
@@ -279,12 +277,7 @@ class EsmCEncoder(nn.Module, _RotaryMixin):
             # length-dispersed protein batches (mean 344 of 1024)
             # measured 2.66x FASTER packed (profiles/RESULTS.md)
             return self._forward_packed(ids, attention_mask, x)
-        mask_f = torch.where(
-            attention_mask.bool(),
-            torch.zeros((), device=ids.device, dtype=torch.float32),
-            torch.full((), float("-inf"), device=ids.device,
-                       dtype=torch.float32),
-        )
+        mask_f = ops.key_bias(attention_mask)
         pos = (
             torch.arange(S, device=ids.device, dtype=torch.int32)
             .repeat(B, 1)
@@ -293,26 +286,33 @@ class EsmCEncoder(nn.Module, _RotaryMixin):
         cs, sn = self._rope(x.device)
         nh, hd = d.num_heads, d.head_dim
         H = d.hidden_size
-        rs = self.residue_scale
-        for layer in self.layers:
-            h = ops.layer_norm(x, layer.ln1_w, layer.ln1_b,
-                               eps=d.layer_norm_eps)
-            qkv = ops.linear(h, layer.wqkv)
-            q = qkv[..., :H].view(B, S, nh, hd)
-            k = qkv[..., H : 2 * H].view(B, S, nh, hd)
-            v = qkv[..., 2 * H :].view(B, S, nh, hd)
-            q = ops.rope_apply(q, cs, sn, pos)
-            k = ops.rope_apply(k, cs, sn, pos)
-            ctx = ops.attn_fwd(q, k, v, mask=mask_f, causal=False,
+        h = self._norm(x, self.layers[0].ln1_w, self.layers[0].ln1_b)
+        for li, layer in enumerate(self.layers):
+            qkv = ops.linear(h, layer.wqkv).view(B, S, 3 * nh, hd)
+            qkv = ops.rope_qk_(qkv, cs, sn, pos, 2 * nh)
+            ctx = ops.attn_fwd(qkv[:, :, :nh], qkv[:, :, nh: 2 * nh],
+                               qkv[:, :, 2 * nh:], mask=mask_f, causal=False,
                                scale=1.0 / math.sqrt(hd))
-            x = x + ops.linear(ctx.reshape(B, S, H), layer.wo) * rs
-            h = ops.layer_norm(x, layer.ln2_w, layer.ln2_b,
-                               eps=d.layer_norm_eps)
-            gate = ops.linear(h, layer.wgate)
-            up = ops.linear(h, layer.wup)
-            x = x + ops.linear(ops.swiglu(gate, up), layer.wdown) * rs
-        return ops.layer_norm(x, self.final_ln_w, self.final_ln_b,
-                              eps=d.layer_norm_eps)
+            h, x = self._rest(li, layer, ctx.reshape(B, S, H), x)
+        return h
+
+    _norm = Esm2Encoder._norm
+    _add_norm = Esm2Encoder._add_norm
+    _next_norm = Esm2Encoder._next_norm
+
+    def _rest(self, li: int, layer, ctx, x):
+        """See Esm2Encoder._rest."""
+        rs = self.residue_scale
+
+        def scaled(y):
+            return y if rs == 1.0 else y * rs
+
+        h, x = self._add_norm(scaled(ops.linear(ctx, layer.wo)), x,
+                              layer.ln2_w, layer.ln2_b)
+        inter = ops.swiglu(ops.linear(h, layer.wgate),
+                           ops.linear(h, layer.wup))
+        return self._add_norm(scaled(ops.linear(inter, layer.wdown)), x,
+                              *self._next_norm(li))
 
     @torch.no_grad()
     def _forward_packed(self, ids, attention_mask, x):
@@ -335,26 +335,14 @@ class EsmCEncoder(nn.Module, _RotaryMixin):
             xp = torch.nn.functional.pad(xp, (0, 0, 0, Tp - T0))
             pos = torch.nn.functional.pad(pos, (0, Tp - T0))
         T = xp.shape[0]
-        rs = self.residue_scale
-        for layer in self.layers:
-            h = ops.layer_norm(xp, layer.ln1_w, layer.ln1_b,
-                               eps=d.layer_norm_eps)
-            qkv = ops.linear(h, layer.wqkv)
-            q = qkv[..., :H].view(T, nh, hd)
-            k = qkv[..., H: 2 * H].view(T, nh, hd)
-            v = qkv[..., 2 * H:].view(T, nh, hd).contiguous()
-            q = ops.rope_apply(q.contiguous(), cs, sn, pos)
-            k = ops.rope_apply(k.contiguous(), cs, sn, pos)
-            ctx = ops.attn_varlen(q, k, v, cu, bmap,
+        h = self._norm(xp, self.layers[0].ln1_w, self.layers[0].ln1_b)
+        for li, layer in enumerate(self.layers):
+            qkv = ops.linear(h, layer.wqkv).view(T, 3 * nh, hd)
+            qkv = ops.rope_qk_(qkv, cs, sn, pos, 2 * nh)
+            ctx = ops.attn_varlen(qkv[:, :nh], qkv[:, nh: 2 * nh],
+                                  qkv[:, 2 * nh:], cu, bmap,
                                   scale=1.0 / math.sqrt(hd))
-            xp = xp + ops.linear(ctx.reshape(T, H), layer.wo) * rs
-            h = ops.layer_norm(xp, layer.ln2_w, layer.ln2_b,
-                               eps=d.layer_norm_eps)
-            gate = ops.linear(h, layer.wgate)
-            up = ops.linear(h, layer.wup)
-            xp = xp + ops.linear(ops.swiglu(gate, up), layer.wdown) * rs
-        xp = ops.layer_norm(xp, self.final_ln_w, self.final_ln_b,
-                            eps=d.layer_norm_eps)
+            h, xp = self._rest(li, layer, ctx.reshape(T, H), xp)
         out = torch.zeros(B, S, H, dtype=xp.dtype, device=xp.device)
-        out[maskb] = xp[:T0]
+        out[maskb] = h[:T0]
         return out

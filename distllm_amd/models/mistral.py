@@ -203,10 +203,10 @@ class DecoderModel(nn.Module):
         B, S, _ = h.shape
         nh, kvh, hd = self.local_heads, self.local_kv_heads, d.head_dim
         cs, sn = self._rope(h.device)
-        # ONE fused qkv GEMM, ONE rope launch (q|k roped, v copied)
+        # ONE fused qkv GEMM, ONE rope launch (q|k in place, v stays)
         qkv = ops.linear(h, layer.wqkv,
                          layer.bqkv).view(B, S, nh + 2 * kvh, hd)
-        qkv = ops.rope_apply(qkv, cs, sn, pos, rope_heads=nh + kvh)
+        qkv = ops.rope_qk_(qkv, cs, sn, pos, nh + kvh)
         q = qkv[:, :, :nh]
         k = qkv[:, :, nh: nh + kvh]
         v = qkv[:, :, nh + kvh:]
@@ -229,12 +229,7 @@ class DecoderModel(nn.Module):
         ids = input_ids.long()
         B, S = ids.shape
         x = self.tok_emb[ids]
-        mask_f = torch.where(
-            attention_mask.bool(),
-            torch.zeros((), device=ids.device, dtype=torch.float32),
-            torch.full((), float("-inf"), device=ids.device,
-                       dtype=torch.float32),
-        )
+        mask_f = ops.key_bias(attention_mask)
         pos = (
             torch.arange(S, device=ids.device, dtype=torch.int32)
             .repeat(B, 1)

@@ -404,6 +404,46 @@ def rope_apply(x, cs, sn, pos, rope_heads: int = -1):
     return torch_ref.rope_apply(x, cs, sn, pos, rope_heads)
 
 
+def rope_qk_(x, cs, sn, pos, heads: int):
+    """Rotates the first `heads` heads of every row of x [..., Hx, D] in
+    place (queries and keys of a fresh projection; values stay) and returns
+    x."""
+    if x.is_cuda and x.shape[-1] in (64, 128) and x.is_contiguous() \
+            and x.data_ptr() % 16 == 0:
+        _require_hip()
+        _hip_ops.rope_inplace(x, cs, sn, pos.int().contiguous(), heads)
+        return x
+    return x.copy_(rope_apply(x, cs, sn, pos, rope_heads=heads))
+
+
+def embed_layer_norm(ids, pos_ids, word, pos, type_row, w, b, eps):
+    """Layer norm of word[ids] + pos[pos_ids] + type_row; pos_ids None:
+    positions 0, 1, ... of every row of ids [B, S]."""
+    if word.is_cuda and word.dtype == torch.bfloat16 \
+            and word.shape[1] % 8 == 0:
+        _require_hip()
+        return _hip_ops.embed_layer_norm(
+            ids.contiguous(), None if pos_ids is None
+            else pos_ids.contiguous(), word, pos, type_row, w, b, eps)
+    p = pos[: ids.shape[1]][None] if pos_ids is None else pos[pos_ids]
+    return layer_norm(word[ids] + p + type_row, w, b, eps=eps)
+
+
+def key_bias(mask):
+    """Additive key mask of the attention: 0 where mask is not zero, -inf
+    where it is."""
+    if mask.is_cuda and not mask.is_floating_point() \
+            and mask.element_size() in (1, 4, 8):
+        _require_hip()
+        return _hip_ops.key_bias(mask.contiguous())
+    return torch.where(
+        mask.bool(),
+        torch.zeros((), device=mask.device, dtype=torch.float32),
+        torch.full((), float("-inf"), device=mask.device,
+                   dtype=torch.float32),
+    )
+
+
 def gateup_swiglu(x, wgup, bias=None):
     """silu(x @ Wg^T) * (x @ Wu^T) with Wg|Wu packed as wgup [2I, K].
     Few rows: ONE product with the swiglu in the same launch; otherwise one

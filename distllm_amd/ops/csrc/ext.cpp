@@ -14,8 +14,16 @@ void launch_bias_gelu(const void*, const void*, void*, long, int, bool,
 void launch_swiglu(const void*, const void*, void*, long, hipStream_t);
 void launch_swiglu_packed(const void*, void*, long, int, hipStream_t);
 void launch_bias_add(const void*, const void*, void*, long, int, hipStream_t);
-void launch_mean_pool(const void*, const int*, float*, int, int, int, bool,
-                      hipStream_t);
+void launch_mean_pool(const void*, const int*, float*, float*, int, int, int,
+                      int, bool, hipStream_t);
+int mean_pool_shares(int, int);
+void launch_embed_layer_norm(const long*, const long*, const void*,
+                             const void*, const void*, const void*,
+                             const void*, void*, long, int, int, long, long,
+                             float, hipStream_t);
+void launch_key_bias(const void*, float*, long, int, hipStream_t);
+void launch_rope_inplace(void*, const float*, const float*, const int*, long,
+                         long, int, int, hipStream_t);
 void launch_last_token_pool(const void*, const int*, float*, int, int, int,
                             bool, bool, hipStream_t);
 void launch_l2_normalize(const float*, float*, int, int, hipStream_t);
@@ -111,8 +119,17 @@ torch::Tensor mean_pool(torch::Tensor hidden, torch::Tensor mask,
   CHECK_DEV(hidden); CHECK_CONT(hidden); CHECK_BF16(hidden); CHECK_I32(mask);
   const int R = hidden.size(0), S = hidden.size(1), H = hidden.size(2);
   auto out = torch::empty({R, H}, hidden.options().dtype(at::kFloat));
+  if (R == 0) return out;
+  TORCH_CHECK(H % 8 == 0 && H <= 16384, "H must be mult of 8, <= 16384");
+  TORCH_CHECK(mask.is_contiguous() && mask.numel() == (long)R * S,
+              "mask must be [R, S]");
+  const int NS = mean_pool_shares(R, S);
+  torch::Tensor parts;
+  if (NS > 1) parts = torch::empty({R, NS, H}, out.options());
   launch_mean_pool(hidden.data_ptr(), mask.data_ptr<int>(),
-                   out.data_ptr<float>(), R, S, H, normalize, cur_stream());
+                   out.data_ptr<float>(),
+                   NS > 1 ? parts.data_ptr<float>() : nullptr, R, S, H, NS,
+                   normalize, cur_stream());
   return out;
 }
 
@@ -239,6 +256,73 @@ torch::Tensor rope_apply(torch::Tensor x, torch::Tensor cs, torch::Tensor sn,
   launch_rope(x.data_ptr(), out.data_ptr(), cs.data_ptr<float>(),
               sn.data_ptr<float>(), pos.data_ptr<int>(), n_rows, Hx, D,
               rope_heads < 0 ? Hx : (int)rope_heads, cur_stream());
+  return out;
+}
+
+// x [..., heads or more, D], rows of equal stride: the first `heads` heads of
+// every row are rotated in place
+void rope_inplace(torch::Tensor x, torch::Tensor cs, torch::Tensor sn,
+                  torch::Tensor pos, int64_t heads) {
+  CHECK_DEV(x); CHECK_CONT(x); CHECK_BF16(x);
+  CHECK_FLOATS(cs); CHECK_FLOATS(sn); CHECK_INTS(pos);
+  const int D = x.size(-1);
+  const long ld = x.size(-2) * (long)D, n_rows = x.numel() / ld;
+  TORCH_CHECK(D == 64 || D == 128, "head_dim must be 64 or 128");
+  TORCH_CHECK(heads >= 0 && heads <= x.size(-2) && pos.numel() == n_rows,
+              "one position per row, at most its heads");
+  TORCH_CHECK(cs.size(-1) == D / 2 && cs.sizes() == sn.sizes() &&
+                  (uintptr_t)x.data_ptr() % 16 == 0,
+              "rotation tables must be [positions, D / 2]");
+  if (n_rows > 0)
+    launch_rope_inplace(x.data_ptr(), cs.data_ptr<float>(),
+                        sn.data_ptr<float>(), pos.data_ptr<int>(), n_rows, ld,
+                        (int)heads, D, cur_stream());
+}
+
+// ---- encoder inputs ---------------------------------------------------------
+torch::Tensor embed_layer_norm(torch::Tensor ids,
+                               c10::optional<torch::Tensor> pos_ids,
+                               torch::Tensor word, torch::Tensor pos,
+                               torch::Tensor type, torch::Tensor w,
+                               torch::Tensor b, double eps) {
+  CHECK_DEV(ids); CHECK_CONT(ids);
+  TORCH_CHECK(ids.scalar_type() == at::kLong && ids.dim() == 2,
+              "ids must be int64 [B, S]");
+  const int S = ids.size(1), H = word.size(1);
+  for (const auto& t : {word, pos, type, w, b}) {
+    CHECK_DEV(t); CHECK_CONT(t); CHECK_BF16(t);
+    TORCH_CHECK(t.size(-1) == H, "equal widths");
+  }
+  TORCH_CHECK(H % 8 == 0 && H <= 8192, "H must be mult of 8, <= 8192");
+  if (pos_ids) {
+    CHECK_DEV(pos_ids.value()); CHECK_CONT(pos_ids.value());
+    TORCH_CHECK(pos_ids->scalar_type() == at::kLong &&
+                    pos_ids->numel() == ids.numel(),
+                "pos_ids must be int64, one per token");
+  } else {
+    TORCH_CHECK(S <= pos.size(0), "more tokens than positions");
+  }
+  auto out = torch::empty({ids.size(0), S, H}, word.options());
+  if (ids.numel() > 0)
+    launch_embed_layer_norm(
+        (const long*)ids.data_ptr<int64_t>(),
+        pos_ids ? (const long*)pos_ids->data_ptr<int64_t>() : nullptr,
+        word.data_ptr(), pos.data_ptr(), type.data_ptr(), w.data_ptr(),
+        b.data_ptr(), out.data_ptr(), ids.numel(), S, H, word.size(0),
+        pos.size(0), (float)eps, cur_stream());
+  return out;
+}
+
+torch::Tensor key_bias(torch::Tensor mask) {
+  CHECK_DEV(mask); CHECK_CONT(mask);
+  const int bytes = mask.element_size();
+  TORCH_CHECK(!mask.is_floating_point() && !mask.is_complex() &&
+                  (bytes == 1 || bytes == 4 || bytes == 8),
+              "mask must be of 8, 32 or 64 bit integers or truth values");
+  auto out = torch::empty(mask.sizes(), mask.options().dtype(at::kFloat));
+  if (mask.numel() > 0)
+    launch_key_bias(mask.data_ptr(), out.data_ptr<float>(), mask.numel(),
+                    bytes, cur_stream());
   return out;
 }
 
@@ -438,6 +522,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("attn_varlen", &attn_varlen);
   m.def("rope_apply", &rope_apply, py::arg("x"), py::arg("cs"),
         py::arg("sn"), py::arg("pos"), py::arg("rope_heads") = -1);
+  m.def("rope_inplace", &rope_inplace);
+  m.def("embed_layer_norm", &embed_layer_norm, py::arg("ids"),
+        py::arg("pos_ids"), py::arg("word"), py::arg("pos"), py::arg("type"),
+        py::arg("w"), py::arg("b"), py::arg("eps"));
+  m.def("key_bias", &key_bias);
   m.def("topk_chunked", &topk_chunked);
   m.def("hamming_score", &hamming_score);
   m.def("ivf_score", &ivf_score);

@@ -1,0 +1,76 @@
+"""What precedes and follows an encoder's layers: embeddings with their norm,
+key masks, rotation in place, pooled means."""
+
+import pytest
+import torch
+
+from distllm_amd import ops
+from distllm_amd.ops import torch_ref
+
+pytestmark = pytest.mark.gpu
+
+
+def _some(device, *s, seed=0):
+    g = torch.Generator(device=device).manual_seed(seed)
+    return torch.randn(*s, device=device, generator=g).to(torch.bfloat16)
+
+
+@pytest.mark.parametrize("H", [8, 512, 520, 768, 1280, 8192])
+@pytest.mark.parametrize("own", [False, True])
+def test_embed_layer_norm(device, H, own):
+    word, pos, row = (_some(device, n, H, seed=n) for n in (50, 12, 1))
+    w, b = _some(device, H, seed=1), _some(device, H, seed=2)
+    ids = torch.randint(-50, 50, (3, 11), device=device)  # negative: from
+    at = torch.randint(0, 12, (3, 11), device=device) if own else None
+    got = ops.embed_layer_norm(ids, at, word, pos, row[0], w, b, 1e-5)
+    p = pos[:11][None] if at is None else pos[at]
+    want = torch.nn.functional.layer_norm(
+        word[ids].float() + p.float() + row[0].float(), (H,), w.float(),
+        b.float(), 1e-5)
+    torch.testing.assert_close(got.float(), want, atol=1e-2, rtol=8e-3)
+
+
+@pytest.mark.parametrize("dtype", [torch.bool, torch.int8, torch.uint8,
+                                   torch.int16, torch.int32, torch.int64,
+                                   torch.float32])
+def test_key_bias(device, dtype):
+    m = (torch.arange(600, device=device).view(2, 300) % 3).to(dtype)
+    want = torch.where(m.bool(), 0.0, float("-inf"))
+    assert torch.equal(ops.key_bias(m), want)
+    assert torch.equal(ops.key_bias(m.t()), want.t())
+
+
+@pytest.mark.parametrize("D", [16, 64, 128])
+@pytest.mark.parametrize("Hx,heads", [(1, 1), (3, 2), (9, 9), (48, 40),
+                                      (20, 0)])
+@pytest.mark.parametrize("rows", [1, 7, 130])
+def test_rope_in_place(device, rows, Hx, heads, D):
+    cs, sn = ops.rope_tables(64, D, device=device)
+    x = _some(device, rows, Hx, D, seed=rows)
+    pos = torch.arange(rows, device=device, dtype=torch.int32) * 5 % 64
+    want = torch_ref.rope_apply(x, cs, sn, pos, rope_heads=heads)
+    if heads == 0:
+        want = x.clone()
+    got = ops.rope_qk_(x, cs, sn, pos, heads)
+    assert got is x
+    assert torch.equal(x[:, heads:], want[:, heads:])
+    # one rounding of sums of two products that may cancel
+    torch.testing.assert_close(x.float(), want.float(), atol=4e-3,
+                               rtol=2 ** -7)
+
+
+@pytest.mark.parametrize("normalize", [False, True])
+@pytest.mark.parametrize("H", [8, 320, 768, 1280, 4096])
+@pytest.mark.parametrize("R,S", [(1, 1), (1, 24), (3, 33), (2, 700),
+                                 (600, 40)])
+def test_mean_pool(device, R, S, H, normalize):
+    x = _some(device, R, S, H, seed=S)
+    mask = torch.zeros(R, S, device=device, dtype=torch.int32)
+    for r in range(R):
+        mask[r, : max(1, S - 5 * r % S)] = 1
+    got = ops.mean_pool(x, mask, normalize)
+    want = torch_ref.mean_pool(x.double(), mask, False).double()
+    if normalize:
+        want = torch.nn.functional.normalize(want, dim=-1)
+    # fp32 sums of up to 700 numbers of unit size
+    torch.testing.assert_close(got.double(), want, atol=2e-6, rtol=2e-5)
