@@ -314,8 +314,7 @@ class DecoderModel(nn.Module):
             h2, x = ops.norm_fwd_sum(attn, x, layer.post_norm,
                                      eps=d.rms_norm_eps, rms=True)
             if fp8 is not None:
-                gu = ops.gemv_fp8(h2[:, 0], *f["wgup"])
-                inter = ops._hip_ops.swiglu_packed(gu)
+                inter = ops.gateup_swiglu_fp8(h2[:, 0], *f["wgup"])
                 down = self._allreduce(
                     ops.gemv_fp8(inter, *f["wdown"])).unsqueeze(1)
             else:

@@ -491,11 +491,20 @@ def quantize_fp8_rows(w: torch.Tensor):
 
 def gemv_fp8(x, wq, scale, bias=None):
     """out = x @ (dequant(wq) * scale)^T (+bias). x bf16 [M<=8, K],
-    wq uint8 fp8-e4m3 [N, K], scale f32 [N]. One wave per output
-    column; the fp32 dot runs on the quantized values, the channel
-    scale applies after — see csrc/gemv_fp8.hip."""
+    wq uint8 fp8-e4m3 [N, K], scale f32 [N]. The fp32 dot runs on the
+    quantized values, the channel scale applies after — see
+    csrc/gemv_fp8.hip."""
     _require_hip()
     return _hip_ops.gemv_fp8(x.contiguous(), wq, scale, bias)
+
+
+def gateup_swiglu_fp8(x, wq, scale):
+    """silu(x @ Wg^T) * (x @ Wu^T) with Wg|Wu packed and quantized as for
+    gemv_fp8."""
+    _require_hip()
+    if wq.shape[1] % 128 == 0:
+        return _hip_ops.gemv_fp8(x.contiguous(), wq, scale, None, True)
+    return _hip_ops.swiglu_packed(gemv_fp8(x, wq, scale))
 
 
 rope_tables = torch_ref.rope_tables

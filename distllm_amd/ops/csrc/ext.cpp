@@ -43,7 +43,7 @@ void launch_hamming_score(const void*, const void*, float*, int, long, int,
 void launch_ivf_score(const void*, const int*, const int*, const float*,
                       float*, int, int, int, int, hipStream_t);
 void launch_gemv_fp8(const void*, const void*, const float*, const void*,
-                     void*, int, int, long, hipStream_t);
+                     void*, int, int, long, bool, hipStream_t);
 void launch_sample(const float*, const float*, int*, int, int, float, float,
                    hipStream_t);
 void launch_paged_attn(const void*, long, const void*, const void*,
@@ -483,7 +483,7 @@ torch::Tensor ivf_score(torch::Tensor slabs, torch::Tensor lens,
 
 torch::Tensor gemv_fp8(torch::Tensor x, torch::Tensor wq,
                        torch::Tensor scale,
-                       c10::optional<torch::Tensor> bias) {
+                       c10::optional<torch::Tensor> bias, bool swiglu) {
   CHECK_DEV(x); CHECK_CONT(x); CHECK_BF16(x);
   CHECK_DEV(wq); CHECK_CONT(wq);
   TORCH_CHECK(wq.scalar_type() == at::kByte, "wq must be uint8 (fp8)");
@@ -501,10 +501,12 @@ torch::Tensor gemv_fp8(torch::Tensor x, torch::Tensor wq,
     TORCH_CHECK(bias->size(0) == N, "bias shape");
     bptr = bias->data_ptr();
   }
-  auto out = torch::empty({M, N}, x.options());
+  TORCH_CHECK(!swiglu || (N % 2 == 0 && K % 128 == 0),
+              "swiglu needs two halves and K % 128 == 0");
+  auto out = torch::empty({M, swiglu ? N / 2 : N}, x.options());
   launch_gemv_fp8(x.data_ptr(), wq.data_ptr(),
                   scale.data_ptr<float>(), bptr, out.data_ptr(), M, N,
-                  K, cur_stream());
+                  K, swiglu, cur_stream());
   return out;
 }
 
@@ -531,7 +533,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("hamming_score", &hamming_score);
   m.def("ivf_score", &ivf_score);
   m.def("gemv_fp8", &gemv_fp8, py::arg("x"), py::arg("wq"),
-        py::arg("scale"), py::arg("bias") = py::none());
+        py::arg("scale"), py::arg("bias") = py::none(),
+        py::arg("swiglu") = false);
   m.def("sample_tokens", &sample_tokens);
   m.def("paged_attn", &paged_attn);
   m.def("cache_put", &cache_put);
