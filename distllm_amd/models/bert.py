@@ -22,6 +22,17 @@ from .. import ops
 from .config import ModelDims
 
 
+def _watched(layers) -> bool:
+    """Whether hooks on a layer's call, or a layer of another make, want it
+    called."""
+    from torch.nn.modules import module as m
+
+    return bool(m._global_forward_hooks or m._global_forward_pre_hooks
+                or any(type(x) is not BertLayer or x._forward_hooks
+                       or x._forward_pre_hooks or "forward" in x.__dict__
+                       for x in layers))
+
+
 class BertLayer(nn.Module):
     def __init__(self, d: ModelDims):
         super().__init__()
@@ -39,6 +50,12 @@ class BertLayer(nn.Module):
         self.b2 = nn.Parameter(torch.empty(H))
         self.ln2_w = nn.Parameter(torch.empty(H))
         self.ln2_b = nn.Parameter(torch.empty(H))
+
+    def tensors(self) -> tuple[torch.Tensor, ...]:
+        """In the order of ops.bert_few_rows."""
+        return (self.wqkv, self.bqkv, self.wo, self.bo, self.ln1_w,
+                self.ln1_b, self.w1, self.b1, self.w2, self.b2, self.ln2_w,
+                self.ln2_b)
 
     def forward(self, x: torch.Tensor, mask_f: torch.Tensor | None):
         d = self.d
@@ -143,9 +160,24 @@ class BertEncoder(nn.Module):
             x = ops.layer_norm(x, self.emb_ln_w, self.emb_ln_b,
                                eps=self.dims.layer_norm_eps)
         mask_f = ops.key_bias(attention_mask)
+        out = self._few_rows(x, mask_f)
+        if out is not None:
+            return out
         for layer in self.layers:
             x = layer(x, mask_f)
         return x
+
+    def _few_rows(self, x, mask_f):
+        """The layers' output from one native call, None where that does not
+        apply (ops.bert_few_rows) or a layer's call is watched."""
+        if (not x.is_cuda or x.shape[0] * x.shape[1] > 64
+                or not self.layers or _watched(self.layers)):
+            return None
+        d = self.dims
+        return ops.bert_few_rows(
+            x, mask_f, [layer.tensors() for layer in self.layers],
+            d.num_heads, d.layer_norm_eps,
+            ops.ACT_GELU_ERF if d.gelu == "erf" else ops.ACT_GELU_TANH)
 
     @torch.no_grad()
     def _forward_packed(self, ids, attention_mask):

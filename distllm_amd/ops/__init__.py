@@ -11,6 +11,7 @@ numerics ground truth in tests.
 from __future__ import annotations
 
 import math
+import os
 
 import torch
 
@@ -177,9 +178,9 @@ def _autotune_gemm(x2, weight, bias, act):
 _DECODE_ACT = {ACT_NONE: 0, ACT_GELU_TANH: 6, ACT_GELU_ERF: 7, ACT_SILU: 8}
 
 
-def _few_rows(x2, N, columns=64):
-    """Whether a product of x2 with N columns and an activation in the same
-    launch takes decode_gemm (csrc/decode_gemm.hip): up to 64 rows it is
+def _few_rows(x2, weight, bias=None, columns=64):
+    """Whether a product of x2 with the rows of weight (in multiples of
+    `columns`) and an activation in the same launch takes decode_gemm (csrc/decode_gemm.hip): up to 64 rows it is
     faster than the library's product at every size measured (64 rows of
     28672 x 4096, gated: 51 against 57 us; 768 x 768: 3.8 against 7), up to 256
     where the product is narrow enough for the launch that it saves to count
@@ -187,9 +188,14 @@ def _few_rows(x2, N, columns=64):
     against 59). K of a single 64-wide chunk, which would leave three of a
     workgroup's four waves idle, keeps its general path."""
     M, K = x2.shape
-    return (x2.dtype == torch.bfloat16 and x2.is_contiguous()
+    N = weight.shape[0]
+    return ((M <= 64 or (M <= 256 and N <= 16384))
             and K % 64 == 0 and K >= 128 and N % columns == 0
-            and (M <= 64 or (M <= 256 and N <= 16384)))
+            and x2.dtype == weight.dtype == torch.bfloat16
+            and x2.is_contiguous() and weight.is_contiguous()
+            and x2.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0
+            and (bias is None or (bias.dtype == torch.bfloat16
+                                  and bias.is_contiguous())))
 
 
 def linear(x, weight, bias=None, act=ACT_NONE):
@@ -199,8 +205,6 @@ def linear(x, weight, bias=None, act=ACT_NONE):
     (decode_gemm.hip, with the activation) for M <= 64 and among the
     choices for M <= 256. Override with
     DISTLLM_GEMM=blaslt|gemm8|gemm16|decode."""
-    import os
-
     orig_shape = x.shape
     x2 = x.reshape(-1, orig_shape[-1])
     M, K = x2.shape
@@ -210,7 +214,7 @@ def linear(x, weight, bias=None, act=ACT_NONE):
         mode = os.environ.get("DISTLLM_GEMM", "auto")
         if x2.dtype == torch.float32:  # true 32-bit products
             mode = "blaslt"
-        if mode != "blaslt" and M <= 64 and _few_rows(x2, N):
+        if mode != "blaslt" and M <= 64 and _few_rows(x2, weight, bias):
             out = _hip_ops.decode_gemm(x2, weight, bias, 0, _DECODE_ACT[act])
             return out.reshape(*orig_shape[:-1], N)
         if (mode != "blaslt" and act == ACT_NONE and M <= 256
@@ -444,6 +448,32 @@ def key_bias(mask):
     )
 
 
+def bert_few_rows(x, mask_f, layers, heads, eps, act):
+    """All layers (post-normed, each a tuple of its twelve tensors, see
+    csrc/encoder_layers.cpp) of a BERT-class encoder on x [B, S, H] in one
+    call; None where rows, types or sizes want the general path, layer by
+    layer: the rules are those of linear's products of few rows, with which
+    every product here would be made, and of the attention's native head
+    sizes."""
+    M, H = x.shape[0] * x.shape[1], x.shape[2]
+    if not (x.is_cuda and x.dtype == torch.bfloat16 and 0 < M <= 64
+            and act in (ACT_GELU_TANH, ACT_GELU_ERF)
+            and H // heads in (64, 128) and H % heads == 0
+            and "DISTLLM_GEMM" not in os.environ):
+        return None
+    w1, w2 = layers[0][6], layers[0][8]
+    for w in (layers[0][0], w1, w2):
+        if w.shape[0] % 64 or w.shape[1] % 64 or w.shape[1] < 128:
+            return None
+    if not all(t.dtype == torch.bfloat16 and t.is_contiguous()
+               and t.device == x.device for p in layers for t in p):
+        return None
+    _require_hip()
+    return _hip_ops.bert_few_rows(x.contiguous(), mask_f,
+                                  [t for p in layers for t in p], heads, eps,
+                                  _DECODE_ACT[act])
+
+
 def gateup_swiglu(x, wgup, bias=None):
     """silu(x @ Wg^T) * (x @ Wu^T) with Wg|Wu packed as wgup [2I, K].
     Few rows: ONE product with the swiglu in the same launch; otherwise one
@@ -454,7 +484,7 @@ def gateup_swiglu(x, wgup, bias=None):
     I = wgup.shape[0] // 2
     if x.is_cuda:
         _require_hip("_hip_gemm")
-        if _few_rows(x2, wgup.shape[0], 128):
+        if _few_rows(x2, wgup, bias, 128):
             out = _hip_ops.decode_gemm(x2, wgup, bias, 0, 1)
             return out.reshape(*orig_shape[:-1], I)
     gu = linear(x2, wgup, bias)
@@ -471,7 +501,7 @@ def gateup_clamped_glu(x, wgup, limit, alpha, shift):
     with the clamped g. For few rows ONE launch, as gateup_swiglu."""
     if x.is_cuda:
         _require_hip("_hip_gemm")
-        if _few_rows(x, wgup.shape[0], 128):
+        if _few_rows(x, wgup, None, 128):
             return _hip_ops.decode_gemm(x, wgup, None, 0, 2, limit, alpha,
                                         shift)
         return _hip_ops.clamped_glu(linear(x, wgup), limit, alpha, shift)
@@ -819,7 +849,7 @@ def up_xielu(x, wup, act):
     if x.is_cuda:
         _require_hip("_hip_gemm")
         _require_hip("_hip_experts")
-        if _few_rows(x, wup.shape[0]):
+        if _few_rows(x, wup):
             return _hip_ops.decode_gemm(x, wup, None, 0, 3, act_nums=act)
         return _hip_ops.xielu(linear(x, wup), act)
     return torch_ref.xielu(linear(x, wup), act)
@@ -871,7 +901,7 @@ def up_relu2(x, wup):
     """The square of relu(x @ wup^T)."""
     if x.is_cuda:
         _require_hip("_hip_gemm")
-        if _few_rows(x, wup.shape[0]):
+        if _few_rows(x, wup):
             return _hip_ops.decode_gemm(x, wup, None, 0, 5)
         return _hip_ops.relu2(linear(x, wup))
     return torch_ref.relu2(linear(x, wup))
@@ -910,7 +940,7 @@ def gated_rows(x, wgate, tokens, table, col0, n):
     columns of wgate behind n."""
     if x.is_cuda:
         _require_hip("_hip_gemm")
-        if _few_rows(x, wgate.shape[0]):
+        if _few_rows(x, wgate):
             return _hip_ops.decode_gemm_rows(x, wgate, 0, tokens, table,
                                              col0, n)
         return _hip_ops.gelu_rows(linear(x, wgate), tokens, table, col0, n)

@@ -1,0 +1,93 @@
+// All layers of a BERT-class encoder on few rows (a question: one text, a few
+// dozen tokens) in one call. Seven launches a layer of 2 to 5 us each were
+// issued one by one from Python at 8 us apiece, so the GPU waited for the
+// host: 1 x 24 tokens through 12 layers of 768 took 750 us, of which it
+// computed 300. Here they follow each other at the cost of a launch, on
+// buffers that live as long as the call.
+#include "ext_common.h"
+#include "gelu_rows.h"
+
+extern "C" {
+void launch_norm_fwd(const void*, const void*, const void*, const void*,
+                     void*, void*, int, int, float, bool, hipStream_t);
+void launch_attn_fwd(const void*, const void*, const void*, const float*,
+                     void*, int, int, int, int, int, int, bool, float, long,
+                     long, long, long, hipStream_t);
+void launch_decode_gemm(const void*, const void*, const void*, void*, void*,
+                        int, int, int, int, bool, int, float, float, float,
+                        const float*, const RowsArgs*, hipStream_t);
+int decode_gemm_shares(int, int, int);
+}
+
+// x [B, S, H]; mask [B, S] additive; layers: wqkv, bqkv, wo, bo, ln1_w, ln1_b,
+// w1, b1, w2, b2, ln2_w, ln2_b of every layer in turn; act: decode_gemm's code
+// of the feed-forward's activation.
+torch::Tensor bert_few_rows(torch::Tensor x, torch::Tensor mask,
+                            std::vector<torch::Tensor> layers, int64_t heads,
+                            double eps, int64_t act) {
+  CHECK_DEV(x); CHECK_CONT(x); CHECK_BF16(x);
+  CHECK_FLOATS(mask);
+  TORCH_CHECK(x.dim() == 3, "x must be [B, S, H]");
+  const int B = x.size(0), S = x.size(1), H = x.size(2), M = B * S;
+  const int D = H / (int)heads;
+  TORCH_CHECK(H % heads == 0 && (D == 64 || D == 128), "head size");
+  TORCH_CHECK(mask.numel() == M && mask.size(0) == B, "mask must be [B, S]");
+  TORCH_CHECK(M >= 1 && M <= 64 && H % 64 == 0 && H <= 8192, "x size");
+  TORCH_CHECK(layers.size() % 12 == 0 && !layers.empty(),
+              "twelve tensors per layer");
+  TORCH_CHECK(act == 6 || act == 7, "activation");
+  const long I = layers[6].size(0);
+  TORCH_CHECK(I % 64 == 0, "feed-forward size");
+  const long rows[12] = {3L * H, 3L * H, H, H, H, H, I, I, H, H, H, H};
+  const long cols[12] = {H, 0, H, 0, 0, 0, H, 0, I, 0, 0, 0};
+  for (size_t i = 0; i < layers.size(); ++i) {
+    const auto& t = layers[i];
+    const int k = i % 12;
+    TORCH_CHECK(t.is_cuda() && t.device() == x.device() &&
+                    t.scalar_type() == at::kBFloat16 && t.is_contiguous() &&
+                    t.size(0) == rows[k] && t.dim() == (cols[k] ? 2 : 1) &&
+                    (cols[k] == 0 || t.size(1) == cols[k]),
+                "layer tensor ", k, " of layer ", i / 12);
+  }
+  auto some = [&](long n) { return torch::empty({M, n}, x.options()); };
+  auto qkv = some(3 * H), ctx = some(H), y = some(H), a = some(H),
+       h = some(I), z = torch::empty_like(x);
+  auto shares = [&](int n, int k) { return decode_gemm_shares(M, n, k); };
+  const long slab = std::max(
+      std::max((long)shares(3 * H, H) * 3 * H, (long)shares(H, H) * H),
+      std::max((long)shares(I, H) * I, (long)shares(H, I) * H));
+  auto slabs = torch::empty({slab, (long)M}, x.options().dtype(at::kFloat));
+  const hipStream_t st = cur_stream();
+  auto gemm = [&](const torch::Tensor& in, const torch::Tensor& w,
+                  const torch::Tensor& b, torch::Tensor& out, int code) {
+    const int n = w.size(0), k = w.size(1);
+    launch_decode_gemm(in.data_ptr(), w.data_ptr(), b.data_ptr(),
+                       out.data_ptr(), slabs.data_ptr(), M, n, k,
+                       shares(n, k), false, code, 0.f, 0.f, 0.f, nullptr,
+                       nullptr, st);
+  };
+  auto norm = [&](const torch::Tensor& in, const torch::Tensor& res,
+                  const torch::Tensor& w, const torch::Tensor& b,
+                  torch::Tensor& out) {
+    launch_norm_fwd(in.data_ptr(), res.data_ptr(), w.data_ptr(), b.data_ptr(),
+                    out.data_ptr(), nullptr, M, H, (float)eps, false, st);
+  };
+  const long row = 3L * H;
+  torch::Tensor in = x;
+  for (size_t i = 0; i < layers.size(); i += 12) {
+    const torch::Tensor* p = &layers[i];
+    gemm(in, p[0], p[1], qkv, 0);
+    const char* q = (const char*)qkv.data_ptr();
+    launch_attn_fwd(q, q + 2L * H, q + 4L * H, mask.data_ptr<float>(),
+                    ctx.data_ptr(), B, S, S, (int)heads, (int)heads, D, false,
+                    (float)(1.0 / std::sqrt((double)D)), S * row, row,
+                    S * row, row, st);
+    gemm(ctx, p[2], p[3], y, 0);
+    norm(y, in, p[4], p[5], a);
+    gemm(a, p[6], p[7], h, (int)act);
+    gemm(h, p[8], p[9], y, 0);
+    norm(y, a, p[10], p[11], z);
+    in = z;
+  }
+  return z;
+}

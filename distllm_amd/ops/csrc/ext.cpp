@@ -510,6 +510,11 @@ torch::Tensor gemv_fp8(torch::Tensor x, torch::Tensor wq,
   return out;
 }
 
+// encoder_layers.cpp
+torch::Tensor bert_few_rows(torch::Tensor x, torch::Tensor mask,
+                            std::vector<torch::Tensor> layers, int64_t heads,
+                            double eps, int64_t act);
+
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("norm_fwd", &norm_fwd, "fused residual+LayerNorm/RMSNorm");
   m.def("bias_gelu", &bias_gelu);
@@ -529,6 +534,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("pos_ids"), py::arg("word"), py::arg("pos"), py::arg("type"),
         py::arg("w"), py::arg("b"), py::arg("eps"));
   m.def("key_bias", &key_bias);
+  m.def("bert_few_rows", &bert_few_rows);
   m.def("topk_chunked", &topk_chunked);
   m.def("hamming_score", &hamming_score);
   m.def("ivf_score", &ivf_score);

@@ -47,7 +47,9 @@ GROUPS = {
 }
 _taken = {s for group in GROUPS.values() for s in group}
 # *_hip.hip files are torch-hipify build artifacts — exclude them.
-GROUPS["_hip_ops"] = ["ext.cpp"] + sorted(
+# (with the products of few rows, for the encoder layers)
+GROUPS["_hip_ops"] = ["ext.cpp", "encoder_layers.cpp",
+                      "decode_gemm.hip"] + sorted(
     p.name for p in CSRC.glob("*.hip")
     if not p.name.endswith("_hip.hip") and p.name not in _taken
 )

@@ -89,3 +89,15 @@ def test_linear(device, M, act):
     x, w, b = _inputs(M, 192, 256, device, M)
     _close(ops.linear(x[None], w, b, act)[0],
            torch_ref.gemm(x.float(), w.float(), b.float(), act).float())
+
+
+@pytest.mark.parametrize("act", [ops.ACT_GELU_ERF, ops.ACT_SILU])
+def test_strided_weights(device, act):
+    """Weights and biases that the form does not read as they lie."""
+    x, w, b = _inputs(20, 192, 256, device, 5)
+    want = torch_ref.gemm(x.float(), w.float(), b.float(), act).float()
+    _close(ops.linear(x, w.t().contiguous().t(), b, act), want)
+    _close(ops.linear(x, w, torch.stack([b, b], 1)[:, 0], act), want)
+    wide = torch.zeros(20, 257, device=device, dtype=torch.bfloat16)
+    wide[:, 1:] = x
+    _close(ops.linear(wide[:, 1:], w, b, act), want)
