@@ -226,19 +226,23 @@ torch::Tensor latent_attn(torch::Tensor q, torch::Tensor cache,
                             e.ld_gate, is_f32(q), cur_stream());
     return out;
   }
-  // Split each row's keys until the CUs are full (two workgroups each, one
-  // of the largest), as long as a split keeps four tiles. All sizes are
-  // known on the host, so a captured graph stays valid as contexts grow.
+  // Split each row's keys until the 256 CUs have a workgroup each (its
+  // buffers take a CU's LDS; more than fit would be a second round), as long
+  // as a share keeps two tiles of 64 keys; four tiles are not worth the second
+  // launch. Measured at rank 512, 32 heads, us: 16 rows of 100 to 4000 keys
+  // 12 shares 28, 16 25, 24 35; 32 rows of 300 to 2048 4 30, 8 25, 12 32; 64
+  // rows of 60 to 200 1 14, 2 16, 4 17; 1 row of 2048 8 17.6, 16 16.2, 32 18.
+  // All sizes are known on the host, so a captured graph stays valid as
+  // contexts grow.
   long NS = nsplit;
   if (NS <= 0) {
     const long per_wg = latent_decode_heads(H);
     const long wgs = (long)M * ((H + per_wg - 1) / per_wg);
     const long keys = std::min<long>(win, bt.size(1) * 16L);
-    const long tiles = keys / 32 + 1;
-    const long fill = per_wg > 32 ? 256 : 512;
-    NS = std::min<long>({(fill + wgs - 1) / wgs, (tiles + 3) / 4, 64L});
+    const long tiles = keys / 64 + 1;
+    NS = tiles <= 4 ? 1 : std::min<long>(256 / wgs, (tiles + 1) / 2);
   }
-  NS = std::max<long>(NS, 1);
+  NS = std::min<long>(std::max<long>(NS, 1), 64);
   torch::Tensor pacc, pml;
   void *pa = nullptr, *pm = nullptr;
   if (NS > 1) {

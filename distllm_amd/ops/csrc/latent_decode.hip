@@ -6,37 +6,64 @@
 // from HBM once for all of them; the visible keys of a row are split over NS
 // workgroups whose partial results a second kernel joins.
 //
-// Tiles of 32 keys go global -> registers -> LDS, where each tile is kept
-// twice: row-major (key operand of the score product) and transposed (the
-// same numbers as value operand). The next tile's loads are in flight while
-// the current one is used.
-//
-// KS waves work on each head group. For the scores they split the keys of
-// the tile (and, when KS is 4, the latent columns, whose partial sums meet
-// in LDS); for the output each owns R / KS latent columns, which keeps the
-// accumulators of a wave small. Both products use
-// mfma_f32_16x16x32_bf16 with keys (then latent columns) as rows and heads
-// as columns, so softmax state and rescaling are lane-local.
-//
 // Cache rows and queries have RR = R + ROT numbers, of which all take part in
-// the scores and the first R are the value. The others need no transposed
-// copy: they go to LDS directly, while the tile before is weighted.
+// the scores and the first R are the value. The same bytes are key and value,
+// so a tile of 64 keys goes to LDS once, as it lies in the cache, by
+// global_load_lds (the next tile's loads are in flight behind the current
+// one); values are transposed on their way out of LDS.
+//  - scores: each of the 4 waves of a head group has 16 keys (one page) and
+//    a softmax state of its own;
+//  - the waves exchange their weights and maxima through LDS;
+//  - output: each wave has R / 4 latent columns, for all keys.
+// Both products are mfma_f32_16x16x32_bf16 with keys (then latent columns) as
+// rows and heads as columns, so that states and rescaling are lane-local; a
+// lane's weights of the exchange are its operand of the second product.
+//
+// At many keys bound by reading the cache, at few by the chain through a tile
+// (0.7 us of it barriers, maxima and exchange) and the two launches. One wave
+// for two head groups reads LDS half as often, but has nobody to fill its
+// waits: 2.9 us a tile against 1.9. Tiles of 32 keys that passed through
+// registers and were kept twice, one copy transposed, with 64 heads in a
+// workgroup, took (rank 512, 32 heads, us, then and now) 1 row of 2048 keys
+// 28 -> 16, 32 rows of 300 to 2048 38 -> 25, 16 of 100 to 4000 47 -> 25, 64 of
+// 200 to 2000 44 -> 35; 64 heads: 32 rows of 2048 41 -> 34, 64 rows of 200 to
+// 2000 53 -> 51, for the second group of 32 heads reads the tiles from L2.
 #include "common.h"
 
 #define PBLK 16
-#define KT 32
+#define KT 64  // keys of a tile: a page for each wave
 #define LOG2E 1.4426950408889634f
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
 
 extern __shared__ __attribute__((aligned(16))) char smem[];
 
-#define SROW 36  // padded row of 32 scores
+union ld_frag {
+  bf16x8 v;
+  s16x4 h[2];
+  unsigned int d[4];
+};
 
-// byte address of the 16-byte slot (4 per row: 32 keys) of latent column r;
-// 64 bytes of padding per 8 rows and the slot swizzle spread the banks
-__device__ __forceinline__ int ct_slot(int r, int slot) {
-  return r * 64 + (r >> 3) * 64 + ((slot ^ ((r >> 2) & 3)) * 16);
+__device__ __forceinline__ unsigned int ld_pack(float a, float b) {
+  return __builtin_bit_cast(
+      unsigned int, __builtin_convertvector(f32x2{a, b}, bf16x2));
+}
+
+// LDS of the workgroup is done with what it read or written by all
+__device__ __forceinline__ void ld_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// Where the 16-byte piece c of row r of R numbers lies in the row. Pieces are
+// read by 16 rows at a time (keys) and by 4 rows x 2 neighbours (values): the
+// low bits of the row move pairs, the next one swaps within a pair.
+template <int R>
+__device__ __forceinline__ int ld_piece(int r, int c) {
+  return R % 128 == 0 ? c ^ ((r & 7) << 1 | (r >> 3 & 1))
+                      : c ^ ((r & 3) << 1 | (r >> 2 & 1));
 }
 
 // Weight of a row's sum: 1 / l with the softmax's state m (log2 units), l and
@@ -55,8 +82,13 @@ __device__ __forceinline__ float row_weight(float m, float l, long row,
   return inv;
 }
 
-template <int R, int ROT, int HG, int KS>
-__global__ void __launch_bounds__(64 * HG * KS, 2)
+template <int R, int ROT, int HG>
+constexpr int ld_lds() {
+  return 2 * KT * (R + ROT) * 2 + 4 * HG * (1024 + 64);
+}
+
+template <int R, int ROT, int HG>
+__global__ void __launch_bounds__(256 * HG, R + ROT <= 256 ? 2 * HG : HG)
 latent_decode_kernel(const unsigned short* __restrict__ q,
                      const unsigned short* __restrict__ cache,
                      const int* __restrict__ block_table,
@@ -64,32 +96,47 @@ latent_decode_kernel(const unsigned short* __restrict__ q,
                      const int* __restrict__ ctx,
                      unsigned short* __restrict__ out,
                      float* __restrict__ pacc, float* __restrict__ pml,
-                     int H, int NG, int NS, int max_blocks, int window,
+                     int M, int H, int NG, int NS, int max_blocks, int window,
                      float scale, const float* __restrict__ sink,
                      const unsigned short* __restrict__ gate, int ld_gate) {
-  constexpr int NT = 64 * HG * KS;
+  static_assert(ROT == 0 || ROT == 64, "eight 16-byte pieces per key");
   constexpr int RR = R + ROT;
-  constexpr int UNITS = R;  // a unit: 4 keys x 8 latent columns
-  constexpr int UPT = (UNITS + NT - 1) / NT;
-  constexpr int SW = R % 128 == 0 ? 15 : 7;
-  constexpr int CT = KT * R * 2;        // LDS offset of the transposed copy
-  constexpr int SC = CT + R * 72;       // LDS offset of the scores
-  constexpr int RSPLIT = KS / 2;       // column parts, besides key halves
-  constexpr int RO = SC + HG * RSPLIT * 16 * SROW * 4;  // of the key parts
-  constexpr int QS = R / 32 / RSPLIT;  // score steps of a wave
-  constexpr int TS = ROT / 32 / RSPLIT;  // and those behind the latent
-  constexpr int OB = R / 16 / KS;      // output blocks of a wave
-  static_assert(KS == 2 || KS == 4, "two key halves");
+  constexpr int MAIN = KT * R * 2;  // of a buffer; its key parts follow
+  constexpr int BUF = KT * RR * 2;
+  constexpr int RP = R / 8;         // 16-byte pieces of a row
+  constexpr int NP = R / 32 / HG;   // copies of a wave: 16 / HG rows' values
+  constexpr int NR = ROT / 32 / HG; // and their key parts
+  constexpr int QS = R / 32, TS = ROT / 32;  // score steps
+  constexpr int OB = R / 64;        // output blocks of a wave
 
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  const int i16 = lane & 15, g = lane >> 4;
-  const int hgrp = wid / KS, ks = wid % KS;
-  const int khalf = ks % 2, rhalf = ks / 2;
-  const int split = blockIdx.x % NS;
-  const int grp = blockIdx.x / NS % NG;
-  const int row = blockIdx.x / NS / NG;
-  const int head = (grp * HG + hgrp) * 16 + i16;
-  const bool live = head < H;
+  const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int w = wid & 3, hg = wid >> 2;  // page of the tile, head group
+  const int c16 = lane & 15, g = lane >> 4;
+  // the workgroups of the same keys follow on one XCD, which reads them once
+  const int share = blockIdx.x / (8 * NG) * 8 + blockIdx.x % 8;
+  const int grp = blockIdx.x / 8 % NG;
+  const int split = share % NS, row = share / NS;
+  if (row >= M) return;
+  const int head0 = grp * HG * 16;
+  float* weights =
+      reinterpret_cast<float*>(smem + 2 * BUF) + hg * 4 * 256;
+  float* maxima =
+      reinterpret_cast<float*>(smem + 2 * BUF) + HG * 4 * 256 + hg * 64;
+
+  // queries pass through the second buffer
+  char* qb = smem + BUF;
+  auto from = [&](int r) {
+    return q + ((long)row * H + min(head0 + r, H - 1)) * RR;
+  };
+  for (int p = wid; p < HG * QS; p += 4 * HG) {
+    const int at = p * 64 + lane, r = at / RP, c = at % RP;
+    copy_to_lds(from(r) + ld_piece<R>(r & 15, c) * 8, qb + p * 1024);
+  }
+  for (int p = wid; p < HG * TS; p += 4 * HG) {
+    const int r = p * 8 + (lane >> 3), c = (lane & 7) ^ (r & 7);
+    copy_to_lds(from(r) + R + c * 8, qb + MAIN + p * 1024);
+  }
 
   const int L = min(ctx[row], max_blocks * PBLK);
   const int lo = L > window ? L - window : 0;
@@ -99,222 +146,201 @@ latent_decode_kernel(const unsigned short* __restrict__ q,
   const int last_page = L > 0 ? (L - 1) / PBLK : 0;
   const int* bt = block_table + (long)row_seq[row] * max_blocks;
 
-  const int kg = (threadIdx.x >> 3) & 7;  // key group of all my units
-  auto page_of = [&](int t) {
-    return bt[min(t * (KT / PBLK) + (kg >> 2), last_page)];
+  // page w of each of the next 64 tiles, on the lanes
+  int pages = 0;
+  auto fetch_pages = [&](int t) {
+    pages = bt[max(min((t + lane) * 4 + w, last_page), lo / PBLK)];
   };
-  i32x4 kv[UPT][4];
-  auto issue = [&](int page) {
-    const unsigned short* base =
-        cache + ((long)page * PBLK + (kg & 3) * 4) * RR;
+  auto issue = [&](int t) {
+    if (((t - ts) & 63) == 0) fetch_pages(t);
+    const unsigned short* src =
+        cache +
+        (long)__builtin_amdgcn_readlane(pages, (t - ts) & 63) * PBLK * RR;
+    char* dst = smem + ((t - ts) & 1) * BUF;
 #pragma unroll
-    for (int i = 0; i < UPT; ++i) {
-      const int u = threadIdx.x + i * NT;
-      if (UNITS % NT == 0 || u < UNITS) {
-        const int c = (u >> 6) * 8 + (u & 7);
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          kv[i][j] =
-              *reinterpret_cast<const i32x4*>(base + (long)j * RR + c * 8);
-      }
+    for (int i = 0; i < NP; ++i) {
+      const int p = hg * NP + i;
+      const int at = p * 64 + lane, r = at / RP, c = at % RP;
+      copy_to_lds(src + r * RR + ld_piece<R>(r, c) * 8,
+                  dst + (w * NP * HG + p) * 1024);
     }
-  };
-  auto stage = [&]() {
 #pragma unroll
-    for (int i = 0; i < UPT; ++i) {
-      const int u = threadIdx.x + i * NT;
-      if (UNITS % NT == 0 || u < UNITS) {
-        const int c = (u >> 6) * 8 + (u & 7);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int key = kg * 4 + j;
-          *reinterpret_cast<i32x4*>(smem + key * (R * 2) +
-                                    ((c ^ (key & SW)) * 16)) = kv[i][j];
-        }
-#pragma unroll
-        for (int w = 0; w < 4; ++w) {
-          i32x2 even, odd;
-          even[0] = __builtin_amdgcn_perm(kv[i][1][w], kv[i][0][w],
-                                          0x05040100);
-          even[1] = __builtin_amdgcn_perm(kv[i][3][w], kv[i][2][w],
-                                          0x05040100);
-          odd[0] = __builtin_amdgcn_perm(kv[i][1][w], kv[i][0][w],
-                                         0x07060302);
-          odd[1] = __builtin_amdgcn_perm(kv[i][3][w], kv[i][2][w],
-                                         0x07060302);
-          const int r = c * 8 + w * 2;
-          char* dst = smem + CT + (kg & 1) * 8;
-          *reinterpret_cast<i32x2*>(dst + ct_slot(r, kg >> 1)) = even;
-          *reinterpret_cast<i32x2*>(dst + ct_slot(r + 1, kg >> 1)) = odd;
-        }
-      }
+    for (int i = 0; i < NR; ++i) {
+      const int p = hg * NR + i;
+      const int r = p * 8 + (lane >> 3), c = (lane & 7) ^ (r & 7);
+      copy_to_lds(src + r * RR + R + c * 8,
+                  dst + MAIN + (w * NR * HG + p) * 1024);
     }
   };
 
-  // key parts: four waves copy eight keys each
-  auto part_page = [&](int t) {
-    return bt[min(t * (KT / PBLK) + (wid >> 1), last_page)];
-  };
-  auto stage_part = [&](int page) {
-    static_assert(ROT == 0 || ROT == 64, "eight 16-byte pieces per key");
-    if (wid >= 4) return;
-    const int key = wid * 8 + (lane >> 3);
-    const unsigned short* src = cache +
-                                ((long)page * PBLK + (key & 15)) * RR + R +
-                                ((lane & 7) ^ (key & 7)) * 8;
-    auto dst = (__attribute__((address_space(3))) unsigned int*)(
-        smem + RO + wid * 1024 + lane * 16);
-    __builtin_amdgcn_global_load_lds(
-        (const __attribute__((address_space(1))) unsigned int*)src, dst, 16,
-        0, 0);
-  };
-
-  int page = 0, ppage = 0;
-  if (ts < te) {
-    issue(page_of(ts));
-    page = page_of(min(ts + 1, te - 1));
-    if (ROT > 0) {
-      stage_part(part_page(ts));
-      ppage = part_page(min(ts + 1, te - 1));
-    }
-  }
   bf16x8 qf[QS + TS];
-  {
-    const unsigned short* qr =
-        q + ((long)row * H + (live ? head : 0)) * RR + g * 8;
+  if (ts < te) {
+    issue(ts);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"i"(NP + NR) : "memory");
+    ld_barrier();
 #pragma unroll
-    for (int s = 0; s < QS + TS; ++s) {
-      s16x8 v = *reinterpret_cast<const s16x8*>(
-          qr + (s < QS ? (rhalf * QS + s) * 32
-                       : R + (rhalf * TS + s - QS) * 32));
-      if (!live) v = (s16x8)(short)0;
-      qf[s] = __builtin_bit_cast(bf16x8, v);
+    for (int s = 0; s < QS; ++s)
+      qf[s] = *reinterpret_cast<const bf16x8*>(
+          qb + (hg * 16 + c16) * (R * 2) +
+          ld_piece<R>(c16, s * 4 + g) * 16);
+#pragma unroll
+    for (int s = 0; s < TS; ++s)
+      qf[QS + s] = *reinterpret_cast<const bf16x8*>(
+          qb + MAIN + (hg * 16 + c16) * (ROT * 2) +
+          (((s * 4 + g) ^ (c16 & 7)) * 16));
+    ld_barrier();
+    if (ts + 1 < te) {
+      issue(ts + 1);
+      asm volatile("s_waitcnt vmcnt(%0)" ::"i"(NP + NR) : "memory");
     }
   }
+  if (ts + 1 >= te) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
-  float m = -1e30f, l = 0.f;
+  const float scale2 = scale * LOG2E;
+  float m = -1e30f;              // of the sums: the largest of all waves
+  float mw = -1e30f, lw = 0.f;   // of this wave's keys
   f32x4 acc[OB];
 #pragma unroll
   for (int i = 0; i < OB; ++i) acc[i] = {0.f, 0.f, 0.f, 0.f};
-  const float scale2 = scale * LOG2E;
-  float* scores = reinterpret_cast<float*>(smem + SC) +
-                  hgrp * (RSPLIT * 16 * SROW) + i16 * SROW;
 
   for (int t = ts; t < te; ++t) {
-    __syncthreads();  // every wave is done with the previous tile
-    if (ROT > 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    stage();
-    if (t + 1 < te) {
-      issue(page);
-      page = page_of(min(t + 2, te - 1));
+    char* buf = smem + ((t - ts) & 1) * BUF;
+    const int key0 = t * KT + w * 16;
+    if (key0 + 16 > L) {
+      // what lies behind the last key must not meet its zero weight; each
+      // wave clears what it copied
+      for (int at = max(max(L - key0, 0) * (R * 2), hg * NP * 1024) +
+                    lane * 16;
+           at < (hg + 1) * NP * 1024; at += 1024)
+        *reinterpret_cast<i32x4*>(buf + w * (QS * 1024) + at) =
+            i32x4{0, 0, 0, 0};
     }
-    __syncthreads();
+    // this tile is there and the other buffer is free
+    ld_barrier();
+    if (t > ts && t + 1 < te) issue(t + 1);
 
-    // scores of my keys over my columns, in two chains
-    f32x4 sa[2];
-    sa[0] = {0.f, 0.f, 0.f, 0.f};
-    sa[1] = {0.f, 0.f, 0.f, 0.f};
+    // scores of my 16 keys, in two chains
+    f32x4 sc = {0.f, 0.f, 0.f, 0.f}, sc2 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int s = 0; s < QS; ++s) {
-      const int chunk = (rhalf * QS + s) * 4 + g;
-      const char* a = smem + (khalf * 16 + i16) * (R * 2) +
-                      ((chunk ^ (i16 & SW)) * 16);
-      const bf16x8 k0 = *reinterpret_cast<const bf16x8*>(a);
-      sa[s & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-          k0, qf[s], sa[s & 1], 0, 0, 0);
+    for (int s = 0; s < QS + TS; ++s) {
+      const char* a =
+          s < QS ? buf + (w * 16 + c16) * (R * 2) +
+                       ld_piece<R>(c16, s * 4 + g) * 16
+                 : buf + MAIN + (w * 16 + c16) * (ROT * 2) +
+                       ((((s - QS) * 4 + g) ^ (c16 & 7)) * 16);
+      const bf16x8 kf = *reinterpret_cast<const bf16x8*>(a);
+      f32x4& to = s & 1 ? sc2 : sc;
+      to = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[s], to, 0, 0, 0);
     }
+    float top = -INFINITY;
 #pragma unroll
-    for (int s = 0; s < TS; ++s) {
-      const int chunk = (rhalf * TS + s) * 4 + g;
-      const bf16x8 k0 = *reinterpret_cast<const bf16x8*>(
-          smem + RO + (khalf * 16 + i16) * 128 + ((chunk ^ (i16 & 7)) * 16));
-      sa[s & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-          k0, qf[QS + s], sa[s & 1], 0, 0, 0);
+    for (int r = 0; r < 4; ++r) {
+      const int key = key0 + g * 4 + r;
+      sc[r] = key >= lo && key < L ? (sc[r] + sc2[r]) * scale2 : -INFINITY;
+      top = fmaxf(top, sc[r]);
     }
+    top = fmaxf(top, __shfl_xor(top, 16, 64));
+    top = fmaxf(top, __shfl_xor(top, 32, 64));
+    const float mn = fmaxf(mw, top);
+    lw *= __builtin_amdgcn_exp2f(mw - mn);
+    mw = mn;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) sa[0][r] += sa[1][r];
-    *reinterpret_cast<f32x4*>(scores + rhalf * (16 * SROW) + khalf * 16 +
-                              g * 4) = sa[0];
-    __syncthreads();
-    if (ROT > 0 && t + 1 < te) {
-      stage_part(ppage);
-      ppage = part_page(min(t + 2, te - 1));
+    for (int r = 0; r < 4; ++r) {
+      sc[r] = __builtin_amdgcn_exp2f(sc[r] - mn);
+      lw += sc[r];  // of the keys of this lane
     }
+    *reinterpret_cast<f32x4*>(weights + (w * 64 + lane) * 4) = sc;
+    if (g == 0) maxima[w * 16 + c16] = mn;
+    ld_barrier();
 
-    // weights of all 32 keys for my head: lane group g has keys g*8 .. + 7
-    float p[8];
-    float pmax = -INFINITY;
+    // all weights, relative to the largest maximum so far
+    ld_frag pf[2];
+    float mx[4], ma = m;
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      f32x4 v = *reinterpret_cast<const f32x4*>(scores + g * 8 + h * 4);
-      if (RSPLIT == 2) {
-        const f32x4 v2 = *reinterpret_cast<const f32x4*>(
-            scores + 16 * SROW + g * 8 + h * 4);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] += v2[r];
-      }
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int key = t * KT + g * 8 + h * 4 + r;
-        p[h * 4 + r] = key >= lo && key < L ? v[r] * scale2 : -INFINITY;
-        pmax = fmaxf(pmax, p[h * 4 + r]);
-      }
+    for (int i = 0; i < 4; ++i) {
+      mx[i] = maxima[i * 16 + c16];
+      ma = fmaxf(ma, mx[i]);
     }
-    pmax = fmaxf(pmax, __shfl_xor(pmax, 16, 64));
-    pmax = fmaxf(pmax, __shfl_xor(pmax, 32, 64));
-    if (!__all(pmax <= m)) {
-      const float mn = fmaxf(m, pmax);
-      const float alpha = __builtin_amdgcn_exp2f(m - mn);
-      m = mn;
-      l *= alpha;
+    if (!__all(ma <= m)) {
+      const float alpha = __builtin_amdgcn_exp2f(m - ma);
+      m = ma;
 #pragma unroll
       for (int i = 0; i < OB; ++i)
 #pragma unroll
         for (int r = 0; r < 4; ++r) acc[i][r] *= alpha;
     }
-    s16x8 pb;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const float e = __builtin_amdgcn_exp2f(p[i] - m);
-      l += e;  // this lane's keys only; lanes are joined at the end
-      pb[i] = (short)f2bf(e);
+    for (int i = 0; i < 4; ++i) {
+      const f32x4 p =
+          *reinterpret_cast<const f32x4*>(weights + (i * 64 + lane) * 4);
+      const float f = __builtin_amdgcn_exp2f(mx[i] - m);
+      pf[i >> 1].d[(i & 1) * 2] = ld_pack(p[0] * f, p[1] * f);
+      pf[i >> 1].d[(i & 1) * 2 + 1] = ld_pack(p[2] * f, p[3] * f);
     }
-    const bf16x8 pf = __builtin_bit_cast(bf16x8, pb);
+    // keys 4 g .. 4 g + 3 of two pages at a time, as the weights lie
+    const int vr = g * 4 + (c16 >> 2);
 #pragma unroll
     for (int i = 0; i < OB; ++i) {
-      const bf16x8 v = *reinterpret_cast<const bf16x8*>(
-          smem + CT + ct_slot((ks * OB + i) * 16 + i16, g));
-      acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, pf, acc[i], 0, 0,
-                                                       0);
+      const int c = (w * OB + i) * 2 + (c16 >> 1 & 1);
+      const char* a =
+          buf + vr * (R * 2) + ld_piece<R>(vr, c) * 16 + (c16 & 1) * 8;
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb) {
+        ld_frag vf;
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+          vf.h[e] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+              (__attribute__((address_space(3))) s16x4*)(
+                  a + (kb * 2 + e) * (16 * R * 2)));
+        acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf.v, pf[kb].v,
+                                                         acc[i], 0, 0, 0);
+      }
     }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
-  l += __shfl_xor(l, 16, 64);
-  l += __shfl_xor(l, 32, 64);
-  if (!live) return;
+
+  // sums of the weights of all waves
+  lw += __shfl_xor(lw, 16, 64);
+  lw += __shfl_xor(lw, 32, 64);
+  ld_barrier();
+  if (g == 0) {
+    weights[w * 16 + c16] = lw;
+    maxima[w * 16 + c16] = mw;
+  }
+  ld_barrier();
+  const int head = head0 + hg * 16 + c16;
+  if (head >= H) return;
+  float l = 0.f;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    l += weights[i * 16 + c16] *
+         __builtin_amdgcn_exp2f(maxima[i * 16 + c16] - m);
   const long rh = (long)row * H + head;
-  const int col = ks * (OB * 16) + g * 4;
+  const int col = w * (OB * 16) + g * 4;
   if (NS == 1) {
     const float inv = row_weight(m, l, row, head, sink, gate, ld_gate);
 #pragma unroll
     for (int i = 0; i < OB; ++i) {
-      s16x4 o;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) o[r] = (short)f2bf(acc[i][r] * inv);
-      *reinterpret_cast<s16x4*>(out + rh * R + col + i * 16) = o;
+      const i32x2 o = {(int)ld_pack(acc[i][0] * inv, acc[i][1] * inv),
+                       (int)ld_pack(acc[i][2] * inv, acc[i][3] * inv)};
+      *reinterpret_cast<i32x2*>(out + rh * R + col + i * 16) = o;
     }
   } else {
     const long part = rh * NS + split;
 #pragma unroll
     for (int i = 0; i < OB; ++i)
       *reinterpret_cast<f32x4*>(pacc + part * R + col + i * 16) = acc[i];
-    if (g == 0 && ks == 0) {
+    if (g == 0 && w == 0) {
       pml[part * 2] = m;
       pml[part * 2 + 1] = l;
     }
   }
 }
 
-// one wave per (row, head): join NS partial results
+// Join NS <= 64 partial results: a wave per (row, head) and 256 columns, the
+// shares' states on its lanes. With a wave per (row, head) that went through
+// the states one by one: 32 rows of 32 heads, 8 shares of rank 512, 12.7 us,
+// now 4.8.
 __global__ void __launch_bounds__(256)
 latent_combine_kernel(const float* __restrict__ pacc,
                       const float* __restrict__ pml,
@@ -322,36 +348,38 @@ latent_combine_kernel(const float* __restrict__ pacc,
                       int NS, int H, const float* __restrict__ sink,
                       const unsigned short* __restrict__ gate, int ld_gate) {
   const int lane = threadIdx.x & 63;
-  const long rh = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int parts = (R + 255) / 256;
+  const int at = blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int rh = at / parts, c = at % parts * 256 + lane * 4;
   if (rh >= RH) return;
-  float M = -1e30f;
-  for (int s = 0; s < NS; ++s) M = fmaxf(M, pml[(rh * NS + s) * 2]);
-  float l = 0.f;
-  for (int s = 0; s < NS; ++s)
-    l += pml[(rh * NS + s) * 2 + 1] *
-         __builtin_amdgcn_exp2f(pml[(rh * NS + s) * 2] - M);
-  const float inv =
-      row_weight(M, l, rh / H, (int)(rh % H), sink, gate, ld_gate);
-  for (int c = lane * 4; c < R; c += 256) {
-    f32x4 o = {0.f, 0.f, 0.f, 0.f};
-    for (int s = 0; s < NS; ++s) {
-      const float a =
-          __builtin_amdgcn_exp2f(pml[(rh * NS + s) * 2] - M) * inv;
-      const f32x4 v =
-          *reinterpret_cast<const f32x4*>(pacc + (rh * NS + s) * R + c);
+  float m = -1e30f, l = 0.f;
+  if (lane < NS) {
+    m = pml[((long)rh * NS + lane) * 2];
+    l = pml[((long)rh * NS + lane) * 2 + 1];
+  }
+  const float M = wave_reduce_max(m);
+  float a = __builtin_amdgcn_exp2f(m - M);
+  const float sum = wave_reduce_sum(l * a);
+  a *= row_weight(M, sum, rh / H, rh % H, sink, gate, ld_gate);
+  const float* p = pacc + (long)rh * NS * R + min(c, R - 4);
+  f32x4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
+  for (int s = 0; s < NS; ++s) {
+    const float w = __builtin_bit_cast(
+        float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, a), s));
+    const f32x4 v = *reinterpret_cast<const f32x4*>(p + (long)s * R);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) o[i] += a * v[i];
-    }
-    s16x4 ov;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) ov[i] = (short)f2bf(o[i]);
-    *reinterpret_cast<s16x4*>(out + rh * R + c) = ov;
+    for (int i = 0; i < 4; ++i) o[i] += w * v[i];
+  }
+  if (c < R) {
+    const i32x2 two = {(int)ld_pack(o[0], o[1]), (int)ld_pack(o[2], o[3])};
+    *reinterpret_cast<i32x2*>(out + (long)rh * R + c) = two;
   }
 }
 
 // heads that one workgroup serves
 extern "C" int latent_decode_heads(int H) {
-  return H <= 16 ? 16 : H <= 32 ? 32 : 64;
+  return H <= 16 ? 16 : 32;
 }
 
 extern "C" bool latent_decode_covers(int R, int rot) {
@@ -367,21 +395,19 @@ extern "C" void launch_latent_decode(
     hipStream_t stream) {
   const int heads = latent_decode_heads(H);
   const int ng = (H + heads - 1) / heads;
-#define LD(RR, RO, HG, KS)                                                    \
-  hipLaunchKernelGGL((latent_decode_kernel<RR, RO, HG, KS>),                  \
-                     dim3(M * ng * NS), dim3(64 * HG * KS),                   \
-                     KT * (RR + RO) * 2 + RR * 72 +                           \
-                         HG * (KS == 4 ? 2 : 1) * 16 * SROW * 4,              \
-                     stream, (const unsigned short*)q,                        \
-                     (const unsigned short*)cache, block_table, row_seq, ctx, \
-                     (unsigned short*)out, (float*)pacc, (float*)pml, H, ng,  \
-                     NS, max_blocks, window, scale, sink,                     \
-                     (const unsigned short*)gate, ld_gate)
-#define LD_H(RR, RO)                      \
-  do {                                    \
-    if (heads == 16) LD(RR, RO, 1, 4);    \
-    else if (heads == 32) LD(RR, RO, 2, 2); \
-    else LD(RR, RO, 4, 2);                \
+#define LD(RR, RO, HG)                                                        \
+  hipLaunchKernelGGL((latent_decode_kernel<RR, RO, HG>),                      \
+                     dim3((M * NS + 7) / 8 * 8 * ng), dim3(256 * HG),         \
+                     (ld_lds<RR, RO, HG>()), stream,                          \
+                     (const unsigned short*)q, (const unsigned short*)cache,  \
+                     block_table, row_seq, ctx, (unsigned short*)out,         \
+                     (float*)pacc, (float*)pml, M, H, ng, NS, max_blocks,     \
+                     window, scale, sink, (const unsigned short*)gate,        \
+                     ld_gate)
+#define LD_H(RR, RO)                 \
+  do {                               \
+    if (heads == 16) LD(RR, RO, 1);  \
+    else LD(RR, RO, 2);              \
   } while (0)
 #define LD_R(RR)              \
   do {                        \
@@ -400,8 +426,9 @@ extern "C" void launch_latent_decode(
 #undef LD_H
 #undef LD
   if (NS > 1)
-    hipLaunchKernelGGL(latent_combine_kernel, dim3((M * H + 3) / 4),
-                       dim3(256), 0, stream, (const float*)pacc,
+    hipLaunchKernelGGL(latent_combine_kernel,
+                       dim3((M * H * ((R + 255) / 256) + 3) / 4), dim3(256),
+                       0, stream, (const float*)pacc,
                        (const float*)pml, (unsigned short*)out, M * H, R, NS,
                        H, sink, (const unsigned short*)gate, ld_gate);
 }
