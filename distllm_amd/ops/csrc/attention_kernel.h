@@ -68,7 +68,10 @@ __device__ __forceinline__ unsigned int pack_bf16(float a, float b) {
   return __builtin_bit_cast(unsigned int, v);
 }
 
-__device__ __forceinline__ void copy_to_lds(const unsigned short* src,
+// The builtin and not copy_to_lds(): here the compiler's wait ahead of the
+// transposing reads costs nothing (several workgroups a CU), and knowing the
+// copies it orders the rest better: 4 x 4096 causal 649 us against 692.
+__device__ __forceinline__ void stage_piece(const unsigned short* src,
                                             char* dst) {
   __builtin_amdgcn_global_load_lds(
       (const __attribute__((address_space(1))) unsigned int*)src,
@@ -229,7 +232,7 @@ attn_fwd_kernel(const unsigned short* __restrict__ Q,
     for (int p = 0; p < KVBLK / KROWS / NWAVE; ++p) {
       const int row = (p * NWAVE + wid) * KROWS + lane / NCH;
       const int c = (lane % NCH) ^ (row & (NCH - 1));
-      copy_to_lds(Kb + (long)min(k0 + row, SKV - 1) * tstr_k + c * 8,
+      stage_piece(Kb + (long)min(k0 + row, SKV - 1) * tstr_k + c * 8,
                   smem + offK[buf] + (p * NWAVE + wid) * 1024 + lane * 16);
     }
     if constexpr (ROT > 0) {
@@ -237,7 +240,7 @@ attn_fwd_kernel(const unsigned short* __restrict__ Q,
 #pragma unroll
       for (int p = 0; p < KVBLK / 8 / NWAVE; ++p) {
         const int row = (p * NWAVE + wid) * 8 + (lane >> 3);
-        copy_to_lds(Kr + (long)(cu_k[b] + min(k0 + row, SKV - 1)) * ROT +
+        stage_piece(Kr + (long)(cu_k[b] + min(k0 + row, SKV - 1)) * ROT +
                         ((lane & 7) ^ (row & 7)) * 8,
                     smem + offR + buf * RTILE_B + (p * NWAVE + wid) * 1024 +
                         lane * 16);
@@ -247,7 +250,7 @@ attn_fwd_kernel(const unsigned short* __restrict__ Q,
     for (int p = 0; p < KVBLK / VROWS / NWAVE; ++p) {
       const int row = (p * NWAVE + wid) * VROWS + lane / NCHV;
       const int c = (lane % NCHV) ^ ((row & 3) << 1);
-      copy_to_lds(Vb + (long)min(k0 + row, SKV - 1) * tstr_k + c * 8,
+      stage_piece(Vb + (long)min(k0 + row, SKV - 1) * tstr_k + c * 8,
                   smem + offV[buf] + (p * NWAVE + wid) * 1024 + lane * 16);
     }
   };

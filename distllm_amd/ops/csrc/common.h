@@ -58,24 +58,36 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// 16 bytes a lane from global memory to LDS: lane i's to base + 16 i, base the
-// same for the whole wave. In assembly, for the compiler must not know of it:
-// it lets a transposing read of LDS (ds_read_b64_tr_b16) wait for every copy
-// that it knows to be in flight, also those into other buffers. So nothing
-// waits by itself, __syncthreads() neither: the caller counts its copies and
-// waits (s_waitcnt vmcnt) before a barrier or a read of the bytes.
+// 16 or 4 bytes a lane from global memory to LDS: lane i's to base + i times
+// as many, base the same for the whole wave. In assembly, for the compiler
+// must not know of it: it lets a transposing read of LDS (ds_read_b64_tr_b16)
+// wait for every copy that it knows to be in flight, also those into other
+// buffers. So nothing waits by itself, __syncthreads() neither: the caller
+// counts its copies and waits (s_waitcnt vmcnt) before a barrier or a read of
+// the bytes.
+template <int BYTES = 16>
 __device__ __forceinline__ void copy_to_lds(const void* src,
                                             const void* base) {
   const unsigned int at = __builtin_amdgcn_readfirstlane(
       (unsigned int)(uintptr_t)(const __attribute__((address_space(3)))
                                     char*)base);
-  asm volatile(
-      "s_mov_b32 m0, %0\n\t"
-      "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %1, off"
-      :
-      : "s"(at), "v"(src)
-      : "memory", "m0");
+  static_assert(BYTES == 16 || BYTES == 4, "a copy's width");
+  if constexpr (BYTES == 16)
+    asm volatile(
+        "s_mov_b32 m0, %0\n\t"
+        "s_nop 0\n\t"
+        "global_load_lds_dwordx4 %1, off"
+        :
+        : "s"(at), "v"(src)
+        : "memory", "m0");
+  else
+    asm volatile(
+        "s_mov_b32 m0, %0\n\t"
+        "s_nop 0\n\t"
+        "global_load_lds_dword %1, off"
+        :
+        : "s"(at), "v"(src)
+        : "memory", "m0");
 }
 
 // Workgroups go round the eight XCDs one by one: number b of n such that

@@ -20,14 +20,16 @@
 //    way out of LDS. Softmax state and rescaling are lane-local but for the
 //    maximum over the four groups of lanes that share a head.
 //  - probabilities stay fp32: each goes in as the sum of two bf16 numbers,
-//    which leaves 2^-17 of it, against the 2^-9 of the bf16 result.
+//    which leaves 2^-16 of it, against the 2^-8 of the bf16 result.
 //  - NS workgroups share a sequence where B * HKV is small; a second launch
 //    joins them.
 // Measured, us, with kernels that read a key row per lane and a value element
 // per lane, and now (32 heads on 8 of 128, bf16; fp8): B = 1, 2048 cached
-// tokens 32 -> 11.2 (31 -> 11.1); B = 16 of 100 to 4000 115 -> 39 (104 -> 24);
-// B = 64 of 200 to 2048 137 -> 65, 4.5 TB/s (117 -> 38); B = 128 of 1000 150 ->
-// 100, 5.2 TB/s (96 -> 56). The 128 KiB of buffers leave one workgroup per CU.
+// tokens 32 -> 11.0 (31 -> 11.1); B = 16 of 100 to 4000 115 -> 36.5 (104 ->
+// 24); B = 64 of 200 to 2048 137 -> 61, 4.8 TB/s (117 -> 38); B = 128 of 1000
+// 150 -> 98, 5.3 TB/s (96 -> 56). With copies that the compiler knows of, which
+// the reads of V then wait for, also for the next tile's: 39, 65 and 101. The
+// 128 KiB of buffers leave one workgroup per CU.
 #include "common.h"
 #include <hip/hip_fp8.h>
 
@@ -82,7 +84,8 @@ paged_attn_kernel(const unsigned short* __restrict__ q, long q_stride,
   constexpr int TILE = KT * D * 2;      // bytes of K or V of a tile
   constexpr int R = pa_ring(D, FP8);
   constexpr int DB = D / 16;
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int c16 = lane & 15, g = lane >> 4;
   const int GR = H / HKV, NG = (GR + 15) / 16;
   const int split = blockIdx.x % NS;
@@ -126,21 +129,17 @@ paged_attn_kernel(const unsigned short* __restrict__ q, long q_stride,
   // bf16: pieces of K and V of tile i, pieces of 16 bytes XOR-ed with the
   // row in K, of 32 bytes in V
   auto issue = [&](int i) {
-    char* dst = ring + (i % R) * 2 * TILE + lane * 16;
+    char* dst = ring + (i % R) * 2 * TILE;
     const int r = lane / NCH, c = lane % NCH;
 #pragma unroll
     for (int p = 0; p < PIECES; ++p) {
       const int row = p * ROWS + r;
       const long at = page(i, p * ROWS / PBLK) * page_bytes + head_bytes +
                       (row % PBLK) * (D * 2);
-      auto go = [&](const char* src, char* to) {
-        __builtin_amdgcn_global_load_lds(
-            (const __attribute__((address_space(1))) unsigned int*)src,
-            (__attribute__((address_space(3))) unsigned int*)to, 16, 0, 0);
-      };
-      go(kcache + at + ((c ^ (row & (NCH - 1))) * 16), dst + p * 1024);
-      go(vcache + at + ((c ^ ((row & 3) << 1)) * 16),
-         dst + TILE + p * 1024);
+      copy_to_lds(kcache + at + ((c ^ (row & (NCH - 1))) * 16),
+                  dst + p * 1024);
+      copy_to_lds(vcache + at + ((c ^ ((row & 3) << 1)) * 16),
+                  dst + TILE + p * 1024);
     }
   };
   // fp8: the same rows through registers, 16 numbers a load
