@@ -68,16 +68,6 @@ __device__ __forceinline__ unsigned int pack_bf16(float a, float b) {
   return __builtin_bit_cast(unsigned int, v);
 }
 
-// The builtin and not copy_to_lds(): here the compiler's wait ahead of the
-// transposing reads costs nothing (several workgroups a CU), and knowing the
-// copies it orders the rest better: 4 x 4096 causal 649 us against 692.
-__device__ __forceinline__ void stage_piece(const unsigned short* src,
-                                            char* dst) {
-  __builtin_amdgcn_global_load_lds(
-      (const __attribute__((address_space(1))) unsigned int*)src,
-      (__attribute__((address_space(3))) unsigned int*)dst, 16, 0, 0);
-}
-
 // LDS of a workgroup: two buffers of keys (and their shared part), values
 // and mask numbers.
 constexpr int attn_lds(int D, int DV, int ROT, bool mask) {
@@ -131,7 +121,13 @@ attn_fwd_kernel(const unsigned short* __restrict__ Q,
   constexpr int VTILE_B = KVBLK * DV * 2;  // V tile bytes
 
   const int lane = threadIdx.x & 63;
-  const int wid = threadIdx.x >> 6;
+  // A wave number that the compiler knows to be uniform, and copies that it
+  // does not know of (copy_to_lds), take fewer registers: packed proteins, 20
+  // heads of 64, 108.5 -> 104 us. Heads of 128 are ordered worse with the
+  // first: 4 x 4096 causal 655 against 692.
+  const int wid = D + DV <= 192
+                      ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)
+                      : threadIdx.x >> 6;
   const int h = lane >> 5;   // half index within wave
   const int qcol = lane & 31;
 
@@ -199,6 +195,17 @@ attn_fwd_kernel(const unsigned short* __restrict__ Q,
   const float scale2 = fabsf(scale) * LOG2E;
   const unsigned int flip = scale < 0.f ? 0x80008000u : 0u;
 
+  int ntile = (SKV + KVBLK - 1) / KVBLK;
+  if (CAUSAL) {
+    const int qmax_blk = min(qb * QBLK + QBLK - 1, SQ - 1);
+    ntile = min(ntile, (qmax_blk + shift) / KVBLK + 1);
+  }
+  unsigned long long some = 0;  // of the first 64 tiles
+  auto holed = [&](int t) { return t >= 64 || (some >> t & 1); };
+  auto mask_read = [&](int t) {
+    return CAUSAL || holed(t) || (t + 1) * KVBLK > SKV;
+  };
+
   // ---- Q fragments in registers ---------------------------------------
   bf16x8 qf[(D + ROT) / 16];
 #pragma unroll
@@ -220,45 +227,35 @@ attn_fwd_kernel(const unsigned short* __restrict__ Q,
 
   // ---- staging: 1 KiB pieces of whole rows, swizzled source -------------
   auto stage = [&](int k0, int buf) {
-    if (HAS_MASK && wid == 0)
-      __builtin_amdgcn_global_load_lds(
-          (const __attribute__((address_space(1))) unsigned int*)(
-              maskp + (long)b * SKV + min(k0 + lane, SKV - 1)),
-          (__attribute__((address_space(3))) unsigned int*)(
-              smem + offM + buf * KVBLK * 4 + lane * 4),
-          4, 0, 0);
+    if (HAS_MASK && wid == 0 && (k0 == 0 || mask_read(k0 / KVBLK)))
+      copy_to_lds<4>(maskp + (long)b * SKV + min(k0 + lane, SKV - 1),
+                     smem + offM + buf * KVBLK * 4);
     constexpr int KROWS = 1024 / (2 * D), VROWS = 1024 / (2 * DV);
 #pragma unroll
     for (int p = 0; p < KVBLK / KROWS / NWAVE; ++p) {
       const int row = (p * NWAVE + wid) * KROWS + lane / NCH;
       const int c = (lane % NCH) ^ (row & (NCH - 1));
-      stage_piece(Kb + (long)min(k0 + row, SKV - 1) * tstr_k + c * 8,
-                  smem + offK[buf] + (p * NWAVE + wid) * 1024 + lane * 16);
+      copy_to_lds(Kb + (long)min(k0 + row, SKV - 1) * tstr_k + c * 8,
+                  smem + offK[buf] + (p * NWAVE + wid) * 1024);
     }
     if constexpr (ROT > 0) {
       static_assert(ROT == 64, "eight 16-byte pieces per row");
 #pragma unroll
       for (int p = 0; p < KVBLK / 8 / NWAVE; ++p) {
         const int row = (p * NWAVE + wid) * 8 + (lane >> 3);
-        stage_piece(Kr + (long)(cu_k[b] + min(k0 + row, SKV - 1)) * ROT +
+        copy_to_lds(Kr + (long)(cu_k[b] + min(k0 + row, SKV - 1)) * ROT +
                         ((lane & 7) ^ (row & 7)) * 8,
-                    smem + offR + buf * RTILE_B + (p * NWAVE + wid) * 1024 +
-                        lane * 16);
+                    smem + offR + buf * RTILE_B + (p * NWAVE + wid) * 1024);
       }
     }
 #pragma unroll
     for (int p = 0; p < KVBLK / VROWS / NWAVE; ++p) {
       const int row = (p * NWAVE + wid) * VROWS + lane / NCHV;
       const int c = (lane % NCHV) ^ ((row & 3) << 1);
-      stage_piece(Vb + (long)min(k0 + row, SKV - 1) * tstr_k + c * 8,
-                  smem + offV[buf] + (p * NWAVE + wid) * 1024 + lane * 16);
+      copy_to_lds(Vb + (long)min(k0 + row, SKV - 1) * tstr_k + c * 8,
+                  smem + offV[buf] + (p * NWAVE + wid) * 1024);
     }
   };
-  int ntile = (SKV + KVBLK - 1) / KVBLK;
-  if (CAUSAL) {
-    const int qmax_blk = min(qb * QBLK + QBLK - 1, SQ - 1);
-    ntile = min(ntile, (qmax_blk + shift) / KVBLK + 1);
-  }
   int tile0 = 0;  // first tile that any row of this workgroup sees
   if (WINDOW) {
     const int first = qb * QBLK + shift - window + 1;
@@ -275,6 +272,24 @@ attn_fwd_kernel(const unsigned short* __restrict__ Q,
                ((d * 2 + ((lane >> 4) & 1)) ^ (vi >> 2)) * 32 + (vi & 3) * 8;
 
   if (tile0 < ntile) stage(tile0 * KVBLK, 0);
+  // ---- mask: which tiles have a number at all, and where the last key lies
+  // that is not -inf in log2 units: the weight of those behind it is 0, their
+  // tiles are left out. 64 x 203 with a quarter of the keys masked, 12 heads
+  // of 64, 33 -> 27 us; 16 x 1024, 32 heads of 128, causal, 264 -> 234; with
+  // nothing masked 512 x 512 takes the same 690 as when a flag was read per
+  // tile, for what the tiles save the first look costs -------------------
+  if constexpr (HAS_MASK) {
+    const float* mrow = maskp + (long)b * SKV;
+    int live = 0;
+#pragma unroll 8
+    for (int t = 0; t < ntile; ++t) {
+      const int k = t * KVBLK + lane;
+      const float v = mrow[min(k, SKV - 1)];
+      if (__any(!(v * LOG2E == -INFINITY))) live = t + 1;
+      if (t < 64 && __any(v != 0.f)) some |= 1ull << t;
+    }
+    ntile = live;
+  }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
 
@@ -322,7 +337,7 @@ attn_fwd_kernel(const unsigned short* __restrict__ Q,
                  k0 <= q0w + QWAVE - 1 + shift - window;
       else
         masked = k0 + KVBLK > SKV || (CAUSAL && k0 + KVBLK - 1 > q0w) ||
-                 (HAS_MASK && __any(mask_lds[cur * KVBLK + lane] != 0.f));
+                 (HAS_MASK && holed(t));
       float pmax = -INFINITY, off, mul;
       if (masked) {
         const unsigned int wspan = WINDOW ? qpos - qlo : 0;

@@ -15,7 +15,7 @@ from distllm_amd.ops import torch_ref
 
 pytestmark = pytest.mark.gpu
 
-# bf16 probabilities and outputs: 2^-9 each, and values of a few units
+# bf16 probabilities and outputs: 2^-8 each, and values of a few units
 TOL = 2e-2
 
 
@@ -51,6 +51,22 @@ def test_general_masks(device, causal, D):
     mask[0, 70:100] = -1.5
     mask[1, 64:128] = -math.inf
     mask[2, 100:] = torch.finfo(torch.float32).min
+    _close(ops.attn_fwd(q, k, v, mask=mask, causal=causal), q, k, v, mask,
+           causal, 1 / math.sqrt(D))
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("S", [193, 512, 4400])
+def test_masked_ends(device, S, causal, D):
+    """Last tiles that no row sees, a last key at either side of a tile's
+    border, masked keys ahead and past the first 64 tiles, no masked key."""
+    q, k, v = _qkv(4, S, 2, 1, D, 9, device)
+    mask = torch.zeros(4, S, device=device)
+    mask[0, 64:] = -math.inf
+    mask[1, 65:] = torch.finfo(torch.float32).min
+    mask[2, S - 100: S - 65] = -math.inf
+    mask[2, S - 64:] = -math.inf
     _close(ops.attn_fwd(q, k, v, mask=mask, causal=causal), q, k, v, mask,
            causal, 1 / math.sqrt(D))
 
