@@ -36,6 +36,9 @@ void launch_attn_varlen(const void*, const void*, const void*, void*,
                         int, int, int, long, long, float, hipStream_t);
 void launch_rope(const void*, void*, const float*, const float*, const int*,
                  long, int, int, int, hipStream_t);
+int score_tile(int);
+void launch_score(const float*, void*, const float*, float*, int, int, int,
+                  hipStream_t);
 void launch_topk_chunk(const float*, const int*, float*, int*, int, long, int,
                        int, hipStream_t);
 void launch_hamming_score(const void*, const void*, float*, int, long, int,
@@ -327,6 +330,28 @@ torch::Tensor key_bias(torch::Tensor mask) {
 }
 
 // ---- search ----------------------------------------------------------------
+torch::Tensor score(torch::Tensor q, torch::Tensor corpus) {
+  CHECK_DEV(q); CHECK_CONT(q); CHECK_F32(q);
+  CHECK_DEV(corpus); CHECK_CONT(corpus); CHECK_F32(corpus);
+  TORCH_CHECK(q.dim() == 2 && corpus.dim() == 2, "matrices");
+  const long Q = q.size(0), K = q.size(1), N = corpus.size(0);
+  TORCH_CHECK(corpus.size(1) == K && K >= 32 && K % 32 == 0, "K % 32");
+  TORCH_CHECK(Q < (1L << 20) && N < (1L << 31) && K < (1L << 20) &&
+                  Q * N < (1L << 39),  // 2^31 workgroups of 64 x 128
+              "score: too large");
+  TORCH_CHECK((uintptr_t)q.data_ptr() % 16 == 0 &&
+                  (uintptr_t)corpus.data_ptr() % 16 == 0,
+              "score: 16-byte alignment");
+  auto out = torch::empty({Q, N}, q.options());
+  if (out.numel() == 0) return out;
+  const long QT = score_tile((int)Q), rows = (Q + QT - 1) / QT * QT;
+  auto planes = torch::empty({rows * K * 6}, q.options().dtype(at::kByte));
+  launch_score(q.data_ptr<float>(), planes.data_ptr(),
+               corpus.data_ptr<float>(), out.data_ptr<float>(), (int)Q,
+               (int)N, (int)K, cur_stream());
+  return out;
+}
+
 std::vector<torch::Tensor> topk_chunked(torch::Tensor scores,
                                         c10::optional<torch::Tensor> in_idx,
                                         int64_t k, int64_t chunk) {
@@ -535,6 +560,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("w"), py::arg("b"), py::arg("eps"));
   m.def("key_bias", &key_bias);
   m.def("bert_few_rows", &bert_few_rows);
+  m.def("score", &score);
   m.def("topk_chunked", &topk_chunked);
   m.def("hamming_score", &hamming_score);
   m.def("ivf_score", &ivf_score);

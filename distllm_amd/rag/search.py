@@ -302,25 +302,20 @@ class HipFlatIndex:
         return normalize_L2(embeddings)
 
     def _topk_exact(self, q: torch.Tensor, k: int):
-        """Chunked GEMM + HIP top-k over the fp32 corpus.
-
-        The scoring GEMM stays a library call by policy: scores are
-        fp32 (faiss-parity exactness) and fp32 GEMM peaks at 157 TF on
-        gfx950 (the f32-input MFMA rate) — rocBLAS's tuned SGEMM
-        (~147 TF) is already at that roofline, so a hand-written f32
-        kernel has nothing to win here. The hand-written kernels own
-        the top-k selection (radix-select, topk_search.hip), the
-        Hamming path and the IVF chunk scorer."""
+        """Chunked scores + HIP top-k over the fp32 corpus. Scores keep
+        fp32 exactness (faiss parity): for batches of queries the product of
+        score.hip, which splits each number into three bf16 parts, for a few
+        the library's fp32 product."""
         N = self.n
         k = min(k, N)
         chunk = self.score_chunk_rows
         if N <= chunk:
-            scores = q @ self.corpus.t()
+            scores = ops.score(q, self.corpus)
             return ops.topk(scores.contiguous(), k)
         vs, is_ = [], []
         for c0 in range(0, N, chunk):
             c1 = min(c0 + chunk, N)
-            scores = q @ self.corpus[c0:c1].t()
+            scores = ops.score(q, self.corpus[c0:c1])
             v, i = ops.topk(scores.contiguous(), min(k, c1 - c0))
             vs.append(v)
             is_.append(i + c0)
