@@ -292,6 +292,8 @@ class DecoderModel(nn.Module):
         # W8A16 small-batch path: fp8 weight GEMV (enable_fp8_decode)
         fp8 = (self._fp8w if self._fp8w is not None and B <= 8
                and x.is_cuda else None)
+        # products whose shares of K the next kernel sums (on one rank)
+        parts = ops.linear_parts if self.tp == 1 else ops.linear
         h = ops.rms_norm(x, self.layers[0].in_norm, eps=d.rms_norm_eps)
         for li, layer in enumerate(self.layers):
             # ONE fused qkv GEMM + ONE launch that rotates q and k and
@@ -300,29 +302,29 @@ class DecoderModel(nn.Module):
                 f = fp8[li]
                 qkv = ops.gemv_fp8(h[:, 0], *f["wqkv"], layer.bqkv)
             else:
-                qkv = ops.linear(h, layer.wqkv, layer.bqkv)
-            q = ops.rope_put(qkv.view(B, nh + 2 * kvh, hd), cs, sn, ctx_lens,
-                             kcaches[li], vcaches[li], block_tables)
+                qkv = (parts if hd in (64, 128) else ops.linear)(
+                    h[:, 0], layer.wqkv, layer.bqkv)
+            q = ops.rope_put(
+                qkv.view(*qkv.shape[:-1], nh + 2 * kvh, hd), cs, sn,
+                ctx_lens, kcaches[li], vcaches[li], block_tables, layer.bqkv)
             ctx = ops.paged_attn(q, kcaches[li], vcaches[li], block_tables,
                                  ctx_lens, scale=1.0 / math.sqrt(hd))
             if fp8 is not None:
                 attn = self._allreduce(ops.gemv_fp8(
-                    ctx.reshape(B, nh * hd), *f["wo"])).unsqueeze(1)
+                    ctx.reshape(B, nh * hd), *f["wo"]))
             else:
                 attn = self._allreduce(
-                    ops.linear(ctx.reshape(B, 1, nh * hd), layer.wo))
-            h2, x = ops.norm_fwd_sum(attn, x, layer.post_norm,
-                                     eps=d.rms_norm_eps, rms=True)
+                    parts(ctx.reshape(B, nh * hd), layer.wo))
+            h2, x = ops.norm_parts_sum(attn, x, layer.post_norm,
+                                       eps=d.rms_norm_eps)
             if fp8 is not None:
                 inter = ops.gateup_swiglu_fp8(h2[:, 0], *f["wgup"])
-                down = self._allreduce(
-                    ops.gemv_fp8(inter, *f["wdown"])).unsqueeze(1)
+                down = self._allreduce(ops.gemv_fp8(inter, *f["wdown"]))
             else:
                 down = self._allreduce(
-                    ops.linear(ops.gateup_swiglu(h2, layer.wgup),
-                               layer.wdown))
+                    parts(ops.gateup_swiglu(h2, layer.wgup)[:, 0],
+                          layer.wdown))
             next_w = (self.layers[li + 1].in_norm
                       if li + 1 < len(self.layers) else self.final_norm)
-            h, x = ops.norm_fwd_sum(down, x, next_w,
-                                    eps=d.rms_norm_eps, rms=True)
+            h, x = ops.norm_parts_sum(down, x, next_w, eps=d.rms_norm_eps)
         return self.logits(h[:, 0])

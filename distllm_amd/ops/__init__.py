@@ -50,6 +50,13 @@ def norm_fwd_sum(x, res, w, b=None, eps=1e-5, rms=False):
     return torch_ref.norm_fwd(x, res, w, b, eps, rms, return_sum=True)
 
 
+def norm_parts_sum(x, res, w, eps=1e-5):
+    """norm_fwd_sum (RMS) of what linear_parts returned."""
+    if x.dtype == torch.float32 and x.is_cuda:
+        return _hip_ops.norm_parts(x, res, w, eps)
+    return norm_fwd_sum(x.view(res.shape), res, w, eps=eps, rms=True)
+
+
 def layer_norm(x, w, b, eps=1e-12, res=None):
     return norm_fwd(x, res=res, w=w, b=b, eps=eps, rms=False)
 
@@ -289,6 +296,22 @@ def linear(x, weight, bias=None, act=ACT_NONE):
     else:
         out = _blaslt_path(x2, weight, bias, act)
     return out.reshape(*orig_shape[:-1], N)
+
+
+def linear_parts(x, weight, bias=None):
+    """linear, for a consumer that can sum: where few rows share K among
+    workgroups (17 to 64 rows, csrc/decode_gemm.hip), the fp32 slabs
+    [shares, M, N] without their sum and without the bias, which saves the
+    summing launch; else linear's output [M, N]."""
+    x2 = x.reshape(-1, x.shape[-1])
+    M, K = x2.shape
+    if (x.is_cuda and 0 < M <= 64
+            and os.environ.get("DISTLLM_GEMM", "auto") != "blaslt"):
+        _require_hip("_hip_gemm")
+        if (_few_rows(x2, weight, bias)
+                and _hip_ops.decode_gemm_shares(M, weight.shape[0], K) > 1):
+            return _hip_ops.decode_gemm_parts(x2, weight)
+    return linear(x2, weight, bias)
 
 
 def _silu_gpu(x):
@@ -635,15 +658,18 @@ def cache_put(knew, vnew, kcache, vcache, block_table, slot):
         vcache[blk, :, pos % BLK] = vnew[b]
 
 
-def rope_put(qkv, cs, sn, ctx, kcache, vcache, block_table):
+def rope_put(qkv, cs, sn, ctx, kcache, vcache, block_table, bias=None):
     """A decode step's projections [B, H + 2 HKV, D]: queries and keys are
     rotated by position ctx - 1; queries are returned [B, H, D], keys and
-    values go to that position of the cache, in one launch."""
-    H = qkv.shape[1] - 2 * kcache.shape[1]
-    if qkv.is_cuda and qkv.shape[2] in (64, 128):
+    values go to that position of the cache, in one launch. qkv may be the
+    fp32 slabs [S, B, H + 2 HKV, D] of linear_parts (heads of 64 and 128),
+    with the bias that they lack."""
+    if qkv.is_cuda and qkv.shape[-1] in (64, 128):
         _require_hip()
         return _hip_ops.rope_put(qkv.contiguous(), cs, sn, ctx.int(), kcache,
-                                 vcache, block_table.int())
+                                 vcache, block_table.int(),
+                                 bias if qkv.dim() == 4 else None)
+    H = qkv.shape[1] - 2 * kcache.shape[1]
     slot = (ctx - 1).int()
     qkv = rope_apply(qkv, cs, sn, slot, rope_heads=H + kcache.shape[1])
     cache_put(qkv[:, H: H + kcache.shape[1]].contiguous(),

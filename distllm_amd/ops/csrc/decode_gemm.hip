@@ -432,14 +432,15 @@ static void dg_launch(const u16* X, const u16* W, float* slabs, int K,
   else if (e.M <= 128) DG_TILE(128, 3);
   else DG_TILE(256, 3);
 #undef DG_TILE
-  if (splitk > 1) {
+  if (splitk > 1 && e.out != nullptr) {
     const long four = (long)e.M * (GLU ? e.N / 2 : e.N) / 4;
     hipLaunchKernelGGL(dg_reduce_kernel<ACT>, dim3((four + 255) / 256),
                        dim3(256), 0, st, slabs, splitk, e);
   }
 }
 
-// tile: the tile form whatever M is; splitk workgroups share K there.
+// tile: the tile form whatever M is; splitk workgroups share K there. Without
+// an out the slabs are left for the next kernel to sum.
 extern "C" void launch_decode_gemm(const void* X, const void* W,
                                    const void* bias, void* out, void* slabs,
                                    int M, int N, int K, int splitk, bool tile,

@@ -52,8 +52,10 @@ void launch_sample(const float*, const float*, int*, int, int, float, float,
 void launch_paged_attn(const void*, long, const void*, const void*,
                        const int*, const int*, void*, void*, void*, int, int,
                        int, int, int, int, float, bool, hipStream_t);
-void launch_rope_put(const void*, const float*, const float*, const int*,
-                     void*, void*, void*, const int*, int, int, int, int, int,
+void launch_norm_parts(const float*, int, const void*, const void*, void*,
+                       void*, int, int, float, hipStream_t);
+void launch_rope_put(const void*, const float*, int, const void*,
+                     const float*, const float*, const int*, void*, void*, void*, const int*, int, int, int, int, int,
                      bool, hipStream_t);
 void launch_cache_put(const void*, const void*, void*, void*, const int*,
                       const int*, int, int, int, int, bool, hipStream_t);
@@ -74,6 +76,26 @@ torch::Tensor norm_fwd(torch::Tensor x, c10::optional<torch::Tensor> res,
                   sum_out ? sum_out->data_ptr() : nullptr, (int)n_rows, H,
                   (float)eps, rms, cur_stream());
   return out;
+}
+
+// slabs [S, rows, H] of a product, res [..., H] -> norm of their sum, the sum
+std::vector<torch::Tensor> norm_parts(torch::Tensor parts, torch::Tensor res,
+                                      torch::Tensor w, double eps) {
+  CHECK_DEV(parts); CHECK_CONT(parts); CHECK_F32(parts);
+  CHECK_DEV(res); CHECK_CONT(res); CHECK_BF16(res);
+  CHECK_DEV(w); CHECK_CONT(w); CHECK_BF16(w);
+  TORCH_CHECK(parts.dim() == 3, "parts must be [S, rows, H]");
+  const int S = parts.size(0), rows = parts.size(1), H = parts.size(2);
+  TORCH_CHECK(H % 8 == 0 && H <= 8192, "H must be mult of 8, <= 8192");
+  TORCH_CHECK(res.numel() == (long)rows * H && res.size(-1) == H &&
+                  w.numel() == H,
+              "norm_parts: shape mismatch");
+  auto out = torch::empty_like(res), sum = torch::empty_like(res);
+  if (rows > 0)
+    launch_norm_parts(parts.data_ptr<float>(), S, res.data_ptr(),
+                      w.data_ptr(), out.data_ptr(), sum.data_ptr(), rows, H,
+                      (float)eps, cur_stream());
+  return {out, sum};
 }
 
 // ---- activations ----------------------------------------------------------
@@ -452,21 +474,36 @@ torch::Tensor paged_attn(torch::Tensor q, torch::Tensor kcache,
 
 // qkv [B, H + 2 HKV, D] of a decode step -> rotated q [B, H, D]; rotated keys
 // and the values to their places (position ctx - 1) in the cache
+// qkv [B, H + 2 HKV, D] bf16, or the slabs [S, B, H + 2 HKV, D] fp32 of the
+// product that it would be, and its bias
 torch::Tensor rope_put(torch::Tensor qkv, torch::Tensor cs, torch::Tensor sn,
                        torch::Tensor ctx, torch::Tensor kcache,
-                       torch::Tensor vcache, torch::Tensor block_table) {
-  CHECK_DEV(qkv); CHECK_CONT(qkv); CHECK_BF16(qkv);
+                       torch::Tensor vcache, torch::Tensor block_table,
+                       c10::optional<torch::Tensor> bias) {
+  CHECK_DEV(qkv); CHECK_CONT(qkv);
   CHECK_FLOATS(cs); CHECK_FLOATS(sn);
-  const int B = qkv.size(0), D = qkv.size(2), HKV = kcache.size(1);
-  const int H = (int)qkv.size(1) - 2 * HKV;
+  const bool parts = qkv.scalar_type() == at::kFloat;
+  if (!parts) CHECK_BF16(qkv);
+  TORCH_CHECK(qkv.dim() == 3 + parts, "qkv must be [B, H + 2 HKV, D]");
+  TORCH_CHECK(!bias || parts, "a bias goes with slabs");
+  const int B = qkv.size(parts), D = qkv.size(2 + parts);
+  const int HKV = kcache.size(1), H = (int)qkv.size(1 + parts) - 2 * HKV;
   TORCH_CHECK(D == 64 || D == 128, "head_dim must be 64 or 128");
-  TORCH_CHECK(qkv.dim() == 3 && H > 0, "qkv must be [B, H + 2 HKV, D]");
+  TORCH_CHECK(H > 0, "qkv must be [B, H + 2 HKV, D]");
   TORCH_CHECK(cs.size(-1) == D / 2 && cs.sizes() == sn.sizes(),
               "rotation tables must be [positions, D / 2]");
   check_kv_pages(kcache, vcache, block_table, ctx, B, D);
-  auto q = torch::empty({B, H, D}, qkv.options());
+  if (bias) {
+    CHECK_DEV(bias.value()); CHECK_CONT(bias.value());
+    CHECK_BF16(bias.value());
+    TORCH_CHECK(bias->numel() == (long)(H + 2 * HKV) * D, "bias");
+  }
+  auto q = torch::empty({B, H, D}, qkv.options().dtype(at::kBFloat16));
   if (B > 0)
-    launch_rope_put(qkv.data_ptr(), cs.data_ptr<float>(),
+    launch_rope_put(parts ? nullptr : qkv.data_ptr(),
+                    parts ? qkv.data_ptr<float>() : nullptr,
+                    parts ? (int)qkv.size(0) : 0,
+                    bias ? bias->data_ptr() : nullptr, cs.data_ptr<float>(),
                     sn.data_ptr<float>(), ctx.data_ptr<int>(), q.data_ptr(),
                     kcache.data_ptr(), vcache.data_ptr(),
                     block_table.data_ptr<int>(), B, H, HKV, D,
@@ -570,5 +607,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("sample_tokens", &sample_tokens);
   m.def("paged_attn", &paged_attn);
   m.def("cache_put", &cache_put);
-  m.def("rope_put", &rope_put);
+  m.def("norm_parts", &norm_parts);
+  m.def("rope_put", &rope_put, py::arg("qkv"), py::arg("cs"), py::arg("sn"),
+        py::arg("ctx"), py::arg("kcache"), py::arg("vcache"),
+        py::arg("block_table"), py::arg("bias") = py::none());
 }

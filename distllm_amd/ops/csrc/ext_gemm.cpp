@@ -128,6 +128,24 @@ torch::Tensor decode_gemm(torch::Tensor X, torch::Tensor W,
                          act_nums, nullptr);
 }
 
+// X W^T as the fp32 slabs [shares, M, N] of the workgroups that share K, for
+// kernels that sum them as they read; shares > 1 (decode_gemm_shares).
+torch::Tensor decode_gemm_parts(torch::Tensor X, torch::Tensor W) {
+  CHECK_DEV(X); CHECK_CONT(X); CHECK_BF16(X);
+  CHECK_DEV(W); CHECK_CONT(W); CHECK_BF16(W);
+  const int M = X.size(0), K = X.size(1), N = W.size(0);
+  TORCH_CHECK(W.size(1) == K, "K mismatch");
+  TORCH_CHECK(M > 0 && M <= 256 && N % 64 == 0 && K % 64 == 0, "shape");
+  const int shares = decode_gemm_shares(M, N, K);
+  TORCH_CHECK(shares > 1, "K is not shared at this shape");
+  auto slabs =
+      torch::empty({shares, M, N}, X.options().dtype(at::kFloat));
+  launch_decode_gemm(X.data_ptr(), W.data_ptr(), nullptr, nullptr,
+                     slabs.data_ptr(), M, N, K, shares, false, 0, 0.f, 0.f,
+                     0.f, nullptr, nullptr, cur_stream());
+  return slabs;
+}
+
 static RowsArgs rows_args(const torch::Tensor& tokens,
                           const torch::Tensor& table, long M, int64_t col0,
                           int64_t n, long N) {
@@ -203,6 +221,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("bias"), py::arg("splitk"), py::arg("act") = 0,
         py::arg("limit") = 0.0, py::arg("alpha") = 0.0,
         py::arg("shift") = 0.0, py::arg("act_nums") = py::none());
+  m.def("decode_gemm_parts", &decode_gemm_parts);
+  m.def("decode_gemm_shares", &decode_gemm_shares);
   m.def("decode_gemm_rows", &decode_gemm_rows);
   m.def("gelu_rows", &gelu_rows);
   m.def("clamped_glu", &clamped_glu);

@@ -479,10 +479,15 @@ extern "C" void launch_cache_put(const void* knew, const void* vnew,
 // tables [positions, D / 2]); queries go to q [B, H, D], keys and values to
 // their place in the cache. One launch for what a rotation, three copies and
 // a cache write took (5 launches of 4 us each, in a graph). A thread has
-// columns c .. c + 3 of either half of a head.
+// columns c .. c + 3 of either half of a head. With S > 0 the projections come
+// as the S fp32 slabs of a product whose K was shared, and are summed, given
+// their bias and rounded here: a launch less (product of 6144 x 4096 and this,
+// in a graph, 64 rows 20.8 -> 18.6 us, 17 rows 18.4 -> 15.7).
 template <int D, typename CT>
 __global__ void __launch_bounds__(256)
 rope_put_kernel(const unsigned short* __restrict__ qkv,
+                const float* __restrict__ parts, int S,
+                const unsigned short* __restrict__ bias,
                 const float* __restrict__ cs, const float* __restrict__ sn,
                 const int* __restrict__ ctx, unsigned short* __restrict__ q,
                 CT* __restrict__ kcache, CT* __restrict__ vcache,
@@ -497,8 +502,33 @@ rope_put_kernel(const unsigned short* __restrict__ qkv,
   const int pos = ctx[b] - 1;
   const unsigned short* x = qkv + ((long)b * heads + h) * D + c;
   unsigned short a[4], e[4];
-  *reinterpret_cast<i32x2*>(a) = *reinterpret_cast<const i32x2*>(x);
-  *reinterpret_cast<i32x2*>(e) = *reinterpret_cast<const i32x2*>(x + D / 2);
+  if (S == 0) {
+    *reinterpret_cast<i32x2*>(a) = *reinterpret_cast<const i32x2*>(x);
+    *reinterpret_cast<i32x2*>(e) = *reinterpret_cast<const i32x2*>(x + D / 2);
+  } else {
+    f32x4 va = {0.f, 0.f, 0.f, 0.f}, ve = va;
+    const float* p = parts + ((long)b * heads + h) * D + c;
+#pragma unroll 4
+    for (int s = 0; s < S; ++s) {
+      const f32x4 pa = *reinterpret_cast<const f32x4*>(p);
+      const f32x4 pe = *reinterpret_cast<const f32x4*>(p + D / 2);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        va[j] += pa[j];
+        ve[j] += pe[j];
+      }
+      p += (long)B * heads * D;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (bias != nullptr) {
+        va[j] += bf2f(bias[h * D + c + j]);
+        ve[j] += bf2f(bias[h * D + D / 2 + c + j]);
+      }
+      a[j] = f2bf(va[j]);
+      e[j] = f2bf(ve[j]);
+    }
+  }
   if (h < H + HKV) {
     const f32x4 co = *reinterpret_cast<const f32x4*>(cs + (long)pos * (D / 2) + c);
     const f32x4 si = *reinterpret_cast<const f32x4*>(sn + (long)pos * (D / 2) + c);
@@ -526,7 +556,8 @@ rope_put_kernel(const unsigned short* __restrict__ qkv,
   }
 }
 
-extern "C" void launch_rope_put(const void* qkv, const float* cs,
+extern "C" void launch_rope_put(const void* qkv, const float* parts, int S,
+                                const void* bias, const float* cs,
                                 const float* sn, const int* ctx, void* q,
                                 void* kcache, void* vcache,
                                 const int* block_table, int B, int H, int HKV,
@@ -535,8 +566,9 @@ extern "C" void launch_rope_put(const void* qkv, const float* cs,
   const long total = (long)B * (H + 2 * HKV) * (D / 8);
 #define RP(DD, CT)                                                            \
   hipLaunchKernelGGL((rope_put_kernel<DD, CT>), dim3((total + 255) / 256),    \
-                     dim3(256), 0, stream, (const unsigned short*)qkv, cs,    \
-                     sn, ctx, (unsigned short*)q, (CT*)kcache, (CT*)vcache,   \
+                     dim3(256), 0, stream, (const unsigned short*)qkv, parts, \
+                     S, (const unsigned short*)bias, cs, sn, ctx,             \
+                     (unsigned short*)q, (CT*)kcache, (CT*)vcache,            \
                      block_table, B, H, HKV, max_blocks)
   if (D == 64) {
     if (fp8) RP(64, unsigned char); else RP(64, unsigned short);

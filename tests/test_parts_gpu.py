@@ -1,0 +1,61 @@
+"""Products whose shares of K the next kernel sums: against the summed product
+and the same kernels on it."""
+import pytest
+import torch
+
+from distllm_amd import ops
+
+pytestmark = pytest.mark.gpu
+BF16 = torch.bfloat16
+
+
+def _rand(*shape, seed=0):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    return torch.randn(*shape, device="cuda", generator=g).to(BF16)
+
+
+@pytest.mark.parametrize("M", [1, 16, 17, 33, 64, 65])
+@pytest.mark.parametrize("N, K", [(4096, 14336), (1024, 4096), (8192, 1536),
+                                  (4160, 768)])
+def test_norm(device, M, N, K):
+    x, w, res = _rand(M, K), _rand(N, K, seed=1), _rand(M, 1, N, seed=2)
+    nw = _rand(N, seed=3)
+    got, total = ops.norm_parts_sum(ops.linear_parts(x, w), res, nw)
+    want, sums = ops.norm_fwd_sum(ops.linear(x, w).view_as(res), res, nw,
+                                  rms=True)
+    assert torch.equal(total, sums) and got.shape == res.shape
+    # the squares are summed in another order: the last of bf16's 7 bits
+    torch.testing.assert_close(got, want, rtol=2 ** -7, atol=1e-6)
+
+
+@pytest.mark.parametrize("bias", [False, True])
+@pytest.mark.parametrize("cache", ["bf16", "fp8"])
+@pytest.mark.parametrize("B, H, HKV, D, K", [
+    (1, 32, 8, 128, 4096), (17, 32, 8, 128, 4096), (64, 32, 8, 128, 4096),
+    (40, 3, 1, 64, 8192), (64, 5, 2, 128, 3072)])
+def test_rope_put(device, B, H, HKV, D, K, cache, bias):
+    heads = H + 2 * HKV
+    x, w = _rand(B, K), _rand(heads * D, K, seed=1)
+    b = _rand(heads * D, seed=2) * 30 if bias else None
+    cs, sn = (torch.randn(300, D // 2, device="cuda") for _ in range(2))
+    ctx = torch.randint(1, 300, (B,), device="cuda", dtype=torch.int32)
+    bt = torch.arange(B * 19, dtype=torch.int32, device="cuda").view(B, 19)
+    out = []
+    for f in (ops.linear, ops.linear_parts):
+        kc, vc = (torch.zeros(B * 19, HKV, 16, D, device="cuda", dtype=BF16
+                              if cache == "bf16" else torch.uint8)
+                  for _ in range(2))
+        qkv = f(x, w, b)
+        q = ops.rope_put(qkv.view(*qkv.shape[:-1], heads, D), cs, sn, ctx, kc,
+                         vc, bt, b)
+        out.append((q, kc, vc))
+    assert all(torch.equal(a, c) for a, c in zip(*out))
+    assert out[0][1].any() and out[0][2].any()
+
+
+def test_shares_taken(device):
+    """Slabs where K is shared, the product elsewhere."""
+    w = _rand(4096, 4096)
+    assert ops.linear_parts(_rand(64, 4096), w).dim() == 3
+    assert ops.linear_parts(_rand(16, 4096), w).dim() == 2
+    assert ops.linear_parts(_rand(65, 4096), w).dim() == 2
