@@ -20,6 +20,7 @@ The resulting distllm_amd/ops/_hip_*.so are git-ignored.
 """
 
 import os
+import zlib
 from pathlib import Path
 
 os.environ.setdefault("PYTORCH_ROCM_ARCH", "gfx950")
@@ -62,6 +63,12 @@ names = [n for n in wanted.split(",") if n] or list(GROUPS)
 # feature is off for every kernel.
 HIPCC_FLAGS = ["-O3", "--offload-arch=gfx950", "-std=c++17",
                "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
+# ninja does not see which headers a kernel file includes: a number of their
+# contents in the command makes it build again what is older than a header
+_headers = sorted(p for p in CSRC.glob("*.h")
+                  if not p.name.endswith("_hip.h"))
+HIPCC_FLAGS.append("-DDISTLLM_HEADERS=%d" % zlib.crc32(
+    b"".join(p.read_bytes() for p in _headers)))
 
 setup(
     name="distllm_amd_ops",
