@@ -183,7 +183,7 @@ class Esm2Encoder(nn.Module, _RotaryMixin):
         lens = attention_mask.int().sum(1)
         cu = torch.zeros(B + 1, dtype=torch.int32, device=x.device)
         cu[1:] = lens.cumsum(0)
-        pos = (attention_mask.int().cumsum(1) - 1).clamp(min=0)[maskb]
+        pos = (attention_mask.int().cumsum(1) - 1).clamp(min=0)[maskb].int()
         bmap = ops.varlen_block_map(cu)
         xp = x[maskb]  # [T, H]
         if self.token_dropout:
@@ -323,7 +323,7 @@ class EsmCEncoder(nn.Module, _RotaryMixin):
         lens = attention_mask.int().sum(1)
         cu = torch.zeros(B + 1, dtype=torch.int32, device=x.device)
         cu[1:] = lens.cumsum(0)
-        pos = (attention_mask.int().cumsum(1) - 1).clamp(min=0)[maskb]
+        pos = (attention_mask.int().cumsum(1) - 1).clamp(min=0)[maskb].int()
         bmap = ops.varlen_block_map(cu)
         xp = x[maskb]
         cs, sn = self._rope(x.device)
