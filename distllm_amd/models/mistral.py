@@ -294,37 +294,39 @@ class DecoderModel(nn.Module):
                and x.is_cuda else None)
         # products whose shares of K the next kernel sums (on one rank)
         parts = ops.linear_parts if self.tp == 1 else ops.linear
-        h = ops.rms_norm(x, self.layers[0].in_norm, eps=d.rms_norm_eps)
+        eps = d.rms_norm_eps
+        down = None
         for li, layer in enumerate(self.layers):
-            # ONE fused qkv GEMM + ONE launch that rotates q and k and
-            # writes k and v to their pages
-            if fp8 is not None:
-                f = fp8[li]
-                qkv = ops.gemv_fp8(h[:, 0], *f["wqkv"], layer.bqkv)
+            # norm and ONE fused qkv GEMM (one launch for one sequence), ONE
+            # launch that rotates q and k and writes k and v to their pages
+            f = fp8[li] if fp8 is not None else None
+            if down is None:
+                h = ops.rms_norm(x, layer.in_norm, eps=eps)[:, 0]
+                qkv = (ops.gemv_fp8(h, *f["wqkv"], layer.bqkv)
+                       if f is not None
+                       else ops.linear(h, layer.wqkv, layer.bqkv))
+            elif f is not None:
+                qkv, x = ops.norm_linear_fp8(down, x, layer.in_norm, eps,
+                                             *f["wqkv"], layer.bqkv)
             else:
-                qkv = (parts if hd in (64, 128) else ops.linear)(
-                    h[:, 0], layer.wqkv, layer.bqkv)
+                qkv, x = ops.norm_linear(down, x, layer.in_norm, eps,
+                                         layer.wqkv, layer.bqkv,
+                                         shares=hd in (64, 128))
             q = ops.rope_put(
                 qkv.view(*qkv.shape[:-1], nh + 2 * kvh, hd), cs, sn,
                 ctx_lens, kcaches[li], vcaches[li], block_tables, layer.bqkv)
             ctx = ops.paged_attn(q, kcaches[li], vcaches[li], block_tables,
                                  ctx_lens, scale=1.0 / math.sqrt(hd))
-            if fp8 is not None:
-                attn = self._allreduce(ops.gemv_fp8(
-                    ctx.reshape(B, nh * hd), *f["wo"]))
-            else:
-                attn = self._allreduce(
-                    parts(ctx.reshape(B, nh * hd), layer.wo))
-            h2, x = ops.norm_parts_sum(attn, x, layer.post_norm,
-                                       eps=d.rms_norm_eps)
-            if fp8 is not None:
-                inter = ops.gateup_swiglu_fp8(h2[:, 0], *f["wgup"])
+            ctx = ctx.reshape(B, nh * hd)
+            if f is not None:
+                attn = self._allreduce(ops.gemv_fp8(ctx, *f["wo"]))
+                inter, x = ops.norm_linear_fp8(attn, x, layer.post_norm, eps,
+                                               *f["wgup"], gated=True)
                 down = self._allreduce(ops.gemv_fp8(inter, *f["wdown"]))
             else:
-                down = self._allreduce(
-                    parts(ops.gateup_swiglu(h2, layer.wgup)[:, 0],
-                          layer.wdown))
-            next_w = (self.layers[li + 1].in_norm
-                      if li + 1 < len(self.layers) else self.final_norm)
-            h, x = ops.norm_parts_sum(down, x, next_w, eps=d.rms_norm_eps)
+                attn = self._allreduce(parts(ctx, layer.wo))
+                inter, x = ops.norm_linear(attn, x, layer.post_norm, eps,
+                                           layer.wgup, gated=True)
+                down = self._allreduce(parts(inter, layer.wdown))
+        h, x = ops.norm_parts_sum(down, x, self.final_norm, eps=eps)
         return self.logits(h[:, 0])

@@ -314,6 +314,56 @@ def linear_parts(x, weight, bias=None):
     return linear(x2, weight, bias)
 
 
+def _norm_in_product(a, b, w_norm, weight, least):
+    """Whether a + b is one row whose norm the product of it with `weight`
+    takes into its launch (csrc/norm_row.h): up to 8192 columns, at least
+    `least`, so that every wave has five chunks. Two rows already cost every
+    workgroup more than the launch saves."""
+    K = weight.shape[1]
+    return (a.is_cuda and a.numel() == b.numel() == K
+            and a.shape[-1] == b.shape[-1] == K
+            and least <= K <= 8192
+            and a.dtype == b.dtype == w_norm.dtype == torch.bfloat16
+            and all(t.is_contiguous() and t.data_ptr() % 16 == 0
+                    for t in (a, b, w_norm, weight)))
+
+
+def norm_linear(a, b, w_norm, eps, weight, bias=None, gated=False,
+                shares=False):
+    """x = a + b, and the linear (or, gated, the SwiGLU of the packed gate and
+    up rows) of its RMS norm times w_norm -> (linear [M, N], x like b); a may
+    be what linear_parts returned, and with `shares` the linear is of that
+    kind. One row is one launch."""
+    N = weight.shape[0]
+    if (os.environ.get("DISTLLM_GEMM", "auto") != "blaslt"
+            and weight.dtype == torch.bfloat16 and weight.shape[1] % 64 == 0
+            and N % (128 if gated else 64) == 0
+            and (bias is None or (bias.dtype == torch.bfloat16
+                                  and bias.is_contiguous()))
+            and _norm_in_product(a, b, w_norm, weight, 1280)):
+        _require_hip("_hip_gemm")
+        return tuple(_hip_ops.norm_gemm(a, b, w_norm, eps, weight, bias,
+                                        int(gated)))
+    h, x = norm_parts_sum(a, b, w_norm, eps=eps)
+    h = h.reshape(-1, h.shape[-1])
+    if gated:
+        return gateup_swiglu(h, weight, bias), x
+    return (linear_parts if shares else linear)(h, weight, bias), x
+
+
+def norm_linear_fp8(a, b, w_norm, eps, wq, scale, bias=None, gated=False):
+    """norm_linear on weights quantized as for gemv_fp8."""
+    if wq.shape[1] % 128 == 0 and _norm_in_product(a, b, w_norm, wq, 2560):
+        _require_hip()
+        return tuple(_hip_ops.gemv_fp8_norm(a, b, w_norm, eps, wq, scale,
+                                            bias, gated))
+    h, x = norm_parts_sum(a, b, w_norm, eps=eps)
+    h = h.reshape(-1, h.shape[-1])
+    if gated:
+        return gateup_swiglu_fp8(h, wq, scale), x
+    return gemv_fp8(h, wq, scale, bias), x
+
+
 def _silu_gpu(x):
     # standalone silu via the swiglu kernel with up=1 is wasteful; use a
     # dedicated path: silu(x) = swiglu(x, ones) avoided — bias_gelu

@@ -64,7 +64,9 @@ __device__ __forceinline__ void wave_sync() {
 // wait for every copy that it knows to be in flight, also those into other
 // buffers. So nothing waits by itself, __syncthreads() neither: the caller
 // counts its copies and waits (s_waitcnt vmcnt) before a barrier or a read of
-// the bytes.
+// the bytes. M0 is a register that the compiler keeps to itself and does not
+// save around assembly: nothing else in the kernels that use this needs it (no
+// copies by the builtin beside these).
 template <int BYTES = 16>
 __device__ __forceinline__ void copy_to_lds(const void* src,
                                             const void* base) {

@@ -34,6 +34,7 @@
 // with the row, on the source address of the copies.
 #include "common.h"
 #include "gelu_rows.h"
+#include "norm_row.h"
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef unsigned short u16;
@@ -228,6 +229,111 @@ dg_ring_kernel(const u16* __restrict__ X, const u16* __restrict__ W, int K,
   }
   __syncthreads();
   dg_join<ACT, MT, NT, NW, NT * MT>(e, n0, wid * NT * MT, &acc[0][0]);
+}
+
+// ---- ring with the norm ahead of the product --------------------------------
+// One row (norm_row.h). The normed row stays in LDS, so that the rings hold
+// weights only: more of them. Measured in a graph, us, norm and product in two
+// launches and in one: 28672 x 4096 gated 44.6 and 41.8, 6144 x 4096 13.3 and
+// 10.8, 4096 x 2048 7.9 and 7.0; two rows normed by every workgroup 46.5 and
+// 49.1 at the first.
+constexpr int dg_norm_lds(int K, int NT, int R) {
+  return 128 + K * 2 + 4 * R * NT * 2048;
+}
+// chunks that every wave has at least: R - 1 are started ahead of the norm
+constexpr int dg_norm_ring(int NT) { return NT == 2 ? 4 : 6; }
+
+template <int ACT, int NT, int NC>
+__global__ void __launch_bounds__(256)
+dg_norm_ring_kernel(const NormRow n, const u16* __restrict__ W, int K,
+                    const DgEnd e) {
+  constexpr bool GLU = dg_glu(ACT);
+  constexpr int NW = 4, R = dg_norm_ring(NT);
+  constexpr int STAGE = NT * 2048, LOADS = NT * 2;
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  const int r = lane & 15, g = lane >> 4;
+  const int n0 = blockIdx.x * (GLU ? NT * 8 : NT * 16);
+  char* hs = smem + 128;
+  char* ring = hs + K * 2 + wid * R * STAGE;
+  const int lr = lane >> 3, lc = ((lane & 7) ^ lr) * 8;
+  const u16* src[NT][2];
+#pragma unroll
+  for (int p = 0; p < 2; ++p)
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+      src[t][p] = W + (long)(dg_wrow<GLU>(n0, t, e.N) + p * 8 + lr) * K +
+                  wid * 64 + lc;
+  const int mine = (K / 64 - wid + NW - 1) / NW;  // chunks wid, wid + NW, ...
+  auto issue = [&](int c) {
+    char* dst = ring + (c % R) * STAGE + lane * 16;
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int p = 0; p < 2; ++p)
+        dg_copy(src[t][p] + (long)c * (NW * 64), dst + t * 2048 + p * 1024);
+  };
+  norm_row<NC>(n, K, reinterpret_cast<float*>(smem), hs, [&]() {
+#pragma unroll
+    for (int c = 0; c < R - 1; ++c) issue(c);
+  });
+
+  f32x4 acc[NT];
+#pragma unroll
+  for (int i = 0; i < NT; ++i) acc[i] = {0.f, 0.f, 0.f, 0.f};
+  auto compute = [&](int c) {
+    const char* b = ring + (c % R) * STAGE;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const bf16x8 x = *reinterpret_cast<const bf16x8*>(
+          hs + (c * NW + wid) * 128 + (h * 4 + g) * 16);
+#pragma unroll
+      for (int i = 0; i < NT; ++i)
+        acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            *reinterpret_cast<const bf16x8*>(
+                b + i * 2048 + r * 128 + (((h * 4 + g) ^ (r & 7)) * 16)),
+            x, acc[i], 0, 0, 0);
+    }
+    // the buffer is read before the wave fills it again
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  };
+  int c = 0;
+  for (; c + R - 1 < mine; ++c) {
+    issue(c + R - 1);
+    dg_wait<(R - 1) * LOADS>();
+    compute(c);
+  }
+  dg_wait<0>();
+  for (; c < mine; ++c) compute(c);
+  __syncthreads();
+  dg_join<ACT, 1, NT, NW, NT>(e, n0, wid * NT, acc);
+}
+
+template <int ACT>
+static void dg_norm_launch(const NormRow& n, const u16* W, int K,
+                           const DgEnd& e, hipStream_t st) {
+  constexpr int NT = dg_glu(ACT) ? 2 : 1;
+#define DG_NR(NC)                                                          \
+  hipLaunchKernelGGL((dg_norm_ring_kernel<ACT, NT, NC>),                   \
+                     dim3(e.N / (NT * 16)), dim3(256),                     \
+                     dg_norm_lds(K, NT, dg_norm_ring(NT)), st, n, W, K, e)
+  if (K <= 2048) DG_NR(1);
+  else if (K <= 4096) DG_NR(2);
+  else DG_NR(4);  // up to 8192
+#undef DG_NR
+}
+
+// act 0 or 1: product or gated unit (SwiGLU) of the norm of one row. K from
+// 1280 (five chunks of 64 for each of four waves) to 8192.
+extern "C" void launch_norm_gemm(const void* a, const void* b,
+                                 const void* w_norm, void* sum, float eps,
+                                 const void* W, const void* bias, void* out,
+                                 int N, int K, int act, hipStream_t stream) {
+  const NormRow n = {(const u16*)a, (const u16*)b, (const u16*)w_norm,
+                     (u16*)sum, eps};
+  const DgEnd e = {(const u16*)bias, (u16*)out, 1, N, 0.f, 0.f, 0.f, nullptr,
+                   {}};
+  if (act == 1) dg_norm_launch<DG_SWIGLU>(n, (const u16*)W, K, e, stream);
+  else dg_norm_launch<DG_NONE>(n, (const u16*)W, K, e, stream);
 }
 
 // ---- tile -------------------------------------------------------------------

@@ -47,6 +47,9 @@ void launch_ivf_score(const void*, const int*, const int*, const float*,
                       float*, int, int, int, int, hipStream_t);
 void launch_gemv_fp8(const void*, const void*, const float*, const void*,
                      void*, int, int, long, bool, hipStream_t);
+void launch_gemv_fp8_norm(const void*, const void*, const void*, void*, float,
+                          const void*, const float*, const void*, void*, int,
+                          int, bool, hipStream_t);
 void launch_sample(const float*, const float*, int*, int, int, float, float,
                    hipStream_t);
 void launch_paged_attn(const void*, long, const void*, const void*,
@@ -55,8 +58,9 @@ void launch_paged_attn(const void*, long, const void*, const void*,
 void launch_norm_parts(const float*, int, const void*, const void*, void*,
                        void*, int, int, float, hipStream_t);
 void launch_rope_put(const void*, const float*, int, const void*,
-                     const float*, const float*, const int*, void*, void*, void*, const int*, int, int, int, int, int,
-                     bool, hipStream_t);
+                     const float*, const float*, const int*, void*, void*,
+                     void*, const int*, int, int, int, int, int, bool,
+                     hipStream_t);
 void launch_cache_put(const void*, const void*, void*, void*, const int*,
                       const int*, int, int, int, int, bool, hipStream_t);
 }
@@ -572,6 +576,43 @@ torch::Tensor gemv_fp8(torch::Tensor x, torch::Tensor wq,
   return out;
 }
 
+// x = a + b, one row, and the quantized product of its RMS norm
+std::vector<torch::Tensor> gemv_fp8_norm(torch::Tensor a, torch::Tensor b,
+                                         torch::Tensor w_norm, double eps,
+                                         torch::Tensor wq,
+                                         torch::Tensor scale,
+                                         c10::optional<torch::Tensor> bias,
+                                         bool swiglu) {
+  for (const auto& t : {a, b, w_norm}) {
+    CHECK_DEV(t); CHECK_CONT(t); CHECK_BF16(t);
+    TORCH_CHECK((uintptr_t)t.data_ptr() % 16 == 0, "16-byte alignment");
+  }
+  CHECK_DEV(wq); CHECK_CONT(wq);
+  TORCH_CHECK(wq.scalar_type() == at::kByte && wq.dim() == 2 &&
+                  (uintptr_t)wq.data_ptr() % 16 == 0,
+              "wq must be uint8 (fp8)");
+  CHECK_DEV(scale); CHECK_CONT(scale); CHECK_F32(scale);
+  const int N = wq.size(0), K = wq.size(1);
+  TORCH_CHECK(K % 128 == 0 && K >= 2560 && K <= 8192 && a.numel() == K &&
+                  b.numel() == K && w_norm.numel() == K,
+              "gemv_fp8_norm: one row of 2560 to 8192 numbers");
+  TORCH_CHECK(scale.numel() == N && N > 0 && (!swiglu || N % 2 == 0),
+              "scale must be per output channel");
+  if (bias) {
+    CHECK_DEV(bias.value()); CHECK_CONT(bias.value());
+    CHECK_BF16(bias.value());
+    TORCH_CHECK(bias->numel() == N, "bias");
+  }
+  auto out = torch::empty({1, swiglu ? N / 2 : N}, a.options());
+  auto sum = torch::empty_like(b);
+  launch_gemv_fp8_norm(a.data_ptr(), b.data_ptr(), w_norm.data_ptr(),
+                       sum.data_ptr(), (float)eps, wq.data_ptr(),
+                       scale.data_ptr<float>(),
+                       bias ? bias->data_ptr() : nullptr, out.data_ptr(), N,
+                       K, swiglu, cur_stream());
+  return {out, sum};
+}
+
 // encoder_layers.cpp
 torch::Tensor bert_few_rows(torch::Tensor x, torch::Tensor mask,
                             std::vector<torch::Tensor> layers, int64_t heads,
@@ -604,6 +645,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gemv_fp8", &gemv_fp8, py::arg("x"), py::arg("wq"),
         py::arg("scale"), py::arg("bias") = py::none(),
         py::arg("swiglu") = false);
+  m.def("gemv_fp8_norm", &gemv_fp8_norm);
   m.def("sample_tokens", &sample_tokens);
   m.def("paged_attn", &paged_attn);
   m.def("cache_put", &cache_put);

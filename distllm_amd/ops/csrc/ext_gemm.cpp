@@ -15,6 +15,9 @@ void launch_decode_gemm(const void*, const void*, const void*, void*, void*,
                         int, int, int, int, bool, int, float, float, float,
                         const float*, const RowsArgs*, hipStream_t);
 int decode_gemm_shares(int, int, int);
+void launch_norm_gemm(const void*, const void*, const void*, void*, float,
+                      const void*, const void*, void*, int, int, int,
+                      hipStream_t);
 void launch_clamped_glu(const void*, void*, long, int, float, float, float,
                         bool, hipStream_t);
 void launch_relu2(const void*, void*, long, bool, hipStream_t);
@@ -146,6 +149,37 @@ torch::Tensor decode_gemm_parts(torch::Tensor X, torch::Tensor W) {
   return slabs;
 }
 
+// x = a + b, one row, and the product of its RMS norm (act 1: gated unit)
+std::vector<torch::Tensor> norm_gemm(torch::Tensor a, torch::Tensor b,
+                                     torch::Tensor w_norm, double eps,
+                                     torch::Tensor W,
+                                     c10::optional<torch::Tensor> bias,
+                                     int64_t act) {
+  for (const auto& t : {a, b, w_norm, W}) {
+    CHECK_DEV(t); CHECK_CONT(t); CHECK_BF16(t);
+    TORCH_CHECK((uintptr_t)t.data_ptr() % 16 == 0, "16-byte alignment");
+  }
+  TORCH_CHECK(W.dim() == 2, "W");
+  const int K = W.size(1), N = W.size(0);
+  TORCH_CHECK(K % 64 == 0 && K >= 1280 && K <= 8192 && a.numel() == K &&
+                  b.numel() == K && w_norm.numel() == K,
+              "norm_gemm: one row of 1280 to 8192 numbers");
+  TORCH_CHECK(act == 0 || act == 1, "activation");
+  TORCH_CHECK(N > 0 && N % (act ? 128 : 64) == 0, "columns");
+  if (bias) {
+    CHECK_DEV(bias.value()); CHECK_CONT(bias.value());
+    CHECK_BF16(bias.value());
+    TORCH_CHECK(bias->numel() == N, "bias");
+  }
+  auto out = torch::empty({1, act ? N / 2 : N}, a.options());
+  auto sum = torch::empty_like(b);
+  launch_norm_gemm(a.data_ptr(), b.data_ptr(), w_norm.data_ptr(),
+                   sum.data_ptr(), (float)eps, W.data_ptr(),
+                   bias ? bias->data_ptr() : nullptr, out.data_ptr(), N, K,
+                   (int)act, cur_stream());
+  return {out, sum};
+}
+
 static RowsArgs rows_args(const torch::Tensor& tokens,
                           const torch::Tensor& table, long M, int64_t col0,
                           int64_t n, long N) {
@@ -221,6 +255,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("bias"), py::arg("splitk"), py::arg("act") = 0,
         py::arg("limit") = 0.0, py::arg("alpha") = 0.0,
         py::arg("shift") = 0.0, py::arg("act_nums") = py::none());
+  m.def("norm_gemm", &norm_gemm);
   m.def("decode_gemm_parts", &decode_gemm_parts);
   m.def("decode_gemm_shares", &decode_gemm_shares);
   m.def("decode_gemm_rows", &decode_gemm_rows);

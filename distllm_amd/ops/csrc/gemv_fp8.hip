@@ -20,7 +20,7 @@
 // (distllm/generate/generators/vllm_backend.py:62-93).
 #include <hip/hip_fp8.h>
 
-#include "common.h"
+#include "norm_row.h"
 
 #define GV_MAXM 8
 
@@ -207,6 +207,134 @@ gemv_fp8_ring_kernel(const unsigned short* __restrict__ X,
     if (bias != nullptr) v[t] += bf2f(bias[n0 + n + t * cols]);
   }
   OUT[(long)m * cols + n0 + n] = f2bf(GLU ? silu(v[0]) * v[NT - 1] : v[0]);
+}
+
+// One row with its residual sum and norm ahead (norm_row.h). The normed row
+// stays in LDS, the rings hold weights only. In a graph, us, in two launches
+// and in one: 28672 x 4096 gated 27.5 and 25.5, 6144 x 4096 10.7 and 8.7.
+constexpr int gv_norm_ring(bool glu) { return glu ? 4 : 6; }
+constexpr int gv_norm_lds(bool glu, int K) {
+  return 128 + K * 2 + 4 * gv_norm_ring(glu) * (glu ? 4096 : 2048);
+}
+
+template <bool GLU, int NC>
+__global__ void __launch_bounds__(256)
+gemv_fp8_norm_kernel(const NormRow nr, const unsigned char* __restrict__ W,
+                     const float* __restrict__ scale,
+                     const unsigned short* __restrict__ bias,
+                     unsigned short* __restrict__ OUT, int N, int K) {
+  constexpr int NT = GLU ? 2 : 1, R = gv_norm_ring(GLU);
+  constexpr int STAGE = NT * 2048, LOADS = NT * 2;
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  const int r = lane & 15, g = lane >> 4;
+  const int cols = GLU ? N / 2 : N, n0 = blockIdx.x * 16;
+  char* hs = smem + 128;
+  char* ring = hs + K * 2 + wid * R * STAGE;
+  const int mine = (K / 128 - wid + 3) / 4;  // chunks wid, wid + 4, ...
+  const unsigned char* src[NT][2];
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {
+    const int row = p * 8 + (lane >> 3);
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+      src[t][p] = W + (long)(min(n0 + row, cols - 1) + t * cols) * K +
+                  wid * 128 + ((lane & 7) ^ (row & 7)) * 16;
+  }
+  auto issue = [&](int c) {
+    char* dst = ring + (c % R) * STAGE + lane * 16;
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int p = 0; p < 2; ++p)
+        __builtin_amdgcn_global_load_lds(
+            (const __attribute__((address_space(1))) unsigned int*)(
+                src[t][p] + (long)c * 512),
+            (__attribute__((address_space(3))) unsigned int*)(
+                dst + (t * 2 + p) * 1024),
+            16, 0, 0);
+  };
+  norm_row<NC>(nr, K, reinterpret_cast<float*>(smem), hs, [&]() {
+#pragma unroll
+    for (int c = 0; c < R - 1; ++c) issue(c);
+  });
+  f32x4 acc[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) acc[t] = {0.f, 0.f, 0.f, 0.f};
+  auto compute = [&](int c) {
+    const char* b = ring + (c % R) * STAGE;
+    const char* xb = hs + (c * 4 + wid) * 256;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      bf16x8 x[2];
+#pragma unroll
+      for (int e = 0; e < 2; ++e)
+        x[e] = *reinterpret_cast<const bf16x8*>(xb +
+                                                (j * 8 + g * 2 + e) * 16);
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        const i32x4 w = *reinterpret_cast<const i32x4*>(
+            b + t * 2048 + r * 128 + (((j * 4 + g) ^ (r & 7)) * 16));
+        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            gv_widen(w[0], w[1]), x[0], acc[t], 0, 0, 0);
+        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            gv_widen(w[2], w[3]), x[1], acc[t], 0, 0, 0);
+      }
+    }
+    // the buffer is read before the wave fills it again
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  };
+  int c = 0;
+  for (; c + R - 1 < mine; ++c) {
+    issue(c + R - 1);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"i"((R - 1) * LOADS) : "memory");
+    compute(c);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  for (; c < mine; ++c) compute(c);
+  __syncthreads();
+  float* red = reinterpret_cast<float*>(smem);  // [4][NT][256]
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+    *reinterpret_cast<f32x4*>(red + (wid * NT + t) * 256 + lane * 4) = acc[t];
+  __syncthreads();
+  const int n = threadIdx.x;  // column n0 + n
+  if (n >= 16 || n0 + n >= cols) return;
+  float v[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    v[t] = 0.f;
+#pragma unroll
+    for (int w = 0; w < 4; ++w)
+      v[t] += red[(w * NT + t) * 256 + (n >> 2) * 64 + (n & 3)];
+    v[t] *= scale[n0 + n + t * cols];
+    if (bias != nullptr) v[t] += bf2f(bias[n0 + n + t * cols]);
+  }
+  OUT[n0 + n] = f2bf(GLU ? silu(v[0]) * v[NT - 1] : v[0]);
+}
+
+// K % 128 == 0 from 2560 (five chunks of 128 for each of four waves) to 8192
+extern "C" void launch_gemv_fp8_norm(const void* a, const void* b,
+                                     const void* w_norm, void* sum, float eps,
+                                     const void* W, const float* scale,
+                                     const void* bias, void* out, int N,
+                                     int K, bool glu, hipStream_t stream) {
+  const NormRow n = {(const unsigned short*)a, (const unsigned short*)b,
+                     (const unsigned short*)w_norm, (unsigned short*)sum,
+                     eps};
+#define GVN(G, NC)                                                          \
+  hipLaunchKernelGGL((gemv_fp8_norm_kernel<G, NC>),                         \
+                     dim3(((G ? N / 2 : N) + 15) / 16), dim3(256),          \
+                     gv_norm_lds(G, K), stream, n, (const unsigned char*)W, \
+                     scale, (const unsigned short*)bias,                    \
+                     (unsigned short*)out, N, K)
+  if (K <= 4096) {
+    if (glu) GVN(true, 2);
+    else GVN(false, 2);
+  } else {
+    if (glu) GVN(true, 4);
+    else GVN(false, 4);
+  }
+#undef GVN
 }
 
 // glu: W holds gate rows, then up rows; out [M, N / 2]. Needs K % 128 == 0.

@@ -59,3 +59,40 @@ def test_shares_taken(device):
     assert ops.linear_parts(_rand(64, 4096), w).dim() == 3
     assert ops.linear_parts(_rand(16, 4096), w).dim() == 2
     assert ops.linear_parts(_rand(65, 4096), w).dim() == 2
+
+
+@pytest.mark.parametrize("rows", [1, 2])
+@pytest.mark.parametrize("gated", [False, True])
+@pytest.mark.parametrize("N, K", [(128, 1280), (1152, 1344), (256, 2048),
+                                  (384, 2560), (6144, 4096), (128, 4160),
+                                  (256, 8192), (128, 1216)])
+def test_norm_linear(device, rows, gated, N, K):
+    """Norm and product in one launch, bit for bit as in two, at the ends of
+    its range and outside."""
+    a, b = _rand(rows, K), _rand(rows, 1, K, seed=1)
+    w, nw = _rand(N, K, seed=2), _rand(K, seed=3)
+    bias = None if gated else _rand(N, seed=4) * 9
+    got, x = ops.norm_linear(a, b, nw, 1e-5, w, bias, gated)
+    h, want_x = ops.norm_fwd_sum(a.view_as(b), b, nw, rms=True)
+    want = (ops.gateup_swiglu(h[:, 0], w) if gated
+            else ops.linear(h[:, 0], w, bias))
+    assert torch.equal(x, want_x) and torch.equal(got, want)
+
+
+@pytest.mark.parametrize("rows", [1, 2])
+@pytest.mark.parametrize("gated", [False, True])
+@pytest.mark.parametrize("N, K", [(32, 2560), (1040, 2688), (6144, 4096),
+                                  (24, 4224), (256, 8192), (64, 2432),
+                                  (64, 2576)])
+def test_norm_linear_fp8(device, rows, gated, N, K):
+    if gated and K % 128:
+        N = 64  # the gated unit of other K is a kernel of its own
+    a, b = _rand(rows, K), _rand(rows, 1, K, seed=1)
+    nw, scale = _rand(K, seed=3), torch.rand(N, device="cuda") + 0.1
+    w = _rand(N, K, seed=2).to(torch.float8_e4m3fn).view(torch.uint8)
+    bias = None if gated else _rand(N, seed=4) * 9
+    got, x = ops.norm_linear_fp8(a, b, nw, 1e-5, w, scale, bias, gated)
+    h, want_x = ops.norm_fwd_sum(a.view_as(b), b, nw, rms=True)
+    want = (ops.gateup_swiglu_fp8(h[:, 0], w, scale) if gated
+            else ops.gemv_fp8(h[:, 0], w, scale, bias))
+    assert torch.equal(x, want_x) and torch.equal(got, want)
