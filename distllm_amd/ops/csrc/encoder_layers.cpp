@@ -48,6 +48,7 @@ torch::Tensor bert_few_rows(torch::Tensor x, torch::Tensor mask,
                     t.size(0) == rows[k] && t.dim() == (cols[k] ? 2 : 1) &&
                     (cols[k] == 0 || t.size(1) == cols[k]),
                 "layer tensor ", k, " of layer ", i / 12);
+    if (cols[k]) layers[i] = aligned16(t);
   }
   auto some = [&](long n) { return torch::empty({M, n}, x.options()); };
   auto qkv = some(3 * H), ctx = some(H), y = some(H), a = some(H),
@@ -73,7 +74,7 @@ torch::Tensor bert_few_rows(torch::Tensor x, torch::Tensor mask,
                     out.data_ptr(), nullptr, M, H, (float)eps, false, st);
   };
   const long row = 3L * H;
-  torch::Tensor in = x;
+  torch::Tensor in = aligned16(x);
   for (size_t i = 0; i < layers.size(); i += 12) {
     const torch::Tensor* p = &layers[i];
     gemm(in, p[0], p[1], qkv, 0);

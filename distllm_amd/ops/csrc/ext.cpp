@@ -453,6 +453,9 @@ torch::Tensor paged_attn(torch::Tensor q, torch::Tensor kcache,
   const bool fp8 = kcache.scalar_type() == at::kByte;
   auto out = torch::empty_like(q);
   if (B == 0) return out;
+  q = aligned16(q);
+  kcache = aligned16(kcache);
+  vcache = aligned16(vcache);
   // Workgroups that share a sequence: as many as make two for every CU, each
   // with at least 256 of the positions that the block table has room for. In
   // us, 1, 2, 4, 8, 16 shares: B = 1 of 2048 25, 18, 13, 11.2, 11.9; B = 8 of
@@ -476,10 +479,9 @@ torch::Tensor paged_attn(torch::Tensor q, torch::Tensor kcache,
   return out;
 }
 
-// qkv [B, H + 2 HKV, D] of a decode step -> rotated q [B, H, D]; rotated keys
-// and the values to their places (position ctx - 1) in the cache
-// qkv [B, H + 2 HKV, D] bf16, or the slabs [S, B, H + 2 HKV, D] fp32 of the
-// product that it would be, and its bias
+// qkv [B, H + 2 HKV, D] of a decode step (or the slabs [S, B, H + 2 HKV, D]
+// fp32 of the product that it would be, and its bias) -> rotated q [B, H, D];
+// rotated keys and the values to their places (position ctx - 1) in the cache
 torch::Tensor rope_put(torch::Tensor qkv, torch::Tensor cs, torch::Tensor sn,
                        torch::Tensor ctx, torch::Tensor kcache,
                        torch::Tensor vcache, torch::Tensor block_table,
@@ -570,6 +572,8 @@ torch::Tensor gemv_fp8(torch::Tensor x, torch::Tensor wq,
   TORCH_CHECK(!swiglu || (N % 2 == 0 && K % 128 == 0),
               "swiglu needs two halves and K % 128 == 0");
   auto out = torch::empty({M, swiglu ? N / 2 : N}, x.options());
+  x = aligned16(x);
+  wq = aligned16(wq);
   launch_gemv_fp8(x.data_ptr(), wq.data_ptr(),
                   scale.data_ptr<float>(), bptr, out.data_ptr(), M, N,
                   K, swiglu, cur_stream());

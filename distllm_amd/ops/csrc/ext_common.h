@@ -44,3 +44,9 @@ static inline int row_stride(const torch::Tensor& t) {
   TORCH_CHECK(t.dim() == 2 && t.stride(1) == 1, "rows must be contiguous");
   return (int)t.stride(0);
 }
+
+// A contiguous operand of kernels that copy 16 bytes a lane to LDS, which asks
+// for their alignment: itself, or a copy where its storage starts elsewhere.
+static inline torch::Tensor aligned16(const torch::Tensor& t) {
+  return (uintptr_t)t.data_ptr() % 16 ? t.clone() : t;
+}

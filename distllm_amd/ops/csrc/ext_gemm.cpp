@@ -105,6 +105,8 @@ static torch::Tensor decode_gemm_act(torch::Tensor X, torch::Tensor W,
   }
   auto out = torch::empty({M, glu ? N / 2 : N}, X.options());
   if (M == 0) return out;
+  X = aligned16(X);
+  W = aligned16(W);
   torch::Tensor slabs;
   void* slabp = nullptr;
   if (splitk > 1) {
@@ -141,6 +143,8 @@ torch::Tensor decode_gemm_parts(torch::Tensor X, torch::Tensor W) {
   TORCH_CHECK(M > 0 && M <= 256 && N % 64 == 0 && K % 64 == 0, "shape");
   const int shares = decode_gemm_shares(M, N, K);
   TORCH_CHECK(shares > 1, "K is not shared at this shape");
+  X = aligned16(X);
+  W = aligned16(W);
   auto slabs =
       torch::empty({shares, M, N}, X.options().dtype(at::kFloat));
   launch_decode_gemm(X.data_ptr(), W.data_ptr(), nullptr, nullptr,

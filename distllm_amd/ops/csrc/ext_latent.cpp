@@ -226,6 +226,8 @@ torch::Tensor latent_attn(torch::Tensor q, torch::Tensor cache,
                             e.ld_gate, is_f32(q), cur_stream());
     return out;
   }
+  q = aligned16(q);
+  cache = aligned16(cache);
   // Split each row's keys until the 256 CUs have a workgroup each (its
   // buffers take a CU's LDS; more than fit would be a second round), as long
   // as a share keeps two tiles of 64 keys; four tiles are not worth the second

@@ -1,0 +1,54 @@
+"""Operands whose storage does not start at a multiple of 16 bytes, for the
+kernels that copy whole pieces to LDS: the same numbers as from aligned ones."""
+import pytest
+import torch
+
+from distllm_amd import ops
+from distllm_amd.ops import _hip_ops
+
+pytestmark = pytest.mark.gpu
+BF16 = torch.bfloat16
+
+
+def _off(t):
+    """t in storage that starts one element late."""
+    flat = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)
+    flat[1:] = t.flatten()
+    return flat[1:].view(t.shape)
+
+
+def _rand(*shape, seed=0):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    return torch.randn(*shape, device="cuda", generator=g).to(BF16)
+
+
+def _same(f, *args):
+    want = f(*args)
+    for i in range(len(args)):
+        got = f(*[_off(a) if i == j else a for j, a in enumerate(args)])
+        assert torch.equal(got, want), i
+
+
+def test_paged_attn(device):
+    bt = torch.arange(12, dtype=torch.int32, device="cuda").view(2, 6)
+    ctx = torch.tensor([90, 17], dtype=torch.int32, device="cuda")
+    _same(lambda q, k, v: ops.paged_attn(q, k, v, bt, ctx), _rand(2, 8, 64),
+          _rand(12, 2, 16, 64, seed=1), _rand(12, 2, 16, 64, seed=2))
+
+
+def test_latent_attn(device):
+    bt = torch.arange(12, dtype=torch.int32, device="cuda").view(2, 6)
+    ctx = torch.tensor([90, 17], dtype=torch.int32, device="cuda")
+    seq = torch.tensor([0, 1], dtype=torch.int32, device="cuda")
+    _same(lambda q, c: ops.latent_attn(q, c, bt, seq, ctx, 64, 0.1),
+          _rand(2, 20, 128), _rand(12, 16, 128, seed=1))
+
+
+def test_products(device):
+    _same(lambda x, w: _hip_ops.decode_gemm(x, w, None, 0), _rand(3, 256),
+          _rand(128, 256, seed=1))
+    _same(lambda x, w: _hip_ops.decode_gemm(x, w, None, 0, 1), _rand(40, 256),
+          _rand(128, 256, seed=1))
+    scale = torch.rand(128, device="cuda")
+    w = _rand(128, 256, seed=1).to(torch.float8_e4m3fn).view(torch.uint8)
+    _same(lambda x, w: ops.gemv_fp8(x, w, scale), _rand(3, 256), w)
