@@ -187,12 +187,12 @@ _DECODE_ACT = {ACT_NONE: 0, ACT_GELU_TANH: 6, ACT_GELU_ERF: 7, ACT_SILU: 8}
 
 def _few_rows(x2, weight, bias=None, columns=64):
     """Whether a product of x2 with the rows of weight (in multiples of
-    `columns`) and an activation in the same launch takes decode_gemm (csrc/decode_gemm.hip): up to 64 rows it is
-    faster than the library's product at every size measured (64 rows of
-    28672 x 4096, gated: 51 against 57 us; 768 x 768: 3.8 against 7), up to 256
-    where the product is narrow enough for the launch that it saves to count
-    (128 rows of 16384 x 2048, gated: 20 against 23 us, of 28672 x 4096: 64
-    against 59). K of a single 64-wide chunk, which would leave three of a
+    `columns`) and an activation in the same launch takes decode_gemm
+    (csrc/decode_gemm.hip): up to 64 rows it is faster than the library's
+    product at every size measured (64 rows of 28672 x 4096, gated: 51 against
+    57 us; 768 x 768: 3.8 against 7), up to 256 where the product is narrow
+    enough for the launch that it saves to count (128 rows of 16384 x 2048,
+    gated: 20 against 23 us, of 28672 x 4096: 64 against 59). K of a single 64-wide chunk, which would leave three of a
     workgroup's four waves idle, keeps its general path."""
     M, K = x2.shape
     N = weight.shape[0]

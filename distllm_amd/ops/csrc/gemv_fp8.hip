@@ -10,9 +10,9 @@
 //
 // The ring kernel takes K % 128 == 0: a workgroup has 16 columns (of a gated
 // unit 16 gate and the 16 up columns), its 4 waves take the 128-wide chunks of
-// K in turn, W (2 KiB a chunk) and x (8 rows) pass through LDS buffers of the
-// wave's own by global_load_lds, three or four chunks ahead, and W is widened to bf16
-// (exact) on its way to the MFMA. The vector-unit kernel below it, a wave per
+// K in turn, W (2 KiB a chunk) and x (4 or 8 rows) pass through LDS buffers of
+// the wave's own by global_load_lds, three or four chunks ahead, and W is widened
+// to bf16 (exact) on its way to the MFMA. The vector-unit kernel below it, a wave per
 // column with one 16-byte load a lane in flight, keeps the other K. Measured
 // in a decode graph, us: 28672 x 4096 with swiglu 31 + 5 -> 24.6, 4096 x 14336
 // and 4096 x 4096 together 29 -> 19, 6144 x 4096 9.8 -> 7.6.
