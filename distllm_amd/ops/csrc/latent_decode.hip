@@ -146,7 +146,8 @@ latent_decode_kernel(const unsigned short* __restrict__ q,
   const int last_page = L > 0 ? (L - 1) / PBLK : 0;
   const int* bt = block_table + (long)row_seq[row] * max_blocks;
 
-  // page w of each of the next 64 tiles, on the lanes
+  // page w of each of the next 64 tiles, on the lanes; the window's first page
+  // in the place of those ahead of it, which may be in use elsewhere
   int pages = 0;
   auto fetch_pages = [&](int t) {
     pages = bt[max(min((t + lane) * 4 + w, last_page), lo / PBLK)];
@@ -206,11 +207,12 @@ latent_decode_kernel(const unsigned short* __restrict__ q,
   for (int t = ts; t < te; ++t) {
     char* buf = smem + ((t - ts) & 1) * BUF;
     const int key0 = t * KT + w * 16;
-    if (key0 + 16 > L) {
-      // what lies behind the last key must not meet its zero weight; each
-      // wave clears what it copied
-      for (int at = max(max(L - key0, 0) * (R * 2), hg * NP * 1024) +
-                    lane * 16;
+    if (key0 + 16 > L || key0 + 16 <= lo) {
+      // what lies behind the last key, or was copied in the place of a page
+      // ahead of the window, must not meet its zero weight; each wave clears
+      // what it copied
+      const int from = key0 + 16 <= lo ? 0 : max(L - key0, 0);
+      for (int at = max(from * (R * 2), hg * NP * 1024) + lane * 16;
            at < (hg + 1) * NP * 1024; at += 1024)
         *reinterpret_cast<i32x4*>(buf + w * (QS * 1024) + at) =
             i32x4{0, 0, 0, 0};

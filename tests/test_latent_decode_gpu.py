@@ -60,3 +60,32 @@ def test_tiles_and_shares(device, rank, rot, H):
             bound = size * (2 ** -8 + 2 ** -8 + 1e-4) + 1e-6
             assert ((got - want).abs() <= bound).all(), (window, nsplit)
             assert not got[4].any()
+
+
+@pytest.mark.parametrize("H", [3, 20])
+@pytest.mark.parametrize("rank, rot", [(64, 0), (192, 64), (512, 64)])
+def test_window_within_the_last_page(device, rank, rot, H):
+    """Windows of up to a page that start in the page of the last key: the
+    pages ahead of it are not looked up, and what lies behind the last key must
+    not reach the result from the rows that stand in for them."""
+    ctx = [60, 52, 63, 64, 49, 15, 4090]
+    width = 256
+    g = torch.Generator().manual_seed(rank + H)
+    bt = torch.arange(len(ctx) * width, dtype=torch.int32).view(-1, width)
+    cache = torch.randn(bt.numel(), 16, rank + rot, generator=g).to(BF16)
+    for r, L in enumerate(ctx):
+        if L % 16:
+            cache[bt[r, L // 16], L % 16:] = float("nan")
+    q = torch.randn(len(ctx), H, rank + rot, generator=g).to(BF16)
+    scale = 2.0 / (rank + rot) ** 0.5
+    seq = torch.arange(len(ctx), dtype=torch.int32, device="cuda")
+    lens = torch.tensor(ctx, dtype=torch.int32, device="cuda")
+    for window in (1, 3, 8, 16, 17):
+        want, size = _exact(q, cache.nan_to_num(), bt, ctx, window, scale,
+                            rank)
+        for nsplit in (0, 1, 3):
+            got = ops.latent_attn(q.cuda(), cache.cuda(), bt.cuda(), seq,
+                                  lens, window, scale, nsplit,
+                                  rank).cpu().double()
+            bound = size * (2 ** -7 + 1e-4) + 1e-6  # as above
+            assert ((got - want).abs() <= bound).all(), (window, nsplit)
