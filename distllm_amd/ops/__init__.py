@@ -360,7 +360,7 @@ def norm_linear_fp8(a, b, w_norm, eps, wq, scale, bias=None, gated=False):
     h, x = norm_parts_sum(a, b, w_norm, eps=eps)
     h = h.reshape(-1, h.shape[-1])
     if gated:
-        return gateup_swiglu_fp8(h, wq, scale), x
+        return gateup_swiglu_fp8(h, wq, scale, bias), x
     return gemv_fp8(h, wq, scale, bias), x
 
 
@@ -601,13 +601,13 @@ def gemv_fp8(x, wq, scale, bias=None):
     return _hip_ops.gemv_fp8(x.contiguous(), wq, scale, bias)
 
 
-def gateup_swiglu_fp8(x, wq, scale):
+def gateup_swiglu_fp8(x, wq, scale, bias=None):
     """silu(x @ Wg^T) * (x @ Wu^T) with Wg|Wu packed and quantized as for
-    gemv_fp8."""
+    gemv_fp8; bias, of both, is added ahead of the unit."""
     _require_hip()
     if wq.shape[1] % 128 == 0:
-        return _hip_ops.gemv_fp8(x.contiguous(), wq, scale, None, True)
-    return _hip_ops.swiglu_packed(gemv_fp8(x, wq, scale))
+        return _hip_ops.gemv_fp8(x.contiguous(), wq, scale, bias, True)
+    return _hip_ops.swiglu_packed(gemv_fp8(x, wq, scale, bias))
 
 
 rope_tables = torch_ref.rope_tables

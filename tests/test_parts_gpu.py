@@ -96,3 +96,22 @@ def test_norm_linear_fp8(device, rows, gated, N, K):
     want = (ops.gateup_swiglu_fp8(h[:, 0], w, scale) if gated
             else ops.gemv_fp8(h[:, 0], w, scale, bias))
     assert torch.equal(x, want_x) and torch.equal(got, want)
+
+
+@pytest.mark.parametrize("rows", [1, 2, 8])
+@pytest.mark.parametrize("K", [2560, 2432, 2576])
+def test_gated_bias_fp8(device, rows, K):
+    """The bias of a quantized gated unit, in one launch, in two, and at a K
+    that the ring form does not take."""
+    N = 64
+    a, b = _rand(rows, K), _rand(rows, 1, K, seed=1)
+    nw, scale = _rand(K, seed=3), torch.rand(N, device="cuda") * 0.01 + 0.01
+    w = _rand(N, K, seed=2).to(torch.float8_e4m3fn)
+    bias = _rand(N, seed=4) * 9
+    got, _ = ops.norm_linear_fp8(a, b, nw, 1e-5, w.view(torch.uint8), scale,
+                                 bias, True)
+    h, _ = ops.norm_fwd_sum(a.view_as(b), b, nw, rms=True)
+    z = (h[:, 0].double() @ w.double().T * scale.double() + bias.double())
+    want = torch.nn.functional.silu(z[:, : N // 2]) * z[:, N // 2:]
+    # the output's bf16, and at other K that of gate and up before the product
+    torch.testing.assert_close(got.double(), want, rtol=2 ** -6, atol=2e-2)
