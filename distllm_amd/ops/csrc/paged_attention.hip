@@ -19,8 +19,9 @@
 //    mfma(V^T, P), columns on rows and heads on lanes, V transposed on its
 //    way out of LDS. Softmax state and rescaling are lane-local but for the
 //    maximum over the four groups of lanes that share a head.
-//  - probabilities stay fp32: each goes in as the sum of two bf16 numbers,
-//    which leaves 2^-16 of it, against the 2^-8 of the bf16 result.
+//  - probabilities stay fp32: each goes in as the sum of three bf16 numbers,
+//    which is exactly it (two leave 2^-18 of it, and what two values that
+//    cancel leave can be less than that).
 //  - NS workgroups share a sequence where B * HKV is small; a second launch
 //    joins them.
 // Measured, us, with kernels that read a key row per lane and a value element
@@ -224,19 +225,21 @@ paged_attn_kernel(const unsigned short* __restrict__ q, long q_stride,
 #pragma unroll
         for (int r = 0; r < 4; ++r) acc[d][r] *= alpha;
     }
-    pa_frag hi, lo;
+    pa_frag part[3];
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
       for (int r = 0; r < 4; r += 2) {
-        const float p0 = __builtin_amdgcn_exp2f(sc[kb][r] - m);
-        const float p1 = __builtin_amdgcn_exp2f(sc[kb][r + 1] - m);
+        float p0 = __builtin_amdgcn_exp2f(sc[kb][r] - m);
+        float p1 = __builtin_amdgcn_exp2f(sc[kb][r + 1] - m);
         l += p0 + p1;
-        const unsigned int h = pa_pack(p0, p1);
-        hi.d[kb * 2 + r / 2] = h;
-        lo.d[kb * 2 + r / 2] =
-            pa_pack(p0 - __builtin_bit_cast(float, h << 16),
-                    p1 - __builtin_bit_cast(float, h & 0xffff0000u));
+#pragma unroll
+        for (int e = 0; e < 3; ++e) {
+          const unsigned int h = pa_pack(p0, p1);
+          part[e].d[kb * 2 + r / 2] = h;
+          p0 -= __builtin_bit_cast(float, h << 16);
+          p1 -= __builtin_bit_cast(float, h & 0xffff0000u);
+        }
       }
     // columns 16 d .. of V, keys 4 g .. 4 g + 3 of both halves: the order in
     // which a lane holds its probabilities
@@ -250,10 +253,10 @@ paged_attn_kernel(const unsigned short* __restrict__ q, long q_stride,
             (__attribute__((address_space(3))) s16x4*)(
                 vt + (kb * 16 + row) * (2 * D) +
                 ((d ^ (row & 3)) * 32) + (c16 & 3) * 8));
-      acc[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf.v, hi.v, acc[d], 0,
-                                                       0, 0);
-      acc[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf.v, lo.v, acc[d], 0,
-                                                       0, 0);
+#pragma unroll
+      for (int e = 0; e < 3; ++e)
+        acc[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf.v, part[e].v,
+                                                         acc[d], 0, 0, 0);
     }
     // the buffer is read before the wave fills it again
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");

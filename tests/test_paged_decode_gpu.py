@@ -82,15 +82,57 @@ def test_shares(device, B, width, lens):
                                    _want(q, k, v, table, lens, scale), **TOL)
 
 
-def test_probabilities_in_32_bits(device):
-    """One large score and many small ones: what 16-bit probabilities would
-    lose in their sum is more than a bf16 step of the result."""
-    L, D = 4096, 64
+def _two_scores(device, D, L, scores, values):
+    """Pages of L keys whose scores (scale 1) are scores[i], in steps of
+    2^-26, and whose values are values[i]."""
     k, v, table = _pages(1, 1, D, [L], L // 16, False, 3, device)
-    q = torch.randn(1, 1, D, device=device).to(torch.bfloat16)
+    q = torch.zeros(1, 1, D, device=device, dtype=torch.bfloat16)
+    q[0, 0, :4] = torch.tensor([1.0, 2 ** -8, 2 ** -14, 2 ** -20])
+    rows = torch.zeros(L, D, dtype=torch.float64)
+    left = torch.tensor(scores, dtype=torch.float64)
+    for i in range(4):
+        rows[:, i] = (left / q[0, 0, i].item()).float().bfloat16().double()
+        left = left - rows[:, i] * q[0, 0, i].item()
+    vals = torch.tensor(values, dtype=torch.float64)[:, None].expand(L, D)
+    at = table[0].long()
+    k[at, 0] = rows.to(k.dtype).to(device).view(-1, 16, D)
+    v[at, 0] = vals.to(v.dtype).to(device).view(-1, 16, D)
     ctx = torch.tensor([L], dtype=torch.int32, device=device)
-    out = ops.paged_attn(q, k, v.fill_(1.0), table, ctx)
-    assert (out == 1).all()
+    out = ops.paged_attn(q, k, v, table, ctx, 1.0)
+    s = (rows @ q[0, 0].double().cpu())
+    want = s.softmax(0) @ vals[:, 0].bfloat16().double()
+    return out.double().cpu().flatten(), want
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("p", [2.0 ** -9 * 1.00390625 + 1e-6, 2 ** -9 * 1.0039])
+def test_probabilities_keep_more_than_bf16(device, D, p):
+    """One large score of value -1 and thousands of the same small
+    probability of value 1: rounded to bf16 each is off by up to 2^-9 to the
+    same side, and the sum by more than a bf16 step of what is left."""
+    L = 4096
+    out, want = _two_scores(device, D, L, [0.0] + [math.log(p)] * (L - 1),
+                            [-7.0] + [1.0] * (L - 1))
+    assert abs(want) < 0.2  # of parts of 0.5 and more
+    # bf16 of the result, 2^-9; sums of 32 bits, 2^-24 of the parts (about 1)
+    assert ((out - want).abs() <= abs(want) * 2 ** -8 + 2 ** -22).all()
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_probabilities_in_32_bits(device, D):
+    """Two probabilities that differ in their 17th bit and lower, of values 1
+    and -1, beside the largest of value 0: what is left of them has 2^-24 of
+    each as its error, not the 2^-18 of a sum of two bf16 numbers."""
+    worst = 0.0
+    for i in range(40):
+        s = -0.03 - 0.02 * i
+        d = 3e-5
+        out, want = _two_scores(device, D, 16, [0.0, s, s - d] + [-60.0] * 13,
+                                [0.0, 1.0, -1.0] + [0.0] * 13)
+        worst = max(worst, ((out - want) / want).abs().max().item())
+    # 2^-9 of bf16 and 4 * 2^-24 / 3e-5 of the probabilities (the exponential
+    # to two units in the last place)
+    assert worst <= 2 ** -9 + 4 * 2 ** -24 / 3e-5
 
 
 @pytest.mark.parametrize("fp8", [False, True])
