@@ -148,9 +148,10 @@ topk_chunk_kernel(const float* __restrict__ scores,
 // chain of conflicting atomics). The k-th largest of the 256 threads' largest
 // scores (k <= 64: of those of 64 fours of threads) bounds the k-th largest of
 // the chunk from below; what reaches it is gathered and ranked, by score and,
-// among equals, by place. If more than the
-// candidate buffer holds reach it (few threads have all the large scores, or
-// many scores are equal), the k-th largest itself is found byte by byte.
+// among equals, by place. If more than the candidate buffer holds reach it (few
+// threads have all the large scores, or many scores are equal), the k-th
+// largest itself is found byte by byte, and its equals are counted in the order
+// of their places. (topk_chunk_kernel leaves the order of equals open.)
 // Bound by reading the scores: 256 x 250000, k = 10, both rounds, 210 -> 61 us
 // (4.2 TB/s); 1 x 250000, k = 5, which had 8 workgroups and now has 31, 110 ->
 // 14 us. (Ranking all 256 threads' largest for any k: 167 and 35 us.)
@@ -249,17 +250,42 @@ topk_regs_kernel(const float* __restrict__ scores,
     }
     if (tid == 0) ncand = 0;
     __syncthreads();
-    // those above it (fewer than k) first, then as many equals as fit
+    // those above it (fewer than k) first, then the first `want` of its equals:
+    // how many of them lie ahead of each 64 scores of a wave
     if (T != 0xffffffffu) gather(T + 1);
+    const int lane = tid & 63, wid = tid >> 6;
+    auto equals = [&](int j) {
+      return __ballot(tid + j * 256 < len && u[j] == T);
+    };
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
-      const int i = tid + j * 256;
-      if (i < len && u[j] == T) {
-        const unsigned int slot = atomicAdd(&ncand, 1u);
-        if (slot < TR_CAP)
-          key[slot] = ((unsigned long long)T << 32) | (unsigned int)~i;
-      }
+      const unsigned long long m = equals(j);
+      if (lane == 0) hist[j * 4 + wid] = __popcll(m);
     }
+    __syncthreads();
+    if (tid < 64) {
+      const unsigned int a = hist[2 * tid], b = hist[2 * tid + 1];
+      unsigned int sum = a + b;
+      for (int d = 1; d < 64; d *= 2) {
+        const unsigned int o = __shfl_up(sum, d, 64);
+        if (tid >= d) sum += o;
+      }
+      hist[2 * tid] = sum - a - b;
+      hist[2 * tid + 1] = sum - b;
+    }
+    __syncthreads();
+    const unsigned int first = ncand;
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+      const unsigned long long m = equals(j);
+      const unsigned int at =
+          hist[j * 4 + wid] + __popcll(m & ((1ull << lane) - 1));
+      if ((m >> lane & 1) && at < want)
+        key[first + at] =
+            ((unsigned long long)T << 32) | (unsigned int)~(tid + j * 256);
+    }
+    __syncthreads();
+    if (tid == 0) ncand = first + want;
     __syncthreads();
   }
   const int n = (int)min(ncand, (unsigned int)TR_CAP);

@@ -56,3 +56,20 @@ def test_equal_scores_by_place(device):
     s[0, 100::500] = 9.0
     _, i = ops.topk(s, 5)
     assert i[0].tolist() == [100, 600, 1100, 1600, 2100]
+
+
+@pytest.mark.parametrize("k", [1, 7, 48, 100])
+@pytest.mark.parametrize("N", [5000, 8192, 30000])
+def test_many_equal_scores_by_place(device, N, k):
+    """Also among more equals than the buffer of candidates holds, with and
+    without larger scores ahead of them; the same on every call."""
+    s = torch.zeros(3, N, device=device)
+    s[1, N // 2] = s[1, 11] = 1.0
+    s[2, ::2] = -1.0
+    want = torch.stack([
+        torch.arange(k), torch.tensor(([11, N // 2] + [
+            i for i in range(k + 2) if i != 11])[:k]),
+        torch.arange(k) * 2 + 1])
+    for _ in range(3):
+        _, i = ops.topk(s, k)
+        assert torch.equal(i.cpu().long(), want)
