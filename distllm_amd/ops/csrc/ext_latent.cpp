@@ -274,6 +274,7 @@ void attn_window(torch::Tensor q, torch::Tensor kv, torch::Tensor out,
   for (const auto& t : {cu_q, cu_k, blk_seq, blk_qb}) {
     CHECK_DEV(t); CHECK_CONT(t); CHECK_I32(t);
   }
+  kv = aligned16(kv);
   const void* krp = nullptr;
   int DR = 0;
   if (kr) {
@@ -281,6 +282,7 @@ void attn_window(torch::Tensor q, torch::Tensor kv, torch::Tensor out,
     DR = kr->size(1);
     TORCH_CHECK(kr->size(0) == kv.size(0) && DR == 64,
                 "shared key numbers: 64 per key");
+    kr = aligned16(kr.value());
     krp = kr->data_ptr();
   }
   const int H = q.size(1), DK = q.size(2) - DR, DV = out.size(2);

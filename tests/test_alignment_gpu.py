@@ -44,6 +44,19 @@ def test_latent_attn(device):
           _rand(2, 20, 128), _rand(12, 16, 128, seed=1))
 
 
+def test_attn_window(device):
+    cu = torch.tensor([0, 100, 130], dtype=torch.int32, device="cuda")
+    maps = ops.varlen_block_map(cu)
+
+    def run(q, kv, kr):
+        out = torch.zeros(130, 2, 128, device="cuda", dtype=BF16)
+        return ops.attn_window(q, kv, out, cu, cu, maps, 40, 0.1, kr)
+
+    q = _rand(130, 2, 128)
+    _same(lambda kv, kr: run(q, kv, kr), _rand(130, 2 * 192, seed=1),
+          _rand(130, 64, seed=2))
+
+
 def test_products(device):
     _same(lambda x, w: _hip_ops.decode_gemm(x, w, None, 0), _rand(3, 256),
           _rand(128, 256, seed=1))
