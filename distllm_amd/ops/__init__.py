@@ -202,6 +202,7 @@ def _few_rows(x2, weight, bias=None, columns=64):
             and x2.is_contiguous() and weight.is_contiguous()
             and x2.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0
             and (bias is None or (bias.dtype == torch.bfloat16
+                                  and bias.shape == (N,)
                                   and bias.is_contiguous())))
 
 
@@ -225,7 +226,8 @@ def linear(x, weight, bias=None, act=ACT_NONE):
             out = _hip_ops.decode_gemm(x2, weight, bias, 0, _DECODE_ACT[act])
             return out.reshape(*orig_shape[:-1], N)
         if (mode != "blaslt" and act == ACT_NONE and M <= 256
-                and N % 64 == 0 and K % 64 == 0 and x2.is_contiguous()):
+                and N % 64 == 0 and K % 64 == 0 and x2.is_contiguous()
+                and (bias is None or bias.shape == (N,))):
             if mode == "decode":  # forced in-chain A/B (profiling)
                 out = _hip_ops.decode_gemm(x2, weight, bias, 0)
                 return out.reshape(*orig_shape[:-1], N)
@@ -339,6 +341,7 @@ def norm_linear(a, b, w_norm, eps, weight, bias=None, gated=False,
             and weight.dtype == torch.bfloat16 and weight.shape[1] % 64 == 0
             and N % (128 if gated else 64) == 0
             and (bias is None or (bias.dtype == torch.bfloat16
+                                  and bias.shape == (N,)
                                   and bias.is_contiguous()))
             and _norm_in_product(a, b, w_norm, weight, 1280)):
         _require_hip("_hip_gemm")

@@ -97,6 +97,11 @@ static torch::Tensor decode_gemm_act(torch::Tensor X, torch::Tensor W,
   TORCH_CHECK(act == 0 || !tile || splitk > 1,
               "a fused activation needs splitk > 1");
   TORCH_CHECK(!glu || N % 128 == 0, "gated-unit fusion needs N % 128 == 0");
+  if (bias) {
+    CHECK_DEV(bias.value()); CHECK_CONT(bias.value());
+    CHECK_BF16(bias.value());
+    TORCH_CHECK(bias->numel() == N, "bias must be [N]");
+  }
   const float* nums = nullptr;
   if (act == 3) {
     TORCH_CHECK(act_nums.has_value() && act_nums->numel() == 2, "act_nums");

@@ -101,3 +101,19 @@ def test_strided_weights(device, act):
     wide = torch.zeros(20, 257, device=device, dtype=torch.bfloat16)
     wide[:, 1:] = x
     _close(ops.linear(wide[:, 1:], w, b, act), want)
+
+
+@pytest.mark.parametrize("act", [ops.ACT_NONE, ops.ACT_GELU_ERF])
+@pytest.mark.parametrize("M", [1, 20, 100])
+def test_bias_sizes(device, M, act):
+    """A bias that is not one number per column is refused, or spread, by the
+    library's product, whose rules hold for every number of rows."""
+    x, w, b = _inputs(M, 192, 256, device, 5)
+    for wrong in (b[:100].contiguous(), b[:0].contiguous(), b.cpu()):
+        with pytest.raises(RuntimeError):
+            ops.linear(x, w, wrong, act)
+        with pytest.raises(RuntimeError):
+            ops._hip_ops.decode_gemm(x, w, wrong, 0)
+    want = torch_ref.gemm(x.float(), w.float(), b[:1].float().expand(192),
+                          act).float()
+    _close(ops.linear(x, w, b[:1].contiguous(), act), want)
