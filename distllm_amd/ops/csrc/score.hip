@@ -11,9 +11,11 @@
 // A workgroup of 8 waves has QT queries and 128 rows of the corpus, in steps
 // of 32 columns. Queries are split once ahead (split_kernel) and go to LDS as
 // they lie; rows of the corpus pass through registers, where they are split:
-// once each for up to 256 queries. Two buffers; the next step's copies and
-// loads are in flight, one barrier a step. A wave has QT / 4 queries by 64
-// rows: the 24 fragments of a step feed 96 products, which bound it.
+// once each for up to 256 queries. Two buffers, one barrier a step; the next
+// step's copies and rows are in flight behind the products of this one, and
+// there when the rows are split (the wait for the rows is one for the younger
+// copies too). A wave has QT / 4 queries by 64 rows: the 24 fragments of a step
+// feed 96 products, which bound it.
 // Where a sum comes out infinite or NaN (numbers of the operands that are, or
 // that exceed bf16), it is done again in plain float32.
 //
@@ -81,11 +83,15 @@ score_split_kernel(const float* __restrict__ q, char* __restrict__ planes,
     *reinterpret_cast<i32x2*>(dst + p * QT * 64) = s[p];
 }
 
+// corpus is not __restrict__: its loads are counted by the waits in the loop,
+// together with the copies in assembly, so they must stay in their place among
+// those. Memory that assembly may write orders them; memory that nothing else
+// reaches would not.
 template <int QT>
 __global__ void __launch_bounds__(512, 2)
 score_kernel(const float* __restrict__ q, const char* __restrict__ planes,
-             const float* __restrict__ corpus, float* __restrict__ out,
-             int Q, int N, int K, int tiles) {
+             const float* corpus, float* __restrict__ out, int Q, int N,
+             int K, int tiles) {
   constexpr int MI = QT / 64;            // query blocks of a wave
   constexpr int QB = 3 * QT * 64;        // bytes of the queries of a step
   constexpr int BUF = QB + 3 * SC_CT * 64;
