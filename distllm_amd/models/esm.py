@@ -136,7 +136,7 @@ class Esm2Encoder(nn.Module, _RotaryMixin):
         cs, sn = self._rope(x.device)
         nh, hd = d.num_heads, d.head_dim
         H = d.hidden_size
-        h = self._norm(x, self.layers[0].ln1_w, self.layers[0].ln1_b)
+        h = self._norm(x, *self._next_norm(-1))
         for li, layer in enumerate(self.layers):
             qkv = ops.linear(h, layer.wqkv, layer.bqkv).view(B, S, 3 * nh, hd)
             qkv = ops.rope_qk_(qkv, cs, sn, pos, 2 * nh)
@@ -154,7 +154,7 @@ class Esm2Encoder(nn.Module, _RotaryMixin):
         return ops.norm_fwd_sum(y, x, w, b, eps=self.dims.layer_norm_eps)
 
     def _next_norm(self, li: int):
-        """Weights of the norm that follows layer li."""
+        """Weights of the norm that follows layer li (-1: the embeddings)."""
         if li + 1 < len(self.layers):
             n = self.layers[li + 1]
             return n.ln1_w, n.ln1_b
@@ -207,7 +207,7 @@ class Esm2Encoder(nn.Module, _RotaryMixin):
             xp = torch.nn.functional.pad(xp, (0, 0, 0, Tp - T0))
             pos = torch.nn.functional.pad(pos, (0, Tp - T0))
         T = xp.shape[0]
-        h = self._norm(xp, self.layers[0].ln1_w, self.layers[0].ln1_b)
+        h = self._norm(xp, *self._next_norm(-1))
         for li, layer in enumerate(self.layers):
             qkv = ops.linear(h, layer.wqkv, layer.bqkv).view(T, 3 * nh, hd)
             qkv = ops.rope_qk_(qkv, cs, sn, pos, 2 * nh)
@@ -286,7 +286,7 @@ class EsmCEncoder(nn.Module, _RotaryMixin):
         cs, sn = self._rope(x.device)
         nh, hd = d.num_heads, d.head_dim
         H = d.hidden_size
-        h = self._norm(x, self.layers[0].ln1_w, self.layers[0].ln1_b)
+        h = self._norm(x, *self._next_norm(-1))
         for li, layer in enumerate(self.layers):
             qkv = ops.linear(h, layer.wqkv).view(B, S, 3 * nh, hd)
             qkv = ops.rope_qk_(qkv, cs, sn, pos, 2 * nh)
@@ -335,7 +335,7 @@ class EsmCEncoder(nn.Module, _RotaryMixin):
             xp = torch.nn.functional.pad(xp, (0, 0, 0, Tp - T0))
             pos = torch.nn.functional.pad(pos, (0, Tp - T0))
         T = xp.shape[0]
-        h = self._norm(xp, self.layers[0].ln1_w, self.layers[0].ln1_b)
+        h = self._norm(xp, *self._next_norm(-1))
         for li, layer in enumerate(self.layers):
             qkv = ops.linear(h, layer.wqkv).view(T, 3 * nh, hd)
             qkv = ops.rope_qk_(qkv, cs, sn, pos, 2 * nh)

@@ -1,0 +1,27 @@
+"""Which way calls go, where that can be seen without a GPU: calls that a
+special form does not cover reach the general one."""
+
+import pytest
+import torch
+
+from distllm_amd.models import ModelDims, build_model
+
+
+@pytest.mark.parametrize("arch", ["esm2", "esmc"])
+@pytest.mark.parametrize("packed", ["", "1"])
+def test_encoder_without_layers(arch, packed, monkeypatch):
+    """Embeddings and the last norm are left."""
+    if packed:
+        monkeypatch.setenv("DISTLLM_FORCE_VARLEN", packed)
+    m = build_model(ModelDims(arch=arch, vocab_size=40, hidden_size=32,
+                              num_layers=1, num_heads=2,
+                              intermediate_size=64), dtype=torch.float32)
+    m.layers = m.layers[:0]
+    ids = torch.randint(4, 30, (2, 7))
+    mask = torch.ones_like(ids)
+    mask[1, 5:] = 0
+    out = m(ids, mask)
+    assert out.shape == (2, 7, 32)
+    # the norm's mean and variance, with its weights as they start
+    assert out[0].mean(-1).abs().max() < 1e-5
+    assert (out[0].var(-1, unbiased=False) - 1).abs().max() < 0.1
