@@ -626,7 +626,7 @@ def score(q, corpus):
     against 5000 (80 tiles) 34, 59."""
     Q, K = q.shape
     N = corpus.shape[0]
-    if (q.is_cuda and corpus.is_cuda and 32 < Q < 1 << 20
+    if (q.is_cuda and q.device == corpus.device and 32 < Q < 1 << 20
             and q.dtype == corpus.dtype == torch.float32
             and K % 32 == 0 and 32 <= K < 1 << 20 and N < 1 << 31
             and -(-Q // 256) * -(-N // 128) >= 128 and Q * N < 1 << 39

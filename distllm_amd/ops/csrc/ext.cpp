@@ -360,10 +360,13 @@ torch::Tensor score(torch::Tensor q, torch::Tensor corpus) {
   CHECK_DEV(q); CHECK_CONT(q); CHECK_F32(q);
   CHECK_DEV(corpus); CHECK_CONT(corpus); CHECK_F32(corpus);
   TORCH_CHECK(q.dim() == 2 && corpus.dim() == 2, "matrices");
+  TORCH_CHECK(q.device() == corpus.device(), "score: two devices");
+  // as the library's product that this stands in for
+  const c10::DeviceGuard guard(q.device());
   const long Q = q.size(0), K = q.size(1), N = corpus.size(0);
   TORCH_CHECK(corpus.size(1) == K && K >= 32 && K % 32 == 0, "K % 32");
   TORCH_CHECK(Q < (1L << 20) && N < (1L << 31) && K < (1L << 20) &&
-                  Q * N < (1L << 39),  // 2^31 workgroups of 64 x 128
+                  Q * N < (1L << 39),  // 2^24 workgroups of 256 x 128
               "score: too large");
   TORCH_CHECK((uintptr_t)q.data_ptr() % 16 == 0 &&
                   (uintptr_t)corpus.data_ptr() % 16 == 0,

@@ -4,6 +4,7 @@ special form does not cover reach the general one."""
 import pytest
 import torch
 
+from distllm_amd import ops
 from distllm_amd.models import ModelDims, build_model
 
 
@@ -25,3 +26,41 @@ def test_encoder_without_layers(arch, packed, monkeypatch):
     # the norm's mean and variance, with its weights as they start
     assert out[0].mean(-1).abs().max() < 1e-5
     assert (out[0].var(-1, unbiased=False) - 1).abs().max() < 0.1
+
+
+class _OnGpu:
+    """What ops.score asks of a float32 matrix on a GPU."""
+
+    is_cuda, dtype = True, torch.float32
+
+    def __init__(self, rows, device):
+        self.shape, self.device = (rows, 64), torch.device(device)
+
+    def is_contiguous(self):
+        return True
+
+    def data_ptr(self):
+        return 1 << 20
+
+    def t(self):
+        return self
+
+    def __matmul__(self, other):
+        assert self.device != other.device
+        raise RuntimeError("tensors on two devices")
+
+
+def test_score_of_two_devices(monkeypatch):
+    """Refused by the product, as ever, and not handed to a kernel."""
+    class Ops:
+        def require(self, name):
+            pass
+
+        def score(self, q, corpus):
+            return "kernel"
+
+    monkeypatch.setattr(ops, "_hip_ops", Ops())
+    q = _OnGpu(256, "cuda:0")
+    assert ops.score(q, _OnGpu(50000, "cuda:0")) == "kernel"
+    with pytest.raises(RuntimeError, match="two devices"):
+        ops.score(q, _OnGpu(50000, "cuda:1"))
