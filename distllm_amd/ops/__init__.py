@@ -628,7 +628,7 @@ def score(q, corpus):
     N = corpus.shape[0]
     if (q.is_cuda and q.device == corpus.device and 32 < Q < 1 << 20
             and q.dtype == corpus.dtype == torch.float32
-            and K % 32 == 0 and 32 <= K < 1 << 20 and N < 1 << 31
+            and K % 32 == 0 and 32 <= K < 1 << 20 and N <= (1 << 31) - 256
             and -(-Q // 256) * -(-N // 128) >= 128 and Q * N < 1 << 39
             and corpus.is_contiguous() and q.is_contiguous()
             and q.data_ptr() % 16 == 0 and corpus.data_ptr() % 16 == 0):

@@ -365,7 +365,8 @@ torch::Tensor score(torch::Tensor q, torch::Tensor corpus) {
   const c10::DeviceGuard guard(q.device());
   const long Q = q.size(0), K = q.size(1), N = corpus.size(0);
   TORCH_CHECK(corpus.size(1) == K && K >= 32 && K % 32 == 0, "K % 32");
-  TORCH_CHECK(Q < (1L << 20) && N < (1L << 31) && K < (1L << 20) &&
+  // rows are counted in 32 bits up to the end of the last tile
+  TORCH_CHECK(Q < (1L << 20) && N <= (1L << 31) - 256 && K < (1L << 20) &&
                   Q * N < (1L << 39),  // 2^24 workgroups of 256 x 128
               "score: too large");
   TORCH_CHECK((uintptr_t)q.data_ptr() % 16 == 0 &&

@@ -46,12 +46,13 @@ class _OnGpu:
         return self
 
     def __matmul__(self, other):
-        assert self.device != other.device
-        raise RuntimeError("tensors on two devices")
+        if self.device != other.device:
+            raise RuntimeError("tensors on two devices")
+        return "product"
 
 
-def test_score_of_two_devices(monkeypatch):
-    """Refused by the product, as ever, and not handed to a kernel."""
+@pytest.fixture
+def kernels(monkeypatch):
     class Ops:
         def require(self, name):
             pass
@@ -60,7 +61,19 @@ def test_score_of_two_devices(monkeypatch):
             return "kernel"
 
     monkeypatch.setattr(ops, "_hip_ops", Ops())
+
+
+def test_score_of_two_devices(kernels):
+    """Refused by the product, as ever, and not handed to a kernel."""
     q = _OnGpu(256, "cuda:0")
     assert ops.score(q, _OnGpu(50000, "cuda:0")) == "kernel"
     with pytest.raises(RuntimeError, match="two devices"):
         ops.score(q, _OnGpu(50000, "cuda:1"))
+
+
+def test_score_of_as_many_rows_as_32_bits_count(kernels):
+    """A tile's rows past the last one are counted, too."""
+    q = _OnGpu(200, "cuda:0")
+    assert ops.score(q, _OnGpu((1 << 31) - 256, "cuda:0")) == "kernel"
+    for n in ((1 << 31) - 255, (1 << 31) - 1, 1 << 31):
+        assert ops.score(q, _OnGpu(n, "cuda:0")) == "product"
