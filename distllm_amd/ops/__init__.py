@@ -206,23 +206,34 @@ def _few_rows(x2, weight, bias=None, columns=64):
                                   and bias.is_contiguous())))
 
 
+# values of DISTLLM_GEMM that ask for another form than that of few rows
+_OTHER_FORMS = ("blaslt", "gemm8", "gemm16")
+
+
+def _gemm_mode() -> str:
+    return os.environ.get("DISTLLM_GEMM", "auto")
+
+
 def linear(x, weight, bias=None, act=ACT_NONE):
     """Linear layer entry used by models. GPU path: autotuned choice
     between hipBLASLt (plain and fused-epilogue) and the hand-written
     MFMA GEMMs (gemm8.hip, 8-phase gemm16.hip); the products of few rows
     (decode_gemm.hip, with the activation) for M <= 64 and among the
     choices for M <= 256. Override with
-    DISTLLM_GEMM=blaslt|gemm8|gemm16|decode."""
+    DISTLLM_GEMM=blaslt|gemm8|gemm16|decode (the last for M <= 256, gemm8 and
+    gemm16 at their multiples of 256 rows; without an activation M <= 256
+    stays a choice for those two, at other sizes they mean the library)."""
     orig_shape = x.shape
     x2 = x.reshape(-1, orig_shape[-1])
     M, K = x2.shape
     N = weight.shape[0]
     if x.is_cuda:
         _require_hip("_hip_gemm")
-        mode = os.environ.get("DISTLLM_GEMM", "auto")
+        mode = _gemm_mode()
         if x2.dtype == torch.float32:  # true 32-bit products
             mode = "blaslt"
-        if mode != "blaslt" and M <= 64 and _few_rows(x2, weight, bias):
+        if (mode not in _OTHER_FORMS and M <= 64
+                and _few_rows(x2, weight, bias)):
             out = _hip_ops.decode_gemm(x2, weight, bias, 0, _DECODE_ACT[act])
             return out.reshape(*orig_shape[:-1], N)
         if (mode != "blaslt" and act == ACT_NONE and M <= 256
@@ -308,7 +319,7 @@ def linear_parts(x, weight, bias=None):
     x2 = x.reshape(-1, x.shape[-1])
     M, K = x2.shape
     if (x.is_cuda and 0 < M <= 64
-            and os.environ.get("DISTLLM_GEMM", "auto") != "blaslt"):
+            and _gemm_mode() not in _OTHER_FORMS):
         _require_hip("_hip_gemm")
         if (_few_rows(x2, weight, bias)
                 and _hip_ops.decode_gemm_shares(M, weight.shape[0], K) > 1):
@@ -337,7 +348,7 @@ def norm_linear(a, b, w_norm, eps, weight, bias=None, gated=False,
     be what linear_parts returned, and with `shares` the linear is of that
     kind. One row is one launch."""
     N = weight.shape[0]
-    if (os.environ.get("DISTLLM_GEMM", "auto") != "blaslt"
+    if (_gemm_mode() not in _OTHER_FORMS
             and weight.dtype == torch.bfloat16 and weight.shape[1] % 64 == 0
             and N % (128 if gated else 64) == 0
             and (bias is None or (bias.dtype == torch.bfloat16

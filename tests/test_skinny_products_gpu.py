@@ -103,6 +103,30 @@ def test_strided_weights(device, act):
     _close(ops.linear(wide[:, 1:], w, b, act), want)
 
 
+@pytest.mark.parametrize("mode", ["gemm8", "gemm16", "blaslt"])
+@pytest.mark.parametrize("act", [ops.ACT_NONE, ops.ACT_GELU_ERF])
+def test_forced_form(device, mode, act, monkeypatch):
+    """A form that the caller asks for is not overruled for few rows of a
+    product with an activation; without one the choice stays measured."""
+    x, w, b = _inputs(20, 192, 256, device, 5)
+    calls, real = [], ops._hip_ops
+
+    class Spy:
+        def __getattr__(self, name):
+            if name == "decode_gemm":
+                calls.append(name)
+            return getattr(real, name)
+
+    monkeypatch.setenv("DISTLLM_GEMM", mode)
+    monkeypatch.setattr(ops, "_hip_ops", Spy())
+    monkeypatch.setattr(ops, "_GEMM_CHOICE", {})
+    out = ops.linear(x, w, b, act)
+    _close(out, torch_ref.gemm(x.float(), w.float(), b.float(), act).float())
+    assert not calls or (act == ops.ACT_NONE and mode != "blaslt")
+    measured = bool(ops._GEMM_CHOICE)
+    assert measured == (act == ops.ACT_NONE and mode != "blaslt")
+
+
 @pytest.mark.parametrize("act", [ops.ACT_NONE, ops.ACT_GELU_ERF])
 @pytest.mark.parametrize("M", [1, 20, 100])
 def test_bias_sizes(device, M, act):
