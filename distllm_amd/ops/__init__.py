@@ -538,10 +538,10 @@ def key_bias(mask):
 def bert_few_rows(x, mask_f, layers, heads, eps, act):
     """All layers (post-normed, each a tuple of its twelve tensors, see
     csrc/encoder_layers.cpp) of a BERT-class encoder on x [B, S, H] in one
-    call; None where rows, types or sizes want the general path, layer by
-    layer: the rules are those of linear's products of few rows, with which
-    every product here would be made, and of the attention's native head
-    sizes."""
+    call; None where rows, types, layouts or sizes (one layer's or another's)
+    want the general path, layer by layer: the rules are those of linear's
+    products of few rows, with which every product here would be made, and of
+    the attention's native head sizes."""
     M, H = x.shape[0] * x.shape[1], x.shape[2]
     if not (x.is_cuda and x.dtype == torch.bfloat16 and 0 < M <= 64
             and act in (ACT_GELU_TANH, ACT_GELU_ERF)
@@ -552,9 +552,6 @@ def bert_few_rows(x, mask_f, layers, heads, eps, act):
     for w in (layers[0][0], w1, w2):
         if w.shape[0] % 64 or w.shape[1] % 64 or w.shape[1] < 128:
             return None
-    if not all(t.dtype == torch.bfloat16 and t.is_contiguous()
-               and t.device == x.device for p in layers for t in p):
-        return None
     _require_hip()
     return _hip_ops.bert_few_rows(x.contiguous(), mask_f,
                                   [t for p in layers for t in p], heads, eps,

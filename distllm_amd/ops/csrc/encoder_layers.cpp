@@ -21,10 +21,13 @@ int decode_gemm_shares(int, int, int);
 
 // x [B, S, H]; mask [B, S] additive; layers: wqkv, bqkv, wo, bo, ln1_w, ln1_b,
 // w1, b1, w2, b2, ln2_w, ln2_b of every layer in turn; act: decode_gemm's code
-// of the feed-forward's activation.
-torch::Tensor bert_few_rows(torch::Tensor x, torch::Tensor mask,
-                            std::vector<torch::Tensor> layers, int64_t heads,
-                            double eps, int64_t act) {
+// of the feed-forward's activation. Nothing where a layer's tensors are not
+// contiguous bf16 ones of the first layer's sizes: layers one by one take those.
+c10::optional<torch::Tensor> bert_few_rows(torch::Tensor x,
+                                           torch::Tensor mask,
+                                           std::vector<torch::Tensor> layers,
+                                           int64_t heads, double eps,
+                                           int64_t act) {
   CHECK_DEV(x); CHECK_CONT(x); CHECK_BF16(x);
   CHECK_FLOATS(mask);
   TORCH_CHECK(x.dim() == 3, "x must be [B, S, H]");
@@ -36,18 +39,18 @@ torch::Tensor bert_few_rows(torch::Tensor x, torch::Tensor mask,
   TORCH_CHECK(layers.size() % 12 == 0 && !layers.empty(),
               "twelve tensors per layer");
   TORCH_CHECK(act == 6 || act == 7, "activation");
+  TORCH_CHECK(layers[6].dim() == 2 && layers[6].size(0) % 64 == 0,
+              "feed-forward size");
   const long I = layers[6].size(0);
-  TORCH_CHECK(I % 64 == 0, "feed-forward size");
   const long rows[12] = {3L * H, 3L * H, H, H, H, H, I, I, H, H, H, H};
   const long cols[12] = {H, 0, H, 0, 0, 0, H, 0, I, 0, 0, 0};
   for (size_t i = 0; i < layers.size(); ++i) {
     const auto& t = layers[i];
     const int k = i % 12;
-    TORCH_CHECK(t.is_cuda() && t.device() == x.device() &&
-                    t.scalar_type() == at::kBFloat16 && t.is_contiguous() &&
-                    t.size(0) == rows[k] && t.dim() == (cols[k] ? 2 : 1) &&
-                    (cols[k] == 0 || t.size(1) == cols[k]),
-                "layer tensor ", k, " of layer ", i / 12);
+    if (!(t.device() == x.device() && t.scalar_type() == at::kBFloat16 &&
+          t.is_contiguous() && t.dim() == (cols[k] ? 2 : 1) &&
+          t.size(0) == rows[k] && (cols[k] == 0 || t.size(1) == cols[k])))
+      return c10::nullopt;
     if (cols[k]) layers[i] = aligned16(t);
   }
   auto some = [&](long n) { return torch::empty({M, n}, x.options()); };

@@ -622,9 +622,11 @@ std::vector<torch::Tensor> gemv_fp8_norm(torch::Tensor a, torch::Tensor b,
 }
 
 // encoder_layers.cpp
-torch::Tensor bert_few_rows(torch::Tensor x, torch::Tensor mask,
-                            std::vector<torch::Tensor> layers, int64_t heads,
-                            double eps, int64_t act);
+c10::optional<torch::Tensor> bert_few_rows(torch::Tensor x,
+                                           torch::Tensor mask,
+                                           std::vector<torch::Tensor> layers,
+                                           int64_t heads, double eps,
+                                           int64_t act);
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("norm_fwd", &norm_fwd, "fused residual+LayerNorm/RMSNorm");

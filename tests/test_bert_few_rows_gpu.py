@@ -90,3 +90,16 @@ def test_streams(device):
                 got.append(m(i, torch.ones_like(i)))
         torch.cuda.synchronize()
         assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+def test_layers_of_different_sizes(device):
+    """A layer whose feed-forward is of another size than the first's."""
+    m = _model(device)
+    ids = torch.randint(0, 300, (1, 20), device=device)
+    mask = torch.ones_like(ids)
+    x = m.layers[1]
+    with torch.no_grad():
+        x.w1 = torch.nn.Parameter(x.w1[:192].clone())
+        x.b1 = torch.nn.Parameter(x.b1[:192].clone())
+        x.w2 = torch.nn.Parameter(x.w2[:, :192].contiguous())
+    assert torch.equal(m(ids, mask), _layers(m, ids, mask))
