@@ -510,8 +510,9 @@ def rope_qk_(x, cs, sn, pos, heads: int):
 def embed_layer_norm(ids, pos_ids, word, pos, type_row, w, b, eps):
     """Layer norm of word[ids] + pos[pos_ids] + type_row; pos_ids None:
     positions 0, 1, ... of every row of ids [B, S]."""
-    if word.is_cuda and word.dtype == torch.bfloat16 \
-            and word.shape[1] % 8 == 0:
+    if (word.is_cuda and word.dtype == torch.bfloat16
+            and word.shape[1] % 8 == 0
+            and all(t.is_contiguous() for t in (word, pos, type_row))):
         _require_hip()
         return _hip_ops.embed_layer_norm(
             ids.contiguous(), None if pos_ids is None

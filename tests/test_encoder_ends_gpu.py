@@ -30,6 +30,20 @@ def test_embed_layer_norm(device, H, own):
     torch.testing.assert_close(got.float(), want, atol=1e-2, rtol=8e-3)
 
 
+@pytest.mark.parametrize("strided", range(3))
+def test_embed_layer_norm_of_strided_tables(device, strided):
+    """Tables that are views of others."""
+    args = [_some(device, 50, 64), _some(device, 12, 64, seed=1),
+            *(_some(device, 64, seed=n) for n in (2, 3, 4))]
+    ids = torch.randint(0, 50, (3, 11), device=device)
+    want = ops.embed_layer_norm(ids, None, *args, 1e-5)
+    t = args[strided]
+    args[strided] = torch.stack([t, t], -1)[..., 0]
+    got = ops.embed_layer_norm(ids, None, *args, 1e-5)
+    # here sums are rounded to bf16 ahead of the norm
+    torch.testing.assert_close(got, want, atol=4e-2, rtol=2e-2)
+
+
 @pytest.mark.parametrize("dtype", [torch.bool, torch.int8, torch.uint8,
                                    torch.int16, torch.int32, torch.int64,
                                    torch.float32])
