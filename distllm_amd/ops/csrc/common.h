@@ -92,6 +92,20 @@ __device__ __forceinline__ void copy_to_lds(const void* src,
         : "memory", "m0");
 }
 
+// 16 bytes at any address
+typedef __attribute__((ext_vector_type(4), aligned(1))) int i32x4_any;
+
+// The same copy of 16 bytes a lane where the sources need not start at their
+// multiples, as that asks: through a register, and waited for.
+template <bool ALIGNED>
+__device__ __forceinline__ void to_lds(const void* src, char* base) {
+  if constexpr (ALIGNED)
+    copy_to_lds(src, base);
+  else
+    *reinterpret_cast<i32x4*>(base + (threadIdx.x & 63) * 16) =
+        *reinterpret_cast<const i32x4_any*>(src);
+}
+
 // Workgroups go round the eight XCDs one by one: number b of n such that
 // each XCD (an L2 cache of its own) gets a contiguous run of numbers.
 __device__ __forceinline__ int xcd_run(int b, int n) {

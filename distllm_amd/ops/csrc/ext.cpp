@@ -54,7 +54,7 @@ void launch_sample(const float*, const float*, int*, int, int, float, float,
                    hipStream_t);
 void launch_paged_attn(const void*, long, const void*, const void*,
                        const int*, const int*, void*, void*, void*, int, int,
-                       int, int, int, int, float, bool, hipStream_t);
+                       int, int, int, int, float, bool, bool, hipStream_t);
 void launch_norm_parts(const float*, int, const void*, const void*, void*,
                        void*, int, int, float, hipStream_t);
 void launch_rope_put(const void*, const float*, int, const void*,
@@ -458,8 +458,8 @@ torch::Tensor paged_attn(torch::Tensor q, torch::Tensor kcache,
   auto out = torch::empty_like(q);
   if (B == 0) return out;
   q = aligned16(q);
-  kcache = aligned16(kcache);
-  vcache = aligned16(vcache);
+  const bool aligned = (uintptr_t)kcache.data_ptr() % 16 == 0 &&
+                       (uintptr_t)vcache.data_ptr() % 16 == 0;
   // Workgroups that share a sequence: as many as make two for every CU, each
   // with at least 256 of the positions that the block table has room for. In
   // us, 1, 2, 4, 8, 16 shares: B = 1 of 2048 25, 18, 13, 11.2, 11.9; B = 8 of
@@ -479,7 +479,7 @@ torch::Tensor paged_attn(torch::Tensor q, torch::Tensor kcache,
                     ctx_len.data_ptr<int>(), out.data_ptr(),
                     NS > 1 ? pacc.data_ptr() : nullptr,
                     NS > 1 ? pml.data_ptr() : nullptr, B, H, HKV, D,
-                    max_blocks, NS, (float)scale, fp8, cur_stream());
+                    max_blocks, NS, (float)scale, fp8, aligned, cur_stream());
   return out;
 }
 

@@ -25,7 +25,7 @@ bool latent_decode_covers(int, int);
 void launch_latent_decode(const void*, const void*, const int*, const int*,
                           const int*, void*, void*, void*, int, int, int, int,
                           int, int, int, float, const float*, const void*,
-                          int, hipStream_t);
+                          int, bool, hipStream_t);
 void launch_attn_window(const void*, const void*, const void*, const void*,
                         void*, const int*, const int*, const int*, const int*,
                         int, int, int, int, int, long, long, int, float,
@@ -227,7 +227,7 @@ torch::Tensor latent_attn(torch::Tensor q, torch::Tensor cache,
     return out;
   }
   q = aligned16(q);
-  cache = aligned16(cache);
+  const bool aligned = (uintptr_t)cache.data_ptr() % 16 == 0;
   // Split each row's keys until the 256 CUs have a workgroup each (its
   // buffers take a CU's LDS; more than fit would be a second round), as long
   // as a share keeps two tiles of 64 keys; four tiles are not worth the second
@@ -258,7 +258,7 @@ torch::Tensor latent_attn(torch::Tensor q, torch::Tensor cache,
                        row_seq.data_ptr<int>(), ctx.data_ptr<int>(),
                        out.data_ptr(), pa, pm, M, H, R, RT - R, (int)NS,
                        bt.size(1), win, (float)scale, e.sink, e.gate,
-                       e.ld_gate, cur_stream());
+                       e.ld_gate, aligned, cur_stream());
   return out;
 }
 

@@ -87,7 +87,9 @@ constexpr int ld_lds() {
   return 2 * KT * (R + ROT) * 2 + 4 * HG * (1024 + 64);
 }
 
-template <int R, int ROT, int HG>
+// ALIGNED: the cache starts at a multiple of 16 bytes, as the copies to LDS ask;
+// else its rows pass through registers, one tile after another.
+template <int R, int ROT, int HG, bool ALIGNED = true>
 __global__ void __launch_bounds__(256 * HG, R + ROT <= 256 ? 2 * HG : HG)
 latent_decode_kernel(const unsigned short* __restrict__ q,
                      const unsigned short* __restrict__ cache,
@@ -162,22 +164,23 @@ latent_decode_kernel(const unsigned short* __restrict__ q,
     for (int i = 0; i < NP; ++i) {
       const int p = hg * NP + i;
       const int at = p * 64 + lane, r = at / RP, c = at % RP;
-      copy_to_lds(src + r * RR + ld_piece<R>(r, c) * 8,
-                  dst + (w * NP * HG + p) * 1024);
+      to_lds<ALIGNED>(src + r * RR + ld_piece<R>(r, c) * 8,
+                      dst + (w * NP * HG + p) * 1024);
     }
 #pragma unroll
     for (int i = 0; i < NR; ++i) {
       const int p = hg * NR + i;
       const int r = p * 8 + (lane >> 3), c = (lane & 7) ^ (r & 7);
-      copy_to_lds(src + r * RR + R + c * 8,
-                  dst + MAIN + (w * NR * HG + p) * 1024);
+      to_lds<ALIGNED>(src + r * RR + R + c * 8,
+                      dst + MAIN + (w * NR * HG + p) * 1024);
     }
   };
 
+  constexpr int COPIES = ALIGNED ? NP + NR : 0;  // in flight, of a tile
   bf16x8 qf[QS + TS];
   if (ts < te) {
     issue(ts);
-    asm volatile("s_waitcnt vmcnt(%0)" ::"i"(NP + NR) : "memory");
+    asm volatile("s_waitcnt vmcnt(%0)" ::"i"(COPIES) : "memory");
     ld_barrier();
 #pragma unroll
     for (int s = 0; s < QS; ++s)
@@ -192,7 +195,7 @@ latent_decode_kernel(const unsigned short* __restrict__ q,
     ld_barrier();
     if (ts + 1 < te) {
       issue(ts + 1);
-      asm volatile("s_waitcnt vmcnt(%0)" ::"i"(NP + NR) : "memory");
+      asm volatile("s_waitcnt vmcnt(%0)" ::"i"(COPIES) : "memory");
     }
   }
   if (ts + 1 >= te) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -394,11 +397,11 @@ extern "C" void launch_latent_decode(
     const int* row_seq, const int* ctx, void* out, void* pacc, void* pml,
     int M, int H, int R, int rot, int NS, int max_blocks, int window,
     float scale, const float* sink, const void* gate, int ld_gate,
-    hipStream_t stream) {
-  const int heads = latent_decode_heads(H);
+    bool aligned, hipStream_t stream) {
+  const int heads = aligned ? latent_decode_heads(H) : 16;
   const int ng = (H + heads - 1) / heads;
-#define LD(RR, RO, HG)                                                        \
-  hipLaunchKernelGGL((latent_decode_kernel<RR, RO, HG>),                      \
+#define LD(RR, RO, HG, AL)                                                    \
+  hipLaunchKernelGGL((latent_decode_kernel<RR, RO, HG, AL>),                  \
                      dim3((M * NS + 7) / 8 * 8 * ng), dim3(256 * HG),         \
                      (ld_lds<RR, RO, HG>()), stream,                          \
                      (const unsigned short*)q, (const unsigned short*)cache,  \
@@ -406,10 +409,11 @@ extern "C" void launch_latent_decode(
                      (float*)pacc, (float*)pml, M, H, ng, NS, max_blocks,     \
                      window, scale, sink, (const unsigned short*)gate,        \
                      ld_gate)
-#define LD_H(RR, RO)                 \
-  do {                               \
-    if (heads == 16) LD(RR, RO, 1);  \
-    else LD(RR, RO, 2);              \
+#define LD_H(RR, RO)                             \
+  do {                                           \
+    if (!aligned) LD(RR, RO, 1, false);          \
+    else if (heads == 16) LD(RR, RO, 1, true);   \
+    else LD(RR, RO, 2, true);                    \
   } while (0)
 #define LD_R(RR)              \
   do {                        \

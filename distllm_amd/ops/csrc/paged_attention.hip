@@ -69,7 +69,9 @@ constexpr int pa_lds(int D, bool fp8) {
   return 4 * pa_ring(D, fp8) * 2 * KT * D * 2;
 }
 
-template <int D, bool FP8>
+// ALIGNED: the pages start at a multiple of 16 bytes, as the copies to LDS ask;
+// else bf16 pages pass through registers like fp8 ones, one tile after another.
+template <int D, bool FP8, bool ALIGNED = true>
 __global__ void __launch_bounds__(256)
 paged_attn_kernel(const unsigned short* __restrict__ q, long q_stride,
                   const char* __restrict__ kcache,
@@ -137,10 +139,10 @@ paged_attn_kernel(const unsigned short* __restrict__ q, long q_stride,
       const int row = p * ROWS + r;
       const long at = page(i, p * ROWS / PBLK) * page_bytes + head_bytes +
                       (row % PBLK) * (D * 2);
-      copy_to_lds(kcache + at + ((c ^ (row & (NCH - 1))) * 16),
-                  dst + p * 1024);
-      copy_to_lds(vcache + at + ((c ^ ((row & 3) << 1)) * 16),
-                  dst + TILE + p * 1024);
+      to_lds<ALIGNED>(kcache + at + ((c ^ (row & (NCH - 1))) * 16),
+                      dst + p * 1024);
+      to_lds<ALIGNED>(vcache + at + ((c ^ ((row & 3) << 1)) * 16),
+                      dst + TILE + p * 1024);
     }
   };
   // fp8: the same rows through registers, 16 numbers a load
@@ -152,8 +154,8 @@ paged_attn_kernel(const unsigned short* __restrict__ q, long q_stride,
       const int at = (j * 64 + lane) * 16, row = at / D, col = at % D;
       const int pg = row < PBLK ? page(i, 0) : page(i, 1);
       const long off = pg * page_bytes + head_bytes + (row % PBLK) * D + col;
-      kreg[j] = *reinterpret_cast<const i32x4*>(kcache + off);
-      vreg[j] = *reinterpret_cast<const i32x4*>(vcache + off);
+      kreg[j] = *reinterpret_cast<const i32x4_any*>(kcache + off);
+      vreg[j] = *reinterpret_cast<const i32x4_any*>(vcache + off);
     }
   };
   auto store8 = [&]() {
@@ -291,6 +293,7 @@ paged_attn_kernel(const unsigned short* __restrict__ q, long q_stride,
       } else {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       }
+      if constexpr (!ALIGNED) wave_sync();
       compute(i);
     }
   }
@@ -388,11 +391,11 @@ extern "C" void launch_paged_attn(const void* q, long q_stride,
                                   void* out, void* pacc, void* pml, int B,
                                   int H, int HKV, int D, int max_blocks,
                                   int NS, float scale, bool fp8,
-                                  hipStream_t stream) {
+                                  bool aligned, hipStream_t stream) {
   const int GR = H / HKV, NG = (GR + 15) / 16;
   const int grid = B * HKV * NG * NS;
-#define PA(DD, F8)                                                            \
-  hipLaunchKernelGGL((paged_attn_kernel<DD, F8>), dim3(grid), dim3(256),      \
+#define PA(DD, F8, AL)                                                        \
+  hipLaunchKernelGGL((paged_attn_kernel<DD, F8, AL>), dim3(grid), dim3(256),  \
                      pa_lds(DD, F8) > 4 * 16 * (DD + 2) * 4                   \
                          ? pa_lds(DD, F8)                                     \
                          : 4 * 16 * (DD + 2) * 4,                             \
@@ -400,11 +403,15 @@ extern "C" void launch_paged_attn(const void* q, long q_stride,
                      (const char*)kcache, (const char*)vcache, block_table,   \
                      ctx_len, (unsigned short*)out, (float*)pacc,             \
                      (float*)pml, H, HKV, max_blocks, NS, scale)
-  if (D == 64) {
-    if (fp8) PA(64, true); else PA(64, false);
-  } else {
-    if (fp8) PA(128, true); else PA(128, false);
-  }
+#define PA_D(DD)                      \
+  do {                                \
+    if (fp8) PA(DD, true, true);      \
+    else if (aligned) PA(DD, false, true); \
+    else PA(DD, false, false);        \
+  } while (0)
+  if (D == 64) PA_D(64);
+  else PA_D(128);
+#undef PA_D
 #undef PA
   if (NS > 1) {
     const int rows = B * H;

@@ -34,6 +34,12 @@ def test_paged_attn(device):
     ctx = torch.tensor([90, 17], dtype=torch.int32, device="cuda")
     _same(lambda q, k, v: ops.paged_attn(q, k, v, bt, ctx), _rand(2, 8, 64),
           _rand(12, 2, 16, 64, seed=1), _rand(12, 2, 16, 64, seed=2))
+    eight = [_rand(12, 2, 16, 128, seed=n).to(torch.float8_e4m3fn)
+             .view(torch.uint8) for n in (1, 2)]
+    q = _rand(2, 8, 128)
+    _same(lambda k, v: ops.paged_attn(q, k, v, bt, ctx), *eight)
+    _same(lambda k, v: ops.paged_attn(q, k, v, bt, ctx),
+          _rand(12, 2, 16, 128, seed=1), _rand(12, 2, 16, 128, seed=2))
 
 
 def test_latent_attn(device):
@@ -42,6 +48,29 @@ def test_latent_attn(device):
     seq = torch.tensor([0, 1], dtype=torch.int32, device="cuda")
     _same(lambda q, c: ops.latent_attn(q, c, bt, seq, ctx, 64, 0.1),
           _rand(2, 20, 128), _rand(12, 16, 128, seed=1))
+
+
+def test_caches_are_not_copied(device):
+    """Pages that start between 16-byte pieces are read where they are."""
+    bt = torch.zeros(1, 4, dtype=torch.int32, device="cuda")
+    ctx = torch.tensor([50], dtype=torch.int32, device="cuda")
+    seq = torch.zeros(1, dtype=torch.int32, device="cuda")
+    pages, latents = (_off(torch.zeros(2000, 1, 16, 128, device="cuda",
+                                       dtype=BF16)) for _ in range(2))
+    eight = _off(torch.zeros(4000, 1, 16, 128, device="cuda",
+                             dtype=torch.uint8))
+    q = _rand(1, 8, 128)
+    for f in (lambda: ops.paged_attn(q, pages, pages, bt, ctx),
+              lambda: ops.paged_attn(q, eight, eight, bt, ctx),
+              lambda: ops.latent_attn(q, latents[:, 0], bt, seq, ctx, 64,
+                                      0.1)):
+        f()
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        f()
+        used = torch.cuda.max_memory_allocated() - before
+        assert used < 4000 * 2048 / 2  # half of the least of them
 
 
 def test_attn_window(device):
