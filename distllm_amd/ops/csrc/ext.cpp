@@ -444,6 +444,23 @@ static void check_kv_pages(const torch::Tensor& kcache,
               "one block-table row and context length per sequence");
 }
 
+// Workgroups that share a sequence in paged_attn: as many as make two for every
+// CU, each with at least 256 of the positions that the block table has room
+// for. In us, 1, 2, 4, 8, 16 shares: B = 1 of 2048 25, 18, 13, 11.2, 11.9; B = 8
+// of 1000 19, 16, 15, 18; B = 16 of 100 to 4000 55, 39, 38, 41, 55; B = 64 of
+// 1124 59, 68, 82. DISTLLM_PA_NSPLIT > 0 asks for a number (1: none; at most a
+// page each, and 64, which is what the joining kernel has lanes for).
+int64_t paged_attn_shares(int64_t B, int64_t H, int64_t HKV,
+                          int64_t max_blocks) {
+  const char* e = getenv("DISTLLM_PA_NSPLIT");
+  const long asked = e ? atol(e) : 0;
+  const long groups = std::max<long>(B * HKV * ((H / HKV + 15) / 16), 1);
+  return std::max<long>(asked > 0 ? std::min<long>({asked, max_blocks, 64})
+                                  : std::min<long>({512 / groups,
+                                                    max_blocks / 16, 32}),
+                        1);
+}
+
 torch::Tensor paged_attn(torch::Tensor q, torch::Tensor kcache,
                          torch::Tensor vcache, torch::Tensor block_table,
                          torch::Tensor ctx_len, double scale) {
@@ -460,14 +477,7 @@ torch::Tensor paged_attn(torch::Tensor q, torch::Tensor kcache,
   q = aligned16(q);
   const bool aligned = (uintptr_t)kcache.data_ptr() % 16 == 0 &&
                        (uintptr_t)vcache.data_ptr() % 16 == 0;
-  // Workgroups that share a sequence: as many as make two for every CU, each
-  // with at least 256 of the positions that the block table has room for. In
-  // us, 1, 2, 4, 8, 16 shares: B = 1 of 2048 25, 18, 13, 11.2, 11.9; B = 8 of
-  // 1000 19, 16, 15, 18; B = 16 of 100 to 4000 55, 39, 38, 41, 55; B = 64 of
-  // 1124 59, 68, 82.
-  const long groups = (long)B * HKV * ((H / HKV + 15) / 16);
-  const int NS = (int)std::max<long>(
-      std::min<long>({512 / groups, max_blocks / 16, 32}), 1);
+  const int NS = (int)paged_attn_shares(B, H, HKV, max_blocks);
   torch::Tensor pacc, pml;
   if (NS > 1) {
     auto f32 = q.options().dtype(at::kFloat);
@@ -658,6 +668,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gemv_fp8_norm", &gemv_fp8_norm);
   m.def("sample_tokens", &sample_tokens);
   m.def("paged_attn", &paged_attn);
+  m.def("paged_attn_shares", &paged_attn_shares);
   m.def("cache_put", &cache_put);
   m.def("norm_parts", &norm_parts);
   m.def("rope_put", &rope_put, py::arg("qkv"), py::arg("cs"), py::arg("sn"),

@@ -82,6 +82,23 @@ def test_shares(device, B, width, lens):
                                    _want(q, k, v, table, lens, scale), **TOL)
 
 
+@pytest.mark.parametrize("asked", ["0", "1", "2", "7", "64", "1000"])
+def test_shares_asked_for(device, asked, monkeypatch):
+    """DISTLLM_PA_NSPLIT, for few long sequences and for many short ones."""
+    monkeypatch.setenv("DISTLLM_PA_NSPLIT", asked)
+    for lens, width in (([4000, 70], 300), ([20] * 40, 2)):
+        B = len(lens)
+        want = {"0": 300 // 16 if B == 2 else 1}.get(
+            asked, min(int(asked), width, 64))
+        assert ops._hip_ops.paged_attn_shares(B, 8, 2, width) == want
+        k, v, table = _pages(B, 2, 64, lens, width, False, B, device)
+        q = torch.randn(B, 8, 64, device=device).to(torch.bfloat16)
+        ctx = torch.tensor(lens, dtype=torch.int32, device=device)
+        out = ops.paged_attn(q, k, v, table, ctx)
+        torch.testing.assert_close(out.float().cpu(),
+                                   _want(q, k, v, table, lens, 0.125), **TOL)
+
+
 def _two_scores(device, D, L, scores, values):
     """Pages of L keys whose scores (scale 1) are scores[i], in steps of
     2^-26, and whose values are values[i]."""
