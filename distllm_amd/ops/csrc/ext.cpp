@@ -444,21 +444,28 @@ static void check_kv_pages(const torch::Tensor& kcache,
               "one block-table row and context length per sequence");
 }
 
-// Workgroups that share a sequence in paged_attn: as many as make two for every
-// CU, each with at least 256 of the positions that the block table has room
-// for. In us, 1, 2, 4, 8, 16 shares: B = 1 of 2048 25, 18, 13, 11.2, 11.9; B = 8
-// of 1000 19, 16, 15, 18; B = 16 of 100 to 4000 55, 39, 38, 41, 55; B = 64 of
-// 1124 59, 68, 82. DISTLLM_PA_NSPLIT > 0 asks for a number (1: none; at most a
-// page each, and 64, which is what the joining kernel has lanes for).
+// Workgroups that share a sequence in paged_attn: as many as make one for every
+// CU (two where pages are fp8, whose buffers leave a CU to two), each with at
+// least 256 of the positions that the block table has room for, 512 beyond eight
+// of them: the table may be wide and the context short, and then every share
+// costs and none gains. In us, at contexts of 64 to 200, 500, 2000 (bf16, heads
+// of 128): 8 x 8 grouped heads 1 share 5.0, 9.3, 27; 4 8.3, 8.8, 19; 8 12.7, 13,
+// 22. 8 x 32 heads 1 5.1, 15, 44; 2 11, 21, 46. 1 x 8 grouped heads of 2048 1 24,
+// 8 10.5, 12 11.5, 16 11.1; of 8000 15 17.6, 31 19.0. 16 x 8 grouped of 100 to
+// 3745 1 45, 2 31, 4 31; fp8 2 31, 4 25, 8 26. DISTLLM_PA_NSPLIT > 0 asks for a
+// number (1: none; at most a page each, and 64, which is what the joining kernel
+// has lanes for).
 int64_t paged_attn_shares(int64_t B, int64_t H, int64_t HKV,
-                          int64_t max_blocks) {
+                          int64_t max_blocks, bool fp8) {
   const char* e = getenv("DISTLLM_PA_NSPLIT");
   const long asked = e ? atol(e) : 0;
   const long groups = std::max<long>(B * HKV * ((H / HKV + 15) / 16), 1);
-  return std::max<long>(asked > 0 ? std::min<long>({asked, max_blocks, 64})
-                                  : std::min<long>({512 / groups,
-                                                    max_blocks / 16, 32}),
-                        1);
+  const long room =
+      std::max(std::min(max_blocks / 16, (int64_t)8), max_blocks / 32);
+  return std::max<long>(
+      asked > 0 ? std::min<long>({asked, max_blocks, 64})
+                : std::min<long>({(fp8 ? 512 : 256) / groups, room, 32}),
+      1);
 }
 
 torch::Tensor paged_attn(torch::Tensor q, torch::Tensor kcache,
@@ -477,7 +484,7 @@ torch::Tensor paged_attn(torch::Tensor q, torch::Tensor kcache,
   q = aligned16(q);
   const bool aligned = (uintptr_t)kcache.data_ptr() % 16 == 0 &&
                        (uintptr_t)vcache.data_ptr() % 16 == 0;
-  const int NS = (int)paged_attn_shares(B, H, HKV, max_blocks);
+  const int NS = (int)paged_attn_shares(B, H, HKV, max_blocks, fp8);
   torch::Tensor pacc, pml;
   if (NS > 1) {
     auto f32 = q.options().dtype(at::kFloat);

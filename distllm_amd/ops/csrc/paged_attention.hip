@@ -29,8 +29,10 @@
 // tokens 32 -> 11.0 (31 -> 11.1); B = 16 of 100 to 4000 115 -> 36.5 (104 ->
 // 24); B = 64 of 200 to 2048 137 -> 61, 4.8 TB/s (117 -> 38); B = 128 of 1000
 // 150 -> 98, 5.3 TB/s (96 -> 56). With copies that the compiler knows of, which
-// the reads of V then wait for, also for the next tile's: 39, 65 and 101. The
-// 128 KiB of buffers leave one workgroup per CU.
+// the reads of V then wait for, also for the next tile's: 39, 65 and 101.
+// Those kernels are still the faster ones where contexts of a page or two meet
+// 16 key heads and rows or more (64 x 32 heads of 128, of 16: 11, now 19), for
+// which the lengths, on the device only, would have to be known ahead.
 #include "common.h"
 #include <hip/hip_fp8.h>
 
@@ -64,14 +66,16 @@ __device__ __forceinline__ void pa_widen(const i32x4 v, i32x4 (&out)[2]) {
   }
 }
 
-constexpr int pa_ring(int D, bool fp8) { return fp8 ? 1 : D == 64 ? 4 : 2; }
-constexpr int pa_lds(int D, bool fp8) {
-  return 4 * pa_ring(D, fp8) * 2 * KT * D * 2;
+// LDS of a workgroup: the waves' rings of R tiles of K and V, then their states
+constexpr int NW = 4;  // waves of a workgroup
+constexpr int pa_lds(int D, int R) {
+  const int ring = NW * R * 2 * KT * D * 2, states = NW * 16 * (D + 2) * 4;
+  return ring > states ? ring : states;
 }
 
 // ALIGNED: the pages start at a multiple of 16 bytes, as the copies to LDS ask;
 // else bf16 pages pass through registers like fp8 ones, one tile after another.
-template <int D, bool FP8, bool ALIGNED = true>
+template <int D, bool FP8, bool ALIGNED, int R>
 __global__ void __launch_bounds__(256)
 paged_attn_kernel(const unsigned short* __restrict__ q, long q_stride,
                   const char* __restrict__ kcache,
@@ -85,7 +89,6 @@ paged_attn_kernel(const unsigned short* __restrict__ q, long q_stride,
   constexpr int ROWS = 1024 / (2 * D);  // rows of a 1 KiB piece of a tile
   constexpr int PIECES = KT / ROWS;     // pieces of K or V of a tile
   constexpr int TILE = KT * D * 2;      // bytes of K or V of a tile
-  constexpr int R = pa_ring(D, FP8);
   constexpr int DB = D / 16;
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -100,7 +103,7 @@ paged_attn_kernel(const unsigned short* __restrict__ q, long q_stride,
   const int L = min(ctx_len[b], max_blocks * PBLK);
   const int T = (L + KT - 1) / KT, per = (T + NS - 1) / NS;
   const int t0 = split * per + wid, t1 = min(T, split * per + per);
-  const int mine = t1 > t0 ? (t1 - t0 + 3) / 4 : 0;  // tiles t0, t0 + 4, ...
+  const int mine = t1 > t0 ? (t1 - t0 + NW - 1) / NW : 0;  // t0, t0 + NW, ...
   const int last_page = max(L - 1, 0) / PBLK;
   const int* bt = block_table + (long)b * max_blocks;
   const long page_bytes = (long)HKV * PBLK * D * (FP8 ? 1 : 2);
@@ -121,7 +124,7 @@ paged_attn_kernel(const unsigned short* __restrict__ q, long q_stride,
   // page numbers of the wave's next 32 tiles, two a tile, on the lanes
   int pages = 0;
   auto fetch_pages = [&](int i) {
-    const int p = (t0 + (i + (lane >> 1)) * 4) * 2 + (lane & 1);
+    const int p = (t0 + (i + (lane >> 1)) * NW) * 2 + (lane & 1);
     pages = mine > 0 ? bt[min(p, last_page)] : 0;
   };
   auto page = [&](int i, int half) {
@@ -186,7 +189,7 @@ paged_attn_kernel(const unsigned short* __restrict__ q, long q_stride,
   auto compute = [&](int i) {
     char* kt = ring + (i % R) * 2 * TILE;
     char* vt = kt + TILE;
-    const int left = L - (t0 + i * 4) * KT;  // keys of the tile, if < 32
+    const int left = L - (t0 + i * NW) * KT;  // keys of the tile, if < 32
     if (left < KT) {
       // what lies behind the last key must not meet its zero probability
       for (int k = left * (2 * D) + lane * 16; k < TILE; k += 1024)
@@ -302,8 +305,8 @@ paged_attn_kernel(const unsigned short* __restrict__ q, long q_stride,
   l += __shfl_xor(l, 16, 64);
   l += __shfl_xor(l, 32, 64);
   __syncthreads();
-  float* ml = reinterpret_cast<float*>(smem);  // [4][16][2]
-  float* wacc = ml + 4 * 16 * 2;               // [4][16][D]
+  float* ml = reinterpret_cast<float*>(smem);  // [NW][16][2]
+  float* wacc = ml + NW * 16 * 2;              // [NW][16][D]
   if (g == 0) {
     ml[(wid * 16 + c16) * 2] = m;
     ml[(wid * 16 + c16) * 2 + 1] = l;
@@ -314,15 +317,15 @@ paged_attn_kernel(const unsigned short* __restrict__ q, long q_stride,
         acc[d];
   __syncthreads();
   const long part = ((long)(b * HKV + kvh) * NS + split) * GR + hg * 16;
-  for (int i = threadIdx.x; i < nh * (D / 4); i += 256) {
+  for (int i = threadIdx.x; i < nh * (D / 4); i += NW * 64) {
     const int head = i / (D / 4), col = i % (D / 4) * 4;
     float M = -1e30f;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) M = fmaxf(M, ml[(w * 16 + head) * 2]);
+    for (int w = 0; w < NW; ++w) M = fmaxf(M, ml[(w * 16 + head) * 2]);
     float sum = 0.f;
     f32x4 o = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
+    for (int w = 0; w < NW; ++w) {
       const float a = __builtin_amdgcn_exp2f(ml[(w * 16 + head) * 2] - M);
       sum += ml[(w * 16 + head) * 2 + 1] * a;
       const f32x4 v =
@@ -394,20 +397,26 @@ extern "C" void launch_paged_attn(const void* q, long q_stride,
                                   bool aligned, hipStream_t stream) {
   const int GR = H / HKV, NG = (GR + 15) / 16;
   const int grid = B * HKV * NG * NS;
-#define PA(DD, F8, AL)                                                        \
-  hipLaunchKernelGGL((paged_attn_kernel<DD, F8, AL>), dim3(grid), dim3(256),  \
-                     pa_lds(DD, F8) > 4 * 16 * (DD + 2) * 4                   \
-                         ? pa_lds(DD, F8)                                     \
-                         : 4 * 16 * (DD + 2) * 4,                             \
-                     stream, (const unsigned short*)q, q_stride,              \
-                     (const char*)kcache, (const char*)vcache, block_table,   \
-                     ctx_len, (unsigned short*)out, (float*)pacc,             \
-                     (float*)pml, H, HKV, max_blocks, NS, scale)
-#define PA_D(DD)                      \
-  do {                                \
-    if (fp8) PA(DD, true, true);      \
-    else if (aligned) PA(DD, false, true); \
-    else PA(DD, false, false);        \
+#define PA(DD, F8, AL, R)                                                     \
+  hipLaunchKernelGGL((paged_attn_kernel<DD, F8, AL, R>), dim3(grid),          \
+                     dim3(256), pa_lds(DD, R), stream,                        \
+                     (const unsigned short*)q, q_stride, (const char*)kcache, \
+                     (const char*)vcache, block_table, ctx_len,               \
+                     (unsigned short*)out, (float*)pacc, (float*)pml, H, HKV, \
+                     max_blocks, NS, scale)
+// Tiles in a wave's ring. Two tiles of 128 columns leave a CU to one workgroup;
+// from 1024 workgroups on, four for every CU, a second one on the CU counts for
+// more, for short contexts are a chain of three reads each. In us, 64 x 32 heads
+// of 128, contexts of 16, of 200, of 200 to 2027: two tiles 30, 51, 211; one 20,
+// 40, 213 (two waves 12, 38, 217 to 226: the long ones wait for each other).
+// 64 x 8 heads, grouped: two 8.8, 16.9, 53; one 6.4, 14.6, 55. With heads of 64,
+// 64 x 32: four tiles 22, 38, 120; two 14, 24, 109.
+#define PA_D(DD)                                                      \
+  do {                                                                \
+    if (fp8) PA(DD, true, true, 1);                                   \
+    else if (!aligned) PA(DD, false, false, 1);                       \
+    else if (DD == 128 && grid >= 1024) PA(DD, false, true, 1);       \
+    else PA(DD, false, true, 2);                                      \
   } while (0)
   if (D == 64) PA_D(64);
   else PA_D(128);

@@ -82,15 +82,31 @@ def test_shares(device, B, width, lens):
                                    _want(q, k, v, table, lens, scale), **TOL)
 
 
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("D", [64, 128])
+def test_many_workgroups(device, D, fp8):
+    """As many as change the buffers, and one row less."""
+    for B in (127, 128):
+        lens = [(37 * b) % 150 for b in range(B)]
+        k, v, table = _pages(B, 8, D, lens, 10, fp8, B, device)
+        raw = [t.view(torch.uint8) if fp8 else t for t in (k, v)]
+        q = torch.randn(B, 16, D, device=device).to(torch.bfloat16)
+        ctx = torch.tensor(lens, dtype=torch.int32, device=device)
+        out = ops.paged_attn(q, *raw, table, ctx)
+        torch.testing.assert_close(
+            out.float().cpu(), _want(q, k, v, table, lens, D ** -0.5), **TOL)
+
+
 @pytest.mark.parametrize("asked", ["0", "1", "2", "7", "64", "1000"])
 def test_shares_asked_for(device, asked, monkeypatch):
     """DISTLLM_PA_NSPLIT, for few long sequences and for many short ones."""
     monkeypatch.setenv("DISTLLM_PA_NSPLIT", asked)
     for lens, width in (([4000, 70], 300), ([20] * 40, 2)):
         B = len(lens)
-        want = {"0": 300 // 16 if B == 2 else 1}.get(
+        want = {"0": 300 // 32 if B == 2 else 1}.get(
             asked, min(int(asked), width, 64))
-        assert ops._hip_ops.paged_attn_shares(B, 8, 2, width) == want
+        assert ops._hip_ops.paged_attn_shares(B, 8, 2, width,
+                                              False) == want
         k, v, table = _pages(B, 2, 64, lens, width, False, B, device)
         q = torch.randn(B, 8, 64, device=device).to(torch.bfloat16)
         ctx = torch.tensor(lens, dtype=torch.int32, device=device)
