@@ -646,26 +646,37 @@ def score(q, corpus):
     return q @ corpus.t()
 
 
+def _topk_in_registers(Q, N, k):
+    """Whether workgroups hold their chunks in registers (topk_regs_kernel).
+    Measured, both rounds, against the radix select: k up to 60 0.2 to 0.9 of
+    its time everywhere (1 to 5000 rows of 300 to 4 million); k = 65, 100, 128
+    from 4096 scores on 0.3 to 0.9, 2048 rows of 1000 1.4, 1.4, 1.2, 64 rows of
+    1000 0.7; k = 200 of 1 to 512 rows 0.4 to 1.0, of 2048 rows 0.9 to 1.6;
+    k = 255 1.3 to 4."""
+    return 0 < k <= 60 or (k <= 128 and N >= 4000) or (k <= 200 and Q <= 512)
+
+
 def topk(scores, k, chunk=1 << 15):
     """Row-wise top-k over a [Q, N] f32 score matrix.
 
     GPU: chunks of scores by workgroups, then rounds over the candidates.
-    Up to k = 256 a workgroup holds its chunk of 8192 in registers; beyond, a
-    radix select reads chunks of `chunk` (the 32k default keeps the grid >=
-    1024 workgroups even for a few queries).
+    Chunks of 8192 in registers for small k (_topk_in_registers); else a radix
+    select reads chunks of `chunk` (the 32k default keeps the grid >= 1024
+    workgroups even for a few queries).
     Returns (values [Q,k] f32 desc-sorted, indices [Q,k] int32).
     """
     if scores.is_cuda:
         _require_hip()
         Q, N = scores.shape
         k_eff = min(k, N)
-        few = 0 < k_eff <= 256
+        few = k_eff > 0 and _topk_in_registers(Q, N, k_eff)
         if few:
             chunk = min(chunk, 8192)
-        v, i = _hip_ops.topk_chunked(scores.contiguous(), None, k_eff, chunk)
+        v, i = _hip_ops.topk_chunked(scores.contiguous(), None, k_eff, chunk,
+                                     few)
         while v.shape[1] > k_eff:  # candidates of several chunks
             v, i = _hip_ops.topk_chunked(
-                v, i, k_eff, 8192 if few else v.shape[1])
+                v, i, k_eff, 8192 if few else v.shape[1], few)
         if k_eff < k:
             pad_v = torch.full((Q, k - k_eff), float("-inf"),
                                device=v.device)

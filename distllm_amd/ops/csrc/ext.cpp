@@ -40,7 +40,7 @@ int score_tile(int);
 void launch_score(const float*, void*, const float*, float*, int, int, int,
                   hipStream_t);
 void launch_topk_chunk(const float*, const int*, float*, int*, int, long, int,
-                       int, hipStream_t);
+                       int, bool, hipStream_t);
 void launch_hamming_score(const void*, const void*, float*, int, long, int,
                           hipStream_t);
 void launch_ivf_score(const void*, const int*, const int*, const float*,
@@ -384,8 +384,12 @@ torch::Tensor score(torch::Tensor q, torch::Tensor corpus) {
 
 std::vector<torch::Tensor> topk_chunked(torch::Tensor scores,
                                         c10::optional<torch::Tensor> in_idx,
-                                        int64_t k, int64_t chunk) {
+                                        int64_t k, int64_t chunk, bool regs) {
+  // regs: a workgroup holds its chunk in registers; else it is read by rounds
+  // of a radix select
   CHECK_DEV(scores); CHECK_CONT(scores); CHECK_F32(scores);
+  TORCH_CHECK(!regs || (chunk > 0 && chunk <= 8192 && k > 0 && k <= 256),
+              "chunks of up to 8192 scores and k up to 256 in registers");
   const int Q = scores.size(0);
   const long N = scores.size(1);
   const int nchunks = (int)((N + chunk - 1) / chunk);
@@ -396,7 +400,7 @@ std::vector<torch::Tensor> topk_chunked(torch::Tensor scores,
   launch_topk_chunk(scores.data_ptr<float>(),
                     in_idx ? in_idx->data_ptr<int>() : nullptr,
                     ov.data_ptr<float>(), oi.data_ptr<int>(), Q, N, (int)chunk,
-                    (int)k, cur_stream());
+                    (int)k, regs, cur_stream());
   return {ov, oi};
 }
 
@@ -666,7 +670,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("key_bias", &key_bias);
   m.def("bert_few_rows", &bert_few_rows);
   m.def("score", &score);
-  m.def("topk_chunked", &topk_chunked);
+  m.def("topk_chunked", &topk_chunked, py::arg("scores"), py::arg("in_idx"),
+        py::arg("k"), py::arg("chunk"), py::arg("regs") = false);
   m.def("hamming_score", &hamming_score);
   m.def("ivf_score", &ivf_score);
   m.def("gemv_fp8", &gemv_fp8, py::arg("x"), py::arg("wq"),

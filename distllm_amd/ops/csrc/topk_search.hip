@@ -7,7 +7,7 @@
 //   topk_chunk_kernel -> per-chunk candidates
 //   topk over concatenated candidates (same kernel, with idx indirection)
 //
-// topk_regs_kernel takes k <= 256; beyond it,
+// topk_regs_kernel takes small k (the caller's choice); beyond,
 // topk_chunk_kernel: one 256-thread block per (query, chunk). Two-round
 // 8-bit radix select over monotonic uint32 keys finds a threshold, a
 // compact pass gathers candidates (cap 2048) into LDS, a bitonic sort
@@ -146,7 +146,7 @@ topk_chunk_kernel(const float* __restrict__ scores,
 // holds in registers: the scores are read once, and no histogram is needed as
 // long as scores are not piled up (a histogram of scores of one magnitude is a
 // chain of conflicting atomics). The k-th largest of the 256 threads' largest
-// scores (k <= 64: of those of 64 fours of threads) bounds the k-th largest of
+// scores (k <= 60: of those of 64 fours of threads) bounds the k-th largest of
 // the chunk from below; what reaches it is gathered and ranked, by score and,
 // among equals, by place. If more than the candidate buffer holds reach it (few
 // threads have all the large scores, or many scores are equal), the k-th
@@ -154,7 +154,9 @@ topk_chunk_kernel(const float* __restrict__ scores,
 // of their places. (topk_chunk_kernel leaves the order of equals open.)
 // Bound by reading the scores: 256 x 250000, k = 10, both rounds, 210 -> 61 us
 // (4.2 TB/s); 1 x 250000, k = 5, which had 8 workgroups and now has 31, 110 ->
-// 14 us. (Ranking all 256 threads' largest for any k: 167 and 35 us.)
+// 14 us. (Ranking all 256 threads' largest for any k: 167 and 35 us.) The bound
+// is a poor one when k comes near the number that it is taken of: hundreds of
+// scores reach it, and each is compared with all of them.
 #define TR_CHUNK 8192
 #define TR_CAP 1024
 
@@ -187,7 +189,7 @@ topk_regs_kernel(const float* __restrict__ scores,
   if (tid == 0) ncand = 0;
   __syncthreads();
   // every rank is taken once
-  if (k <= 64) {  // of 64 fours of threads, on the lanes of one wave
+  if (k <= 60) {  // of 64 fours of threads, on the lanes of one wave
     if (tid < 64) {
       const unsigned int four = max(max(top[tid], top[tid + 64]),
                                     max(top[tid + 128], top[tid + 192]));
@@ -309,10 +311,11 @@ topk_regs_kernel(const float* __restrict__ scores,
 
 extern "C" void launch_topk_chunk(const float* scores, const int* in_idx,
                                   float* out_v, int* out_i, int Qn, long N,
-                                  int chunk, int k, hipStream_t stream) {
+                                  int chunk, int k, bool regs,
+                                  hipStream_t stream) {
   const int nchunks = (int)((N + chunk - 1) / chunk);
   dim3 grid(nchunks, Qn);
-  if (chunk <= TR_CHUNK && k <= 256) {
+  if (regs) {  // chunk <= TR_CHUNK, k <= 256
     hipLaunchKernelGGL(topk_regs_kernel, grid, dim3(256), 0, stream, scores,
                        in_idx, out_v, out_i, N, chunk, k, nchunks);
     return;

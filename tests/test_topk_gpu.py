@@ -27,6 +27,22 @@ def test_sizes(device, N, k):
     _check(torch.randn(3, N, device=device, generator=g), k)
 
 
+@pytest.mark.parametrize("k", [59, 60, 61, 64, 65, 128, 129, 200, 201])
+@pytest.mark.parametrize("Q, N", [(3, 300), (3, 9000), (512, 300),
+                                  (513, 300), (513, 3999), (513, 4000)])
+def test_rule(device, Q, N, k):
+    """Both sides of where the form changes."""
+    g = torch.Generator(device=device).manual_seed(N + k)
+    _check(torch.randn(Q, N, device=device, generator=g), k)
+
+
+def test_refusals(device):
+    s = torch.randn(2, 20000, device=device)
+    for k, chunk in ((257, 8192), (0, 8192), (5, 8193), (5, 0)):
+        with pytest.raises(RuntimeError):
+            ops._hip_ops.topk_chunked(s, None, k, chunk, True)
+
+
 @pytest.mark.parametrize("k", [1, 10, 256])
 def test_few_threads_have_the_large_scores(device, k):
     """All large scores at places of one residue mod 256: far more than the
@@ -58,7 +74,7 @@ def test_equal_scores_by_place(device):
     assert i[0].tolist() == [100, 600, 1100, 1600, 2100]
 
 
-@pytest.mark.parametrize("k", [1, 7, 48, 100])
+@pytest.mark.parametrize("k", [1, 7, 60, 61, 100, 200])
 @pytest.mark.parametrize("N", [5000, 8192, 30000])
 def test_many_equal_scores_by_place(device, N, k):
     """Also among more equals than the buffer of candidates holds, with and
