@@ -625,20 +625,40 @@ def gateup_swiglu_fp8(x, wq, scale, bias=None):
 rope_tables = torch_ref.rope_tables
 
 
+def _score_fills(Q, N, K):
+    """Whether the tiles of score.hip (64, 128 or 256 queries by 128 rows, a
+    workgroup each) use the card well enough: by rounds of 256 of them, the
+    share of the scores among what the rounds could make. Measured against the
+    library's product over 33 to 1000 queries, 8000 to 250000 rows, K of 64 to
+    4096, own time over its: from 65 queries on a share of 0.55 and more 0.55 to
+    1.08, of 0.4 to 0.55 0.55 to 1.4, below up to 1.6; up to 64, where both are
+    bound by the rows, of 0.65 and more 0.65 to 1.0, 63 of 20000 x 4096 (0.6)
+    1.39, 33 of 16384 x 4096 1.75. Short sums, which the library's launches cost
+    more: up to 64 queries at K <= 384 0.45 to 1.0, one tile of queries at K <=
+    128 of up to 66000 rows 0.45 to 0.95. Fewer than 128 workgroups were not
+    worth it at all."""
+    tile = 64 if Q <= 64 else 128 if Q <= 128 else 256
+    wgs = -(-Q // tile) * -(-N // 128)
+    if wgs < 128:
+        return False
+    share = Q * N / (-(-wgs // 256) * 256 * tile * 128)
+    return (share >= (0.65 if Q <= 64 else 0.55) or (Q <= 64 and K <= 384)
+            or (Q <= 256 and K <= 128 and N <= 1 << 16))
+
+
 def score(q, corpus):
     """q [Q, K] against the rows of corpus [N, K], float32.
 
-    From 33 queries on, and where tiles of up to 256 queries by 128 rows fill
-    half of the card, the product of score.hip; else the library's. Measured
-    against 250000 rows of 768, us, library and own: 32 queries 168, 171; 64
-    214, 185; 128 404, 279; 256 716, 487; 256 against 20000 68, 59; 300
-    against 5000 (80 tiles) 34, 59."""
+    From 33 queries on, and where its tiles fill the card (_score_fills), the
+    product of score.hip; else the library's. Measured against 250000 rows of
+    768, us, library and own: 32 queries 168, 171; 64 214, 185; 128 404, 279;
+    256 716, 487."""
     Q, K = q.shape
     N = corpus.shape[0]
     if (q.is_cuda and q.device == corpus.device and 32 < Q < 1 << 20
             and q.dtype == corpus.dtype == torch.float32
             and K % 32 == 0 and 32 <= K < 1 << 20 and N <= (1 << 31) - 256
-            and -(-Q // 256) * -(-N // 128) >= 128 and Q * N < 1 << 39
+            and Q * N < 1 << 39 and _score_fills(Q, N, K)
             and corpus.is_contiguous() and q.is_contiguous()
             and q.data_ptr() % 16 == 0 and corpus.data_ptr() % 16 == 0):
         _require_hip()

@@ -33,8 +33,8 @@ class _OnGpu:
 
     is_cuda, dtype = True, torch.float32
 
-    def __init__(self, rows, device):
-        self.shape, self.device = (rows, 64), torch.device(device)
+    def __init__(self, rows, device="cuda:0", columns=64):
+        self.shape, self.device = (rows, columns), torch.device(device)
 
     def is_contiguous(self):
         return True
@@ -77,3 +77,17 @@ def test_score_of_as_many_rows_as_32_bits_count(kernels):
     assert ops.score(q, _OnGpu((1 << 31) - 256, "cuda:0")) == "kernel"
     for n in ((1 << 31) - 255, (1 << 31) - 1, 1 << 31):
         assert ops.score(q, _OnGpu(n, "cuda:0")) == "product"
+
+
+@pytest.mark.parametrize("Q, N, K, way", [
+    (256, 250000, 768, "kernel"), (128, 250000, 768, "kernel"),
+    (64, 250000, 768, "kernel"), (129, 250000, 768, "product"),
+    (257, 250000, 768, "product"), (33, 20000, 1024, "product"),
+    (33, 20000, 384, "kernel"), (64, 16384, 4096, "product"),
+    (64, 20000, 1024, "product"), (64, 50000, 1024, "kernel"),
+    (129, 20000, 128, "kernel"), (257, 20000, 128, "product"),
+    (129, 250000, 128, "product"),
+    (400, 5000, 64, "product"), (1000, 20000, 768, "kernel"),
+    (32, 250000, 768, "product")])
+def test_score_where_tiles_fill_the_card(kernels, Q, N, K, way):
+    assert ops.score(_OnGpu(Q, columns=K), _OnGpu(N, columns=K)) == way
