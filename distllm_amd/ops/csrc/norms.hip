@@ -193,12 +193,19 @@ norm_fwd_small_kernel(const unsigned short* __restrict__ x,
   }
 }
 
-// Up to how many rows each takes a workgroup. Measured in a graph with
-// residual and sum, us, workgroup and wave per row: 64 rows of 768 2.6 and
-// 3.3, of 4096 3.4 and 6.6, of 8192 4.6 and 11.1; 1024 rows 3.2 and 3.7, 6.0
-// and 8.2, 9.4 and 17.0; 2048 rows 4.2 and 4.3, 9.2 and 11.5, 15.7 and 20.4;
-// 4096 rows 6.4 and 5.5, 16.1 and 20.7, 30.3 and 37.9.
-#define NORM_ROWS_BLOCK 2048
+// Whether a row gets a workgroup: few rows leave most CUs without a wave, wide
+// rows leave a wave with many loads; narrow ones leave most of a workgroup's
+// threads without any. Measured in a graph with residual and sum, us, workgroup
+// and wave per row: 64 rows of 768 2.6 and 3.3, of 4096 3.4 and 6.6, of 8192
+// 4.6 and 11.1; 2048 rows of 128 3.1 and 2.4, of 512 3.4 and 2.8, of 640 1.03
+// times the wave's, of 768 4.2 and 4.3, of 4096 9.2 and 11.5, of 8192 15.7 and
+// 20.4; 4096 rows of 768 6.4 and 5.5, of 4096 16.1 and 20.7, of 8192 30.3 and
+// 37.9. Widths up to 512 are within 4% of each other up to 1024 rows; 3072 to
+// 65536 rows of 2048 are 0.91 to 1.14 of the wave's time, of 3072 0.87 to 1.00,
+// of 4096 0.83 to 0.96, of 5120 and 8192 0.79 to 0.92.
+static bool norm_row_block(int n_rows, int H) {
+  return n_rows <= 8 || (H > 512 && n_rows <= 2048) || H >= 3072;
+}
 
 extern "C" void launch_norm_fwd(const void* x, const void* res, const void* w,
                                 const void* b, void* out, void* sum_out,
@@ -216,7 +223,7 @@ extern "C" void launch_norm_fwd(const void* x, const void* res, const void* w,
   int blocks = min((n_rows + 3) / 4, cap);
   bool has_res = res != nullptr;
   bool write_sum = sum_out != nullptr;
-  const bool small = n_rows <= NORM_ROWS_BLOCK;
+  const bool small = norm_row_block(n_rows, H);
   int ncl = small ? (H / 8 + 255) / 256 : (H / 8 + WAVE - 1) / WAVE;
 
 #define DISPATCH3(NCL, HR, WS, RM)                                             \

@@ -1,5 +1,5 @@
-"""Residual norms on both sides of the row count where a row gets a wave
-instead of a workgroup, at sizes of one and of many loads a thread."""
+"""Residual norms on both sides of where a row gets a wave instead of a
+workgroup, at sizes of one and of many loads a thread."""
 
 import pytest
 import torch
@@ -11,8 +11,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("rms", [False, True])
-@pytest.mark.parametrize("H", [8, 768, 2056, 4096, 8192])
-@pytest.mark.parametrize("rows", [9, 2048, 2049])
+@pytest.mark.parametrize("H", [8, 512, 520, 768, 2056, 3064, 3072, 4096, 8192])
+@pytest.mark.parametrize("rows", [8, 9, 2048, 2049])
 def test_rows(device, rows, H, rms):
     g = torch.Generator(device=device).manual_seed(rows + H)
     x, r = (torch.randn(rows, H, device=device, generator=g)
