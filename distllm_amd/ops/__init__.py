@@ -188,11 +188,16 @@ _DECODE_ACT = {ACT_NONE: 0, ACT_GELU_TANH: 6, ACT_GELU_ERF: 7, ACT_SILU: 8}
 def _few_rows(x2, weight, bias=None, columns=64):
     """Whether a product of x2 with the rows of weight (in multiples of
     `columns`) and an activation in the same launch takes decode_gemm
-    (csrc/decode_gemm.hip): up to 64 rows it is faster than the library's
-    product at every size measured (64 rows of 28672 x 4096, gated: 51 against
-    57 us; 768 x 768: 3.8 against 7), up to 256 where the product is narrow
-    enough for the launch that it saves to count (128 rows of 16384 x 2048,
-    gated: 20 against 23 us, of 28672 x 4096: 64 against 59). K of a single 64-wide chunk, which would leave three of a
+    (csrc/decode_gemm.hip). Up to 64 rows: measured against the library's
+    product, 64 rows of 28672 x 4096, gated, 51 and 57 us, of 768 x 768 3.8 and
+    7; the slowest gated one of 14 sizes is 16384 x 8192 (61 and 56). Up to 256
+    rows of up to 16384 columns, in which gate and up-projection reach the
+    activation in 32 bits: against the library's product and the unit as a
+    launch of its own, which round them to 16 in between, 128 rows of 16384 x
+    1024 9.8 and 14, of 8192 x 2048 14 and 16, of 4096 x 1024 10.6 and 11.8, of
+    2048 x 1024 9.1 and 8.1; 256 rows 13.7 and 19, 21 and 23, 15 and 11.7, 12.5
+    and 11.1. Wider ones are the library's above 64 rows (28672 x 4096, 128 rows:
+    64 and 58). K of a single 64-wide chunk, which would leave three of a
     workgroup's four waves idle, keeps its general path."""
     M, K = x2.shape
     N = weight.shape[0]
@@ -210,6 +215,14 @@ def _few_rows(x2, weight, bias=None, columns=64):
 _OTHER_FORMS = ("blaslt", "gemm8", "gemm16")
 
 
+def _wide_logits(M, N, K) -> bool:
+    """Columns of a vocabulary, for which decode_gemm and the library take
+    turns from 17 rows on (64 rows, us: 151936 x 4096 269 and 237, 128256 x
+    4096 223 and 200, 250000 x 1536 176 and 161, 151936 x 2048 139 and 152): the
+    choice is measured."""
+    return M > 16 and N > 32768 and K >= 1536
+
+
 def _gemm_mode() -> str:
     return os.environ.get("DISTLLM_GEMM", "auto")
 
@@ -218,8 +231,8 @@ def linear(x, weight, bias=None, act=ACT_NONE):
     """Linear layer entry used by models. GPU path: autotuned choice
     between hipBLASLt (plain and fused-epilogue) and the hand-written
     MFMA GEMMs (gemm8.hip, 8-phase gemm16.hip); the products of few rows
-    (decode_gemm.hip, with the activation) for M <= 64 and among the
-    choices for M <= 256. Override with
+    (decode_gemm.hip, with the activation) for M <= 64 (_few_rows) and
+    among the choices for M <= 256. Override with
     DISTLLM_GEMM=blaslt|gemm8|gemm16|decode (the last for M <= 256, gemm8 and
     gemm16 at their multiples of 256 rows; without an activation M <= 256
     stays a choice for those two, at other sizes they mean the library)."""
@@ -233,6 +246,7 @@ def linear(x, weight, bias=None, act=ACT_NONE):
         if x2.dtype == torch.float32:  # true 32-bit products
             mode = "blaslt"
         if (mode not in _OTHER_FORMS and M <= 64
+                and not (act == ACT_NONE and _wide_logits(M, N, K))
                 and _few_rows(x2, weight, bias)):
             out = _hip_ops.decode_gemm(x2, weight, bias, 0, _DECODE_ACT[act])
             return out.reshape(*orig_shape[:-1], N)

@@ -10,9 +10,9 @@
 // operand wants, takes it 64 cycles for 1 KiB where whole lines take 16, and
 // 6 TB/s leave about 100 cycles per KiB of weights.
 //
-//  ring    M <= 16, and up to 64 where columns are few. A workgroup has 16
-//          columns (rows of W) and its 4 waves take the 64-wide chunks of K
-//          in turn; W and x pass through a ring of LDS buffers that belongs
+//  ring    M <= 16 but for many columns of a short K, and up to 64 where
+//          columns are few. A workgroup has 16 columns (rows of W) and its 4
+//          waves take the 64-wide chunks of K in turn; W and x pass through a ring of LDS buffers that belongs
 //          to the wave alone: whole lines by global_load_lds, counted waits,
 //          no barriers. The waves' sums meet in LDS: no slabs, no second
 //          launch. (W straight to operand registers is 2% faster for one row
@@ -483,6 +483,16 @@ static bool dg_few_columns(int rows, int N, int K) {
          (long)N * K <= (rows <= 32 ? 4096L * 4096 : 4096L * 1536);
 }
 
+// Whether up to 16 rows take the tile form: a ring's workgroup has 16 columns,
+// and with many columns of a short K it has hardly begun when it ends. Measured,
+// ring and tile, us, 1 to 16 rows: 16384 x 128 4 and 3, 128256 x 128 19 and 9,
+// 250000 x 256 53 and 28, 151936 x 512 42 and 31, 65536 x 768 20 to 22 and 18,
+// 250000 x 1024 89 to 112 and 91, 65536 x 1536 34 to 41 and 38, 151936 x 1536 73
+// to 95 and 87, 151936 x 2048 103 to 115 and 116.
+static bool dg_short_sums(int rows, int N, int K) {
+  return N >= 16384 && K <= (rows <= 8 ? 1024 : 1536);
+}
+
 // How many workgroups share K in the tile form: the least that give 150 of
 // them, each with at least 384 of K (48 rows, in us: 4096 x 4096 2 shares
 // 15.1, 4 shares 12.0, 8 shares 13.7; 4096 x 14336 39, 26.7, 29.5; 5120 x
@@ -508,7 +518,7 @@ static void dg_launch(const u16* X, const u16* W, float* slabs, int K,
                      dim3(e.N / (NT * 16)), dim3(256),                       \
                      dg_ring_lds(MT, NT, 4, R), st, X, W, K, e)
   // two rows of W per stage: three stages let two workgroups share a CU
-  if (!tile && e.M <= 16) {
+  if (!tile && e.M <= 16 && !dg_short_sums(e.M, e.N, K)) {
     DG_RING(1, GLU ? 3 : 4);
     return;
   }

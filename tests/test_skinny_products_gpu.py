@@ -141,3 +141,28 @@ def test_bias_sizes(device, M, act):
     want = torch_ref.gemm(x.float(), w.float(), b[:1].float().expand(192),
                           act).float()
     _close(ops.linear(x, w, b[:1].contiguous(), act), want)
+
+
+@pytest.mark.parametrize("M", [1, 8, 9, 16, 17])
+@pytest.mark.parametrize("N,K", [(16320, 128), (16384, 128), (16384, 1024),
+                                 (16384, 1088), (16448, 1536), (16384, 1600)])
+def test_short_sums(device, M, N, K):
+    """Both sides of where up to 16 rows leave the ring."""
+    x, w, b = _inputs(M, N, K, device, M * N + K)
+    ref = x.float() @ w.float().T + b.float()
+    _close(ops.linear(x, w, b), ref)
+    _close(ops.linear(x, w, b, ops.ACT_GELU_ERF),
+           torch.nn.functional.gelu(ref))
+
+
+def test_vocabulary(device, monkeypatch):
+    """The choice for wide products without an activation is measured."""
+    monkeypatch.setattr(ops, "_GEMM_CHOICE", {})
+    for M, N, K, measured in ((16, 32832, 1536, 0), (17, 32768, 1536, 0),
+                              (17, 32832, 1472, 0), (17, 32832, 1536, 1),
+                              (64, 32832, 1536, 1)):
+        x, w, b = _inputs(M, N, K, device, M)
+        _close(ops.linear(x, w, b), x.float() @ w.float().T + b.float())
+        assert len(ops._GEMM_CHOICE) == measured
+        ops.linear(x, w, b, ops.ACT_SILU)
+        assert len(ops._GEMM_CHOICE) == measured
