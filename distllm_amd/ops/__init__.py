@@ -380,8 +380,11 @@ def norm_linear(a, b, w_norm, eps, weight, bias=None, gated=False,
 
 
 def norm_linear_fp8(a, b, w_norm, eps, wq, scale, bias=None, gated=False):
-    """norm_linear on weights quantized as for gemv_fp8."""
-    if wq.shape[1] % 128 == 0 and _norm_in_product(a, b, w_norm, wq, 2560):
+    """norm_linear on weights quantized as for gemv_fp8 (but for the few
+    columns of a long K that gemv_fp8 takes by column)."""
+    N, K = wq.shape
+    if (K % 128 == 0 and (gated or N > 512 or K < 4096)
+            and _norm_in_product(a, b, w_norm, wq, 2560)):
         _require_hip()
         return tuple(_hip_ops.gemv_fp8_norm(a, b, w_norm, eps, wq, scale,
                                             bias, gated))

@@ -12,10 +12,11 @@
 // unit 16 gate and the 16 up columns), its 4 waves take the 128-wide chunks of
 // K in turn, W (2 KiB a chunk) and x (4 or 8 rows) pass through LDS buffers of
 // the wave's own by global_load_lds, three or four chunks ahead, and W is widened
-// to bf16 (exact) on its way to the MFMA. The vector-unit kernel below it, a wave per
-// column with one 16-byte load a lane in flight, keeps the other K. Measured
-// in a decode graph, us: 28672 x 4096 with swiglu 31 + 5 -> 24.6, 4096 x 14336
-// and 4096 x 4096 together 29 -> 19, 6144 x 4096 9.8 -> 7.6.
+// to bf16 (exact) on its way to the MFMA. The vector-unit kernel above it, a
+// wave per column with one 16-byte load a lane in flight, keeps the other K and
+// one row of few columns. Measured in a decode graph, us: 28672 x 4096 with
+// swiglu 31 + 5 -> 24.6, 4096 x 14336 and 4096 x 4096 together 29 -> 19, 6144 x
+// 4096 9.8 -> 7.6.
 // Reference anchor: the vLLM latency role the reference delegated
 // (distllm/generate/generators/vllm_backend.py:62-93).
 #include <hip/hip_fp8.h>
@@ -354,7 +355,11 @@ extern "C" void launch_gemv_fp8(const void* X, const void* W,
     else GVR(true, 8);
     return;
   }
-  if (K % 128 == 0) {
+  // One row and few columns of a long K: the ring's 16 columns a workgroup leave
+  // most CUs without one, a wave per column does not. us, ring and column: 512 x
+  // 4096 4.5 and 4.1, x 8192 7.2 and 5.9, x 16384 12.7 and 11.0; 64 x 28672 20.4
+  // and 14.4; two rows the same or slower by column.
+  if (K % 128 == 0 && !(M == 1 && N <= 512 && K >= 4096)) {
     if (M <= 4) GVR(false, 4);
     else GVR(false, 8);
     return;

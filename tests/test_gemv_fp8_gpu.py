@@ -41,3 +41,13 @@ def test_gated(device, M, I, K):
     out = ops.gateup_swiglu_fp8(x, wq, s)
     want = torch.nn.functional.silu(z[:, :I]) * z[:, I:]
     torch.testing.assert_close(out.float(), want, atol=2e-2, rtol=1.6e-2)
+
+
+@pytest.mark.parametrize("N,K", [(512, 4096), (513, 4096), (512, 3968),
+                                 (5, 16384), (3, 4224)])
+@pytest.mark.parametrize("M", [1, 2])
+def test_few_columns(device, M, N, K):
+    """Both sides of where one row goes by column."""
+    x, wq, s, z = _inputs(M, N, K, device)
+    b = torch.randn(N, device=device).to(torch.bfloat16)
+    _close(ops.gemv_fp8(x, wq, s, b), z + b.float())
