@@ -64,9 +64,10 @@ __device__ __forceinline__ void wave_sync() {
 // wait for every copy that it knows to be in flight, also those into other
 // buffers. So nothing waits by itself, __syncthreads() neither: the caller
 // counts its copies and waits (s_waitcnt vmcnt) before a barrier or a read of
-// the bytes. M0 is a register that the compiler keeps to itself and does not
-// save around assembly: nothing else in the kernels that use this needs it (no
-// copies by the builtin beside these).
+// the bytes. M0 is reserved: the compiler sets it ahead of each of its own uses
+// and neither keeps nor expects anything in it across assembly, for which a
+// clobber would do nothing but warn. (Copies by the builtin would be such uses;
+// the kernels that take this have none.)
 template <int BYTES = 16>
 __device__ __forceinline__ void copy_to_lds(const void* src,
                                             const void* base) {
@@ -81,7 +82,7 @@ __device__ __forceinline__ void copy_to_lds(const void* src,
         "global_load_lds_dwordx4 %1, off"
         :
         : "s"(at), "v"(src)
-        : "memory", "m0");
+        : "memory");
   else
     asm volatile(
         "s_mov_b32 m0, %0\n\t"
@@ -89,7 +90,7 @@ __device__ __forceinline__ void copy_to_lds(const void* src,
         "global_load_lds_dword %1, off"
         :
         : "s"(at), "v"(src)
-        : "memory", "m0");
+        : "memory");
 }
 
 // 16 bytes at any address
