@@ -88,15 +88,16 @@ mean_pool_kernel(const unsigned short* __restrict__ hidden,
       parts[(long)blockIdx.x * H + c] = sums[c];
     return;
   }
-  const float inv = 1.f / fmaxf((float)L - 2.f, 1.f);
+  // (a quotient, rounded once; a product with 1 / count is rounded twice more)
+  const float count = fmaxf((float)L - 2.f, 1.f);
   float sq = 0.f;
   for (int c = threadIdx.x; c < H; c += 256) {
-    const float m = sums[c] * inv;
+    const float m = sums[c] / count;
+    sums[c] = m;
     sq += m * m;
   }
-  float scale = inv;
-  if (normalize)
-    scale *= rsqrtf(fmaxf(block_reduce_sum<4>(sq, lds), 1e-24f));
+  const float scale =
+      normalize ? rsqrtf(fmaxf(block_reduce_sum<4>(sq, lds), 1e-24f)) : 1.f;
   for (int c = threadIdx.x; c < H; c += 256)
     out[(long)r * H + c] = sums[c] * scale;
 }
@@ -111,18 +112,18 @@ mean_join_kernel(const float* __restrict__ parts, const int* __restrict__ mask,
   int lsum = 0;
   for (int s = threadIdx.x; s < S; s += 256) lsum += mask[(long)r * S + s];
   const int L = (int)(block_reduce_sum<4>((float)lsum, lds) + 0.5f);
-  const float inv = 1.f / fmaxf((float)L - 2.f, 1.f);
+  const float count = fmaxf((float)L - 2.f, 1.f);
   float sq = 0.f;
   for (int c = threadIdx.x; c < H; c += 256) {
     float m = 0.f;
 #pragma unroll 4
     for (int p = 0; p < NS; ++p) m += parts[((long)r * NS + p) * H + c];
+    m /= count;
     sums[c] = m;
-    sq += m * inv * (m * inv);
+    sq += m * m;
   }
-  float scale = inv;
-  if (normalize)
-    scale *= rsqrtf(fmaxf(block_reduce_sum<4>(sq, lds), 1e-24f));
+  const float scale =
+      normalize ? rsqrtf(fmaxf(block_reduce_sum<4>(sq, lds), 1e-24f)) : 1.f;
   for (int c = threadIdx.x; c < H; c += 256)
     out[(long)r * H + c] = sums[c] * scale;
 }

@@ -88,3 +88,13 @@ def test_mean_pool(device, R, S, H, normalize):
         want = torch.nn.functional.normalize(want, dim=-1)
     # fp32 sums of up to 700 numbers of unit size
     torch.testing.assert_close(got.double(), want, atol=2e-6, rtol=2e-5)
+
+
+@pytest.mark.parametrize("R,S", [(1, 9), (3, 40), (2, 300), (600, 24)])
+def test_mean_pool_is_rounded_once(device, R, S):
+    """Sums of small whole numbers have no error, so a mean is their quotient
+    to the last bit."""
+    x = torch.randint(-99, 100, (R, S, 320), device=device).to(torch.bfloat16)
+    mask = torch.ones(R, S, device=device, dtype=torch.int32)
+    total = x[:, 1:-1].double().sum(1)
+    assert torch.equal(ops.mean_pool(x, mask), (total / (S - 2)).float())
