@@ -232,8 +232,8 @@ torch::Tensor latent_attn(torch::Tensor q, torch::Tensor cache,
   // buffers take a CU's LDS; more than fit would be a second round), as long
   // as a share keeps two tiles of 64 keys; four tiles are not worth the second
   // launch. Measured at rank 512, 32 heads, us: 16 rows of 100 to 4000 keys
-  // 12 shares 28, 16 25, 24 35; 32 rows of 300 to 2048 4 30, 8 25, 12 32; 64
-  // rows of 60 to 200 1 14, 2 16, 4 17; 1 row of 2048 8 17.6, 16 16.2, 32 18.
+  // 12 shares 29, 16 25.5, 24 32; 32 rows of 300 to 2048 4 31, 8 25.5, 12 32; 64
+  // rows of 60 to 200 1 13, 2 15, 4 17; 1 row of 2048 8 19.0, 16 16.6, 32 18.2.
   // All sizes are known on the host, so a captured graph stays valid as
   // contexts grow.
   long NS = nsplit;

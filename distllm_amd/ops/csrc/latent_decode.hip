@@ -14,7 +14,11 @@
 //  - scores: each of the 4 waves of a head group has 16 keys (one page) and
 //    a softmax state of its own;
 //  - the waves exchange their weights and maxima through LDS;
-//  - output: each wave has R / 4 latent columns, for all keys.
+//  - output: each wave has R / 4 latent columns, for all keys. A weight goes in
+//    as the sum of two bf16 numbers: with one, a tile of 64 keys, which has
+//    fewer weights of exactly 1 than two of 32 had, was 0.3 to 1.3% further off
+//    64 bits than those (2.0e-3 of the result; with two 1.66e-3, what its own
+//    rounding leaves). Up to 11% of the kernel at many keys.
 // Both products are mfma_f32_16x16x32_bf16 with keys (then latent columns) as
 // rows and heads as columns, so that states and rescaling are lane-local; a
 // lane's weights of the exchange are its operand of the second product.
@@ -25,9 +29,9 @@
 // waits: 2.9 us a tile against 1.9. Tiles of 32 keys that passed through
 // registers and were kept twice, one copy transposed, with 64 heads in a
 // workgroup, took (rank 512, 32 heads, us, then and now) 1 row of 2048 keys
-// 28 -> 16, 32 rows of 300 to 2048 38 -> 25, 16 of 100 to 4000 47 -> 25, 64 of
-// 200 to 2000 44 -> 35; 64 heads: 32 rows of 2048 41 -> 34, 64 rows of 200 to
-// 2000 53 -> 51, for the second group of 32 heads reads the tiles from L2.
+// 28 -> 17, 32 rows of 300 to 2048 37 -> 25.5, 16 of 100 to 4000 46 -> 25.5, 64
+// of 200 to 2000 43 -> 36; 64 heads: 32 rows of 2048 40 -> 35, 64 rows of 200 to
+// 2000 51 -> 51, for the second group of 32 heads reads the tiles from L2.
 #include "common.h"
 
 #define PBLK 16
@@ -201,8 +205,8 @@ latent_decode_kernel(const unsigned short* __restrict__ q,
   if (ts + 1 >= te) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
   const float scale2 = scale * LOG2E;
-  float m = -1e30f;              // of the sums: the largest of all waves
-  float mw = -1e30f, lw = 0.f;   // of this wave's keys
+  float m = -1e30f, l = 0.f;  // of the sums, l: of this lane's keys
+  float mw = -1e30f;          // the largest of this wave's keys
   f32x4 acc[OB];
 #pragma unroll
   for (int i = 0; i < OB; ++i) acc[i] = {0.f, 0.f, 0.f, 0.f};
@@ -246,20 +250,15 @@ latent_decode_kernel(const unsigned short* __restrict__ q,
     }
     top = fmaxf(top, __shfl_xor(top, 16, 64));
     top = fmaxf(top, __shfl_xor(top, 32, 64));
-    const float mn = fmaxf(mw, top);
-    lw *= __builtin_amdgcn_exp2f(mw - mn);
-    mw = mn;
+    mw = fmaxf(mw, top);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      sc[r] = __builtin_amdgcn_exp2f(sc[r] - mn);
-      lw += sc[r];  // of the keys of this lane
-    }
+    for (int r = 0; r < 4; ++r) sc[r] = __builtin_amdgcn_exp2f(sc[r] - mw);
     *reinterpret_cast<f32x4*>(weights + (w * 64 + lane) * 4) = sc;
-    if (g == 0) maxima[w * 16 + c16] = mn;
+    if (g == 0) maxima[w * 16 + c16] = mw;
     ld_barrier();
 
     // all weights, relative to the largest maximum so far
-    ld_frag pf[2];
+    ld_frag pf[2], pl[2];  // high and low parts
     float mx[4], ma = m;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -269,6 +268,7 @@ latent_decode_kernel(const unsigned short* __restrict__ q,
     if (!__all(ma <= m)) {
       const float alpha = __builtin_amdgcn_exp2f(m - ma);
       m = ma;
+      l *= alpha;
 #pragma unroll
       for (int i = 0; i < OB; ++i)
 #pragma unroll
@@ -279,8 +279,16 @@ latent_decode_kernel(const unsigned short* __restrict__ q,
       const f32x4 p =
           *reinterpret_cast<const f32x4*>(weights + (i * 64 + lane) * 4);
       const float f = __builtin_amdgcn_exp2f(mx[i] - m);
-      pf[i >> 1].d[(i & 1) * 2] = ld_pack(p[0] * f, p[1] * f);
-      pf[i >> 1].d[(i & 1) * 2 + 1] = ld_pack(p[2] * f, p[3] * f);
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const float a = p[e * 2] * f, b = p[e * 2 + 1] * f;
+        l += a + b;
+        const unsigned int h = ld_pack(a, b);
+        pf[i >> 1].d[(i & 1) * 2 + e] = h;
+        pl[i >> 1].d[(i & 1) * 2 + e] =
+            ld_pack(a - __builtin_bit_cast(float, h << 16),
+                    b - __builtin_bit_cast(float, h & 0xffff0000u));
+      }
     }
     // keys 4 g .. 4 g + 3 of two pages at a time, as the weights lie
     const int vr = g * 4 + (c16 >> 2);
@@ -299,27 +307,18 @@ latent_decode_kernel(const unsigned short* __restrict__ q,
                   a + (kb * 2 + e) * (16 * R * 2)));
         acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf.v, pf[kb].v,
                                                          acc[i], 0, 0, 0);
+        acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf.v, pl[kb].v,
+                                                         acc[i], 0, 0, 0);
       }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
 
-  // sums of the weights of all waves
-  lw += __shfl_xor(lw, 16, 64);
-  lw += __shfl_xor(lw, 32, 64);
-  ld_barrier();
-  if (g == 0) {
-    weights[w * 16 + c16] = lw;
-    maxima[w * 16 + c16] = mw;
-  }
-  ld_barrier();
+  // (every wave has the weights of all keys)
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
   const int head = head0 + hg * 16 + c16;
   if (head >= H) return;
-  float l = 0.f;
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-    l += weights[i * 16 + c16] *
-         __builtin_amdgcn_exp2f(maxima[i * 16 + c16] - m);
   const long rh = (long)row * H + head;
   const int col = w * (OB * 16) + g * 4;
   if (NS == 1) {

@@ -1,5 +1,7 @@
 """Attention of single-token rows over paged latents at the edges of its
 tiles, shares and head groups, against float64."""
+import math
+
 import pytest
 import torch
 
@@ -89,3 +91,34 @@ def test_window_within_the_last_page(device, rank, rot, H):
                                   rank).cpu().double()
             bound = size * (2 ** -7 + 1e-4) + 1e-6  # as above
             assert ((got - want).abs() <= bound).all(), (window, nsplit)
+
+
+@pytest.mark.parametrize("H", [16, 40])
+@pytest.mark.parametrize("rank", [64, 512])
+@pytest.mark.parametrize("p", [2.0 ** -9 * 1.00390625 + 1e-6, 2 ** -9 * 1.0039])
+def test_weights_keep_more_than_bf16(device, rank, H, p):
+    """One large score of value -7 and thousands of the same small weight of
+    value 1: rounded to bf16 each is off by up to 2^-9 to the same side, which
+    is 3% of what is left of the sum."""
+    L = 4096
+    q = torch.zeros(1, H, rank + 64, dtype=BF16)
+    q[0, :, rank: rank + 3] = torch.tensor([1.0, 2 ** -8, 2 ** -14])
+    left = torch.full((L,), math.log(p), dtype=torch.float64)
+    left[0] = 0.0
+    score = torch.zeros_like(left)
+    cache = torch.zeros(L, rank + 64, dtype=BF16)
+    cache[:, :rank] = 1.0
+    cache[0, :rank] = -7.0
+    for i in range(3):
+        unit = q[0, 0, rank + i].item()
+        cache[:, rank + i] = ((left - score) / unit).to(BF16)
+        score += cache[:, rank + i].double() * unit
+    want = score.softmax(0) @ cache[:, 0].double()
+    bt = torch.arange(L // 16, dtype=torch.int32, device="cuda")[None]
+    got = ops.latent_attn(
+        q.cuda(), cache.view(-1, 16, rank + 64).cuda(), bt,
+        torch.zeros(1, dtype=torch.int32, device="cuda"),
+        torch.tensor([L], dtype=torch.int32, device="cuda"), 1 << 30, 1.0, 1,
+        rank).double().cpu()
+    # bf16 of the result and 2^-18 of parts of together 1
+    assert ((got - want).abs() <= abs(want) * 2 ** -8 + 2 ** -18).all()
