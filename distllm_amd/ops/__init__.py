@@ -202,7 +202,7 @@ def _few_rows(x2, weight, bias=None, columns=64):
     M, K = x2.shape
     N = weight.shape[0]
     return ((M <= 64 or (M <= 256 and N <= 16384))
-            and K % 64 == 0 and K >= 128 and N % columns == 0
+            and K % 64 == 0 and K >= 128 and N % columns == 0 and N > 0
             and x2.dtype == weight.dtype == torch.bfloat16
             and x2.is_contiguous() and weight.is_contiguous()
             and x2.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0

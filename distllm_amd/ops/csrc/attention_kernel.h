@@ -31,7 +31,7 @@
 // by LDS reads (32 KB per wave and tile). Measured, before (V transposed
 // through registers at D = 64, read element by element from memory at 128,
 // every score scaled and masked by itself) and now: 512 x 512 tokens, 12
-// heads of 64, masked 1341 -> 640 us (640 TFLOP/s); packed proteins of 64 to
+// heads of 64, masked 1240 -> 600 us (690 TFLOP/s); packed proteins of 64 to
 // 1024, 20 heads of 64, 248 -> 111 us; causal, 32 heads of 128 on 8,
 // 16 x 1024 536 -> 260 us and 4 x 4096 2354 -> 621 us (885 TFLOP/s); window
 // 1024 of 6 x 2048, 32 heads of 128, 370 -> 289 us. Four waves a SIMD at
@@ -276,8 +276,8 @@ attn_fwd_kernel(const unsigned short* __restrict__ Q,
   // that is not -inf in log2 units: the weight of those behind it is 0, their
   // tiles are left out. 64 x 203 with a quarter of the keys masked, 12 heads
   // of 64, 33 -> 27 us; 16 x 1024, 32 heads of 128, causal, 264 -> 234; with
-  // nothing masked 512 x 512 takes the same 690 as when a flag was read per
-  // tile, for what the tiles save the first look costs -------------------
+  // nothing masked 512 x 512 takes as long as when a flag was read per tile,
+  // for what the tiles save the first look costs ---------------------------
   if constexpr (HAS_MASK) {
     const float* mrow = maskp + (long)b * SKV;
     int live = 0;

@@ -109,7 +109,7 @@ static torch::Tensor decode_gemm_act(torch::Tensor X, torch::Tensor W,
     nums = act_nums->data_ptr<float>();
   }
   auto out = torch::empty({M, glu ? N / 2 : N}, X.options());
-  if (M == 0) return out;
+  if (out.numel() == 0) return out;
   X = aligned16(X);
   W = aligned16(W);
   torch::Tensor slabs;

@@ -166,3 +166,15 @@ def test_vocabulary(device, monkeypatch):
         assert len(ops._GEMM_CHOICE) == measured
         ops.linear(x, w, b, ops.ACT_SILU)
         assert len(ops._GEMM_CHOICE) == measured
+
+
+@pytest.mark.parametrize("act", [ops.ACT_NONE, ops.ACT_GELU_ERF])
+@pytest.mark.parametrize("M, N", [(0, 128), (5, 0), (0, 0)])
+def test_nothing_to_do(device, M, N, act):
+    x = torch.zeros(M, 128, device=device, dtype=torch.bfloat16)
+    w = torch.zeros(N, 128, device=device, dtype=torch.bfloat16)
+    assert ops._hip_ops.decode_gemm(x, w, None, 0).shape == (M, N)
+    if N:
+        assert ops.linear(x, w, None, act).shape == (M, N)
+        assert ops.gateup_swiglu(x, w).shape == (M, N // 2)
+    torch.cuda.synchronize()
