@@ -58,6 +58,19 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// The leading 8 bits of a and b, not negative, as bf16 numbers (a's in the low
+// half); a and b become what is left of them, or the least normal number where
+// nothing is, which counts for nothing in a sum but keeps a product with infinity
+// from being NaN.
+__device__ __forceinline__ unsigned int split_bf16(float& a, float& b) {
+  const unsigned int h = __builtin_amdgcn_perm(
+      __builtin_bit_cast(unsigned int, b), __builtin_bit_cast(unsigned int, a),
+      0x07060302);
+  a = fmaxf(a - __builtin_bit_cast(float, h << 16), 0x1p-126f);
+  b = fmaxf(b - __builtin_bit_cast(float, h & 0xffff0000u), 0x1p-126f);
+  return h;
+}
+
 // 16 or 4 bytes a lane from global memory to LDS: lane i's to base + i times
 // as many, base the same for the whole wave. In assembly, for the compiler
 // must not know of it: it lets a transposing read of LDS (ds_read_b64_tr_b16)

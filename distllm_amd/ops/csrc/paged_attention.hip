@@ -20,8 +20,10 @@
 //    way out of LDS. Softmax state and rescaling are lane-local but for the
 //    maximum over the four groups of lanes that share a head.
 //  - probabilities stay fp32: each goes in as the sum of three bf16 numbers,
-//    which is exactly it (two leave 2^-18 of it, and what two values that
-//    cancel leave can be less than that).
+//    which is exactly it (two leave 2^-17 of it, and what two values that
+//    cancel leave can be less than that). With bf16 pages no part is negative
+//    or, but for a first one, 0: an infinite value gives an infinite result. fp8
+//    has no infinities.
 //  - NS workgroups share a sequence where B * HKV is small; a second launch
 //    joins them.
 // Measured, us, with kernels that read a key row per lane and a value element
@@ -240,10 +242,14 @@ paged_attn_kernel(const unsigned short* __restrict__ q, long q_stride,
         l += p0 + p1;
 #pragma unroll
         for (int e = 0; e < 3; ++e) {
-          const unsigned int h = pa_pack(p0, p1);
-          part[e].d[kb * 2 + r / 2] = h;
-          p0 -= __builtin_bit_cast(float, h << 16);
-          p1 -= __builtin_bit_cast(float, h & 0xffff0000u);
+          if constexpr (FP8) {  // no infinities, and rounding costs less
+            const unsigned int h = pa_pack(p0, p1);
+            part[e].d[kb * 2 + r / 2] = h;
+            p0 -= __builtin_bit_cast(float, h << 16);
+            p1 -= __builtin_bit_cast(float, h & 0xffff0000u);
+          } else {
+            part[e].d[kb * 2 + r / 2] = split_bf16(p0, p1);
+          }
         }
       }
     // columns 16 d .. of V, keys 4 g .. 4 g + 3 of both halves: the order in

@@ -189,3 +189,24 @@ def test_rope_put(device, B, H, HKV, D, fp8):
             assert (got.int() - want.int()).abs().max() <= 1
         else:
             torch.testing.assert_close(got, want, atol=0, rtol=2 ** -7)
+
+
+@pytest.mark.parametrize("shares", ["1", "3"])
+@pytest.mark.parametrize("D", [64, 128])
+def test_infinite_values(device, D, shares, monkeypatch):
+    """Infinite values come out as from sums of 32 bits: infinite, with their
+    sign, and NaN only where both signs meet."""
+    monkeypatch.setenv("DISTLLM_PA_NSPLIT", shares)
+    lens = [200, 33, 16]
+    k, v, table = _pages(3, 2, D, lens, 13, False, 1, device, 0.0)
+    inf = float("inf")
+    for b, key, col, x in ((0, 7, 3, inf), (0, 190, 5, -inf), (1, 32, 0, inf),
+                           (2, 0, 9, inf), (2, 1, 9, -inf), (2, 3, 11, -inf)):
+        v[table[b, key // 16], :, key % 16, col] = x
+    # the largest probability is 1, whose low parts are nothing
+    q = torch.randn(3, 8, D, device=device).to(torch.bfloat16) * 0.2
+    ctx = torch.tensor(lens, dtype=torch.int32, device=device)
+    out = ops.paged_attn(q, k, v, table, ctx).float().cpu()
+    want = _want(q, k, v, table, lens, D ** -0.5)
+    assert torch.equal(out.isnan(), want.isnan()) and want.isnan().any()
+    torch.testing.assert_close(out, want, equal_nan=True, **TOL)
