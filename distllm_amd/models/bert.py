@@ -131,13 +131,12 @@ class BertEncoder(nn.Module):
 
         ids = input_ids.long()
         B, S = ids.shape
-        # BERT packed/varlen is opt-in only: on its realistic padded
-        # workloads (semantic-chunk buffers AND chunk re-embeds, 12
-        # light layers, ~200-400-token rows) the padded path measured
-        # FASTER (73 vs 47-50 docs/s on the pipeline bench) — the
-        # per-layer pack overheads beat the skipped pad FLOPs at this
-        # depth/width. The deep/wide ESM encoders auto-pack instead
-        # (x3.0 measured, profiles/RESULTS.md).
+        # Packed on request only. 64 texts of 40 to 203 tokens, 60% of the
+        # padded rows: 2.93 ms packed, 3.53 padded. An earlier attention
+        # made padded batches the faster ones (73 against 47-50 docs/s of
+        # semantic chunks); other lengths and shares of padding have not
+        # been measured since. The deep and wide ESM encoders pack by a rule
+        # of their own (x3.0 measured, profiles/RESULTS.md).
         if (ids.is_cuda and ops.HAVE_HIP and attention_mask is not None
                 and token_type_ids is None
                 and os.environ.get("DISTLLM_FORCE_VARLEN")):
