@@ -223,6 +223,19 @@ def _wide_logits(M, N, K) -> bool:
     return M > 16 and N > 32768 and K >= 1536
 
 
+# sizes (M, N, K, bias or not) of such products that ran with their choice
+_WIDE_RUN: set[tuple] = set()
+
+
+def _to_choose(M, N, K, bias) -> bool:
+    """Whether a product of up to 64 rows goes by the measured choice. While a
+    graph is captured nothing can be measured, neither the choice nor the
+    library's algorithm for a new M: only sizes that ran before go by it."""
+    return _wide_logits(M, N, K) and (
+        (M, N, K, bias is not None) in _WIDE_RUN
+        or not torch.cuda.is_current_stream_capturing())
+
+
 def _gemm_mode() -> str:
     return os.environ.get("DISTLLM_GEMM", "auto")
 
@@ -246,7 +259,7 @@ def linear(x, weight, bias=None, act=ACT_NONE):
         if x2.dtype == torch.float32:  # true 32-bit products
             mode = "blaslt"
         if (mode not in _OTHER_FORMS and M <= 64
-                and not (act == ACT_NONE and _wide_logits(M, N, K))
+                and not (act == ACT_NONE and _to_choose(M, N, K, bias))
                 and _few_rows(x2, weight, bias)):
             out = _hip_ops.decode_gemm(x2, weight, bias, 0, _DECODE_ACT[act])
             return out.reshape(*orig_shape[:-1], N)
@@ -292,6 +305,8 @@ def linear(x, weight, bias=None, act=ACT_NONE):
                 out = _blt_fused_path(x2, weight, bias, act)
             else:
                 out = torch.nn.functional.linear(x2, weight, bias)
+            if M <= 64 and _wide_logits(M, N, K):
+                _WIDE_RUN.add((M, N, K, bias is not None))
             return out.reshape(*orig_shape[:-1], N)
         shapes_ok = (M % 256 == 0 and N % 256 == 0 and K % 64 == 0
                      and x2.is_contiguous())

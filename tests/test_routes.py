@@ -91,3 +91,62 @@ def test_score_of_as_many_rows_as_32_bits_count(kernels):
     (32, 250000, 768, "product")])
 def test_score_where_tiles_fill_the_card(kernels, Q, N, K, way):
     assert ops.score(_OnGpu(Q, columns=K), _OnGpu(N, columns=K)) == way
+
+
+class _Cuda(torch.Tensor):
+    is_cuda = True
+
+
+@pytest.mark.parametrize("choice", ["decode", "blt_fused", "blaslt"])
+def test_wide_logits_are_not_measured_in_a_capture(monkeypatch, choice):
+    """Capture takes a product whose choice, or whose library algorithm at this
+    row count, is not there yet: by the form that needs neither."""
+    capturing, took = False, []
+
+    def ran(name):
+        def run(x, weight, *rest):
+            took.append(name)
+            if capturing and name == "blt_fused" and not x.shape[0] in known:
+                raise RuntimeError("waits in a capture")
+            known.add(x.shape[0])
+            return torch.empty(x.shape[0], weight.shape[0],
+                               dtype=torch.bfloat16)
+        return run
+
+    def synchronize():
+        if capturing:
+            raise RuntimeError("waits in a capture")
+
+    class Ops:
+        def require(self, name):
+            pass
+
+        decode_gemm = staticmethod(ran("decode"))
+
+    known = set()
+    monkeypatch.setattr(ops, "_hip_ops", Ops())
+    monkeypatch.setattr(ops, "_blt_fused_path", ran("blt_fused"))
+    monkeypatch.setattr(torch.nn.functional, "linear", ran("blaslt"))
+    monkeypatch.setattr(torch.cuda, "synchronize", synchronize)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing",
+                        lambda: capturing)
+    monkeypatch.setattr(ops, "_GEMM_CHOICE", {})
+    monkeypatch.setattr(ops, "_WIDE_RUN", set(), raising=False)
+    K, N = 1536, 33024
+    w = torch.empty(N, K, dtype=torch.bfloat16).as_subclass(_Cuda)
+    x = {M: torch.zeros(M, K, dtype=torch.bfloat16).as_subclass(_Cuda)
+         for M in (20, 40)}
+
+    def last(M):
+        took.clear()
+        assert ops.linear(x[M], w).shape == (M, N)
+        return took[-1]
+
+    capturing = True  # nothing ran yet
+    assert last(20) == "decode" and not ops._GEMM_CHOICE
+    ops._GEMM_CHOICE["dec", 128, N, K, False] = choice
+    capturing = False
+    assert last(20) == choice
+    capturing = True
+    assert last(20) == choice
+    assert last(40) == "decode"

@@ -178,3 +178,21 @@ def test_nothing_to_do(device, M, N, act):
         assert ops.linear(x, w, None, act).shape == (M, N)
         assert ops.gateup_swiglu(x, w).shape == (M, N // 2)
     torch.cuda.synchronize()
+
+
+def test_vocabulary_in_a_capture(device, monkeypatch):
+    """A wide product that was never measured can be captured."""
+    monkeypatch.setattr(ops, "_GEMM_CHOICE", {})
+    monkeypatch.setattr(ops, "_WIDE_RUN", set())
+    ops.linear(*_inputs(20, 64, 128, device, 0))
+    x, w, b = _inputs(20, 32832, 1536, device, 5)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = ops.linear(x, w, b)
+    assert not ops._GEMM_CHOICE
+    for seed in range(3):
+        x.copy_(_inputs(20, 64, 1536, device, seed)[0])
+        graph.replay()
+        torch.cuda.synchronize()
+        _close(out, x.float() @ w.float().T + b.float())
