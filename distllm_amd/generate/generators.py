@@ -73,7 +73,7 @@ class NativeGeneratorConfig(BaseConfig):
     max_batch_size: int = 64
     max_model_len: int = 4096
     # accepted for reference-YAML compatibility; single-GPU engine per
-    # rank (data-parallel across ranks) in this round:
+    # rank (data-parallel across ranks):
     tensor_parallel_size: int = 1
     trust_remote_code: bool = True
     # reference `quantization: true` meant NF4 capacity quantization;
@@ -111,7 +111,7 @@ class NativeGenerator:
             if dist.get_world_size() != config.tensor_parallel_size:
                 raise RuntimeError(
                     "tensor_parallel_size must equal the world size "
-                    "(TP subgroups are not split out in this round)"
+                    "(TP subgroups are not split out)"
                 )
             kw["tp_group"] = dist.group.WORLD
         self.model = build_model(dims, device=device, dtype=dtype, **kw)
