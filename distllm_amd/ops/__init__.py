@@ -240,12 +240,50 @@ def _gemm_mode() -> str:
     return os.environ.get("DISTLLM_GEMM", "auto")
 
 
+def _recorded(*tensors) -> bool:
+    """Whether something follows these tensors that a native kernel would
+    pass by: gradients, transforms, dispatch modes, tensors of another make."""
+    grad = torch.is_grad_enabled()
+    return (torch._C._len_torch_dispatch_stack() > 0
+            or torch._C._functorch.peek_interpreter_stack() is not None
+            or torch.autograd.forward_ad._current_level >= 0
+            or any(type(t) not in (torch.Tensor, torch.nn.Parameter)
+                   or (grad and t.requires_grad)
+                   for t in tensors if t is not None))
+
+
+# activation codes of wide_gemm behind those of linear
+_WIDE_SWIGLU, _WIDE_CLAMPED = 4, 5
+
+
+def _wide_tile(x2, weight, bias, act) -> int:
+    """The tile with which x2 @ weight^T, bias and activation or gated unit go
+    in one launch of csrc/wide_gemm.hip, 0 where another way is faster (the
+    measurements are there, at wide_gemm_tile) or has to be taken."""
+    M, K = x2.shape
+    N = weight.shape[0]
+    if M <= 64 or (act == ACT_NONE and M <= 256):
+        return 0
+    tile = _hip_ops.wide_gemm_tile(M, N, K, act)
+    if (tile and x2.dtype == weight.dtype == torch.bfloat16
+            and x2.is_contiguous() and weight.is_contiguous()
+            and x2.device == weight.device
+            and (bias is None or (
+                bias.dtype == torch.bfloat16 and bias.shape == (N,)
+                and bias.is_contiguous() and bias.device == x2.device))
+            and _gemm_mode() not in _OTHER_FORMS
+            and not _recorded(x2, weight, bias)):
+        return tile
+    return 0
+
+
 def linear(x, weight, bias=None, act=ACT_NONE):
-    """Linear layer entry used by models. GPU path: autotuned choice
-    between hipBLASLt (plain and fused-epilogue) and the hand-written
-    MFMA GEMMs (gemm8.hip, 8-phase gemm16.hip); the products of few rows
-    (decode_gemm.hip, with the activation) for M <= 64 (_few_rows) and
-    among the choices for M <= 256. Override with
+    """Linear layer entry used by models. GPU path: the products of few rows
+    (decode_gemm.hip, with the activation) for M <= 64 (_few_rows), those of
+    many rows (wide_gemm.hip, with the activation) where _wide_tile says so;
+    else an autotuned choice between hipBLASLt (plain and fused-epilogue), the
+    other hand-written MFMA GEMMs (gemm8.hip, 8-phase gemm16.hip) and, for M
+    <= 256, decode_gemm.hip. Override with
     DISTLLM_GEMM=blaslt|gemm8|gemm16|decode (the last for M <= 256, gemm8 and
     gemm16 at their multiples of 256 rows; without an activation M <= 256
     stays a choice for those two, at other sizes they mean the library)."""
@@ -263,6 +301,10 @@ def linear(x, weight, bias=None, act=ACT_NONE):
                 and _few_rows(x2, weight, bias)):
             out = _hip_ops.decode_gemm(x2, weight, bias, 0, _DECODE_ACT[act])
             return out.reshape(*orig_shape[:-1], N)
+        tile = _wide_tile(x2, weight, bias, act)
+        if tile:
+            return _hip_ops.wide_gemm(x2, weight, bias, act, tile).view(
+                *orig_shape[:-1], N)
         if (mode != "blaslt" and act == ACT_NONE and M <= 256
                 and N % 64 == 0 and K % 64 == 0 and x2.is_contiguous()
                 and (bias is None or bias.shape == (N,))):
@@ -593,8 +635,8 @@ def bert_few_rows(x, mask_f, layers, heads, eps, act):
 
 def gateup_swiglu(x, wgup, bias=None):
     """silu(x @ Wg^T) * (x @ Wu^T) with Wg|Wu packed as wgup [2I, K].
-    Few rows: ONE product with the swiglu in the same launch; otherwise one
-    big GEMM + packed swiglu."""
+    Few rows, and many where _wide_tile says so: ONE product with the swiglu in
+    the same launch; otherwise one big GEMM + packed swiglu."""
     orig_shape = x.shape
     x2 = x.reshape(-1, orig_shape[-1])
     M, K = x2.shape
@@ -604,6 +646,10 @@ def gateup_swiglu(x, wgup, bias=None):
         if _few_rows(x2, wgup, bias, 128):
             out = _hip_ops.decode_gemm(x2, wgup, bias, 0, 1)
             return out.reshape(*orig_shape[:-1], I)
+        tile = _wide_tile(x2, wgup, bias, _WIDE_SWIGLU)
+        if tile:
+            return _hip_ops.wide_gemm(x2, wgup, bias, _WIDE_SWIGLU,
+                                      tile).view(*orig_shape[:-1], I)
     gu = linear(x2, wgup, bias)
     if gu.is_cuda:
         out = _hip_ops.swiglu_packed(gu.contiguous())
@@ -615,12 +661,16 @@ def gateup_swiglu(x, wgup, bias=None):
 def gateup_clamped_glu(x, wgup, limit, alpha, shift):
     """Clamped gated unit of x @ Wg^T and x @ Wu^T, Wg|Wu packed as wgup
     [2I, K]: min(g, limit) * sigmoid(alpha * g) * (clamp(u) + shift), all
-    with the clamped g. For few rows ONE launch, as gateup_swiglu."""
+    with the clamped g. ONE launch where gateup_swiglu has one."""
     if x.is_cuda:
         _require_hip("_hip_gemm")
         if _few_rows(x, wgup, None, 128):
             return _hip_ops.decode_gemm(x, wgup, None, 0, 2, limit, alpha,
                                         shift)
+        tile = _wide_tile(x, wgup, None, _WIDE_CLAMPED)
+        if tile:
+            return _hip_ops.wide_gemm(x, wgup, None, _WIDE_CLAMPED, tile,
+                                      limit, alpha, shift)
         return _hip_ops.clamped_glu(linear(x, wgup), limit, alpha, shift)
     return torch_ref.clamped_glu(linear(x, wgup), limit, alpha, shift)
 

@@ -18,6 +18,9 @@ int decode_gemm_shares(int, int, int);
 void launch_norm_gemm(const void*, const void*, const void*, void*, float,
                       const void*, const void*, void*, int, int, int,
                       hipStream_t);
+void launch_wide_gemm(const void*, const void*, const void*, void*, int, int,
+                      int, int, float, float, float, int, hipStream_t);
+int wide_gemm_tile(int, int, int, int);
 void launch_clamped_glu(const void*, void*, long, int, float, float, float,
                         bool, hipStream_t);
 void launch_relu2(const void*, void*, long, bool, hipStream_t);
@@ -158,6 +161,44 @@ torch::Tensor decode_gemm_parts(torch::Tensor X, torch::Tensor W) {
   return slabs;
 }
 
+// X W^T of many rows. act 0 to 3 as of the 256-row tiles (GELU by erf in 32
+// bits), 4 and 5 = SwiGLU and clamped unit of packed gate and up rows; tile as
+// wide_gemm_tile gives it.
+torch::Tensor wide_gemm(torch::Tensor X, torch::Tensor W,
+                        c10::optional<torch::Tensor> bias, int64_t act,
+                        int64_t tile, double limit = 0.0, double alpha = 0.0,
+                        double shift = 0.0) {
+  CHECK_DEV(X); CHECK_CONT(X); CHECK_BF16(X);
+  CHECK_DEV(W); CHECK_CONT(W); CHECK_BF16(W);
+  TORCH_CHECK(X.dim() == 2 && W.dim() == 2 && W.size(1) == X.size(1) &&
+                  X.device() == W.device(),
+              "operands");
+  const int64_t M = X.size(0), K = X.size(1), N = W.size(0);
+  TORCH_CHECK(M > 0 && M < 1 << 30 && N > 0 && N % 256 == 0 && K % 64 == 0 &&
+                  K >= 128 && N * K < 1L << 30,
+              "wide_gemm: sizes");
+  TORCH_CHECK(act >= 0 && act <= 5 && tile >= 4 && tile <= 8, "wide_gemm");
+  const int64_t rows = (M + 32 * tile - 1) / (32 * tile);
+  TORCH_CHECK(rows * (N / 256) * (N / 256) * 8 < 1L << 32,
+              "wide_gemm: too many tiles");
+  const c10::DeviceGuard guard(X.device());
+  if (bias) {
+    CHECK_DEV(bias.value()); CHECK_CONT(bias.value());
+    CHECK_BF16(bias.value());
+    TORCH_CHECK(bias->numel() == N && bias->device() == X.device(),
+                "bias must be [N]");
+    bias = aligned16(bias.value());
+  }
+  auto out = torch::empty({M, act >= 4 ? N / 2 : N}, X.options());
+  X = aligned16(X);
+  W = aligned16(W);
+  launch_wide_gemm(X.data_ptr(), W.data_ptr(),
+                   bias ? bias->data_ptr() : nullptr, out.data_ptr(), (int)M,
+                   (int)N, (int)K, (int)act, (float)limit, (float)alpha,
+                   (float)shift, (int)tile, cur_stream());
+  return out;
+}
+
 // x = a + b, one row, and the product of its RMS norm (act 1: gated unit)
 std::vector<torch::Tensor> norm_gemm(torch::Tensor a, torch::Tensor b,
                                      torch::Tensor w_norm, double eps,
@@ -264,6 +305,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("bias"), py::arg("splitk"), py::arg("act") = 0,
         py::arg("limit") = 0.0, py::arg("alpha") = 0.0,
         py::arg("shift") = 0.0, py::arg("act_nums") = py::none());
+  m.def("wide_gemm", &wide_gemm, py::arg("X"), py::arg("W"), py::arg("bias"),
+        py::arg("act"), py::arg("tile"), py::arg("limit") = 0.0,
+        py::arg("alpha") = 0.0, py::arg("shift") = 0.0);
+  m.def("wide_gemm_tile", &wide_gemm_tile);
   m.def("norm_gemm", &norm_gemm);
   m.def("decode_gemm_parts", &decode_gemm_parts);
   m.def("decode_gemm_shares", &decode_gemm_shares);

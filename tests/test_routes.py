@@ -150,3 +150,34 @@ def test_wide_logits_are_not_measured_in_a_capture(monkeypatch, choice):
     capturing = True
     assert last(20) == choice
     assert last(40) == "decode"
+
+
+def test_many_rows_go_by_tiles_and_sums():
+    """wide_gemm_tile: sizes that the kernel cannot take, rounds of the card's
+    CUs, and what is followed stays with torch."""
+    tile = ops._hip_ops.wide_gemm_tile
+    for sizes in [(5000, 2200, 768, 0), (5000, 2304, 760, 0),
+                  (5000, 2304, 64, 0), (0, 256, 128, 0), (5000, 0, 128, 0),
+                  (100000, 1 << 20, 1024, 0), (1 << 29, 1 << 20, 128, 0)]:
+        assert tile(*sizes) == 0
+    assert tile(12992, 768, 768, 0) == 5   # 246 tiles of 160 rows
+    assert tile(8448, 4096, 14336, 0) == 6  # 704 of 192 rows, 2.75 rounds
+    assert tile(262144, 2304, 768, 0) == 8
+    assert tile(300, 768, 768, 0) == 0     # too few tiles
+    assert tile(1000, 3072, 768, 2) == 4   # and enough with an activation
+    assert tile(16384, 4096, 4096, 0) == 0  # whole rounds of long sums
+    assert tile(16384, 28672, 4096, 4) == 8
+    x = torch.zeros(2)
+    p = torch.nn.Parameter(x)
+    assert ops._recorded(p) and not ops._recorded(x, None)
+    with torch.no_grad():
+        assert not ops._recorded(x, p)
+        assert ops._recorded(type("Sub", (torch.Tensor,), {})(2))
+        seen = []
+        torch.func.vmap(lambda t: seen.append(ops._recorded(t)) or t)(x)
+        with torch.autograd.forward_ad.dual_level():
+            seen.append(ops._recorded(x))
+        from torch.utils.flop_counter import FlopCounterMode
+        with FlopCounterMode(display=False):
+            seen.append(ops._recorded(x))
+        assert seen == [True] * 3

@@ -1,0 +1,159 @@
+"""Products of many rows (csrc/wide_gemm.hip): tiles, remainders, activations
+and units against fp32 references, and which calls linear sends there."""
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+import distllm_amd.ops as ops
+
+pytestmark = pytest.mark.gpu
+
+
+def _operands(M, N, K, seed=0):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    x = torch.randn(M, K, device="cuda", generator=g).bfloat16()
+    w = (torch.randn(N, K, device="cuda", generator=g) * K ** -0.5).bfloat16()
+    b = torch.randn(N, device="cuda", generator=g).bfloat16()
+    return x, w, b
+
+
+def _reference(x, w, b, act):
+    y = x.double() @ w.double().T
+    if b is not None:
+        y = y + b.double()
+    if act == ops.ACT_GELU_TANH:
+        return F.gelu(y, approximate="tanh")
+    if act == ops.ACT_GELU_ERF:
+        return F.gelu(y)
+    if act == ops.ACT_SILU:
+        return F.silu(y)
+    if act >= 4:
+        g, u = y.chunk(2, 1)
+        if act == 4:
+            return F.silu(g) * u
+        g, u = g.clamp(max=1.5), u.clamp(-1.5, 1.5)
+        return g * torch.sigmoid(1.702 * g) * (u + 1)
+    return y
+
+
+def _check(got, want):
+    # the result's rounding to 8 bits, and sums of at most 1024 terms of size
+    # 1 in 32 bits ahead of an activation whose slope is below 2 x its factor
+    bound = want.abs() * 2.0 ** -8 + 2e-5 * (1 + want.abs().amax())
+    assert ((got.double() - want).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("tile", [4, 5, 6, 7, 8])
+@pytest.mark.parametrize("M,N,K", [
+    (1, 256, 128),      # one row of one tile, two stages
+    (257, 512, 192),    # a row behind a tile's edge, an odd count of stages
+    (2049, 768, 128),   # more row tiles than go together, some in the last
+    (9001, 2304, 256),  # workgroups with more tiles than one
+    (300, 256, 1024),   # more stages than slots, a few times
+])
+def test_tiles(tile, M, N, K):
+    x, w, b = _operands(M, N, K)
+    _check(ops._hip_ops.wide_gemm(x, w, b, 0, tile), _reference(x, w, b, 0))
+
+
+@pytest.mark.parametrize("act", [1, 2, 3, 4, 5])
+@pytest.mark.parametrize("bias", [False, True])
+@pytest.mark.parametrize("M,tile", [(70, 8), (4099, 6)])
+def test_ends(act, bias, M, tile):
+    x, w, b = _operands(M, 1024, 320)
+    b = b if bias else None
+    got = ops._hip_ops.wide_gemm(x, w, b, act, tile, 1.5, 1.702, 1.0)
+    _check(got, _reference(x, w, b, act))
+
+
+def test_large_result():
+    """Above 256 MiB the result is written past the caches."""
+    x, w, b = _operands(46000, 3072, 128)
+    got = ops._hip_ops.wide_gemm(x, w, b, 0, 8)
+    at = torch.arange(0, 46000, 97, device="cuda")
+    _check(got[at], _reference(x[at], w, b, 0))
+    _check(got[-300:], _reference(x[-300:], w, b, 0))
+
+
+def test_gelu_of_large_and_not_finite():
+    x, w, b = _operands(300, 256, 128)
+    x[:, 0], w[:, 1:] = 1.0, 0.0
+    special = torch.tensor([float("inf"), float("nan"), 3e38, 80.0, 9.0, 5.5,
+                            4.0, 1e-3, 1e-30, 0.0, -1e-3, -4.0, -5.5, -9.0,
+                            -80.0, -3e38], device="cuda").bfloat16()
+    w[:, 0] = 0
+    b[:] = special.repeat(16)
+    got = ops._hip_ops.wide_gemm(x, w, b, 2, 8).double()
+    want = F.gelu(b.double()).expand(300, -1)
+    assert torch.equal(got.isnan(), want.isnan())
+    ok = ~want.isnan()
+    same = got[ok] == want[ok]  # infinities among them
+    close = (got[ok] - want[ok]).abs() <= want[ok].abs() * 2.0 ** -8 + 1e-6
+    assert (same | close).all()
+
+
+def test_linear_takes_it_and_gives_the_library_s_result(monkeypatch):
+    """Over the forms that linear accepts: shapes with leading dimensions,
+    strided inputs and biases, storage that starts between 16-byte pieces."""
+    calls = []
+    own = ops._hip_ops.wide_gemm
+    monkeypatch.setattr(ops._hip_ops, "wide_gemm",
+                        lambda *a: calls.append(a) or own(*a), raising=False)
+    x, w, b = _operands(6000, 2304, 256)
+
+    def same(x, w, b, wide):
+        calls.clear()
+        got = ops.linear(x, w, b)
+        assert got.shape == (*x.shape[:-1], w.shape[0])
+        assert bool(calls) == wide
+        _check(got.reshape(-1, w.shape[0]),
+               _reference(x.reshape(-1, x.shape[-1]), w, b, 0))
+
+    with torch.no_grad():
+        same(x, w, b, True)
+        same(x.view(6, 1000, 256), w, None, True)
+        same(torch.nn.Parameter(x), torch.nn.Parameter(w), b, True)
+        wide = torch.randn(6000, 512, device="cuda").bfloat16()
+        same(wide[:, :256], w, b, False if not wide[:, :256].is_contiguous()
+             else True)
+        same(wide.view(3000, 4, 256).transpose(0, 1), w, b, True)  # a copy
+        same(x, w, torch.stack([b, b], 1)[:, 0], False)
+        flat = torch.empty(6000 * 256 + 1, device="cuda").bfloat16()
+        flat[1:] = x.reshape(-1)
+        same(flat[1:].view(6000, 256), w, b, True)
+        same(x[:300], w, b, False)
+        monkeypatch.setenv("DISTLLM_GEMM", "blaslt")
+        same(x, w, b, False)
+        monkeypatch.delenv("DISTLLM_GEMM")
+    # gradients are the library's
+    w = torch.nn.Parameter(w)
+    calls.clear()
+    y = ops.linear(x[:5999], w, b)
+    assert y.requires_grad and not calls
+    y.float().sum().backward()
+    assert w.grad is not None
+
+
+def test_units_take_it():
+    x, w, _ = _operands(3000, 6144, 256)
+    with torch.no_grad():
+        assert ops._wide_tile(x, w, None, 4)
+        _check(ops.gateup_swiglu(x, w), _reference(x, w, None, 4))
+        _check(ops.gateup_clamped_glu(x, w, 1.5, 1.702, 1.0),
+               _reference(x, w, None, 5))
+
+
+def test_in_a_graph():
+    x, w, b = _operands(3000, 2304, 768)
+    with torch.no_grad():
+        want = ops.linear(x, w, b, act=ops.ACT_GELU_ERF)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            got = ops.linear(x, w, b, act=ops.ACT_GELU_ERF)
+        for _ in range(3):
+            got.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(got, want)
