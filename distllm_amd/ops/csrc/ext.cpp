@@ -393,10 +393,10 @@ std::vector<torch::Tensor> topk_chunked(torch::Tensor scores,
   const int Q = scores.size(0);
   const long N = scores.size(1);
   const int nchunks = (int)((N + chunk - 1) / chunk);
-  auto ov = torch::empty({Q, (long)nchunks * k},
-                         scores.options().dtype(at::kFloat));
-  auto oi = torch::empty({Q, (long)nchunks * k},
-                         scores.options().dtype(at::kInt));
+  // one behind the other, so that one copy takes both to the host
+  auto both = torch::empty({2, Q, (long)nchunks * k},
+                           scores.options().dtype(at::kInt));
+  auto ov = both.select(0, 0).view(at::kFloat), oi = both.select(0, 1);
   launch_topk_chunk(scores.data_ptr<float>(),
                     in_idx ? in_idx->data_ptr<int>() : nullptr,
                     ov.data_ptr<float>(), oi.data_ptr<int>(), Q, N, (int)chunk,

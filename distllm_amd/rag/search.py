@@ -54,6 +54,17 @@ def quantize_embeddings(emb: np.ndarray, precision: str) -> np.ndarray:
     raise ValueError(f"unsupported precision {precision}")
 
 
+def _one_tensor(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
+    """[2, ...] of two tensors of one shape and type: where they lie one
+    behind the other, as ops.topk leaves them, as they lie."""
+    if (a.is_contiguous() and b.is_contiguous()
+            and a.untyped_storage().data_ptr() == b.untyped_storage().data_ptr()
+            and b.storage_offset() == a.storage_offset() + a.numel()):
+        return b.as_strided((2, *b.shape), (b.numel(), *b.stride()),
+                            a.storage_offset())
+    return torch.stack((a, b))
+
+
 class HipIndexConfig(BaseConfig):
     name: str = Field("hip_index",
                       description="'hip_index' (alias: 'faiss_index_v2')")
@@ -356,17 +367,20 @@ class HipFlatIndex:
             v, i = self._topk_ivf(q, top_k)
         else:
             v, i = self._topk_exact(q, top_k)
-        v = v.cpu().tolist()
-        i = i.cpu().tolist()
+        # scores and indices in one copy: it costs 25 us whatever it holds
+        both = _one_tensor(v.float().view(torch.int32), i.int()).cpu().numpy()
+        scores, indices = both[0].view(np.float32), both[1]
         print(f"Search time: {time.perf_counter() - t0:.6f} seconds")
         # IVF pads short candidate lists with index -1 / score -inf;
         # drop those unconditionally (not only under score_threshold) so
-        # -1 never reaches get()/dataset indexing as "last row".
-        vv, ii = [], []
-        for scores, indices in zip(v, i):
-            keep = [(s, ix) for s, ix in zip(scores, indices) if ix >= 0]
-            vv.append([s for s, _ in keep])
-            ii.append([ix for _, ix in keep])
+        # -1 never reaches get()/dataset indexing as "last row". Lists without
+        # any are taken as they are (256 by 10 of them: 240 us entry by entry).
+        keep = indices >= 0
+        if keep.all():
+            vv, ii = scores.tolist(), indices.tolist()
+        else:
+            vv = [s[k].tolist() for s, k in zip(scores, keep)]
+            ii = [x[k].tolist() for x, k in zip(indices, keep)]
         results = BatchedSearchResults(total_scores=vv, total_indices=ii)
         return self._filter_search_by_score(results, score_threshold)
 

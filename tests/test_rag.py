@@ -3,6 +3,7 @@ search vs numpy reference, retriever, end-to-end RagGenerator."""
 
 import numpy as np
 import pytest
+import torch
 
 from distllm_amd.rag.search import (
     HipFlatIndex,
@@ -212,3 +213,30 @@ download_dir: /data/benchmarks
     assert len(c.rag_configs) == 1
     fc = c.rag_configs[0].retriever_config.faiss_config
     assert str(fc.faiss_index_path).endswith("hip_index.npz")
+
+
+def test_search_takes_scores_and_indices_together(tmp_path, monkeypatch):
+    """Answers that lie one behind the other go as they lie, others are
+    joined; short lists lose their -1 entries, row by row."""
+    from distllm_amd.rag import search
+
+    both = torch.arange(12, dtype=torch.int32).view(2, 2, 3)
+    one = search._one_tensor(both[0], both[1])
+    assert one.data_ptr() == both.data_ptr() and torch.equal(one, both)
+    for a, b in [(both[1], both[0]), (both[0].clone(), both[1]),
+                 (both[0, :, :2], both[1, :, :2]), (both[0, :0], both[1, :0])]:
+        assert torch.equal(search._one_tensor(a, b), torch.stack((a, b)))
+
+    index = search.HipFlatIndex.__new__(search.HipFlatIndex)
+    index.corpus = torch.zeros(1, 4)
+    index.precision, index.search_algorithm = "float32", "exact"
+    v = torch.tensor([[3.0, 2.0, float("-inf")], [9.0, 8.5, 8.25]])
+    i = torch.tensor([[4, 7, -1], [0, 1, 2]])
+    monkeypatch.setattr(index, "_topk_exact", lambda q, k: (v, i))
+    found = index.search(np.zeros((2, 4), np.float32), top_k=3)
+    assert found.total_scores == [[3.0, 2.0], [9.0, 8.5, 8.25]]
+    assert found.total_indices == [[4, 7], [0, 1, 2]]
+    assert type(found.total_indices[0][0]) is int
+    i[0, 2] = 9
+    assert index.search(np.zeros((2, 4), np.float32), top_k=3,
+                        score_threshold=8.4).total_indices == [[], [0, 1]]
