@@ -295,10 +295,13 @@ class DecoderModel(nn.Module):
         # products whose shares of K the next kernel sums (on one rank)
         parts = ops.linear_parts if self.tp == 1 else ops.linear
         eps = d.rms_norm_eps
+        zeros = (ops.step_zeros(len(self.layers), B, nh, kcaches[0],
+                                block_tables) if len(self.layers) else None)
         down = None
         for li, layer in enumerate(self.layers):
             # norm and ONE fused qkv GEMM (one launch for one sequence), ONE
-            # launch that rotates q and k and writes k and v to their pages
+            # launch that rotates q and k, writes k and v to their pages and
+            # attends
             f = fp8[li] if fp8 is not None else None
             if down is None:
                 h = ops.rms_norm(x, layer.in_norm, eps=eps)[:, 0]
@@ -312,11 +315,10 @@ class DecoderModel(nn.Module):
                 qkv, x = ops.norm_linear(down, x, layer.in_norm, eps,
                                          layer.wqkv, layer.bqkv,
                                          shares=hd in (64, 128))
-            q = ops.rope_put(
+            ctx = ops.step_attn(
                 qkv.view(*qkv.shape[:-1], nh + 2 * kvh, hd), cs, sn,
-                ctx_lens, kcaches[li], vcaches[li], block_tables, layer.bqkv)
-            ctx = ops.paged_attn(q, kcaches[li], vcaches[li], block_tables,
-                                 ctx_lens, scale=1.0 / math.sqrt(hd))
+                ctx_lens, kcaches[li], vcaches[li], block_tables, layer.bqkv,
+                1.0 / math.sqrt(hd), zeros[li] if zeros is not None else None)
             ctx = ctx.reshape(B, nh * hd)
             if f is not None:
                 attn = self._allreduce(ops.gemv_fp8(ctx, *f["wo"]))

@@ -853,6 +853,33 @@ def rope_put(qkv, cs, sn, ctx, kcache, vcache, block_table, bias=None):
     return qkv[:, :H].contiguous()
 
 
+def step_zeros(layers, B, H, kcache, block_table):
+    """What step_attn of so many layers needs cleared, a row for each, None
+    where it needs nothing."""
+    HKV, D = kcache.shape[1], kcache.shape[3]
+    if (not kcache.is_cuda or D not in (64, 128)
+            or _hip_ops.step_attn_shares(B, H, HKV, block_table.shape[1],
+                                         kcache.dtype == torch.uint8) <= 1):
+        return None
+    return torch.zeros(layers, B * HKV * -(-(H // HKV) // 16),
+                       dtype=torch.int32, device=kcache.device)
+
+
+def step_attn(qkv, cs, sn, ctx, kcache, vcache, block_table, bias, scale,
+              zeros):
+    """rope_put and the attention of its queries over the cache, the new token
+    among it -> [B, H, D]; one launch for heads of 64 and 128. zeros: a row of
+    step_zeros, used up."""
+    if qkv.is_cuda and qkv.shape[-1] in (64, 128):
+        _require_hip()
+        return _hip_ops.step_attn(qkv.contiguous(), cs, sn, ctx.int(), kcache,
+                                  vcache, block_table.int(),
+                                  bias if qkv.dim() == 4 else None, scale,
+                                  zeros)
+    q = rope_put(qkv, cs, sn, ctx, kcache, vcache, block_table, bias)
+    return paged_attn(q, kcache, vcache, block_table, ctx, scale)
+
+
 # ---- sandwich-norm / latent-attention decoder -----------------------------
 
 def embed_norm(tokens, table, w_next, n, eps):

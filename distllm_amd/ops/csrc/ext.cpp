@@ -52,9 +52,13 @@ void launch_gemv_fp8_norm(const void*, const void*, const void*, void*, float,
                           int, bool, hipStream_t);
 void launch_sample(const float*, const float*, int*, int, int, float, float,
                    hipStream_t);
-void launch_paged_attn(const void*, long, const void*, const void*,
-                       const int*, const int*, void*, void*, void*, int, int,
-                       int, int, int, int, float, bool, bool, hipStream_t);
+void launch_paged_attn(const void*, long, void*, void*, const int*,
+                       const int*, void*, void*, void*, int, int, int, int,
+                       int, int, float, bool, bool, hipStream_t);
+void launch_step_attn(const void*, const float*, int, const void*,
+                      const float*, const float*, void*, void*, const int*,
+                      const int*, void*, void*, void*, int*, int, int, int,
+                      int, int, int, float, bool, bool, hipStream_t);
 void launch_norm_parts(const float*, int, const void*, const void*, void*,
                        void*, int, int, float, hipStream_t);
 void launch_rope_put(const void*, const float*, int, const void*,
@@ -472,6 +476,23 @@ int64_t paged_attn_shares(int64_t B, int64_t H, int64_t HKV,
       1);
 }
 
+// The same for step_attn, whose shares join in the launch, so that one that
+// finds no keys costs next to nothing: every CU one, each with 128 of the table's
+// positions (a tile for each of its waves); fp8 pages two, with 256. In us, shares
+// of 4, 8, 16, 32 (two launches as above): 1 x 8 grouped heads, contexts of 64
+// 6.2, 6.3, 6.3, 7.4 (10.9); 2048 11.2, 8.3, 7.6, 8.8 (12.7); 8000 30, 18, 12.2,
+// 10.6 (21); 8 x 8 of 2000 15.6, 20, 21 (22); 8 x 8 fp8 of 500 7.5, 9.5, 17 (11),
+// of 2000 12.4, 12.1, 18.5 (18).
+int64_t step_attn_shares(int64_t B, int64_t H, int64_t HKV,
+                         int64_t max_blocks, bool fp8) {
+  const char* e = getenv("DISTLLM_PA_NSPLIT");
+  if (e && atol(e) > 0) return paged_attn_shares(B, H, HKV, max_blocks, fp8);
+  const long groups = std::max<long>(B * HKV * ((H / HKV + 15) / 16), 1);
+  long n = std::min<long>(256 / groups, max_blocks / 8);
+  if (fp8) n = std::max(n, std::min<long>(512 / groups, max_blocks / 16));
+  return std::max<long>(std::min<long>(n, 32), 1);
+}
+
 torch::Tensor paged_attn(torch::Tensor q, torch::Tensor kcache,
                          torch::Tensor vcache, torch::Tensor block_table,
                          torch::Tensor ctx_len, double scale) {
@@ -504,13 +525,18 @@ torch::Tensor paged_attn(torch::Tensor q, torch::Tensor kcache,
   return out;
 }
 
-// qkv [B, H + 2 HKV, D] of a decode step (or the slabs [S, B, H + 2 HKV, D]
-// fp32 of the product that it would be, and its bias) -> rotated q [B, H, D];
-// rotated keys and the values to their places (position ctx - 1) in the cache
-torch::Tensor rope_put(torch::Tensor qkv, torch::Tensor cs, torch::Tensor sn,
-                       torch::Tensor ctx, torch::Tensor kcache,
-                       torch::Tensor vcache, torch::Tensor block_table,
-                       c10::optional<torch::Tensor> bias) {
+// qkv [B, H + 2 HKV, D] of a decode step, or the slabs [S, B, H + 2 HKV, D]
+// fp32 of the product that it would be, and its bias
+struct StepSizes {
+  bool parts;
+  int B, H, HKV, D;
+};
+static StepSizes check_step(const torch::Tensor& qkv, const torch::Tensor& cs,
+                            const torch::Tensor& sn, const torch::Tensor& ctx,
+                            const torch::Tensor& kcache,
+                            const torch::Tensor& vcache,
+                            const torch::Tensor& block_table,
+                            const c10::optional<torch::Tensor>& bias) {
   CHECK_DEV(qkv); CHECK_CONT(qkv);
   CHECK_FLOATS(cs); CHECK_FLOATS(sn);
   const bool parts = qkv.scalar_type() == at::kFloat;
@@ -529,18 +555,76 @@ torch::Tensor rope_put(torch::Tensor qkv, torch::Tensor cs, torch::Tensor sn,
     CHECK_BF16(bias.value());
     TORCH_CHECK(bias->numel() == (long)(H + 2 * HKV) * D, "bias");
   }
-  auto q = torch::empty({B, H, D}, qkv.options().dtype(at::kBFloat16));
-  if (B > 0)
-    launch_rope_put(parts ? nullptr : qkv.data_ptr(),
-                    parts ? qkv.data_ptr<float>() : nullptr,
-                    parts ? (int)qkv.size(0) : 0,
+  return {parts, B, H, HKV, D};
+}
+
+// -> rotated q [B, H, D]; rotated keys and the values to their places (position
+// ctx - 1) in the cache
+torch::Tensor rope_put(torch::Tensor qkv, torch::Tensor cs, torch::Tensor sn,
+                       torch::Tensor ctx, torch::Tensor kcache,
+                       torch::Tensor vcache, torch::Tensor block_table,
+                       c10::optional<torch::Tensor> bias) {
+  const StepSizes z =
+      check_step(qkv, cs, sn, ctx, kcache, vcache, block_table, bias);
+  auto q = torch::empty({z.B, z.H, z.D}, qkv.options().dtype(at::kBFloat16));
+  if (z.B > 0)
+    launch_rope_put(z.parts ? nullptr : qkv.data_ptr(),
+                    z.parts ? qkv.data_ptr<float>() : nullptr,
+                    z.parts ? (int)qkv.size(0) : 0,
                     bias ? bias->data_ptr() : nullptr, cs.data_ptr<float>(),
                     sn.data_ptr<float>(), ctx.data_ptr<int>(), q.data_ptr(),
                     kcache.data_ptr(), vcache.data_ptr(),
-                    block_table.data_ptr<int>(), B, H, HKV, D,
+                    block_table.data_ptr<int>(), z.B, z.H, z.HKV, z.D,
                     block_table.size(1), kcache.scalar_type() == at::kByte,
                     cur_stream());
   return q;
+}
+
+// rope_put and the attention of its queries [B, H, D] in one launch. arrived:
+// zeros (int32, B * HKV * ceil(H / HKV / 16) of them, used up by the call) where
+// step_attn_shares of the sizes is above 1.
+torch::Tensor step_attn(torch::Tensor qkv, torch::Tensor cs, torch::Tensor sn,
+                        torch::Tensor ctx, torch::Tensor kcache,
+                        torch::Tensor vcache, torch::Tensor block_table,
+                        c10::optional<torch::Tensor> bias, double scale,
+                        c10::optional<torch::Tensor> arrived) {
+  const StepSizes z =
+      check_step(qkv, cs, sn, ctx, kcache, vcache, block_table, bias);
+  TORCH_CHECK(z.H % z.HKV == 0, "GQA requires H % HKV == 0");
+  const int max_blocks = block_table.size(1);
+  const bool fp8 = kcache.scalar_type() == at::kByte;
+  auto out =
+      torch::empty({z.B, z.H, z.D}, qkv.options().dtype(at::kBFloat16));
+  if (z.B == 0) return out;
+  const int NS = (int)step_attn_shares(z.B, z.H, z.HKV, max_blocks, fp8);
+  torch::Tensor pacc, pml;
+  if (NS > 1) {
+    TORCH_CHECK(arrived.has_value(), "arrived");
+    CHECK_INTS(arrived.value());
+    TORCH_CHECK(arrived->numel() >=
+                    (long)z.B * z.HKV * ((z.H / z.HKV + 15) / 16),
+                "arrived: one for every group of heads");
+    auto f32 = qkv.options().dtype(at::kFloat);
+    pacc = torch::empty({(long)z.B * z.H * NS, z.D}, f32);
+    pml = torch::empty({(long)z.B * z.H * NS, 2}, f32);
+  }
+  qkv = aligned16(qkv);
+  cs = aligned16(cs);
+  sn = aligned16(sn);
+  const bool aligned = (uintptr_t)kcache.data_ptr() % 16 == 0 &&
+                       (uintptr_t)vcache.data_ptr() % 16 == 0;
+  launch_step_attn(z.parts ? nullptr : qkv.data_ptr(),
+                   z.parts ? qkv.data_ptr<float>() : nullptr,
+                   z.parts ? (int)qkv.size(0) : 0,
+                   bias ? bias->data_ptr() : nullptr, cs.data_ptr<float>(),
+                   sn.data_ptr<float>(), kcache.data_ptr(), vcache.data_ptr(),
+                   block_table.data_ptr<int>(), ctx.data_ptr<int>(),
+                   out.data_ptr(), NS > 1 ? pacc.data_ptr() : nullptr,
+                   NS > 1 ? pml.data_ptr() : nullptr,
+                   NS > 1 ? arrived->data_ptr<int>() : nullptr, z.B, z.H,
+                   z.HKV, z.D, max_blocks, NS, (float)scale, fp8, aligned,
+                   cur_stream());
+  return out;
 }
 
 void cache_put(torch::Tensor knew, torch::Tensor vnew, torch::Tensor kcache,
@@ -683,6 +767,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("paged_attn_shares", &paged_attn_shares);
   m.def("cache_put", &cache_put);
   m.def("norm_parts", &norm_parts);
+  m.def("step_attn", &step_attn);
+  m.def("step_attn_shares", &step_attn_shares);
   m.def("rope_put", &rope_put, py::arg("qkv"), py::arg("cs"), py::arg("sn"),
         py::arg("ctx"), py::arg("kcache"), py::arg("vcache"),
         py::arg("block_table"), py::arg("bias") = py::none());

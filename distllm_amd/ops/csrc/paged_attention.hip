@@ -25,7 +25,11 @@
 //    or, but for a first one, 0: an infinite value gives an infinite result. fp8
 //    has no infinities.
 //  - NS workgroups share a sequence where B * HKV is small; a second launch
-//    joins them.
+//    joins them or, in a decode step, the last of them.
+//  - a decode step's queries are rotated and its key and value put into the
+//    cache in the same launch (STEP): us in a graph, three launches and one,
+//    32 heads on 8, B = 1, 2048 tokens 12.7 -> 7.6, 64 tokens 10.9 -> 6.3, B = 8
+//    of 500 11.0 -> 7.4, B = 64 of 200 to 2027 70 -> 56.
 // Measured, us, with kernels that read a key row per lane and a value element
 // per lane, and now (32 heads on 8 of 128, bf16; fp8): B = 1, 2048 cached
 // tokens 32 -> 11.0 (31 -> 11.1); B = 16 of 100 to 4000 115 -> 36.5 (104 ->
@@ -68,6 +72,105 @@ __device__ __forceinline__ void pa_widen(const i32x4 v, i32x4 (&out)[2]) {
   }
 }
 
+// Cache element of a bf16 number.
+__device__ __forceinline__ void cache_store(unsigned short* p,
+                                            unsigned short v) {
+  *p = v;
+}
+__device__ __forceinline__ void cache_store(unsigned char* p,
+                                            unsigned short v) {
+  *p = __hip_fp8_e4m3(bf2f(v)).__x;
+}
+
+// A decode step's projections [B, H + 2 HKV, D], as bf16 numbers or, S > 0, as
+// the S fp32 slabs of a product whose K was shared, without its bias; rotation
+// tables [positions, D / 2].
+struct PaStep {
+  const unsigned short* qkv;
+  const float* parts;
+  int S;
+  const unsigned short* bias;
+  const float *cs, *sn;
+};
+
+// Columns c .. c + 3 and D / 2 + c .. of head h of row b, as bf16 numbers; ROT:
+// rotated (half-split, fp32) by the angles of position pos.
+template <int D>
+__device__ __forceinline__ void step_columns(const PaStep& p, int B,
+                                             int heads, int b, int h, int c,
+                                             bool rotate, int pos,
+                                             unsigned short* a,
+                                             unsigned short* e) {
+  const long at = ((long)b * heads + h) * D + c;
+  f32x4 co = {1.f, 1.f, 1.f, 1.f}, si = {0.f, 0.f, 0.f, 0.f};
+  if (rotate) {
+    co = *reinterpret_cast<const f32x4*>(p.cs + (long)pos * (D / 2) + c);
+    si = *reinterpret_cast<const f32x4*>(p.sn + (long)pos * (D / 2) + c);
+  }
+  if (p.S == 0) {
+    *reinterpret_cast<i32x2*>(a) = *reinterpret_cast<const i32x2*>(p.qkv + at);
+    *reinterpret_cast<i32x2*>(e) =
+        *reinterpret_cast<const i32x2*>(p.qkv + at + D / 2);
+  } else {
+    f32x4 va = {0.f, 0.f, 0.f, 0.f}, ve = va;
+    const long slab = (long)B * heads * D;
+    // four slabs at once are on their way
+    for (int s0 = 0; s0 < p.S; s0 += 4) {
+      f32x4 pa[4], pe[4];
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        const float* from = p.parts + min(s0 + s, p.S - 1) * slab + at;
+        pa[s] = *reinterpret_cast<const f32x4*>(from);
+        pe[s] = *reinterpret_cast<const f32x4*>(from + D / 2);
+      }
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          va[j] = s0 + s < p.S ? va[j] + pa[s][j] : va[j];
+          ve[j] = s0 + s < p.S ? ve[j] + pe[s][j] : ve[j];
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (p.bias != nullptr) {
+        va[j] += bf2f(p.bias[h * D + c + j]);
+        ve[j] += bf2f(p.bias[h * D + D / 2 + c + j]);
+      }
+      a[j] = f2bf(va[j]);
+      e[j] = f2bf(ve[j]);
+    }
+  }
+  if (rotate) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float x = bf2f(a[j]), y = bf2f(e[j]);
+      // fused as written, in every kernel alike
+      a[j] = f2bf(fmaf(x, co[j], -(y * si[j])));
+      e[j] = f2bf(fmaf(y, co[j], x * si[j]));
+    }
+  }
+}
+
+// Two results of a workgroup for the kernel, or (JOIN) the workgroup, that joins
+// them.
+template <bool JOIN>
+__device__ __forceinline__ void pa_put(float* to, float a, float b) {
+  const f32x2 v = {a, b};
+  if constexpr (JOIN)
+    __hip_atomic_store(reinterpret_cast<unsigned long long*>(to),
+                       __builtin_bit_cast(unsigned long long, v),
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  else
+    *reinterpret_cast<f32x2*>(to) = v;
+}
+__device__ __forceinline__ f32x2 pa_get(const float* from) {
+  return __builtin_bit_cast(
+      f32x2, __hip_atomic_load(
+                 reinterpret_cast<const unsigned long long*>(from),
+                 __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+}
+
 // LDS of a workgroup: the waves' rings of R tiles of K and V, then their states
 constexpr int NW = 4;  // waves of a workgroup
 constexpr int pa_lds(int D, int R) {
@@ -77,16 +180,20 @@ constexpr int pa_lds(int D, int R) {
 
 // ALIGNED: the pages start at a multiple of 16 bytes, as the copies to LDS ask;
 // else bf16 pages pass through registers like fp8 ones, one tile after another.
-template <int D, bool FP8, bool ALIGNED, int R>
+// STEP: queries come out of the step's projections and are rotated here, into
+// LDS, while the first tile is on its way, and so are the new token's key and
+// value where the share ends with it: the wave that has the last tile puts them
+// into it, and they go to the cache (from the first of several groups of heads).
+// A launch that did this ahead (rope_put_kernel) took 4.7 us.
+template <int D, bool FP8, bool ALIGNED, int R, bool STEP>
 __global__ void __launch_bounds__(256)
 paged_attn_kernel(const unsigned short* __restrict__ q, long q_stride,
-                  const char* __restrict__ kcache,
-                  const char* __restrict__ vcache,
+                  const PaStep step, char* kcache, char* vcache,
                   const int* __restrict__ block_table,
                   const int* __restrict__ ctx_len,
                   unsigned short* __restrict__ out,
-                  float* __restrict__ pacc, float* __restrict__ pml, int H,
-                  int HKV, int max_blocks, int NS, float scale) {
+                  float* pacc, float* pml, int* arrived, int H, int HKV,
+                  int max_blocks, int NS, float scale) {
   constexpr int NCH = D / 8;            // 16-byte pieces of a bf16 row
   constexpr int ROWS = 1024 / (2 * D);  // rows of a 1 KiB piece of a tile
   constexpr int PIECES = KT / ROWS;     // pieces of K or V of a tile
@@ -110,18 +217,6 @@ paged_attn_kernel(const unsigned short* __restrict__ q, long q_stride,
   const int* bt = block_table + (long)b * max_blocks;
   const long page_bytes = (long)HKV * PBLK * D * (FP8 ? 1 : 2);
   const long head_bytes = (long)kvh * PBLK * D * (FP8 ? 1 : 2);
-
-  bf16x8 qf[D / 32];
-#pragma unroll
-  for (int s = 0; s < D / 32; ++s) {
-    pa_frag f;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) f.d[i] = 0;
-    if (c16 < nh)
-      f.v = *reinterpret_cast<const bf16x8*>(
-          q + b * q_stride + (long)(head0 + c16) * D + s * 32 + g * 8);
-    qf[s] = f.v;
-  }
 
   // page numbers of the wave's next 32 tiles, two a tile, on the lanes
   int pages = 0;
@@ -180,6 +275,100 @@ paged_attn_kernel(const unsigned short* __restrict__ q, long q_stride,
             ring + TILE + row * (2 * D) + ((c + e) ^ ((row & 3) << 1)) * 16) =
             w[e];
     }
+  };
+
+  // the first tile is on its way while the queries come
+  int at = 0;  // tiles issued
+  auto next = [&]() {
+    if ((at & 31) == 0) fetch_pages(at);
+    if constexpr (FP8) issue8(at++);
+    else issue(at++);
+  };
+  while (at < (R > 1 ? R - 1 : 1) && at < mine) next();
+
+  const int pos = STEP ? ctx_len[b] - 1 : 0;
+  // of the workgroup, of the wave: its share ends with the new token
+  const bool newest = STEP && pos >= 0 && pos < max_blocks * PBLK && T > 0 &&
+                      T - 1 >= split * per && T - 1 < split * per + per;
+  const bool renews = newest && mine > 0 && t0 + (mine - 1) * NW == T - 1;
+  // rotated queries, the new key and value: rows of D in LDS
+  char* rows = smem + pa_lds(D, R);
+  if constexpr (STEP) {
+    const int nb = gridDim.x / NS / NG / HKV, heads = H + 2 * HKV;
+    const int units = (nh + (newest ? 2 : 0)) * (D / 8);
+    for (int u = threadIdx.x; u < units && pos >= 0; u += NW * 64) {
+      const int row = u / (D / 8), c = u % (D / 8) * 4;
+      const int h = row < nh ? head0 + row
+                             : H + (row - nh) * HKV + kvh;
+      unsigned short a[4], e[4];
+      step_columns<D>(step, nb, heads, b, h, c, row <= nh, pos, a, e);
+      if (row >= nh) {
+        char* to = (row == nh ? kcache : vcache) +
+                   bt[pos / PBLK] * page_bytes + head_bytes +
+                   (long)(pos % PBLK) * D * (FP8 ? 1 : 2);
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+          unsigned short* x = half ? e : a;
+          const int col = c + half * (D / 2);
+          if constexpr (FP8) {
+            unsigned char eight[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              cache_store(&eight[i], x[i]);
+              __hip_fp8_e4m3 f;
+              f.__x = eight[i];
+              x[i] = f2bf((float)f);
+            }
+            if (hg == 0)
+#pragma unroll
+              for (int i = 0; i < 4; ++i) to[col + i] = (char)eight[i];
+          } else if (hg == 0) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              reinterpret_cast<unsigned short*>(to)[col + i] = x[i];
+          }
+        }
+      }
+      *reinterpret_cast<i32x2*>(rows + (row * D + c) * 2) =
+          *reinterpret_cast<const i32x2*>(a);
+      *reinterpret_cast<i32x2*>(rows + (row * D + c + D / 2) * 2) =
+          *reinterpret_cast<const i32x2*>(e);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  }
+  bf16x8 qf[D / 32];
+#pragma unroll
+  for (int s = 0; s < D / 32; ++s) {
+    pa_frag f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) f.d[i] = 0;
+    if (c16 < nh) {
+      if constexpr (STEP)
+        f.v = *reinterpret_cast<const bf16x8*>(
+            rows + (c16 * D + s * 32 + g * 8) * 2);
+      else
+        f.v = *reinterpret_cast<const bf16x8*>(
+            q + b * q_stride + (long)(head0 + c16) * D + s * 32 + g * 8);
+    }
+    qf[s] = f.v;
+  }
+
+  // the new token's row of the last tile, which holds what was in the cache
+  auto renew = [&](int i) {
+    const int row = (L - 1) % KT, c = lane % NCH;
+    char* kt = ring + (i % R) * 2 * TILE + row * (2 * D);
+    if (lane < 2 * NCH) {
+      const i32x4 x = *reinterpret_cast<const i32x4*>(
+          rows + (nh + lane / NCH) * (2 * D) + c * 16);
+      if (lane < NCH)
+        *reinterpret_cast<i32x4*>(kt + ((c ^ (row & (NCH - 1))) * 16)) = x;
+      else
+        *reinterpret_cast<i32x4*>(kt + TILE + ((c ^ ((row & 3) << 1)) * 16)) =
+            x;
+    }
+    wave_sync();
   };
 
   const float scale2 = scale * 1.4426950408889634f;
@@ -273,38 +462,22 @@ paged_attn_kernel(const unsigned short* __restrict__ q, long q_stride,
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   };
 
-  if constexpr (FP8) {
-    if (mine > 0) {
-      fetch_pages(0);
-      issue8(0);
-    }
-    for (int i = 0; i < mine; ++i) {
+  for (int i = 0; i < mine; ++i) {
+    if constexpr (FP8) {
       store8();
-      if (i + 1 < mine) {
-        if (((i + 1) & 31) == 0) fetch_pages(i + 1);
-        issue8(i + 1);
-      }
+      if (at < mine) next();
       wave_sync();
-      compute(i);
-    }
-  } else {
-    int at = 0;  // tiles issued
-    auto next = [&]() {
-      if ((at & 31) == 0) fetch_pages(at);
-      issue(at++);
-    };
-    while (at < R - 1 && at < mine) next();
-    for (int i = 0; i < mine; ++i) {
-      if (at < mine) {
-        next();
+    } else {
+      if (at < mine && at < i + R) next();
+      if (at == i + R)
         asm volatile("s_waitcnt vmcnt(%0)" ::"i"((R - 1) * 2 * PIECES)
                      : "memory");
-      } else {
+      else
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      }
       if constexpr (!ALIGNED) wave_sync();
-      compute(i);
     }
+    if (renews && i == mine - 1) renew(i);
+    compute(i);
   }
 
   // ---- the waves' states meet ---------------------------------------------
@@ -346,11 +519,51 @@ paged_attn_kernel(const unsigned short* __restrict__ q, long q_stride,
       *reinterpret_cast<i32x2*>(out + ((long)b * H + head0 + head) * D + col) =
           two;
     } else {
-      *reinterpret_cast<f32x4*>(pacc + (part + head) * D + col) = o;
-      if (col == 0) {
-        pml[(part + head) * 2] = M;
-        pml[(part + head) * 2 + 1] = sum;
+      float* to = pacc + (part + head) * D + col;
+      pa_put<STEP>(to, o[0], o[1]);
+      pa_put<STEP>(to + 2, o[2], o[3]);
+      if (col == 0) pa_put<STEP>(pml + (part + head) * 2, M, sum);
+    }
+  }
+  if constexpr (STEP) {
+    // The last of a sequence's workgroups joins their results, which saves a
+    // launch (4.7 us). Results and count are agent-scope atomics, which meet in
+    // memory that all XCDs see; every wave's are there before the barrier ahead of
+    // the count.
+    if (NS == 1) return;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    int* last = reinterpret_cast<int*>(smem);
+    if (threadIdx.x == 0)
+      *last = __hip_atomic_fetch_add(arrived + (b * HKV + kvh) * NG + hg, 1,
+                                     __ATOMIC_RELAXED,
+                                     __HIP_MEMORY_SCOPE_AGENT) == NS - 1;
+    __syncthreads();
+    if (!*last) return;
+    const long first = (long)(b * HKV + kvh) * NS * GR + hg * 16;
+    float* state = reinterpret_cast<float*>(smem) + 4;  // [NS][nh][2]
+    for (int i = threadIdx.x; i < NS * nh; i += NW * 64)
+      *reinterpret_cast<f32x2*>(state + i * 2) =
+          pa_get(pml + (first + (long)(i / nh) * GR + i % nh) * 2);
+    __syncthreads();
+    for (int i = threadIdx.x; i < nh * (D / 2); i += NW * 64) {
+      const int head = i / (D / 2), col = i % (D / 2) * 2;
+      const float* from = pacc + (first + head) * D + col;
+      const float* st = state + head * 2;
+      float M = -1e30f, sum = 0.f;
+      for (int s = 0; s < NS; ++s) M = fmaxf(M, st[s * nh * 2]);
+      f32x2 o = {0.f, 0.f};
+#pragma unroll 8
+      for (int s = 0; s < NS; ++s) {
+        const float a = __builtin_amdgcn_exp2f(st[s * nh * 2] - M);
+        const f32x2 v = pa_get(from + (long)s * GR * D);
+        sum += a * st[s * nh * 2 + 1];
+        o[0] += a * v[0];
+        o[1] += a * v[1];
       }
+      const float inv = sum > 0.f ? 1.f / sum : 0.f;
+      *reinterpret_cast<unsigned int*>(out + ((long)b * H + head0 + head) * D +
+                                       col) = pa_pack(o[0] * inv, o[1] * inv);
     }
   }
 }
@@ -394,22 +607,24 @@ paged_attn_combine_kernel(const float* __restrict__ pacc,
     out[(long)row * D + lane * DPL + i] = f2bf(o[i] * inv);
 }
 
-extern "C" void launch_paged_attn(const void* q, long q_stride,
-                                  const void* kcache, const void* vcache,
-                                  const int* block_table, const int* ctx_len,
-                                  void* out, void* pacc, void* pml, int B,
-                                  int H, int HKV, int D, int max_blocks,
-                                  int NS, float scale, bool fp8,
-                                  bool aligned, hipStream_t stream) {
+// step: a decode step's projections in the place of q, arrived: a zero for every
+// B * HKV * groups of 16 query heads, where NS > 1
+static void pa_launch(const void* q, long q_stride, const PaStep* step,
+                      void* kcache, void* vcache, const int* block_table,
+                      const int* ctx_len, void* out, void* pacc, void* pml,
+                      int* arrived, int B, int H, int HKV, int D,
+                      int max_blocks, int NS, float scale, bool fp8,
+                      bool aligned, hipStream_t stream) {
   const int GR = H / HKV, NG = (GR + 15) / 16;
   const int grid = B * HKV * NG * NS;
-#define PA(DD, F8, AL, R)                                                     \
-  hipLaunchKernelGGL((paged_attn_kernel<DD, F8, AL, R>), dim3(grid),          \
-                     dim3(256), pa_lds(DD, R), stream,                        \
-                     (const unsigned short*)q, q_stride, (const char*)kcache, \
-                     (const char*)vcache, block_table, ctx_len,               \
-                     (unsigned short*)out, (float*)pacc, (float*)pml, H, HKV, \
-                     max_blocks, NS, scale)
+  const PaStep in = step != nullptr ? *step : PaStep{};
+#define PA(DD, F8, AL, R, ST)                                                 \
+  hipLaunchKernelGGL((paged_attn_kernel<DD, F8, AL, R, ST>), dim3(grid),      \
+                     dim3(256), pa_lds(DD, R) + (ST ? 18 * DD * 2 : 0), stream, \
+                     (const unsigned short*)q, q_stride, in, (char*)kcache,   \
+                     (char*)vcache, block_table, ctx_len,                     \
+                     (unsigned short*)out, (float*)pacc, (float*)pml,         \
+                     arrived, H, HKV, max_blocks, NS, scale)
 // Tiles in a wave's ring. Two tiles of 128 columns leave a CU to one workgroup;
 // from 1024 workgroups on, four for every CU, a second one on the CU counts for
 // more, for short contexts are a chain of three reads each. In us, 64 x 32 heads
@@ -417,17 +632,33 @@ extern "C" void launch_paged_attn(const void* q, long q_stride,
 // 40, 213 (two waves 12, 38, 217 to 226: the long ones wait for each other).
 // 64 x 8 heads, grouped: two 8.8, 16.9, 53; one 6.4, 14.6, 55. With heads of 64,
 // 64 x 32: four tiles 22, 38, 120; two 14, 24, 109.
-#define PA_D(DD)                                                      \
+#define PA_D(DD, ST)                                                  \
   do {                                                                \
-    if (fp8) PA(DD, true, true, 1);                                   \
-    else if (!aligned) PA(DD, false, false, 1);                       \
-    else if (DD == 128 && grid >= 1024) PA(DD, false, true, 1);       \
-    else PA(DD, false, true, 2);                                      \
+    if (fp8) PA(DD, true, true, 1, ST);                               \
+    else if (!aligned) PA(DD, false, false, 1, ST);                   \
+    else if (DD == 128 && grid >= 1024) PA(DD, false, true, 1, ST);   \
+    else PA(DD, false, true, 2, ST);                                  \
   } while (0)
-  if (D == 64) PA_D(64);
-  else PA_D(128);
+  if (step != nullptr) {
+    if (D == 64) PA_D(64, true);
+    else PA_D(128, true);
+  } else {
+    if (D == 64) PA_D(64, false);
+    else PA_D(128, false);
+  }
 #undef PA_D
 #undef PA
+}
+
+extern "C" void launch_paged_attn(const void* q, long q_stride, void* kcache,
+                                  void* vcache, const int* block_table,
+                                  const int* ctx_len, void* out, void* pacc,
+                                  void* pml, int B, int H, int HKV, int D,
+                                  int max_blocks, int NS, float scale,
+                                  bool fp8, bool aligned, hipStream_t stream) {
+  pa_launch(q, q_stride, nullptr, kcache, vcache, block_table, ctx_len, out,
+            pacc, pml, nullptr, B, H, HKV, D, max_blocks, NS, scale, fp8,
+            aligned, stream);
   if (NS > 1) {
     const int rows = B * H;
 #define PC(DD)                                                                \
@@ -441,14 +672,19 @@ extern "C" void launch_paged_attn(const void* q, long q_stride,
   }
 }
 
-// Cache element of a bf16 number.
-__device__ __forceinline__ void cache_store(unsigned short* p,
-                                            unsigned short v) {
-  *p = v;
-}
-__device__ __forceinline__ void cache_store(unsigned char* p,
-                                            unsigned short v) {
-  *p = __hip_fp8_e4m3(bf2f(v)).__x;
+extern "C" void launch_step_attn(const void* qkv, const float* parts, int S,
+                                 const void* bias, const float* cs,
+                                 const float* sn, void* kcache, void* vcache,
+                                 const int* block_table, const int* ctx_len,
+                                 void* out, void* pacc, void* pml,
+                                 int* arrived, int B, int H, int HKV, int D,
+                                 int max_blocks, int NS, float scale, bool fp8,
+                                 bool aligned, hipStream_t stream) {
+  const PaStep step = {(const unsigned short*)qkv, parts, S,
+                       (const unsigned short*)bias, cs, sn};
+  pa_launch(nullptr, 0, &step, kcache, vcache, block_table, ctx_len, out, pacc,
+            pml, arrived, B, H, HKV, D, max_blocks, NS, scale, fp8, aligned,
+            stream);
 }
 
 // Write one new token's K/V into the paged cache (decode step).
@@ -499,7 +735,8 @@ extern "C" void launch_cache_put(const void* knew, const void* vnew,
 #undef CP
 }
 
-// A decode step's projections qkv [B, H + 2 HKV, D] on their way: queries and
+// A decode step's projections qkv [B, H + 2 HKV, D] on their way, for callers
+// that attend by themselves (the attention kernel does this too): queries and
 // keys are rotated by the position ctx - 1 of the new token (half-split, fp32,
 // tables [positions, D / 2]); queries go to q [B, H, D], keys and values to
 // their place in the cache. One launch for what a rotation, three copies and
@@ -510,11 +747,8 @@ extern "C" void launch_cache_put(const void* knew, const void* vnew,
 // in a graph, 64 rows 20.8 -> 18.6 us, 17 rows 18.4 -> 15.7).
 template <int D, typename CT>
 __global__ void __launch_bounds__(256)
-rope_put_kernel(const unsigned short* __restrict__ qkv,
-                const float* __restrict__ parts, int S,
-                const unsigned short* __restrict__ bias,
-                const float* __restrict__ cs, const float* __restrict__ sn,
-                const int* __restrict__ ctx, unsigned short* __restrict__ q,
+rope_put_kernel(const PaStep p, const int* __restrict__ ctx,
+                unsigned short* __restrict__ q,
                 CT* __restrict__ kcache, CT* __restrict__ vcache,
                 const int* __restrict__ block_table, int B, int H, int HKV,
                 int max_blocks) {
@@ -525,45 +759,8 @@ rope_put_kernel(const unsigned short* __restrict__ qkv,
   const int c = (int)(i % PER) * 4;
   const int h = (int)(i / PER % heads), b = (int)(i / PER / heads);
   const int pos = ctx[b] - 1;
-  const unsigned short* x = qkv + ((long)b * heads + h) * D + c;
   unsigned short a[4], e[4];
-  if (S == 0) {
-    *reinterpret_cast<i32x2*>(a) = *reinterpret_cast<const i32x2*>(x);
-    *reinterpret_cast<i32x2*>(e) = *reinterpret_cast<const i32x2*>(x + D / 2);
-  } else {
-    f32x4 va = {0.f, 0.f, 0.f, 0.f}, ve = va;
-    const float* p = parts + ((long)b * heads + h) * D + c;
-#pragma unroll 4
-    for (int s = 0; s < S; ++s) {
-      const f32x4 pa = *reinterpret_cast<const f32x4*>(p);
-      const f32x4 pe = *reinterpret_cast<const f32x4*>(p + D / 2);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        va[j] += pa[j];
-        ve[j] += pe[j];
-      }
-      p += (long)B * heads * D;
-    }
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      if (bias != nullptr) {
-        va[j] += bf2f(bias[h * D + c + j]);
-        ve[j] += bf2f(bias[h * D + D / 2 + c + j]);
-      }
-      a[j] = f2bf(va[j]);
-      e[j] = f2bf(ve[j]);
-    }
-  }
-  if (h < H + HKV) {
-    const f32x4 co = *reinterpret_cast<const f32x4*>(cs + (long)pos * (D / 2) + c);
-    const f32x4 si = *reinterpret_cast<const f32x4*>(sn + (long)pos * (D / 2) + c);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const float x1 = bf2f(a[j]), x2 = bf2f(e[j]);
-      a[j] = f2bf(x1 * co[j] - x2 * si[j]);
-      e[j] = f2bf(x2 * co[j] + x1 * si[j]);
-    }
-  }
+  step_columns<D>(p, B, heads, b, h, c, h < H + HKV, pos, a, e);
   if (h < H) {
     unsigned short* o = q + ((long)b * H + h) * D + c;
     *reinterpret_cast<i32x2*>(o) = *reinterpret_cast<const i32x2*>(a);
@@ -589,11 +786,12 @@ extern "C" void launch_rope_put(const void* qkv, const float* parts, int S,
                                 int D, int max_blocks, bool fp8,
                                 hipStream_t stream) {
   const long total = (long)B * (H + 2 * HKV) * (D / 8);
+  const PaStep p = {(const unsigned short*)qkv, parts, S,
+                    (const unsigned short*)bias, cs, sn};
 #define RP(DD, CT)                                                            \
   hipLaunchKernelGGL((rope_put_kernel<DD, CT>), dim3((total + 255) / 256),    \
-                     dim3(256), 0, stream, (const unsigned short*)qkv, parts, \
-                     S, (const unsigned short*)bias, cs, sn, ctx,             \
-                     (unsigned short*)q, (CT*)kcache, (CT*)vcache,            \
+                     dim3(256), 0, stream, p, ctx, (unsigned short*)q,        \
+                     (CT*)kcache, (CT*)vcache,            \
                      block_table, B, H, HKV, max_blocks)
   if (D == 64) {
     if (fp8) RP(64, unsigned char); else RP(64, unsigned short);

@@ -210,3 +210,96 @@ def test_infinite_values(device, D, shares, monkeypatch):
     want = _want(q, k, v, table, lens, D ** -0.5)
     assert torch.equal(out.isnan(), want.isnan()) and want.isnan().any()
     torch.testing.assert_close(out, want, equal_nan=True, **TOL)
+
+
+def _step(device, lens, H, HKV, D, fp8, width, slabs=0, seed=0):
+    """A step's projections and pages whose new rows hold NaN."""
+    k, v, table = _pages(len(lens), HKV, D, [n - 1 for n in lens], width, fp8,
+                         seed, device)
+    raw = [t.view(torch.uint8) if fp8 else t for t in (k, v)]
+    cs, sn = ops.rope_tables(width * 16, D, device=device)
+    g = torch.Generator().manual_seed(seed)
+    shape = (len(lens), H + 2 * HKV, D)
+    if slabs:
+        qkv = torch.randn(slabs, *shape, generator=g).to(device)
+        bias = torch.randn(shape[1] * D, generator=g).bfloat16().to(device)
+    else:
+        qkv, bias = torch.randn(*shape, generator=g).bfloat16().to(device), None
+    ctx = torch.tensor(lens, dtype=torch.int32, device=device)
+    return qkv, cs, sn, ctx, raw, table, bias
+
+
+def _same_step(device, qkv, cs, sn, ctx, raw, table, bias):
+    """In one launch as in two."""
+    two = [t.clone() for t in raw]
+    HKV, D = raw[0].shape[1], raw[0].shape[3]
+    H = qkv.shape[-2] - 2 * HKV
+    scale = D ** -0.5
+    q = ops.rope_put(qkv, cs, sn, ctx, *two, table, bias)
+    want = ops.paged_attn(q, *two, table, ctx, scale)
+    zeros = ops.step_zeros(1, len(ctx), H, raw[0], table)
+    got = ops.step_attn(qkv, cs, sn, ctx, *raw, table, bias, scale,
+                        None if zeros is None else zeros[0])
+    assert not got.isnan().any()
+    torch.testing.assert_close(got.float(), want.float(), **TOL)
+    for a, b in zip(raw, two):
+        torch.testing.assert_close(a, b, atol=0, rtol=0, equal_nan=True)
+    return zeros
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("H,HKV", [(4, 4), (10, 2), (20, 1), (32, 8)])
+@pytest.mark.parametrize("slabs", [0, 3])
+def test_step(device, H, HKV, D, fp8, slabs):
+    lens = [1, 2, 16, 17, 31, 32, 33, 127, 128, 129, 257, 320]
+    _same_step(device, *_step(device, lens, H, HKV, D, fp8, 20, slabs))
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("shares", ["", "2", "7", "64"])
+@pytest.mark.parametrize("lens,width,H,HKV", [
+    ([4800], 300, 32, 8), ([33], 300, 8, 2), ([1, 1600, 777], 100, 20, 1)])
+def test_step_shares(device, lens, width, H, HKV, shares, fp8, monkeypatch):
+    """Shares joined by the last of them, those without keys among them."""
+    if shares:
+        monkeypatch.setenv("DISTLLM_PA_NSPLIT", shares)
+    args = _step(device, lens, H, HKV, 128, fp8, width)
+    zeros = _same_step(device, *args)
+    n = ops._hip_ops.step_attn_shares(len(lens), H, HKV, width, fp8)
+    assert (zeros == n).all() if n > 1 else zeros is None
+
+
+def test_step_unaligned_pages(device):
+    args = list(_step(device, [50, 300], 8, 2, 64, False, 20))
+    odd = []
+    for t in args[4]:
+        flat = torch.empty(t.numel() + 1, dtype=t.dtype, device=device)
+        flat[1:] = t.reshape(-1)
+        odd.append(flat[1:].view(t.shape))
+    args[4] = odd
+    _same_step(device, *args)
+
+
+def test_step_in_a_graph(device):
+    """Replayed, with other work between, as run."""
+    qkv, cs, sn, ctx, raw, table, _ = _step(device, [2000, 1, 640], 32, 8, 128,
+                                            False, 128)
+
+    def run():
+        zeros = ops.step_zeros(2, 3, 32, raw[0], table)
+        return [ops.step_attn(qkv * f, cs, sn, ctx, *raw, table, None, 0.1,
+                              zeros[i]) for i, f in enumerate((1.0, 0.5))]
+
+    want = [t.clone() for t in run()]
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = run()
+    for _ in range(4):
+        for t in got:
+            t.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
+        run()
