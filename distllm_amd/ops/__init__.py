@@ -256,31 +256,50 @@ def _recorded(*tensors) -> bool:
 _WIDE_SWIGLU, _WIDE_CLAMPED = 4, 5
 
 
+def _own_product(x2, weight, bias) -> bool:
+    """Whether the operands are as mid_gemm and wide_gemm take them and nothing
+    asks for another product."""
+    return (x2.dtype == weight.dtype == torch.bfloat16
+            and x2.is_contiguous() and weight.is_contiguous()
+            and x2.device == weight.device
+            and (bias is None or (
+                bias.dtype == torch.bfloat16
+                and bias.shape == weight.shape[:1]
+                and bias.is_contiguous() and bias.device == x2.device))
+            and _gemm_mode() not in _OTHER_FORMS
+            and not _recorded(x2, weight, bias))
+
+
+def _mid_shares(x2, weight, bias) -> int:
+    """The shares of K with which x2 @ weight^T goes by csrc/decode_gemm.hip's
+    blocks of 64 rows, 0 where it does not (mid_gemm_shares there has the
+    measurements)."""
+    M, K = x2.shape
+    N = weight.shape[0]
+    if M <= 64 or M * N > 512 * 4096:  # tiles of 64 x 64
+        return 0
+    shares = _hip_ops.mid_gemm_shares(M, N, K)
+    return shares if shares and _own_product(x2, weight, bias) else 0
+
+
 def _wide_tile(x2, weight, bias, act) -> int:
     """The tile with which x2 @ weight^T, bias and activation or gated unit go
     in one launch of csrc/wide_gemm.hip, 0 where another way is faster (the
     measurements are there, at wide_gemm_tile) or has to be taken."""
     M, K = x2.shape
     N = weight.shape[0]
-    if M <= 64 or (act == ACT_NONE and M <= 256):
+    if (M <= 64 or M * N < 96 * 127 * 256  # its least tiles
+            or (act == ACT_NONE and M <= 256)):
         return 0
     tile = _hip_ops.wide_gemm_tile(M, N, K, act)
-    if (tile and x2.dtype == weight.dtype == torch.bfloat16
-            and x2.is_contiguous() and weight.is_contiguous()
-            and x2.device == weight.device
-            and (bias is None or (
-                bias.dtype == torch.bfloat16 and bias.shape == (N,)
-                and bias.is_contiguous() and bias.device == x2.device))
-            and _gemm_mode() not in _OTHER_FORMS
-            and not _recorded(x2, weight, bias)):
-        return tile
-    return 0
+    return tile if tile and _own_product(x2, weight, bias) else 0
 
 
 def linear(x, weight, bias=None, act=ACT_NONE):
     """Linear layer entry used by models. GPU path: the products of few rows
-    (decode_gemm.hip, with the activation) for M <= 64 (_few_rows), those of
-    many rows (wide_gemm.hip, with the activation) where _wide_tile says so;
+    (decode_gemm.hip, with the activation) for M <= 64 (_few_rows) and, by
+    blocks of them, where _mid_shares says so, those of many rows
+    (wide_gemm.hip, with the activation) where _wide_tile says so;
     else an autotuned choice between hipBLASLt (plain and fused-epilogue), the
     other hand-written MFMA GEMMs (gemm8.hip, 8-phase gemm16.hip) and, for M
     <= 256, decode_gemm.hip. Override with
@@ -301,6 +320,11 @@ def linear(x, weight, bias=None, act=ACT_NONE):
                 and _few_rows(x2, weight, bias)):
             out = _hip_ops.decode_gemm(x2, weight, bias, 0, _DECODE_ACT[act])
             return out.reshape(*orig_shape[:-1], N)
+        shares = _mid_shares(x2, weight, bias)
+        if shares:
+            return _hip_ops.mid_gemm(x2, weight, bias, shares,
+                                     _DECODE_ACT[act]).view(
+                *orig_shape[:-1], N)
         tile = _wide_tile(x2, weight, bias, act)
         if tile:
             return _hip_ops.wide_gemm(x2, weight, bias, act, tile).view(

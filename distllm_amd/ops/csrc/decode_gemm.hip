@@ -1,4 +1,5 @@
-// Products of few rows: out[M,N] = x[M,K] @ W[N,K]^T, M <= 256, with bias
+// Products of few rows: out[M,N] = x[M,K] @ W[N,K]^T, M <= 256 and, of few
+// columns or a short K, up to some thousand, with bias
 // and activation in the same launch where K is not split over workgroups.
 // Replaces the skinny-M GEMMs vLLM issues per decode step (reference
 // delegated generation to vLLM, distllm/generate/generators/
@@ -20,7 +21,7 @@
 //  tile    above: W and x tiles of 64 columns of K in a ring that 4 or 8
 //          waves share, one barrier per chunk; where N alone does not fill
 //          the chip K is split over workgroups and a second launch sums fp32
-//          slabs.
+//          slabs. Some hundred rows go by blocks of 64 (mid_gemm_shares).
 //
 // Measured in a graph over fresh weights, us (GB/s of weights); before: the
 // faster of a two-stage tile of 128 rows with slabs and the library:
@@ -354,7 +355,8 @@ dg_tile_kernel(const u16* __restrict__ X, const u16* __restrict__ W,
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   const int r = lane & 15, g = lane >> 4;
   const int ncb = e.N / 64;
-  const int cb = blockIdx.x % ncb, ks = blockIdx.x / ncb;
+  const int cb = blockIdx.x % ncb, ks = blockIdx.x / ncb % splitk;
+  const int m0 = blockIdx.x / ncb / splitk * MP;  // the tile's first row
   const int nt = K / splitk / 64, n0 = cb * (GLU ? 32 : 64);
   const int lr = lane >> 3, lc = ((lane & 7) ^ lr) * 8;
   const u16* src[LOADS];
@@ -363,7 +365,7 @@ dg_tile_kernel(const u16* __restrict__ X, const u16* __restrict__ W,
     const int row = (wid * LOADS + p) * 8 + lr;
     src[p] = (row < 64
                   ? W + (long)(dg_wrow<GLU>(n0, row >> 4, e.N) + (row & 15)) * K
-                  : X + (long)min(row - 64, e.M - 1) * K) +
+                  : X + (long)min(m0 + row - 64, e.M - 1) * K) +
              ks * (K / splitk) + lc;
   }
   auto issue = [&](int c) {
@@ -436,7 +438,7 @@ dg_tile_kernel(const u16* __restrict__ X, const u16* __restrict__ W,
   }
 #pragma unroll
   for (int j = 0; j < FM; ++j) {
-    const int m = (wm * FM + j) * 16 + r;
+    const int m = m0 + (wm * FM + j) * 16 + r;
     if (m >= e.M) continue;
     if constexpr (SLAB) {
 #pragma unroll
@@ -508,9 +510,38 @@ extern "C" int decode_gemm_shares(int M, int N, int K) {
   return best;
 }
 
+// How many workgroups share K where 65 rows and more go by tiles of 64 x 64, 0
+// where another product is to be taken. Tiles have to fit the card twice over,
+// and the sums, 0.22 us for 64 of K and 4.5 for the launch that joins shares, have
+// to stay below what the library's product costs the host alone, 19 us a call
+// (this one 6): an encoder of some hundred rows issues its layers slower than it
+// runs them. Measured in a graph, us, library and this: 300 rows of 2304 x 768 6.8
+// and 6.0, 768 x 768 4.9 and 5.6, 3072 x 768 with GELU 10.0 and 6.5, 768 x 3072
+// (4 shares) 8.4 and 10.1, 1280 x 5120 (2) 16.7 and 15.2; 800 rows 8.6 and 8.3, 6.6
+// and 5.8, 14.7 and 12.8, 14.1 and 14.6; 2000 rows of 768 x 768 8.6 and 8.0. With
+// more tiles it is the slower one: 1300 rows of 2304 x 768 10.2 and 12.8, 800 of
+// 3840 x 1280 14.8 and 20.7.
+extern "C" int mid_gemm_shares(int M, int N, int K) {
+  if (M <= 64 || N <= 0 || N % 64 || K % 64 || K < 128) return 0;
+  const long tiles = (long)((M + 63) / 64) * (N / 64);
+  if (tiles > 512) return 0;
+  if (K <= 1536) return 1;
+  int best = 0;
+  float least = 16.f;
+  for (int s = 1; s <= 4; s *= 2) {
+    if (K % (64 * s) || (s > 1 && tiles * s > 256)) continue;
+    const float us = 2.5f + 0.22f * (K / 64 / s) * (tiles > 256 ? 1.5f : 1.f) +
+                     (s > 1 ? 4.5f : 0.f);
+    if (us >= least) continue;
+    least = us;
+    best = s;
+  }
+  return best;
+}
+
 template <int ACT>
 static void dg_launch(const u16* X, const u16* W, float* slabs, int K,
-                      int splitk, bool tile, const DgEnd& e, hipStream_t st) {
+                      int splitk, int tile, const DgEnd& e, hipStream_t st) {
   constexpr bool GLU = dg_glu(ACT);
   constexpr int NT = GLU ? 2 : 1;
 #define DG_RING(MT, R)                                                       \
@@ -531,9 +562,9 @@ static void dg_launch(const u16* X, const u16* W, float* slabs, int K,
     return;
   }
 #undef DG_RING
-  const int grid = e.N / 64 * splitk;
 #define DG_TILE(MP, R)                                                       \
   do {                                                                       \
+    const int grid = e.N / 64 * splitk * ((e.M + MP - 1) / MP);              \
     if (splitk > 1)                                                          \
       hipLaunchKernelGGL((dg_tile_kernel<ACT, MP, R, true>), dim3(grid),     \
                          dim3(MP == 32 ? 256 : 512), dg_tile_lds(MP, R), st, \
@@ -543,9 +574,10 @@ static void dg_launch(const u16* X, const u16* W, float* slabs, int K,
                          dim3(MP == 32 ? 256 : 512), dg_tile_lds(MP, R), st, \
                          X, W, slabs, K, splitk, e);                         \
   } while (0)
-  if (e.M <= 32) DG_TILE(32, 4);
-  else if (e.M <= 64) DG_TILE(64, 4);
-  else if (e.M <= 128) DG_TILE(128, 3);
+  const int rows = tile > 1 ? tile : e.M;
+  if (rows <= 32) DG_TILE(32, 4);
+  else if (rows <= 64) DG_TILE(64, 4);
+  else if (rows <= 128) DG_TILE(128, 3);
   else DG_TILE(256, 3);
 #undef DG_TILE
   if (splitk > 1 && e.out != nullptr) {
@@ -555,11 +587,12 @@ static void dg_launch(const u16* X, const u16* W, float* slabs, int K,
   }
 }
 
-// tile: the tile form whatever M is; splitk workgroups share K there. Without
+// tile: the tile form whatever M is; splitk workgroups share K there. 64: by
+// blocks of 64 rows. Without
 // an out the slabs are left for the next kernel to sum.
 extern "C" void launch_decode_gemm(const void* X, const void* W,
                                    const void* bias, void* out, void* slabs,
-                                   int M, int N, int K, int splitk, bool tile,
+                                   int M, int N, int K, int splitk, int tile,
                                    int act, float limit, float alpha,
                                    float shift, const float* act_nums,
                                    const RowsArgs* rows,

@@ -14,7 +14,7 @@ void launch_attn_fwd(const void*, const void*, const void*, const float*,
                      void*, int, int, int, int, int, int, bool, float, long,
                      long, long, long, hipStream_t);
 void launch_decode_gemm(const void*, const void*, const void*, void*, void*,
-                        int, int, int, int, bool, int, float, float, float,
+                        int, int, int, int, int, int, float, float, float,
                         const float*, const RowsArgs*, hipStream_t);
 int decode_gemm_shares(int, int, int);
 }

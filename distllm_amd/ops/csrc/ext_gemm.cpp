@@ -12,9 +12,10 @@ void launch_gemm8_bf16(const void*, const void*, const void*, void*, int, int,
 void launch_gemm16_bf16(const void*, const void*, const void*, void*, int,
                         int, int, int, hipStream_t);
 void launch_decode_gemm(const void*, const void*, const void*, void*, void*,
-                        int, int, int, int, bool, int, float, float, float,
+                        int, int, int, int, int, int, float, float, float,
                         const float*, const RowsArgs*, hipStream_t);
 int decode_gemm_shares(int, int, int);
+int mid_gemm_shares(int, int, int);
 void launch_norm_gemm(const void*, const void*, const void*, void*, float,
                       const void*, const void*, void*, int, int, int,
                       hipStream_t);
@@ -199,6 +200,43 @@ torch::Tensor wide_gemm(torch::Tensor X, torch::Tensor W,
   return out;
 }
 
+// X W^T of 65 rows and more by tiles of 64 x 64; shares as mid_gemm_shares
+// gives them; act 0, 6, 7, 8 as of decode_gemm.
+torch::Tensor mid_gemm(torch::Tensor X, torch::Tensor W,
+                       c10::optional<torch::Tensor> bias, int64_t shares,
+                       int64_t act) {
+  CHECK_DEV(X); CHECK_CONT(X); CHECK_BF16(X);
+  CHECK_DEV(W); CHECK_CONT(W); CHECK_BF16(W);
+  TORCH_CHECK(X.dim() == 2 && W.dim() == 2 && W.size(1) == X.size(1) &&
+                  X.device() == W.device(),
+              "operands");
+  const int64_t M = X.size(0), K = X.size(1), N = W.size(0);
+  TORCH_CHECK(M > 0 && N > 0 && N % 64 == 0 && K >= 128 && shares >= 1 &&
+                  shares <= 4 && K % (64 * shares) == 0 &&
+                  M * N < 1L << 30,
+              "mid_gemm: sizes");
+  TORCH_CHECK(act == 0 || (act >= 6 && act <= 8), "activation");
+  const c10::DeviceGuard guard(X.device());
+  if (bias) {
+    CHECK_DEV(bias.value()); CHECK_CONT(bias.value());
+    CHECK_BF16(bias.value());
+    TORCH_CHECK(bias->numel() == N && bias->device() == X.device(),
+                "bias must be [N]");
+  }
+  auto out = torch::empty({M, N}, X.options());
+  X = aligned16(X);
+  W = aligned16(W);
+  torch::Tensor slabs;
+  if (shares > 1)
+    slabs = torch::empty({shares, M, N}, X.options().dtype(at::kFloat));
+  launch_decode_gemm(X.data_ptr(), W.data_ptr(),
+                     bias ? bias->data_ptr() : nullptr, out.data_ptr(),
+                     shares > 1 ? slabs.data_ptr() : nullptr, (int)M, (int)N,
+                     (int)K, (int)shares, 64, (int)act, 0.f, 0.f, 0.f, nullptr,
+                     nullptr, cur_stream());
+  return out;
+}
+
 // x = a + b, one row, and the product of its RMS norm (act 1: gated unit)
 std::vector<torch::Tensor> norm_gemm(torch::Tensor a, torch::Tensor b,
                                      torch::Tensor w_norm, double eps,
@@ -309,6 +347,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("act"), py::arg("tile"), py::arg("limit") = 0.0,
         py::arg("alpha") = 0.0, py::arg("shift") = 0.0);
   m.def("wide_gemm_tile", &wide_gemm_tile);
+  m.def("mid_gemm", &mid_gemm);
+  m.def("mid_gemm_shares", &mid_gemm_shares);
   m.def("norm_gemm", &norm_gemm);
   m.def("decode_gemm_parts", &decode_gemm_parts);
   m.def("decode_gemm_shares", &decode_gemm_shares);

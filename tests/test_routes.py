@@ -167,6 +167,13 @@ def test_many_rows_go_by_tiles_and_sums():
     assert tile(1000, 3072, 768, 2) == 4   # and enough with an activation
     assert tile(16384, 4096, 4096, 0) == 0  # whole rounds of long sums
     assert tile(16384, 28672, 4096, 4) == 8
+    shares = ops._hip_ops.mid_gemm_shares
+    for sizes in [(64, 768, 768), (300, 760, 768), (300, 768, 760),
+                  (300, 768, 64), (300, 0, 768), (1300, 2304, 768),
+                  (300, 4096, 4096), (300, 4096, 14336)]:
+        assert shares(*sizes) == 0
+    assert shares(300, 2304, 768) == shares(2000, 768, 768) == 1
+    assert shares(200, 768, 3072) == 4
     x = torch.zeros(2)
     p = torch.nn.Parameter(x)
     assert ops._recorded(p) and not ops._recorded(x, None)

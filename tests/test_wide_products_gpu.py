@@ -144,6 +144,53 @@ def test_units_take_it():
                _reference(x, w, None, 5))
 
 
+@pytest.mark.parametrize("M,N,K,shares", [
+    (65, 64, 128, 1),      # a row behind a block's edge, two chunks
+    (128, 192, 448, 1),    # fewer chunks and as many as a ring's
+    (300, 768, 768, 1),
+    (1000, 1280, 1280, 1),
+    (129, 128, 512, 2),    # shares of K, joined by a second launch
+    (200, 768, 3072, 4),
+])
+@pytest.mark.parametrize("act", [ops.ACT_NONE, ops.ACT_GELU_TANH,
+                                 ops.ACT_GELU_ERF, ops.ACT_SILU])
+@pytest.mark.parametrize("bias", [False, True])
+def test_blocks_of_64_rows(M, N, K, shares, act, bias):
+    x, w, b = _operands(M, N, K)
+    b = b if bias else None
+    _check(ops._hip_ops.mid_gemm(x, w, b, shares, ops._DECODE_ACT[act]),
+           _reference(x, w, b, act))
+
+
+def test_linear_of_some_hundred_rows(monkeypatch):
+    """By blocks of 64 where they fit, with the general path's results."""
+    calls = []
+    own = ops._hip_ops.mid_gemm
+    monkeypatch.setattr(ops._hip_ops, "mid_gemm",
+                        lambda *a: calls.append(a) or own(*a), raising=False)
+    with torch.no_grad():
+        for M, N, K, act, mid in [(65, 768, 768, 0, True),
+                                  (300, 2304, 768, 2, True),
+                                  (200, 768, 3072, 0, True),
+                                  (64, 768, 768, 0, False),
+                                  (1000, 3840, 1280, 0, False),
+                                  (300, 4096, 4096, 0, False),
+                                  (300, 2304, 800, 0, False)]:
+            x, w, b = _operands(M, N, K)
+            calls.clear()
+            _check(ops.linear(x, w, b, act), _reference(x, w, b, act))
+            assert bool(calls) == mid
+        x, w, b = _operands(4 * 50, 768, 768)
+        strided = torch.cat([x, x], 1)[:, :768].view(4, 50, 768)
+        calls.clear()
+        _check(ops.linear(strided, w, b).view(200, 768),
+               _reference(x, w, b, 0))
+        assert bool(calls) == strided.reshape(200, 768).is_contiguous()
+    w.requires_grad_()
+    calls.clear()
+    assert ops.linear(x, w, b).requires_grad or not calls
+
+
 def test_in_a_graph():
     x, w, b = _operands(3000, 2304, 768)
     with torch.no_grad():
