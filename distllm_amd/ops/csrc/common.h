@@ -128,6 +128,19 @@ __device__ __forceinline__ int xcd_run(int b, int n) {
          b / 8;
 }
 
+// The chunk of n, of 128 bytes of a row, with which workgroup b of a product of
+// few rows begins; it goes round from there. Workgroups that all begin at the
+// start of rows whose strides are large powers of two ask the same few memory
+// channels: us, that and this, 32 rows of 32768 x 4096 59.8 and 51.4, 64 of 16384 x
+// 8192 gated 65.0 and 54.0, of 28672 x 4096 gated 55.7 and 51.1, one row 45.3 and
+// 42.5, of 4096 x 14336 25.6 and 23.0. STEP is the best of a dozen odd numbers in a
+// form, most of them within 3%. Rows of less than 32 chunks gain nothing (151936 x
+// 1536 115.0, 114.3) and are spared the division (24 rows of 768 x 768 3.24, 3.33).
+template <int STEP>
+__device__ __forceinline__ int chunk_turn(int b, int n) {
+  return n < 32 ? 0 : (int)((unsigned)(b * STEP) % (unsigned)n);
+}
+
 // Block-level reduce across NW waves using LDS scratch (NW <= 16).
 template <int NW>
 __device__ __forceinline__ float block_reduce_sum(float v, float* lds_scratch) {

@@ -166,21 +166,24 @@ dg_ring_kernel(const u16* __restrict__ X, const u16* __restrict__ W, int K,
   for (int p = 0; p < 2; ++p) {
 #pragma unroll
     for (int t = 0; t < NT; ++t)
-      src[t][p] = W + (long)(dg_wrow<GLU>(n0, t, e.N) + p * 8 + lr) * K +
-                  wid * 64 + lc;
+      src[t][p] = W + (long)(dg_wrow<GLU>(n0, t, e.N) + p * 8 + lr) * K + lc;
 #pragma unroll
     for (int t = 0; t < MT; ++t)
       src[NT + t][p] =
-          X + (long)min(t * 16 + p * 8 + lr, e.M - 1) * K + wid * 64 + lc;
+          X + (long)min(t * 16 + p * 8 + lr, e.M - 1) * K + lc;
   }
-  const int mine = (K / 64 - wid + NW - 1) / NW;  // chunks wid, wid + NW, ...
+  // chunks wid, wid + NW, ... from the block's first one on
+  const int nch = K / 64, mine = (nch - wid + NW - 1) / NW;
+  const int turn = chunk_turn<37>(blockIdx.x, nch) + wid;
   auto issue = [&](int c) {
     char* dst = ring + (c % R) * STAGE + lane * 16;
+    int k = c * NW + turn;
+    if (k >= nch) k -= nch;
 #pragma unroll
     for (int t = 0; t < NT + MT; ++t)
 #pragma unroll
       for (int p = 0; p < 2; ++p)
-        dg_copy(src[t][p] + (long)c * (NW * 64), dst + t * 2048 + p * 1024);
+        dg_copy(src[t][p] + (long)k * 64, dst + t * 2048 + p * 1024);
   };
   f32x4 acc[NT][MT];
 #pragma unroll
@@ -262,16 +265,22 @@ dg_norm_ring_kernel(const NormRow n, const u16* __restrict__ W, int K,
   for (int p = 0; p < 2; ++p)
 #pragma unroll
     for (int t = 0; t < NT; ++t)
-      src[t][p] = W + (long)(dg_wrow<GLU>(n0, t, e.N) + p * 8 + lr) * K +
-                  wid * 64 + lc;
-  const int mine = (K / 64 - wid + NW - 1) / NW;  // chunks wid, wid + NW, ...
+      src[t][p] = W + (long)(dg_wrow<GLU>(n0, t, e.N) + p * 8 + lr) * K + lc;
+  // chunks wid, wid + NW, ... from the block's first one on
+  const int nch = K / 64, mine = (nch - wid + NW - 1) / NW;
+  const int turn = chunk_turn<37>(blockIdx.x, nch) + wid;
+  auto chunk = [&](int c) {
+    const int k = c * NW + turn;
+    return k >= nch ? k - nch : k;
+  };
   auto issue = [&](int c) {
     char* dst = ring + (c % R) * STAGE + lane * 16;
+    const long k = chunk(c) * 64;
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
       for (int p = 0; p < 2; ++p)
-        dg_copy(src[t][p] + (long)c * (NW * 64), dst + t * 2048 + p * 1024);
+        dg_copy(src[t][p] + k, dst + t * 2048 + p * 1024);
   };
   norm_row<NC>(n, K, reinterpret_cast<float*>(smem), hs, [&]() {
 #pragma unroll
@@ -283,10 +292,11 @@ dg_norm_ring_kernel(const NormRow n, const u16* __restrict__ W, int K,
   for (int i = 0; i < NT; ++i) acc[i] = {0.f, 0.f, 0.f, 0.f};
   auto compute = [&](int c) {
     const char* b = ring + (c % R) * STAGE;
+    const char* xs = hs + chunk(c) * 128;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      const bf16x8 x = *reinterpret_cast<const bf16x8*>(
-          hs + (c * NW + wid) * 128 + (h * 4 + g) * 16);
+      const bf16x8 x =
+          *reinterpret_cast<const bf16x8*>(xs + (h * 4 + g) * 16);
 #pragma unroll
       for (int i = 0; i < NT; ++i)
         acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
@@ -368,11 +378,13 @@ dg_tile_kernel(const u16* __restrict__ X, const u16* __restrict__ W,
                   : X + (long)min(m0 + row - 64, e.M - 1) * K) +
              ks * (K / splitk) + lc;
   }
+  const int turn = chunk_turn<19>(cb, nt);
   auto issue = [&](int c) {
     char* dst = smem + (c % R) * STAGE + wid * LOADS * 1024 + lane * 16;
+    const int k = c + turn < nt ? c + turn : c + turn - nt;
 #pragma unroll
     for (int p = 0; p < LOADS; ++p)
-      dg_copy(src[p] + (long)c * 64, dst + p * 1024);
+      dg_copy(src[p] + (long)k * 64, dst + p * 1024);
   };
   const int wn = wid % WN, wm = wid / WN;
   f32x4 acc[FN][FM];
@@ -409,7 +421,6 @@ dg_tile_kernel(const u16* __restrict__ X, const u16* __restrict__ W,
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
   };
-  static_assert(R == 3 || R == 4, "tail");
   if (nt >= R - 1) {
     for (int c = 0; c < R - 1; ++c) issue(c);
     int c = 0;
@@ -419,17 +430,12 @@ dg_tile_kernel(const u16* __restrict__ X, const u16* __restrict__ W,
       issue(c + R - 1);
       compute(c);
     }
-    if constexpr (R == 4) {
-      dg_wait<2 * LOADS>();
+#pragma unroll
+    for (int left = R - 2; left >= 0; --left) {
+      asm volatile("s_waitcnt vmcnt(%0)" ::"i"(left * LOADS) : "memory");
       arrive();
       compute(c++);
     }
-    dg_wait<LOADS>();
-    arrive();
-    compute(c++);
-    dg_wait<0>();
-    arrive();
-    compute(c);
   } else {
     for (int c = 0; c < nt; ++c) issue(c);
     dg_wait<0>();

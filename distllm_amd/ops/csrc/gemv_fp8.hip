@@ -120,7 +120,13 @@ gemv_fp8_ring_kernel(const unsigned short* __restrict__ X,
   const int r = lane & 15, g = lane >> 4;
   const int cols = GLU ? N / 2 : N, n0 = blockIdx.x * 16;
   char* ring = smem + wid * GV_R * STAGE;
-  const int mine = (K / 128 - wid + 3) / 4;  // chunks wid, wid + 4, ...
+  // chunks wid, wid + 4, ... from the workgroup's first one on
+  const int nch = K / 128, mine = (nch - wid + 3) / 4;
+  const int turn = chunk_turn<37>(blockIdx.x, nch) + wid;
+  auto chunk = [&](int c) {
+    const int k = c * 4 + turn;
+    return k >= nch ? k - nch : k;
+  };
   const char* src[LOADS];
 #pragma unroll
   for (int p = 0; p < 2; ++p) {
@@ -129,22 +135,23 @@ gemv_fp8_ring_kernel(const unsigned short* __restrict__ X,
     for (int t = 0; t < NT; ++t)
       src[t * 2 + p] =
           (const char*)W +
-          (long)(min(n0 + row, cols - 1) + t * cols) * K + wid * 128 +
+          (long)(min(n0 + row, cols - 1) + t * cols) * K +
           ((lane & 7) ^ (row & 7)) * 16;
   }
 #pragma unroll
   for (int p = 0; p < XL; ++p) {
     const int row = p * 4 + (lane >> 4);
-    src[NT * 2 + p] = (const char*)(X + (long)min(row, M - 1) * K + wid * 128) +
+    src[NT * 2 + p] = (const char*)(X + (long)min(row, M - 1) * K) +
                       ((lane & 15) ^ row) * 16;
   }
   auto issue = [&](int c) {
     char* dst = ring + (c % GV_R) * STAGE + lane * 16;
+    const long k = chunk(c) * 128;
 #pragma unroll
     for (int i = 0; i < LOADS; ++i)
       __builtin_amdgcn_global_load_lds(
           (const __attribute__((address_space(1))) unsigned int*)(
-              src[i] + (long)c * 512 * (i < NT * 2 ? 1 : 2)),
+              src[i] + k * (i < NT * 2 ? 1 : 2)),
           (__attribute__((address_space(3))) unsigned int*)(dst + i * 1024),
           16, 0, 0);
   };
@@ -231,7 +238,13 @@ gemv_fp8_norm_kernel(const NormRow nr, const unsigned char* __restrict__ W,
   const int cols = GLU ? N / 2 : N, n0 = blockIdx.x * 16;
   char* hs = smem + 128;
   char* ring = hs + K * 2 + wid * R * STAGE;
-  const int mine = (K / 128 - wid + 3) / 4;  // chunks wid, wid + 4, ...
+  // chunks wid, wid + 4, ... from the workgroup's first one on
+  const int nch = K / 128, mine = (nch - wid + 3) / 4;
+  const int turn = chunk_turn<37>(blockIdx.x, nch) + wid;
+  auto chunk = [&](int c) {
+    const int k = c * 4 + turn;
+    return k >= nch ? k - nch : k;
+  };
   const unsigned char* src[NT][2];
 #pragma unroll
   for (int p = 0; p < 2; ++p) {
@@ -239,17 +252,18 @@ gemv_fp8_norm_kernel(const NormRow nr, const unsigned char* __restrict__ W,
 #pragma unroll
     for (int t = 0; t < NT; ++t)
       src[t][p] = W + (long)(min(n0 + row, cols - 1) + t * cols) * K +
-                  wid * 128 + ((lane & 7) ^ (row & 7)) * 16;
+                  ((lane & 7) ^ (row & 7)) * 16;
   }
   auto issue = [&](int c) {
     char* dst = ring + (c % R) * STAGE + lane * 16;
+    const long k = chunk(c) * 128;
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
       for (int p = 0; p < 2; ++p)
         __builtin_amdgcn_global_load_lds(
             (const __attribute__((address_space(1))) unsigned int*)(
-                src[t][p] + (long)c * 512),
+                src[t][p] + k),
             (__attribute__((address_space(3))) unsigned int*)(
                 dst + (t * 2 + p) * 1024),
             16, 0, 0);
@@ -263,7 +277,7 @@ gemv_fp8_norm_kernel(const NormRow nr, const unsigned char* __restrict__ W,
   for (int t = 0; t < NT; ++t) acc[t] = {0.f, 0.f, 0.f, 0.f};
   auto compute = [&](int c) {
     const char* b = ring + (c % R) * STAGE;
-    const char* xb = hs + (c * 4 + wid) * 256;
+    const char* xb = hs + chunk(c) * 256;
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       bf16x8 x[2];
