@@ -295,8 +295,8 @@ class DecoderModel(nn.Module):
         # products whose shares of K the next kernel sums (on one rank)
         parts = ops.linear_parts if self.tp == 1 else ops.linear
         eps = d.rms_norm_eps
-        zeros = (ops.step_zeros(len(self.layers), B, nh, kcaches[0],
-                                block_tables) if len(self.layers) else None)
+        plan = (ops.step_plan(len(self.layers), ctx_lens, nh, kcaches[0],
+                              block_tables) if len(self.layers) else [])
         down = None
         for li, layer in enumerate(self.layers):
             # norm and ONE fused qkv GEMM (one launch for one sequence), ONE
@@ -318,7 +318,7 @@ class DecoderModel(nn.Module):
             ctx = ops.step_attn(
                 qkv.view(*qkv.shape[:-1], nh + 2 * kvh, hd), cs, sn,
                 ctx_lens, kcaches[li], vcaches[li], block_tables, layer.bqkv,
-                1.0 / math.sqrt(hd), zeros[li] if zeros is not None else None)
+                1.0 / math.sqrt(hd), plan[li])
             ctx = ctx.reshape(B, nh * hd)
             if f is not None:
                 attn = self._allreduce(ops.gemv_fp8(ctx, *f["wo"]))

@@ -877,29 +877,31 @@ def rope_put(qkv, cs, sn, ctx, kcache, vcache, block_table, bias=None):
     return qkv[:, :H].contiguous()
 
 
-def step_zeros(layers, B, H, kcache, block_table):
-    """What step_attn of so many layers needs cleared, a row for each, None
-    where it needs nothing."""
+def step_plan(layers, ctx, H, kcache, block_table):
+    """What step_attn of so many layers needs, an item for each: the shares of
+    the sequences, cut by their lengths, and its counters. None for heads and
+    devices that need nothing."""
     HKV, D = kcache.shape[1], kcache.shape[3]
-    if (not kcache.is_cuda or D not in (64, 128)
-            or _hip_ops.step_attn_shares(B, H, HKV, block_table.shape[1],
-                                         kcache.dtype == torch.uint8) <= 1):
-        return None
-    return torch.zeros(layers, B * HKV * -(-(H // HKV) // 16),
-                       dtype=torch.int32, device=kcache.device)
+    if not kcache.is_cuda or D not in (64, 128):
+        return [None] * layers
+    _require_hip()
+    slots, zeros = _hip_ops.step_plan(ctx.int(), layers, H, HKV,
+                                      block_table.shape[1],
+                                      kcache.dtype == torch.uint8)
+    return [(slots, row) for row in zeros.unbind()]
 
 
 def step_attn(qkv, cs, sn, ctx, kcache, vcache, block_table, bias, scale,
-              zeros):
+              plan):
     """rope_put and the attention of its queries over the cache, the new token
-    among it -> [B, H, D]; one launch for heads of 64 and 128. zeros: a row of
-    step_zeros, used up."""
+    among it -> [B, H, D]; one launch for heads of 64 and 128. plan: an item of
+    step_plan, used up."""
     if qkv.is_cuda and qkv.shape[-1] in (64, 128):
         _require_hip()
         return _hip_ops.step_attn(qkv.contiguous(), cs, sn, ctx.int(), kcache,
                                   vcache, block_table.int(),
                                   bias if qkv.dim() == 4 else None, scale,
-                                  zeros)
+                                  *plan)
     q = rope_put(qkv, cs, sn, ctx, kcache, vcache, block_table, bias)
     return paged_attn(q, kcache, vcache, block_table, ctx, scale)
 

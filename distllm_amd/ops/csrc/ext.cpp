@@ -57,8 +57,11 @@ void launch_paged_attn(const void*, long, void*, void*, const int*,
                        int, int, float, bool, bool, hipStream_t);
 void launch_step_attn(const void*, const float*, int, const void*,
                       const float*, const float*, void*, void*, const int*,
-                      const int*, void*, void*, void*, int*, int, int, int,
-                      int, int, int, float, bool, bool, hipStream_t);
+                      const int*, void*, void*, void*, int*, const int*, int,
+                      int, int, int, int, int, float, bool, bool, hipStream_t);
+void launch_step_plan(const int*, int, int, int, int, int, int, int*, int*,
+                      long, hipStream_t);
+int step_plan_room(int, int, int, int);
 void launch_norm_parts(const float*, int, const void*, const void*, void*,
                        void*, int, int, float, hipStream_t);
 void launch_rope_put(const void*, const float*, int, const void*,
@@ -476,21 +479,49 @@ int64_t paged_attn_shares(int64_t B, int64_t H, int64_t HKV,
       1);
 }
 
-// The same for step_attn, whose shares join in the launch, so that one that
-// finds no keys costs next to nothing: every CU one, each with 128 of the table's
-// positions (a tile for each of its waves); fp8 pages two, with 256. In us, shares
-// of 4, 8, 16, 32 (two launches as above): 1 x 8 grouped heads, contexts of 64
-// 6.2, 6.3, 6.3, 7.4 (10.9); 2048 11.2, 8.3, 7.6, 8.8 (12.7); 8000 30, 18, 12.2,
-// 10.6 (21); 8 x 8 of 2000 15.6, 20, 21 (22); 8 x 8 fp8 of 500 7.5, 9.5, 17 (11),
-// of 2000 12.4, 12.1, 18.5 (18).
-int64_t step_attn_shares(int64_t B, int64_t H, int64_t HKV,
-                         int64_t max_blocks, bool fp8) {
+// What step_plan has to know of a decode step's attention, whose shares join in
+// the launch, so that one that finds no keys costs next to nothing: the shares of
+// a head group that give every CU one, of fp8 pages two (else 0), and a number
+// that is asked for by DISTLLM_PA_NSPLIT (else 0). In us, shares of 4, 8, 16, 32
+// (two launches, as above): 1 x 8 grouped heads, contexts of 64 6.2, 6.3, 6.3, 7.4
+// (10.9); 2048 11.2, 8.3, 7.6, 8.8 (12.7); 8000 30, 18, 12.2, 10.6 (21); 8 x 8 of
+// 2000 15.6, 20, 21 (22); 8 x 8 fp8 of 500 7.5, 9.5, 17 (11), of 2000 12.4, 12.1,
+// 18.5 (18).
+struct StepShares {
+  int narrow, wide, asked, room;
+};
+static StepShares step_shares(int64_t B, int64_t H, int64_t HKV,
+                              int64_t max_blocks, bool fp8) {
   const char* e = getenv("DISTLLM_PA_NSPLIT");
-  if (e && atol(e) > 0) return paged_attn_shares(B, H, HKV, max_blocks, fp8);
-  const long groups = std::max<long>(B * HKV * ((H / HKV + 15) / 16), 1);
-  long n = std::min<long>(256 / groups, max_blocks / 8);
-  if (fp8) n = std::max(n, std::min<long>(512 / groups, max_blocks / 16));
-  return std::max<long>(std::min<long>(n, 32), 1);
+  const long groups = std::max<long>(HKV * ((H / HKV + 15) / 16), 1);
+  StepShares s;
+  s.narrow = (int)std::max<long>(256 / groups, 1);
+  s.wide = fp8 ? (int)std::max<long>(512 / groups, 1) : 0;
+  s.asked = e && atol(e) > 0
+                ? (int)std::min<long>({atol(e), std::max<long>(max_blocks, 1), 64})
+                : 0;
+  s.room = step_plan_room((int)B, s.narrow, s.wide, s.asked);
+  return s;
+}
+
+// What the attention launches of a decode step of `layers` layers need:
+// [room, 8] shares, and zeros [layers, B * HKV * groups of 16 query heads], a row
+// of which each launch uses up.
+std::vector<torch::Tensor> step_plan(torch::Tensor ctx, int64_t layers,
+                                     int64_t H, int64_t HKV,
+                                     int64_t max_blocks, bool fp8) {
+  CHECK_INTS(ctx);
+  TORCH_CHECK(HKV > 0 && H % HKV == 0, "GQA requires H % HKV == 0");
+  const int64_t B = ctx.numel();
+  const StepShares s = step_shares(B, H, HKV, max_blocks, fp8);
+  auto slots = torch::empty({s.room, 8}, ctx.options());
+  auto arrived = torch::empty({layers, B * HKV * ((H / HKV + 15) / 16)},
+                              ctx.options());
+  if (B > 0)
+    launch_step_plan(ctx.data_ptr<int>(), (int)B, (int)max_blocks, s.room,
+                     s.narrow, s.wide, s.asked, slots.data_ptr<int>(),
+                     arrived.data_ptr<int>(), arrived.numel(), cur_stream());
+  return {slots, arrived};
 }
 
 torch::Tensor paged_attn(torch::Tensor q, torch::Tensor kcache,
@@ -580,14 +611,13 @@ torch::Tensor rope_put(torch::Tensor qkv, torch::Tensor cs, torch::Tensor sn,
   return q;
 }
 
-// rope_put and the attention of its queries [B, H, D] in one launch. arrived:
-// zeros (int32, B * HKV * ceil(H / HKV / 16) of them, used up by the call) where
-// step_attn_shares of the sizes is above 1.
+// rope_put and the attention of its queries [B, H, D] in one launch. slots and
+// arrived: of step_plan for the same lengths, heads and block table.
 torch::Tensor step_attn(torch::Tensor qkv, torch::Tensor cs, torch::Tensor sn,
                         torch::Tensor ctx, torch::Tensor kcache,
                         torch::Tensor vcache, torch::Tensor block_table,
                         c10::optional<torch::Tensor> bias, double scale,
-                        c10::optional<torch::Tensor> arrived) {
+                        torch::Tensor slots, torch::Tensor arrived) {
   const StepSizes z =
       check_step(qkv, cs, sn, ctx, kcache, vcache, block_table, bias);
   TORCH_CHECK(z.H % z.HKV == 0, "GQA requires H % HKV == 0");
@@ -596,18 +626,17 @@ torch::Tensor step_attn(torch::Tensor qkv, torch::Tensor cs, torch::Tensor sn,
   auto out =
       torch::empty({z.B, z.H, z.D}, qkv.options().dtype(at::kBFloat16));
   if (z.B == 0) return out;
-  const int NS = (int)step_attn_shares(z.B, z.H, z.HKV, max_blocks, fp8);
-  torch::Tensor pacc, pml;
-  if (NS > 1) {
-    TORCH_CHECK(arrived.has_value(), "arrived");
-    CHECK_INTS(arrived.value());
-    TORCH_CHECK(arrived->numel() >=
-                    (long)z.B * z.HKV * ((z.H / z.HKV + 15) / 16),
-                "arrived: one for every group of heads");
-    auto f32 = qkv.options().dtype(at::kFloat);
-    pacc = torch::empty({(long)z.B * z.H * NS, z.D}, f32);
-    pml = torch::empty({(long)z.B * z.H * NS, 2}, f32);
-  }
+  CHECK_INTS(slots);
+  CHECK_INTS(arrived);
+  const int room = slots.size(0);
+  TORCH_CHECK(slots.dim() == 2 && slots.size(1) == 8 && room >= z.B &&
+                  (uintptr_t)slots.data_ptr() % 16 == 0,
+              "slots: those of step_plan");
+  TORCH_CHECK(arrived.numel() >= (long)z.B * z.HKV * ((z.H / z.HKV + 15) / 16),
+              "arrived: one for every group of heads");
+  auto f32 = qkv.options().dtype(at::kFloat);
+  auto pacc = torch::empty({(long)room * z.H, z.D}, f32);
+  auto pml = torch::empty({(long)room * z.H, 2}, f32);
   qkv = aligned16(qkv);
   cs = aligned16(cs);
   sn = aligned16(sn);
@@ -619,10 +648,9 @@ torch::Tensor step_attn(torch::Tensor qkv, torch::Tensor cs, torch::Tensor sn,
                    bias ? bias->data_ptr() : nullptr, cs.data_ptr<float>(),
                    sn.data_ptr<float>(), kcache.data_ptr(), vcache.data_ptr(),
                    block_table.data_ptr<int>(), ctx.data_ptr<int>(),
-                   out.data_ptr(), NS > 1 ? pacc.data_ptr() : nullptr,
-                   NS > 1 ? pml.data_ptr() : nullptr,
-                   NS > 1 ? arrived->data_ptr<int>() : nullptr, z.B, z.H,
-                   z.HKV, z.D, max_blocks, NS, (float)scale, fp8, aligned,
+                   out.data_ptr(), pacc.data_ptr(), pml.data_ptr(),
+                   arrived.data_ptr<int>(), slots.data_ptr<int>(), room, z.B,
+                   z.H, z.HKV, z.D, max_blocks, (float)scale, fp8, aligned,
                    cur_stream());
   return out;
 }
@@ -768,7 +796,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("cache_put", &cache_put);
   m.def("norm_parts", &norm_parts);
   m.def("step_attn", &step_attn);
-  m.def("step_attn_shares", &step_attn_shares);
+  m.def("step_plan", &step_plan);
   m.def("rope_put", &rope_put, py::arg("qkv"), py::arg("cs"), py::arg("sn"),
         py::arg("ctx"), py::arg("kcache"), py::arg("vcache"),
         py::arg("block_table"), py::arg("bias") = py::none());

@@ -29,7 +29,8 @@
 //  - a decode step's queries are rotated and its key and value put into the
 //    cache in the same launch (STEP): us in a graph, three launches and one,
 //    32 heads on 8, B = 1, 2048 tokens 12.7 -> 7.6, 64 tokens 10.9 -> 6.3, B = 8
-//    of 500 11.0 -> 7.4, B = 64 of 200 to 2027 70 -> 56.
+//    of 500 11.0 -> 7.4, B = 64 of 200 to 2027 70 -> 56, and 51 with the sequences
+//    cut and ordered by their lengths (step_plan_kernel).
 // Measured, us, with kernels that read a key row per lane and a value element
 // per lane, and now (32 heads on 8 of 128, bf16; fp8): B = 1, 2048 cached
 // tokens 32 -> 11.0 (31 -> 11.1); B = 16 of 100 to 4000 115 -> 36.5 (104 ->
@@ -91,6 +92,10 @@ struct PaStep {
   int S;
   const unsigned short* bias;
   const float *cs, *sn;
+  // the launch's shares (step_plan_kernel), eight numbers each: sequence or -1,
+  // its length, first tile, the one behind the last; of the sequence, the first
+  // share and their number
+  const int* slots;
 };
 
 // Columns c .. c + 3 and D / 2 + c .. of head h of row b, as bf16 numbers; ROT:
@@ -192,7 +197,7 @@ paged_attn_kernel(const unsigned short* __restrict__ q, long q_stride,
                   const int* __restrict__ block_table,
                   const int* __restrict__ ctx_len,
                   unsigned short* __restrict__ out,
-                  float* pacc, float* pml, int* arrived, int H, int HKV,
+                  float* pacc, float* pml, int* arrived, int B, int H, int HKV,
                   int max_blocks, int NS, float scale) {
   constexpr int NCH = D / 8;            // 16-byte pieces of a bf16 row
   constexpr int ROWS = 1024 / (2 * D);  // rows of a 1 KiB piece of a tile
@@ -203,15 +208,27 @@ paged_attn_kernel(const unsigned short* __restrict__ q, long q_stride,
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int c16 = lane & 15, g = lane >> 4;
   const int GR = H / HKV, NG = (GR + 15) / 16;
-  const int split = blockIdx.x % NS;
-  const int hg = blockIdx.x / NS % NG;
-  const int kvh = blockIdx.x / NS / NG % HKV;
-  const int b = blockIdx.x / NS / NG / HKV;
+  const int slot = STEP ? blockIdx.x / (NG * HKV) : 0;
+  const int split = STEP ? 0 : blockIdx.x % NS;
+  const int hg = STEP ? blockIdx.x % NG : blockIdx.x / NS % NG;
+  const int kvh = STEP ? blockIdx.x / NG % HKV : blockIdx.x / NS / NG % HKV;
+  int share[6] = {};
+  if constexpr (STEP) {
+#pragma unroll
+    for (int i = 0; i < 6; ++i)
+      share[i] = __builtin_amdgcn_readfirstlane(step.slots[slot * 8 + i]);
+    if ((unsigned)share[0] >= (unsigned)B) return;
+    NS = share[5];
+  }
+  const int b = STEP ? share[0] : blockIdx.x / NS / NG / HKV;
   const int head0 = kvh * GR + hg * 16, nh = min(GR - hg * 16, 16);
 
-  const int L = min(ctx_len[b], max_blocks * PBLK);
+  const int ctx = STEP ? share[1] : ctx_len[b];
+  const int L = min(ctx, max_blocks * PBLK);
   const int T = (L + KT - 1) / KT, per = (T + NS - 1) / NS;
-  const int t0 = split * per + wid, t1 = min(T, split * per + per);
+  const int first_tile = STEP ? share[2] : split * per;
+  const int t0 = first_tile + wid;
+  const int t1 = STEP ? share[3] : min(T, split * per + per);
   const int mine = t1 > t0 ? (t1 - t0 + NW - 1) / NW : 0;  // t0, t0 + NW, ...
   const int last_page = max(L - 1, 0) / PBLK;
   const int* bt = block_table + (long)b * max_blocks;
@@ -286,22 +303,22 @@ paged_attn_kernel(const unsigned short* __restrict__ q, long q_stride,
   };
   while (at < (R > 1 ? R - 1 : 1) && at < mine) next();
 
-  const int pos = STEP ? ctx_len[b] - 1 : 0;
+  const int pos = ctx - 1;
   // of the workgroup, of the wave: its share ends with the new token
   const bool newest = STEP && pos >= 0 && pos < max_blocks * PBLK && T > 0 &&
-                      T - 1 >= split * per && T - 1 < split * per + per;
+                      T - 1 >= first_tile && T - 1 < t1;
   const bool renews = newest && mine > 0 && t0 + (mine - 1) * NW == T - 1;
   // rotated queries, the new key and value: rows of D in LDS
   char* rows = smem + pa_lds(D, R);
   if constexpr (STEP) {
-    const int nb = gridDim.x / NS / NG / HKV, heads = H + 2 * HKV;
+    const int heads = H + 2 * HKV;
     const int units = (nh + (newest ? 2 : 0)) * (D / 8);
     for (int u = threadIdx.x; u < units && pos >= 0; u += NW * 64) {
       const int row = u / (D / 8), c = u % (D / 8) * 4;
       const int h = row < nh ? head0 + row
                              : H + (row - nh) * HKV + kvh;
       unsigned short a[4], e[4];
-      step_columns<D>(step, nb, heads, b, h, c, row <= nh, pos, a, e);
+      step_columns<D>(step, B, heads, b, h, c, row <= nh, pos, a, e);
       if (row >= nh) {
         char* to = (row == nh ? kcache : vcache) +
                    bt[pos / PBLK] * page_bytes + head_bytes +
@@ -495,7 +512,9 @@ paged_attn_kernel(const unsigned short* __restrict__ q, long q_stride,
     *reinterpret_cast<f32x4*>(wacc + (wid * 16 + c16) * D + d * 16 + g * 4) =
         acc[d];
   __syncthreads();
-  const long part = ((long)(b * HKV + kvh) * NS + split) * GR + hg * 16;
+  // row of the share's first head among the partial results
+  const long part = STEP ? (long)slot * H + head0
+                         : ((long)(b * HKV + kvh) * NS + split) * GR + hg * 16;
   for (int i = threadIdx.x; i < nh * (D / 4); i += NW * 64) {
     const int head = i / (D / 4), col = i % (D / 4) * 4;
     float M = -1e30f;
@@ -540,11 +559,11 @@ paged_attn_kernel(const unsigned short* __restrict__ q, long q_stride,
                                      __HIP_MEMORY_SCOPE_AGENT) == NS - 1;
     __syncthreads();
     if (!*last) return;
-    const long first = (long)(b * HKV + kvh) * NS * GR + hg * 16;
+    const long first = (long)share[4] * H + head0;
     float* state = reinterpret_cast<float*>(smem) + 4;  // [NS][nh][2]
     for (int i = threadIdx.x; i < NS * nh; i += NW * 64)
       *reinterpret_cast<f32x2*>(state + i * 2) =
-          pa_get(pml + (first + (long)(i / nh) * GR + i % nh) * 2);
+          pa_get(pml + (first + (long)(i / nh) * H + i % nh) * 2);
     __syncthreads();
     for (int i = threadIdx.x; i < nh * (D / 2); i += NW * 64) {
       const int head = i / (D / 2), col = i % (D / 2) * 2;
@@ -556,7 +575,7 @@ paged_attn_kernel(const unsigned short* __restrict__ q, long q_stride,
 #pragma unroll 8
       for (int s = 0; s < NS; ++s) {
         const float a = __builtin_amdgcn_exp2f(st[s * nh * 2] - M);
-        const f32x2 v = pa_get(from + (long)s * GR * D);
+        const f32x2 v = pa_get(from + (long)s * H * D);
         sum += a * st[s * nh * 2 + 1];
         o[0] += a * v[0];
         o[1] += a * v[1];
@@ -607,8 +626,8 @@ paged_attn_combine_kernel(const float* __restrict__ pacc,
     out[(long)row * D + lane * DPL + i] = f2bf(o[i] * inv);
 }
 
-// step: a decode step's projections in the place of q, arrived: a zero for every
-// B * HKV * groups of 16 query heads, where NS > 1
+// step: a decode step's projections in the place of q, NS the shares of all
+// sequences; arrived: a zero for every B * HKV * groups of 16 query heads
 static void pa_launch(const void* q, long q_stride, const PaStep* step,
                       void* kcache, void* vcache, const int* block_table,
                       const int* ctx_len, void* out, void* pacc, void* pml,
@@ -616,7 +635,7 @@ static void pa_launch(const void* q, long q_stride, const PaStep* step,
                       int max_blocks, int NS, float scale, bool fp8,
                       bool aligned, hipStream_t stream) {
   const int GR = H / HKV, NG = (GR + 15) / 16;
-  const int grid = B * HKV * NG * NS;
+  const int grid = (step != nullptr ? 1 : B) * HKV * NG * NS;
   const PaStep in = step != nullptr ? *step : PaStep{};
 #define PA(DD, F8, AL, R, ST)                                                 \
   hipLaunchKernelGGL((paged_attn_kernel<DD, F8, AL, R, ST>), dim3(grid),      \
@@ -624,7 +643,7 @@ static void pa_launch(const void* q, long q_stride, const PaStep* step,
                      (const unsigned short*)q, q_stride, in, (char*)kcache,   \
                      (char*)vcache, block_table, ctx_len,                     \
                      (unsigned short*)out, (float*)pacc, (float*)pml,         \
-                     arrived, H, HKV, max_blocks, NS, scale)
+                     arrived, B, H, HKV, max_blocks, NS, scale)
 // Tiles in a wave's ring. Two tiles of 128 columns leave a CU to one workgroup;
 // from 1024 workgroups on, four for every CU, a second one on the CU counts for
 // more, for short contexts are a chain of three reads each. In us, 64 x 32 heads
@@ -636,7 +655,7 @@ static void pa_launch(const void* q, long q_stride, const PaStep* step,
   do {                                                                \
     if (fp8) PA(DD, true, true, 1, ST);                               \
     else if (!aligned) PA(DD, false, false, 1, ST);                   \
-    else if (DD == 128 && grid >= 1024) PA(DD, false, true, 1, ST);   \
+    else if (DD == 128 && B * HKV * NG >= 1024) PA(DD, false, true, 1, ST);   \
     else PA(DD, false, true, 2, ST);                                  \
   } while (0)
   if (step != nullptr) {
@@ -677,14 +696,143 @@ extern "C" void launch_step_attn(const void* qkv, const float* parts, int S,
                                  const float* sn, void* kcache, void* vcache,
                                  const int* block_table, const int* ctx_len,
                                  void* out, void* pacc, void* pml,
-                                 int* arrived, int B, int H, int HKV, int D,
-                                 int max_blocks, int NS, float scale, bool fp8,
-                                 bool aligned, hipStream_t stream) {
+                                 int* arrived, const int* slots, int G, int B,
+                                 int H, int HKV, int D, int max_blocks,
+                                 float scale, bool fp8, bool aligned,
+                                 hipStream_t stream) {
   const PaStep step = {(const unsigned short*)qkv, parts, S,
-                       (const unsigned short*)bias, cs, sn};
+                       (const unsigned short*)bias, cs, sn,
+                       slots};
   pa_launch(nullptr, 0, &step, kcache, vcache, block_table, ctx_len, out, pacc,
-            pml, arrived, B, H, HKV, D, max_blocks, NS, scale, fp8, aligned,
+            pml, arrived, B, H, HKV, D, max_blocks, G, scale, fp8, aligned,
             stream);
+}
+
+// Who takes what in the attention launches of a decode step, which know the
+// lengths only on the device. `wide` and `narrow` are the shares of a head group
+// that fill the CUs with one workgroup and, of fp8 pages, with two (else 0).
+//  - Up to 7/8 of that many sequences are cut into tiles of 32 keys so that all shares
+//    run at once and the largest is as small as can be (256 sizes are tried); of
+//    fp8 pages no further than 8 tiles where one workgroup a CU does with less.
+//  - Of more sequences only those are cut that are above one and a half times
+//    what a CU has to read; a CU alone reads nearly twice as fast as all at once.
+//  - The largest come first: a CU that got a long one late is what all the
+//    others waited for.
+// Measured, us in a graph, 32 heads on 8 of 128, equal shares in the batch's
+// order and these (bf16; fp8), lengths spread evenly and mixed: 8 of 200 to 4096
+// 20.3 -> 17.1 (14.4 -> 13.9); of 200 to 2048, 20 30.6 -> 21.9 (17.9 -> 15.7), 30
+// 32.9 -> 30.7 (23 -> 20.5), 42 46.4 -> 36.2 (38.5 -> 23.6), 64 60.5 -> 51.1 (37.4
+// -> 33.7); lengths all alike take what they took. One launch per step, 5 us, which
+// clears the counters of all layers too, as one did before.
+// Shares have 4 tiles or more, one for each wave, a sequence 32 shares or less.
+// asked > 0: that many for each.
+__host__ __device__ constexpr bool plan_many(int B, int p) {
+  return B > p - p / 8;
+}
+constexpr int PLAN_ROWS = 1024;  // beyond, each sequence is a share, in order
+__global__ void __launch_bounds__(256)
+step_plan_kernel(const int* __restrict__ ctx, int B, int max_blocks, int G,
+                 int narrow, int wide, int asked, int4* __restrict__ slots,
+                 int* __restrict__ arrived, long zeros) {
+  const int tid = threadIdx.x;
+  if (blockIdx.x > 0) {
+    for (long i = (blockIdx.x - 1) * 256L + tid; i < zeros;
+         i += (gridDim.x - 1) * 256L)
+      arrived[i] = 0;
+    return;
+  }
+  auto length = [&](int b) { return min(max(ctx[b], 0), max_blocks * PBLK); };
+  if (B > PLAN_ROWS) {
+    for (int i = tid; i < G; i += 256) {
+      const bool is = i < B;
+      slots[i * 2] = int4{is ? i : -1, is ? ctx[i] : 0, 0,
+                          is ? (length(i) + KT - 1) / KT : 0};
+      slots[i * 2 + 1] = int4{i, 1, 0, 0};
+    }
+    return;
+  }
+  int* tiles = reinterpret_cast<int*>(smem);  // [B]
+  int* some = tiles + B;                      // [B]: shares
+  int* each = some + B;                       // [B]: tiles of a share
+  __shared__ int sum, most, best[2];
+  if (tid == 0) sum = most = 0, best[0] = best[1] = 1 << 30;
+  __syncthreads();
+  int s = 0, m = 0;
+  for (int b = tid; b < B; b += 256) {
+    const int t = (length(b) + KT - 1) / KT;
+    tiles[b] = t;
+    s += t;
+    m = max(m, t);
+  }
+  atomicAdd(&sum, s);
+  atomicMax(&most, m);
+  __syncthreads();
+  // tiles of a share so that there are p shares or less; of many sequences, two
+  // thirds of p more than them. Quotients by a multiplication, exact below 2^16
+  // tiles and never too small: the largest size is always one that does.
+  auto cut = [&](int p, int* found) {
+    if (plan_many(B, p)) return (3 * sum + 2 * p - 1) / (2 * p);
+    const int lo = max((sum + p - 1) / p, NW), hi = max(most, lo);
+    const int c = lo + (int)(((long)(hi - lo) * tid + 254) / 255);
+    const unsigned int inv = 0xffffffffu / (unsigned)c + 1;
+    int n = 0;
+    for (int b = 0; b < B; ++b)
+      n += max((int)__umulhi((unsigned)(tiles[b] + c - 1), inv), 1);
+    if (n <= p) atomicMin(found, c);
+    __syncthreads();
+    return min(*found, hi);
+  };
+  int c = 1;
+  if (asked <= 0) {
+    c = cut(narrow, &best[0]);
+    if (wide > 0) c = max(cut(wide, &best[1]), min(c, 8));
+    c = max(max(c, NW), (most + 31) / 32);
+  }
+  for (int b = tid; b < B; b += 256) {
+    const int t = tiles[b], n = asked > 0 ? asked : max((t + c - 1) / c, 1);
+    const int per = max((t + n - 1) / n, 1);
+    some[b] = asked > 0 ? n : max((t + per - 1) / per, 1);
+    each[b] = per;
+  }
+  __syncthreads();
+  int all = 0;
+  for (int b = tid; b < B; b += 256) {
+    const int t = tiles[b], n = some[b], per = each[b];
+    int first = 0;
+    all = 0;
+    for (int j = 0; j < B; ++j) {
+      const int nj = some[j], pj = each[j];
+      all += nj;
+      if (pj > per || (pj == per && j < b)) first += nj;
+    }
+    for (int i = 0; i < n && first + i < G; ++i) {
+      slots[(first + i) * 2] =
+          int4{b, ctx[b], min(i * per, t), min((i + 1) * per, t)};
+      slots[(first + i) * 2 + 1] = int4{first, n, 0, 0};
+    }
+  }
+  // thread 0 has a sequence
+  if (tid == 0) sum = all;
+  __syncthreads();
+  for (int i = sum + tid; i < G; i += 256) slots[i * 2] = int4{-1, 0, 0, 0};
+}
+
+// Shares that a launch has room for; asked is taken up to PLAN_ROWS sequences.
+extern "C" int step_plan_room(int B, int narrow, int wide, int asked) {
+  if (B > PLAN_ROWS) return B;
+  if (asked > 0) return B * asked;
+  const int p = std::max(narrow, wide);
+  return plan_many(B, p) ? B + 2 * p / 3 : p;
+}
+
+extern "C" void launch_step_plan(const int* ctx, int B, int max_blocks, int G,
+                                 int narrow, int wide, int asked, int* slots,
+                                 int* arrived, long zeros,
+                                 hipStream_t stream) {
+  const int clear = (int)std::min((zeros + 1023) / 1024, 256L);
+  hipLaunchKernelGGL(step_plan_kernel, dim3(1 + clear), dim3(256),
+                     B > PLAN_ROWS ? 0 : B * 12, stream, ctx, B, max_blocks, G,
+                     narrow, wide, asked, (int4*)slots, arrived, zeros);
 }
 
 // Write one new token's K/V into the paged cache (decode step).

@@ -237,14 +237,33 @@ def _same_step(device, qkv, cs, sn, ctx, raw, table, bias):
     scale = D ** -0.5
     q = ops.rope_put(qkv, cs, sn, ctx, *two, table, bias)
     want = ops.paged_attn(q, *two, table, ctx, scale)
-    zeros = ops.step_zeros(1, len(ctx), H, raw[0], table)
-    got = ops.step_attn(qkv, cs, sn, ctx, *raw, table, bias, scale,
-                        None if zeros is None else zeros[0])
+    plan = ops.step_plan(1, ctx, H, raw[0], table)[0]
+    got = ops.step_attn(qkv, cs, sn, ctx, *raw, table, bias, scale, plan)
     assert not got.isnan().any()
     torch.testing.assert_close(got.float(), want.float(), **TOL)
     for a, b in zip(raw, two):
         torch.testing.assert_close(a, b, atol=0, rtol=0, equal_nan=True)
-    return zeros
+    return plan
+
+
+def _shares(slots, lens, width):
+    """Every tile of 32 keys once, a sequence's shares side by side; -> the
+    numbers of shares and, in their order, the sizes of the first ones."""
+    cut = [[] for _ in lens]
+    sizes = []
+    for i, (b, n, t0, t1, first, shares) in enumerate(slots[:, :6].tolist()):
+        if b < 0:
+            continue
+        assert n == lens[b] and first + len(cut[b]) == i < first + shares
+        cut[b].append((t0, t1, shares))
+        if i == first:
+            sizes.append(max(t1 - t0, 1))
+    for n, c in zip(lens, cut):
+        tiles = -(-min(n, width * 16) // 32)
+        ends = [0] + [t1 for _, t1, _ in c]
+        assert [t0 for t0, _, _ in c] == ends[:-1] and ends[-1] == tiles
+        assert all(shares == len(c) for _, _, shares in c)
+    return [len(c) for c in cut], sizes
 
 
 @pytest.mark.parametrize("fp8", [False, True])
@@ -265,9 +284,41 @@ def test_step_shares(device, lens, width, H, HKV, shares, fp8, monkeypatch):
     if shares:
         monkeypatch.setenv("DISTLLM_PA_NSPLIT", shares)
     args = _step(device, lens, H, HKV, 128, fp8, width)
-    zeros = _same_step(device, *args)
-    n = ops._hip_ops.step_attn_shares(len(lens), H, HKV, width, fp8)
-    assert (zeros == n).all() if n > 1 else zeros is None
+    slots, zeros = _same_step(device, *args)
+    n, _ = _shares(slots, lens, width)
+    assert not shares or n == [int(shares)] * len(lens)
+    want = [k if k > 1 else 0 for k in n]
+    assert zeros.view(len(lens), -1).tolist() == [
+        [k] * (zeros.numel() // len(lens)) for k in want]
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("HKV,groups", [(8, 8), (1, 2), (32, 32)])
+@pytest.mark.parametrize("lens", [
+    [1], [8000], [0, 33], [300] * 20, list(range(1, 2048, 66)),
+    [200 + 56 * (7 * i % 33) for i in range(33)], [4096] + [16] * 63,
+    [3 * i for i in range(300)], [40] * 1025])
+def test_step_plan(device, lens, HKV, groups, fp8):
+    """The cut of the lengths that a decode step's attention goes by, at and
+    around as many sequences as fill the CUs and as many as are sorted."""
+    B, width = len(lens), 256
+    H = 20 if HKV == 1 else 32
+    pages = torch.empty(2, HKV, 16, 128, device=device,
+                        dtype=torch.uint8 if fp8 else torch.bfloat16)
+    table = torch.zeros(B, width, dtype=torch.int32, device=device)
+    ctx = torch.tensor(lens, dtype=torch.int32, device=device)
+    plan = ops.step_plan(3, ctx, H, pages, table)
+    assert len(plan) == 3 and all(not row.any() for _, row in plan)
+    assert plan[0][1].numel() == B * groups
+    n, sizes = _shares(plan[0][0], lens, width)
+    full = (512 if fp8 else 256) // groups
+    if B <= 1024:
+        assert sizes == sorted(sizes, reverse=True)
+        assert max(n) <= 32 and sum(n) <= max(full, B + full * 2 // 3)
+        for k, x in zip(n, lens):  # four tiles, but for what halving leaves
+            assert k == 1 or -(-min(x, width * 16) // 32) > 4 * (k - 1)
+    if lens == [8000] and groups == 8:
+        assert n == [32]
 
 
 def test_step_unaligned_pages(device):
@@ -287,9 +338,9 @@ def test_step_in_a_graph(device):
                                             False, 128)
 
     def run():
-        zeros = ops.step_zeros(2, 3, 32, raw[0], table)
+        plan = ops.step_plan(2, ctx, 32, raw[0], table)
         return [ops.step_attn(qkv * f, cs, sn, ctx, *raw, table, None, 0.1,
-                              zeros[i]) for i, f in enumerate((1.0, 0.5))]
+                              plan[i]) for i, f in enumerate((1.0, 0.5))]
 
     want = [t.clone() for t in run()]
     torch.cuda.synchronize()
