@@ -516,6 +516,12 @@ extern "C" int decode_gemm_shares(int M, int N, int K) {
   return best;
 }
 
+// Whether a product of M <= 64 rows takes the ring.
+extern "C" bool decode_gemm_rings(int M, int N, int K) {
+  return M <= 16 ? !dg_short_sums(M, N, K)
+                 : M <= 64 && dg_few_columns(M, N, K);
+}
+
 // How many workgroups share K where 65 rows and more go by tiles of 64 x 64, 0
 // where another product is to be taken. Tiles have to fit the card twice over,
 // and the sums, 0.22 us for 64 of K and 4.5 for the launch that joins shares, have
@@ -555,16 +561,10 @@ static void dg_launch(const u16* X, const u16* W, float* slabs, int K,
                      dim3(e.N / (NT * 16)), dim3(256),                       \
                      dg_ring_lds(MT, NT, 4, R), st, X, W, K, e)
   // two rows of W per stage: three stages let two workgroups share a CU
-  if (!tile && e.M <= 16 && !dg_short_sums(e.M, e.N, K)) {
-    DG_RING(1, GLU ? 3 : 4);
-    return;
-  }
-  if (!tile && e.M <= 32 && dg_few_columns(32, e.N, K)) {
-    DG_RING(2, 4);
-    return;
-  }
-  if (!tile && e.M <= 64 && dg_few_columns(64, e.N, K)) {
-    DG_RING(4, 3);
+  if (!tile && decode_gemm_rings(e.M, e.N, K)) {
+    if (e.M <= 16) DG_RING(1, GLU ? 3 : 4);
+    else if (e.M <= 32) DG_RING(2, 4);
+    else DG_RING(4, 3);
     return;
   }
 #undef DG_RING

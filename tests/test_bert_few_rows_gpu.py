@@ -61,6 +61,23 @@ def test_same_as_layers(device, B, S, H, heads, ff):
     assert torch.equal(out, _layers(m, ids, mask))
 
 
+@pytest.mark.parametrize("B,S,H,heads,ff", [
+    (1, 9, 768, 12, 768), (1, 25, 768, 12, 3072), (1, 32, 1024, 16, 4096),
+    (1, 33, 768, 12, 3072), (2, 12, 1024, 16, 1024), (2, 16, 768, 12, 3072),
+    (2, 24, 512, 8, 2048), (3, 15, 512, 8, 512), (4, 8, 384, 6, 1536),
+    (24, 1, 64, 1, 128), (6, 10, 256, 4, 256), (5, 8, 832, 13, 128)])
+def test_joined_launches(device, B, S, H, heads, ff):
+    """Norms and attention within a product's launch: their edges of rows,
+    width and texts, odd starts of texts, and a text without tokens."""
+    m = _model(device, H, heads, ff, "tanh" if ff == H else "erf")
+    ids = torch.randint(0, 300, (B, S), device=device)
+    at = torch.arange(B, device=device)[:, None]
+    mask = (torch.arange(S, device=device)[None] < (S - at * 3) % (S + 1))
+    if B == 1:
+        mask[:, S // 2] = False
+    assert torch.equal(m(ids, mask.int()), _layers(m, ids, mask.int()))
+
+
 def test_stands_back(device):
     m = _model(device)
     ids = torch.randint(0, 300, (1, 20), device=device)
