@@ -764,8 +764,16 @@ step_plan_kernel(const int* __restrict__ ctx, int B, int max_blocks, int G,
     s += t;
     m = max(m, t);
   }
-  atomicAdd(&sum, s);
-  atomicMax(&most, m);
+  // (256 threads' atomics on one number were half of the launch)
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    s += __shfl_xor(s, off, 64);
+    m = max(m, __shfl_xor(m, off, 64));
+  }
+  if ((tid & 63) == 0) {
+    atomicAdd(&sum, s);
+    atomicMax(&most, m);
+  }
   __syncthreads();
   // tiles of a share so that there are p shares or less; of many sequences, two
   // thirds of p more than them. Quotients by a multiplication, exact below 2^16
@@ -778,7 +786,11 @@ step_plan_kernel(const int* __restrict__ ctx, int B, int max_blocks, int G,
     int n = 0;
     for (int b = 0; b < B; ++b)
       n += max((int)__umulhi((unsigned)(tiles[b] + c - 1), inv), 1);
-    if (n <= p) atomicMin(found, c);
+    const unsigned long long does = __ballot(n <= p);
+    if (does) {
+      const int least = __shfl(c, __ffsll(does) - 1, 64);
+      if ((tid & 63) == 0) atomicMin(found, least);
+    }
     __syncthreads();
     return min(*found, hi);
   };
