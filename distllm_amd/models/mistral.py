@@ -318,7 +318,8 @@ class DecoderModel(nn.Module):
             ctx = ops.step_attn(
                 qkv.view(*qkv.shape[:-1], nh + 2 * kvh, hd), cs, sn,
                 ctx_lens, kcaches[li], vcaches[li], block_tables, layer.bqkv,
-                1.0 / math.sqrt(hd), plan[li])
+                1.0 / math.sqrt(hd), plan[li],
+                f["wo"][0] if f is not None else layer.wo)
             ctx = ctx.reshape(B, nh * hd)
             if f is not None:
                 attn = self._allreduce(ops.gemv_fp8(ctx, *f["wo"]))

@@ -892,16 +892,17 @@ def step_plan(layers, ctx, H, kcache, block_table):
 
 
 def step_attn(qkv, cs, sn, ctx, kcache, vcache, block_table, bias, scale,
-              plan):
+              plan, ahead=None):
     """rope_put and the attention of its queries over the cache, the new token
     among it -> [B, H, D]; one launch for heads of 64 and 128. plan: an item of
-    step_plan, used up."""
+    step_plan, used up. ahead: weights of the product that follows, which few
+    sequences leave the time to fetch into the caches."""
     if qkv.is_cuda and qkv.shape[-1] in (64, 128):
         _require_hip()
         return _hip_ops.step_attn(qkv.contiguous(), cs, sn, ctx.int(), kcache,
                                   vcache, block_table.int(),
                                   bias if qkv.dim() == 4 else None, scale,
-                                  *plan)
+                                  *plan, ahead)
     q = rope_put(qkv, cs, sn, ctx, kcache, vcache, block_table, bias)
     return paged_attn(q, kcache, vcache, block_table, ctx, scale)
 

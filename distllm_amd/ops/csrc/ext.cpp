@@ -4,6 +4,7 @@
 // if this extension is missing — no silent eager fallback.
 // All kernels are hand-written CDNA4 HIP (see *.hip in this directory);
 // this file only validates tensors and forwards device pointers.
+#include "ahead.h"
 #include "ext_common.h"
 
 extern "C" {
@@ -58,7 +59,8 @@ void launch_paged_attn(const void*, long, void*, void*, const int*,
 void launch_step_attn(const void*, const float*, int, const void*,
                       const float*, const float*, void*, void*, const int*,
                       const int*, void*, void*, void*, int*, const int*, int,
-                      int, int, int, int, int, float, bool, bool, hipStream_t);
+                      int, int, int, int, int, float, bool, bool, const Ahead*,
+                      hipStream_t);
 void launch_step_plan(const int*, int, int, int, int, int, int, int*, int*,
                       long, hipStream_t);
 int step_plan_room(int, int, int, int);
@@ -611,13 +613,31 @@ torch::Tensor rope_put(torch::Tensor qkv, torch::Tensor cs, torch::Tensor sn,
   return q;
 }
 
+// Weights [N, K] that a product of few rows reads next, as runs of the 16 rows that
+// its workgroups have; nothing where they cannot be read in pieces of 1 KiB. Of
+// large ones the first 40 MiB, what an attention of 8 us leaves the time for.
+static Ahead ahead_of(const c10::optional<torch::Tensor>& w,
+                      const torch::Tensor& like) {
+  if (!w || w->dim() != 2 || !w->is_contiguous() ||
+      w->device() != like.device() || (uintptr_t)w->data_ptr() % 16)
+    return Ahead{};
+  const long run = 16 * w->size(1) * w->element_size();
+  if (run == 0 || run % 1024) return Ahead{};
+  const long chunks = std::min<long>(w->size(0) / 16, (40l << 20) / run);
+  if (chunks < 8) return Ahead{};
+  return Ahead{(const char*)w->data_ptr(), 192, (int)chunks,
+               (int)(run / 1024)};
+}
+
 // rope_put and the attention of its queries [B, H, D] in one launch. slots and
-// arrived: of step_plan for the same lengths, heads and block table.
+// arrived: of step_plan for the same lengths, heads and block table. ahead: the
+// weights [N, K] of the product that follows, for the caches.
 torch::Tensor step_attn(torch::Tensor qkv, torch::Tensor cs, torch::Tensor sn,
                         torch::Tensor ctx, torch::Tensor kcache,
                         torch::Tensor vcache, torch::Tensor block_table,
                         c10::optional<torch::Tensor> bias, double scale,
-                        torch::Tensor slots, torch::Tensor arrived) {
+                        torch::Tensor slots, torch::Tensor arrived,
+                        c10::optional<torch::Tensor> ahead) {
   const StepSizes z =
       check_step(qkv, cs, sn, ctx, kcache, vcache, block_table, bias);
   TORCH_CHECK(z.H % z.HKV == 0, "GQA requires H % HKV == 0");
@@ -642,6 +662,7 @@ torch::Tensor step_attn(torch::Tensor qkv, torch::Tensor cs, torch::Tensor sn,
   sn = aligned16(sn);
   const bool aligned = (uintptr_t)kcache.data_ptr() % 16 == 0 &&
                        (uintptr_t)vcache.data_ptr() % 16 == 0;
+  const Ahead next = z.B <= 8 ? ahead_of(ahead, qkv) : Ahead{};
   launch_step_attn(z.parts ? nullptr : qkv.data_ptr(),
                    z.parts ? qkv.data_ptr<float>() : nullptr,
                    z.parts ? (int)qkv.size(0) : 0,
@@ -651,7 +672,7 @@ torch::Tensor step_attn(torch::Tensor qkv, torch::Tensor cs, torch::Tensor sn,
                    out.data_ptr(), pacc.data_ptr(), pml.data_ptr(),
                    arrived.data_ptr<int>(), slots.data_ptr<int>(), room, z.B,
                    z.H, z.HKV, z.D, max_blocks, (float)scale, fp8, aligned,
-                   cur_stream());
+                   &next, cur_stream());
   return out;
 }
 
@@ -795,7 +816,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("paged_attn_shares", &paged_attn_shares);
   m.def("cache_put", &cache_put);
   m.def("norm_parts", &norm_parts);
-  m.def("step_attn", &step_attn);
+  m.def("step_attn", &step_attn, py::arg("qkv"), py::arg("cs"), py::arg("sn"),
+        py::arg("ctx"), py::arg("kcache"), py::arg("vcache"),
+        py::arg("block_table"), py::arg("bias"), py::arg("scale"),
+        py::arg("slots"), py::arg("arrived"), py::arg("ahead") = py::none());
   m.def("step_plan", &step_plan);
   m.def("rope_put", &rope_put, py::arg("qkv"), py::arg("cs"), py::arg("sn"),
         py::arg("ctx"), py::arg("kcache"), py::arg("vcache"),

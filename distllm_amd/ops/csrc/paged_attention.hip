@@ -40,6 +40,7 @@
 // Those kernels are still the faster ones where contexts of a page or two meet
 // 16 key heads and rows or more (64 x 32 heads of 128, of 16: 11, now 19), for
 // which the lengths, on the device only, would have to be known ahead.
+#include "ahead.h"
 #include "common.h"
 #include <hip/hip_fp8.h>
 
@@ -96,6 +97,7 @@ struct PaStep {
   // its length, first tile, the one behind the last; of the sequence, the first
   // share and their number
   const int* slots;
+  Ahead ahead;
 };
 
 // Columns c .. c + 3 and D / 2 + c .. of head h of row b, as bf16 numbers; ROT:
@@ -183,6 +185,33 @@ constexpr int pa_lds(int D, int R) {
   return ring > states ? ring : states;
 }
 
+// The attention of a few sequences is latency and leaves the memory idle. The
+// last workgroups of its launch read the weights of the product behind it
+// meanwhile, each run of 16 rows into the L2 of the XCD on which the product's
+// workgroup will be (they go round), and so into the cache that all share. A CU
+// takes in some 50 GB/s this way, so it wants most of them: us of a step of 8
+// layers, one sequence of 2048, 32 workgroups 928, 64 840, 128 801, 192 803, none
+// 821; of 32 tokens 925, 832, 786, 760 and 778; 8 of 100 1005, 912, 850, 840, 867;
+// 8-bit weights, 2048 606, 572, 576, 571, 578. (The same behind norms of 5 us
+// shortened the products by less than it lengthened the norms.)
+__device__ __forceinline__ void fetch_ahead(const Ahead& a) {
+  const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int xcd = blockIdx.x % 8, waves = a.blocks / 8 * NW;
+  const int turn = (blockIdx.x - (gridDim.x - a.blocks)) / 8;
+  const int n = (a.chunks - xcd + 7) / 8 * a.pieces;
+  int k = 0;
+  for (int i = turn * NW + wid; i < n; i += waves) {
+    const long piece =
+        (xcd + (long)(i / a.pieces) * 8) * a.pieces + i % a.pieces;
+    // all to one place in LDS, where nobody looks: through registers, eight at a
+    // time, a step of one sequence of 2048 took 836
+    copy_to_lds(a.from + piece * 1024 + lane * 16, smem + wid * 1024);
+    if ((++k & 7) == 0) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
 // ALIGNED: the pages start at a multiple of 16 bytes, as the copies to LDS ask;
 // else bf16 pages pass through registers like fp8 ones, one tile after another.
 // STEP: queries come out of the step's projections and are rotated here, into
@@ -204,6 +233,18 @@ paged_attn_kernel(const unsigned short* __restrict__ q, long q_stride,
   constexpr int PIECES = KT / ROWS;     // pieces of K or V of a tile
   constexpr int TILE = KT * D * 2;      // bytes of K or V of a tile
   constexpr int DB = D / 16;
+  if constexpr (STEP) {
+    if (blockIdx.x >= gridDim.x - step.ahead.blocks) {
+      // where there are more pages than weights to read, the time is theirs: us
+      // of a step of 8 sequences of 2048 990 without, 995 with
+      long cached = 0;
+      for (int i = 0; i < B; ++i) cached += ctx_len[i];
+      if (cached * HKV * D * (FP8 ? 2 : 4) <=
+          (long)step.ahead.chunks * step.ahead.pieces * 1024)
+        fetch_ahead(step.ahead);
+      return;
+    }
+  }
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int c16 = lane & 15, g = lane >> 4;
@@ -635,8 +676,9 @@ static void pa_launch(const void* q, long q_stride, const PaStep* step,
                       int max_blocks, int NS, float scale, bool fp8,
                       bool aligned, hipStream_t stream) {
   const int GR = H / HKV, NG = (GR + 15) / 16;
-  const int grid = (step != nullptr ? 1 : B) * HKV * NG * NS;
   const PaStep in = step != nullptr ? *step : PaStep{};
+  const int grid =
+      (step != nullptr ? 1 : B) * HKV * NG * NS + in.ahead.blocks;
 #define PA(DD, F8, AL, R, ST)                                                 \
   hipLaunchKernelGGL((paged_attn_kernel<DD, F8, AL, R, ST>), dim3(grid),      \
                      dim3(256), pa_lds(DD, R) + (ST ? 18 * DD * 2 : 0), stream, \
@@ -699,10 +741,10 @@ extern "C" void launch_step_attn(const void* qkv, const float* parts, int S,
                                  int* arrived, const int* slots, int G, int B,
                                  int H, int HKV, int D, int max_blocks,
                                  float scale, bool fp8, bool aligned,
-                                 hipStream_t stream) {
+                                 const Ahead* ahead, hipStream_t stream) {
   const PaStep step = {(const unsigned short*)qkv, parts, S,
-                       (const unsigned short*)bias, cs, sn,
-                       slots};
+                       (const unsigned short*)bias, cs, sn, slots,
+                       *ahead};
   pa_launch(nullptr, 0, &step, kcache, vcache, block_table, ctx_len, out, pacc,
             pml, arrived, B, H, HKV, D, max_blocks, G, scale, fp8, aligned,
             stream);

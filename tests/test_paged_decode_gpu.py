@@ -354,3 +354,23 @@ def test_step_in_a_graph(device):
         torch.cuda.synchronize()
         assert all(torch.equal(a, b) for a, b in zip(got, want))
         run()
+
+
+@pytest.mark.parametrize("shape,dtype,step", [
+    ((128, 64), torch.uint8, 1), ((136, 64), torch.bfloat16, 1),
+    ((4099, 2048), torch.bfloat16, 1), ((127, 64), torch.bfloat16, 1),
+    ((512, 96), torch.uint8, 1), ((512, 128), torch.bfloat16, 2),
+    ((40000, 1024), torch.bfloat16, 1)])
+def test_step_fetches_ahead(device, shape, dtype, step):
+    """Weights that come to the caches beside the attention change nothing,
+    also where their rows or pieces do not divide, and past the most."""
+    qkv, cs, sn, ctx, raw, table, _ = _step(device, [70, 1, 33], 32, 8, 128,
+                                            False, 8)
+    w = torch.ones(shape, device=device).to(dtype)[:, ::step]
+    outs = []
+    for ahead in (None, w):
+        plan = ops.step_plan(1, ctx, 32, raw[0], table)[0]
+        outs.append(ops.step_attn(qkv, cs, sn, ctx, *raw, table, None, 0.1,
+                                  plan, ahead))
+    assert torch.equal(*outs)
+    assert bool((w == 1).all())
