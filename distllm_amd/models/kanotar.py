@@ -11,9 +11,21 @@ sublayer.
 from __future__ import annotations
 
 import torch
+from torch.nn.modules import module
 
 from .. import ops
+from .blocks import ClampedGlu, LatentAttention
 from .layered import LayeredCache, LayeredModel
+
+
+def _shared(part) -> dict:
+    """Arguments with which a sublayer leaves the sum over shares of K to the
+    norm behind it; none where a hook sees its output, or it has other forms."""
+    return ({"linear": ops.linear_parts}
+            if type(part) in (ClampedGlu, LatentAttention)
+            and "forward" not in part.__dict__
+            and not (part._forward_hooks or module._global_forward_hooks)
+            else {})
 
 
 class KanotarModel(LayeredModel):
@@ -29,14 +41,15 @@ class KanotarModel(LayeredModel):
         for i, layer in enumerate(self.layers):
             after = (self.layers[i + 1].norm1 if i + 1 < len(self.layers)
                      else self.final_norm)
-            y = layer.mixer(h, batch, cache.layers[i])
+            y = layer.mixer(h, batch, cache.layers[i],
+                            **_shared(layer.mixer))
             if layer.mlp is None:
                 h = ops.post_norm_add(y, x, layer.norm1b, after, W, eps)
             else:
                 h = ops.post_norm_add(y, x, layer.norm1b, layer.norm2, W,
                                       eps)
-                h = ops.post_norm_add(layer.mlp(h), x, layer.norm2b, after,
-                                      W, eps)
+                h = ops.post_norm_add(layer.mlp(h, **_shared(layer.mlp)), x,
+                                      layer.norm2b, after, W, eps)
             if trace is not None:
                 trace.append(x[:, :W].clone())
         return h

@@ -923,7 +923,8 @@ def embed_norm(tokens, table, w_next, n, eps):
 
 def post_norm_add(y, x, w_post, w_next, n, eps):
     """End of a sandwich-normed sublayer: x += rms(y) * w_post (x fp32,
-    in place), returns the next sublayer's input rms(x) * w_next."""
+    in place), returns the next sublayer's input rms(x) * w_next. y may be
+    what linear_parts returned."""
     if y.is_cuda:
         _require_hip("_hip_residual")
         return _hip_ops.sandwich_norm(y, None, x, w_post, w_next, n, eps)

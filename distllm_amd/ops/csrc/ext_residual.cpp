@@ -3,7 +3,7 @@
 #include "ext_common.h"
 
 extern "C" {
-void launch_sandwich_norm(const void*, const long*, float*, const float*,
+void launch_sandwich_norm(const void*, int, const long*, float*, const float*,
                           const float*, void*, int, int, int, float, bool,
                           hipStream_t);
 void launch_embed_positions(const void*, const void*, const long*, const int*,
@@ -25,7 +25,8 @@ void launch_rotation_table(const int*, const double*, float, float*, int, int,
                            hipStream_t);
 }
 
-// y == embedding table when tokens are given
+// y == embedding table when tokens are given; else it may be the fp32 slabs
+// [shares, M, W] of a bf16 product
 torch::Tensor sandwich_norm(torch::Tensor y,
                             c10::optional<torch::Tensor> tokens,
                             torch::Tensor x,
@@ -35,7 +36,9 @@ torch::Tensor sandwich_norm(torch::Tensor y,
   CHECK_DEV(x); CHECK_CONT(x); CHECK_F32(x);
   CHECK_DEV(w_next); CHECK_CONT(w_next); CHECK_F32(w_next);
   const int M = x.size(0), W = x.size(1);
-  TORCH_CHECK(x.dim() == 2 && y.dim() == 2 && y.size(1) == W, "row sizes");
+  const int shares = y.dim() == 3 && !tokens && is_f32(y) ? y.size(0) : 0;
+  TORCH_CHECK(x.dim() == 2 && (y.dim() == 2 || shares > 0) && y.size(-1) == W,
+              "row sizes");
   TORCH_CHECK(W % 8 == 0 && W <= 16384 && n > 0 && n <= W,
               "width must be a multiple of 8, at most 16384");
   TORCH_CHECK(w_next.numel() == W, "w_next size");
@@ -46,17 +49,19 @@ torch::Tensor sandwich_norm(torch::Tensor y,
                 "tokens must be int64, one per row");
     tok = (const long*)tokens->data_ptr<int64_t>();
   } else {
-    TORCH_CHECK(y.size(0) == M, "y rows");
+    TORCH_CHECK(y.size(-2) == M, "y rows");
     TORCH_CHECK(w_post.has_value() && w_post->numel() == W, "w_post size");
     CHECK_DEV(w_post.value()); CHECK_CONT(w_post.value());
     CHECK_F32(w_post.value());
   }
-  auto h = torch::empty({M, W}, y.options());
+  auto h = torch::empty({M, W}, shares ? y.options().dtype(at::kBFloat16)
+                                       : y.options());
   if (M > 0)
-    launch_sandwich_norm(y.data_ptr(), tok, x.data_ptr<float>(),
+    launch_sandwich_norm(y.data_ptr(), shares, tok, x.data_ptr<float>(),
                          tok ? nullptr : w_post->data_ptr<float>(),
                          w_next.data_ptr<float>(), h.data_ptr(), M, W,
-                         (int)n, (float)eps, is_f32(y), cur_stream());
+                         (int)n, (float)eps, is_f32(y) && !shares,
+                         cur_stream());
   return h;
 }
 

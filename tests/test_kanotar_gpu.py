@@ -13,6 +13,8 @@ import torch
 import kanotar_cases as cases
 import kanotar_oracle as oracle
 from distllm_amd import ops
+from distllm_amd.models import build_model, kanotar
+from distllm_amd.models.config import layered_preset
 from distllm_amd.ops import torch_ref
 
 pytestmark = pytest.mark.gpu
@@ -166,6 +168,46 @@ def test_sandwich_norm(device, dtype, M, W, n):
     h_ref = torch_ref.post_norm_add(y.float(), x_ref, wp, wn, n, 0.01)
     _close(x, x_ref, F32)
     _close(h, h_ref, dtype)
+
+
+@pytest.mark.parametrize("S, M, W, n", [(2, 17, 64, 60), (5, 64, 1088, 1088),
+                                        (1, 33, 4096, 4000), (9, 20, 8192, 8192)])
+def test_sandwich_norm_of_parts(device, S, M, W, n):
+    """Slabs of a product, summed in their order and rounded to bf16."""
+    parts = _rand(S, M, W)
+    parts[..., n:] = 0
+    wn, wp, x = _rand(W, seed=2), _rand(W, seed=3), _rand(M, W, seed=4)
+    y = torch.zeros_like(parts[0])
+    for p in parts:
+        y += p
+    want = x.clone()
+    h_want = ops.post_norm_add(y.bfloat16(), want, wp, wn, n, 0.01)
+    h = ops.post_norm_add(parts, x, wp, wn, n, 0.01)
+    assert torch.equal(h, h_want) and torch.equal(x, want)
+
+
+def test_sublayers_that_are_watched(device):
+    """A hook on a sublayer sees its output, and changes no result."""
+    model = build_model(layered_preset(
+        2, 1024, 64, 8, 64, 64, 64, 512, 8192, [64], limit=7.0),
+        device=device)
+    with torch.no_grad():
+        for p in model.layers[0].mlp.parameters():
+            p.normal_(0, 0.03)
+    h = _rand(20, 1024, dtype=torch.bfloat16)
+    mlp = model.layers[0].mlp
+    seen = []
+    hook = mlp.register_forward_hook(lambda m, i, o: seen.append(o))
+    assert kanotar._shared(mlp) == {}
+    want = mlp(h)
+    hook.remove()
+    assert seen[0].shape == want.shape == (20, 1024)
+    parts = mlp(h, **kanotar._shared(mlp))
+    assert parts.dtype == torch.float32 and parts.dim() == 3
+    total = torch.zeros_like(parts[0])
+    for p in parts:
+        total += p
+    assert torch.equal(total.bfloat16(), want)
 
 
 @pytest.mark.parametrize("dtype", DTYPES, ids=ids)
