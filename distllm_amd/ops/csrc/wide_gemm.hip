@@ -368,31 +368,34 @@ __global__ void __launch_bounds__(256, 1) wide_gemm_kernel(const WgArgs p) {
 }
 
 // Rows of a tile / 32: those with the least rounds of the card's 256 CUs times
-// what a tile costs, which is its rows and as much as 32 more (768 x 768 of
-// 12992 rows, us: fm 8 to 4 19.8, 18.7, 17.9, 17.3, 22.6, by this rule 9, 8, 7,
-// 6, 10; 4096 x 14336 of 8448 rows 850, 794, 749, 894, 1004: 27, 24, 21, 24,
-// 25). Ties go to the larger tile. *full: the share of the CUs that a single
-// round takes, or 1.
-static int wg_tile(int M, int N, float* full) {
+// what a tile costs, which is its rows and, for W and the turn to the next tile, as
+// much as 192 more. us, fm 8 to 4: 12992 x 768 x 768 19.8, 18.7, 17.9, 17.3, 22.6, by
+// this rule 14, 13, 12, 11, 20; 8448 x 4096 x 14336 850, 794, 749, 894, 1004: 42, 39,
+// 36, 44, 50. A round of 28672 x 4096 gated 80, 73, 68, 65, 62. Ties go to the larger
+// tile. *tiles: their number.
+static int wg_tile(int M, int N, long* tiles) {
   int best = 8;
   long least = -1;
   for (int fm = 8; fm >= 4; --fm) {
-    const long tiles = (long)((M + 32 * fm - 1) / (32 * fm)) * (N / 256);
-    const long cost = ((tiles + 7) / 8 + 31) / 32 * (fm + 1);
+    const long n = (long)((M + 32 * fm - 1) / (32 * fm)) * (N / 256);
+    const long cost = ((n + 7) / 8 + 31) / 32 * (fm + 6);
     if (least >= 0 && cost >= least) continue;
     least = cost;
     best = fm;
-    *full = tiles < 256 ? tiles / 256.f : 1.f;
+    *tiles = n;
   }
   return best;
 }
 
 // The tile with which this product is the faster one, 0 where another is.
 // Measured against the library's product (and the activation's or unit's own
-// launch), own time over its, in a graph:
-// - A first round that leaves CUs idle: without activation 176 tiles and more
-//   0.88 to 1.0, 120 to 160 1.0 to 1.15, fewer up to 3; with one, K <= 1536, 96
-//   and more 0.7 to 0.92, 60 1.02.
+// launch), own time over its, in a graph, over weights that come from memory:
+// - A single round, by the share of the card's 256 tiles of 256 rows that its tiles
+//   make: without activation and K of 1536 and more 0.58 to 0.9 0.75 to 1.02, 0.5 to
+//   0.55 1.04 to 1.08, below 1.1 to 1.4; a gated unit of long rows 0.54 and more 0.83
+//   to 1.0, 0.44 1.02 to 1.23. Shorter sums: without activation 216 tiles and more
+//   0.79 to 1.0, 120 to 200 1.0 to 1.23, fewer up to 3; with one 96 tiles and more
+//   0.7 to 0.92, 60 1.02.
 // - Long sums whose 256 x 256 tiles fill their rounds, which is the library's
 //   best case: K of 1536 and more, a share of 0.87 and more 1.01 to 1.09, below
 //   0.73 to 0.99. With K to 1280 0.86 to 1.0 all the same, and with an
@@ -401,15 +404,21 @@ extern "C" int wide_gemm_tile(int M, int N, int K, int act) {
   if (M <= 0 || N <= 0 || N % 256 || K % 64 || K < 128 ||
       (long)N * K >= 1L << 30 || M >= 1 << 30)
     return 0;
-  float full = 0.f;
-  const int fm = wg_tile(M, N, &full);
+  long tiles = 0;
+  const int fm = wg_tile(M, N, &tiles);
   const long ntn = N / 256;
-  if ((long)((M + 32 * fm - 1) / (32 * fm)) * ntn * ntn * WG_GROUP >= 1L << 32)
+  if (tiles * ntn * WG_GROUP >= 1L << 32)
     return 0;  // divisions by multiplication
-  if (full < (act != WG_NONE && K <= 1536 ? 0.375f : 0.6875f)) return 0;
+  if (tiles <= 256) {
+    if (K >= 1536 && !(act != WG_NONE && K == 1536)) {
+      if (tiles * fm < (act == WG_NONE ? 0.58f : 0.5f) * 2048) return 0;
+    } else if (tiles < (act != WG_NONE ? 96 : 208)) {
+      return 0;
+    }
+  }
   if (act == WG_NONE && K >= 1536) {
-    const long tiles = (long)((M + 255) / 256) * ntn;
-    if (tiles >= 0.87f * ((tiles + 255) / 256 * 256)) return 0;
+    const long most = (long)((M + 255) / 256) * ntn;
+    if (most >= 0.87f * ((most + 255) / 256 * 256)) return 0;
   }
   return fm;
 }

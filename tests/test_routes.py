@@ -167,6 +167,11 @@ def test_many_rows_go_by_tiles_and_sums():
     assert tile(1000, 3072, 768, 2) == 4   # and enough with an activation
     assert tile(16384, 4096, 4096, 0) == 0  # whole rounds of long sums
     assert tile(16384, 28672, 4096, 4) == 8
+    # a round of low tiles reads the weights too often
+    assert tile(1500, 4096, 4096, 0) == tile(1025, 6144, 4096, 0) == 0
+    assert tile(200, 28672, 4096, 4) == tile(1500, 3840, 1280, 0) == 0
+    assert tile(300, 28672, 4096, 4) == 5 and tile(1025, 28672, 4096, 4) == 6
+    assert tile(3000, 4096, 4096, 0) == 6 and tile(12992, 768, 3072, 0) == 5
     shares = ops._hip_ops.mid_gemm_shares
     for sizes in [(64, 768, 768), (300, 760, 768), (300, 768, 760),
                   (300, 768, 64), (300, 0, 768), (1300, 2304, 768),
