@@ -56,8 +56,10 @@ __device__ __forceinline__ float wg_gelu(float x) {
   p = fmaf(p, y, -0.45967310667037964f);
   p = fmaf(p, y, -1.1509627103805542f);
   p = fmaf(p, y, -1.000006079673767f);
-  // infinity times zero is kept out, NaN is in p
-  return fmaf(-fminf(y, 3e38f), __builtin_amdgcn_exp2f(p), fmaxf(x, 0.f));
+  // infinity times zero is kept out of a positive x; minus infinity gives NaN,
+  // as x Phi(x) written down does, and NaN is in p
+  return fmaf(-fabsf(fminf(x, 3e38f)), __builtin_amdgcn_exp2f(p),
+              fmaxf(x, 0.f));
 }
 
 template <int ACT>

@@ -93,6 +93,20 @@ def test_gelu_of_large_and_not_finite():
     assert (same | close).all()
 
 
+@pytest.mark.parametrize("act", [ops.ACT_GELU_TANH, ops.ACT_GELU_ERF,
+                                 ops.ACT_SILU])
+def test_activations_of_infinities(act):
+    """As torch has them, NaN for minus infinity among them."""
+    x, w, b = _operands(300, 256, 128)
+    x[:], w[:] = 1.0, 0.0
+    b[:] = torch.tensor([float("inf"), float("-inf"), float("nan"), 0.0],
+                        device="cuda").repeat(64)
+    got = ops._hip_ops.wide_gemm(x, w, b, act, 8).double()
+    want = _reference(x, w, b, act)
+    assert want[0, 1].isnan()
+    torch.testing.assert_close(got, want, rtol=0, atol=0, equal_nan=True)
+
+
 def test_linear_takes_it_and_gives_the_library_s_result(monkeypatch):
     """Over the forms that linear accepts: shapes with leading dimensions,
     strided inputs and biases, storage that starts between 16-byte pieces."""
