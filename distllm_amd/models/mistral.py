@@ -279,7 +279,8 @@ class DecoderModel(nn.Module):
 
         tokens: [B] int; cache: per-layer paged [nblk, HKV, BLK, D];
         ctx_lens: [B] int32 length INCLUDING the new token (the new
-        token's kv is written at position ctx_lens-1 by this call).
+        token's kv is written at position ctx_lens-1 by this call; rows may
+        be tokens of one sequence that follow each other, with one block table).
         Returns logits [B, V] f32.
         """
         d = self.dims

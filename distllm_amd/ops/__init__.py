@@ -885,16 +885,16 @@ def step_plan(layers, ctx, H, kcache, block_table):
     if not kcache.is_cuda or D not in (64, 128):
         return [None] * layers
     _require_hip()
-    slots, zeros = _hip_ops.step_plan(ctx.int(), layers, H, HKV,
-                                      block_table.shape[1],
-                                      kcache.dtype == torch.uint8)
+    slots, zeros = _hip_ops.step_plan(ctx.int(), block_table.int(), layers, H,
+                                      HKV, kcache.dtype == torch.uint8)
     return [(slots, row) for row in zeros.unbind()]
 
 
 def step_attn(qkv, cs, sn, ctx, kcache, vcache, block_table, bias, scale,
               plan, ahead=None):
-    """rope_put and the attention of its queries over the cache, the new token
-    among it -> [B, H, D]; one launch for heads of 64 and 128. plan: an item of
+    """rope_put and the attention of its queries over the cache, the new tokens
+    of all rows among it (of a sequence several rows may be one token each, in
+    any order) -> [B, H, D]; one launch for heads of 64 and 128. plan: an item of
     step_plan, used up. ahead: weights of the product that follows, which few
     sequences leave the time to fetch into the caches."""
     if qkv.is_cuda and qkv.shape[-1] in (64, 128):

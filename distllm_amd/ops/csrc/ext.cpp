@@ -61,8 +61,8 @@ void launch_step_attn(const void*, const float*, int, const void*,
                       const int*, void*, void*, void*, int*, const int*, int,
                       int, int, int, int, int, float, bool, bool, const Ahead*,
                       hipStream_t);
-void launch_step_plan(const int*, int, int, int, int, int, int, int*, int*,
-                      long, hipStream_t);
+void launch_step_plan(const int*, const int*, int, int, int, int, int, int,
+                      int*, int*, long, hipStream_t);
 int step_plan_room(int, int, int, int);
 void launch_norm_parts(const float*, int, const void*, const void*, void*,
                        void*, int, int, float, hipStream_t);
@@ -507,20 +507,25 @@ static StepShares step_shares(int64_t B, int64_t H, int64_t HKV,
 }
 
 // What the attention launches of a decode step of `layers` layers need:
-// [room, 8] shares, and zeros [layers, B * HKV * groups of 16 query heads], a row
+// [room, 8] shares and what PaStep says of them, and zeros [layers, B * HKV * groups of 16 query heads], a row
 // of which each launch uses up.
-std::vector<torch::Tensor> step_plan(torch::Tensor ctx, int64_t layers,
-                                     int64_t H, int64_t HKV,
-                                     int64_t max_blocks, bool fp8) {
+std::vector<torch::Tensor> step_plan(torch::Tensor ctx,
+                                     torch::Tensor block_table, int64_t layers,
+                                     int64_t H, int64_t HKV, bool fp8) {
   CHECK_INTS(ctx);
+  CHECK_INTS(block_table);
   TORCH_CHECK(HKV > 0 && H % HKV == 0, "GQA requires H % HKV == 0");
   const int64_t B = ctx.numel();
+  TORCH_CHECK(block_table.dim() == 2 && block_table.size(0) == B &&
+                  block_table.device() == ctx.device(),
+              "block_table must be [B, blocks]");
+  const int64_t max_blocks = block_table.size(1);
   const StepShares s = step_shares(B, H, HKV, max_blocks, fp8);
   auto slots = torch::empty({s.room, 8}, ctx.options());
   auto arrived = torch::empty({layers, B * HKV * ((H / HKV + 15) / 16)},
                               ctx.options());
   if (B > 0)
-    launch_step_plan(ctx.data_ptr<int>(), (int)B, (int)max_blocks, s.room,
+    launch_step_plan(ctx.data_ptr<int>(), block_table.data_ptr<int>(), (int)B, (int)max_blocks, s.room,
                      s.narrow, s.wide, s.asked, slots.data_ptr<int>(),
                      arrived.data_ptr<int>(), arrived.numel(), cur_stream());
   return {slots, arrived};

@@ -95,7 +95,8 @@ struct PaStep {
   const float *cs, *sn;
   // the launch's shares (step_plan_kernel), eight numbers each: sequence or -1,
   // its length, first tile, the one behind the last; of the sequence, the first
-  // share and their number
+  // share and their number. The seventh of the first B is not a share's but that
+  // row's: whether another row of the step is an earlier token of its sequence
   const int* slots;
   Ahead ahead;
 };
@@ -219,6 +220,9 @@ __device__ __forceinline__ void fetch_ahead(const Ahead& a) {
 // value where the share ends with it: the wave that has the last tile puts them
 // into it, and they go to the cache (from the first of several groups of heads).
 // A launch that did this ahead (rope_put_kernel) took 4.7 us.
+// Rows of one step may be tokens of one sequence that follow each other. Nothing
+// orders this launch's workgroups, so those of a later token put the earlier ones
+// into the cache themselves, too, with the same numbers, ahead of their first tile.
 template <int D, bool FP8, bool ALIGNED, int R, bool STEP>
 __global__ void __launch_bounds__(256)
 paged_attn_kernel(const unsigned short* __restrict__ q, long q_stride,
@@ -335,16 +339,65 @@ paged_attn_kernel(const unsigned short* __restrict__ q, long q_stride,
     }
   };
 
+  const int pos = ctx - 1, heads = H + 2 * HKV;
+  // Numbers c .. and D / 2 + c .. of a row of the cache; of fp8 pages they come
+  // back as what the cache then holds.
+  auto put = [&](char* to, int c, unsigned short* a, unsigned short* e,
+                 bool write) {
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      unsigned short* x = half ? e : a;
+      const int col = c + half * (D / 2);
+      if constexpr (FP8) {
+        unsigned char eight[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          cache_store(&eight[i], x[i]);
+          __hip_fp8_e4m3 f;
+          f.__x = eight[i];
+          x[i] = f2bf((float)f);
+        }
+        if (write)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) to[col + i] = (char)eight[i];
+      } else if (write) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          reinterpret_cast<unsigned short*>(to)[col + i] = x[i];
+      }
+    }
+  };
+  fetch_pages(0);
+  if constexpr (STEP) {
+    if (B > 1 && step.slots[b * 8 + 6] != 0) {
+      for (int j = 0; j < B; ++j) {
+        const int p = ctx_len[j] - 1;
+        if (j == b || p < 0 || p >= pos || p / PBLK >= max_blocks) continue;
+        const int pg = block_table[(long)j * max_blocks + p / PBLK];
+        if (bt[p / PBLK] != pg || threadIdx.x >= D / 4) continue;
+        const int row = threadIdx.x / (D / 8), c = threadIdx.x % (D / 8) * 4;
+        unsigned short a[4], e[4];
+        step_columns<D>(step, B, heads, j, H + row * HKV + kvh, c, row == 0, p,
+                        a, e);
+        put((row == 0 ? kcache : vcache) + pg * page_bytes + head_bytes +
+                (long)(p % PBLK) * D * (FP8 ? 1 : 2),
+            c, a, e, true);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+      __syncthreads();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    }
+  }
+
   // the first tile is on its way while the queries come
   int at = 0;  // tiles issued
   auto next = [&]() {
-    if ((at & 31) == 0) fetch_pages(at);
+    if (at > 0 && (at & 31) == 0) fetch_pages(at);
     if constexpr (FP8) issue8(at++);
     else issue(at++);
   };
   while (at < (R > 1 ? R - 1 : 1) && at < mine) next();
 
-  const int pos = ctx - 1;
   // of the workgroup, of the wave: its share ends with the new token
   const bool newest = STEP && pos >= 0 && pos < max_blocks * PBLK && T > 0 &&
                       T - 1 >= first_tile && T - 1 < t1;
@@ -352,7 +405,6 @@ paged_attn_kernel(const unsigned short* __restrict__ q, long q_stride,
   // rotated queries, the new key and value: rows of D in LDS
   char* rows = smem + pa_lds(D, R);
   if constexpr (STEP) {
-    const int heads = H + 2 * HKV;
     const int units = (nh + (newest ? 2 : 0)) * (D / 8);
     for (int u = threadIdx.x; u < units && pos >= 0; u += NW * 64) {
       const int row = u / (D / 8), c = u % (D / 8) * 4;
@@ -360,33 +412,10 @@ paged_attn_kernel(const unsigned short* __restrict__ q, long q_stride,
                              : H + (row - nh) * HKV + kvh;
       unsigned short a[4], e[4];
       step_columns<D>(step, B, heads, b, h, c, row <= nh, pos, a, e);
-      if (row >= nh) {
-        char* to = (row == nh ? kcache : vcache) +
-                   bt[pos / PBLK] * page_bytes + head_bytes +
-                   (long)(pos % PBLK) * D * (FP8 ? 1 : 2);
-#pragma unroll
-        for (int half = 0; half < 2; ++half) {
-          unsigned short* x = half ? e : a;
-          const int col = c + half * (D / 2);
-          if constexpr (FP8) {
-            unsigned char eight[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              cache_store(&eight[i], x[i]);
-              __hip_fp8_e4m3 f;
-              f.__x = eight[i];
-              x[i] = f2bf((float)f);
-            }
-            if (hg == 0)
-#pragma unroll
-              for (int i = 0; i < 4; ++i) to[col + i] = (char)eight[i];
-          } else if (hg == 0) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-              reinterpret_cast<unsigned short*>(to)[col + i] = x[i];
-          }
-        }
-      }
+      if (row >= nh)
+        put((row == nh ? kcache : vcache) + bt[pos / PBLK] * page_bytes +
+                head_bytes + (long)(pos % PBLK) * D * (FP8 ? 1 : 2),
+            c, a, e, hg == 0);
       *reinterpret_cast<i32x2*>(rows + (row * D + c) * 2) =
           *reinterpret_cast<const i32x2*>(a);
       *reinterpret_cast<i32x2*>(rows + (row * D + c + D / 2) * 2) =
@@ -773,23 +802,44 @@ __host__ __device__ constexpr bool plan_many(int B, int p) {
 }
 constexpr int PLAN_ROWS = 1024;  // beyond, each sequence is a share, in order
 __global__ void __launch_bounds__(256)
-step_plan_kernel(const int* __restrict__ ctx, int B, int max_blocks, int G,
-                 int narrow, int wide, int asked, int4* __restrict__ slots,
-                 int* __restrict__ arrived, long zeros) {
+step_plan_kernel(const int* __restrict__ ctx, const int* __restrict__ table,
+                 int B, int max_blocks, int G, int narrow, int wide, int asked,
+                 int4* __restrict__ slots, int* __restrict__ arrived,
+                 long zeros, int clear) {
   const int tid = threadIdx.x;
+  if (blockIdx.x > clear) {
+    // a wave for each row: does another one put a token into a page that it
+    // reads, ahead of its own
+    const int i = (blockIdx.x - 1 - clear) * 4 + (tid >> 6);
+    if (i >= B) return;
+    const int pos = ctx[i] - 1;
+    bool found = false;
+    for (int j = tid & 63; j < B; j += 64) {
+      const int p = ctx[j] - 1, pg = p / PBLK;
+      if (j != i && p >= 0 && p < pos && pg < max_blocks)
+        found |= table[(long)i * max_blocks + pg] ==
+                 table[(long)j * max_blocks + pg];
+    }
+    found = __any(found);
+    if ((tid & 63) == 0) reinterpret_cast<int*>(slots)[i * 8 + 6] = found;
+    return;
+  }
   if (blockIdx.x > 0) {
-    for (long i = (blockIdx.x - 1) * 256L + tid; i < zeros;
-         i += (gridDim.x - 1) * 256L)
+    for (long i = (blockIdx.x - 1) * 256L + tid; i < zeros; i += clear * 256L)
       arrived[i] = 0;
     return;
   }
+  // (of the second four of a share's numbers two are other workgroups')
+  auto of_sequence = [&](int slot, int first, int n) {
+    *reinterpret_cast<int2*>(slots + slot * 2 + 1) = int2{first, n};
+  };
   auto length = [&](int b) { return min(max(ctx[b], 0), max_blocks * PBLK); };
   if (B > PLAN_ROWS) {
     for (int i = tid; i < G; i += 256) {
       const bool is = i < B;
       slots[i * 2] = int4{is ? i : -1, is ? ctx[i] : 0, 0,
                           is ? (length(i) + KT - 1) / KT : 0};
-      slots[i * 2 + 1] = int4{i, 1, 0, 0};
+      of_sequence(i, i, 1);
     }
     return;
   }
@@ -862,7 +912,7 @@ step_plan_kernel(const int* __restrict__ ctx, int B, int max_blocks, int G,
     for (int i = 0; i < n && first + i < G; ++i) {
       slots[(first + i) * 2] =
           int4{b, ctx[b], min(i * per, t), min((i + 1) * per, t)};
-      slots[(first + i) * 2 + 1] = int4{first, n, 0, 0};
+      of_sequence(first + i, first, n);
     }
   }
   // thread 0 has a sequence
@@ -879,14 +929,15 @@ extern "C" int step_plan_room(int B, int narrow, int wide, int asked) {
   return plan_many(B, p) ? B + 2 * p / 3 : p;
 }
 
-extern "C" void launch_step_plan(const int* ctx, int B, int max_blocks, int G,
-                                 int narrow, int wide, int asked, int* slots,
-                                 int* arrived, long zeros,
-                                 hipStream_t stream) {
+extern "C" void launch_step_plan(const int* ctx, const int* table, int B,
+                                 int max_blocks, int G, int narrow, int wide,
+                                 int asked, int* slots, int* arrived,
+                                 long zeros, hipStream_t stream) {
   const int clear = (int)std::min((zeros + 1023) / 1024, 256L);
-  hipLaunchKernelGGL(step_plan_kernel, dim3(1 + clear), dim3(256),
-                     B > PLAN_ROWS ? 0 : B * 12, stream, ctx, B, max_blocks, G,
-                     narrow, wide, asked, (int4*)slots, arrived, zeros);
+  hipLaunchKernelGGL(step_plan_kernel, dim3(1 + clear + (B + 3) / 4),
+                     dim3(256), B > PLAN_ROWS ? 0 : B * 12, stream, ctx, table,
+                     B, max_blocks, G, narrow, wide, asked, (int4*)slots,
+                     arrived, zeros, clear);
 }
 
 // Write one new token's K/V into the paged cache (decode step).

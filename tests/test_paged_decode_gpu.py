@@ -321,6 +321,41 @@ def test_step_plan(device, lens, HKV, groups, fp8):
         assert n == [32]
 
 
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("H,HKV,D", [(32, 8, 128), (20, 1, 64)])
+@pytest.mark.parametrize("slabs", [0, 3])
+def test_step_rows_of_one_sequence(device, H, HKV, D, fp8, slabs):
+    """Tokens of one sequence that follow each other, in any order, over the
+    edge of a page and in a share of their own; and two sequences that have but
+    their first page in common."""
+    lens = [33, 31, 20, 34, 2001, 32, 2000, 40, 25]
+    qkv, cs, sn, ctx, raw, table, bias = _step(device, lens, H, HKV, D, fp8,
+                                               128, slabs)
+    table[[0, 3, 5]] = table[1].clone()
+    table[4] = table[6].clone()
+    table[8, 0] = table[7, 0]
+    slots, _ = _same_step(device, qkv, cs, sn, ctx, raw, table, bias)
+    assert slots[:9, 6].tolist() == [1, 0, 0, 1, 1, 1, 0, 0, 0]
+
+
+@pytest.mark.parametrize("B", [1, 5, 70, 1030])
+def test_plan_finds_rows_of_one_sequence(device, B):
+    g = torch.Generator().manual_seed(B)
+    ctx = torch.randint(0, 70, (B,), generator=g).int()
+    table = torch.randint(0, 2 * B, (B, 4), generator=g).int()
+    pos = ctx.long() - 1
+    page = pos.clamp(min=0) // 16
+    ok = (pos >= 0) & (page < 4)
+    at = page.clamp(max=3)
+    same = table[:, at] == table[torch.arange(B), at]  # [row, writer]
+    want = (same & ok & (pos < pos[:, None])).fill_diagonal_(False).any(1)
+    pages = torch.empty(2, 8, 16, 128, device=device, dtype=torch.bfloat16)
+    slots, _ = ops.step_plan(1, ctx.to(device), 32, pages,
+                             table.to(device))[0]
+    assert torch.equal(slots[:B, 6].cpu().bool(), want)
+    assert B == 1 or want.any()
+
+
 def test_step_unaligned_pages(device):
     args = list(_step(device, [50, 300], 8, 2, 64, False, 20))
     odd = []
