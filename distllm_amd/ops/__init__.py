@@ -14,6 +14,8 @@ import math
 import os
 
 import torch
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 
 from . import torch_ref
 from .native import Native
@@ -242,11 +244,19 @@ def _gemm_mode() -> str:
 
 def _recorded(*tensors) -> bool:
     """Whether something follows these tensors that a native kernel would
-    pass by: gradients, transforms, dispatch modes, tensors of another make."""
+    pass by: gradients, transforms, traces, modes of dispatch or of functions
+    (but for the one of a default device), tensors of another make, a cast to
+    another 16-bit type."""
     grad = torch.is_grad_enabled()
     return (torch._C._len_torch_dispatch_stack() > 0
             or torch._C._functorch.peek_interpreter_stack() is not None
             or torch.autograd.forward_ad._current_level >= 0
+            or torch._C._get_tracing_state() is not None
+            or (torch._C._len_torch_function_stack() > 0
+                and any(type(m) is not DeviceContext
+                        for m in _get_current_function_mode_stack()))
+            or (torch.is_autocast_enabled("cuda")
+                and torch.get_autocast_dtype("cuda") != torch.bfloat16)
             or any(type(t) not in (torch.Tensor, torch.nn.Parameter)
                    or (grad and t.requires_grad)
                    for t in tensors if t is not None))

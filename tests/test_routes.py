@@ -193,3 +193,31 @@ def test_many_rows_go_by_tiles_and_sums():
         with FlopCounterMode(display=False):
             seen.append(ops._recorded(x))
         assert seen == [True] * 3
+
+
+def test_traces_modes_and_casts_are_followed(monkeypatch):
+    """A kernel would be a constant of a trace, unseen by a mode of functions,
+    and of bf16 where half precision is asked for."""
+    from torch.overrides import TorchFunctionMode
+
+    class Sees(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    x, seen = torch.zeros(2), []
+
+    def f(t):
+        seen.append(ops._recorded(t))
+        return t + 1
+
+    torch.jit.trace(f, x, check_trace=False)
+    with Sees():
+        f(x)
+    with torch.device("cpu"):
+        f(x)
+    # (no autocast for a GPU that is not there)
+    monkeypatch.setattr(torch, "is_autocast_enabled", lambda kind: True)
+    for dtype in (torch.float16, torch.bfloat16):
+        monkeypatch.setattr(torch, "get_autocast_dtype", lambda kind: dtype)
+        f(x)
+    assert seen == [True, True, False, True, False]
