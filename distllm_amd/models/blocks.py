@@ -228,9 +228,10 @@ class LatentAttention(Part):
         return (max(self.dp, self.vp) <= 256
                 and (w.dtype == torch.bfloat16 or not w.is_cuda))
 
-    def forward(self, h, batch, latents, linear=ops.linear):
+    def forward(self, h, batch, latents, linear=None):
         """h [M, width]; latents: the paged cache [blocks, BLK, rank] of
-        the layer that owns it; linear: the last product's form."""
+        the layer that owns it; linear: the last product's form, ops.linear if
+        none is given."""
         d, H = self.d, self.d.heads
         M = h.shape[0]
         bt, ctx = batch.block_table, batch.ctx
@@ -259,7 +260,7 @@ class LatentAttention(Part):
             kv = ops.linear(c, self.wukv)
             ops.attn_window(q[n:], kv, o[n:], e.cu_q, e.cu_k, e.block_map,
                             d.window, d.scale)
-        return linear(o.view(M, H * self.vp), self.wo)
+        return (linear or ops.linear)(o.view(M, H * self.vp), self.wo)
 
 
 class ClampedGlu(Part):
@@ -282,9 +283,10 @@ class ClampedGlu(Part):
             "wdown": padded(t["down"], self.wp, self.fp),
         }
 
-    def forward(self, h, linear=ops.linear):
-        """linear: the last product's form, for a caller that takes another."""
+    def forward(self, h, linear=None):
+        """linear: the last product's form, for a caller that takes another
+        than ops.linear."""
         d = self.d
-        return linear(
+        return (linear or ops.linear)(
             ops.gateup_clamped_glu(h, self.wgup, d.limit, d.alpha, d.shift),
             self.wdown)

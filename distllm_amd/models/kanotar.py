@@ -18,12 +18,16 @@ from .blocks import ClampedGlu, LatentAttention
 from .layered import LayeredCache, LayeredModel
 
 
+_LINEAR = ops.linear
+
+
 def _shared(part) -> dict:
     """Arguments with which a sublayer leaves the sum over shares of K to the
-    norm behind it; none where a hook sees its output, or it has other forms."""
+    norm behind it; none where a hook sees its output, it has other forms, or
+    ops.linear has been replaced and is to see every product."""
     return ({"linear": ops.linear_parts}
             if type(part) in (ClampedGlu, LatentAttention)
-            and "forward" not in part.__dict__
+            and "forward" not in part.__dict__ and ops.linear is _LINEAR
             and not (part._forward_hooks or module._global_forward_hooks)
             else {})
 

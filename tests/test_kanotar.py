@@ -28,6 +28,27 @@ def test_residual_stream(case):
     cases.check_residuals(case)
 
 
+@pytest.mark.parametrize("hooked", [False, True])
+def test_a_replaced_linear_sees_every_product(case, monkeypatch, hooked):
+    """The output products of attention and feed-forward among them, and none
+    is left for the norm behind it to sum."""
+    seen, own = [], ops.linear
+    monkeypatch.setattr(ops, "linear",
+                        lambda x, w, *a, **k: seen.append(w) or own(
+                            x, w, *a, **k))
+    monkeypatch.setattr(ops, "linear_parts", None)
+    parts = [p for layer in case.model.layers
+             for p in (layer.mixer, layer.mlp) if p is not None]
+    hooks = [p.register_forward_hook(lambda *a: None)
+             for p in parts if hooked]
+    cases.check_whole(case)
+    for h in hooks:
+        h.remove()
+    for p in parts:
+        w = p.wo if hasattr(p, "wo") else p.wdown
+        assert any(w is s for s in seen)
+
+
 def test_portions(case):
     cases.check_portions(case)
 
