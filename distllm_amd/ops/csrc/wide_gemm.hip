@@ -45,17 +45,24 @@ struct WgArgs {
 constexpr int WG_SLOT = 32768;
 constexpr int WG_GROUP = 8;  // row tiles that go over the columns together
 
-// x Phi(x) in 32 bits. Phi(-|x|) is 2 to a polynomial of |x| of degree 5, fitted
-// with the least largest |x| Phi error: below 7e-7 everywhere, 5e-5 of results
-// above 0.01, a tenth of what the rounding to 16 bits leaves. 12 issue slots
-// where erf by a reciprocal and an exponential takes 22.
+// x Phi(x) in 32 bits. Phi(-|x|) is 2 to a polynomial of |x| of degree 7 that is
+// -1 at 0 and falls everywhere, fitted with the least largest error of Phi, below
+// 2e-7 or 3e-5 of it. Against 64 bits, and gelu_erf (erf by a reciprocal and an
+// exponential, 22 issue slots where this takes 14): largest error 2.7e-7 (4.7e-7); of
+// results above 0.01 1.9e-6 of them (1.6e-5), above 1e-4 3.4e-4 (1.1e-3); for |x|
+// below 1e-3 1.4e-7 (3.5e-7). Degree 5 leaves 6.7e-7, 5.2e-5, 4.2e-3 and 4.3e-6, at
+// -3.5 and below as much as the rounding to 16 bits; us, degree 5 and 7: 262144 x
+// 3072 x 768 1217, 1250; 12992 x 3072 x 768 69.6, 72.5; 16384 x 5120 x 1280 183.5,
+// 186.6. Degree 6 cannot fall everywhere and be closer than 5.
 __device__ __forceinline__ float wg_gelu(float x) {
   const float y = fabsf(x);
-  float p = fmaf(y, -0.0004843742644879967f, 0.007172281388193369f);
-  p = fmaf(p, y, -0.05207876116037369f);
-  p = fmaf(p, y, -0.45967310667037964f);
-  p = fmaf(p, y, -1.1509627103805542f);
-  p = fmaf(p, y, -1.000006079673767f);
+  float p = fmaf(y, -7.365080705312721e-07f, 4.1180137486662716e-05f);
+  p = fmaf(p, y, -0.000798956782091409f);
+  p = fmaf(p, y, 0.008115779608488083f);
+  p = fmaf(p, y, -0.05338641256093979f);
+  p = fmaf(p, y, -0.4588525891304016f);
+  p = fmaf(p, y, -1.1511530876159668f);
+  p = fmaf(p, y, -1.f);
   // infinity times zero is kept out of a positive x; minus infinity gives NaN,
   // as x Phi(x) written down does, and NaN is in p
   return fmaf(-fabsf(fminf(x, 3e38f)), __builtin_amdgcn_exp2f(p),

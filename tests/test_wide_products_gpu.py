@@ -93,6 +93,19 @@ def test_gelu_of_large_and_not_finite():
     assert (same | close).all()
 
 
+def test_gelu_of_small_results():
+    """To the rounding of the result, half a unit of its eighth bit, also where
+    little is left of x: 4e-4 of results above 1e-4 and 3e-7 are the function's
+    own."""
+    x, w, b = _operands(300, 2048, 128)
+    x[:], w[:] = 1.0, 0.0
+    b[:] = torch.linspace(-4.2, 9, 2048, device="cuda")
+    got = ops._hip_ops.wide_gemm(x, w, b, ops.ACT_GELU_ERF, 8).double()
+    want = F.gelu(b.double())
+    half = torch.ldexp(torch.ones_like(want), want.frexp().exponent - 9)
+    assert ((got - want).abs() <= half + want.abs() * 4e-4 + 3e-7).all()
+
+
 @pytest.mark.parametrize("act", [ops.ACT_GELU_TANH, ops.ACT_GELU_ERF,
                                  ops.ACT_SILU])
 def test_activations_of_infinities(act):
