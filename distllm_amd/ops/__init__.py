@@ -330,12 +330,13 @@ def linear(x, weight, bias=None, act=ACT_NONE):
                 and _few_rows(x2, weight, bias)):
             out = _hip_ops.decode_gemm(x2, weight, bias, 0, _DECODE_ACT[act])
             return out.reshape(*orig_shape[:-1], N)
-        shares = _mid_shares(x2, weight, bias)
+        asked = mode == "decode" and M <= 256  # for that form alone
+        shares = 0 if asked else _mid_shares(x2, weight, bias)
         if shares:
             return _hip_ops.mid_gemm(x2, weight, bias, shares,
                                      _DECODE_ACT[act]).view(
                 *orig_shape[:-1], N)
-        tile = _wide_tile(x2, weight, bias, act)
+        tile = 0 if asked else _wide_tile(x2, weight, bias, act)
         if tile:
             return _hip_ops.wide_gemm(x2, weight, bias, act, tile).view(
                 *orig_shape[:-1], N)

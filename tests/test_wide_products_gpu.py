@@ -218,6 +218,32 @@ def test_linear_of_some_hundred_rows(monkeypatch):
     assert ops.linear(x, w, b).requires_grad or not calls
 
 
+@pytest.mark.parametrize("mode", ["decode", "blaslt", "gemm8", "gemm16"])
+@pytest.mark.parametrize("M", [65, 128, 200, 256])
+@pytest.mark.parametrize("act", [ops.ACT_NONE, ops.ACT_GELU_ERF])
+def test_forms_that_are_asked_for(monkeypatch, mode, M, act):
+    """DISTLLM_GEMM holds where blocks of 64 rows and tiles are the rule."""
+    calls = []
+    for name in ("mid_gemm", "wide_gemm", "decode_gemm"):
+        own = getattr(ops._hip_ops, name)
+        monkeypatch.setattr(
+            ops._hip_ops, name, lambda *a, own=own, name=name:
+            calls.append(name) or own(*a), raising=False)
+    monkeypatch.setattr(ops, "_GEMM_CHOICE", {
+        ("dec", n, 768, 768, True): "blaslt" for n in (128, 256)})
+    x, w, b = _operands(M, 768, 768)
+    with torch.no_grad():
+        ops.linear(x, w, b, act)
+        assert calls == ["mid_gemm"]
+        calls.clear()
+        monkeypatch.setenv("DISTLLM_GEMM", mode)
+        got = ops.linear(x, w, b, act)
+    if act == ops.ACT_NONE:  # else the library's sums are rounded ahead of it
+        _check(got, _reference(x, w, b, act))
+    # (an activation has no form in a launch of decode_gemm here)
+    assert calls == (["decode_gemm"] if (mode, act) == ("decode", 0) else [])
+
+
 def test_in_a_graph():
     x, w, b = _operands(3000, 2304, 768)
     with torch.no_grad():
