@@ -242,24 +242,33 @@ def _gemm_mode() -> str:
     return os.environ.get("DISTLLM_GEMM", "auto")
 
 
+# what _recorded asks in every call, found once
+_grad_enabled, _autocast = torch.is_grad_enabled, torch.is_autocast_enabled
+_tracing, _function_modes = torch._C._is_tracing, torch._C._len_torch_function_stack
+_dispatch_modes = torch._C._len_torch_dispatch_stack
+_transforms = torch._C._functorch.peek_interpreter_stack
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+
+
 def _recorded(*tensors) -> bool:
     """Whether something follows these tensors that a native kernel would
     pass by: gradients, transforms, traces, modes of dispatch or of functions
     (but for the one of a default device), tensors of another make, a cast to
     another 16-bit type."""
-    grad = torch.is_grad_enabled()
-    return (torch._C._len_torch_dispatch_stack() > 0
-            or torch._C._functorch.peek_interpreter_stack() is not None
-            or torch.autograd.forward_ad._current_level >= 0
-            or torch._C._get_tracing_state() is not None
-            or (torch._C._len_torch_function_stack() > 0
+    if (_dispatch_modes() or _transforms() is not None
+            or torch.autograd.forward_ad._current_level >= 0 or _tracing()
+            or (_function_modes()
                 and any(type(m) is not DeviceContext
                         for m in _get_current_function_mode_stack()))
-            or (torch.is_autocast_enabled("cuda")
-                and torch.get_autocast_dtype("cuda") != torch.bfloat16)
-            or any(type(t) not in (torch.Tensor, torch.nn.Parameter)
-                   or (grad and t.requires_grad)
-                   for t in tensors if t is not None))
+            or (_autocast()
+                and torch.get_autocast_dtype("cuda") != torch.bfloat16)):
+        return True
+    grad = _grad_enabled()
+    for t in tensors:
+        if t is not None and (type(t) not in _PLAIN
+                              or (grad and t.requires_grad)):
+            return True
+    return False
 
 
 # activation codes of wide_gemm behind those of linear

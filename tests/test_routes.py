@@ -216,7 +216,7 @@ def test_traces_modes_and_casts_are_followed(monkeypatch):
     with torch.device("cpu"):
         f(x)
     # (no autocast for a GPU that is not there)
-    monkeypatch.setattr(torch, "is_autocast_enabled", lambda kind: True)
+    monkeypatch.setattr(ops, "_autocast", lambda: True)
     for dtype in (torch.float16, torch.bfloat16):
         monkeypatch.setattr(torch, "get_autocast_dtype", lambda kind: dtype)
         f(x)

@@ -244,6 +244,18 @@ def test_forms_that_are_asked_for(monkeypatch, mode, M, act):
     assert calls == (["decode_gemm"] if (mode, act) == ("decode", 0) else [])
 
 
+def test_linear_under_autocast():
+    """To half precision by torch, as ever; to bf16 it is the same product."""
+    x, w, b = _operands(300, 768, 768)
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.float16):
+        got = ops.linear(x, w, b)
+    assert got.dtype == torch.float16
+    with torch.no_grad():
+        want = ops.linear(x, w, b)
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            assert torch.equal(ops.linear(x, w, b), want)
+
+
 def test_in_a_graph():
     x, w, b = _operands(3000, 2304, 768)
     with torch.no_grad():
