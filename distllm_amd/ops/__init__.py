@@ -225,17 +225,22 @@ def _wide_logits(M, N, K) -> bool:
     return M > 16 and N > 32768 and K >= 1536
 
 
-# sizes (M, N, K, bias or not) of such products that ran with their choice
+# sizes (M, N, K, bias or not) of products that ran with their measured choice
+# and have another form to go by
 _WIDE_RUN: set[tuple] = set()
 
 
+def _measurable(M, N, K, bias) -> bool:
+    """While a graph is captured nothing can be measured, neither the choice
+    nor the library's algorithm for a new M: only sizes that ran before go by
+    the measured choice."""
+    return ((M, N, K, bias is not None) in _WIDE_RUN
+            or not torch.cuda.is_current_stream_capturing())
+
+
 def _to_choose(M, N, K, bias) -> bool:
-    """Whether a product of up to 64 rows goes by the measured choice. While a
-    graph is captured nothing can be measured, neither the choice nor the
-    library's algorithm for a new M: only sizes that ran before go by it."""
-    return _wide_logits(M, N, K) and (
-        (M, N, K, bias is not None) in _WIDE_RUN
-        or not torch.cuda.is_current_stream_capturing())
+    """Whether a product of up to 64 rows goes by the measured choice."""
+    return _wide_logits(M, N, K) and _measurable(M, N, K, bias)
 
 
 def _gemm_mode() -> str:
@@ -321,7 +326,7 @@ def linear(x, weight, bias=None, act=ACT_NONE):
     (wide_gemm.hip, with the activation) where _wide_tile says so;
     else an autotuned choice between hipBLASLt (plain and fused-epilogue), the
     other hand-written MFMA GEMMs (gemm8.hip, 8-phase gemm16.hip) and, for M
-    <= 256, decode_gemm.hip. Override with
+    <= 256, decode_gemm.hip and blocks that share K. Override with
     DISTLLM_GEMM=blaslt|gemm8|gemm16|decode (the last for M <= 256, gemm8 and
     gemm16 at their multiples of 256 rows; without an activation M <= 256
     stays a choice for those two, at other sizes they mean the library)."""
@@ -341,7 +346,12 @@ def linear(x, weight, bias=None, act=ACT_NONE):
             return out.reshape(*orig_shape[:-1], N)
         asked = mode == "decode" and M <= 256  # for that form alone
         shares = 0 if asked else _mid_shares(x2, weight, bias)
-        if shares:
+        # up to 256 rows whose K is shared, a second launch, it is one of the
+        # measured choices: us in a graph, this and decode_gemm, 80 rows of 4096 x
+        # 4096 16.4 and 15.4, of 2048 x 8192 16.6 and 17.0, of 768 x 3072 9.6 and
+        # 10.7, 160 rows 10.2 and 12.9 (and the library's 9.6)
+        if shares and not (shares > 1 and act == ACT_NONE and M <= 256
+                           and _measurable(M, N, K, bias)):
             return _hip_ops.mid_gemm(x2, weight, bias, shares,
                                      _DECODE_ACT[act]).view(
                 *orig_shape[:-1], N)
@@ -358,7 +368,7 @@ def linear(x, weight, bias=None, act=ACT_NONE):
             # bucket by padded M so varying decode/prefill
             # batch sizes reuse one tuning decision
             key = ("dec", 128 if M <= 128 else 256, N, K,
-                   bias is not None)
+                   bias is not None) + (("mid",) if shares else ())
             choice = _GEMM_CHOICE.get(key)
             if choice is None:
                 import time as _t
@@ -378,6 +388,9 @@ def linear(x, weight, bias=None, act=ACT_NONE):
                     "decode": timeit(lambda: _hip_ops.decode_gemm(
                         x2, weight, bias, 0)),
                 }
+                if shares:
+                    times["mid"] = timeit(lambda: _hip_ops.mid_gemm(
+                        x2, weight, bias, shares, 0))
                 try:  # hipBLASLt with measured algo search (blt_gemm.cpp)
                     times["blt_fused"] = timeit(
                         lambda: _blt_fused_path(x2, weight, bias, act))
@@ -387,11 +400,13 @@ def linear(x, weight, bias=None, act=ACT_NONE):
                 _GEMM_CHOICE[key] = choice
             if choice == "decode":
                 out = _hip_ops.decode_gemm(x2, weight, bias, 0)
+            elif choice == "mid":
+                out = _hip_ops.mid_gemm(x2, weight, bias, shares, 0)
             elif choice == "blt_fused":
                 out = _blt_fused_path(x2, weight, bias, act)
             else:
                 out = torch.nn.functional.linear(x2, weight, bias)
-            if M <= 64 and _wide_logits(M, N, K):
+            if shares or (M <= 64 and _wide_logits(M, N, K)):
                 _WIDE_RUN.add((M, N, K, bias is not None))
             return out.reshape(*orig_shape[:-1], N)
         shapes_ok = (M % 256 == 0 and N % 256 == 0 and K % 64 == 0

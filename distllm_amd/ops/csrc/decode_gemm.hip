@@ -378,9 +378,11 @@ dg_tile_kernel(const u16* __restrict__ X, const u16* __restrict__ W,
                   : X + (long)min(m0 + row - 64, e.M - 1) * K) +
              ks * (K / splitk) + lc;
   }
-  // beyond 64 rows it is x that all read, and do so together: us from the first
-  // columns on and from different ones, 120 rows of 4096 x 14336 41.3 and 48.9, 100
-  // rows 39.9 and 42.2
+  // with more than 64 rows in a tile it is x that all read, and do so together: us
+  // from the first columns on and from different ones, 120 rows of 4096 x 14336 41.3
+  // and 48.9, 100 rows 39.9 and 42.2. Not so in blocks of 64 of more rows: 128 rows
+  // of 2048 x 8192 18.2 and 17.3, 66 rows 17.1 and 16.6, 128 of 4096 x 4096 17.2 and
+  // 16.8, 160 of 2048 x 4096 15.2 and 15.2
   const int turn = MP <= 64 ? chunk_turn<19>(cb, nt) : 0;
   auto issue = [&](int c) {
     char* dst = smem + (c % R) * STAGE + wid * LOADS * 1024 + lane * 16;
@@ -527,26 +529,28 @@ extern "C" bool decode_gemm_rings(int M, int N, int K) {
 
 // How many workgroups share K where 65 rows and more go by tiles of 64 x 64, 0
 // where another product is to be taken. Tiles have to fit the card twice over,
-// and the sums, 0.22 us for 64 of K and 4.5 for the launch that joins shares, have
-// to stay below what the library's product costs the host alone, 19 us a call
-// (this one 6): an encoder of some hundred rows issues its layers slower than it
-// runs them. Measured in a graph, us, library and this: 300 rows of 2304 x 768 6.8
-// and 6.0, 768 x 768 4.9 and 5.6, 3072 x 768 with GELU 10.0 and 6.5, 768 x 3072
-// (4 shares) 8.4 and 10.1, 1280 x 5120 (2) 16.7 and 15.2; 800 rows 8.6 and 8.3, 6.6
-// and 5.8, 14.7 and 12.8, 14.1 and 14.6; 2000 rows of 768 x 768 8.6 and 8.0. With
-// more tiles it is the slower one: 1300 rows of 2304 x 768 10.2 and 12.8, 800 of
-// 3840 x 1280 14.8 and 20.7.
+// and the time, 0.28 us for 64 of K (more with more than a tile a CU) and 4.5 for the
+// launch that joins shares, has to stay below what the library's product costs
+// either way: on the host alone 14 to 25 us a call (this one 6), and an encoder of
+// some hundred rows issues its layers slower than it runs them; in a graph, over
+// weights from memory, us, library (the faster of two calls) and this: 300 rows of
+// 2304 x 768 10.1 and 6.9, 768 x 768 7.8 and 6.1, 3072 x 768 with GELU 10.4 and 7.4,
+// 768 x 3072 (4 shares) 10.0 and 10.9, 1280 x 5120 (2) 19.6 and 17.6; 160 rows of
+// 6144 x 1024 12.7 and 9.9, of 1280 x 1280 8.4 and 8.7; 1000 rows of 1024 x 1024 11.4
+// and 7.9, of 768 x 3072 16.4 and 16.1. Where it is the slower one by both: 600 rows
+// of 3072 x 2048 16.8 and 19.2, 1000 of 2048 x 2048 17.3 and 19.7.
 extern "C" int mid_gemm_shares(int M, int N, int K) {
   if (M <= 64 || N <= 0 || N % 64 || K % 64 || K < 128) return 0;
   const long tiles = (long)((M + 63) / 64) * (N / 64);
   if (tiles > 512) return 0;
   if (K <= 1536) return 1;
   int best = 0;
-  float least = 16.f;
+  float least = 18.5f;
   for (int s = 1; s <= 4; s *= 2) {
     if (K % (64 * s) || (s > 1 && tiles * s > 256)) continue;
-    const float us = 2.5f + 0.22f * (K / 64 / s) * (tiles > 256 ? 1.5f : 1.f) +
-                     (s > 1 ? 4.5f : 0.f);
+    const float each = tiles > 256 ? std::max(1.5f, tiles / 256.f) : 1.f;
+    const float us =
+        2.5f + 0.28f * (K / 64 / s) * each + (s > 1 ? 4.5f : 0.f);
     if (us >= least) continue;
     least = us;
     best = s;

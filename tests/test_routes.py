@@ -152,6 +152,66 @@ def test_wide_logits_are_not_measured_in_a_capture(monkeypatch, choice):
     assert last(40) == "decode"
 
 
+def test_shares_of_k_are_one_of_the_measured_choices(monkeypatch):
+    """Blocks of 64 rows that share K: taken by the choice, and where a graph is
+    captured before the size ran, for they need no measurement."""
+    capturing, took = False, []
+
+    def ran(name):
+        def run(x, weight, *rest):
+            took.append(name)
+            return torch.empty(x.shape[0], weight.shape[0],
+                               dtype=torch.bfloat16)
+        return run
+
+    def synchronize():
+        assert not capturing
+
+    class Ops:
+        mid_gemm_shares = staticmethod(lambda M, N, K: int(M > 64) * 2)
+        wide_gemm_tile = staticmethod(lambda *sizes: 0)
+        decode_gemm = staticmethod(ran("decode"))
+        mid_gemm = staticmethod(ran("mid"))
+
+        def require(self, name):
+            pass
+
+    monkeypatch.setattr(ops, "_hip_ops", Ops())
+    monkeypatch.setattr(ops, "_own_product", lambda *a: True)
+    monkeypatch.setattr(ops, "_blt_fused_path", ran("blt_fused"))
+    monkeypatch.setattr(torch.nn.functional, "linear", ran("blaslt"))
+    monkeypatch.setattr(torch.cuda, "synchronize", synchronize)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing",
+                        lambda: capturing)
+    monkeypatch.setattr(ops, "_GEMM_CHOICE", {})
+    monkeypatch.setattr(ops, "_WIDE_RUN", set())
+    w = torch.empty(4096, 4096, dtype=torch.bfloat16).as_subclass(_Cuda)
+
+    def last(M, act=ops.ACT_NONE):
+        took.clear()
+        x = torch.zeros(M, 4096, dtype=torch.bfloat16).as_subclass(_Cuda)
+        assert ops.linear(x, w, None, act).shape == (M, 4096)
+        return took[-1]
+
+    capturing = True
+    assert last(80) == "mid" and not ops._GEMM_CHOICE
+    capturing = False
+    last(80)
+    assert {"mid", "decode", "blaslt", "blt_fused"} == set(took)
+    (key,) = ops._GEMM_CHOICE
+    for choice in ("decode", "blt_fused", "blaslt", "mid"):
+        ops._GEMM_CHOICE[key] = choice
+        assert last(80) == choice
+        capturing = True
+        assert last(80) == choice
+        assert last(100) == "mid"
+        capturing = False
+    ops._GEMM_CHOICE[key] = "decode"
+    assert last(80, ops.ACT_SILU) == last(300) == "mid"
+    monkeypatch.setenv("DISTLLM_GEMM", "decode")
+    assert last(200) == "decode"
+
+
 def test_many_rows_go_by_tiles_and_sums():
     """wide_gemm_tile: sizes that the kernel cannot take, rounds of the card's
     CUs, and what is followed stays with torch."""
@@ -179,6 +239,11 @@ def test_many_rows_go_by_tiles_and_sums():
         assert shares(*sizes) == 0
     assert shares(300, 2304, 768) == shares(2000, 768, 768) == 1
     assert shares(200, 768, 3072) == 4
+    # by both measures the slower ones, and some that are not
+    assert shares(600, 3072, 2048) == shares(1000, 2048, 2048) == 0
+    assert shares(600, 2048, 2048) == shares(1000, 768, 3072) == 1
+    assert shares(200, 1280, 5120) == shares(80, 4096, 4096) == 2
+    assert shares(80, 2048, 8192) == 4
     x = torch.zeros(2)
     p = torch.nn.Parameter(x)
     assert ops._recorded(p) and not ops._recorded(x, None)

@@ -244,6 +244,32 @@ def test_forms_that_are_asked_for(monkeypatch, mode, M, act):
     assert calls == (["decode_gemm"] if (mode, act) == ("decode", 0) else [])
 
 
+@pytest.mark.parametrize("M,N,K", [
+    (66, 4096, 4096), (128, 4096, 4096), (100, 2048, 8192), (256, 1280, 5120)])
+def test_shares_of_k_in_a_graph(M, N, K):
+    """As a captured step of so many sequences has them, 32 chunks of 64 of K
+    and more a share."""
+    x, w, b = _operands(M, N, K)
+    with torch.no_grad():
+        shares = ops._mid_shares(x, w, b)
+        assert shares > 1 and K // shares >= 2048
+        forms = [lambda: ops.linear(x, w, b),
+                 lambda: ops._hip_ops.mid_gemm(x, w, b, shares, 0)]
+        for run in forms:
+            want = run()
+            # of K terms in 32 bits, whose errors add up as steps at random
+            _check(want, _reference(x, w, b, 0))
+            torch.cuda.synchronize()
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph):
+                got = run()
+            for _ in range(3):
+                got.zero_()
+                graph.replay()
+                torch.cuda.synchronize()
+                assert torch.equal(got, want)
+
+
 def test_linear_under_autocast():
     """To half precision by torch, as ever; to bf16 it is the same product."""
     x, w, b = _operands(300, 768, 768)
