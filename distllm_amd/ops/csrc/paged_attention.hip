@@ -721,12 +721,21 @@ static void pa_launch(const void* q, long q_stride, const PaStep* step,
 // of 128, contexts of 16, of 200, of 200 to 2027: two tiles 30, 51, 211; one 20,
 // 40, 213 (two waves 12, 38, 217 to 226: the long ones wait for each other).
 // 64 x 8 heads, grouped: two 8.8, 16.9, 53; one 6.4, 14.6, 55. With heads of 64,
-// 64 x 32: four tiles 22, 38, 120; two 14, 24, 109.
+// 64 x 32: four tiles 22, 38, 120; two 14, 24, 109. A decode step's workgroups wait
+// longer, for their share and their rotated queries, so a second one is worth more:
+// us a layer, 8 key heads, two tiles and one, contexts of 16, of 200, of 100 to 500,
+// of 200 to 2048: 64 sequences 12.3, 22.0, 26.1, 60.2 and 8.9, 18.4, 24.3, 65.5; 66
+// 16.5, 28.2, 30.2, 66.1 and 12.2, 23.3, 24.6, 67.1 (three launches 15.2, 25.7, 27.0,
+// 67.8); 80 16.9, 29.1, 34.0, 79.3 and 12.6, 24.9, 30.8, 76.9; 112 21.7, 38.1, 45.0,
+// 105 and 15.0, 30.2, 37.9, 102. Of fp8 pages, which always have one, the step is the
+// slower one for many short contexts (128 of 200 25.4, three launches 23.0) and the
+// faster one for mixed ones (80 of 200 to 2048 43, 52).
 #define PA_D(DD, ST)                                                  \
   do {                                                                \
     if (fp8) PA(DD, true, true, 1, ST);                               \
     else if (!aligned) PA(DD, false, false, 1, ST);                   \
-    else if (DD == 128 && B * HKV * NG >= 1024) PA(DD, false, true, 1, ST);   \
+    else if (DD == 128 && B * HKV * NG >= (ST ? 513 : 1024))          \
+      PA(DD, false, true, 1, ST);                                     \
     else PA(DD, false, true, 2, ST);                                  \
   } while (0)
   if (step != nullptr) {

@@ -338,6 +338,28 @@ def test_step_rows_of_one_sequence(device, H, HKV, D, fp8, slabs):
     assert slots[:9, 6].tolist() == [1, 0, 0, 1, 1, 1, 0, 0, 0]
 
 
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("B,H,HKV", [(64, 32, 8), (65, 32, 8), (128, 32, 8),
+                                     (33, 32, 32)])
+def test_step_of_many_sequences(device, B, H, HKV, fp8):
+    """From 513 groups of heads on bf16 tiles have one place in a wave's ring;
+    lengths of a token to several tiles a wave, and rows without any."""
+    lens = [(1, 17, 32, 0, 33, 150, 300, 600)[i % 8] for i in range(B)]
+    qkv, cs, sn, ctx, raw, table, _ = _step(device, lens, H, HKV, 128, fp8, 38)
+    scale, two = 128 ** -0.5, [t.clone() for t in raw]
+    plan = ops.step_plan(1, ctx, H, raw[0], table)[0]
+    got = ops.step_attn(qkv, cs, sn, ctx, *raw, table, None, scale, plan)
+    has = ctx > 0
+    assert not got[~has].any()
+    some = [t[has].contiguous() for t in (qkv, ctx, table)]
+    q = ops.rope_put(some[0], cs, sn, some[1], *two, some[2])
+    want = ops.paged_attn(q, *two, some[2], some[1], scale)
+    assert not want.isnan().any()
+    torch.testing.assert_close(got[has].float(), want.float(), **TOL)
+    for a, b in zip(raw, two):
+        torch.testing.assert_close(a, b, atol=0, rtol=0, equal_nan=True)
+
+
 @pytest.mark.parametrize("B", [1, 5, 70, 1030])
 def test_plan_finds_rows_of_one_sequence(device, B):
     g = torch.Generator().manual_seed(B)
