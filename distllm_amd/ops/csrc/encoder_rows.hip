@@ -1,7 +1,7 @@
 // Products of an encoder's few rows (width H <= 1024) with what came ahead of
-// them in launches of their own: the norm of a sum (launch_norm_rows, M <= 32)
-// and the attention of short texts (launch_attn_rows, M <= 64). On so few rows a
-// launch is latency: 2.9 us a norm, 4.8 the attention of 24 tokens, and the
+// them in launches of their own: the norm of a sum (launch_norm_rows, M <= 32 or
+// 24) and the attention of short texts (launch_attn_rows, M <= 64). On so few rows
+// a launch is latency: 2.9 us a norm, 4.8 the attention of 24 tokens, and the
 // products 3 to 4. Here every workgroup norms, or attends, all rows again while
 // its weights are on their way; 16 columns of W are a workgroup: 24 KiB of
 // weights, and 74 KiB of rows to norm (24 x 768) or 110 KiB to attend, from L2.
@@ -391,11 +391,16 @@ constexpr int LDS_MOST = 160 * 1024;
 }  // namespace
 
 // Whether M rows of H numbers are normed by every workgroup. They fit up to 56
-// rows of 1024, but from 33 on that takes as long as a launch (768, 12 layers,
-// both ways: 48 rows 384 and 381 us, 64 rows 423 and 390).
+// rows of 1024, but every workgroup norms them all, and a launch of its own costs
+// the same whatever they are. From 25 rows on a wave has a second pair of rows;
+// 12 layers, own launches and joined, us: 24 rows of 512 273 and 229, 768 290 and
+// 261, 832 306 and 289, 896 311 and 294, 960 360 and 345, 1024 369 and 351; 25 rows
+// 512 275 and 246, 768 326 and 312, 832 334 and 337, 896 336 and 342, 1024 403 and
+// 404; 32 rows 768 333 and 320, 832 339 and 346, 960 415 and 417, 1024 415 and 419;
+// 48 rows of 768 381 and 384, 64 rows 390 and 423.
 extern "C" bool norm_rows_fit(int M, int H) {
-  return M >= 1 && M <= 32 && H % 64 == 0 && H >= 64 && H <= 1024 &&
-         rows_lds(M, H, 0) <= LDS_MOST;
+  return M >= 1 && M <= (H <= 768 ? 32 : 24) && H % 64 == 0 && H >= 64 &&
+         H <= 1024 && rows_lds(M, H, 0) <= LDS_MOST;
 }
 
 // Whether the attention fits the twelve waves in at most two turns, and LDS
@@ -418,22 +423,18 @@ extern "C" void launch_norm_rows(const void* y, const void* res, const void* w,
   hipLaunchKernelGGL((norm_rows_kernel<A, MT, NC, P>), dim3(N / COLS),      \
                      dim3(NW * 64), rows_lds(M, H, 0), stream, n,       \
                      (const u16*)W, H, e)
-#define NR_M(A, NC)                                                         \
-  do {                                                                      \
-    if (M <= 16) NR(A, 1, NC, 1);                                           \
-    else if (M <= 24) NR(A, 2, NC, 1);                                      \
-    else NR(A, 2, NC, 2);                                                   \
-  } while (0)
 #define NR_A(A)                                                             \
   do {                                                                      \
-    if (H <= 768) NR_M(A, 3);                                               \
-    else NR_M(A, 4);                                                        \
+    if (H > 768 && M <= 16) NR(A, 1, 4, 1);                                 \
+    else if (H > 768) NR(A, 2, 4, 1);                                       \
+    else if (M <= 16) NR(A, 1, 3, 1);                                       \
+    else if (M <= 24) NR(A, 2, 3, 1);                                       \
+    else NR(A, 2, 3, 2);                                                    \
   } while (0)
   if (act == 6) NR_A(6);
   else if (act == 7) NR_A(7);
   else NR_A(0);
 #undef NR_A
-#undef NR_M
 #undef NR
 }
 

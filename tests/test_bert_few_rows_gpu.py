@@ -78,6 +78,16 @@ def test_joined_launches(device, B, S, H, heads, ff):
     assert torch.equal(m(ids, mask.int()), _layers(m, ids, mask.int()))
 
 
+@pytest.mark.parametrize("S", [16, 24, 25, 32])
+@pytest.mark.parametrize("H,heads", [(768, 12), (832, 13), (1024, 16)])
+def test_norms_on_both_sides_of_their_bound(device, S, H, heads):
+    """Joined with a product up to 32 rows of 768, 24 of more."""
+    m = _model(device, H, heads, 256)
+    ids = torch.randint(0, 300, (1, S), device=device)
+    mask = torch.ones_like(ids)
+    assert torch.equal(m(ids, mask), _layers(m, ids, mask))
+
+
 def test_stands_back(device):
     m = _model(device)
     ids = torch.randint(0, 300, (1, 20), device=device)
