@@ -401,10 +401,17 @@ static int wg_tile(int M, int N, long* tiles) {
 // launch), own time over its, in a graph, over weights that come from memory:
 // - A single round, by the share of the card's 256 tiles of 256 rows that its tiles
 //   make: without activation and K of 1536 and more 0.58 to 0.9 0.75 to 1.02, 0.5 to
-//   0.55 1.04 to 1.08, below 1.1 to 1.4; a gated unit of long rows 0.54 and more 0.83
-//   to 1.0, 0.44 1.02 to 1.23. Shorter sums: without activation 216 tiles and more
-//   0.79 to 1.0, 120 to 200 1.0 to 1.23, fewer up to 3; with one 96 tiles and more
-//   0.7 to 0.92, 60 1.02.
+//   0.55 1.04 to 1.08, below 1.1 to 1.9; a gated unit of K from 4096 on 0.54 and more
+//   0.83 to 1.0, 0.44 1.02 to 1.23; with either and K of 1536 to 2048 0.43 and more
+//   0.75 to 1.03, 0.38 1.0 to 1.09, 0.19 to 0.31 1.07 to 1.39. Shorter sums: without
+//   activation 216 tiles and more 0.52 to 1.03, 120 to 192 0.67 to 1.24, fewer up to
+//   1.55; with one, K to 1024, 96 tiles and more 0.5 to 1.09, K of 1280 to 1472 96 to
+//   160 tiles 1.05 to 1.36, 176 to 192 0.95 to 1.1, more below that. Those 96 to 192
+//   are taken for the host, which two or three calls cost 21 to 30 us and this one 6:
+//   issued one after the other 0.78 to 1.0 (K of 1536 0.98 to 1.1), and an encoder
+//   of 650 M weights on 700 to 1300 tokens 4840 and 4120 us.
+// - Several rounds that fill less than half of the card without an activation: K of
+//   1024 and more 1.08 to 1.1.
 // - Long sums whose 256 x 256 tiles fill their rounds, which is the library's
 //   best case: K of 1536 and more, a share of 0.87 and more 1.01 to 1.09, below
 //   0.73 to 0.99. With K to 1280 0.86 to 1.0 all the same, and with an
@@ -418,12 +425,17 @@ extern "C" int wide_gemm_tile(int M, int N, int K, int act) {
   const long ntn = N / 256;
   if (tiles * ntn * WG_GROUP >= 1L << 32)
     return 0;  // divisions by multiplication
+  const long filled = tiles * fm;  // 2048 are a round of 256 tiles of 256 rows
   if (tiles <= 256) {
-    if (K >= 1536 && !(act != WG_NONE && K == 1536)) {
-      if (tiles * fm < (act == WG_NONE ? 0.58f : 0.5f) * 2048) return 0;
-    } else if (tiles < (act != WG_NONE ? 96 : 208)) {
+    if (K < 1536) {
+      if (tiles < (act != WG_NONE ? 96 : 208)) return 0;
+    } else if (filled <
+               (act == WG_NONE ? 0.58f : K <= 2048 ? 0.43f : 0.5f) * 2048) {
       return 0;
     }
+  } else if (act == WG_NONE && K >= 1024 &&
+             filled < ((tiles + 7) / 8 + 31) / 32 * 1024) {
+    return 0;
   }
   if (act == WG_NONE && K >= 1536) {
     const long most = (long)((M + 255) / 256) * ntn;

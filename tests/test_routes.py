@@ -231,6 +231,16 @@ def test_many_rows_go_by_tiles_and_sums():
     assert tile(1500, 4096, 4096, 0) == tile(1025, 6144, 4096, 0) == 0
     assert tile(200, 28672, 4096, 4) == tile(1500, 3840, 1280, 0) == 0
     assert tile(300, 28672, 4096, 4) == 5 and tile(1025, 28672, 4096, 4) == 6
+    # K of 1536 and more by the share of the card, shorter ones by tiles
+    for act in (1, 2, 3, 4, 5):
+        assert tile(700, 4096, 1472, act) == 4  # 96 tiles of 128 rows
+        assert tile(700, 4096, 1536, act) == tile(1500, 4096, 1536, act) == 0
+        assert tile(1700, 4096, 1536, act) == tile(1700, 4096, 2048, act) == 4
+        assert tile(1700, 4096, 2112, act) == 0
+        assert tile(2600, 6144, 4096, act) == 4
+    # two rounds of tiles of 128 rows
+    assert tile(2600, 6144, 1024, 0) == tile(2600, 6144, 4096, 0) == 0
+    assert tile(2600, 6144, 960, 0) == 4
     assert tile(3000, 4096, 4096, 0) == 6 and tile(12992, 768, 3072, 0) == 5
     shares = ops._hip_ops.mid_gemm_shares
     for sizes in [(64, 768, 768), (300, 760, 768), (300, 768, 760),
