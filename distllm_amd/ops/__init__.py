@@ -849,6 +849,13 @@ def topk(scores, k, chunk=1 << 15):
     return torch_ref.topk(scores, min(k, scores.shape[1]))
 
 
+def found_lists(v, i):
+    """Scores and indices [Q, k] on a GPU (float32, int32) as lists of their
+    rows, without the entries whose index is negative."""
+    _require_hip()
+    return _hip_ops.found_lists(v, i)
+
+
 def hamming_score(qcodes, codes_t):
     if qcodes.is_cuda:
         _require_hip()

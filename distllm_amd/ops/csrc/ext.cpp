@@ -787,6 +787,49 @@ c10::optional<torch::Tensor> bert_few_rows(torch::Tensor x,
                                            int64_t heads, double eps,
                                            int64_t act);
 
+// Scores and indices [Q, k] of a search as lists of their rows, without the
+// entries whose index is negative. One copy to the host (25 us whatever it holds)
+// of both, joined on the way if they do not lie one behind the other. As steps of
+// Python this took a first call on a new question, which finds the host's caches
+// full of other things, 60 us longer than two copies.
+static std::pair<py::list, py::list> found_lists(torch::Tensor v,
+                                                 torch::Tensor i) {
+  CHECK_DEV(v); CHECK_F32(v);
+  CHECK_DEV(i); CHECK_I32(i);
+  TORCH_CHECK(v.dim() == 2 && v.sizes() == i.sizes() &&
+                  v.device() == i.device(),
+              "scores and indices must be [Q, k]");
+  const int64_t Q = v.size(0), k = v.size(1), n = Q * k;
+  torch::Tensor host;
+  {
+    py::gil_scoped_release others;
+    const c10::DeviceGuard guard(v.device());
+    const bool lie = v.is_contiguous() && i.is_contiguous() &&
+                     i.is_alias_of(v) &&
+                     i.storage_offset() == v.storage_offset() + n;
+    host = (lie ? torch::as_strided(i, {2, Q, k}, {n, k, 1},
+                                    v.storage_offset())
+                : torch::stack({v.contiguous().view(at::kInt), i}))
+               .cpu();
+  }
+  const int* indices = host.data_ptr<int>() + n;
+  const float* scores = reinterpret_cast<const float*>(host.data_ptr<int>());
+  py::list all_scores(Q), all_indices(Q);
+  for (int64_t q = 0; q < Q; ++q, scores += k, indices += k) {
+    const int64_t kept =
+        k - std::count_if(indices, indices + k, [](int x) { return x < 0; });
+    py::list s(kept), x(kept);
+    for (int64_t j = 0, to = 0; j < k; ++j) {
+      if (indices[j] < 0) continue;
+      s[to] = py::float_(scores[j]);
+      x[to++] = py::int_(indices[j]);
+    }
+    all_scores[q] = std::move(s);
+    all_indices[q] = std::move(x);
+  }
+  return {all_scores, all_indices};
+}
+
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("norm_fwd", &norm_fwd, "fused residual+LayerNorm/RMSNorm");
   m.def("bias_gelu", &bias_gelu);
@@ -826,6 +869,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("block_table"), py::arg("bias"), py::arg("scale"),
         py::arg("slots"), py::arg("arrived"), py::arg("ahead") = py::none());
   m.def("step_plan", &step_plan);
+  m.def("found_lists", &found_lists);
   m.def("rope_put", &rope_put, py::arg("qkv"), py::arg("cs"), py::arg("sn"),
         py::arg("ctx"), py::arg("kcache"), py::arg("vcache"),
         py::arg("block_table"), py::arg("bias") = py::none());

@@ -367,20 +367,21 @@ class HipFlatIndex:
             v, i = self._topk_ivf(q, top_k)
         else:
             v, i = self._topk_exact(q, top_k)
-        # scores and indices in one copy: it costs 25 us whatever it holds
-        both = _one_tensor(v.float().view(torch.int32), i.int()).cpu().numpy()
-        scores, indices = both[0].view(np.float32), both[1]
-        print(f"Search time: {time.perf_counter() - t0:.6f} seconds")
         # IVF pads short candidate lists with index -1 / score -inf;
         # drop those unconditionally (not only under score_threshold) so
-        # -1 never reaches get()/dataset indexing as "last row". Lists without
-        # any are taken as they are (256 by 10 of them: 240 us entry by entry).
-        keep = indices >= 0
-        if keep.all():
-            vv, ii = scores.tolist(), indices.tolist()
+        # -1 never reaches get()/dataset indexing as "last row".
+        if v.is_cuda:
+            vv, ii = ops.found_lists(v.float(), i.int())
         else:
-            vv = [s[k].tolist() for s, k in zip(scores, keep)]
-            ii = [x[k].tolist() for x, k in zip(indices, keep)]
+            both = _one_tensor(v.float().view(torch.int32), i.int()).numpy()
+            scores, indices = both[0].view(np.float32), both[1]
+            keep = indices >= 0
+            if keep.all():
+                vv, ii = scores.tolist(), indices.tolist()
+            else:
+                vv = [s[k].tolist() for s, k in zip(scores, keep)]
+                ii = [x[k].tolist() for x, k in zip(indices, keep)]
+        print(f"Search time: {time.perf_counter() - t0:.6f} seconds")
         results = BatchedSearchResults(total_scores=vv, total_indices=ii)
         return self._filter_search_by_score(results, score_threshold)
 

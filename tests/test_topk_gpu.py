@@ -89,3 +89,41 @@ def test_many_equal_scores_by_place(device, N, k):
     for _ in range(3):
         _, i = ops.topk(s, k)
         assert torch.equal(i.cpu().long(), want)
+
+
+def _lists(v, i):
+    v, i = v.cpu(), i.cpu()
+    keep = [row >= 0 for row in i]
+    return ([s[k].tolist() for s, k in zip(v, keep)],
+            [x[k].tolist() for x, k in zip(i, keep)])
+
+
+@pytest.mark.parametrize("Q,k", [(0, 3), (1, 0), (1, 5), (256, 10), (3, 1000)])
+@pytest.mark.parametrize("form", ["topk", "apart", "swapped", "strided"])
+def test_found_lists(device, Q, k, form):
+    """However scores and indices lie, with entries that are none."""
+    g = torch.Generator(device=device).manual_seed(Q + k)
+    both = torch.empty(2, Q, k, dtype=torch.int32, device=device)
+    if form == "strided":
+        both = torch.empty(2, Q, 2 * k, dtype=torch.int32,
+                           device=device)[:, :, ::2]
+    v, i = both[0].view(torch.float32), both[1]
+    if form == "apart":
+        i = torch.empty_like(i)
+    if form == "swapped":
+        v, i = both[1].view(torch.float32), both[0]
+    v.copy_(torch.randn(Q, k, device=device, generator=g))
+    i.copy_(torch.randint(-2, 9, (Q, k), device=device, generator=g))
+    if Q > 1:
+        i[0] = -1
+        i[1] = 7
+        v[1, 0] = float("inf")
+        v[1, -1] = float("-inf")
+    want = _lists(v, i)
+    got = ops.found_lists(v, i)
+    assert got == want
+    assert all(type(x) is int for row in got[1] for x in row)
+    assert all(type(x) is float for row in got[0] for x in row)
+    if form == "topk" and k:
+        found = ops.topk(torch.randn(max(Q, 1), 5000, device=device), k)
+        assert ops.found_lists(*found) == _lists(*found)
