@@ -821,8 +821,8 @@ static std::pair<py::list, py::list> found_lists(torch::Tensor v,
     py::list s(kept), x(kept);
     for (int64_t j = 0, to = 0; j < k; ++j) {
       if (indices[j] < 0) continue;
-      s[to] = py::float_(scores[j]);
-      x[to++] = py::int_(indices[j]);
+      PyList_SET_ITEM(s.ptr(), to, py::float_(scores[j]).release().ptr());
+      PyList_SET_ITEM(x.ptr(), to++, py::int_(indices[j]).release().ptr());
     }
     all_scores[q] = std::move(s);
     all_indices[q] = std::move(x);
