@@ -431,3 +431,25 @@ def test_step_fetches_ahead(device, shape, dtype, step):
                                   plan, ahead))
     assert torch.equal(*outs)
     assert bool((w == 1).all())
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("lens", [[1], [5, 0, 2], [1] * 8])
+@pytest.mark.parametrize("shape,dtype", [
+    ((128, 64), torch.uint8),     # eight runs of one piece, the fewest
+    ((213, 64), torch.uint8),     # thirteen, and rows that are no run
+    ((136, 64), torch.bfloat16), ((400, 192), torch.bfloat16),
+    ((4099, 2048), torch.bfloat16)])
+def test_step_fetches_ahead_of_short_contexts(device, lens, shape, dtype, fp8):
+    """Where the pages are less than the weights, so that these are fetched."""
+    qkv, cs, sn, ctx, raw, table, _ = _step(device, lens, 4, 1, 64, fp8, 4)
+    w = torch.ones(shape, device=device).to(dtype)
+    runs = shape[0] // 16 * 16 * shape[1] * w.element_size()
+    assert sum(lens) * 64 * (2 if fp8 else 4) <= runs
+    outs = []
+    for ahead in (None, w):
+        plan = ops.step_plan(1, ctx, 4, raw[0], table)[0]
+        outs.append(ops.step_attn(qkv, cs, sn, ctx, *raw, table, None, 0.1,
+                                  plan, ahead))
+    assert torch.equal(*outs) and not outs[0].isnan().any()
+    assert bool((w == 1).all())

@@ -57,6 +57,20 @@ def test_tiles(tile, M, N, K):
     _check(ops._hip_ops.wide_gemm(x, w, b, 0, tile), _reference(x, w, b, 0))
 
 
+@pytest.mark.parametrize("tile", [4, 6, 8])
+@pytest.mark.parametrize("M,N,K,act", [
+    (1100, 512, 4096, 0), (300, 512, 14336, 0), (2100, 4096, 4096, 0),
+    (1100, 1024, 4096, 4), (300, 512, 14336, 2)])
+def test_long_sums(tile, M, N, K, act):
+    """K of a decoder's products, with one round of tiles and several. Errors
+    of the terms' sums are as steps at random, sqrt(K) 2^-24 of 4 or so: 3e-5."""
+    x, w, b = _operands(M, N, K)
+    got = ops._hip_ops.wide_gemm(x, w, b, act, tile)
+    want = _reference(x, w, b, act)
+    bound = want.abs() * 2.0 ** -8 + 6e-5 * (1 + want.abs().amax())
+    assert ((got.double() - want).abs() <= bound).all()
+
+
 @pytest.mark.parametrize("act", [1, 2, 3, 4, 5])
 @pytest.mark.parametrize("bias", [False, True])
 @pytest.mark.parametrize("M,tile", [(70, 8), (4099, 6)])
@@ -280,6 +294,41 @@ def test_linear_under_autocast():
         want = ops.linear(x, w, b)
         with torch.autocast("cuda", dtype=torch.bfloat16):
             assert torch.equal(ops.linear(x, w, b), want)
+
+
+@pytest.mark.parametrize("B", [66, 128])
+def test_captured_step_of_some_hundred_sequences(B, monkeypatch):
+    """A decoder's step, whose products of short K go by blocks of 64 rows and
+    whose last one, of a long K, by the choice that the first run measured."""
+    from distllm_amd.models import ModelDims, build_model
+
+    calls = []
+    own = ops._hip_ops.mid_gemm
+    monkeypatch.setattr(ops._hip_ops, "mid_gemm",
+                        lambda *a: calls.append(a[0].shape[1]) or own(*a),
+                        raising=False)
+    monkeypatch.setattr(ops, "_GEMM_CHOICE", {})
+    torch.manual_seed(B)
+    m = build_model(ModelDims(
+        arch="llama", vocab_size=512, hidden_size=512, num_layers=2,
+        num_heads=8, num_kv_heads=2, intermediate_size=4096,
+        max_position_embeddings=256), device="cuda")
+    cache = m.make_cache(4 * B + 1, 16, "bf16")
+    table = torch.randperm(4 * B, device="cuda").int().view(B, 4) + 1
+    ctx = torch.randint(1, 65, (B,), device="cuda").int()
+    tokens = torch.randint(0, 512, (B,), device="cuda")
+    want = m.decode_step(tokens, cache, table, ctx)
+    assert 512 in calls and 4096 in calls
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = m.decode_step(tokens, cache, table, ctx)
+    for _ in range(3):
+        got.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)
+        m.decode_step(tokens, cache, table, ctx)
 
 
 def test_in_a_graph():
