@@ -26,6 +26,9 @@
 //    has no infinities.
 //  - NS workgroups share a sequence where B * HKV is small; a second launch
 //    joins them or, in a decode step, the last of them.
+//  - a decode step goes by the STEP form alone (launch_step_attn). launch_paged_attn
+//    and launch_rope_put are what ops.paged_attn and ops.rope_put have for callers
+//    that attend by themselves; no model of this package does.
 //  - a decode step's queries are rotated and its key and value put into the
 //    cache in the same launch (STEP): us in a graph, three launches and one,
 //    32 heads on 8, B = 1, 2048 tokens 12.7 -> 7.6, 64 tokens 10.9 -> 6.3, B = 8
@@ -38,8 +41,9 @@
 // 150 -> 98, 5.3 TB/s (96 -> 56). With copies that the compiler knows of, which
 // the reads of V then wait for, also for the next tile's: 39, 65 and 101.
 // Those kernels are still the faster ones where contexts of a page or two meet
-// 16 key heads and rows or more (64 x 32 heads of 128, of 16: 11, now 19), for
-// which the lengths, on the device only, would have to be known ahead.
+// 16 key heads and rows or more (64 x 32 heads of 128, of 16: 11, now 19): which
+// kernel runs is the host's choice, and the lengths are on the device only (where
+// step_plan_kernel deals a step's shares by them).
 #include "ahead.h"
 #include "common.h"
 #include <hip/hip_fp8.h>
@@ -804,8 +808,9 @@ extern "C" void launch_step_attn(const void* qkv, const float* parts, int S,
 // 32.9 -> 30.7 (23 -> 20.5), 42 46.4 -> 36.2 (38.5 -> 23.6), 64 60.5 -> 51.1 (37.4
 // -> 33.7); lengths all alike take what they took. One launch per step, 5 us, which
 // clears the counters of all layers too, as one did before.
-// Shares have 4 tiles or more, one for each wave, a sequence 32 shares or less.
-// asked > 0: that many for each.
+// A sequence is cut at 4 tiles or more, one for each wave, into 32 shares or less;
+// the shares are then made even, so that n of them have more than 4 (n - 1) tiles (5
+// tiles are shares of 3 and 2). asked > 0: that many for each.
 __host__ __device__ constexpr bool plan_many(int B, int p) {
   return B > p - p / 8;
 }
