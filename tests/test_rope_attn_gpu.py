@@ -93,3 +93,24 @@ def test_general(D):
         out = ops.rope_attn_(qkv, cs, sn, pos, H, HKV, causal=True)
         flat = keep
         _same(out, want)
+
+
+@pytest.mark.parametrize("S", [32, 300, 1000])
+@pytest.mark.parametrize("H,HKV,D", [(6, 6, 64), (8, 2, 128)])
+def test_bits(S, H, HKV, D):
+    """The queries that attention rotates are those of the launch that rotates keys,
+    bit for bit: no output depends on which of them a call took."""
+    qkv = _qkv(3, S, H + 2 * HKV, D)
+    cs, sn = _tables(D)
+    pos = _positions(3 * S)
+    turned = ops.rope_qk_(qkv.clone(), cs, sn, pos, H + HKV)
+    want = ops.attn_fwd(turned[:, :, :H], turned[:, :, H: H + HKV],
+                        turned[:, :, H + HKV:], causal=True)
+    assert torch.equal(want, ops.rope_attn_(qkv.clone(), cs, sn, pos, H, HKV,
+                                            causal=True))
+    cu = torch.tensor([0, S, 3 * S], device="cuda", dtype=torch.int32)
+    flat = turned.view(3 * S, H + 2 * HKV, D)
+    want = ops.attn_varlen(flat[:, :H], flat[:, H: H + HKV],
+                           flat[:, H + HKV:], cu)
+    assert torch.equal(want, ops.rope_attn_varlen_(
+        qkv.view(flat.shape).clone(), cs, sn, pos, H, HKV, cu))
