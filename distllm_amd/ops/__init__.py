@@ -863,8 +863,8 @@ def score(q, corpus):
 
     From 33 queries on, and where its tiles fill the card (_score_fills), the
     product of score.hip; else the library's. Measured against 250000 rows of
-    768, us, library and own: 32 queries 168, 171; 64 214, 186; 128 399, 221;
-    256 722, 316."""
+    768, us, library and own: 32 queries 168, 171; 64 214, 190; 128 399, 293;
+    256 722, 489."""
     Q, K = q.shape
     N = corpus.shape[0]
     if (q.is_cuda and q.device == corpus.device and 32 < Q < 1 << 20
@@ -924,7 +924,8 @@ def score_topk(q, corpus, k):
     For 33 and more queries and k to 60 without the matrix of scores, where
     _score_topk_fills: the largest score of every four rows, the k best of these
     fours, and their rows once more in float32. 250000 rows of 768, k = 10, us,
-    with the matrix and without: 64 queries 211, 197; 128 333, 234; 256 565, 339."""
+    with the matrix and without: 64 queries 211, 202; 128 333, 228; 256 565, 333
+    (833 where f16 parts do not do and the tiles are made again, see score.hip)."""
     Q, K = q.shape
     N = corpus.shape[0]
     if (0 < Q <= 4 and 0 < k <= min(30, N) and q.is_cuda

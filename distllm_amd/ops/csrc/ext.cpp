@@ -39,11 +39,14 @@ void launch_attn_varlen(const void*, const void*, const void*, void*,
                         const float*, const int*, hipStream_t);
 void launch_rope(const void*, void*, const float*, const float*, const int*,
                  long, int, int, int, hipStream_t);
-long score_bytes(int, int);
+long score_bytes(int, int, bool);
 void launch_score(const float*, void*, const float*, void*, bool, int, int, int,
-                  hipStream_t);
+                  const float**, int**, hipStream_t);
+void launch_score_again(const float*, const void*, const float*, void*,
+                        const int*, int, int, int, hipStream_t);
 void launch_search_top(const unsigned int*, const float*, const float*, float*,
-                       int*, int, int, int, int, int, hipStream_t);
+                       int*, int, int, int, int, int, const float*, int*, bool,
+                       hipStream_t);
 int search_few_groups(int);
 void launch_search_few(const float*, const float*, float*, int*, int, int, int,
                        int, hipStream_t);
@@ -429,11 +432,13 @@ torch::Tensor score(torch::Tensor q, torch::Tensor corpus) {
   const long Q = q.size(0), K = q.size(1), N = corpus.size(0);
   auto out = torch::empty({Q, N}, q.options());
   if (out.numel() == 0) return out;
-  auto planes = torch::empty({score_bytes((int)Q, (int)K)},
+  auto planes = torch::empty({score_bytes((int)Q, (int)K, true)},
                              q.options().dtype(at::kByte));
+  const float* lost;
+  int* again;
   launch_score(q.data_ptr<float>(), planes.data_ptr(),
                corpus.data_ptr<float>(), out.data_ptr(), true, (int)Q, (int)N,
-               (int)K, cur_stream());
+               (int)K, &lost, &again, cur_stream());
   return out;
 }
 
@@ -451,14 +456,23 @@ std::vector<torch::Tensor> score_topk(torch::Tensor q, torch::Tensor corpus,
   auto both = torch::empty({2, Q, k}, words);
   auto ov = both.select(0, 0).view(at::kFloat), oi = both.select(0, 1);
   auto* at = reinterpret_cast<unsigned int*>(most.data_ptr<int>());
-  auto planes = torch::empty({score_bytes((int)Q, (int)K)},
+  auto planes = torch::empty({score_bytes((int)Q, (int)K, false)},
                              q.options().dtype(at::kByte));
-  launch_score(q.data_ptr<float>(), planes.data_ptr(),
-               corpus.data_ptr<float>(), at, false, (int)Q, (int)N, (int)K,
-               cur_stream());
-  launch_search_top(at, q.data_ptr<float>(), corpus.data_ptr<float>(),
-                    ov.data_ptr<float>(), oi.data_ptr<int>(), (int)Q, (int)N,
-                    (int)groups, (int)K, (int)k, cur_stream());
+  const float *qp = q.data_ptr<float>(), *cp = corpus.data_ptr<float>(), *lost;
+  int* again;
+  launch_score(qp, planes.data_ptr(), cp, at, false, (int)Q, (int)N, (int)K,
+               &lost, &again, cur_stream());
+  auto top = [&](bool second) {
+    launch_search_top(at, qp, cp, ov.data_ptr<float>(), oi.data_ptr<int>(),
+                      (int)Q, (int)N, (int)groups, (int)K, (int)k, lost, again,
+                      second, cur_stream());
+  };
+  top(false);
+  if (again) {
+    launch_score_again(qp, planes.data_ptr(), cp, at, again, (int)Q, (int)N,
+                       (int)K, cur_stream());
+    top(true);
+  }
   return {ov, oi};
 }
 

@@ -566,6 +566,10 @@ extern "C" void launch_search_few(const float* q, const float* corpus,
 // float32, so the groups' numbers need only be near: a row that is left out for a
 // group's is within their error of it. Equals go by place, groups as rows. A
 // workgroup per query; k <= 60.
+// lost and again, null where the groups' numbers have float32's error: lost[q] is what
+// those of query q may be off beyond that (score_scale_kernel). Where it is more than
+// 2^-22 of the k-th largest, again[q] is set to 1, and the groups made again and chosen
+// from by a second launch (`second`: of such queries only).
 // The k-th largest of 64 sixteens of threads bounds the k-th largest group from
 // below, as in topk_regs_kernel; likewise, more than the buffer holds are selected
 // byte by byte.
@@ -578,13 +582,16 @@ __global__ void __launch_bounds__(ST_THREADS)
 search_top_kernel(const unsigned int* __restrict__ most,
                   const float* __restrict__ q,
                   const float* __restrict__ corpus, float* __restrict__ out_v,
-                  int* __restrict__ out_i, int N, int groups, int K, int k) {
+                  int* __restrict__ out_i, int N, int groups, int K, int k,
+                  const float* __restrict__ lost, int* __restrict__ again,
+                  bool second) {
   __shared__ unsigned int top[16][64], hist[256], thresh, ncand, found, above,
       counts[16];
   __shared__ unsigned long long key[ST_CAP];
   __shared__ int chosen[64];
   __shared__ unsigned long long rows[256];
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  if (second && again[blockIdx.x] == 0) return;
   const unsigned int* row = most + (long)blockIdx.x * groups;
 
   // f(number, place) for all groups of this thread
@@ -679,6 +686,11 @@ search_top_kernel(const unsigned int* __restrict__ most,
 #pragma unroll 8
     for (int j = 0; j < n; ++j) r += key[j] > own;
     if (r < take) chosen[r] = (int)~(unsigned int)own;
+    // (fewer groups than k have all rows)
+    if (r == k - 1 && lost != nullptr && !second &&
+        !(lost[blockIdx.x] <=
+          0x1p-22f * fabsf(ord_to_f32((unsigned int)(own >> 32)))))
+      again[blockIdx.x] = 1;
   }
   __syncthreads();
   const float* query = q + (long)blockIdx.x * K;
@@ -721,9 +733,11 @@ search_top_kernel(const unsigned int* __restrict__ most,
 extern "C" void launch_search_top(const unsigned int* most, const float* q,
                                   const float* corpus, float* out_v,
                                   int* out_i, int Q, int N, int groups, int K,
-                                  int k, hipStream_t stream) {
+                                  int k, const float* lost, int* again,
+                                  bool second, hipStream_t stream) {
   hipLaunchKernelGGL(search_top_kernel, dim3(Q), dim3(ST_THREADS), 0, stream,
-                     most, q, corpus, out_v, out_i, N, groups, K, k);
+                     most, q, corpus, out_v, out_i, N, groups, K, k, lost, again,
+                     second);
 }
 
 extern "C" void launch_topk_chunk(const float* scores, const int* in_idx,

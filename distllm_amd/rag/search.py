@@ -314,10 +314,11 @@ class HipFlatIndex:
 
     def _topk_exact(self, q: torch.Tensor, k: int):
         """Chunked scores + HIP top-k over the fp32 corpus. Scores keep
-        fp32 exactness (faiss parity): for batches of queries score.hip's
-        products of parts choose rows that are scored again in fp32, up to
-        four are multiplied where their rows are chosen, others by the
-        library's fp32 product."""
+        fp32 exactness (faiss parity). For batches of queries products of
+        score.hip's parts choose up to 60 rows, which are scored again in
+        fp32; of more rows the scores are its sums of three bf16 parts, all
+        24 bits of each number. Up to four queries are multiplied in fp32
+        where their rows are chosen, others by the library's product."""
         N = self.n
         k = min(k, N)
         chunk = self.score_chunk_rows

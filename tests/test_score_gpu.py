@@ -42,6 +42,15 @@ def test_all_bits(device):
     assert torch.equal(out, c.t())
 
 
+@pytest.mark.parametrize("K", [256, 288])
+def test_all_bits_of_small_numbers(device, K):
+    """As test_all_bits, beside numbers of other sizes in the same row."""
+    c = torch.randn(300, K, device="cuda") * torch.logspace(
+        0, -20, K, device="cuda")
+    out = _hip_ops.score(torch.eye(K, device="cuda"), c)
+    assert torch.equal(out, c.t())
+
+
 def test_not_finite(device):
     """Infinities, NaN and numbers that bf16 rounds to infinity come out as
     from float32 sums."""

@@ -56,6 +56,25 @@ def test_ranges(device, Q, form):
     _check(q, c, 10)
 
 
+@pytest.mark.parametrize("Q, N, K", [(100, 30001, 288), (256, 40000, 256),
+                                     (520, 20000, 320)])
+@pytest.mark.parametrize("small", [1e-3, 1e-6, 1e-9, 1e-11, 1e-13])
+@pytest.mark.parametrize("form", ["corpus", "queries", "some"])
+def test_wide_range(device, Q, N, K, small, form):
+    """A number in every row of the corpus beside which the others, which decide, are
+    small, and which the queries do not weigh; the other way round; queries that do
+    among those that do not."""
+    q, c = _unit(Q, K, 1), _unit(N, K, 2)
+    wide, other = (q, c) if form == "queries" else (c, q)
+    wide *= small
+    wide[:, 0] = 1
+    if form == "some":
+        other[::3, 0] = 0
+    else:
+        other[:, 0] = 0
+    _check(q, c, 10)
+
+
 @pytest.mark.parametrize("Q", [64, 70, 200])
 def test_equal_scores_by_place(device, Q):
     """Rows that occur several times; a query of zeros, for which more groups are
