@@ -109,3 +109,15 @@ def test_refusals(device):
             _hip_ops.score_topk(q, c, k)
     v, i = ops.score_topk(q, c, 55)
     assert v.shape == (40, 55) and (i[:, 50:] == -1).all()
+
+
+def test_place_of_a_query(device):
+    """What a query finds does not depend on its place in the batch, with rows beyond
+    f16 parts in one share of the corpus (every tile of queries looks at all of it)."""
+    q, c = _unit(256, 256, 9), _unit(40000, 256, 10)
+    c[:10000] *= 1e3
+    v, i = _hip_ops.score_topk(q.repeat(4, 1), c, 10)
+    for at in (256, 512, 768):
+        assert torch.equal(v[at: at + 256], v[:256])
+        assert torch.equal(i[at: at + 256], i[:256])
+    _check(q, c, 10)
