@@ -612,7 +612,7 @@ class _GraphRunner:
         # pinned, so that the copy has its turn on the stream and nothing waits
         # for it; the allocator keeps the memory until it is through
         host = torch.empty(self.inputs.shape, dtype=torch.int32,
-                           pin_memory=True)
+                           device="cpu", pin_memory=True)
         ops.step_inputs(self._views(host), tokens, lengths, slots, blocks)
         self.inputs.copy_(host, non_blocking=True)
 

@@ -167,3 +167,20 @@ def test_qwen2_engine_greedy_gpu(device):
             if a != b and mg > 0.05:
                 bad.append((p[:3], a, b, mg))
     assert not bad, f"clear-margin disagreements: {bad}"
+
+
+def test_captured_steps_under_a_default_device(model):
+    """Steps are captured, and graphs from outside replayed, where tensors that
+    name no device are on the GPU."""
+    def engine():
+        return LLMEngine(model, max_batch_size=4, max_model_len=128,
+                         num_blocks=128)
+
+    params = SamplingParams(temperature=0.0, min_p=0.0, max_tokens=8)
+    prompts = [[5, 9, 100, 42], [7, 7, 3, 900, 12, 4], list(range(10, 40))]
+    first = engine()
+    want = first.generate(prompts, params)
+    with torch.device("cuda"):
+        for e in (first, engine()):
+            assert e.generate(prompts, params) == want
+            assert e.use_graphs and e._graphs
