@@ -443,16 +443,18 @@ def linear(x, weight, bias=None, act=ACT_NONE):
 
 # decode_gemm's code for linear(...).float()
 _DECODE_F32 = 9
+_LINEAR = linear
 
 
 def linear_f32(x, weight):
     """linear(x, weight).float(). Up to 64 rows that take decode_gemm are stored as
-    32 bits by the product, without a launch of 4 to 5 us that widens them."""
+    32 bits by the product, without a launch of 4 to 5 us that widens them, unless
+    ops.linear has been replaced and is to see every product."""
     x2 = x.reshape(-1, x.shape[-1])
     M, K = x2.shape
     N = weight.shape[0]
     if (x.is_cuda and M <= 64 and x2.dtype == torch.bfloat16
-            and _gemm_mode() not in _OTHER_FORMS
+            and linear is _LINEAR and _gemm_mode() not in _OTHER_FORMS
             and not _to_choose(M, N, K, None) and _few_rows(x2, weight)
             and not _recorded(x2, weight)):
         _require_hip("_hip_gemm")
@@ -498,7 +500,7 @@ def norm_linear(a, b, w_norm, eps, weight, bias=None, gated=False,
     be what linear_parts returned, and with `shares` the linear is of that
     kind; with `f32` (no bias) it is linear_f32. One row is one launch."""
     N = weight.shape[0]
-    if (_gemm_mode() not in _OTHER_FORMS
+    if (_gemm_mode() not in _OTHER_FORMS and not (f32 and linear is not _LINEAR)
             and weight.dtype == torch.bfloat16 and weight.shape[1] % 64 == 0
             and N % (128 if gated else 64) == 0
             and (bias is None or (bias.dtype == torch.bfloat16

@@ -80,3 +80,19 @@ def test_norm_linear_f32(rows, N, K):
     want, sums = ops.norm_linear(a, b, w_norm, 1e-5, w)
     assert out.dtype == torch.float32 and torch.equal(x, sums)
     assert torch.equal(out, want.float())
+
+
+@pytest.mark.parametrize("rows", [1, 3])
+def test_a_replaced_linear_sees_the_logits(rows, monkeypatch):
+    """Of both ways to make them, one row's with the norm in its launch."""
+    a, b = _randn(rows, 1280), _randn(rows, 1, 1280, seed=1)
+    w_norm, w = _randn(1280, seed=2), _randn(512, 1280, seed=3)
+    first = ops.norm_linear(a, b, w_norm, 1e-5, w, f32=True)
+    last = ops.linear_f32(a, w)
+    seen, own = [], ops.linear
+    monkeypatch.setattr(ops, "linear", lambda x, w, *r, **k: seen.append(
+        w) or own(x, w, *r, **k))
+    for g, v in zip(first, ops.norm_linear(a, b, w_norm, 1e-5, w, f32=True)):
+        assert torch.equal(g, v)
+    assert torch.equal(last, ops.linear_f32(a, w))
+    assert len(seen) == 2 and all(s is w for s in seen)
