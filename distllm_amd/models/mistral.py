@@ -332,5 +332,12 @@ class DecoderModel(nn.Module):
                 inter, x = ops.norm_linear(attn, x, layer.post_norm, eps,
                                            layer.wgup, gated=True)
                 down = self._allreduce(parts(inter, layer.wdown))
+        if type(self).logits is not _LOGITS or "logits" in self.__dict__:
+            h, _ = ops.norm_parts_sum(down, x, self.final_norm, eps=eps)
+            return self.logits(h[:, 0])
+        # logits of the norm, which one row's product takes into its launch
         w = self.lm_head if self.lm_head is not None else self.tok_emb
         return ops.norm_linear(down, x, self.final_norm, eps, w, f32=True)[0]
+
+
+_LOGITS = DecoderModel.logits

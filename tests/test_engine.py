@@ -251,3 +251,27 @@ def test_block_manager_invariants():
         bm.alloc(1)
     bm.release(a)
     assert bm.can_alloc(3) and not bm.can_alloc(4)
+
+
+@pytest.mark.parametrize("where", ["instance", "class", "subclass"])
+def test_replaced_logits_hold_for_every_step(model, monkeypatch, where):
+    """One token only is left to choose, after the prompt as in decoding."""
+    own = type(model).logits
+
+    def logits(self, hidden):
+        out = torch.full_like(own(self, hidden), -1e9)
+        out[..., 77] = 0
+        return out
+
+    if where == "instance":
+        monkeypatch.setitem(model.__dict__, "logits",
+                            lambda hidden: logits(model, hidden))
+    elif where == "class":
+        monkeypatch.setattr(type(model), "logits", logits)
+    else:
+        sub = type("Own", (type(model),), {"logits": logits})
+        monkeypatch.setattr(model, "__class__", sub)
+    engine = LLMEngine(model, max_batch_size=2, max_model_len=64,
+                       num_blocks=16)
+    params = SamplingParams(temperature=0.0, min_p=0.0, max_tokens=4)
+    assert engine.generate([[5, 9], [7, 3, 8]], params) == [[77] * 4] * 2
