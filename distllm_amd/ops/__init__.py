@@ -1078,25 +1078,24 @@ def step_plan(layers, ctx, H, kcache, block_table):
 
 def step_begin(tokens, emb, w_norm, eps, layers, ctx, H, kcache, block_table):
     """The rows x [B, 1, n] of tokens [B] in the table emb, the RMS norm of x times
-    w_norm, and step_plan of the others: where the step has a plan, in its launch.
-    With this and the head's product by norm_linear(..., f32=True) a step of eight
-    layers of 4096 takes, us, one row of 2048 tokens 792 -> 780, with 8-bit weights
-    583 -> 572, 64 rows 1476 -> 1454."""
-    if (layers > 0 and kcache.is_cuda and kcache.shape[3] in (64, 128)
-            and tokens.device == emb.device == w_norm.device == kcache.device
-            and tokens.dim() == 1 and tokens.dtype in (torch.int64, torch.int32)
-            and emb.dim() == 2 and 0 < emb.shape[1] <= 8192
-            and emb.shape[1] % 8 == 0 and w_norm.shape == emb.shape[1:]
-            and all(t.dtype == torch.bfloat16 and t.is_contiguous()
-                    and t.data_ptr() % 16 == 0 for t in (emb, w_norm))
-            and not _recorded(tokens, emb, w_norm)):
-        _require_hip()
-        slots, zeros, x, h = _hip_ops.step_plan(
-            ctx.int(), block_table.int(), layers, H, kcache.shape[1],
-            kcache.dtype == torch.uint8, tokens.long().contiguous(), emb,
-            w_norm, eps)
-        return x, h, [(slots, row) for row in zeros.unbind()]
+    w_norm, and step_plan of the others: where the step has a plan, the norm in its
+    launch. (The rows are torch's to take, which refuses a token outside the table; a
+    launch that took them too was 3 to 6 us less.) With this and the head's product by
+    norm_linear(..., f32=True) a step of eight layers of 4096 takes, us, one row of
+    2048 tokens 792 -> 786, with 8-bit weights 583 -> 577, 64 rows 1476 -> 1457."""
     x = emb[tokens.long()].unsqueeze(1)
+    if (layers > 0 and kcache.is_cuda and kcache.shape[3] in (64, 128)
+            and x.device == w_norm.device == kcache.device
+            and x.dim() == 3 and 0 < x.shape[2] <= 8192
+            and x.shape[2] % 8 == 0 and w_norm.shape == x.shape[2:]
+            and all(t.dtype == torch.bfloat16 and t.is_contiguous()
+                    and t.data_ptr() % 16 == 0 for t in (x, w_norm))
+            and not _recorded(x, w_norm)):
+        _require_hip()
+        slots, zeros, h = _hip_ops.step_plan(
+            ctx.int(), block_table.int(), layers, H, kcache.shape[1],
+            kcache.dtype == torch.uint8, x, w_norm, eps)
+        return x, h, [(slots, row) for row in zeros.unbind()]
     return (x, rms_norm(x, w_norm, eps=eps),
             step_plan(layers, ctx, H, kcache, block_table))
 

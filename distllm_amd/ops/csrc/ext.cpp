@@ -72,8 +72,8 @@ void launch_step_attn(const void*, const float*, int, const void*,
                       int, int, int, int, int, float, bool, bool, const Ahead*,
                       hipStream_t);
 void launch_step_plan(const int*, const int*, int, int, int, int, int, int,
-                      int*, int*, long, const long*, const void*, const void*,
-                      void*, void*, long, int, float, hipStream_t);
+                      int*, int*, long, const void*, const void*, void*, int,
+                      float, hipStream_t);
 int step_plan_room(int, int, int, int);
 void launch_norm_parts(const float*, int, const void*, const void*, void*,
                        void*, int, int, float, hipStream_t);
@@ -623,13 +623,11 @@ static StepShares step_shares(int64_t B, int64_t H, int64_t HKV,
 // What the attention launches of a decode step of `layers` layers need:
 // [room, 8] shares and what PaStep says of them, and zeros [layers, B * HKV * groups of 16 query heads], a row
 // of which each launch uses up.
-// With tokens [B], also x [B, 1, n], their rows of emb [V, n], and the RMS norm of x
-// times w.
+// With x [B, 1, n], also its RMS norm times w.
 std::vector<torch::Tensor> step_plan(torch::Tensor ctx,
                                      torch::Tensor block_table, int64_t layers,
                                      int64_t H, int64_t HKV, bool fp8,
-                                     c10::optional<torch::Tensor> tokens,
-                                     c10::optional<torch::Tensor> emb,
+                                     c10::optional<torch::Tensor> x,
                                      c10::optional<torch::Tensor> w,
                                      double eps) {
   CHECK_INTS(ctx);
@@ -645,26 +643,20 @@ std::vector<torch::Tensor> step_plan(torch::Tensor ctx,
   auto arrived = torch::empty({layers, B * HKV * ((H / HKV + 15) / 16)},
                               ctx.options());
   std::vector<torch::Tensor> out = {slots, arrived};
-  torch::Tensor x, h;
-  if (tokens) {
-    TORCH_CHECK(emb && w, "tokens come with a table and the norm's weights");
-    CHECK_DEV(tokens.value()); CHECK_CONT(tokens.value());
-    for (const auto& t : {*emb, *w}) {
+  torch::Tensor h;
+  if (x) {
+    TORCH_CHECK(w, "rows come with the norm's weights");
+    for (const auto& t : {*x, *w}) {
       CHECK_DEV(t); CHECK_CONT(t); CHECK_BF16(t);
       TORCH_CHECK((uintptr_t)t.data_ptr() % 16 == 0 &&
                       t.device() == ctx.device(),
                   "16-byte alignment");
     }
-    TORCH_CHECK(tokens->scalar_type() == at::kLong && tokens->numel() == B &&
-                    tokens->device() == ctx.device(),
-                "tokens must be [B] int64");
-    TORCH_CHECK(emb->dim() == 2 && emb->size(1) == w->numel() &&
-                    w->numel() > 0 && w->numel() % 8 == 0 &&
-                    w->numel() <= 8192,
-                "table must be [V, n], n % 8 == 0 and up to 8192");
-    x = torch::empty({B, 1, w->numel()}, emb->options());
-    h = torch::empty_like(x);
-    out.push_back(x);
+    TORCH_CHECK(x->dim() == 3 && x->size(0) == B && x->size(1) == 1 &&
+                    x->size(2) == w->numel() && w->numel() > 0 &&
+                    w->numel() % 8 == 0 && w->numel() <= 8192,
+                "rows must be [B, 1, n], n % 8 == 0 and up to 8192");
+    h = torch::empty_like(*x);
     out.push_back(h);
   }
   if (B > 0)
@@ -672,10 +664,8 @@ std::vector<torch::Tensor> step_plan(torch::Tensor ctx,
         ctx.data_ptr<int>(), block_table.data_ptr<int>(), (int)B,
         (int)max_blocks, s.room, s.narrow, s.wide, s.asked,
         slots.data_ptr<int>(), arrived.data_ptr<int>(), arrived.numel(),
-        tokens ? tokens->data_ptr<int64_t>() : nullptr,
-        tokens ? emb->data_ptr() : nullptr, tokens ? w->data_ptr() : nullptr,
-        tokens ? x.data_ptr() : nullptr, tokens ? h.data_ptr() : nullptr,
-        tokens ? emb->size(0) : 0, tokens ? (int)w->numel() : 0, (float)eps,
+        x ? x->data_ptr() : nullptr, x ? w->data_ptr() : nullptr,
+        x ? h.data_ptr() : nullptr, x ? (int)w->numel() : 0, (float)eps,
         cur_stream());
   return out;
 }
@@ -1028,8 +1018,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("slots"), py::arg("arrived"), py::arg("ahead") = py::none());
   m.def("step_plan", &step_plan, py::arg("ctx"), py::arg("block_table"),
         py::arg("layers"), py::arg("H"), py::arg("HKV"), py::arg("fp8"),
-        py::arg("tokens") = py::none(), py::arg("emb") = py::none(),
-        py::arg("w") = py::none(), py::arg("eps") = 0.0);
+        py::arg("x") = py::none(), py::arg("w") = py::none(),
+        py::arg("eps") = 0.0);
   m.def("found_lists", &found_lists);
   m.def("rope_put", &rope_put, py::arg("qkv"), py::arg("cs"), py::arg("sn"),
         py::arg("ctx"), py::arg("kcache"), py::arg("vcache"),

@@ -814,33 +814,25 @@ __host__ __device__ constexpr bool plan_many(int B, int p) {
 }
 constexpr int PLAN_ROWS = 1024;  // beyond, each sequence is a share, in order
 
-// What else a step begins with, in workgroups of the same launch: x, the rows of
-// its tokens in an embedding table, and their RMS norm. (Launches of their own for
-// both cost 6 to 8 us of a step.) Tokens are counted from the end where negative,
-// and rows of those outside the table NaN. Sums as in norm_fwd_small_kernel.
+// What else a step begins with, in workgroups of the same launch: the RMS norm of its
+// rows x. (A launch of its own costs 3 to 4 us of a step.) Sums as in
+// norm_fwd_small_kernel.
 struct PlanRows {
-  const long* tokens;
-  const unsigned short *emb, *w;
-  unsigned short *x, *h;
-  long V;
+  const unsigned short *x, *w;
+  unsigned short* h;
   int H;  // a multiple of 8, up to 8192; 0: none
   float eps;
 };
 __device__ __forceinline__ void plan_row(const PlanRows& p, int row) {
   __shared__ float red[4];
   const int tid = threadIdx.x;
-  long token = p.tokens[row];
-  if (token < 0) token += p.V;
-  const bool is = token >= 0 && token < p.V;
   s16x8 xv[4];
   float sumsq = 0.f;
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
     const int c = (tid + k * 256) * 8;
-    xv[k] = s16x8{} + (short)0x7fc0;
     if (c < p.H) {
-      if (is) xv[k] = *reinterpret_cast<const s16x8*>(p.emb + token * p.H + c);
-      *reinterpret_cast<s16x8*>(p.x + (long)row * p.H + c) = xv[k];
+      xv[k] = *reinterpret_cast<const s16x8*>(p.x + (long)row * p.H + c);
       float f[8];
       bf8_to_f32(xv[k], f);
 #pragma unroll
@@ -1002,14 +994,12 @@ extern "C" int step_plan_room(int B, int narrow, int wide, int asked) {
 extern "C" void launch_step_plan(const int* ctx, const int* table, int B,
                                  int max_blocks, int G, int narrow, int wide,
                                  int asked, int* slots, int* arrived,
-                                 long zeros, const long* tokens,
-                                 const void* emb, const void* w, void* x,
-                                 void* h, long V, int H, float eps,
+                                 long zeros, const void* x, const void* w,
+                                 void* h, int H, float eps,
                                  hipStream_t stream) {
   const int clear = (int)std::min((zeros + 1023) / 1024, 256L);
-  const PlanRows rows = {tokens, (const unsigned short*)emb,
-                         (const unsigned short*)w, (unsigned short*)x,
-                         (unsigned short*)h, V, H, eps};
+  const PlanRows rows = {(const unsigned short*)x, (const unsigned short*)w,
+                         (unsigned short*)h, H, eps};
   hipLaunchKernelGGL(step_plan_kernel,
                      dim3(1 + clear + (B + 3) / 4 + (H > 0 ? B : 0)),
                      dim3(256), B > PLAN_ROWS ? 0 : B * 12, stream, ctx, table,

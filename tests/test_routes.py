@@ -350,3 +350,32 @@ def test_traces_modes_and_casts_are_followed(monkeypatch):
         monkeypatch.setattr(torch, "get_autocast_dtype", lambda kind: dtype)
         f(x)
     assert seen == [True, True, False, True, False]
+
+
+def test_tokens_outside_the_table_are_refused(monkeypatch):
+    """A decode step's rows are torch's to take, where a launch makes their norm as
+    elsewhere."""
+    class Ops:
+        def require(self, name):
+            pass
+
+        def step_plan(self, ctx, table, layers, H, HKV, fp8, x, w, eps):
+            return torch.zeros(1, 8), torch.zeros(layers, 1), x
+
+    class Cache:
+        is_cuda, device, shape = True, torch.device("cpu"), (4, 2, 16, 64)
+        dtype = torch.bfloat16
+
+    monkeypatch.setattr(ops, "_hip_ops", Ops())
+    emb, w = torch.randn(7, 64).bfloat16(), torch.ones(64).bfloat16()
+    ints = torch.ones(2, dtype=torch.int32)
+    for dtype in (torch.int32, torch.int64):
+        tokens = torch.tensor([-7, 6], dtype=dtype)
+        x, h, plan = ops.step_begin(tokens, emb, w, 1e-5, 3, ints, 4, Cache(),
+                                    ints[:, None])
+        assert torch.equal(x[:, 0], emb[[0, 6]]) and h is x and len(plan) == 3
+        for wrong in (7, -8):
+            tokens[1] = wrong
+            with pytest.raises(IndexError):
+                ops.step_begin(tokens, emb, w, 1e-5, 3, ints, 4, Cache(),
+                               ints[:, None])
