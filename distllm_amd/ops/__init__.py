@@ -884,8 +884,10 @@ def _score_topk_fills(Q, N, K):
     """Whether score_topk's launches are faster than the scores, by the library,
     and topk. By the share of the scores among what the rounds of the card's 256
     CUs could make, own time over theirs, 33 to 513 queries, 4000 to 250000 rows:
-    - two f16 parts (score.hip: from 65 queries and K = 256 on) from 0.3 on 0.37
-      to 0.96, below, which is tiles of a few thousand rows, up to 2.4;
+    - two f16 parts (score.hip: from 65 queries and K = 256 on) from 0.3 on 0.44
+      to 1.01, below, which is tiles of a few thousand rows, up to 1.7; more than
+      256 queries of less than 384 columns, whose launches are the most of it, up
+      to 4 million scores 0.8 to 1.27, beyond 0.52 to 0.85;
     - three bf16 parts, K <= 384, one tile of queries 0.34 to 1.0, several from
       0.5 on 0.5 to 0.8, below up to 1.1; K <= 1024 from 0.25 on 0.63 to 0.98,
       below up to 1.07; K of 1536 from 0.65 on 0.79 to 0.98, below up to 1.7."""
@@ -895,6 +897,8 @@ def _score_topk_fills(Q, N, K):
         each = min(max(256 // queries, 1), rows)
         rounds = -(-queries * each // 256) * -(-rows // each)
         least = 0.3
+        if Q > 256 and K < 384 and Q * N < 4_000_000:
+            return False
     else:
         rounds = -(-queries * rows // 256)
         least = (0.65 if K > 1024 else 0.25 if K > 384 else
@@ -907,10 +911,14 @@ def _search_few_fills(Q, N, K):
     against the library's product and topk, own time over theirs, k to 30. One
     query, 64 to 1024 columns, from 10000 rows on 0.43 to 0.96, 8192 rows 0.88 to
     1.15, below up to 1.3; two, from 128 columns on, 0.47 to 1.0, of 64 up to 1.1.
-    Three and four of 128 to 768 columns to 32768 rows 0.58 to 1.0, beyond, of 768
-    0.53 (100000 rows, where the library's choice is a slow one, as it is of 120000
-    and 170000) to 1.02 at 50000 and 250000, of 384 0.95 to 1.07, of 128 up to 1.3;
-    of 64 up to 1.6, of more than 768, whose sums leave no room for rows, up to 1.5."""
+    Three and four of 128 to 768 columns to 32768 rows 0.58 to 1.0; beyond, of 384
+    0.95 to 1.07, of 128 up to 1.3; of 64 up to 1.6, of more than 768, whose sums
+    leave no room for rows, up to 1.5. Of 544, 640 and 768 columns the library's time
+    jumps by a factor of two from one size to the next beyond 60000 rows, and own
+    time lies between: at 18 sizes from 33000 to 200000 rows 0.45 to 0.97 but for
+    120000 and 180000 of 544 and 130000 and 190000 of all, 1.03 to 1.11. Beyond it is
+    as it is below (215000 to 300000 rows 0.48 to 0.59 and 1.04 to 1.13, 250000 among
+    the latter), and left to the library."""
     if N < 10000 or K % 4 or K < (64 if Q == 1 else 128):
         return False
     return K <= 1024 if Q <= 2 else Q <= 4 and K <= 768 and (

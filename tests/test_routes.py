@@ -98,6 +98,8 @@ def test_score_where_tiles_fill_the_card(kernels, Q, N, K, way):
     (65, 20000, 384, 60, "kernels"), (33, 20000, 768, 1, "kernels"),
     (256, 250000, 768, 61, "scores"), (32, 250000, 768, 10, "scores"),
     (256, 4000, 768, 10, "scores"), (64, 8000, 768, 10, "scores"),
+    (400, 8000, 256, 10, "scores"), (400, 10000, 352, 10, "kernels"),
+    (513, 7700, 384, 10, "kernels"), (256, 10000, 256, 10, "kernels"),
     (64, 40000, 1536, 10, "scores"), (64, 120000, 1536, 10, "kernels"),
     (256, 250000, 784, 10, "scores"), (300, 50000, 128, 10, "scores")])
 def test_topk_of_scores_without_their_matrix(monkeypatch, Q, N, K, k, way):
