@@ -351,11 +351,10 @@ class LLMEngine:
         s.blocks = []
         s.cached = 0
 
-    def _block_table(self, seqs: list[_Seq],
-                     width: int | None = None) -> torch.Tensor:
+    def _block_table(self, seqs: list[_Seq]) -> torch.Tensor:
         # build on the host, upload in ONE copy (a per-row device
         # tensor-from-list costs one tiny H2D copy per sequence/step)
-        maxb = width or max(len(s.blocks) for s in seqs)
+        maxb = max(len(s.blocks) for s in seqs)
         bt = torch.zeros(len(seqs), maxb, dtype=torch.int32)
         for i, s in enumerate(seqs):
             bt[i, : len(s.blocks)] = torch.tensor(s.blocks,

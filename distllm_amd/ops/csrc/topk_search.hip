@@ -464,8 +464,8 @@ search_few_kernel(const float* __restrict__ q,
         row[j] = __builtin_amdgcn_ds_permute(rank * 4, lane < n ? s0 + lane : -1);
         least[j] = __builtin_amdgcn_readlane(best[j], k - 1);
       } else {
-        unsigned long long some =
-            __ballot(lane < n && (u > least[j] || r1 - r0 < k));
+        // (64 rows, more than k, are behind these)
+        unsigned long long some = __ballot(lane < n && u > least[j]);
         while (some) {
           const int i = __ffsll(some) - 1;
           some &= some - 1;
