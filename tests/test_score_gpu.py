@@ -65,6 +65,24 @@ def test_not_finite(device):
                                atol=1e-6)
 
 
+@pytest.mark.parametrize("Q", [65, 128, 256, 520])
+@pytest.mark.parametrize("N, K", [(40000, 256), (40001, 288), (20003, 352)])
+def test_many_tiles(device, Q, N, K):
+    """Bounds as of test_against_64_bits; infinities and NaN stay where they are."""
+    q, c = _unit(Q, K, Q), _unit(N, K, N)
+    c[5000:5300, K - 1] = 70.0
+    c[N // 3: N // 3 + 100] *= 1e-6
+    c[N - 1, 5], c[777, 0] = float("inf"), float("nan")
+    out = _hip_ops.score(q, c)
+    want = q.double() @ c.double().t()
+    size = q.double().abs() @ c.double().abs().t()
+    real = want.isfinite()
+    bound = size * (12 * K / 32 + 3) * 2 ** -24 + 1e-12
+    assert ((out.double() - want).abs() <= bound)[real].all()
+    assert torch.equal(out.isnan(), want.isnan())
+    assert torch.equal(out.isinf(), want.isinf())
+
+
 def test_rule(device):
     """Both sides of the rule agree, as do operands that only one takes."""
     for Q, N, K in ((32, 20000, 64), (33, 20000, 64), (40, 16256, 64),

@@ -121,3 +121,14 @@ def test_place_of_a_query(device):
         assert torch.equal(v[at: at + 256], v[:256])
         assert torch.equal(i[at: at + 256], i[:256])
     _check(q, c, 10)
+
+
+@pytest.mark.parametrize("Q", [65, 128, 256, 520])
+@pytest.mark.parametrize("N, K", [(70001, 288), (66000, 352), (90000, 256)])
+def test_runs_of_tiles(device, Q, N, K):
+    """Workgroups of several tiles: odd and even numbers of steps over their edges, the
+    last tile whole and not, a tile in the middle that is made by bf16 parts."""
+    q, c = _unit(Q, K, Q), _unit(N, K, K)
+    _check(q, c, 12)
+    c[N // 2: N // 2 + 3] *= 1e4
+    _check(q, c, 12)
