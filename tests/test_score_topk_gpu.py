@@ -133,3 +133,27 @@ def test_runs_of_tiles(device, Q, N, K):
     _check(q, c, 12)
     c[N // 2: N // 2 + 3] *= 1e4
     _check(q, c, 12)
+
+
+def test_captured(device):
+    """Replays of one graph over queries that f16 parts do for, that they lose too much
+    of, and back: which launches do the work is decided on the device."""
+    c = _unit(30000, 256, 11)
+    c[:, 0] = 1
+    c[:, 1:] *= 6e-3
+    plain, blind = _unit(100, 256, 12), _unit(100, 256, 13)
+    blind[:, 0] = 0
+    q = plain.clone()
+    _hip_ops.score_topk(q, c, 10)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        v, i = _hip_ops.score_topk(q, c, 10)
+    for now in (plain, blind, plain, blind):
+        q.copy_(now)
+        graph.replay()
+        got = v.clone(), i.clone()
+        want = _hip_ops.score_topk(now, c, 10)
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+        _check(now, c, 10)
+        torch.cuda.synchronize()
