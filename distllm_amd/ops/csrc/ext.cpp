@@ -4,6 +4,10 @@
 // if this extension is missing — no silent eager fallback.
 // All kernels are hand-written CDNA4 HIP (see *.hip in this directory);
 // this file only validates tensors and forwards device pointers.
+#include <climits>
+#include <cmath>
+#include <limits>
+
 #include "ahead.h"
 #include "ext_common.h"
 
@@ -50,6 +54,13 @@ void launch_search_top(const unsigned int*, const float*, const float*, float*,
 int search_few_groups(int);
 void launch_search_few(const float*, const float*, float*, int*, int, int, int,
                        int, hipStream_t);
+void launch_narrow_most(const float*, long, int*, hipStream_t);
+void launch_narrow_rows(const float*, void*, long, int, int, int, float*,
+                        hipStream_t);
+long narrow_bytes(long, long, long, long);
+void launch_narrow_topk(const float*, const float*, const void*, void*, float*,
+                        int*, int, int, int, int, int, float, float, int,
+                        hipStream_t);
 void launch_topk_chunk(const float*, const int*, float*, int*, int, long, int,
                        int, bool, hipStream_t);
 void launch_hamming_score(const void*, const void*, float*, int, long, int,
@@ -505,6 +516,69 @@ std::vector<torch::Tensor> search_few(torch::Tensor q, torch::Tensor corpus,
   return {ov, oi};
 }
 
+// Rows [N, K] times the power of two that brings the largest number to 2^13, as f16
+// in blocks (narrow_search.hip; [N in whole 16s, K in whole 64s] of them), that power, and the largest |row - row as f16| and |row as f16|
+// (and the root of the mean square of the latter) of rows times it. Nothing where a
+// number is infinite or NaN, or all are 0. Waits for the GPU.
+c10::optional<std::tuple<torch::Tensor, int64_t, double, double, double>>
+narrow_rows(torch::Tensor corpus) {
+  CHECK_DEV(corpus); CHECK_CONT(corpus); CHECK_F32(corpus);
+  TORCH_CHECK(corpus.dim() == 2 && corpus.size(0) > 0 && corpus.size(1) > 0 &&
+                  corpus.size(1) % 4 == 0 && corpus.size(1) < (1L << 16) &&
+                  (uintptr_t)corpus.data_ptr() % 16 == 0,
+              "rows of fours, aligned to 16 bytes");
+  const c10::DeviceGuard guard(corpus.device());
+  const long N = corpus.size(0), K = corpus.size(1);
+  const long KP = std::max(128L, (K + 63) / 64 * 64);
+  auto facts = torch::zeros({4}, corpus.options());
+  launch_narrow_most(corpus.data_ptr<float>(), N * K,
+                     reinterpret_cast<int*>(facts.data_ptr<float>()) + 3,
+                     cur_stream());
+  const float most = facts[3].item<float>();
+  if (!(most > 0.f && most <= std::numeric_limits<float>::max()))
+    return c10::nullopt;
+  const int up = std::min(13 - std::ilogb(most), 120);
+  auto rows = torch::empty({(N + 15) / 16 * 16, KP}, corpus.options().dtype(at::kHalf));
+  launch_narrow_rows(corpus.data_ptr<float>(), rows.data_ptr(), N, (int)K,
+                     (int)KP, up, facts.data_ptr<float>(), cur_stream());
+  const auto host = facts.cpu();
+  const float* f = host.data_ptr<float>();
+  return std::make_tuple(rows, (int64_t)up, std::sqrt((double)f[0]),
+                         std::sqrt((double)f[1]), std::sqrt((double)f[2] / N));
+}
+
+// The k best rows for every query, [Q, k] scores and rows one behind the other, by
+// way of the rows that narrow_rows made (narrow_search.hip). A query that they cannot
+// answer has INT_MIN for rows.
+std::vector<torch::Tensor> narrow_topk(torch::Tensor q, torch::Tensor corpus,
+                                       torch::Tensor rows, int64_t up,
+                                       double error, double norm, int64_t k) {
+  for (const auto& t : {q, corpus, rows}) {
+    CHECK_DEV(t); CHECK_CONT(t);
+    TORCH_CHECK(t.dim() == 2 && (uintptr_t)t.data_ptr() % 16 == 0 &&
+                    t.device() == q.device(),
+                "rows aligned to 16 bytes");
+  }
+  CHECK_F32(q); CHECK_F32(corpus);
+  TORCH_CHECK(rows.scalar_type() == at::kHalf, "rows as f16");
+  const long Q = q.size(0), K = q.size(1), N = corpus.size(0),
+             KP = rows.size(1);
+  const long bytes = narrow_bytes(Q, N, K, KP);
+  TORCH_CHECK(bytes > 0 && corpus.size(1) == K && rows.size(0) == (N + 15) / 16 * 16 &&
+                  k > 0 &&
+                  k <= 60 && k <= N && up >= -200 && up <= 200,
+              "narrow_topk: sizes");
+  const c10::DeviceGuard guard(q.device());
+  auto space = torch::empty({bytes}, q.options().dtype(at::kByte));
+  auto both = torch::empty({2, Q, k}, q.options().dtype(at::kInt));
+  auto ov = both.select(0, 0).view(at::kFloat), oi = both.select(0, 1);
+  launch_narrow_topk(q.data_ptr<float>(), corpus.data_ptr<float>(),
+                     rows.data_ptr(), space.data_ptr(), ov.data_ptr<float>(),
+                     oi.data_ptr<int>(), (int)Q, (int)N, (int)K, (int)KP,
+                     (int)up, (float)error, (float)norm, (int)k, cur_stream());
+  return {ov, oi};
+}
+
 std::vector<torch::Tensor> topk_chunked(torch::Tensor scores,
                                         c10::optional<torch::Tensor> in_idx,
                                         int64_t k, int64_t chunk, bool regs) {
@@ -931,8 +1005,8 @@ c10::optional<torch::Tensor> bert_few_rows(torch::Tensor x,
 // of both, joined on the way if they do not lie one behind the other. As steps of
 // Python this took a first call on a new question, which finds the host's caches
 // full of other things, 60 us longer than two copies.
-static std::pair<py::list, py::list> found_lists(torch::Tensor v,
-                                                 torch::Tensor i) {
+// sure: nothing (None) where an index is INT_MIN (see narrow_topk).
+static py::object found_lists(torch::Tensor v, torch::Tensor i, bool sure) {
   CHECK_DEV(v); CHECK_F32(v);
   CHECK_DEV(i); CHECK_I32(i);
   TORCH_CHECK(v.dim() == 2 && v.sizes() == i.sizes() &&
@@ -953,6 +1027,7 @@ static std::pair<py::list, py::list> found_lists(torch::Tensor v,
   }
   const int* indices = host.data_ptr<int>() + n;
   const float* scores = reinterpret_cast<const float*>(host.data_ptr<int>());
+  if (sure && std::count(indices, indices + n, INT_MIN) > 0) return py::none();
   py::list all_scores(Q), all_indices(Q);
   for (int64_t q = 0; q < Q; ++q, scores += k, indices += k) {
     const int64_t kept =
@@ -966,7 +1041,7 @@ static std::pair<py::list, py::list> found_lists(torch::Tensor v,
     all_scores[q] = std::move(s);
     all_indices[q] = std::move(x);
   }
-  return {all_scores, all_indices};
+  return py::make_tuple(all_scores, all_indices);
 }
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -999,6 +1074,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("score", &score);
   m.def("score_topk", &score_topk);
   m.def("search_few", &search_few);
+  m.def("narrow_rows", &narrow_rows);
+  m.def("narrow_topk", &narrow_topk);
+  m.def("narrow_bytes", &narrow_bytes);
   m.def("topk_chunked", &topk_chunked, py::arg("scores"), py::arg("in_idx"),
         py::arg("k"), py::arg("chunk"), py::arg("regs") = false);
   m.def("hamming_score", &hamming_score);
@@ -1020,7 +1098,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("layers"), py::arg("H"), py::arg("HKV"), py::arg("fp8"),
         py::arg("x") = py::none(), py::arg("w") = py::none(),
         py::arg("eps") = 0.0);
-  m.def("found_lists", &found_lists);
+  m.def("found_lists", &found_lists, py::arg("v"), py::arg("i"),
+        py::arg("sure") = false);
   m.def("rope_put", &rope_put, py::arg("qkv"), py::arg("cs"), py::arg("sn"),
         py::arg("ctx"), py::arg("kcache"), py::arg("vcache"),
         py::arg("block_table"), py::arg("bias") = py::none());

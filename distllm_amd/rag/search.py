@@ -2,9 +2,11 @@
 faiss-gpu entirely (reference distllm/rag/search.py:59-928).
 
 Design (MI355X-first): the corpus embedding matrix lives in HBM
-(288 GB/GPU holds ~17B fp32x4 dims); exact inner-product search is a
-chunked GEMM (hipBLASLt) + the hand-written radix-select top-k kernel
-(topk_search.hip); the `ubinary` precision path packs sign bits into
+(288 GB/GPU holds ~17B fp32x4 dims), once in fp32 and once in 16 bits;
+exact inner-product search reads the latter, finds with a bound which
+rows can be among the best, and scores these in fp32 (narrow_search.hip;
+where that is no gain or not certain, products of all rows and top-k,
+score.hip and topk_search.hip); the `ubinary` precision path packs sign bits into
 u64 words (word-major for coalesced candidate reads) and scores with
 the HIP popcount-Hamming kernel, then rescores `top_k *
 rescore_multiplier` candidates against the fp32 queries.
@@ -99,6 +101,8 @@ class HipIndexConfig(BaseConfig):
 class HipFlatIndex:
     """GPU-resident flat index over the HF-dataset interchange format
     (columns `text`, `embeddings` fp32)."""
+
+    narrow: ops.NarrowRows | None = None
 
     def __init__(self, dataset_dir: Path, faiss_index_path: Path,
                  dataset_chunk_paths: list[Path] | None = None,
@@ -195,6 +199,9 @@ class HipFlatIndex:
             self.code_words = W
         if self.search_algorithm == "ivf":
             self._build_ivf()
+        elif self.precision == "float32":
+            # the rows once more in 16 bits, which searches read in their place
+            self.narrow = ops.narrow_rows(self.corpus)
 
     def _assign(self, cent: torch.Tensor) -> torch.Tensor:
         """argmax cluster per corpus row, GEMM-chunked so the score
@@ -335,6 +342,18 @@ class HipFlatIndex:
         v, sel = torch.topk(allv, k, dim=1)
         return v, alli.gather(1, sel.long()).int()
 
+    def _found_narrow(self, q: torch.Tensor, k: int):
+        """What _topk_exact finds, as lists, by way of the rows in 16 bits; None
+        where these do not answer it, for want of speed or of certainty, or
+        where another search has been put in _topk_exact's place."""
+        if (self.narrow is None or q.dim() != 2
+                or getattr(self._topk_exact, "__func__", None)
+                is not HipFlatIndex._topk_exact):
+            return None
+        found = ops.score_topk_narrow(q, self.corpus, min(k, self.n),
+                                      self.narrow)
+        return None if found is None else ops.found_lists(*found, sure=True)
+
     def _topk_ubinary(self, qfp: torch.Tensor, k: int):
         """Hamming candidates (HIP popcount) + fp32 rescore."""
         qb = quantize_embeddings(qfp.cpu().numpy(), "ubinary")
@@ -361,16 +380,21 @@ class HipFlatIndex:
         q = torch.from_numpy(
             np.ascontiguousarray(query_embedding, dtype=np.float32)
         ).to(self.corpus.device)
+        lists = None
         if self.precision == "ubinary":
             v, i = self._topk_ubinary(q, top_k)
         elif self.search_algorithm == "ivf":
             v, i = self._topk_ivf(q, top_k)
         else:
-            v, i = self._topk_exact(q, top_k)
+            lists = self._found_narrow(q, top_k)
+            if lists is None:
+                v, i = self._topk_exact(q, top_k)
         # IVF pads short candidate lists with index -1 / score -inf;
         # drop those unconditionally (not only under score_threshold) so
         # -1 never reaches get()/dataset indexing as "last row".
-        if v.is_cuda:
+        if lists is not None:
+            vv, ii = lists
+        elif v.is_cuda:
             vv, ii = ops.found_lists(v.float(), i.int())
         else:
             both = _one_tensor(v.float().view(torch.int32), i.int()).numpy()
