@@ -22,6 +22,8 @@
 //          waves share, one barrier per chunk; where N alone does not fill
 //          the chip K is split over workgroups and a second launch sums fp32
 //          slabs. Some hundred rows go by blocks of 64 (mid_gemm_shares).
+//  even    17 to 64 rows where tiles of 48 to 128 columns come out even on the
+//          card's CUs and those of 64 do not.
 //
 // Measured in a graph over fresh weights, us (GB/s of weights); before: the
 // faster of a two-stage tile of 128 rows with slabs and the library:
@@ -482,6 +484,144 @@ dg_tile_kernel(const u16* __restrict__ X, const u16* __restrict__ W,
   }
 }
 
+// ---- even -------------------------------------------------------------------
+// 17 to 64 rows (MP = 32 or 64 of them) by C sixteens of columns a workgroup, so many
+// that the columns, or their shares of K, come out even on the card's 256 CUs. Tiles
+// of 64 columns leave CUs with one or two of them beside each other (28672 columns
+// are 448 tiles), and every one reads all of x again: with 112 columns that is half as
+// much. One workgroup a CU, whose ring has all of LDS; 4 or 8 waves, 16 rows and half
+// of the columns each. A gated unit's sixteen rows of W are eight columns of either
+// kind, dealt so that a lane has both of a column.
+// us in a graph over fresh weights, 64 x 64 tiles and these, 17, 32, 64 rows: 28672 x
+// 4096 gated 42.7, 44.7, 49.8 and 43.7, 43.6, 45.1; 22016 x 4096 gated 39.9, 40.1, 45.3
+// and 37.3, 35.8, 38.7; 27648 x 5120 gated 57.2, 60.5, 68.2 and 54.6, 53.7, 57.1; 32768
+// x 4096 53.0, 52.6, 55.1 and 51.2, 50.7, 51.8; with shares of K (without what joins
+// them) 6144 x 4096, 2 and 4 13.2, 12.7, 14.7 and 11.2, 11.6, 13.6; 5120 x 5120, 2 and
+// 4 16.7, 18.0, 18.0 and 12.9, 12.8, 15.4.
+constexpr int dg_even_stages(int MP, int C) {
+  const int r = 160 * 1024 / ((C * 16 + MP) * 128);
+  return r > 8 ? 8 : r;
+}
+constexpr int dg_even_lds(int MP, int C) {
+  return dg_even_stages(MP, C) * (C * 16 + MP) * 128;
+}
+
+template <int ACT, int MP, int C, bool SLAB>
+__global__ void __launch_bounds__(MP * 8)
+dg_even_kernel(const u16* __restrict__ X, const u16* __restrict__ W,
+               float* __restrict__ slabs, int K, int splitk, int G,
+               const DgEnd e) {
+  constexpr bool GLU = dg_glu(ACT);
+  constexpr int NW = MP / 8, WM = MP / 16, CH = (C + 1) / 2;
+  constexpr int R = dg_even_stages(MP, C), STAGE = (C * 16 + MP) * 128;
+  constexpr int PIECES = STAGE / 1024, LOADS = (PIECES + NW - 1) / NW;
+  static_assert((R - 1) * LOADS < 64, "copies that vmcnt counts");
+  const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = lane & 15, g = lane >> 4;
+  const int cb = blockIdx.x % G, ks = blockIdx.x / G;
+  const int F = e.N / 16;
+  const int f0 = (int)((long)F * cb / G), mine = (int)((long)F * (cb + 1) / G) - f0;
+  const int nt = K / splitk / 64;
+  const int lr = lane >> 3, lc = ((lane & 7) ^ lr) * 8;
+  const u16* src[LOADS];
+  int to[LOADS];
+#pragma unroll
+  for (int p = 0; p < LOADS; ++p) {
+    // (of uneven numbers some pieces twice)
+    const int piece = min(wid * LOADS + p, PIECES - 1);
+    to[p] = piece * 1024;
+    const int row = piece * 8 + lr;
+    const u16* from;
+    if (piece < C * 2) {
+      const int f = f0 + min(row >> 4, mine - 1), j = row & 15;
+      const int n = GLU ? (j & 2) * (e.N / 4) + f * 8 + (j >> 2) * 2 + (j & 1)
+                        : f * 16 + j;
+      from = W + (long)n * K;
+    } else {
+      from = X + (long)min(row - C * 16, e.M - 1) * K;
+    }
+    src[p] = from + ks * (K / splitk) + lc;
+  }
+  const int turn = chunk_turn<19>(cb, nt);
+  auto issue = [&](int c) {
+    char* dst = smem + (c % R) * STAGE + lane * 16;
+    const int k = c + turn < nt ? c + turn : c + turn - nt;
+#pragma unroll
+    for (int p = 0; p < LOADS; ++p) dg_copy(src[p] + (long)k * 64, dst + to[p]);
+  };
+  const int wn = wid % 2, wm = wid / 2;
+  f32x4 acc[CH];
+#pragma unroll
+  for (int i = 0; i < CH; ++i) acc[i] = {0.f, 0.f, 0.f, 0.f};
+  auto compute = [&](int c) {
+    const char* b = smem + (c % R) * STAGE;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int piece = ((h * 4 + g) ^ (r & 7)) * 16;
+      const bf16x8 x = *reinterpret_cast<const bf16x8*>(
+          b + (C * 16 + wm * 16 + r) * 128 + piece);
+#pragma unroll
+      for (int i = 0; i < CH; ++i)
+        acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            *reinterpret_cast<const bf16x8*>(
+                b + (min(wn * CH + i, C - 1) * 16 + r) * 128 + piece),
+            x, acc[i], 0, 0, 0);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  };
+  auto arrive = [&]() {
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  for (int c = 0; c < R - 1; ++c) issue(c);
+  int c = 0;
+  for (; c + R - 1 < nt; ++c) {
+    dg_wait<(R - 2) * LOADS>();
+    arrive();
+    issue(c + R - 1);
+    compute(c);
+  }
+#pragma unroll
+  for (int left = R - 2; left >= 0; --left) {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"i"(left * LOADS) : "memory");
+    arrive();
+    compute(c++);
+  }
+  const int m = wm * 16 + r;
+  if (m >= e.M) return;
+#pragma unroll
+  for (int i = 0; i < CH; ++i) {
+    const int t = wn * CH + i;
+    if (t >= mine) continue;
+    if constexpr (SLAB && GLU) {
+      float* to = slabs + ((long)ks * e.M + m) * e.N + (f0 + t) * 8 + g * 2;
+      *reinterpret_cast<f32x2*>(to) = f32x2{acc[i][0], acc[i][1]};
+      *reinterpret_cast<f32x2*>(to + e.N / 2) = f32x2{acc[i][2], acc[i][3]};
+    } else if constexpr (SLAB) {
+      *reinterpret_cast<f32x4*>(slabs + ((long)ks * e.M + m) * e.N +
+                                (f0 + t) * 16 + g * 4) = acc[i];
+    } else if constexpr (GLU) {
+      const int n = (f0 + t) * 8 + g * 2, cols = e.N / 2;
+      unsigned int o = 0;
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        float a = acc[i][q], b = acc[i][2 + q];
+        if (e.bias != nullptr) {
+          a += bf2f(e.bias[n + q]);
+          b += bf2f(e.bias[cols + n + q]);
+        }
+        a = ACT == DG_SWIGLU ? silu(a) * b
+                             : clamped_glu(a, b, e.limit, e.alpha, e.shift);
+        o |= (unsigned int)f2bf(a) << (q * 16);
+      }
+      *reinterpret_cast<unsigned int*>(e.out + (long)m * cols + n) = o;
+    } else {
+      dg_finish<ACT>(e, m, (f0 + t) * 16 + g * 4, acc[i], acc[i]);
+    }
+  }
+}
+
 // sum of fp32 slabs [splitk, M, N], four columns a thread
 template <int ACT>
 __global__ void __launch_bounds__(256)
@@ -521,6 +661,15 @@ static bool dg_short_sums(int rows, int N, int K) {
   return N >= 16384 && K <= (rows <= 8 ? 1024 : 1536);
 }
 
+// Sixteens of columns of a workgroup in the even form where `splitk` share K, 0 where
+// that is another's: 3 and 5 to 8 (4 are the tile form), of which a CU has at least
+// 0.85 on average, and a sum that fills the ring.
+static int dg_even_columns(int rows, int N, int K, int splitk) {
+  if (rows <= 16 || rows > 64 || 256 % splitk || K / splitk < 512) return 0;
+  const int F = N / 16, G = 256 / splitk, C = (F + G - 1) / G;
+  return C >= 3 && C != 4 && C <= 8 && F >= 0.85f * (G * C) ? C : 0;
+}
+
 // How many workgroups share K in the tile form: the least that give 150 of
 // them, each with at least 384 of K (48 rows, in us: 4096 x 4096 2 shares
 // 15.1, 4 shares 12.0, 8 shares 13.7; 4096 x 14336 39, 26.7, 29.5; 5120 x
@@ -533,6 +682,12 @@ extern "C" int decode_gemm_shares(int M, int N, int K) {
     best = s;
     if (N / 64 * s >= 150) break;
   }
+  // twice as many where that makes tiles of 80 columns and more come out even (those
+  // of 64 may be: 64 rows of 4096 x 4096, 4 and 8 shares 9.6 and 11.0)
+  const int twice = best * 2;
+  if (best > 1 && N / 64 * best != 256 && M <= 64 && K % (64 * twice) == 0 &&
+      dg_even_columns(M, N, K, twice) >= 5)
+    return twice;
   return best;
 }
 
@@ -571,6 +726,15 @@ extern "C" int mid_gemm_shares(int M, int N, int K) {
     best = s;
   }
   return best;
+}
+
+template <int ACT>
+static void dg_reduce_launch(const float* slabs, int splitk, const DgEnd& e,
+                             hipStream_t st) {
+  if (splitk <= 1 || e.out == nullptr) return;
+  const long four = (long)e.M * (dg_glu(ACT) ? e.N / 2 : e.N) / 4;
+  hipLaunchKernelGGL(dg_reduce_kernel<ACT>, dim3((four + 255) / 256),
+                     dim3(256), 0, st, slabs, splitk, e);
 }
 
 template <int ACT>
@@ -615,17 +779,39 @@ static void dg_launch(const u16* X, const u16* W, float* slabs, int K,
                          dim3(MP == 32 ? 256 : 512), dg_tile_lds(MP, R), st, \
                          X, W, slabs, K, splitk, e);                         \
   } while (0)
+  if constexpr (ACT == DG_NONE || ACT == DG_F32 || GLU) {
+    const int C = tile ? 0 : dg_even_columns(e.M, e.N, K, splitk);
+    if (C > 0) {
+#define DG_EVEN(MP, CC, SL)                                                 \
+  hipLaunchKernelGGL((dg_even_kernel<ACT, MP, CC, SL>), dim3(256),          \
+                     dim3(MP * 8), dg_even_lds(MP, CC), st, X, W, slabs, K, \
+                     splitk, 256 / splitk, e)
+#define DG_EVEN_C(CC)                        \
+  case CC:                                   \
+    if (splitk == 1) {                       \
+      if (e.M <= 32) DG_EVEN(32, CC, false); \
+      else DG_EVEN(64, CC, false);           \
+    } else {                                 \
+      if (e.M <= 32) DG_EVEN(32, CC, true);  \
+      else DG_EVEN(64, CC, true);            \
+    }                                        \
+    break
+      switch (C) {
+        DG_EVEN_C(3); DG_EVEN_C(5); DG_EVEN_C(6); DG_EVEN_C(7); DG_EVEN_C(8);
+      }
+#undef DG_EVEN_C
+#undef DG_EVEN
+      dg_reduce_launch<ACT>(slabs, splitk, e, st);
+      return;
+    }
+  }
   const int rows = tile > 1 ? tile : e.M;
   if (rows <= 32) DG_TILE(32, 4);
   else if (rows <= 64) DG_TILE(64, 4);
   else if (rows <= 128) DG_TILE(128, 3);
   else DG_TILE(256, 3);
 #undef DG_TILE
-  if (splitk > 1 && e.out != nullptr) {
-    const long four = (long)e.M * (GLU ? e.N / 2 : e.N) / 4;
-    hipLaunchKernelGGL(dg_reduce_kernel<ACT>, dim3((four + 255) / 256),
-                       dim3(256), 0, st, slabs, splitk, e);
-  }
+  dg_reduce_launch<ACT>(slabs, splitk, e, st);
 }
 
 // tile: the tile form whatever M is; splitk workgroups share K there. 64: by

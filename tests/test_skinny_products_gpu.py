@@ -73,6 +73,29 @@ def test_activations(device, M, share):
            rows)
 
 
+@pytest.mark.parametrize("M", [17, 32, 33, 64])
+@pytest.mark.parametrize("N, K, shares", [
+    (12288, 512, 1), (16384 + 3072, 576, 1), (27648, 512, 1), (32768, 640, 1),
+    (6144, 2048, 4), (5120, 2048, 4), (6144, 1024, 2)])
+def test_columns_even_on_the_card(device, M, N, K, shares):
+    """48 to 128 columns a workgroup, all and some with one block less, with the
+    least sum and others, of one share and of several."""
+    run, F = ops._hip_ops.decode_gemm, torch.nn.functional
+    assert ops._hip_ops.decode_gemm_shares(M, N, K) == shares
+    x, w, b = _inputs(M, N, K, device, M + N)
+    z = x.float() @ w.float().T
+    zb = z + b.float()
+    _close(run(x, w, None, 0), z)
+    _close(run(x, w, b, 0), zb)
+    torch.testing.assert_close(run(x, w, b, 0, 9), run(x, w, b, 0).float(),
+                               atol=0, rtol=0)
+    _close(run(x, w, b, 0, 1), F.silu(zb[:, : N // 2]) * zb[:, N // 2:])
+    _close(run(x, w, b, 0, 2, 1.1, 1.702, 1.0),
+           torch_ref.clamped_glu(zb, 1.1, 1.702, 1.0).float())
+    if shares > 1:
+        _close(ops._hip_ops.decode_gemm_parts(x, w).sum(0), z)
+
+
 def test_refusals(device):
     x, w, _ = _inputs(4, 128, 128, device, 1)
     for args in ((x, w, None, 1, 1), (x, w, None, 3), (x, w, None, 0, 4),
