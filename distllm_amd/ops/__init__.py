@@ -475,7 +475,7 @@ def linear_parts(x, weight, bias=None):
             and _gemm_mode() not in _OTHER_FORMS):
         _require_hip("_hip_gemm")
         if (_few_rows(x2, weight, bias)
-                and _hip_ops.decode_gemm_shares(M, weight.shape[0], K) > 1):
+                and _hip_ops.decode_parts_shares(M, weight.shape[0], K) > 1):
             return _hip_ops.decode_gemm_parts(x2, weight)
     return linear(x2, weight, bias)
 
@@ -1232,8 +1232,8 @@ def post_norm_add(y, x, w_post, w_next, n, eps):
 
 def latent_prep(ab, q_cols, q_rank, rank, wq, wc, eps, cache, block_table,
                 row_seq, ctx):
-    """Norm both down-projections of a latent-attention layer in one
-    launch: the query latent (first q_cols columns of ab) is returned,
+    """Norm both down-projections of a latent-attention layer, ab [M, columns]
+    or what linear_parts returned, in one launch: the query latent (first q_cols columns of ab) is returned,
     the key/value latent goes straight to its cache slot (position
     ctx - 1 of block-table row row_seq; ctx 0 writes nothing). cache
     None: the layer has no latent of its own."""

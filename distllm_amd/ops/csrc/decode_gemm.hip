@@ -670,12 +670,11 @@ static int dg_even_columns(int rows, int N, int K, int splitk) {
   return C >= 3 && C != 4 && C <= 8 && F >= 0.85f * (G * C) ? C : 0;
 }
 
-// How many workgroups share K in the tile form: the least that give 150 of
+// How many workgroups share K in the tile and even forms: the least that give 150 of
 // them, each with at least 384 of K (48 rows, in us: 4096 x 4096 2 shares
 // 15.1, 4 shares 12.0, 8 shares 13.7; 4096 x 14336 39, 26.7, 29.5; 5120 x
 // 1280 9.7 and 4 shares 10.6; 16384 x 4096 none 31.3, 2 shares 34.6).
-extern "C" int decode_gemm_shares(int M, int N, int K) {
-  if (M <= 16 || (M <= 64 && dg_few_columns(M, N, K))) return 1;
+static int dg_shares(int M, int N, int K) {
   int best = 1;
   for (int s = 1; s <= 16; ++s) {
     if (K % (64 * s) != 0 || (s > 1 && K / s < 384)) continue;
@@ -689,6 +688,21 @@ extern "C" int decode_gemm_shares(int M, int N, int K) {
       dg_even_columns(M, N, K, twice) >= 5)
     return twice;
   return best;
+}
+extern "C" int decode_gemm_shares(int M, int N, int K) {
+  return M <= 16 || (M <= 64 && dg_few_columns(M, N, K)) ? 1
+                                                         : dg_shares(M, N, K);
+}
+
+// The same where what follows sums the shares as it reads them, without a launch of 4.7
+// us that joins them: of 17 to 32 rows the ring is the slower form then from 2048 x 4096
+// on. us in a graph over fresh weights, ring and tiles, 17 and 32 rows: 2048 x 4096 8.0,
+// 9.3 and 5.8, 6.1; 4096 x 4096 9.0, 11.4 and 8.5, 8.4; 4096 x 1536 5.5, 5.6 and 5.6,
+// 6.0.
+extern "C" int decode_parts_shares(int M, int N, int K) {
+  return M > 16 && M <= 32 && (long)N * K >= 2048L * 4096
+             ? dg_shares(M, N, K)
+             : decode_gemm_shares(M, N, K);
 }
 
 // Whether a product of M <= 64 rows takes the ring.
@@ -747,7 +761,7 @@ static void dg_launch(const u16* X, const u16* W, float* slabs, int K,
                      dim3(e.N / (NT * 16)), dim3(256),                       \
                      dg_ring_lds((XP + 1) / 2, NT, 4, R), st, X, W, K, e)
   // two rows of W per stage: three stages let two workgroups share a CU
-  if (!tile && decode_gemm_rings(e.M, e.N, K)) {
+  if (!tile && splitk == 1 && decode_gemm_rings(e.M, e.N, K)) {
     // (one form for 32 rows and one for 64 will do for what is seldom called)
     if constexpr (ACT == DG_NONE || ACT == DG_F32 || ACT == DG_GELU_TANH ||
                   ACT == DG_GELU_ERF) {

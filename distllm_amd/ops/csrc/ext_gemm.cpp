@@ -17,6 +17,7 @@ void launch_decode_gemm(const void*, const void*, const void*, void*, void*,
                         int, int, int, int, int, int, float, float, float,
                         const float*, const RowsArgs*, hipStream_t);
 int decode_gemm_shares(int, int, int);
+int decode_parts_shares(int, int, int);
 int mid_gemm_shares(int, int, int);
 void launch_norm_gemm(const void*, const void*, const void*, void*, float,
                       const void*, const void*, void*, int, int, int,
@@ -147,14 +148,14 @@ torch::Tensor decode_gemm(torch::Tensor X, torch::Tensor W,
 }
 
 // X W^T as the fp32 slabs [shares, M, N] of the workgroups that share K, for
-// kernels that sum them as they read; shares > 1 (decode_gemm_shares).
+// kernels that sum them as they read; shares > 1 (decode_parts_shares).
 torch::Tensor decode_gemm_parts(torch::Tensor X, torch::Tensor W) {
   CHECK_DEV(X); CHECK_CONT(X); CHECK_BF16(X);
   CHECK_DEV(W); CHECK_CONT(W); CHECK_BF16(W);
   const int M = X.size(0), K = X.size(1), N = W.size(0);
   TORCH_CHECK(W.size(1) == K, "K mismatch");
   TORCH_CHECK(M > 0 && M <= 256 && N % 64 == 0 && K % 64 == 0, "shape");
-  const int shares = decode_gemm_shares(M, N, K);
+  const int shares = decode_parts_shares(M, N, K);
   TORCH_CHECK(shares > 1, "K is not shared at this shape");
   X = aligned16(X);
   W = aligned16(W);
@@ -414,6 +415,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("norm_gemm", &norm_gemm);
   m.def("decode_gemm_parts", &decode_gemm_parts);
   m.def("decode_gemm_shares", &decode_gemm_shares);
+  m.def("decode_parts_shares", &decode_parts_shares);
   m.def("decode_gemm_rows", &decode_gemm_rows);
   m.def("gelu_rows", &gelu_rows);
   m.def("clamped_glu", &clamped_glu);

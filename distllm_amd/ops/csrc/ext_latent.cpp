@@ -7,6 +7,10 @@ void launch_latent_prep(const void*, int, int, int, int, int, int,
                         const float*, const float*, float, void*, void*,
                         const int*, int, int, const int*, const int*, bool,
                         hipStream_t);
+void launch_latent_prep_parts(const float*, int, int, int, int, int, int, int,
+                              const float*, const float*, float, void*, void*,
+                              const int*, int, int, const int*, const int*,
+                              hipStream_t);
 void launch_latent_gather(const void*, const int*, int, int, const int*,
                           const int*, void*, void*, int, int, int,
                           hipStream_t);
@@ -58,7 +62,10 @@ torch::Tensor latent_prep(torch::Tensor ab, int64_t QP, int64_t qn,
                           torch::Tensor ctx) {
   CHECK_DEV(ab); CHECK_CONT(ab); CHECK_T(ab);
   CHECK_DEV(wq); CHECK_CONT(wq); CHECK_F32(wq);
-  const int M = ab.size(0), ld = ab.size(1);
+  // the slabs of a product whose K was shared stand for bf16 numbers
+  const bool parts = ab.dim() == 3;
+  TORCH_CHECK(parts ? is_f32(ab) && ab.size(0) > 0 : ab.dim() == 2, "ab");
+  const int M = ab.size(parts), ld = ab.size(parts + 1);
   const int R = ld - (int)QP;
   TORCH_CHECK(R >= 0 && wq.numel() == QP && qn > 0 && qn <= QP, "q sizes");
   TORCH_CHECK(QP % 8 == 0 && QP <= 8192 && R <= 8192,
@@ -68,7 +75,11 @@ torch::Tensor latent_prep(torch::Tensor ab, int64_t QP, int64_t qn,
   int nblk = 0;
   if (cache) {
     check_pages(cache.value(), bt, row_seq, ctx, M);
-    CHECK_SAME(ab, cache.value());
+    if (parts) {
+      CHECK_DEV(cache.value()); CHECK_BF16(cache.value());
+    } else {
+      CHECK_SAME(ab, cache.value());
+    }
     TORCH_CHECK(cache->size(2) == R && rn > 0 && rn <= R, "rank");
     TORCH_CHECK(wc.has_value() && wc->numel() == R, "latent norm size");
     CHECK_DEV(wc.value()); CHECK_CONT(wc.value()); CHECK_F32(wc.value());
@@ -78,8 +89,16 @@ torch::Tensor latent_prep(torch::Tensor ab, int64_t QP, int64_t qn,
   } else {
     TORCH_CHECK(R == 0, "latent columns without a cache");
   }
-  auto cq = torch::empty({M, QP}, ab.options());
-  if (M > 0)
+  auto cq = torch::empty(
+      {M, QP}, parts ? ab.options().dtype(at::kBFloat16) : ab.options());
+  if (M > 0 && parts) {
+    TORCH_CHECK((uintptr_t)ab.data_ptr() % 16 == 0 && ld % 4 == 0, "slabs");
+    launch_latent_prep_parts(
+        ab.data_ptr<float>(), (int)ab.size(0), M, ld, (int)QP, (int)qn, R,
+        (int)rn, wq.data_ptr<float>(), wcp, (float)eps, cq.data_ptr(), cp,
+        bt.data_ptr<int>(), bt.size(1), nblk, row_seq.data_ptr<int>(),
+        ctx.data_ptr<int>(), cur_stream());
+  } else if (M > 0)
     launch_latent_prep(ab.data_ptr(), M, ld, (int)QP, (int)qn, R, (int)rn,
                        wq.data_ptr<float>(), wcp, (float)eps, cq.data_ptr(),
                        cp, bt.data_ptr<int>(), bt.size(1), nblk,

@@ -14,6 +14,8 @@
 // Every row of a batch is one token: row_seq[row] is its block-table row,
 // ctx[row] its position + 1 (0: padding row, nothing is read or written).
 // A row sees the last `window` positions up to its own.
+#include <algorithm>
+
 #include "common.h"
 
 #define PBLK 16  // tokens per cache block
@@ -81,6 +83,88 @@ latent_prep_kernel(const T* __restrict__ ab, int ld, int QP, int qn, int R,
       store8(dst + c, v[k]);
     }
   }
+}
+
+// The same on the fp32 slabs [S, rows, ld] of a product whose K was shared, whose sums
+// are rounded to bf16 as the product's are: a workgroup for each row's query latent and
+// one for its cached latent, eight columns a thread, four slabs on their way at once.
+template <int NC>
+__global__ void __launch_bounds__(256)
+latent_prep_parts_kernel(const float* __restrict__ ab, int S, int ld, int QP,
+                         int qn, int R, int rn, const float* __restrict__ wq,
+                         const float* __restrict__ wc, float eps,
+                         unsigned short* __restrict__ cq,
+                         unsigned short* __restrict__ cache,
+                         const int* __restrict__ block_table, int max_blocks,
+                         int num_blocks, const int* __restrict__ row_seq,
+                         const int* __restrict__ ctx) {
+  __shared__ float red[4];
+  const int row = blockIdx.x, tid = threadIdx.x;
+  const bool latent = blockIdx.y != 0;
+  const int n = latent ? rn : qn, np = latent ? R : QP;
+  const float* src = ab + (long)row * ld + (latent ? QP : 0);
+  const float* w = latent ? wc : wq;
+  const long slab = (long)gridDim.x * ld;
+  unsigned short* dst = cq + (long)row * QP;
+  if (latent) {
+    const int pos = ctx[row] - 1;
+    if (pos < 0 || pos / PBLK >= max_blocks) return;
+    const int blk = block_table[(long)row_seq[row] * max_blocks + pos / PBLK];
+    if (blk < 0 || blk >= num_blocks) return;
+    dst = cache + ((long)blk * PBLK + pos % PBLK) * R;
+  }
+  float v[NC][8], wv[NC][8];
+  float ss = 0.f;
+#pragma unroll
+  for (int k = 0; k < NC; ++k) {
+    const int c = (k * 256 + tid) * 8;
+    if (c >= np) continue;
+    load8<float>(w + c, wv[k]);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[k][i] = 0.f;
+    for (int s0 = 0; s0 < S; s0 += 4) {
+      float t[4][8];
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+        load8<float>(src + min(s0 + s, S - 1) * slab + c, t[s]);
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          v[k][i] = s0 + s < S ? v[k][i] + t[s][i] : v[k][i];
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      v[k][i] = bf2f(f2bf(v[k][i]));
+      ss += v[k][i] * v[k][i];
+    }
+  }
+  const float inv = 1.f / sqrtf(block_reduce_sum<4>(ss, red) / n + eps);
+#pragma unroll
+  for (int k = 0; k < NC; ++k) {
+    const int c = (k * 256 + tid) * 8;
+    if (c < np) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[k][i] *= inv * wv[k][i];
+      store8(dst + c, v[k]);
+    }
+  }
+}
+
+extern "C" void launch_latent_prep_parts(
+    const float* ab, int S, int M, int ld, int QP, int qn, int R, int rn,
+    const float* wq, const float* wc, float eps, void* cq, void* cache,
+    const int* block_table, int max_blocks, int num_blocks,
+    const int* row_seq, const int* ctx, hipStream_t stream) {
+  const dim3 grid(M, cache != nullptr ? 2 : 1);
+#define LPP(NC)                                                              \
+  hipLaunchKernelGGL((latent_prep_parts_kernel<NC>), grid, dim3(256), 0,     \
+                     stream, ab, S, ld, QP, qn, R, rn, wq, wc, eps,          \
+                     (unsigned short*)cq, (unsigned short*)cache,            \
+                     block_table, max_blocks, num_blocks, row_seq, ctx)
+  if (std::max(QP, R) <= 2048) LPP(1);
+  else LPP(4);
+#undef LPP
 }
 
 extern "C" void launch_latent_prep(

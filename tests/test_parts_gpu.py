@@ -115,3 +115,55 @@ def test_gated_bias_fp8(device, rows, K):
     want = torch.nn.functional.silu(z[:, : N // 2]) * z[:, N // 2:]
     # the output's bf16, and at other K that of gate and up before the product
     torch.testing.assert_close(got.double(), want, rtol=2 ** -6, atol=2e-2)
+
+
+@pytest.mark.parametrize("M", [17, 32])
+@pytest.mark.parametrize("N, K, shares", [(4096, 4096, 4), (2048, 4096, 8),
+                                          (2048, 4032, 1), (4096, 2048, 4)])
+def test_shares_in_place_of_the_ring(device, M, N, K, shares):
+    """Products that a launch of their own would not share K for."""
+    x, w = _rand(M, K), _rand(N, K, seed=1)
+    assert ops._hip_ops.decode_gemm_shares(M, N, K) == 1
+    got = ops.linear_parts(x, w)
+    assert got.shape == ((shares, M, N) if shares > 1 else (M, N))
+    want = x.double() @ w.double().t()
+    total = (got.sum(0) if shares > 1 else got).double()
+    bound = (x.double().abs() @ w.double().abs().t()) * K * 2 ** -24
+    if shares == 1:
+        bound += want.abs() * 2 ** -8
+    assert ((total - want).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("S", [2, 3, 8])
+@pytest.mark.parametrize("QP, qn, R, rn", [(128, 100, 192, 130),
+                                           (1536, 1536, 512, 512),
+                                           (4096, 4000, 2112, 2100)])
+def test_latent_prep(device, S, QP, qn, R, rn):
+    """Both norms of the sum of slabs against those of the sum in bf16; a row
+    without a place in the cache writes nothing."""
+    M = 5
+    ab = torch.randn(S, M, QP + R, device="cuda")
+    ab[:, :, qn:QP] = 0
+    ab[:, :, QP + rn:] = 0
+    wq, wc = torch.randn(QP, device="cuda"), torch.randn(R, device="cuda")
+    bt = torch.tensor([[3, 1, 0], [5, 2, 4]], dtype=torch.int32, device="cuda")
+    seq = torch.tensor([0, 0, 1, 0, 1], dtype=torch.int32, device="cuda")
+    ctx = torch.tensor([40, 17, 7, 0, 1], dtype=torch.int32, device="cuda")
+    total = ab[0].clone()
+    for s in range(1, S):
+        total += ab[s]
+    out = []
+    for x in (ab, total.to(BF16)):
+        cache = torch.zeros(6, 16, R, dtype=BF16, device="cuda")
+        cq = ops.latent_prep(x, QP, qn, rn, wq, wc, 1e-3, cache, bt, seq, ctx)
+        out.append((cq, cache))
+    for a, b in zip(*out):
+        # the squares are summed in another order: the last of bf16's 7 bits
+        torch.testing.assert_close(a, b, rtol=2 ** -7, atol=1e-6)
+        assert torch.equal(a == 0, b == 0)
+    alone = ops.latent_prep(ab[:, :, :QP].contiguous(), QP, qn, rn, wq, None,
+                            1e-3, None, bt, seq, ctx)
+    assert torch.equal(alone, out[0][0])
+    with pytest.raises(RuntimeError):
+        ops.latent_prep(ab, QP, qn, rn, wq, wc, 1e-3, cache.float(), bt, seq,
+                        ctx)
