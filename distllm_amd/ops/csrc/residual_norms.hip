@@ -17,7 +17,7 @@
 // with zeros to W columns. T is the type of y, h and E (bf16 or fp32).
 #include "common.h"
 
-// sum over the TPR threads (one or four waves) that share a row
+// sum over the TPR threads (one, four or eight waves) that share a row
 template <int TPR>
 __device__ __forceinline__ float row_sum(float v, float* scratch) {
   v = wave_reduce_sum(v);
@@ -26,7 +26,10 @@ __device__ __forceinline__ float row_sum(float v, float* scratch) {
   __syncthreads();  // the previous use of scratch is over
   if ((threadIdx.x & 63) == 0) scratch[wid] = v;
   __syncthreads();
-  return scratch[0] + scratch[1] + scratch[2] + scratch[3];
+  float sum = scratch[0] + scratch[1] + scratch[2] + scratch[3];
+#pragma unroll
+  for (int w = 4; w < TPR / 64; ++w) sum += scratch[w];
+  return sum;
 }
 
 // PARTS: y are the S fp32 slabs [S, M, W] of a product whose K was shared, summed
@@ -34,21 +37,35 @@ __device__ __forceinline__ float row_sum(float v, float* scratch) {
 // 32 rows of 4096, four slabs, 9.8 -> 6.8 us; steps of 8 layers (one such product a
 // layer, two from 33 rows on) of 20 sequences 1419 -> 1412 us, 32 1564 -> 1550, 64
 // 1929 -> 1902.
-template <typename T, int NC, int TPR, bool EMBED, bool PARTS>
-__global__ void __launch_bounds__(256)
+// FEW: of rows that leave CUs idle all is asked for at once, also what the sums are
+// followed by, and a row has eight waves: 32 rows of 4096, four slabs, 6.4 -> 4.8 us.
+template <typename T, int NC, int TPR, bool EMBED, bool PARTS, bool FEW = false>
+__global__ void __launch_bounds__(TPR == 512 ? 512 : 256)
 sandwich_norm_kernel(const T* __restrict__ y, const long* __restrict__ tokens,
                      float* __restrict__ x, const float* __restrict__ w_post,
                      const float* __restrict__ w_next, T* __restrict__ h,
                      int M, int W, int n, float eps, int S) {
-  __shared__ float scratch[4];
+  __shared__ float scratch[8];
   const int sub = threadIdx.x % TPR;
-  const int row = blockIdx.x * (256 / TPR) + threadIdx.x / TPR;
-  if (row >= M) return;  // whole waves; whole blocks when TPR == 256
+  const int row = TPR == 512 ? blockIdx.x
+                             : blockIdx.x * (256 / TPR) + threadIdx.x / TPR;
+  if (row >= M) return;  // whole waves; whole blocks from TPR == 256 on
   const T* yr = y + (EMBED ? tokens[row] : (long)row) * W;
   float* xr = x + (long)row * W;
 
   float v[NC][8];
   float ss = 0.f;
+  float xs[NC][8], wp[NC][8], wn[NC][8];
+  if constexpr (FEW)
+#pragma unroll
+    for (int k = 0; k < NC; ++k) {
+      const int c = (sub + k * TPR) * 8;
+      if (c < W) {
+        load8<float>(xr + c, xs[k]);
+        load8<float>(w_post + c, wp[k]);
+        load8<float>(w_next + c, wn[k]);
+      }
+    }
 #pragma unroll
   for (int k = 0; k < NC; ++k) {
     const int c = (sub + k * TPR) * 8;
@@ -87,11 +104,14 @@ sandwich_norm_kernel(const T* __restrict__ y, const long* __restrict__ tokens,
       const int c = (sub + k * TPR) * 8;
       if (c < W) {
         float xv[8], wv[8];
-        load8<float>(xr + c, xv);
-        load8<float>(w_post + c, wv);
+        if constexpr (!FEW) {
+          load8<float>(xr + c, xv);
+          load8<float>(w_post + c, wv);
+        }
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-          v[k][i] = xv[i] + v[k][i] * inv * wv[i];
+          v[k][i] = (FEW ? xs[k][i] : xv[i]) +
+                    v[k][i] * inv * (FEW ? wp[k][i] : wv[i]);
           ss += v[k][i] * v[k][i];
         }
       }
@@ -104,9 +124,10 @@ sandwich_norm_kernel(const T* __restrict__ y, const long* __restrict__ tokens,
     const int c = (sub + k * TPR) * 8;
     if (c < W) {
       float wv[8], o[8];
-      load8<float>(w_next + c, wv);
+      if constexpr (!FEW) load8<float>(w_next + c, wv);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) o[i] = v[k][i] * inv * wv[i];
+      for (int i = 0; i < 8; ++i)
+        o[i] = v[k][i] * inv * (FEW ? wn[k][i] : wv[i]);
       store8(xr + c, v[k]);
       store8(h + (long)row * W + c, o);
     }
@@ -125,6 +146,24 @@ extern "C" void launch_sandwich_norm(const void* y, int shares,
   const int rows = 256 / tpr;
   const dim3 grid((M + rows - 1) / rows);
   const int nc = (W / 8 + tpr - 1) / tpr;
+  if (tokens == nullptr && !fp32 && M <= 256 && W > 1024 && W <= 8192) {
+#define SN_FEW(NC, TPR, PA)                                                   \
+  hipLaunchKernelGGL(                                                         \
+      (sandwich_norm_kernel<unsigned short, NC, TPR, false, PA, true>),       \
+      dim3(M), dim3(TPR), 0, stream, (const unsigned short*)y, tokens, x,     \
+      w_post, w_next, (unsigned short*)h, M, W, n, eps, shares)
+#define SN_FEW_P(NC, TPR)                    \
+  do {                                       \
+    if (shares > 0) SN_FEW(NC, TPR, true);   \
+    else SN_FEW(NC, TPR, false);             \
+  } while (0)
+    if (W <= 2048) SN_FEW_P(1, 256);
+    else if (W <= 4096) SN_FEW_P(1, 512);
+    else SN_FEW_P(2, 512);
+#undef SN_FEW_P
+#undef SN_FEW
+    return;
+  }
 #define SN(T, NC, TPR, EM, PA)                                                \
   hipLaunchKernelGGL((sandwich_norm_kernel<T, NC, TPR, EM, PA>), grid,        \
                      dim3(256), 0, stream, (const T*)y, tokens, x, w_post,    \
