@@ -156,6 +156,23 @@ __device__ __forceinline__ void copy_to_lds(const void* from,
       : "memory");
 }
 
+// The same from a buffer, 16 bytes a lane from byte lane_at + at of it on, and known to
+// the compiler: loads ahead of it that it waits for do not wait for the copies. (As
+// global_load_lds a copy may be one of LDS to the compiler's counts, and it then waits
+// for all that is in flight.)
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t weight_rows(const void* from,
+                                                              int bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(from), 0, bytes,
+                                           0x00020000);
+}
+__device__ __forceinline__ void copy_rows_to_lds(__amdgpu_buffer_rsrc_t from,
+                                                 int lane_at, int at,
+                                                 char* base) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(
+      from, (__attribute__((address_space(3))) void*)base, 16, lane_at, at, 0,
+      0);
+}
+
 // 16 bytes at any address
 typedef __attribute__((ext_vector_type(4), aligned(1))) int i32x4_any;
 

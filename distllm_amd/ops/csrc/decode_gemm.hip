@@ -269,18 +269,18 @@ dg_norm_ring_kernel(const NormRow n, const u16* __restrict__ W, int K,
   constexpr bool GLU = dg_glu(ACT);
   constexpr int NW = 4, R = dg_norm_ring(NT);
   constexpr int STAGE = NT * 2048, LOADS = NT * 2;
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, g = lane >> 4;
   const int n0 = blockIdx.x * (GLU ? NT * 8 : NT * 16);
   char* hs = smem + 128;
   char* ring = hs + K * 2 + wid * R * STAGE;
-  const int lr = lane >> 3, lc = ((lane & 7) ^ lr) * 8;
-  const u16* src[NT][2];
+  const int lr = lane >> 3;
+  const int lane_at = lr * K * 2 + ((lane & 7) ^ lr) * 16;
+  __amdgpu_buffer_rsrc_t src[NT];  // 16 rows of W
 #pragma unroll
-  for (int p = 0; p < 2; ++p)
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-      src[t][p] = W + (long)(dg_wrow<GLU>(n0, t, e.N) + p * 8 + lr) * K + lc;
+  for (int t = 0; t < NT; ++t)
+    src[t] = weight_rows(W + (long)dg_wrow<GLU>(n0, t, e.N) * K, 32 * K);
   // chunks wid, wid + NW, ... from the block's first one on
   const int nch = K / 64, mine = (nch - wid + NW - 1) / NW;
   const int turn = chunk_turn<37>(blockIdx.x, nch) + wid;
@@ -289,13 +289,14 @@ dg_norm_ring_kernel(const NormRow n, const u16* __restrict__ W, int K,
     return k >= nch ? k - nch : k;
   };
   auto issue = [&](int c) {
-    char* dst = ring + (c % R) * STAGE + lane * 16;
-    const long k = chunk(c) * 64;
+    char* dst = ring + (c % R) * STAGE;
+    const int k = chunk(c) * 128;
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
       for (int p = 0; p < 2; ++p)
-        dg_copy(src[t][p] + k, dst + t * 2048 + p * 1024);
+        copy_rows_to_lds(src[t], lane_at, k + p * 16 * K,
+                         dst + t * 2048 + p * 1024);
   };
   norm_row<NC>(n, K, reinterpret_cast<float*>(smem), hs, [&]() {
 #pragma unroll

@@ -44,26 +44,23 @@ __device__ __forceinline__ void lds_barrier() {
 
 // The workgroup's 16 rows of W, as chunks of 64 columns, by copies of 1 KiB.
 // Straight-line code: a wave without a CP-th piece copies the last once more.
-// KNOWN: by the builtin, so that waits for loads ahead of them do not wait for
+// KNOWN: to the compiler, so that waits for loads ahead of them do not wait for
 // them, too; not where others are by copy_to_lds.
 template <int CP, bool KNOWN>
 __device__ __forceinline__ void start_weights(const u16* W, int H, char* ws) {
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lr = lane >> 3, lc = ((lane & 7) ^ lr) * 8;
+  const u16* rows = W + (long)blockIdx.x * COLS * H;
+  const __amdgpu_buffer_rsrc_t buffer = weight_rows(rows, COLS * H * 2);
 #pragma unroll
   for (int i = 0; i < CP; ++i) {
     const int p = min(wid + i * NW, H / 32 - 1);
-    const u16* src = W + (long)(blockIdx.x * COLS + (p & 1) * 8 + lr) * H +
-                     (p >> 1) * 64 + lc;
+    const int at = (p & 1) * 8 * H + (p >> 1) * 64;
     if constexpr (KNOWN)
-      __builtin_amdgcn_global_load_lds(
-          (const __attribute__((address_space(1))) unsigned int*)src,
-          (__attribute__((address_space(3))) unsigned int*)(ws + p * 1024 +
-                                                            lane * 16),
-          16, 0, 0);
+      copy_rows_to_lds(buffer, (lr * H + lc) * 2, at * 2, ws + p * 1024);
     else
-      copy_to_lds(src, ws + p * 1024);
+      copy_to_lds(rows + at + lr * H + lc, ws + p * 1024);
   }
 }
 

@@ -233,7 +233,8 @@ gemv_fp8_norm_kernel(const NormRow nr, const unsigned char* __restrict__ W,
                      unsigned short* __restrict__ OUT, int N, int K) {
   constexpr int NT = GLU ? 2 : 1, R = gv_norm_ring(GLU);
   constexpr int STAGE = NT * 2048, LOADS = NT * 2;
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, g = lane >> 4;
   const int cols = GLU ? N / 2 : N, n0 = blockIdx.x * 16;
   char* hs = smem + 128;
@@ -245,28 +246,25 @@ gemv_fp8_norm_kernel(const NormRow nr, const unsigned char* __restrict__ W,
     const int k = c * 4 + turn;
     return k >= nch ? k - nch : k;
   };
-  const unsigned char* src[NT][2];
+  const int rows = min(16, cols - n0);
+  int lane_at[2];
 #pragma unroll
   for (int p = 0; p < 2; ++p) {
     const int row = p * 8 + (lane >> 3);
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-      src[t][p] = W + (long)(min(n0 + row, cols - 1) + t * cols) * K +
-                  ((lane & 7) ^ (row & 7)) * 16;
+    lane_at[p] = min(row, rows - 1) * K + ((lane & 7) ^ (row & 7)) * 16;
   }
+  __amdgpu_buffer_rsrc_t src[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+    src[t] = weight_rows(W + (long)(n0 + t * cols) * K, rows * K);
   auto issue = [&](int c) {
-    char* dst = ring + (c % R) * STAGE + lane * 16;
-    const long k = chunk(c) * 128;
+    char* dst = ring + (c % R) * STAGE;
+    const int k = chunk(c) * 128;
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
       for (int p = 0; p < 2; ++p)
-        __builtin_amdgcn_global_load_lds(
-            (const __attribute__((address_space(1))) unsigned int*)(
-                src[t][p] + k),
-            (__attribute__((address_space(3))) unsigned int*)(
-                dst + (t * 2 + p) * 1024),
-            16, 0, 0);
+        copy_rows_to_lds(src[t], lane_at[p], k, dst + (t * 2 + p) * 1024);
   };
   norm_row<NC>(nr, K, reinterpret_cast<float*>(smem), hs, [&]() {
 #pragma unroll
