@@ -276,7 +276,9 @@ attn_rows_kernel(const u16* __restrict__ qkv, const float* __restrict__ mask,
     const int b = u / heads, head = u % heads;
     const u16* base = qkv + (long)b * S * ld + head * 64;
     char* qs = xs + (head * MR + b * S) * 128;
-    const float mine = mask[b * S + at];
+    // (by a copy, too: for a load the compiler would wait until nothing is in
+    // flight, the weights among it)
+    if (lane < 32) copy_to_lds<4>(mask + b * S + at, ms);
     for (int p = 0; p < SR / 8; ++p) {
       const int row = p * 8 + lr;
       const u16* src = base + min(row, S - 1) * ld;
@@ -294,7 +296,7 @@ attn_rows_kernel(const u16* __restrict__ qkv, const float* __restrict__ mask,
     } else {
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     }
-    if (lane < 32) ms[lane] = q < S ? mine * LOG2E : -INFINITY;
+    if (lane < 32) ms[lane] = q < S ? ms[lane] * LOG2E : -INFINITY;
     wave_sync();
 
     f32x16 sc = {};
