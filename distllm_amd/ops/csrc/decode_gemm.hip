@@ -124,7 +124,7 @@ __device__ __forceinline__ int dg_wrow(int block0, int t16, int N) {
 
 // The sums of the NW waves that share K, added up: 16 x 16 tiles in LDS,
 // [wave][NT][MT], of which this wave has COUNT from `first` on.
-template <int ACT, int MT, int NT, int NW, int COUNT = 1>
+template <int ACT, int MT, int NT, int NW, int COUNT = 1, bool HALF = false>
 __device__ __forceinline__ void dg_join(const DgEnd& e, int n0, int first,
                                         const f32x4* acc) {
   constexpr bool GLU = dg_glu(ACT);
@@ -138,7 +138,7 @@ __device__ __forceinline__ void dg_join(const DgEnd& e, int n0, int first,
   for (int k = threadIdx.x; k < UNITS; k += blockDim.x) {
     const int l = k & 63, tj = (k >> 6) % MT, ti = (k >> 6) / MT;
     const int m = tj * 16 + (l & 15);
-    if (m >= e.M) continue;
+    if (m >= e.M || (HALF && l >= 32)) continue;
     f32x4 v = {0.f, 0.f, 0.f, 0.f}, u = v;
 #pragma unroll
     for (int w = 0; w < NW; ++w) {
@@ -163,16 +163,24 @@ constexpr int dg_ring_lds(int MT, int NT, int NW, int R) {
 // or 64 copied and those that are: 768 x 3072, 1 row 4.12 and 4.00, 24 5.03 and 4.87,
 // 40 6.98 and 6.04, 48 7.03 and 6.46; 2304 x 768, 24 3.31 and 3.30, 40 3.85 and 3.56;
 // 2048 x 2048, 1 4.37 and 4.24, 40 6.90 and 6.49; 4096 x 14336, 1 23.3 and 23.1.
-template <int ACT, int XP, int NT, int NW, int R>
+// HALF: 8 columns a workgroup, where those of all still fit the card at once. Half of
+// the matrix cores' rows are for nothing, but a CU takes in less: us as above, 16 and 8
+// columns, 1, 8, 24, 64 rows: 768 x 3072 4.6, 5.1, 6.6, 10.1 and 4.5, 4.6, 5.8, 9.4; 768
+// x 768 2.7, 2.8, 3.1, 3.9 and 2.7, 2.8, 3.0, 3.8; 1024 x 4096 5.5, 6.0, 7.9, 12.1 and
+// 5.3, 5.4, 6.9, 11.3; 2048 x 2048 4.3, 4.6, 5.5, 7.7 and 4.1, 4.2, 5.0, 7.4; in two
+// rounds, 2304 x 768, 2.8, 2.9, 3.2, 4.0 and 2.9, 3.0, 4.6, 6.1.
+template <int ACT, int XP, int NT, int NW, int R, bool HALF = false>
 __global__ void __launch_bounds__(NW * 64)
 dg_ring_kernel(const u16* __restrict__ X, const u16* __restrict__ W, int K,
                const DgEnd e) {
   constexpr bool GLU = dg_glu(ACT);
   constexpr int MT = (XP + 1) / 2;
-  constexpr int STAGE = (NT + MT) * 2048, LOADS = NT * 2 + XP;
+  constexpr int WP = HALF ? 1 : 2;  // eights of rows of W
+  static_assert(!HALF || (NT == 1 && !GLU), "one half of 16 columns");
+  constexpr int STAGE = (NT + MT) * 2048, LOADS = NT * WP + XP;
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   const int r = lane & 15, g = lane >> 4;
-  const int n0 = blockIdx.x * (GLU ? NT * 8 : NT * 16);
+  const int n0 = blockIdx.x * (GLU || HALF ? NT * 8 : NT * 16);
   char* ring = smem + wid * R * STAGE;
   const int lr = lane >> 3, lc = ((lane & 7) ^ lr) * 8;
   const u16* src[NT + MT][2];
@@ -197,7 +205,7 @@ dg_ring_kernel(const u16* __restrict__ X, const u16* __restrict__ W, int K,
     for (int t = 0; t < NT + MT; ++t)
 #pragma unroll
       for (int p = 0; p < 2; ++p)
-        if (t < NT || (t - NT) * 2 + p < XP)
+        if (t < NT ? p < WP : (t - NT) * 2 + p < XP)
           dg_copy(src[t][p] + (long)k * 64, dst + t * 2048 + p * 1024);
   };
   f32x4 acc[NT][MT];
@@ -247,7 +255,7 @@ dg_ring_kernel(const u16* __restrict__ X, const u16* __restrict__ W, int K,
     for (int c = 0; c < mine; ++c) compute(c);
   }
   __syncthreads();
-  dg_join<ACT, MT, NT, NW, NT * MT>(e, n0, wid * NT * MT, &acc[0][0]);
+  dg_join<ACT, MT, NT, NW, NT * MT, HALF>(e, n0, wid * NT * MT, &acc[0][0]);
 }
 
 // ---- ring with the norm ahead of the product --------------------------------
@@ -763,6 +771,23 @@ static void dg_launch(const u16* X, const u16* W, float* slabs, int K,
                      dg_ring_lds((XP + 1) / 2, NT, 4, R), st, X, W, K, e)
   // two rows of W per stage: three stages let two workgroups share a CU
   if (!tile && splitk == 1 && decode_gemm_rings(e.M, e.N, K)) {
+    if constexpr (ACT == DG_NONE)
+      if (e.N <= 2048) {
+#define DG_HALF(XP, R)                                                       \
+  hipLaunchKernelGGL((dg_ring_kernel<ACT, XP, 1, 4, R, true>),               \
+                     dim3(e.N / 8), dim3(256),                               \
+                     dg_ring_lds((XP + 1) / 2, 1, 4, R), st, X, W, K, e)
+        if (e.M <= 8) DG_HALF(1, 4);
+        else if (e.M <= 16) DG_HALF(2, 4);
+        else if (e.M <= 24) DG_HALF(3, 4);
+        else if (e.M <= 32) DG_HALF(4, 4);
+        else if (e.M <= 40) DG_HALF(5, 4);
+        else if (e.M <= 48) DG_HALF(6, 4);
+        else if (e.M <= 56) DG_HALF(7, 3);
+        else DG_HALF(8, 3);
+#undef DG_HALF
+        return;
+      }
     // (one form for 32 rows and one for 64 will do for what is seldom called)
     if constexpr (ACT == DG_NONE || ACT == DG_F32 || ACT == DG_GELU_TANH ||
                   ACT == DG_GELU_ERF) {
