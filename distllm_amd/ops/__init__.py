@@ -941,7 +941,7 @@ class NarrowRows(NamedTuple):
 
 
 def narrow_rows(corpus):
-    """NarrowRows of a corpus [N, K] on a GPU, for score_topk; None where they
+    """NarrowRows of a corpus [N, K] on a GPU, for found_narrow; None where they
     would be of no use or there is no room for them: numbers that are infinite
     or NaN, rows whose lengths differ so much that what the longest loses in 16
     bits hides the others, more than an eighth of the memory that is free."""
@@ -968,33 +968,29 @@ def narrow_rows(corpus):
                        version) if norm <= 4 * usual else None)
 
 
-def _narrow_fills(Q, N, K):
-    """Whether score_topk_narrow is faster than score_topk. Measured over 1 to 256
-    queries, 2000 to 250000 rows of 384 and 768, k = 10, own time over its: from
-    five queries on 0.36 to 0.95. Up to four, which score_topk answers by one
-    launch beside its own choice, by the bytes of the rows: from 15 million
-    numbers on 0.52 to 0.95 (two of 20000 rows of 384 1.0), below 10000 rows,
-    where score_topk asks the library, 0.45 to 0.5, between 0.85 to 1.1."""
-    if N < 2048:
-        return False
-    return Q > 4 or N * K >= 15_000_000 or N < 10000
+def _narrow_fills(Q, N):
+    """Whether found_narrow is faster than score_topk of queries copied to the
+    GPU and found_lists of that. Measured over 64 to 250000 rows of 384 and 768,
+    k = 10, own time over theirs: 1 to 4 queries 0.45 to 0.73, 5 to 256 0.32 to
+    0.83, 1000 of 2000 rows on 0.63 to 0.99, of fewer rows 0.94 to 1.08."""
+    return Q <= 256 or N >= 2048
 
 
-def score_topk_narrow(q, corpus, k, narrow):
-    """score_topk by way of the corpus's NarrowRows: None where that is not
-    the faster way, and indices of -2^31 for queries that these cannot answer."""
+def found_narrow(q, corpus, k, narrow):
+    """found_lists of score_topk for queries [Q, K] of the host, by way of the
+    corpus's NarrowRows: None where that is not the faster way, or these cannot
+    answer a query."""
     Q, K = q.shape
     N = corpus.shape[0]
     if not (0 < Q < 1 << 20 and 0 < k <= min(60, N)
-            and q.dtype == torch.float32 and q.device == corpus.device
+            and q.dtype == torch.float32 and q.device.type == "cpu"
             and tuple(corpus.shape[1:]) == (K,) and narrow.holds(corpus)
-            and _narrow_fills(Q, N, K) and q.is_contiguous()
-            and q.data_ptr() % 16 == 0
+            and _narrow_fills(Q, N) and q.is_contiguous()
             and 0 < _hip_ops.narrow_bytes(Q, N, K, narrow.rows.shape[1])
             <= 1 << 31):
         return None
-    return _hip_ops.narrow_topk(q, corpus, narrow.rows, narrow.up,
-                                narrow.error, narrow.norm, k)
+    return _hip_ops.narrow_found(q, corpus, narrow.rows, narrow.up,
+                                 narrow.error, narrow.norm, k)
 
 
 def score_topk(q, corpus, k):
@@ -1073,12 +1069,11 @@ def topk(scores, k, chunk=1 << 15):
     return torch_ref.topk(scores, min(k, scores.shape[1]))
 
 
-def found_lists(v, i, sure=False):
+def found_lists(v, i):
     """Scores and indices [Q, k] on a GPU (float32, int32) as lists of their
-    rows, without the entries whose index is negative; sure: None where one is
-    -2^31 (score_topk_narrow)."""
+    rows, without the entries whose index is negative."""
     _require_hip()
-    return _hip_ops.found_lists(v, i, sure)
+    return _hip_ops.found_lists(v, i)
 
 
 def hamming_score(qcodes, codes_t):

@@ -120,20 +120,22 @@ struct NarrowRows {
 };
 
 // A query as f16, by one wave: times the power of two that brings its largest number to
-// 2^13, zeros behind K, as put(column, four numbers) for KP columns. The margin (see
+// 2^13, zeros behind K, as put(column, four numbers) for KP columns; first as it is to
+// `copy`, from where it is read again (q may be memory of the host). The margin (see
 // above) of products of the scaled numbers, infinite where it cannot be said.
 template <class F>
-__device__ __forceinline__ float narrow_query(const float* q,
+__device__ __forceinline__ float narrow_query(const float* q, float* copy,
                                               const NarrowRows& c, F put) {
   const int lane = threadIdx.x & 63;
   auto four = [&](int i) {
-    const f32x4 x = *reinterpret_cast<const f32x4*>(q + min(i, c.K - 4));
+    const f32x4 x = *reinterpret_cast<const f32x4*>(copy + min(i, c.K - 4));
     return i < c.K ? x : f32x4{0.f, 0.f, 0.f, 0.f};
   };
   int bits = 0;
 #pragma unroll 3
-  for (int i = lane * 4; i < c.KP; i += 256) {
-    const f32x4 x = four(i);
+  for (int i = lane * 4; i < c.K; i += 256) {
+    const f32x4 x = *reinterpret_cast<const f32x4*>(q + i);
+    *reinterpret_cast<f32x4*>(copy + i) = x;
 #pragma unroll
     for (int e = 0; e < 4; ++e)
       bits = max(bits, __builtin_bit_cast(int, (float)x[e]) & 0x7fffffff);
@@ -172,10 +174,11 @@ __device__ __forceinline__ float narrow_query(const float* q,
                    (c.K + 64) * 0x1p-23f * norm * c.norm);
 }
 
-// Queries of a batch in blocks as the rows, a wave each: of 16 FN queries lane r has
-// query FN r + f in the f-th block. Zeros past Q.
+// Queries in blocks as the rows, a wave each: of 16 FN queries lane r has query FN r + f
+// in the f-th block. Zeros past Q. q may be memory of the host: one launch takes it to
+// the GPU and makes what is asked of it.
 __global__ void __launch_bounds__(256)
-narrow_queries_kernel(const float* __restrict__ q, u16* __restrict__ out,
+narrow_queries_kernel(const float* q, float* copy, u16* __restrict__ out,
                       float* __restrict__ margin, const NarrowRows c, int Q,
                       int FN) {
   const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -185,8 +188,9 @@ narrow_queries_kernel(const float* __restrict__ q, u16* __restrict__ out,
                                     ((i >> 3 & 3) * 16 + r) * 8 + (i & 4));
   };
   if (row < Q) {
-    const float m = narrow_query(q + (long)row * c.K, c,
-                                 [&](int i, i32x2 v) { *at(i) = v; });
+    const float m =
+        narrow_query(q + (long)row * c.K, copy + (long)row * c.K, c,
+                     [&](int i, i32x2 v) { *at(i) = v; });
     if ((threadIdx.x & 63) == 0) margin[row] = m;
   } else {
     for (int i = (threadIdx.x & 63) * 4; i < c.KP; i += 256) *at(i) = {0, 0};
@@ -198,8 +202,7 @@ narrow_queries_kernel(const float* __restrict__ q, u16* __restrict__ out,
 // and spans[Q, waves], of a wave's rows. A wave has every W-th sixteen of rows, so
 // that all read beside each other, and a ring of its own in LDS for their chunks of 64
 // columns, filled R - 1 chunks ahead: no barriers, counted waits. The queries are in
-// LDS as a whole, made by every workgroup while its first rows come. Bound by reading
-// the rows: 250000 of 768 66 us, 5.8 TB/s.
+// LDS as a whole. Bound by reading the rows: 250000 of 768 66 us, 5.8 TB/s.
 constexpr int NF_WAVES = 8, NF_RING = 6;
 static int narrow_few_lds(int KP) {
   return KP * 32 + NF_WAVES * NF_RING * 2048;
@@ -214,11 +217,10 @@ __device__ __forceinline__ void narrow_copy(const u16* src, char* dst) {
 }
 
 __global__ void __launch_bounds__(NF_WAVES * 64)
-narrow_few_kernel(const NarrowRows of, const float* __restrict__ q,
-                  float* __restrict__ margin, float* __restrict__ groups,
-                  float* __restrict__ spans, int Q) {
+narrow_few_kernel(const u16* __restrict__ rows, const u16* __restrict__ q16,
+                  float* __restrict__ groups, float* __restrict__ spans, int Q,
+                  int N, int KP) {
   constexpr int R = NF_RING;
-  const int N = of.N, KP = of.KP;
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, g = lane >> 4;
@@ -229,7 +231,7 @@ narrow_few_kernel(const NarrowRows of, const float* __restrict__ q,
   char* ring = smem + KP * 32 + wid * (R * 2048);
 
   // to be copied next: a chunk of a unit's
-  const u16* src = of.rows + (long)own * KP * 16;
+  const u16* src = rows + (long)own * KP * 16;
   const long hop = (long)(W - 1) * KP * 16;
   int chunk = 0;
   auto issue = [&](int slot) {
@@ -244,19 +246,9 @@ narrow_few_kernel(const NarrowRows of, const float* __restrict__ q,
   };
   const int total = mine * nch;
   for (int c = 0; c < R - 1 && c < total; ++c) issue(c);
-  for (int j = wid; j < 16; j += NF_WAVES) {
-    auto at = [&](int i) {
-      return reinterpret_cast<i32x2*>(smem + (i >> 5) * 1024 +
-                                      ((i >> 3 & 3) * 16 + j) * 16 + (i & 4) * 2);
-    };
-    if (j < Q) {
-      const float m = narrow_query(q + (long)j * of.K, of,
-                                   [&](int i, i32x2 v) { *at(i) = v; });
-      if (blockIdx.x == 0 && lane == 0) margin[j] = m;
-    } else {
-      for (int i = lane * 4; i < KP; i += 256) *at(i) = {0, 0};
-    }
-  }
+  for (int c = wid; c < nch * 2; c += NF_WAVES)
+    narrow_copy(q16 + c * 512, smem + c * 1024);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
 
   float top = -INFINITY;
@@ -701,11 +693,11 @@ namespace {
 // Where things lie beside the operands.
 struct NarrowPlan {
   int QP, fm, fn, grid;  // fn 1: a few queries
-  long q16, margin, groups, spans, bytes;
+  long copy, q16, margin, groups, spans, bytes;
   NarrowMost most;
 };
 
-NarrowPlan narrow_plan(int Q, int N, int KP) {
+NarrowPlan narrow_plan(int Q, int N, int K, int KP) {
   NarrowPlan p = {};
   p.fn = Q <= 16 && KP <= 1536 ? 1 : Q <= 128 ? 4 : 8;
   const int tile = p.fn == 1 ? 16 : 32 * p.fn;
@@ -732,7 +724,8 @@ NarrowPlan narrow_plan(int Q, int N, int KP) {
     p.bytes += (bytes + 255) / 256 * 256;
     return at;
   };
-  if (p.fn > 1) p.q16 = place((long)p.QP * KP * 2);
+  p.copy = place((long)Q * K * 4);
+  p.q16 = place((long)p.QP * KP * 2);
   p.margin = place((long)Q * 4);
   p.spans = place(o.S * o.ld * 4);
   p.groups = place(o.G * o.ld * 4);
@@ -748,29 +741,30 @@ extern "C" long narrow_bytes(long Q, long N, long K, long KP) {
       K % 4 || KP % 64 || KP < 128 || KP < K || KP > 1L << 16 ||
       (N + 127) / 128 * ((Q + 127) / 128) >= 1L << 30)
     return 0;
-  return narrow_plan((int)Q, (int)N, (int)KP).bytes;
+  return narrow_plan((int)Q, (int)N, (int)K, (int)KP).bytes;
 }
 
 // rows: of narrow_rows_kernel, with its up and (roots of its) facts; space:
-// narrow_bytes. out_v, out_i [Q, k], k <= 60 and <= N.
+// narrow_bytes. out_v, out_i [Q, k], k <= 60 and <= N. q, out_v and out_i may be memory
+// of the host that the GPU sees.
 extern "C" void launch_narrow_topk(const float* q, const float* corpus,
                                    const void* rows, void* space, float* out_v,
                                    int* out_i, int Q, int N, int K, int KP,
                                    int up, float error, float norm, int k,
                                    hipStream_t stream) {
-  NarrowPlan p = narrow_plan(Q, N, KP);
+  NarrowPlan p = narrow_plan(Q, N, K, KP);
   char* at = (char*)space;
   u16* q16 = (u16*)(at + p.q16);
+  float* copy = (float*)(at + p.copy);
   float *margin = (float*)(at + p.margin), *groups = (float*)(at + p.groups),
         *spans = (float*)(at + p.spans);
   const NarrowRows c = {(const u16*)rows, N, K, KP, up, error, norm};
-  if (p.fn > 1)
-    hipLaunchKernelGGL(narrow_queries_kernel, dim3(p.QP / 4), dim3(256), 0,
-                       stream, q, q16, margin, c, Q, p.fn);
+  hipLaunchKernelGGL(narrow_queries_kernel, dim3(p.QP / 4), dim3(256), 0,
+                     stream, q, copy, q16, margin, c, Q, p.fn);
   if (p.fn == 1)
     hipLaunchKernelGGL(narrow_few_kernel, dim3(p.grid), dim3(NF_WAVES * 64),
-                       narrow_few_lds(KP), stream, c, q, margin, groups,
-                       spans, Q);
+                       narrow_few_lds(KP), stream, c.rows, q16, groups, spans,
+                       Q, N, KP);
 #define NS(M, F)                                                             \
   hipLaunchKernelGGL((narrow_batch_kernel<M, F>), dim3(256), dim3(256),      \
                      nb_lds(M, F), stream, (const char*)c.rows,              \
@@ -789,5 +783,5 @@ extern "C" void launch_narrow_topk(const float* q, const float* corpus,
   p.most.spans = spans;
   p.most.margin = margin;
   hipLaunchKernelGGL(narrow_top_kernel, dim3(Q), dim3(1024), 0, stream, p.most,
-                     q, corpus, out_v, out_i, N, K, k);
+                     copy, corpus, out_v, out_i, N, K, k);
 }

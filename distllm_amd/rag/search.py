@@ -343,16 +343,17 @@ class HipFlatIndex:
         return v, alli.gather(1, sel.long()).int()
 
     def _found_narrow(self, q: torch.Tensor, k: int):
-        """What _topk_exact finds, as lists, by way of the rows in 16 bits; None
-        where these do not answer it, for want of speed or of certainty, or
-        where another search has been put in _topk_exact's place."""
+        """What _topk_exact finds for queries of the host, as lists, by way of the
+        rows in 16 bits; None where these do not answer it, for want of speed or
+        of certainty, or where another search has been put in _topk_exact's
+        place or asked for."""
         if (self.narrow is None or q.dim() != 2
+                or self.precision != "float32"
+                or self.search_algorithm == "ivf"
                 or getattr(self._topk_exact, "__func__", None)
                 is not HipFlatIndex._topk_exact):
             return None
-        found = ops.score_topk_narrow(q, self.corpus, min(k, self.n),
-                                      self.narrow)
-        return None if found is None else ops.found_lists(*found, sure=True)
+        return ops.found_narrow(q, self.corpus, min(k, self.n), self.narrow)
 
     def _topk_ubinary(self, qfp: torch.Tensor, k: int):
         """Hamming candidates (HIP popcount) + fp32 rescore."""
@@ -378,17 +379,18 @@ class HipFlatIndex:
                score_threshold: float = 0.0) -> BatchedSearchResults:
         t0 = time.perf_counter()
         q = torch.from_numpy(
-            np.ascontiguousarray(query_embedding, dtype=np.float32)
-        ).to(self.corpus.device)
-        lists = None
-        if self.precision == "ubinary":
+            np.ascontiguousarray(query_embedding, dtype=np.float32))
+        lists = self._found_narrow(q, top_k)
+        if lists is None:
+            q = q.to(self.corpus.device)
+        if lists is not None:
+            pass
+        elif self.precision == "ubinary":
             v, i = self._topk_ubinary(q, top_k)
         elif self.search_algorithm == "ivf":
             v, i = self._topk_ivf(q, top_k)
         else:
-            lists = self._found_narrow(q, top_k)
-            if lists is None:
-                v, i = self._topk_exact(q, top_k)
+            v, i = self._topk_exact(q, top_k)
         # IVF pads short candidate lists with index -1 / score -inf;
         # drop those unconditionally (not only under score_threshold) so
         # -1 never reaches get()/dataset indexing as "last row".

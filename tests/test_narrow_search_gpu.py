@@ -73,10 +73,20 @@ def test_queries_that_are_not_answered(device, Q):
     v, i = _topk(q, c, 9)
     assert (i[:5] == UNSURE).all()
     assert torch.equal(i[5:], _topk(q[5:].contiguous(), c, 9)[1])
-    assert ops.found_lists(v, i, sure=True) is None
-    assert ops.found_lists(v, i)[1][0] == []
-    assert ops.found_lists(v[5:], i[5:], sure=True) == tuple(
+    n = ops.narrow_rows(c)
+    args = c, n.rows, n.up, n.error, n.norm, 9
+    assert _hip_ops.narrow_found(q.cpu(), *args) is None
+    assert _hip_ops.narrow_found(q[5:].cpu(), *args) == tuple(
         t.tolist() for t in (v[5:], i[5:]))
+
+
+@pytest.mark.parametrize("Q", [4096, 4097])
+def test_host_queries_pinned_or_copied(device, Q):
+    """Q of 1024 numbers: 16 MB, and above it."""
+    q, c = _unit(Q, 1024, 1), _unit(900, 1024, 2)
+    n = ops.narrow_rows(c)
+    found = _hip_ops.narrow_found(q.cpu(), c, n.rows, n.up, n.error, n.norm, 3)
+    assert found == tuple(t.tolist() for t in _topk(q, c, 3))
 
 
 def test_rows_of_no_use(device):
@@ -105,8 +115,8 @@ def test_index(device, tmp_path, monkeypatch, Q):
     np.savez(tmp_path / "i.npz", embeddings=c.cpu().numpy())
     index = HipFlatIndex(tmp_path / "d", tmp_path / "i.npz")
     calls = []
-    own = _hip_ops.narrow_topk
-    monkeypatch.setattr(_hip_ops, "narrow_topk",
+    own = _hip_ops.narrow_found
+    monkeypatch.setattr(_hip_ops, "narrow_found",
                         lambda *a: calls.append(0) or own(*a), raising=False)
 
     def check(by):
