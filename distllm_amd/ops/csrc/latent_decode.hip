@@ -381,20 +381,25 @@ latent_combine_kernel(const float* __restrict__ pacc,
 
 // The same join, and the product of the joined latents with the heads' value
 // weights W [H, N, R], which is what follows: out[m, h, :] = W[h] latent[m, h]. A
-// workgroup has eight rows of a head, one joined by each wave, while the weights come
-// to LDS by whole lines, and then 16 columns a wave; roundings and sums are those of
+// workgroup has ROWS rows of a head, joined while the weights come to LDS by whole
+// lines, and then 16 columns a wave; roundings and sums are those of
 // latent_combine_kernel and head_gemm_kernel, bit for bit. Bound by the way of the
-// shares and the weights into a CU, 128 KiB each at 8 shares of rank 512 and 128
-// columns: the first shares are on their way ahead of the weights (behind them 10.7 us
-// for 8.2). us with the attention, launches of their own and this, 32 heads: rank 512,
-// 128 columns, 32 rows of 2000 keys 33.0, 28.8, one 20.8, 19.3, 64 of 300 23.8, 20.1;
-// rank 256, 64 columns, 32 of 2000 22.4, 17.5.
+// shares and the weights into a CU, of 8 rows 128 KiB each at 8 shares of rank 512 and
+// 128 columns: the first shares are on their way ahead of the weights (behind them 10.7
+// us for 8.2), and there are 4 rows, two waves each, where those of all still fit the
+// card at once. us over fresh weights, 8 and 4 rows, rank 512, 128 columns, 8 shares,
+// 32 heads: 1 row 5.9 and 5.0, 32 6.0 and 5.4, with 16 shares 11.2 and 8.5; in two
+// rounds, 40 6.1 and 9.1; 128 heads, 8 rows 6.9 and 6.9, 12 8.0 and 11.6; rank 384, 64
+// columns, 32 heads, 32 rows 4.5 and 3.9, 40 4.6 and 4.9. us with the attention,
+// launches of their own and this of 8 rows, 32 heads: rank 512, 128 columns, 32 rows of
+// 2000 keys 33.0, 28.8, one 20.8, 19.3, 64 of 300 23.8, 20.1; rank 256, 64 columns, 32
+// of 2000 22.4, 17.5.
 // LDS rows' 16-byte pieces are XOR-ed with the row.
-constexpr int LV_ROWS = 8;
-constexpr int lv_lds(int R, int N) { return (N + LV_ROWS) * R * 2; }
+constexpr int LV_WAVES = 8;
+constexpr int lv_lds(int R, int N, int ROWS) { return (N + ROWS) * R * 2; }
 
-template <int R>
-__global__ void __launch_bounds__(LV_ROWS * 64)
+template <int R, int ROWS>
+__global__ void __launch_bounds__(LV_WAVES * 64)
 latent_values_kernel(const float* __restrict__ pacc,
                      const float* __restrict__ pml,
                      const unsigned short* __restrict__ W,
@@ -405,13 +410,16 @@ latent_values_kernel(const float* __restrict__ pacc,
   constexpr int RP = R / 8;
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int head = blockIdx.x % H, m0 = blockIdx.x / H * LV_ROWS;
+  const int head = blockIdx.x % H, m0 = blockIdx.x / H * ROWS;
   char* xs = smem + N * (R * 2);
-  const long rh = (long)min(m0 + wid, M - 1) * H + head;
+  // of 8 rows a wave joins one, of 4 half of one
+  constexpr int PARTS = (R + 255) / 256 * ROWS / LV_WAVES, AHEAD = 8;
+  static_assert(PARTS * LV_WAVES == (R + 255) / 256 * ROWS, "whole parts");
+  const int mine = wid % ROWS, c0 = wid / ROWS * 256 + lane * 4;
+  const long rh = (long)min(m0 + mine, M - 1) * H + head;
   const float* state = pml + (rh * NS + min(lane, NS - 1)) * 2;
   float m = state[0], l = state[1];
   // the first shares are on their way ahead of the weights: loads arrive in order
-  constexpr int PARTS = (R + 255) / 256, AHEAD = 8;
   f32x4 v[PARTS][AHEAD];
 #pragma unroll
   for (int part = 0; part < PARTS; ++part)
@@ -419,10 +427,10 @@ latent_values_kernel(const float* __restrict__ pacc,
     for (int s = 0; s < AHEAD; ++s)
       v[part][s] = *reinterpret_cast<const f32x4*>(
           pacc + (rh * NS + min(s, NS - 1)) * R +
-          min(part * 256 + lane * 4, R - 4));
+          min(part * 256 + c0, R - 4));
   __builtin_amdgcn_sched_barrier(0);
   const unsigned short* from = W + (long)head * N * R;
-  for (int p = wid; p < N * RP / 64; p += LV_ROWS) {
+  for (int p = wid; p < N * RP / 64; p += LV_WAVES) {
     const int at = p * 64 + lane, r = at / RP, c = at % RP;
     copy_to_lds(from + r * R + (c ^ (r & 7)) * 8, smem + p * 1024);
   }
@@ -438,7 +446,7 @@ latent_values_kernel(const float* __restrict__ pacc,
   };
 #pragma unroll
   for (int part = 0; part < PARTS; ++part) {
-    const int c = part * 256 + lane * 4;
+    const int c = part * 256 + c0;
     f32x4 o = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int s = 0; s < AHEAD; ++s)
@@ -456,15 +464,15 @@ latent_values_kernel(const float* __restrict__ pacc,
       for (int i = 0; i < 4; ++i) o[i] += w * x[i];
     }
     if (c < R)
-      *reinterpret_cast<i32x2*>(xs + wid * (R * 2) + ((c >> 3) ^ wid) * 16 +
-                                (c & 4) * 2) =
+      *reinterpret_cast<i32x2*>(xs + mine * (R * 2) +
+                                ((c >> 3) ^ mine) * 16 + (c & 4) * 2) =
           i32x2{(int)ld_pack(o[0], o[1]), (int)ld_pack(o[2], o[3])};
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
 
-  const int c16 = lane & 15, g = lane >> 4, xrow = c16 & (LV_ROWS - 1);
-  for (int n0 = wid * 16; n0 < N; n0 += LV_ROWS * 16) {
+  const int c16 = lane & 15, g = lane >> 4, xrow = c16 & (ROWS - 1);
+  for (int n0 = wid * 16; n0 < N; n0 += LV_WAVES * 16) {
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int s = 0; s < R / 32; ++s) {
@@ -477,7 +485,7 @@ latent_values_kernel(const float* __restrict__ pacc,
           acc, 0, 0, 0);
     }
     const int row = m0 + c16;
-    if (c16 < LV_ROWS && row < M)
+    if (c16 < ROWS && row < M)
       *reinterpret_cast<i32x2*>(out + row * orow_s + (long)head * ohead_s +
                                 n0 + g * 4) =
           i32x2{(int)ld_pack(acc[0], acc[1]), (int)ld_pack(acc[2], acc[3])};
@@ -486,7 +494,7 @@ latent_values_kernel(const float* __restrict__ pacc,
 
 // Whether the weights of a head have room in LDS.
 extern "C" bool latent_values_fit(int R, int N) {
-  return N % 64 == 0 && lv_lds(R, N) <= 160 * 1024;
+  return N % 64 == 0 && lv_lds(R, N, 8) <= 160 * 1024;
 }
 
 extern "C" void launch_latent_values(const void* pacc, const void* pml,
@@ -495,17 +503,23 @@ extern "C" void launch_latent_values(const void* pacc, const void* pml,
                                      int ohead_s, const float* sink,
                                      const void* gate, int ld_gate,
                                      hipStream_t stream) {
-#define LV(RR)                                                                \
-  case RR:                                                                    \
-    hipLaunchKernelGGL((latent_values_kernel<RR>),                            \
-                       dim3(H * ((M + LV_ROWS - 1) / LV_ROWS)),               \
-                       dim3(LV_ROWS * 64), lv_lds(RR, N), stream,             \
-                       (const float*)pacc, (const float*)pml,                 \
-                       (const unsigned short*)W, (unsigned short*)out, M, H,  \
-                       N, NS, orow_s, ohead_s, sink,                          \
-                       (const unsigned short*)gate, ld_gate);                 \
-    break
-  switch (R) { LV(64); LV(128); LV(192); LV(256); LV(384); LV(512); }
+  // (up to rank 256 a row is one wave's)
+  const bool four = R > 256 && (long)H * ((M + 3) / 4) <= 256;
+#define LV(RR, ROWS)                                                          \
+  hipLaunchKernelGGL((latent_values_kernel<RR, ROWS>),                        \
+                     dim3(H * ((M + ROWS - 1) / ROWS)), dim3(LV_WAVES * 64),  \
+                     lv_lds(RR, N, ROWS), stream, (const float*)pacc,         \
+                     (const float*)pml, (const unsigned short*)W,             \
+                     (unsigned short*)out, M, H, N, NS, orow_s, ohead_s,      \
+                     sink, (const unsigned short*)gate, ld_gate)
+  switch (R) {
+    case 64: LV(64, 8); break;
+    case 128: LV(128, 8); break;
+    case 192: LV(192, 8); break;
+    case 256: LV(256, 8); break;
+    case 384: if (four) LV(384, 4); else LV(384, 8); break;
+    case 512: if (four) LV(512, 4); else LV(512, 8); break;
+  }
 #undef LV
 }
 
