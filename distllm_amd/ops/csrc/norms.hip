@@ -7,6 +7,12 @@
 // Design (guide: Appendix B element-wise/reduction rules):
 //  - one WAVE per row (row = hidden vector of size H), 4 rows per 256-thread
 //    block; bf16 loads vectorized as s16x8 (16 B/lane);
+//  - all that a row needs, weights and bias too, is asked for before its
+//    sums: a row's chunks under branches, then its weights, were a round to
+//    memory each. Lanes past the row's end ask for its last numbers again
+//    (guards instead: 2 to 10% slower). us with a residual, 768 columns,
+//    4096 rows 5.9 -> 5.3, 12992 14.0 -> 12.3 (4.9 TB/s), 131072 104 -> 100,
+//    262144 205 -> 200 (6.0 TB/s).
 //  - fp32 accumulate, single pass, row held in registers. Per-lane chunk
 //    count is a template parameter so every register index is
 //    compile-time (runtime-indexed ext_vector arrays spill to scratch).
@@ -32,19 +38,33 @@ norm_fwd_kernel(const unsigned short* __restrict__ x,
     const unsigned short* xr = x + (long)row * H;
     const unsigned short* rr = HAS_RES ? res + (long)row * H : nullptr;
 
+    s16x8 xv[NCL], rv[NCL], wv[NCL], bv[NCL];
+#pragma unroll
+    for (int k = 0; k < NCL; ++k) {
+      const int c = min(lane + k * WAVE, chunks - 1) * 8;
+      xv[k] = *reinterpret_cast<const s16x8*>(xr + c);
+      if (HAS_RES) rv[k] = *reinterpret_cast<const s16x8*>(rr + c);
+    }
+#pragma unroll
+    for (int k = 0; k < NCL; ++k) {
+      const int c = min(lane + k * WAVE, chunks - 1) * 8;
+      wv[k] = *reinterpret_cast<const s16x8*>(w + c);
+      if (b != nullptr) bv[k] = *reinterpret_cast<const s16x8*>(b + c);
+      else bv[k] = s16x8{0, 0, 0, 0, 0, 0, 0, 0};
+    }
+    __builtin_amdgcn_sched_barrier(0);
+
     float v[NCL][8];
     float sum = 0.f, sumsq = 0.f;
 #pragma unroll
     for (int k = 0; k < NCL; ++k) {
       const int c = lane + k * WAVE;
       if (c < chunks) {
-        s16x8 xv = *reinterpret_cast<const s16x8*>(xr + c * 8);
         float f[8];
-        bf8_to_f32(xv, f);
+        bf8_to_f32(xv[k], f);
         if (HAS_RES) {
-          s16x8 rv = *reinterpret_cast<const s16x8*>(rr + c * 8);
           float g[8];
-          bf8_to_f32(rv, g);
+          bf8_to_f32(rv[k], g);
 #pragma unroll
           for (int i = 0; i < 8; ++i) f[i] += g[i];
         }
@@ -79,14 +99,9 @@ norm_fwd_kernel(const unsigned short* __restrict__ x,
     for (int k = 0; k < NCL; ++k) {
       const int c = lane + k * WAVE;
       if (c < chunks) {
-        s16x8 wv = *reinterpret_cast<const s16x8*>(w + c * 8);
-        float wf[8];
-        bf8_to_f32(wv, wf);
-        float bf[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-        if (b != nullptr) {
-          s16x8 bv = *reinterpret_cast<const s16x8*>(b + c * 8);
-          bf8_to_f32(bv, bf);
-        }
+        float wf[8], bf[8];
+        bf8_to_f32(wv[k], wf);
+        bf8_to_f32(bv[k], bf);
         s16x8 ov;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
@@ -99,13 +114,16 @@ norm_fwd_kernel(const unsigned short* __restrict__ x,
   }
 }
 
-
-
-// Small-batch variant: ONE 256-thread block per row (4 waves split the
-// chunks, LDS cross-wave combine). With few rows the wave-per-row kernel is
-// a few waves doing NCL dependent 16-B load rounds; spreading the row across
-// the block quarters the rounds on the per-token critical path.
-template <int NCL, bool HAS_RES, bool WRITE_SUM, bool RMS>
+// ONE 256-thread block per row (4 waves split the chunks, LDS cross-wave
+// combine): few rows are a few waves in the kernel above, and wide ones a
+// quarter of the waves that a CU could have, for their registers.
+// AHEAD: all is asked for at once, as above; else chunk by chunk, and the
+// weights behind the sums. us, behind and ahead, with residual and sum: 16
+// rows of 4096 2.88 and 2.69, 256 rows of 2048 2.69 and 2.51, 2048 13.8 and
+// 13.1 of 4096, 4096 23.6 and 22.5, 13000 rows of 2048 39.2 and 33.1; but
+// 800 and 1024 rows of 4096 6.27, 7.00 and 6.56, 7.30, of 1024 2.65, 3.10
+// and 2.89, 3.29; 512 rows of 640 to 4096 within 3% either way, 1500 1%.
+template <int NCL, bool HAS_RES, bool WRITE_SUM, bool RMS, bool AHEAD>
 __global__ void __launch_bounds__(256)
 norm_fwd_small_kernel(const unsigned short* __restrict__ x,
                       const unsigned short* __restrict__ res,
@@ -123,19 +141,38 @@ norm_fwd_small_kernel(const unsigned short* __restrict__ x,
   const unsigned short* xr = x + (long)row * H;
   const unsigned short* rr = HAS_RES ? res + (long)row * H : nullptr;
 
+  s16x8 xv[NCL], rv[NCL], wv[NCL], bv[NCL];
+  auto row_at = [&](int k) {
+    const int c = min((int)threadIdx.x + k * 256, chunks - 1) * 8;
+    xv[k] = *reinterpret_cast<const s16x8*>(xr + c);
+    if (HAS_RES) rv[k] = *reinterpret_cast<const s16x8*>(rr + c);
+  };
+  auto weights_at = [&](int k) {
+    const int c = min((int)threadIdx.x + k * 256, chunks - 1) * 8;
+    wv[k] = *reinterpret_cast<const s16x8*>(w + c);
+    if (b != nullptr) bv[k] = *reinterpret_cast<const s16x8*>(b + c);
+    else bv[k] = s16x8{0, 0, 0, 0, 0, 0, 0, 0};
+  };
+  if (AHEAD) {
+#pragma unroll
+    for (int k = 0; k < NCL; ++k) row_at(k);
+#pragma unroll
+    for (int k = 0; k < NCL; ++k) weights_at(k);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+
   float v[NCL][8];
   float sum = 0.f, sumsq = 0.f;
 #pragma unroll
   for (int k = 0; k < NCL; ++k) {
     const int c = threadIdx.x + k * 256;
     if (c < chunks) {
-      s16x8 xv = *reinterpret_cast<const s16x8*>(xr + c * 8);
+      if (!AHEAD) row_at(k);
       float f[8];
-      bf8_to_f32(xv, f);
+      bf8_to_f32(xv[k], f);
       if (HAS_RES) {
-        s16x8 rv = *reinterpret_cast<const s16x8*>(rr + c * 8);
         float g[8];
-        bf8_to_f32(rv, g);
+        bf8_to_f32(rv[k], g);
 #pragma unroll
         for (int i = 0; i < 8; ++i) f[i] += g[i];
       }
@@ -174,14 +211,10 @@ norm_fwd_small_kernel(const unsigned short* __restrict__ x,
   for (int k = 0; k < NCL; ++k) {
     const int c = threadIdx.x + k * 256;
     if (c < chunks) {
-      s16x8 wv = *reinterpret_cast<const s16x8*>(w + c * 8);
-      float wf[8];
-      bf8_to_f32(wv, wf);
-      float bf[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-      if (b != nullptr) {
-        s16x8 bv = *reinterpret_cast<const s16x8*>(b + c * 8);
-        bf8_to_f32(bv, bf);
-      }
+      if (!AHEAD) weights_at(k);
+      float wf[8], bf[8];
+      bf8_to_f32(wv[k], wf);
+      bf8_to_f32(bv[k], bf);
       s16x8 ov;
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
@@ -195,54 +228,53 @@ norm_fwd_small_kernel(const unsigned short* __restrict__ x,
 
 // Whether a row gets a workgroup: few rows leave most CUs without a wave, wide
 // rows leave a wave with many loads; narrow ones leave most of a workgroup's
-// threads without any. Measured in a graph with residual and sum, us, workgroup
-// and wave per row: 64 rows of 768 2.6 and 3.3, of 4096 3.4 and 6.6, of 8192
-// 4.6 and 11.1; 2048 rows of 128 3.1 and 2.4, of 512 3.4 and 2.8, of 640 1.03
-// times the wave's, of 768 4.2 and 4.3, of 4096 9.2 and 11.5, of 8192 15.7 and
-// 20.4; 4096 rows of 768 6.4 and 5.5, of 4096 16.1 and 20.7, of 8192 30.3 and
-// 37.9. Widths up to 512 are within 4% of each other up to 1024 rows; 3072 to
-// 65536 rows of 2048 are 0.91 to 1.14 of the wave's time, of 3072 0.87 to 1.00,
-// of 4096 0.83 to 0.96, of 5120 and 8192 0.79 to 0.92.
+// threads without any. Measured in a graph with residual (and sum, from 1152
+// columns on), us, workgroup and wave per row: 64 rows of 512 2.31 and 2.28, of
+// 768 2.34 and 2.54, of 4096 2.8 and 4.5; 2048 rows of 128 3.2 and 2.6, of 512 3.6
+// and 3.3, of 768 4.0 and 4.1; 4096 rows of 768 5.7 and 5.3, of 1024 6.4 and 6.1,
+// of 1280 8.4 and 8.6, of 2560 15.2 and 17.9; 16384 rows of 768 18.1 and 14.4, of
+// 1024 19.6 and 17.9, of 1152 26.7 and 26.7, of 1280 28.4 and 29.4, of 2048 40.7
+// and 42.5; 65536 rows of 1152 to 2560 0.95 to 1.01 of the wave's time, 131072
+// 0.99 to 1.02; of 4096 always below 0.99.
 static bool norm_row_block(int n_rows, int H) {
-  return n_rows <= 8 || (H > 512 && n_rows <= 2048) || H >= 3072;
+  return n_rows <= 8 || (H > 512 && n_rows <= 2048) ||
+         (H > 1024 && n_rows <= 65536) || H >= 3072;
 }
 
 extern "C" void launch_norm_fwd(const void* x, const void* res, const void* w,
                                 const void* b, void* out, void* sum_out,
                                 int n_rows, int H, float eps, bool rms,
                                 hipStream_t stream) {
-  // Grid cap: measured on MI355X (DISTLLM_NORM_BLOCKS sweep in
-  // profiles/RESULTS.md): deep grids beat a 2048-block grid-stride
-  // loop by ~5%; a 2-rows-per-wave ILP variant was also probed and
-  // REGRESSED (149 -> 172 us plain LN) — tail guards in the unrolled
-  // loops cost more than the overlap wins, so R stays 1.
+  // Waves that go on to a second row pay up to 512 columns only: us, at most
+  // 32768 blocks and all, 262144 rows of 128 50.7 and 63.6, of 384 102.8 and
+  // 105.8, of 768 209 and 200, of 1024 281 and 278, of 1280 466 and 455, of 2048
+  // 763 and 749. (Threads of a grid are counted in 32 bits: at most 2^20 blocks.)
   static const int cap = [] {
     const char* e = getenv("DISTLLM_NORM_BLOCKS");
-    return e ? atoi(e) : 32768;
+    return e ? atoi(e) : 0;
   }();
-  int blocks = min((n_rows + 3) / 4, cap);
+  int blocks = min((n_rows + 3) / 4,
+                   cap != 0 ? cap : H > 512 ? 1 << 20 : 32768);
   bool has_res = res != nullptr;
   bool write_sum = sum_out != nullptr;
   const bool small = norm_row_block(n_rows, H);
+  const bool ahead = n_rows <= 512 || n_rows >= 1500;
   int ncl = small ? (H / 8 + 255) / 256 : (H / 8 + WAVE - 1) / WAVE;
 
+#define DISPATCH4(KERNEL, BLOCKS)                                              \
+  hipLaunchKernelGGL(KERNEL, dim3(BLOCKS), dim3(256), 0, stream,               \
+                     (const unsigned short*)x, (const unsigned short*)res,     \
+                     (const unsigned short*)w, (const unsigned short*)b,       \
+                     (unsigned short*)out, (unsigned short*)sum_out, n_rows,   \
+                     H, eps)
 #define DISPATCH3(NCL, HR, WS, RM)                                             \
   do {                                                                         \
-    if (small)                                                                 \
-      hipLaunchKernelGGL((norm_fwd_small_kernel<NCL, HR, WS, RM>),             \
-                         dim3(n_rows), dim3(256), 0, stream,                   \
-                         (const unsigned short*)x,                             \
-                         (const unsigned short*)res,                           \
-                         (const unsigned short*)w,                             \
-                         (const unsigned short*)b, (unsigned short*)out,       \
-                         (unsigned short*)sum_out, n_rows, H, eps);            \
+    if (small && ahead)                                                        \
+      DISPATCH4((norm_fwd_small_kernel<NCL, HR, WS, RM, true>), n_rows);       \
+    else if (small)                                                            \
+      DISPATCH4((norm_fwd_small_kernel<NCL, HR, WS, RM, false>), n_rows);      \
     else                                                                       \
-      hipLaunchKernelGGL((norm_fwd_kernel<NCL, HR, WS, RM>), dim3(blocks),     \
-                         dim3(256), 0, stream, (const unsigned short*)x,       \
-                         (const unsigned short*)res,                           \
-                         (const unsigned short*)w,                             \
-                         (const unsigned short*)b, (unsigned short*)out,       \
-                         (unsigned short*)sum_out, n_rows, H, eps);            \
+      DISPATCH4((norm_fwd_kernel<NCL, HR, WS, RM>), blocks);                   \
   } while (0)
 #define DISPATCH_FLAGS(NCL)                                                    \
   do {                                                                         \
@@ -268,6 +300,7 @@ extern "C" void launch_norm_fwd(const void* x, const void* res, const void* w,
   }
 #undef DISPATCH_FLAGS
 #undef DISPATCH3
+#undef DISPATCH4
 }
 
 // Sum of the fp32 slabs [S, rows, H] of a product whose K was shared, rounded

@@ -24,3 +24,22 @@ def test_rows(device, rows, H, rms):
     want = torch_ref.norm_fwd(x, r, w, b, 1e-5, rms, return_sum=True)
     for a, e in zip(got, want):  # a bf16 step of results of a few units
         torch.testing.assert_close(a.float(), e.float(), atol=1e-2, rtol=8e-3)
+
+
+@pytest.mark.parametrize("rows, H", [
+    (512, 1032), (513, 1032), (1499, 2056), (1500, 2056),  # ahead of the sums
+    (65536, 1032), (65537, 1032), (65537, 1024),  # workgroup and wave
+    (131076, 512), (131077, 520), (300001, 8)])  # waves of more than a row
+@pytest.mark.parametrize("res, bias", [(False, False), (True, True)])
+def test_all_at_once(device, rows, H, res, bias):
+    g = torch.Generator(device=device).manual_seed(rows + H)
+    x, r = (torch.randn(rows, H, device=device, generator=g)
+            .to(torch.bfloat16) for _ in range(2))
+    w, b = (torch.randn(H, device=device, generator=g).to(torch.bfloat16)
+            for _ in range(2))
+    for rms in (False, True):
+        args = (x, r if res else None, w, b if bias else None, 1e-5, rms)
+        # a bf16 step, as above
+        torch.testing.assert_close(ops.norm_fwd(*args).float(),
+                                   torch_ref.norm_fwd(*args).float(),
+                                   atol=1e-2, rtol=8e-3)
