@@ -978,8 +978,8 @@ def _narrow_fills(Q, N):
 
 def found_narrow(q, corpus, k, narrow):
     """found_lists of score_topk for queries [Q, K] of the host, by way of the
-    corpus's NarrowRows: None where that is not the faster way, or these cannot
-    answer a query."""
+    corpus's NarrowRows: None where that is not the faster way, these cannot
+    answer a query, or there is no room for what it takes."""
     Q, K = q.shape
     N = corpus.shape[0]
     if not (0 < Q < 1 << 20 and 0 < k <= min(60, N)
@@ -989,8 +989,11 @@ def found_narrow(q, corpus, k, narrow):
             and 0 < _hip_ops.narrow_bytes(Q, N, K, narrow.rows.shape[1])
             <= 1 << 31):
         return None
-    return _hip_ops.narrow_found(q, corpus, narrow.rows, narrow.up,
-                                 narrow.error, narrow.norm, k)
+    try:
+        return _hip_ops.narrow_found(q, corpus, narrow.rows, narrow.up,
+                                     narrow.error, narrow.norm, k)
+    except torch.OutOfMemoryError:
+        return None
 
 
 def score_topk(q, corpus, k):

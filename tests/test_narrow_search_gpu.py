@@ -140,6 +140,13 @@ def test_index(device, tmp_path, monkeypatch, Q):
                         lambda x, k: HipFlatIndex._topk_exact(index, x, k))
     check(0)
     monkeypatch.undo()
+
+    def full(*a):
+        raise torch.OutOfMemoryError("no room")
+
+    monkeypatch.setattr(_hip_ops, "narrow_found", full, raising=False)
+    check(0)
+    monkeypatch.undo()
     # rows that are all the same are asked again
     index.corpus = c[:1].repeat(5000, 1)
     index.narrow = ops.narrow_rows(index.corpus)
