@@ -12,10 +12,10 @@
 // 6 TB/s leave about 100 cycles per KiB of weights.
 //
 //  ring    M <= 16 but for many columns of a short K, and up to 64 where
-//          columns are few. A workgroup has 16 columns (rows of W) and its 4
-//          waves take the 64-wide chunks of K in turn; W and x pass through a ring of LDS buffers that belongs
-//          to the wave alone: whole lines by global_load_lds, counted waits,
-//          no barriers. The waves' sums meet in LDS: no slabs, no second
+//          columns are few. A workgroup has 16 columns (rows of W), of up to
+//          2048 columns 8, and its 4 waves take the 64-wide chunks of K in turn;
+//          W and x pass through a ring of LDS buffers that belongs to the wave
+//          alone: whole lines by global_load_lds, counted waits, no barriers. The waves' sums meet in LDS: no slabs, no second
 //          launch. (W straight to operand registers is 2% faster for one row
 //          of 28672 x 4096 and up, and 10 to 60% slower else.)
 //  tile    above: W and x tiles of 64 columns of K in a ring that 4 or 8
@@ -30,8 +30,9 @@
 //   M = 1   28672 x 4096 gated 64 -> 41 (5.7 TB/s), 6144 x 4096 20 -> 11.3,
 //           4096 x 4096 12 -> 8.1, 4096 x 14336 31 -> 23.3, 32768 x 4096 58 ->
 //           45 (6.0 TB/s), 768 x 768 5.1 -> 2.7
-//   M = 64  28672 x 4096 gated 57 -> 51, 6144 x 4096 25 -> 17.7, 4096 x 4096
-//           18 -> 12.4, 4096 x 14336 38 -> 28.4, 768 x 768 7 -> 3.8
+//   M = 64  28672 x 4096 gated 57 -> 51 (as tiles; even 45 to 49), 6144 x 4096
+//           25 -> 17.6, 4096 x 4096 18 -> 12.4, 4096 x 14336 38 -> 28.4, 768 x 768
+//           7 -> 3.8
 //
 // Both LDS images hold rows of 128 bytes whose 16-byte pieces are XOR-ed
 // with the row, on the source address of the copies.
@@ -261,8 +262,9 @@ dg_ring_kernel(const u16* __restrict__ X, const u16* __restrict__ W, int K,
 // ---- ring with the norm ahead of the product --------------------------------
 // One row (norm_row.h). The normed row stays in LDS, so that the rings hold
 // weights only: more of them. Measured in a graph, us, norm and product in two
-// launches and in one: 28672 x 4096 gated 44.6 and 41.8, 6144 x 4096 13.3 and
-// 10.8, 4096 x 2048 7.9 and 7.0; two rows normed by every workgroup 46.5 and
+// launches and in one: 28672 x 4096 gated 45.8 and 41.3, 6144 x 4096 14.3 and
+// 11.8, 4096 x 2048 7.4 and 5.8 (the weights as copies that the compiler counts one
+// by one, so that the norm does not wait for them); two rows normed by every workgroup 46.5 and
 // 49.1 at the first.
 constexpr int dg_norm_lds(int K, int NT, int R) {
   return 128 + K * 2 + 4 * R * NT * 2048;

@@ -12,12 +12,14 @@
 // these. So K is dealt to four waves in chunks of 64, and the other waves take
 // other rows.
 //
-// Of 4.4 us for the norm of 24 rows and 2304 columns 0.8 are the start of the
-// waves, 1.0 the rows' loads, 2.0 the norm (vector units: every workgroup norms
-// all rows) and 0.6 the product. 12 layers in a graph, us, seven launches a
-// layer and four (five where the attention does not fit): 768 on 4 rows 305 and
-// 219, 16 313 and 238, 24 331 and 267, 32 338 and 326, 2 x 16 338 and 304; 1024
-// on 24 389 and 350, 32 405 and 412; 512 on 24 321 and 237, 2 x 24 352 and 322.
+// What a launch is made of: the start of the waves, a round to L2 for the rows, the
+// norm (vector units: every workgroup norms all rows) and the product. The weights
+// are asked for ahead of all that and waited for behind it: as copies that the
+// compiler cannot tell from accesses of LDS they were waited for ahead of the norm
+// (24 rows, 2304 columns, under a profiler 5.5 us, now 4.9). 12 layers in a graph,
+// us, norms in launches of their own and here: 768 on 4 rows 248 and 208, 16 259 and
+// 217, 24 274 and 241, 32 317 and 296, 2 x 16 300 and 278; 1024 on 16 304 and 273,
+// 24 332 and 309; 512 on 24 256 and 215.
 #include "attention_kernel.h"
 #include <algorithm>
 
@@ -384,11 +386,11 @@ constexpr int LDS_MOST = 160 * 1024;
 // Whether M rows of H numbers are normed by every workgroup. They fit up to 56
 // rows of 1024, but every workgroup norms them all, and a launch of its own costs
 // the same whatever they are. From 25 rows on a wave has a second pair of rows;
-// 12 layers, own launches and joined, us: 24 rows of 512 273 and 229, 768 290 and
-// 261, 832 306 and 289, 896 311 and 294, 960 360 and 345, 1024 369 and 351; 25 rows
-// 512 275 and 246, 768 326 and 312, 832 334 and 337, 896 336 and 342, 1024 403 and
-// 404; 32 rows 768 333 and 320, 832 339 and 346, 960 415 and 417, 1024 415 and 419;
-// 48 rows of 768 381 and 384, 64 rows 390 and 423.
+// 12 layers, own launches and joined, us: 24 rows of 512 256 and 215, 768 274 and
+// 241, 832 289 and 270, 1024 332 and 309; 25 rows of 768 313 and 292, 32 317 and 296.
+// Beyond, while the copies were waited for ahead of the norm: 25 rows of 832 334 and
+// 337, 896 336 and 342, 1024 403 and 404; 32 rows of 832 339 and 346, 1024 415 and
+// 419; 48 rows of 768 381 and 384, 64 rows 390 and 423.
 extern "C" bool norm_rows_fit(int M, int H) {
   return M >= 1 && M <= (H <= 768 ? 32 : 24) && H % 64 == 0 && H >= 64 &&
          H <= 1024 && rows_lds(M, H, 0) <= LDS_MOST;

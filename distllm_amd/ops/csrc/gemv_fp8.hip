@@ -219,7 +219,8 @@ gemv_fp8_ring_kernel(const unsigned short* __restrict__ X,
 
 // One row with its residual sum and norm ahead (norm_row.h). The normed row
 // stays in LDS, the rings hold weights only. In a graph, us, in two launches
-// and in one: 28672 x 4096 gated 27.5 and 25.5, 6144 x 4096 10.7 and 8.7.
+// and in one: 28672 x 4096 gated 27.5 and 24.8, 6144 x 4096 10.7 and 8.5 (25.5 and
+// 8.7 while the norm waited for the first weights).
 constexpr int gv_norm_ring(bool glu) { return glu ? 4 : 6; }
 constexpr int gv_norm_lds(bool glu, int K) {
   return 128 + K * 2 + 4 * gv_norm_ring(glu) * (glu ? 4096 : 2048);
