@@ -539,18 +539,21 @@ struct NarrowMost {
 // largest group from below; the spans within the margin of it are looked into, where
 // the same is found of their groups, then the k-th largest itself. Rows of groups
 // within the margin of that are scored in plain float32; equals go by place. k <= 60.
-// 250000 rows of 768, 1 query 10.6 us, a chain of loads, 256 18, which read 44 MB of rows.
+// A chain of loads and barriers, and of 256 queries 44 MB of rows: under the profiler, of
+// 250000 rows of 768, 1 query 7.1 us, 256 16.1 (9.3 and 18.0 with the 64 shares' ranks
+// found by one wave, and the spans read again once there is a bound).
 __global__ void __launch_bounds__(1024)
 narrow_top_kernel(const NarrowMost o, const float* __restrict__ q,
                   const float* __restrict__ corpus,
                   float* __restrict__ out_v, int* __restrict__ out_i, int N,
                   int K, int k) {
   __shared__ float top[16][64], thresh;
-  __shared__ int nspan, nlist, ncand;
+  __shared__ int nspan, nlist, ncand, ranks[64];
   __shared__ int span[NS_SPANS], list[NS_LIST], cand[NS_CAP];
   __shared__ float near[NS_LIST];
   __shared__ unsigned long long rows[NS_CAP * 4];
-  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int me = blockIdx.x;
   const float margin = o.margin[me];
   float* ov = out_v + (long)me * k;
@@ -563,37 +566,51 @@ narrow_top_kernel(const NarrowMost o, const float* __restrict__ q,
   };
   if (!(margin < INFINITY)) return unsure();
   if (tid == 0) nspan = nlist = ncand = 0;
+  if (tid < 64) ranks[tid] = 0;
   // the k-th largest of 64 shares' largest, of all threads' m
   auto bound = [&](float m) {
     top[wid][lane] = m;
     __syncthreads();
+#pragma unroll
+    for (int w = 0; w < 16; ++w) m = fmaxf(m, top[w][lane]);
+    // a wave compares with four of the shares
+    int rank = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int j = wid * 4 + i;
+      const float v = __builtin_bit_cast(
+          float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, m), j));
+      rank += v > m || (v == m && j < lane);
+    }
+    if (rank > 0) atomicAdd(&ranks[lane], rank);
+    __syncthreads();
     if (tid < 64) {
-#pragma unroll
-      for (int w = 0; w < 16; ++w) m = fmaxf(m, top[w][lane]);
-      int rank = 0;
-#pragma unroll
-      for (int j = 0; j < 64; ++j) {
-        const float v = __builtin_bit_cast(
-            float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, m), j));
-        rank += v > m || (v == m && j < lane);
-      }
-      if (rank == k - 1) thresh = m;
+      if (ranks[lane] == k - 1) thresh = m;
+      ranks[lane] = 0;
     }
     __syncthreads();
     return thresh;
   };
 
-  float m = -INFINITY;
+  float m = -INFINITY, first[2];
   const float* spans = o.spans + (long)me * o.S;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int s = tid + i * 1024;
+    first[i] = s < o.S ? spans[s] : -INFINITY;
+    m = fmaxf(m, first[i]);
+  }
 #pragma unroll 2
-  for (int s = tid; s < o.S; s += 1024) m = fmaxf(m, spans[s]);
+  for (int s = tid + 2048; s < o.S; s += 1024) m = fmaxf(m, spans[s]);
   float least = bound(m);
   if (m >= least - margin)
-    for (int s = tid; s < o.S; s += 1024)
-      if (spans[s] >= least - margin) {
+    for (int s = tid, i = 0; s < o.S; s += 1024, ++i) {
+      const float v = i == 0 ? first[0] : i == 1 ? first[1] : spans[s];
+      if (v >= least - margin) {
         const int to = atomicAdd(&nspan, 1);
         if (to < NS_SPANS) span[to] = s;
       }
+    }
   __syncthreads();
   if (nspan > NS_SPANS) return unsure();
 
