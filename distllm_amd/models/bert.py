@@ -147,10 +147,10 @@ class BertEncoder(nn.Module):
             nz = (ids != pad).int()
             pos2d = (nz.cumsum(1) * nz + pad).long()
         if token_type_ids is None:
-            x = ops.embed_layer_norm(ids, pos2d, self.word_emb, self.pos_emb,
-                                     self.type_emb[0], self.emb_ln_w,
-                                     self.emb_ln_b,
-                                     self.dims.layer_norm_eps)
+            x, mask_f = ops.embed_with_bias(
+                ids, pos2d, attention_mask, self.word_emb, self.pos_emb,
+                self.type_emb[0], self.emb_ln_w, self.emb_ln_b,
+                self.dims.layer_norm_eps)
         else:
             if pos2d is None:
                 pos2d = torch.arange(S, device=ids.device)[None, :]
@@ -158,7 +158,7 @@ class BertEncoder(nn.Module):
                  + self.type_emb[token_type_ids.long()])
             x = ops.layer_norm(x, self.emb_ln_w, self.emb_ln_b,
                                eps=self.dims.layer_norm_eps)
-        mask_f = ops.key_bias(attention_mask)
+            mask_f = ops.key_bias(attention_mask)
         out = self._few_rows(x, mask_f)
         if out is not None:
             return out

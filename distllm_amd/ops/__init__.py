@@ -714,18 +714,37 @@ def rope_attn_varlen_(qkv, cs, sn, pos, H, HKV, cu_seqlens, block_map=None,
         cs, sn, pos)
 
 
+def _embeds(word, pos, type_row):
+    return (word.is_cuda and word.dtype == torch.bfloat16
+            and word.shape[1] % 8 == 0
+            and all(t.is_contiguous() for t in (word, pos, type_row)))
+
+
 def embed_layer_norm(ids, pos_ids, word, pos, type_row, w, b, eps):
     """Layer norm of word[ids] + pos[pos_ids] + type_row; pos_ids None:
     positions 0, 1, ... of every row of ids [B, S]."""
-    if (word.is_cuda and word.dtype == torch.bfloat16
-            and word.shape[1] % 8 == 0
-            and all(t.is_contiguous() for t in (word, pos, type_row))):
+    if _embeds(word, pos, type_row):
         _require_hip()
         return _hip_ops.embed_layer_norm(
             ids.contiguous(), None if pos_ids is None
             else pos_ids.contiguous(), word, pos, type_row, w, b, eps)
     p = pos[: ids.shape[1]][None] if pos_ids is None else pos[pos_ids]
     return layer_norm(word[ids] + p + type_row, w, b, eps=eps)
+
+
+def embed_with_bias(ids, pos_ids, mask, word, pos, type_row, w, b, eps):
+    """embed_layer_norm, and key_bias of mask: in one launch where both are the
+    kernels' and mask has a number per token."""
+    if (_embeds(word, pos, type_row) and mask.shape == ids.shape
+            and mask.device == ids.device and not mask.is_floating_point()
+            and not mask.is_complex() and mask.element_size() in (1, 4, 8)):
+        _require_hip()
+        return _hip_ops.embed_with_bias(
+            ids.contiguous(), None if pos_ids is None
+            else pos_ids.contiguous(), word, pos, type_row, w, b, eps,
+            mask.contiguous())
+    return (embed_layer_norm(ids, pos_ids, word, pos, type_row, w, b, eps),
+            key_bias(mask))
 
 
 def key_bias(mask):

@@ -26,7 +26,7 @@ int mean_pool_shares(int, int);
 void launch_embed_layer_norm(const long*, const long*, const void*,
                              const void*, const void*, const void*,
                              const void*, void*, long, int, int, long, long,
-                             float, hipStream_t);
+                             float, const void*, int, float*, hipStream_t);
 void launch_key_bias(const void*, float*, long, int, hipStream_t);
 void launch_rope_inplace(void*, const float*, const float*, const int*, long,
                          long, int, int, hipStream_t);
@@ -373,11 +373,20 @@ void rope_inplace(torch::Tensor x, torch::Tensor cs, torch::Tensor sn,
 }
 
 // ---- encoder inputs ---------------------------------------------------------
-torch::Tensor embed_layer_norm(torch::Tensor ids,
-                               c10::optional<torch::Tensor> pos_ids,
-                               torch::Tensor word, torch::Tensor pos,
-                               torch::Tensor type, torch::Tensor w,
-                               torch::Tensor b, double eps) {
+static int mask_bytes(const torch::Tensor& mask) {
+  CHECK_DEV(mask); CHECK_CONT(mask);
+  const int bytes = mask.element_size();
+  TORCH_CHECK(!mask.is_floating_point() && !mask.is_complex() &&
+                  (bytes == 1 || bytes == 4 || bytes == 8),
+              "mask must be of 8, 32 or 64 bit integers or truth values");
+  return bytes;
+}
+
+// The layer norm, and the key bias of a mask that is there.
+static std::vector<torch::Tensor> embed_tokens(
+    torch::Tensor ids, c10::optional<torch::Tensor> pos_ids,
+    torch::Tensor word, torch::Tensor pos, torch::Tensor type, torch::Tensor w,
+    torch::Tensor b, double eps, c10::optional<torch::Tensor> mask) {
   CHECK_DEV(ids); CHECK_CONT(ids);
   TORCH_CHECK(ids.scalar_type() == at::kLong && ids.dim() == 2,
               "ids must be int64 [B, S]");
@@ -396,22 +405,43 @@ torch::Tensor embed_layer_norm(torch::Tensor ids,
     TORCH_CHECK(S <= pos.size(0), "more tokens than positions");
   }
   auto out = torch::empty({ids.size(0), S, H}, word.options());
+  torch::Tensor bias;
+  int bytes = 0;
+  if (mask) {
+    bytes = mask_bytes(*mask);
+    TORCH_CHECK(mask->sizes() == ids.sizes() && mask->device() == ids.device(),
+                "a mask number per token");
+    bias = torch::empty(ids.sizes(), ids.options().dtype(at::kFloat));
+  }
   if (ids.numel() > 0)
     launch_embed_layer_norm(
         (const long*)ids.data_ptr<int64_t>(),
         pos_ids ? (const long*)pos_ids->data_ptr<int64_t>() : nullptr,
         word.data_ptr(), pos.data_ptr(), type.data_ptr(), w.data_ptr(),
         b.data_ptr(), out.data_ptr(), ids.numel(), S, H, word.size(0),
-        pos.size(0), (float)eps, cur_stream());
-  return out;
+        pos.size(0), (float)eps, mask ? mask->data_ptr() : nullptr, bytes,
+        mask ? bias.data_ptr<float>() : nullptr, cur_stream());
+  return {out, bias};
+}
+
+torch::Tensor embed_layer_norm(torch::Tensor ids,
+                               c10::optional<torch::Tensor> pos_ids,
+                               torch::Tensor word, torch::Tensor pos,
+                               torch::Tensor type, torch::Tensor w,
+                               torch::Tensor b, double eps) {
+  return embed_tokens(ids, pos_ids, word, pos, type, w, b, eps,
+                      c10::nullopt)[0];
+}
+
+std::vector<torch::Tensor> embed_with_bias(
+    torch::Tensor ids, c10::optional<torch::Tensor> pos_ids,
+    torch::Tensor word, torch::Tensor pos, torch::Tensor type, torch::Tensor w,
+    torch::Tensor b, double eps, torch::Tensor mask) {
+  return embed_tokens(ids, pos_ids, word, pos, type, w, b, eps, mask);
 }
 
 torch::Tensor key_bias(torch::Tensor mask) {
-  CHECK_DEV(mask); CHECK_CONT(mask);
-  const int bytes = mask.element_size();
-  TORCH_CHECK(!mask.is_floating_point() && !mask.is_complex() &&
-                  (bytes == 1 || bytes == 4 || bytes == 8),
-              "mask must be of 8, 32 or 64 bit integers or truth values");
+  const int bytes = mask_bytes(mask);
   auto out = torch::empty(mask.sizes(), mask.options().dtype(at::kFloat));
   if (mask.numel() > 0)
     launch_key_bias(mask.data_ptr(), out.data_ptr<float>(), mask.numel(),
@@ -1140,6 +1170,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("embed_layer_norm", &embed_layer_norm, py::arg("ids"),
         py::arg("pos_ids"), py::arg("word"), py::arg("pos"), py::arg("type"),
         py::arg("w"), py::arg("b"), py::arg("eps"));
+  m.def("embed_with_bias", &embed_with_bias);
   m.def("key_bias", &key_bias);
   m.def("bert_few_rows", &bert_few_rows);
   m.def("score", &score);

@@ -98,3 +98,19 @@ def test_mean_pool_is_rounded_once(device, R, S):
     mask = torch.ones(R, S, device=device, dtype=torch.int32)
     total = x[:, 1:-1].double().sum(1)
     assert torch.equal(ops.mean_pool(x, mask), (total / (S - 2)).float())
+
+
+@pytest.mark.parametrize("H", [8, 520, 768, 2048, 2056, 8192])
+@pytest.mark.parametrize("dtype", [torch.bool, torch.int8, torch.int32,
+                                   torch.int64])
+def test_embed_with_bias(device, H, dtype):
+    """As the two ops on their own, bit for bit."""
+    g = torch.Generator(device=device).manual_seed(H)
+    tables = [torch.randn(*n, H, device=device, generator=g).bfloat16()
+              for n in ((50,), (40,), (), (), ())]
+    ids = torch.randint(0, 50, (3, 37), device=device, generator=g)
+    mask = torch.randint(0, 3, (37, 3), device=device, generator=g).t()
+    mask = (mask * 2 ** 33 if dtype == torch.int64 else mask).to(dtype)
+    x, bias = ops.embed_with_bias(ids, None, mask, *tables, 1e-5)
+    assert torch.equal(x, ops.embed_layer_norm(ids, None, *tables, 1e-5))
+    assert torch.equal(bias, ops.key_bias(mask)) and bias.is_contiguous()
