@@ -946,8 +946,10 @@ def _search_few_fills(Q, N, K):
 
 
 class NarrowRows(NamedTuple):
-    """Rows of a corpus in 16 bits beside it (narrow_search.hip), and what
-    tells whether they are still its."""
+    """Rows of a corpus in 16 bits beside it (narrow_search.hip). They are its
+    until it is written to: holds says whether that was counted, and who keeps
+    them sees to it that nothing writes uncounted (through `.data`, by a kernel, by
+    a replayed graph), after which they would choose wrong rows."""
     rows: torch.Tensor      # f16 [N, K in whole 64s], of the rows times 2^up
     up: int
     error: float            # most that a row and its 16 bits are apart

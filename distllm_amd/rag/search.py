@@ -102,7 +102,42 @@ class HipFlatIndex:
     """GPU-resident flat index over the HF-dataset interchange format
     (columns `text`, `embeddings` fp32)."""
 
+    # the rows once more in 16 bits, which searches read in place of `corpus`
     narrow: ops.NarrowRows | None = None
+
+    @property
+    def corpus(self) -> torch.Tensor:
+        """The rows in fp32. Who has them can write to them in ways that nothing
+        counts (through `.data`, by a kernel, by a replayed graph), and rows in 16
+        bits that are no longer theirs would choose wrong ones. So these are given
+        up, and their memory with them, where the rows are handed out or replaced:
+        searches read fp32 from there on, until renew_narrow."""
+        self.narrow = None
+        try:
+            return self.__dict__["corpus"]
+        except KeyError:
+            raise AttributeError("corpus") from None
+
+    @corpus.setter
+    def corpus(self, rows: torch.Tensor) -> None:
+        self.narrow = None
+        self.__dict__["corpus"] = rows
+
+    @property
+    def _rows(self) -> torch.Tensor:
+        """`corpus`, for what only reads it."""
+        rows = self.__dict__.get("corpus")
+        return self.corpus if rows is None else rows
+
+    def renew_narrow(self) -> None:
+        """Makes the rows in 16 bits, of `corpus` as it is: for a caller that has
+        had it or replaced it, and will not write to it any more. Takes half of
+        its memory again; nothing where they are of no use to the index."""
+        self.narrow = None
+        rows = self.__dict__.get("corpus")
+        if (rows is not None and self.precision == "float32"
+                and self.search_algorithm != "ivf"):
+            self.narrow = ops.narrow_rows(rows)
 
     def __init__(self, dataset_dir: Path, faiss_index_path: Path,
                  dataset_chunk_paths: list[Path] | None = None,
@@ -199,9 +234,7 @@ class HipFlatIndex:
             self.code_words = W
         if self.search_algorithm == "ivf":
             self._build_ivf()
-        elif self.precision == "float32":
-            # the rows once more in 16 bits, which searches read in their place
-            self.narrow = ops.narrow_rows(self.corpus)
+        self.renew_narrow()
 
     def _assign(self, cent: torch.Tensor) -> torch.Tensor:
         """argmax cluster per corpus row, GEMM-chunked so the score
@@ -210,7 +243,7 @@ class HipFlatIndex:
         outs = []
         for r0 in range(0, self.n, rows):
             outs.append(
-                (self.corpus[r0:r0 + rows] @ cent.t()).argmax(1))
+                (self._rows[r0:r0 + rows] @ cent.t()).argmax(1))
         return torch.cat(outs)
 
     def _build_ivf(self) -> None:
@@ -224,14 +257,14 @@ class HipFlatIndex:
         resident in 288 GB HBM."""
         C = self.nlist or max(int(self.n ** 0.5), 1)
         C = min(C, self.n)
-        dev = self.corpus.device
+        dev = self._rows.device
         g = torch.Generator().manual_seed(0)
         init = torch.randperm(self.n, generator=g)[:C]
-        cent = self.corpus[init.to(dev)].clone()
+        cent = self._rows[init.to(dev)].clone()
         ar = torch.arange(C, device=dev)
         for _ in range(10):
             assign = self._assign(cent)
-            sums = torch.zeros_like(cent).index_add_(0, assign, self.corpus)
+            sums = torch.zeros_like(cent).index_add_(0, assign, self._rows)
             cnt = torch.bincount(assign, minlength=C).float()
             keep = cnt > 0
             cent[keep] = sums[keep] / cnt[keep].unsqueeze(1)
@@ -264,7 +297,7 @@ class HipFlatIndex:
                             device=dev)
         gather = idx_pad.clamp(min=0).long().to(dev)
         slabs[:, :, :self.dim].copy_(
-            self.corpus[gather.reshape(-1)].reshape(nch, cap, self.dim))
+            self._rows[gather.reshape(-1)].reshape(nch, cap, self.dim))
         # zero the pad rows (the clamp pointed them at corpus[0]): they
         # must not contribute to chunk means nor produce candidates
         valid = (torch.arange(cap, device=dev)[None, :]
@@ -330,11 +363,11 @@ class HipFlatIndex:
         k = min(k, N)
         chunk = self.score_chunk_rows
         if N <= chunk:
-            return ops.score_topk(q, self.corpus, k)
+            return ops.score_topk(q, self._rows, k)
         vs, is_ = [], []
         for c0 in range(0, N, chunk):
             c1 = min(c0 + chunk, N)
-            v, i = ops.score_topk(q, self.corpus[c0:c1], min(k, c1 - c0))
+            v, i = ops.score_topk(q, self._rows[c0:c1], min(k, c1 - c0))
             vs.append(v)
             is_.append(i + c0)
         allv = torch.cat(vs, 1)
@@ -347,13 +380,17 @@ class HipFlatIndex:
         rows in 16 bits; None where these do not answer it, for want of speed or
         of certainty, or where another search has been put in _topk_exact's
         place or asked for."""
-        if (self.narrow is None or q.dim() != 2
+        narrow = self.narrow
+        if (narrow is None or q.dim() != 2
                 or self.precision != "float32"
                 or self.search_algorithm == "ivf"
                 or getattr(self._topk_exact, "__func__", None)
                 is not HipFlatIndex._topk_exact):
             return None
-        return ops.found_narrow(q, self.corpus, min(k, self.n), self.narrow)
+        if not narrow.holds(self._rows):
+            self.narrow = None
+            return None
+        return ops.found_narrow(q, self._rows, min(k, self.n), narrow)
 
     def _topk_ubinary(self, qfp: torch.Tensor, k: int):
         """Hamming candidates (HIP popcount) + fp32 rescore."""
@@ -364,13 +401,13 @@ class HipFlatIndex:
             qb = np.pad(qb, ((0, 0), (0, pad)))
         q64 = qb.reshape(qb.shape[0], W, 8).copy().view(np.uint64)
         q64 = torch.from_numpy(q64.reshape(qb.shape[0], W).view(np.int64))
-        q64 = q64.to(self.corpus.device)
+        q64 = q64.to(self._rows.device)
         scores = ops.hamming_score(q64, self.codes_t)  # [Q, N] = -dist
         kk = min(k * self.rescore_multiplier, self.n)
         _, cand = ops.topk(scores, kk)
         # rescore candidates with fp32 inner product
-        gathered = self.corpus[cand.long()]            # [Q, kk, H]
-        res = torch.einsum("qh,qkh->qk", qfp.to(self.corpus.device),
+        gathered = self._rows[cand.long()]            # [Q, kk, H]
+        res = torch.einsum("qh,qkh->qk", qfp.to(self._rows.device),
                            gathered)
         v, sel = torch.topk(res, min(k, kk), dim=1)
         return v, cand.gather(1, sel).int()
@@ -382,7 +419,7 @@ class HipFlatIndex:
             np.ascontiguousarray(query_embedding, dtype=np.float32))
         lists = self._found_narrow(q, top_k)
         if lists is None:
-            q = q.to(self.corpus.device)
+            q = q.to(self._rows.device)
         if lists is not None:
             pass
         elif self.precision == "ubinary":

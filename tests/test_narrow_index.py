@@ -1,0 +1,85 @@
+"""An index's rows in 16 bits beside its corpus: when they are its, on the CPU with
+a stand-in for the search by them."""
+from contextlib import nullcontext as _nothing
+
+import numpy as np
+import pytest
+import torch
+from datasets import Dataset
+
+from distllm_amd import ops
+from distllm_amd.rag.search import HipFlatIndex
+
+
+@pytest.fixture
+def by_narrow(monkeypatch):
+    """Searches by the rows in 16 bits, which answer nothing here."""
+    calls = []
+
+    def rows(corpus):
+        return ops.NarrowRows(corpus.half(), 0, 0.0, 1.0, corpus,
+                              corpus._version)
+
+    monkeypatch.setattr(ops, "narrow_rows", rows)
+    monkeypatch.setattr(ops, "found_narrow",
+                        lambda *a: calls.append(a) and None)
+    return calls
+
+
+@pytest.fixture
+def index(tmp_path, by_narrow):
+    c = torch.randn(50, 8, generator=torch.Generator().manual_seed(1))
+    Dataset.from_dict({"text": ["a"]}).save_to_disk(str(tmp_path / "d"))
+    np.savez(tmp_path / "i.npz", embeddings=c.numpy())
+    return HipFlatIndex(tmp_path / "d", tmp_path / "i.npz", device="cpu")
+
+
+def _search(index, by_narrow):
+    """Whether the rows in 16 bits were asked; the answer is the corpus's."""
+    q = torch.randn(3, 8, generator=torch.Generator().manual_seed(2))
+    by_narrow.clear()
+    found = index.search(q.numpy(), 4)
+    want = (q @ vars(index)["corpus"].t()).topk(4).indices.tolist()
+    assert found.total_indices == want
+    return len(by_narrow) > 0
+
+
+@pytest.mark.parametrize("write", [
+    lambda c: c.mul_(-1), lambda c: c.data.mul_(-1),
+    lambda c: c.numpy().__imul__(-1)], ids=["counted", "data", "memory"])
+def test_rows_that_may_have_been_written_to(index, by_narrow, write):
+    assert _search(index, by_narrow) and _search(index, by_narrow)
+    write(index.corpus)
+    assert not _search(index, by_narrow)
+    assert index.narrow is None
+    index.renew_narrow()
+    assert _search(index, by_narrow)
+
+
+def test_rows_that_were_replaced(index, by_narrow):
+    index.corpus = -vars(index)["corpus"]
+    assert index.narrow is None and not _search(index, by_narrow)
+    index.renew_narrow()
+    assert index.narrow.corpus is vars(index)["corpus"]
+    assert _search(index, by_narrow)
+
+
+def test_counted_writes_by_who_has_the_rows(index, by_narrow):
+    rows = index.corpus
+    index.renew_narrow()
+    rows.mul_(-1)
+    assert not _search(index, by_narrow) and index.narrow is None
+
+
+@pytest.mark.parametrize("args", [{"precision": "ubinary"},
+                                  {"search_algorithm": "ivf"}])
+def test_indices_without(index, tmp_path, by_narrow, args):
+    with pytest.warns() if "precision" in args else _nothing():
+        other = HipFlatIndex(tmp_path / "d", tmp_path / "i.npz", device="cpu",
+                             **args)
+    assert other.narrow is None
+
+
+def test_no_corpus():
+    with pytest.raises(AttributeError):
+        HipFlatIndex.__new__(HipFlatIndex).corpus
