@@ -228,14 +228,14 @@ class LatentAttention(Part):
         return (max(self.dp, self.vp) <= 256
                 and (w.dtype == torch.bfloat16 or not w.is_cuda))
 
-    def forward(self, h, batch, latents, linear=None):
+    def forward(self, h, batch, latents, linear=None, down=None):
         """h [M, width]; latents: the paged cache [blocks, BLK, rank] of
-        the layer that owns it; linear: the form of the products that a norm
-        follows, the first and the last, ops.linear if none is given."""
+        the layer that owns it; linear and down: the last and the first
+        product's forms, ops.linear if none is given."""
         d, H = self.d, self.d.heads
         M = h.shape[0]
         bt, ctx = batch.block_table, batch.ctx
-        ab = (linear or ops.linear)(h, self.wdown)
+        ab = (down or ops.linear)(h, self.wdown)
         cq = ops.latent_prep(ab, self.qp, d.q_rank, d.kv_rank, self.q_norm,
                              self.kv_norm, self.eps,
                              latents if self.own else None, bt,

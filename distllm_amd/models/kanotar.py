@@ -32,6 +32,19 @@ def _shared(part) -> dict:
             else {})
 
 
+def _forms(part) -> dict:
+    """The forms of a sublayer's products that a norm follows: _shared, and where
+    a hook sees the output the same sums, joined, so that watching changes no
+    result. Nothing sees the product that a mixer's own norms follow."""
+    forms = _shared(part)
+    if (not forms and type(part) in (ClampedGlu, LatentAttention)
+            and "forward" not in part.__dict__ and ops.linear is _LINEAR):
+        forms = {"linear": ops.linear_joined}
+    if forms and type(part) is LatentAttention:
+        forms["down"] = ops.linear_parts
+    return forms
+
+
 class KanotarModel(LayeredModel):
     layer_norms = ("norm1", "norm1b")
     mlp_norms = ("norm2", "norm2b")
@@ -46,13 +59,13 @@ class KanotarModel(LayeredModel):
             after = (self.layers[i + 1].norm1 if i + 1 < len(self.layers)
                      else self.final_norm)
             y = layer.mixer(h, batch, cache.layers[i],
-                            **_shared(layer.mixer))
+                            **_forms(layer.mixer))
             if layer.mlp is None:
                 h = ops.post_norm_add(y, x, layer.norm1b, after, W, eps)
             else:
                 h = ops.post_norm_add(y, x, layer.norm1b, layer.norm2, W,
                                       eps)
-                h = ops.post_norm_add(layer.mlp(h, **_shared(layer.mlp)), x,
+                h = ops.post_norm_add(layer.mlp(h, **_forms(layer.mlp)), x,
                                       layer.norm2b, after, W, eps)
             if trace is not None:
                 trace.append(x[:, :W].clone())

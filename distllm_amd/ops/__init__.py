@@ -480,6 +480,20 @@ def linear_parts(x, weight, bias=None):
     return linear(x2, weight, bias)
 
 
+def linear_joined(x, weight):
+    """linear, whose sums are those of linear_parts' slabs in every bit: for a
+    consumer that wants [M, N] where another of the same numbers takes slabs (of
+    17 to 32 rows linear may be another split of K)."""
+    x2 = x.reshape(-1, x.shape[-1])
+    M, K = x2.shape
+    if x.is_cuda and 0 < M <= 64 and _gemm_mode() not in _OTHER_FORMS:
+        _require_hip("_hip_gemm")
+        if (_few_rows(x2, weight)
+                and _hip_ops.decode_parts_shares(M, weight.shape[0], K) > 1):
+            return _hip_ops.decode_gemm_joined(x2, weight)
+    return linear(x2, weight)
+
+
 def _norm_in_product(a, b, w_norm, weight, least):
     """Whether a + b is one row whose norm the product of it with `weight`
     takes into its launch (csrc/norm_row.h): up to 8192 columns, at least

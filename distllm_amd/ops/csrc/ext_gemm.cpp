@@ -84,13 +84,14 @@ static torch::Tensor decode_gemm_act(torch::Tensor X, torch::Tensor W,
                                      double limit, double alpha,
                                      double shift,
                                      c10::optional<torch::Tensor> act_nums,
-                                     const RowsArgs* rows) {
+                                     const RowsArgs* rows,
+                                     bool as_parts = false) {
   // act 1, 2 = packed gated unit (swiglu, clamped with the given constants):
   // W is [2I, K] (gate rows then up rows), output is [M, I]. act 3 = xIELU
   // with the raw numbers act_nums [2]. act 4 = GELU times a part of a table's
   // row. act 5 = relu(.)^2. act 6, 7, 8 = GELU (tanh, erf), SiLU. splitk
   // workgroups share K (activations: not 1); 0: form and split follow from
-  // the sizes.
+  // the sizes, as_parts: the split of decode_gemm_parts.
   CHECK_DEV(X); CHECK_CONT(X); CHECK_BF16(X);
   CHECK_DEV(W); CHECK_CONT(W); CHECK_BF16(W);
   const int M = X.size(0), K = X.size(1), N = W.size(0);
@@ -98,7 +99,9 @@ static torch::Tensor decode_gemm_act(torch::Tensor X, torch::Tensor W,
   TORCH_CHECK(M <= 256, "decode_gemm is for M <= 256");
   TORCH_CHECK(N % 64 == 0, "N % 64");
   const bool tile = splitk != 0;
-  if (!tile) splitk = decode_gemm_shares(M, N, K);
+  if (!tile)
+    splitk = as_parts ? decode_parts_shares(M, N, K)
+                      : decode_gemm_shares(M, N, K);
   TORCH_CHECK(splitk > 0 && K % (64 * splitk) == 0, "K % (64*splitk)");
   const bool glu = act == 1 || act == 2;
   TORCH_CHECK(act == 0 || !tile || splitk > 1,
@@ -145,6 +148,11 @@ torch::Tensor decode_gemm(torch::Tensor X, torch::Tensor W,
   TORCH_CHECK(act >= 0 && act <= 9 && act != 4, "activation");
   return decode_gemm_act(X, W, bias, splitk, act, limit, alpha, shift,
                          act_nums, nullptr);
+}
+
+// The slabs of decode_gemm_parts, joined.
+torch::Tensor decode_gemm_joined(torch::Tensor X, torch::Tensor W) {
+  return decode_gemm_act(X, W, {}, 0, 0, 0., 0., 0., {}, nullptr, true);
 }
 
 // X W^T as the fp32 slabs [shares, M, N] of the workgroups that share K, for
@@ -414,6 +422,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("mid_gemm_shares", &mid_gemm_shares);
   m.def("norm_gemm", &norm_gemm);
   m.def("decode_gemm_parts", &decode_gemm_parts);
+  m.def("decode_gemm_joined", &decode_gemm_joined);
   m.def("decode_gemm_shares", &decode_gemm_shares);
   m.def("decode_parts_shares", &decode_parts_shares);
   m.def("decode_gemm_rows", &decode_gemm_rows);

@@ -13,6 +13,7 @@ import torch
 import kanotar_cases as cases
 import kanotar_oracle as oracle
 from distllm_amd import ops
+from distllm_amd.engine.engine import LLMEngine, _Seq
 from distllm_amd.models import build_model, kanotar
 from distllm_amd.models.config import layered_preset
 from distllm_amd.ops import torch_ref
@@ -208,6 +209,36 @@ def test_sublayers_that_are_watched(device):
     for p in parts:
         total += p
     assert torch.equal(total.bfloat16(), want)
+
+
+@pytest.mark.parametrize("rows", [16, 17, 32, 40])
+def test_watching_layers_changes_no_logits(device, rows):
+    """Hooks on layers whose every product that a norm follows has another split
+    of K than on its own (17 to 32 rows): bit for bit."""
+    model = build_model(layered_preset(
+        2, 4096, 64, 32, 64, 128, 1536, 512, 2048, [64], limit=7.0),
+        device=device)
+    with torch.no_grad():
+        for p in model.parameters():
+            p.normal_(0, 0.03)
+    prompt = torch.arange(rows).mul(7).remainder(64).tolist()
+    engine = LLMEngine(model, max_batch_size=1, max_model_len=64)
+
+    def logits():
+        seq = _Seq(seq_id=0, prompt_ids=prompt)
+        out = engine.step([(seq, prompt)], [list(range(rows))])
+        engine.release(seq)
+        return out.clone()
+
+    want, seen = logits(), []
+    hooks = [p.register_forward_hook(lambda m, i, o: seen.append(o))
+             for layer in model.layers for p in (layer.mixer, layer.mlp)]
+    got = logits()
+    for h in hooks:
+        h.remove()
+    assert [(o.dtype, o.dim()) for o in seen] == [(BF16, 2)] * 4
+    assert rows <= seen[0].shape[0] <= 64
+    assert torch.equal(got, want)
 
 
 @pytest.mark.parametrize("dtype", DTYPES, ids=ids)

@@ -134,6 +134,19 @@ def test_shares_in_place_of_the_ring(device, M, N, K, shares):
     assert ((total - want).abs() <= bound).all()
 
 
+@pytest.mark.parametrize("M", [1, 16, 17, 32, 33, 64, 65])
+@pytest.mark.parametrize("N, K", [(4096, 4096), (2048, 4096), (6144, 2048),
+                                  (768, 768), (1024, 8192)])
+def test_shares_joined(device, M, N, K):
+    """The slabs' sum, one after the other, rounded once."""
+    x, w = _rand(M, K), _rand(N, K, seed=1)
+    parts = ops.linear_parts(x, w)
+    total = parts if parts.dim() == 2 else torch.zeros_like(parts[0])
+    for p in parts if parts.dim() == 3 else ():
+        total += p
+    assert torch.equal(ops.linear_joined(x, w), total.to(BF16))
+
+
 @pytest.mark.parametrize("S", [2, 3, 8])
 @pytest.mark.parametrize("QP, qn, R, rn", [(128, 100, 192, 130),
                                            (1536, 1536, 512, 512),
