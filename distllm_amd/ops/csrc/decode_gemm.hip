@@ -195,9 +195,11 @@ dg_ring_kernel(const u16* __restrict__ X, const u16* __restrict__ W, int K,
       src[NT + t][p] =
           X + (long)min(t * 16 + p * 8 + lr, e.M - 1) * K + lc;
   }
-  // chunks wid, wid + NW, ... from the block's first one on
+  // chunks wid, wid + NW, ... from the block's first one on: halves have that of the
+  // 16 columns, so that a column's sum has one order in all forms (it costs nothing)
   const int nch = K / 64, mine = (nch - wid + NW - 1) / NW;
-  const int turn = chunk_turn<37>(blockIdx.x, nch) + wid;
+  const int turn =
+      chunk_turn<37>(HALF ? blockIdx.x / 2 : blockIdx.x, nch) + wid;
   auto issue = [&](int c) {
     char* dst = ring + (c % R) * STAGE + lane * 16;
     int k = c * NW + turn;

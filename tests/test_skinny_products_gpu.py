@@ -96,6 +96,35 @@ def test_columns_even_on_the_card(device, M, N, K, shares):
         _close(ops._hip_ops.decode_gemm_parts(x, w).sum(0), z)
 
 
+@pytest.mark.parametrize("M", [1, 8, 24, 64])
+@pytest.mark.parametrize("N, K", [(64, 2048), (1024, 4096), (2048, 2176),
+                                  (2112, 2048)])
+def test_sums_are_in_one_order(device, M, N, K):
+    """Of 8 columns a workgroup (up to 2048) as of 16, which a 32-bit result and
+    a row with its norm ahead have: of products that cancel each other what is
+    left are the roundings on the way."""
+    g = torch.Generator(device=device).manual_seed(N + K + M)
+
+    def randn(*shape):
+        return torch.randn(*shape, device=device, generator=g).bfloat16()
+
+    def twice(t, sign=1):
+        return torch.cat((t, sign * t.flip(-1)), -1).contiguous()
+
+    w = randn(N, K // 2) * 2.0 ** torch.randint(0, 12, (N, K // 2),
+                                                device=device, generator=g)
+    w = twice(w.bfloat16(), -1)
+    x = twice(randn(M, K // 2))
+    want = ops.linear(x, w)
+    assert want.any()
+    assert torch.equal(ops.linear_f32(x, w), want.float())
+    if M == 1:
+        a, nw = twice(randn(1, K // 2)), twice(randn(K // 2))
+        got, _ = ops.norm_linear(a, x, nw, 1e-5, w)
+        h, _ = ops.norm_fwd_sum(a, x, nw, rms=True)
+        assert torch.equal(got, ops.linear(h, w))
+
+
 def test_refusals(device):
     x, w, _ = _inputs(4, 128, 128, device, 1)
     for args in ((x, w, None, 1, 1), (x, w, None, 3), (x, w, None, 0, 4),
