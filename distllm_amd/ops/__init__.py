@@ -1003,12 +1003,29 @@ def narrow_rows(corpus):
                        version) if norm <= 4 * usual else None)
 
 
-def _narrow_fills(Q, N):
+def _narrow_fills(Q, N, K, k):
     """Whether found_narrow is faster than score_topk of queries copied to the
-    GPU and found_lists of that. Measured over 64 to 250000 rows of 384 and 768,
-    k = 10, own time over theirs: 1 to 4 queries 0.45 to 0.73, 5 to 256 0.32 to
-    0.83, 1000 of 2000 rows on 0.63 to 0.99, of fewer rows 0.94 to 1.08."""
-    return Q <= 256 or N >= 2048
+    GPU and found_lists of that: half of the rows' bytes are spared, and the rows
+    that may be among the best, more with k, are read by one workgroup of each
+    query. Unit vectors, own time over theirs:
+    - to 1536 columns, 64 to 250000 rows, up to 256 queries 0.32 to 1.00, but
+      for 17 and more queries of few thousand rows and large k, 0.95 to 1.13
+      (1536 columns, 4000 rows, k = 60, one query 1.04); 600 and 1000 queries
+      from 2048 rows on 0.37 to 1.0 (of 2000 to 4000 and large k up to 1.10),
+      of fewer 0.98 to 1.08;
+    - beyond by k and the rows. 2048 columns, k of 1, 10, 60, the slowest of 1
+      to 256 queries: 1000 rows 1.01, 1.05, 1.40, 4000 0.91, 0.97, 1.52, 32000
+      0.70, 0.77, 0.94; 4096: 4000 rows 1.37, 1.47, 2.28, 16000 0.89, 0.99,
+      1.55, 32000 0.72, 0.78, 1.31, 125000 0.60, 0.64, 0.97; 8192: 4000 rows
+      1.8, 2.1, 3.8, 32000 0.72, 1.03, 2.2, 125000 0.60, 0.70, 1.20; 16384,
+      64000 rows 0.91, 1.43, above 2. 600 and 1000 queries of 4096: 4000 rows
+      0.95, 0.98, 1.21, 16000 0.81, 0.89, 1.04; 8192: 16000 0.75, 0.91, 1.19,
+      64000 0.49, 0.57, 0.93."""
+    if K > 8192 or (Q > 256 and N < 2048):
+        return False
+    if K > 1536:
+        return N >= K * (1 + 0.12 * k if Q > 256 else 2.6 + 0.4 * k)
+    return K * k <= 26000 or N >= 8000 or (Q <= 16 and K * k <= 80000)
 
 
 def found_narrow(q, corpus, k, narrow):
@@ -1020,7 +1037,7 @@ def found_narrow(q, corpus, k, narrow):
     if not (0 < Q < 1 << 20 and 0 < k <= min(60, N)
             and q.dtype == torch.float32 and q.device.type == "cpu"
             and tuple(corpus.shape[1:]) == (K,) and narrow.holds(corpus)
-            and _narrow_fills(Q, N) and q.is_contiguous()
+            and _narrow_fills(Q, N, K, k) and q.is_contiguous()
             and 0 < _hip_ops.narrow_bytes(Q, N, K, narrow.rows.shape[1])
             <= 1 << 31):
         return None

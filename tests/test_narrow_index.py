@@ -83,3 +83,18 @@ def test_indices_without(index, tmp_path, by_narrow, args):
 def test_no_corpus():
     with pytest.raises(AttributeError):
         HipFlatIndex.__new__(HipFlatIndex).corpus
+
+
+@pytest.mark.parametrize("Q, N, K, k, by", [
+    # own time over the general way's, measured
+    (1, 250000, 768, 5, True), (256, 250000, 768, 10, True),  # 0.58, 0.49
+    (4, 64, 384, 10, True), (1000, 4000, 1024, 20, True),  # 0.5, 0.94
+    (1, 32000, 2048, 60, False), (1, 64000, 2048, 60, True),  # 0.94, 0.82
+    (1, 4000, 2048, 60, False), (64, 4000, 8192, 60, False),  # 1.5, 1.9
+    (1, 1000, 4096, 1, False), (1, 4000, 8192, 60, False),  # 1.3, 3.5
+    (16, 20000, 4096, 60, False), (1, 250000, 4096, 60, True),  # 1.25, 0.77
+    (4, 1000, 1536, 20, True), (17, 2000, 1536, 60, False),  # 0.63, 1.13
+    (600, 16000, 4096, 20, True), (600, 4000, 8192, 60, False),  # 0.94, 1.6
+    (1, 32000, 16384, 10, False), (1000, 1000, 384, 10, False)])  # 1.9, 1.0
+def test_where_rows_in_16_bits_are_the_faster_way(Q, N, K, k, by):
+    assert ops._narrow_fills(Q, N, K, k) == by
