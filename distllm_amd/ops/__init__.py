@@ -1028,10 +1028,12 @@ def _narrow_fills(Q, N, K, k):
     return K * k <= 26000 or N >= 8000 or (Q <= 16 and K * k <= 80000)
 
 
-def found_narrow(q, corpus, k, narrow):
+def found_narrow(q, corpus, k, narrow, general=None):
     """found_lists of score_topk for queries [Q, K] of the host, by way of the
-    corpus's NarrowRows: None where that is not the faster way, these cannot
-    answer a query, or there is no room for what it takes."""
+    corpus's NarrowRows: None where that is not the faster way, or there is no room
+    for what it takes. Queries that these cannot answer (infinite or NaN numbers,
+    of far more rows nearly as good as the best) go on to general(queries, k),
+    on the corpus's device, score_topk of them if it is not given."""
     Q, K = q.shape
     N = corpus.shape[0]
     if not (0 < Q < 1 << 20 and 0 < k <= min(60, N)
@@ -1042,10 +1044,18 @@ def found_narrow(q, corpus, k, narrow):
             <= 1 << 31):
         return None
     try:
-        return _hip_ops.narrow_found(q, corpus, narrow.rows, narrow.up,
-                                     narrow.error, narrow.norm, k)
+        found = _hip_ops.narrow_found(q, corpus, narrow.rows, narrow.up,
+                                      narrow.error, narrow.norm, k, True)
     except torch.OutOfMemoryError:
         return None
+    scores, indices, rest = found
+    if rest:
+        left = (q if len(rest) == Q else q[rest]).to(corpus.device)
+        v, i = (general(left, k) if general is not None
+                else score_topk(left, corpus, k))
+        for at, s, x in zip(rest, *found_lists(v.float(), i.int())):
+            scores[at], indices[at] = s, x
+    return scores, indices
 
 
 def score_topk(q, corpus, k):

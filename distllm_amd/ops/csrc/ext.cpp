@@ -8,6 +8,7 @@
 #include <cmath>
 #include <cstring>
 #include <limits>
+#include <numeric>
 
 #include "ahead.h"
 #include "ext_common.h"
@@ -62,6 +63,11 @@ long narrow_bytes(long, long, long, long);
 void launch_narrow_topk(const float*, const float*, const void*, void*, float*,
                         int*, int, int, int, int, int, float, float, int,
                         hipStream_t);
+int narrow_again_most();
+long narrow_again_bytes(int);
+void launch_narrow_again(const float*, void*, const int*, int,
+                         unsigned long long*, float*, int*, int, int, int, int,
+                         int, hipStream_t);
 void launch_topk_chunk(const float*, const int*, float*, int*, int, long, int,
                        int, bool, hipStream_t);
 void launch_hamming_score(const void*, const void*, float*, int, long, int,
@@ -1096,16 +1102,21 @@ static std::pair<py::list, py::list> found_lists(torch::Tensor v,
 // found_lists of narrow_topk of queries that the host has, in one call: the GPU reads
 // them and writes its answer where the host has them (pinned memory of torch's cache,
 // given back when the stream has been waited for), which spares two copies and their
-// waits. Above 16 MB they are copied: pinned memory stays with the process. Nothing
-// (None) where a query is not answered. us of 250000 rows of 768, the same work by way
-// of copies and found_lists, and so: one query 109 and 96, 256 230 and 205.
+// waits. Above 16 MB they are copied: pinned memory stays with the process. us of
+// 250000 rows of 768, the same work by way of copies and found_lists, and so: one query
+// 109 and 96, 256 230 and 205.
+// With rest: queries that narrow_topk left for near rows are asked again, one that is
+// all 0 has the first rows with scores of 0, and those that are still unanswered are
+// returned, as a third list, with nothing in their lists. Without, nothing (None) if
+// narrow_topk left one.
 static py::object narrow_found(torch::Tensor q, torch::Tensor corpus,
                                torch::Tensor rows, int64_t up, double error,
-                               double norm, int64_t k) {
+                               double norm, int64_t k, bool rest) {
   const long bytes = check_narrow(q, corpus, rows, up, k);
   TORCH_CHECK(q.device().is_cpu(), "queries of the host");
   const int64_t Q = q.size(0), K = q.size(1), n = Q * k;
   torch::Tensor answer;
+  std::vector<int> left;
   {
     py::gil_scoped_release others;
     const c10::DeviceGuard guard(corpus.device());
@@ -1116,7 +1127,7 @@ static py::object narrow_found(torch::Tensor q, torch::Tensor corpus,
                                     : corpus.options().dtype(t));
     };
     auto asked = place({Q, K}, at::kFloat);
-    answer = place({2, Q, k}, at::kInt);
+    auto told = place({2, Q, k}, at::kInt);
     if (pin)
       std::memcpy(asked.data_ptr(), q.data_ptr(), Q * K * sizeof(float));
     else
@@ -1127,22 +1138,70 @@ static py::object narrow_found(torch::Tensor q, torch::Tensor corpus,
       return p;
     };
     auto space = torch::empty({bytes}, corpus.options().dtype(at::kByte));
-    int* to = (int*)seen(answer);
+    int* to = (int*)seen(told);
     const hipStream_t stream = cur_stream();
+    const int N = (int)corpus.size(0), KP = (int)rows.size(1);
     launch_narrow_topk((const float*)seen(asked), corpus.data_ptr<float>(),
                        rows.data_ptr(), space.data_ptr(), (float*)to, to + n,
-                       (int)Q, (int)corpus.size(0), (int)K, (int)rows.size(1),
-                       (int)up, (float)error, (float)norm, (int)k, stream);
+                       (int)Q, N, (int)K, KP, (int)up, (float)error,
+                       (float)norm, (int)k, stream);
     // (waited for also where a launch failed: the others read what is given back)
-    const hipError_t launched = hipGetLastError();
-    C10_HIP_CHECK(hipStreamSynchronize(stream));
-    C10_HIP_CHECK(launched);
-    if (!pin) answer = answer.cpu();
+    auto wait = [&]() {
+      const hipError_t launched = hipGetLastError();
+      C10_HIP_CHECK(hipStreamSynchronize(stream));
+      C10_HIP_CHECK(launched);
+      answer = pin ? told : told.cpu();
+    };
+    // of those in question the ones whose last row is not known
+    auto unanswered = [&](const std::vector<int>* asked) {
+      std::vector<int> out;
+      const int* last = answer.data_ptr<int>() + n + k - 1;
+      for (int64_t i = 0; i < (asked ? (int64_t)asked->size() : Q); ++i) {
+        const int query = asked ? (*asked)[i] : (int)i;
+        if (last[query * k] == INT_MIN) out.push_back(query);
+      }
+      return out;
+    };
+    wait();
+    left = unanswered(nullptr);
+    if (rest && !left.empty()) {
+      const auto zeros = std::stable_partition(
+          left.begin(), left.end(), [&](int i) {
+            const float* x = q.data_ptr<float>() + i * K;
+            return !std::all_of(x, x + K, [](float f) { return f == 0.f; });
+          });
+      const std::vector<int> first(zeros, left.end());
+      left.erase(zeros, left.end());
+      // (behind these, those that are left for their numbers)
+      const auto other = std::stable_partition(
+          left.begin(), left.end(), [&](int i) {
+            return answer.data_ptr<int>()[i * k] != 0x7f800000;
+          });
+      const int many = (int)(other - left.begin());
+      if (many > 0 && many <= narrow_again_most()) {
+        auto lists = torch::empty({many * narrow_again_bytes((int)k)},
+                                  space.options());
+        launch_narrow_again(corpus.data_ptr<float>(), space.data_ptr(),
+                            left.data(), many,
+                            (unsigned long long*)lists.data_ptr(), (float*)to,
+                            to + n, (int)Q, N, (int)K, KP, (int)k, stream);
+        wait();
+        left = unanswered(&left);
+      }
+      std::sort(left.begin(), left.end());
+      int* found = answer.data_ptr<int>() + n;
+      for (const int i : first) {
+        std::iota(found + i * k, found + (i + 1) * k, 0);
+        std::fill_n(found - n + i * k, k, 0);  // (the bits of 0.f)
+      }
+      for (const int i : left) std::fill_n(found + i * k, k, INT_MIN);
+    }
   }
+  if (!rest && !left.empty()) return py::none();
   const int* at = answer.data_ptr<int>();
-  if (std::count(at + n, at + 2 * n, INT_MIN) > 0) return py::none();
   const auto lists = lists_of(reinterpret_cast<const float*>(at), at + n, Q, k);
-  return py::make_tuple(lists.first, lists.second);
+  if (!rest) return py::make_tuple(lists.first, lists.second);
+  return py::make_tuple(lists.first, lists.second, py::cast(left));
 }
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -1201,7 +1260,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("x") = py::none(), py::arg("w") = py::none(),
         py::arg("eps") = 0.0);
   m.def("found_lists", &found_lists);
-  m.def("narrow_found", &narrow_found);
+  m.def("narrow_found", &narrow_found, py::arg("q"), py::arg("corpus"),
+        py::arg("rows"), py::arg("up"), py::arg("error"), py::arg("norm"),
+        py::arg("k"), py::arg("rest") = false);
   m.def("rope_put", &rope_put, py::arg("qkv"), py::arg("cs"), py::arg("sn"),
         py::arg("ctx"), py::arg("kcache"), py::arg("vcache"),
         py::arg("block_table"), py::arg("bias") = py::none());

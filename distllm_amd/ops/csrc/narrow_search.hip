@@ -12,8 +12,9 @@
 // k rows have products within half of it below the k-th largest one, so a row whose
 // product is more than the whole below that is not among the k best. Where more than
 // NS_CAP groups of four rows are within it (rows that are nearly the same), or a
-// query's numbers are infinite or NaN, the query's indices say NS_UNSURE, and the
-// caller asks the corpus itself. Unit vectors of 768: the margin is 1.3e-3, within which
+// query's numbers are infinite or NaN or all 0, the query's indices say NS_UNSURE. The
+// former are answered by launch_narrow_again, for the latter, whose scores are infinite,
+// the caller asks the corpus itself. Unit vectors of 768: the margin is 1.3e-3, within which
 // a sixth more rows than the k best are. The scores are those of search_top_kernel.
 //
 // Us in a stream, k = 10, score_topk and this, 250000 rows of 768: 1 query 140, 80; 16
@@ -39,6 +40,9 @@ extern __shared__ __attribute__((aligned(16))) char smem[];
 #define NS_SPANS 1024  // spans of rows that a query may have to look into
 #define NS_LIST 1024   // groups that may be near
 #define NS_CAP 256     // groups that are scored
+#define NS_AGAIN 32    // queries that are asked again in a launch
+#define NS_LISTS 256   // lists of their best rows, a workgroup each
+#define NS_PIECE 128   // groups that these score at a time
 
 // ---- rows -------------------------------------------------------------------
 // Bits of the largest magnitude of n numbers, n % 4 == 0, into *most (0 ahead):
@@ -179,8 +183,9 @@ __device__ __forceinline__ float narrow_query(const float* q, float* copy,
 // the GPU and makes what is asked of it.
 __global__ void __launch_bounds__(256)
 narrow_queries_kernel(const float* q, float* copy, u16* __restrict__ out,
-                      float* __restrict__ margin, const NarrowRows c, int Q,
-                      int FN) {
+                      float* __restrict__ margin, int* __restrict__ spent,
+                      const NarrowRows c, int Q, int FN) {
+  if (blockIdx.x == 0 && threadIdx.x < NS_AGAIN) spent[threadIdx.x] = 0;
   const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
   const int block = row / (16 * FN) * FN + row % FN, r = row / FN % 16;
   auto at = [&](int i) {
@@ -531,9 +536,29 @@ narrow_batch_kernel(const char* rows, const char* q16, float* groups,
 // s has the groups s A + j / A B + j % A for j < each.
 struct NarrowMost {
   const float *groups, *spans, *margin;
+  float* limit;  // of a query that is not answered: its best rows' groups are above
   long ld;
   int S, A, B, each, G;
+  __device__ int group(int s, int j) const { return s * A + j / A * B + j % A; }
 };
+
+// Score and place as one number: the larger score, then the smaller row, is the larger.
+__device__ __forceinline__ unsigned long long narrow_key(float v, int row) {
+  return ((unsigned long long)f32_to_ord(v) << 32) | (unsigned int)~row;
+}
+
+// Keys of the rows r0 to r0 + 3, by one wave; 0 past the last.
+__device__ __forceinline__ void narrow_score(const float* query,
+                                             const float* corpus, int r0, int N,
+                                             int K, unsigned long long* keys) {
+  const int lane = threadIdx.x & 63;
+  float s[4];
+  search_dot(query, corpus, r0, N, K, s);
+  if (lane < 4) {
+    const float v = lane == 0 ? s[0] : lane == 1 ? s[1] : lane == 2 ? s[2] : s[3];
+    keys[lane] = r0 + lane < N ? narrow_key(v, r0 + lane) : 0ull;
+  }
+}
 
 // A workgroup per query. The k-th largest of 64 shares of the spans bounds the k-th
 // largest group from below; the spans within the margin of it are looked into, where
@@ -558,13 +583,14 @@ narrow_top_kernel(const NarrowMost o, const float* __restrict__ q,
   const float margin = o.margin[me];
   float* ov = out_v + (long)me * k;
   int* oi = out_i + (long)me * k;
-  auto unsure = [&]() {
+  auto unsure = [&](float limit) {
     if (tid < k) {
-      ov[tid] = -INFINITY;
+      ov[tid] = limit;
       oi[tid] = NS_UNSURE;
     }
+    if (tid == 0) o.limit[me] = limit;
   };
-  if (!(margin < INFINITY)) return unsure();
+  if (!(margin < INFINITY)) return unsure(INFINITY);
   if (tid == 0) nspan = nlist = ncand = 0;
   if (tid < 64) ranks[tid] = 0;
   // the k-th largest of 64 shares' largest, of all threads' m
@@ -612,15 +638,14 @@ narrow_top_kernel(const NarrowMost o, const float* __restrict__ q,
       }
     }
   __syncthreads();
-  if (nspan > NS_SPANS) return unsure();
+  if (nspan > NS_SPANS) return unsure(least - margin);
 
   const int items = nspan * o.each;
   // those within the margin, and the largest number of this thread's
   auto gather = [&]() {
     float m = -INFINITY;
     for (int i = tid; i < items; i += 1024) {
-      const int j = i % o.each, s = span[i / o.each];
-      const int at = s * o.A + j / o.A * o.B + j % o.A;
+      const int at = o.group(span[i / o.each], i % o.each);
       if (at >= o.G) continue;
       const float v = o.groups[at * o.ld + me];
       m = fmaxf(m, v);
@@ -644,11 +669,19 @@ narrow_top_kernel(const NarrowMost o, const float* __restrict__ q,
     gather();
   }
   const int n = nlist;
- if (n > NS_LIST) return unsure();
+  if (n > NS_LIST) return unsure(least - margin);
+  const float own = tid < n ? near[tid] : -INFINITY;
+  if (n > 2 * NS_CAP) {  // (ranks of 750 take 20 us, a bound of them 1)
+    least = fmaxf(least, bound(own));
+    if (own >= least - margin) atomicAdd(&ncand, 1);
+    __syncthreads();
+    if (ncand > 2 * NS_CAP) return unsure(least - margin);
+    __syncthreads();
+    if (tid == 0) ncand = 0;
+  }
   // (fewer groups than k are all that there are)
   if (tid == 0) thresh = -INFINITY;
   __syncthreads();
-  const float own = tid < n ? near[tid] : -INFINITY;
   if (tid < n) {
     int rank = 0;
     for (int j = 0; j < n; ++j)
@@ -662,22 +695,11 @@ narrow_top_kernel(const NarrowMost o, const float* __restrict__ q,
   }
   __syncthreads();
   const int take = ncand;
-  if (take > NS_CAP) return unsure();
+  if (take > NS_CAP) return unsure(thresh - margin);
 
   const float* query = q + (long)me * K;
-  for (int c = wid; c < take; c += 16) {
-    const int r0 = cand[c] * 4;
-    float s[4];
-    search_dot(query, corpus, r0, N, K, s);
-    if (lane < 4) {
-      const float v = lane == 0 ? s[0] : lane == 1 ? s[1] : lane == 2 ? s[2]
-                                                                      : s[3];
-      rows[c * 4 + lane] =
-          r0 + lane < N ? ((unsigned long long)f32_to_ord(v) << 32) |
-                              (unsigned int)~(r0 + lane)
-                        : 0ull;
-    }
-  }
+  for (int c = wid; c < take; c += 16)
+    narrow_score(query, corpus, cand[c] * 4, N, K, rows + c * 4);
   __syncthreads();
   if (tid >= take * 4) return;
   const unsigned long long key = rows[tid];
@@ -687,6 +709,104 @@ narrow_top_kernel(const NarrowMost o, const float* __restrict__ q,
   if (key != 0 && r < k) {
     ov[r] = ord_to_f32((unsigned int)(key >> 32));
     oi[r] = (int)~(unsigned int)key;
+  }
+}
+
+// ---- queries beside many rows that are nearly as good ---------------------------
+// A query that narrow_top_kernel left for them, by NS_LISTS workgroups: each looks
+// into every NS_LISTS-th span, scores the groups above the limit and keeps the k best
+// rows, largest first, as keys, 0 behind them. spent counts the groups of a query;
+// above `most` (the corpus itself is read in less) it is left unanswered.
+// Bound by reading these rows, and by the launches where they are few thousands: a search
+// of 250000 rows of 768 with a question beside 3000 equal ones, us, all questions asked
+// of the corpus and this: one 173 and 136 (101 without such rows), 256 450 and 257 (218);
+// 20 of 256 292.
+struct NarrowAgain {
+  int who[NS_AGAIN];
+};
+
+__global__ void __launch_bounds__(1024)
+narrow_again_kernel(const NarrowMost o, const NarrowAgain a,
+                    const float* __restrict__ q,
+                    const float* __restrict__ corpus,
+                    unsigned long long* __restrict__ lists, int* spent, int most,
+                    int N, int K, int k) {
+  __shared__ unsigned long long keys[64 + NS_PIECE * 4];  // the best, new ones
+  __shared__ int list[1024], near, before;
+  const int tid = threadIdx.x;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int me = a.who[blockIdx.y], first = blockIdx.x;
+  const float limit = o.limit[me];
+  const float* query = q + (long)me * K;
+  const float* spans = o.spans + (long)me * o.S;
+  if (tid < 64) keys[tid] = 0;
+  const int items =
+      limit < INFINITY && first < o.S
+          ? ((o.S - 1 - first) / NS_LISTS + 1) * o.each
+          : 0;
+  for (int i0 = 0; i0 < items; i0 += 1024) {
+    if (tid == 0) near = 0;
+    __syncthreads();
+    const int i = i0 + tid, s = first + i / o.each * NS_LISTS;
+    if (i < items && spans[s] >= limit) {
+      const int at = o.group(s, i % o.each);
+      if (at < o.G && o.groups[at * o.ld + me] >= limit)
+        list[atomicAdd(&near, 1)] = at;
+    }
+    __syncthreads();
+    const int take = near;
+    if (tid == 0) before = take > 0 ? atomicAdd(spent + blockIdx.y, take) : 0;
+    __syncthreads();
+    if (before + take > most) break;
+    for (int c0 = 0; c0 < take; c0 += NS_PIECE) {
+      const int piece = min(take - c0, NS_PIECE), all = 64 + piece * 4;
+      for (int c = wid; c < piece; c += 16)
+        narrow_score(query, corpus, list[c0 + c] * 4, N, K, keys + 64 + c * 4);
+      __syncthreads();
+      const unsigned long long key = tid < all ? keys[tid] : 0;
+      int r = 0;
+#pragma unroll 8
+      for (int j = 0; j < all; ++j) r += keys[j] > key;
+      __syncthreads();
+      if (key != 0 && r < k) keys[r] = key;
+      __syncthreads();
+    }
+  }
+  __syncthreads();
+  if (tid < k)
+    lists[((long)blockIdx.y * NS_LISTS + first) * k + tid] = keys[tid];
+}
+
+// The k best of a query's lists, a thread each.
+__global__ void __launch_bounds__(NS_LISTS)
+narrow_pick_kernel(const NarrowAgain a,
+                   const unsigned long long* __restrict__ lists,
+                   const int* __restrict__ spent, int most,
+                   float* __restrict__ out_v, int* __restrict__ out_i, int k) {
+  __shared__ unsigned long long top[2][NS_LISTS / 64];
+  if (spent[blockIdx.x] > most) return;
+  const long me = a.who[blockIdx.x];
+  const unsigned long long* mine =
+      lists + ((long)blockIdx.x * NS_LISTS + threadIdx.x) * k;
+  unsigned long long key = mine[0];
+  for (int r = 0, at = 0; r < k; ++r) {
+    unsigned long long m = key;
+#pragma unroll
+    for (int d = 1; d < 64; d *= 2) {
+      const unsigned long long other = __shfl_xor(m, d);
+      m = other > m ? other : m;
+    }
+    if ((threadIdx.x & 63) == 0) top[r & 1][threadIdx.x >> 6] = m;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < NS_LISTS / 64; ++w)
+      m = top[r & 1][w] > m ? top[r & 1][w] : m;
+    if (m == 0) return;  // there are none
+    if (key == m) {
+      out_v[me * k + r] = ord_to_f32((unsigned int)(m >> 32));
+      out_i[me * k + r] = (int)~(unsigned int)m;
+      key = ++at < k ? mine[at] : 0;
+    }
   }
 }
 
@@ -710,7 +830,7 @@ namespace {
 // Where things lie beside the operands.
 struct NarrowPlan {
   int QP, fm, fn, grid;  // fn 1: a few queries
-  long copy, q16, margin, groups, spans, bytes;
+  long copy, q16, margin, limit, spent, groups, spans, bytes;
   NarrowMost most;
 };
 
@@ -744,9 +864,20 @@ NarrowPlan narrow_plan(int Q, int N, int K, int KP) {
   p.copy = place((long)Q * K * 4);
   p.q16 = place((long)p.QP * KP * 2);
   p.margin = place((long)Q * 4);
+  p.limit = place((long)Q * 4);
+  p.spent = place(NS_AGAIN * 4);
   p.spans = place(o.S * o.ld * 4);
   p.groups = place(o.G * o.ld * 4);
   return p;
+}
+
+NarrowMost narrow_most(const NarrowPlan& p, char* space) {
+  NarrowMost o = p.most;
+  o.groups = (const float*)(space + p.groups);
+  o.spans = (const float*)(space + p.spans);
+  o.margin = (const float*)(space + p.margin);
+  o.limit = (float*)(space + p.limit);
+  return o;
 }
 
 }  // namespace
@@ -777,7 +908,8 @@ extern "C" void launch_narrow_topk(const float* q, const float* corpus,
         *spans = (float*)(at + p.spans);
   const NarrowRows c = {(const u16*)rows, N, K, KP, up, error, norm};
   hipLaunchKernelGGL(narrow_queries_kernel, dim3(p.QP / 4), dim3(256), 0,
-                     stream, q, copy, q16, margin, c, Q, p.fn);
+                     stream, q, copy, q16, margin, (int*)(at + p.spent), c, Q,
+                     p.fn);
   if (p.fn == 1)
     hipLaunchKernelGGL(narrow_few_kernel, dim3(p.grid), dim3(NF_WAVES * 64),
                        narrow_few_lds(KP), stream, c.rows, q16, groups, spans,
@@ -796,9 +928,32 @@ extern "C" void launch_narrow_topk(const float* q, const float* corpus,
   else
     NS(8, 8);
 #undef NS
-  p.most.groups = groups;
-  p.most.spans = spans;
-  p.most.margin = margin;
-  hipLaunchKernelGGL(narrow_top_kernel, dim3(Q), dim3(1024), 0, stream, p.most,
-                     copy, corpus, out_v, out_i, N, K, k);
+  hipLaunchKernelGGL(narrow_top_kernel, dim3(Q), dim3(1024), 0, stream,
+                     narrow_most(p, at), copy, corpus, out_v, out_i, N, K, k);
+}
+
+// How many queries launch_narrow_again takes, and the bytes of `lists` for each.
+extern "C" int narrow_again_most() { return NS_AGAIN; }
+extern "C" long narrow_again_bytes(int k) { return (long)NS_LISTS * k * 8; }
+
+// The queries who[0] to who[n - 1] of launch_narrow_topk once more, by the same space
+// and into the same out_v and out_i, if it was for near rows that they were left
+// unanswered, up to a share of the corpus (half of it over all of them, beyond which
+// the corpus itself is read in less). Once for a launch_narrow_topk.
+extern "C" void launch_narrow_again(const float* corpus, void* space,
+                                    const int* who, int n,
+                                    unsigned long long* lists, float* out_v,
+                                    int* out_i, int Q, int N, int K, int KP,
+                                    int k, hipStream_t stream) {
+  const NarrowPlan p = narrow_plan(Q, N, K, KP);
+  char* at = (char*)space;
+  int* spent = (int*)(at + p.spent);
+  NarrowAgain a = {};
+  for (int i = 0; i < n; ++i) a.who[i] = who[i];
+  const int most = N / 8 / n;
+  hipLaunchKernelGGL(narrow_again_kernel, dim3(NS_LISTS, n), dim3(1024), 0,
+                     stream, narrow_most(p, at), a, (const float*)(at + p.copy),
+                     corpus, lists, spent, most, N, K, k);
+  hipLaunchKernelGGL(narrow_pick_kernel, dim3(n), dim3(NS_LISTS), 0, stream, a,
+                     lists, spent, most, out_v, out_i, k);
 }

@@ -85,6 +85,35 @@ def test_no_corpus():
         HipFlatIndex.__new__(HipFlatIndex).corpus
 
 
+def test_rows_that_leave_most_questions_are_spared(index, monkeypatch):
+    """Searches go without after those that had to ask again for two fifths and
+    more, one, two, four, ... of them, until one does better."""
+    left, tried = [3], []
+
+    def found(q, corpus, k, narrow, general):
+        tried.append(True)
+        v, i = general(q, k)
+        if left[0] < len(q):
+            general(q[: left[0]], k)
+        return v.tolist(), i.tolist()
+
+    monkeypatch.setattr(ops, "found_narrow", found)
+
+    def search():
+        tried.clear()
+        q = torch.randn(5, 8, generator=torch.Generator().manual_seed(2))
+        got = index.search(q.numpy(), 4).total_indices
+        assert got == (q @ vars(index)["corpus"].t()).topk(4).indices.tolist()
+        return bool(tried)
+
+    for pause in (1, 2, 4, 8, 16, 32, 64, 64):
+        assert search() and not any(search() for _ in range(pause))
+    left[0] = 2
+    assert all(search() for _ in range(3))
+    left[0] = 3
+    assert search() and not search() and search()
+
+
 @pytest.mark.parametrize("Q, N, K, k, by", [
     # own time over the general way's, measured
     (1, 250000, 768, 5, True), (256, 250000, 768, 10, True),  # 0.58, 0.49
