@@ -1099,10 +1099,24 @@ static std::pair<py::list, py::list> found_lists(torch::Tensor v,
   return lists_of(reinterpret_cast<const float*>(at), at + n, Q, k);
 }
 
+// Pinned memory of torch's cache; none where the host or a limit on locked memory does
+// not give it, and nothing is left of that failure.
+static c10::optional<torch::Tensor> pinned(std::vector<int64_t> size,
+                                           at::ScalarType type) {
+  try {
+    return torch::empty(
+        size, torch::TensorOptions().dtype(type).pinned_memory(true));
+  } catch (const c10::Error&) {
+    (void)hipGetLastError();
+    return c10::nullopt;
+  }
+}
+
 // found_lists of narrow_topk of queries that the host has, in one call: the GPU reads
 // them and writes its answer where the host has them (pinned memory of torch's cache,
 // given back when the stream has been waited for), which spares two copies and their
-// waits. Above 16 MB they are copied: pinned memory stays with the process. us of
+// waits. Above 16 MB they are copied (pinned memory stays with the process), and where
+// there is none. us of
 // 250000 rows of 768, the same work by way of copies and found_lists, and so: one query
 // 109 and 96, 256 230 and 205.
 // With rest: queries that narrow_topk left for near rows are asked again, one that is
@@ -1120,14 +1134,17 @@ static py::object narrow_found(torch::Tensor q, torch::Tensor corpus,
   {
     py::gil_scoped_release others;
     const c10::DeviceGuard guard(corpus.device());
-    const bool pin = std::max(Q * K, 2 * n) <= 1 << 22;
-    auto place = [&](at::IntArrayRef size, at::ScalarType t) {
-      return torch::empty(size, pin ? torch::TensorOptions().dtype(t)
-                                          .pinned_memory(true)
-                                    : corpus.options().dtype(t));
+    c10::optional<torch::Tensor> host[2];
+    if (std::max(Q * K, 2 * n) <= 1 << 22) {
+      host[0] = pinned({Q, K}, at::kFloat);
+      if (host[0]) host[1] = pinned({2, Q, k}, at::kInt);
+    }
+    const bool pin = host[1].has_value();
+    auto place = [&](int i, at::IntArrayRef size, at::ScalarType t) {
+      return pin ? *host[i] : torch::empty(size, corpus.options().dtype(t));
     };
-    auto asked = place({Q, K}, at::kFloat);
-    auto told = place({2, Q, k}, at::kInt);
+    auto asked = place(0, {Q, K}, at::kFloat);
+    auto told = place(1, {2, Q, k}, at::kInt);
     if (pin)
       std::memcpy(asked.data_ptr(), q.data_ptr(), Q * K * sizeof(float));
     else
@@ -1260,6 +1277,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("x") = py::none(), py::arg("w") = py::none(),
         py::arg("eps") = 0.0);
   m.def("found_lists", &found_lists);
+  m.def("pinned", [](int64_t n) { return pinned({n}, at::kByte); });
   m.def("narrow_found", &narrow_found, py::arg("q"), py::arg("corpus"),
         py::arg("rows"), py::arg("up"), py::arg("error"), py::arg("norm"),
         py::arg("k"), py::arg("rest") = false);

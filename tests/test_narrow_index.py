@@ -127,3 +127,12 @@ def test_rows_that_leave_most_questions_are_spared(index, monkeypatch):
     (1, 32000, 16384, 10, False), (1000, 1000, 384, 10, False)])  # 1.9, 1.0
 def test_where_rows_in_16_bits_are_the_faster_way(Q, N, K, k, by):
     assert ops._narrow_fills(Q, N, K, k) == by
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="the failure of a host "
+                    "without a GPU")
+def test_no_pinned_memory():
+    """A search then copies its questions; it does not fail."""
+    with pytest.raises(RuntimeError):
+        torch.empty(64, pin_memory=True)
+    assert ops._hip_ops.pinned(64) is None

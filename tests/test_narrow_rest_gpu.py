@@ -65,7 +65,8 @@ def _check(found, q, c, k, rest, equal):
     (2, 9001, 256, 1100, 1, 7),      # beside a question that is answered
     (40, 40003, 64, 900, 5, 8),      # of a batch
     (32, 70000, 64, 1060, 32, 1),    # as many as are asked again
-    (200, 70001, 128, 1200, 4, 1)])
+    (200, 70001, 128, 1200, 4, 1),
+    (4100, 40000, 1024, 1100, 1, 1)])  # whose answer is copied
 def test_near_rows(device, k, noise, Q, N, K, many, some, every):
     q, c = _unit(Q, K, 1), _unit(N, K, 2)
     at = (torch.arange(many)[None] * every
@@ -163,3 +164,7 @@ def test_streams_and_threads(device, tmp_path):
     for t in threads:
         t.join()
     assert not errors
+
+
+def test_pinned_memory(device):
+    assert _hip_ops.pinned(64).is_pinned()
