@@ -419,7 +419,11 @@ static std::vector<torch::Tensor> embed_tokens(
                 "a mask number per token");
     bias = torch::empty(ids.sizes(), ids.options().dtype(at::kFloat));
   }
-  if (ids.numel() > 0)
+  // (rows without numbers have nothing to be asked for ahead)
+  if (ids.numel() > 0 && H == 0 && mask)
+    launch_key_bias(mask->data_ptr(), bias.data_ptr<float>(), mask->numel(),
+                    bytes, cur_stream());
+  if (ids.numel() > 0 && H > 0)
     launch_embed_layer_norm(
         (const long*)ids.data_ptr<int64_t>(),
         pos_ids ? (const long*)pos_ids->data_ptr<int64_t>() : nullptr,

@@ -114,3 +114,14 @@ def test_embed_with_bias(device, H, dtype):
     x, bias = ops.embed_with_bias(ids, None, mask, *tables, 1e-5)
     assert torch.equal(x, ops.embed_layer_norm(ids, None, *tables, 1e-5))
     assert torch.equal(bias, ops.key_bias(mask)) and bias.is_contiguous()
+
+
+def test_rows_without_numbers(device):
+    """Nothing is read for them, and the mask is as ever."""
+    tables = [torch.zeros(*n, 0, device=device, dtype=torch.bfloat16)
+              for n in ((50,), (40,), (), (), ())]
+    ids = torch.randint(0, 50, (3, 37), device=device)
+    mask = torch.randint(0, 2, (3, 37), device=device)
+    x, bias = ops.embed_with_bias(ids, None, mask, *tables, 1e-5)
+    assert x.shape == (3, 37, 0) and torch.equal(bias, ops.key_bias(mask))
+    assert ops.embed_layer_norm(ids, None, *tables, 1e-5).shape == x.shape
