@@ -748,8 +748,10 @@ def embed_layer_norm(ids, pos_ids, word, pos, type_row, w, b, eps):
 
 def embed_with_bias(ids, pos_ids, mask, word, pos, type_row, w, b, eps):
     """embed_layer_norm, and key_bias of mask: in one launch where both are the
-    kernels' and mask has a number per token."""
-    if (_embeds(word, pos, type_row) and mask.shape == ids.shape
+    kernels' and mask has a number per token, unless one of them has been replaced
+    and is to see its own."""
+    if (embed_layer_norm is _EMBED and key_bias is _KEY_BIAS
+            and _embeds(word, pos, type_row) and mask.shape == ids.shape
             and mask.device == ids.device and not mask.is_floating_point()
             and not mask.is_complex() and mask.element_size() in (1, 4, 8)):
         _require_hip()
@@ -774,6 +776,9 @@ def key_bias(mask):
         torch.full((), float("-inf"), device=mask.device,
                    dtype=torch.float32),
     )
+
+
+_EMBED, _KEY_BIAS = embed_layer_norm, key_bias
 
 
 def bert_few_rows(x, mask_f, layers, heads, eps, act):

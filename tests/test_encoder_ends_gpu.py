@@ -5,6 +5,7 @@ import pytest
 import torch
 
 from distllm_amd import ops
+from distllm_amd.models import build_model
 from distllm_amd.ops import torch_ref
 
 pytestmark = pytest.mark.gpu
@@ -114,6 +115,16 @@ def test_embed_with_bias(device, H, dtype):
     x, bias = ops.embed_with_bias(ids, None, mask, *tables, 1e-5)
     assert torch.equal(x, ops.embed_layer_norm(ids, None, *tables, 1e-5))
     assert torch.equal(bias, ops.key_bias(mask)) and bias.is_contiguous()
+
+
+@pytest.mark.parametrize("name", ["embed_layer_norm", "key_bias"])
+def test_a_replaced_end_sees_its_call(device, monkeypatch, name):
+    model = build_model("bert-tiny", device=device, dtype=torch.bfloat16)
+    ids = torch.randint(1, 50, (2, 9), device=device)
+    mask = torch.ones_like(ids)
+    want, seen, own = model(ids, mask), [], getattr(ops, name)
+    monkeypatch.setattr(ops, name, lambda *a: seen.append(name) or own(*a))
+    assert torch.equal(model(ids, mask), want) and seen == [name]
 
 
 def test_rows_without_numbers(device):
