@@ -187,6 +187,27 @@ def test_sandwich_norm_of_parts(device, S, M, W, n):
     assert torch.equal(h, h_want) and torch.equal(x, want)
 
 
+@pytest.mark.parametrize("M", [256, 257, 300])
+@pytest.mark.parametrize("W, n", [(1032, 1032), (2048, 2048), (2056, 2050),
+                                  (4096, 4096), (4104, 4104), (8192, 8000)])
+def test_sandwich_norm_of_more_rows(device, M, W, n):
+    """Both sides of the rows up to which all is asked for at once, bf16 rows
+    and slabs of them."""
+    y = _rand(3, M, W)
+    wn, wp, x = _rand(W, seed=2), _rand(W, seed=3), _rand(M, W, seed=4)
+    for t in (y, wn, wp, x):
+        t[..., n:] = 0
+    one = (y[0] + y[1] + y[2]).bfloat16()
+    x_ref, x_one = x.cpu(), x.clone()
+    h_ref = torch_ref.post_norm_add(one.float().cpu(), x_ref, wp.cpu(),
+                                    wn.cpu(), n, 0.01)
+    h_one = ops.post_norm_add(one, x_one, wp, wn, n, 0.01)
+    _close(h_one, h_ref, BF16)
+    _close(x_one, x_ref, F32)
+    h = ops.post_norm_add(y, x, wp, wn, n, 0.01)
+    assert torch.equal(h, h_one) and torch.equal(x, x_one)
+
+
 def test_sublayers_that_are_watched(device):
     """A hook on a sublayer sees its output, and changes no result."""
     model = build_model(layered_preset(
