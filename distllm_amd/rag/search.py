@@ -91,6 +91,9 @@ class HipIndexConfig(BaseConfig):
     nlist: int = 0    # ivf: clusters (0 -> ~sqrt(N))
     nprobe: int = 32  # ivf: chunks probed per query (recall@10 0.94
     # at 10M rows/nprobe 32, 0.97 at 64 — profiles/RESULTS.md)
+    narrow_rows: bool = True  # float32, exact: the rows once more in 16 bits
+    # on the GPU, half of their memory again (an eighth of what is free at
+    # most), for searches that take 0.6 of the time
 
     def model_post_init(self, _ctx) -> None:
         if str(self.faiss_index_path) in ("", "."):
@@ -107,6 +110,7 @@ class HipFlatIndex:
     # searches that go without them as these answered few questions, and how many
     # the next time
     _without, _without_next = 0, 1
+    narrow_rows = True  # whether there are to be any
 
     @property
     def corpus(self) -> torch.Tensor:
@@ -150,7 +154,8 @@ class HipFlatIndex:
                  num_quantization_workers: int = 1,
                  device: str | None = None,
                  score_chunk_rows: int = 1 << 21,
-                 nlist: int = 0, nprobe: int = 8):
+                 nlist: int = 0, nprobe: int = 8,
+                 narrow_rows: bool = True):
         if precision not in ("float32", "ubinary"):
             raise ValueError(f"invalid precision {precision}")
         if precision == "ubinary":
@@ -173,6 +178,7 @@ class HipFlatIndex:
         self.search_algorithm = search_algorithm
         self.nlist = nlist
         self.nprobe = nprobe
+        self.narrow_rows = narrow_rows
         self.precision = precision
         self.rescore_multiplier = rescore_multiplier
         self.faiss_index_path = Path(faiss_index_path)
@@ -237,7 +243,8 @@ class HipFlatIndex:
             self.code_words = W
         if self.search_algorithm == "ivf":
             self._build_ivf()
-        self.renew_narrow()
+        if self.narrow_rows:
+            self.renew_narrow()
 
     def _assign(self, cent: torch.Tensor) -> torch.Tensor:
         """argmax cluster per corpus row, GEMM-chunked so the score

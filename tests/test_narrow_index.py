@@ -8,7 +8,7 @@ import torch
 from datasets import Dataset
 
 from distllm_amd import ops
-from distllm_amd.rag.search import HipFlatIndex
+from distllm_amd.rag.search import HipFlatIndex, HipIndexConfig
 
 
 @pytest.fixture
@@ -78,6 +78,18 @@ def test_indices_without(index, tmp_path, by_narrow, args):
         other = HipFlatIndex(tmp_path / "d", tmp_path / "i.npz", device="cpu",
                              **args)
     assert other.narrow is None
+
+
+def test_an_index_told_to_do_without(index, tmp_path, by_narrow):
+    paths = tmp_path / "d", tmp_path / "i.npz"
+    other = HipFlatIndex(*paths, device="cpu", narrow_rows=False)
+    assert other.narrow is None and not _search(other, by_narrow)
+    other.renew_narrow()
+    assert _search(other, by_narrow)
+    config = {"dataset_dir": paths[0], "faiss_index_path": paths[1]}
+    for told in ({}, {"narrow_rows": False}):
+        args = HipIndexConfig(**config, **told).model_dump(exclude={"name"})
+        assert (HipFlatIndex(**args, device="cpu").narrow is None) == bool(told)
 
 
 def test_no_corpus():
