@@ -1298,10 +1298,10 @@ def post_norm_add(y, x, w_post, w_next, n, eps):
 def latent_prep(ab, q_cols, q_rank, rank, wq, wc, eps, cache, block_table,
                 row_seq, ctx):
     """Norm both down-projections of a latent-attention layer, ab [M, columns]
-    or what linear_parts returned, in one launch: the query latent (first q_cols columns of ab) is returned,
-    the key/value latent goes straight to its cache slot (position
-    ctx - 1 of block-table row row_seq; ctx 0 writes nothing). cache
-    None: the layer has no latent of its own."""
+    or what linear_parts returned, in one launch: the query latent (first
+    q_cols columns of ab) is returned, the key/value latent goes straight to
+    its cache slot (position ctx - 1 of block-table row row_seq; ctx 0 writes
+    nothing). cache None: the layer has no latent of its own."""
     if ab.is_cuda:
         _require_hip("_hip_latent")
         return _hip_ops.latent_prep(ab, q_cols, q_rank, rank, wq, wc, eps,

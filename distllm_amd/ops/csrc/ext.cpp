@@ -558,9 +558,10 @@ std::vector<torch::Tensor> search_few(torch::Tensor q, torch::Tensor corpus,
 }
 
 // Rows [N, K] times the power of two that brings the largest number to 2^13, as f16
-// in blocks (narrow_search.hip; [N in whole 16s, K in whole 64s] of them), that power, and the largest |row - row as f16| and |row as f16|
-// (and the root of the mean square of the latter) of rows times it. Nothing where a
-// number is infinite or NaN, or all are 0. Waits for the GPU.
+// in blocks (narrow_search.hip; [N in whole 16s, K in whole 64s] of them), that power,
+// and the largest |row - row as f16| and |row as f16| (and the root of the mean square
+// of the latter) of rows times it. Nothing where a number is infinite or NaN, or all
+// are 0. Waits for the GPU.
 c10::optional<std::tuple<torch::Tensor, int64_t, double, double, double>>
 narrow_rows(torch::Tensor corpus) {
   CHECK_DEV(corpus); CHECK_CONT(corpus); CHECK_F32(corpus);
@@ -1120,9 +1121,8 @@ static c10::optional<torch::Tensor> pinned(std::vector<int64_t> size,
 // them and writes its answer where the host has them (pinned memory of torch's cache,
 // given back when the stream has been waited for), which spares two copies and their
 // waits. Above 16 MB they are copied (pinned memory stays with the process), and where
-// there is none. us of
-// 250000 rows of 768, the same work by way of copies and found_lists, and so: one query
-// 109 and 96, 256 230 and 205.
+// there is none. us of 250000 rows of 768, the same work by way of copies and
+// found_lists, and so: one query 111 and 96, 256 228 and 204 (score_topk 173 and 455).
 // With rest: queries that narrow_topk left for near rows are asked again, one that is
 // all 0 has the first rows with scores of 0, and those that are still unanswered are
 // returned, as a third list, with nothing in their lists. Without, nothing (None) if

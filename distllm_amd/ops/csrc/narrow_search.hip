@@ -17,9 +17,9 @@
 // the caller asks the corpus itself. Unit vectors of 768: the margin is 1.3e-3, within which
 // a sixth more rows than the k best are. The scores are those of search_top_kernel.
 //
-// Us in a stream, k = 10, score_topk and this, 250000 rows of 768: 1 query 140, 80; 16
-// 159, 87; 17 163, 104; 128 233, 107; 256 342, 128; 20000 rows of 384: 1 14, 14; 16 40,
-// 17; 256 42, 27.
+// Us in a stream, k = 10, score_topk and this, 250000 rows of 768: 1 query 138, 79; 16
+// 159, 83; 17 161, 100; 128 239, 102; 256 355, 126; 20000 rows of 384: 1 14, 13; 16 37,
+// 14; 256 41, 24.
 //
 // Rows and queries lie in the order of the matrix cores' operands: blocks of 16 rows
 // by 32 columns, [ceil(N / 16)][KP / 32][64 lanes][8 numbers], lane l with row l % 16
@@ -850,6 +850,10 @@ NarrowPlan narrow_plan(int Q, int N, int K, int KP) {
     o.each = (units + o.S - 1) / o.S * 4;
     o.ld = Q;
   } else {
+    // Tiles of 256 rows that leave half of the CUs without one are halved: 200 sizes
+    // of 128 to 4096 columns, time by 128 rows over that by 256, up to 128 tiles 0.57
+    // to 0.95 (1000 x 4096 1.01), 129 to 256, where the halves are a second round,
+    // 0.88 to 1.02 of 128 columns and 0.95 to 1.23 beyond, above 0.95 to 1.21.
     const long tiles = (N + 255L) / 256 * (p.QP / tile);
     p.fm = tiles <= 128 ? 4 : 8;
     o.S = (N + 32 * p.fm - 1) / (32 * p.fm) * 2;

@@ -96,6 +96,17 @@ def test_columns_even_on_the_card(device, M, N, K, shares):
         _close(ops._hip_ops.decode_gemm_parts(x, w).sum(0), z)
 
 
+@pytest.mark.parametrize("N, K", [(64, 2048), (192, 2112), (1024, 4096),
+                                  (1984, 2048), (2048, 2240)])
+@pytest.mark.parametrize("M", [1, 8, 9, 16, 17, 25, 32, 33, 41, 49, 57, 64])
+def test_eight_columns(device, M, N, K):
+    """Up to 2048 columns with sums that begin in turn."""
+    x, w, b = _inputs(M, N, K, device, M + N)
+    z = x.float() @ w.float().T
+    _close(ops._hip_ops.decode_gemm(x, w, None, 0), z)
+    _close(ops._hip_ops.decode_gemm(x, w, b, 0), z + b.float())
+
+
 @pytest.mark.parametrize("M", [1, 8, 24, 64])
 @pytest.mark.parametrize("N, K", [(64, 2048), (1024, 4096), (2048, 2176),
                                   (2112, 2048)])
