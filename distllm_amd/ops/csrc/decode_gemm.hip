@@ -39,6 +39,7 @@
 #include "common.h"
 #include "gelu_rows.h"
 #include "norm_row.h"
+#include <climits>
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef unsigned short u16;
@@ -676,11 +677,31 @@ static bool dg_short_sums(int rows, int N, int K) {
 
 // Sixteens of columns of a workgroup in the even form where `splitk` share K, 0 where
 // that is another's: 3 and 5 to 8 (4 are the tile form), of which a CU has at least
-// 0.85 on average, and a sum that fills the ring.
-static int dg_even_columns(int rows, int N, int K, int splitk) {
-  if (rows <= 16 || rows > 64 || 256 % splitk || K / splitk < 512) return 0;
-  const int F = N / 16, G = 256 / splitk, C = (F + G - 1) / G;
-  return C >= 3 && C != 4 && C <= 8 && F >= 0.85f * (G * C) ? C : 0;
+// 0.85 on average, and a sum that is long enough for them. Measured over fresh weights
+// at 36 numbers of columns and 13 of K, linear and gated, 17 to 64 rows, time over that
+// of the tiles and shares else taken: short sums are 0.95 to 1.25 (the ring of many
+// columns fills slowly, and 64 x 64 tiles are several a CU that fill each other's
+// pauses), from these lines on it is 0.73 to 1.02 (6144 x 8192 by four shares 1.03):
+//   3 sixteens, up to 32 rows 1536 of K, where K is shared 512; more rows 2560
+//   5, up to 32 rows 768, else 1024
+//   6, up to 32 rows 768, else 1536; where K is shared 1024, by eight and more 1536
+//   7, 2560 (7168 columns by four shares 0.95 to 1.23: not where K is shared)
+//   8, 3072, up to 32 rows 4096 and no gated unit (32768 x 4096 0.97, gated 1.04), and
+//      only if they come out even to 3% (30720 x 4096 1.07)
+static int dg_even_columns(int rows, int N, int K, int splitk,
+                           bool gated = false) {
+  if (rows <= 16 || rows > 64 || 256 % splitk) return 0;
+  const int F = N / 16, G = 256 / splitk, C = (F + G - 1) / G, sum = K / splitk;
+  if (C < 3 || C == 4 || C > 8 || F < 0.85f * (G * C)) return 0;
+  const bool few = rows <= 32, shared = splitk > 1;
+  int least = INT_MAX;
+  if (C == 3) least = !few ? 2560 : shared ? 512 : 1536;
+  else if (C == 5) least = few && !shared ? 768 : 1024;
+  else if (C == 6) least = shared ? (splitk <= 4 ? 1024 : 1536) : few ? 768 : 1536;
+  else if (C == 7) least = shared ? INT_MAX : 2560;
+  else if (!shared && F >= 0.97f * (G * C) && !(few && gated))
+    least = few ? 4096 : 3072;
+  return sum >= least ? C : 0;
 }
 
 // How many workgroups share K in the tile and even forms: the least that give 150 of
@@ -711,11 +732,14 @@ extern "C" int decode_gemm_shares(int M, int N, int K) {
 // us that joins them: of 17 to 32 rows the ring is the slower form then from 2048 x 4096
 // on. us in a graph over fresh weights, ring and tiles, 17 and 32 rows: 2048 x 4096 8.0,
 // 9.3 and 5.8, 6.1; 4096 x 4096 9.0, 11.4 and 8.5, 8.4; 4096 x 1536 5.5, 5.6 and 5.6,
-// 6.0.
+// 6.0. (With the norm that sums them 4096 x 3072, three shares, 17 rows 10.6 and 10.9,
+// 24 11.7 and 11.4.)
 extern "C" int decode_parts_shares(int M, int N, int K) {
-  return M > 16 && M <= 32 && (long)N * K >= 2048L * 4096
-             ? dg_shares(M, N, K)
-             : decode_gemm_shares(M, N, K);
+  if (M > 16 && M <= 32 && (long)N * K >= 2048L * 4096) {
+    const int shares = dg_shares(M, N, K);
+    if (shares != 3 || M >= 24) return shares;
+  }
+  return decode_gemm_shares(M, N, K);
 }
 
 // Whether a product of M <= 64 rows takes the ring.
@@ -824,7 +848,8 @@ static void dg_launch(const u16* X, const u16* W, float* slabs, int K,
                          X, W, slabs, K, splitk, e);                         \
   } while (0)
   if constexpr (ACT == DG_NONE || ACT == DG_F32 || GLU) {
-    const int C = tile ? 0 : dg_even_columns(e.M, e.N, K, splitk);
+    const int C =
+        tile ? 0 : dg_even_columns(e.M, e.N, K, splitk, dg_glu(ACT));
     if (C > 0) {
 #define DG_EVEN(MP, CC, SL)                                                 \
   hipLaunchKernelGGL((dg_even_kernel<ACT, MP, CC, SL>), dim3(256),          \

@@ -76,10 +76,15 @@ def test_activations(device, M, share):
 @pytest.mark.parametrize("M", [17, 32, 33, 64])
 @pytest.mark.parametrize("N, K, shares", [
     (12288, 512, 1), (16384 + 3072, 576, 1), (27648, 512, 1), (32768, 640, 1),
-    (6144, 2048, 4), (5120, 2048, 4), (6144, 1024, 2)])
+    (6144, 2048, 2), (5120, 2048, 2), (6144, 1024, 2),
+    (12288, 1536, 1), (12288, 2560, 1), (19456, 768, 1), (19456, 1088, 1),
+    (24576, 768, 1), (24576, 1600, 1), (28672, 2560, 1), (27648, 2624, 1),
+    (32768, 3072, 1), (32768, 4096, 1), (5632, 1024, 2), (5120, 4096, 4),
+    (5632, 4096, 4), (6144, 4096, 4), (2560, 8192, 8), (3072, 12288, 8)])
 def test_columns_even_on_the_card(device, M, N, K, shares):
-    """48 to 128 columns a workgroup, all and some with one block less, with the
-    least sum and others, of one share and of several."""
+    """48 to 128 columns a workgroup, all and some with one block less, of one
+    share and of several, with the least sums that take them, and short ones
+    that do not."""
     run, F = ops._hip_ops.decode_gemm, torch.nn.functional
     assert ops._hip_ops.decode_gemm_shares(M, N, K) == shares
     x, w, b = _inputs(M, N, K, device, M + N)
