@@ -45,12 +45,22 @@ norm_fwd_kernel(const unsigned short* __restrict__ x,
       xv[k] = *reinterpret_cast<const s16x8*>(xr + c);
       if (HAS_RES) rv[k] = *reinterpret_cast<const s16x8*>(rr + c);
     }
-#pragma unroll
-    for (int k = 0; k < NCL; ++k) {
-      const int c = min(lane + k * WAVE, chunks - 1) * 8;
-      wv[k] = *reinterpret_cast<const s16x8*>(w + c);
+    // The weights behind the row, not ahead of the loop and waited for there (up to
+    // 512 columns the compiler would); the bias, which an RMS norm seldom has, behind
+    // its sums: us without and with these two, RMS norms, 65536 rows of 128 17.9 and
+    // 16.3, with a residual and its sum 26 and 22, 8192 of 640 8.9 and 7.9.
+    int behind = 0;
+    asm volatile("" : "+s"(behind));
+    auto bias_at = [&](int k) {
+      const int c = min(lane + k * WAVE, chunks - 1) * 8 + behind;
       if (b != nullptr) bv[k] = *reinterpret_cast<const s16x8*>(b + c);
       else bv[k] = s16x8{0, 0, 0, 0, 0, 0, 0, 0};
+    };
+#pragma unroll
+    for (int k = 0; k < NCL; ++k) {
+      const int c = min(lane + k * WAVE, chunks - 1) * 8 + behind;
+      wv[k] = *reinterpret_cast<const s16x8*>(w + c);
+      if (!RMS) bias_at(k);
     }
     __builtin_amdgcn_sched_barrier(0);
 
@@ -100,6 +110,7 @@ norm_fwd_kernel(const unsigned short* __restrict__ x,
       const int c = lane + k * WAVE;
       if (c < chunks) {
         float wf[8], bf[8];
+        if (RMS) bias_at(k);
         bf8_to_f32(wv[k], wf);
         bf8_to_f32(bv[k], bf);
         s16x8 ov;
@@ -235,10 +246,14 @@ norm_fwd_small_kernel(const unsigned short* __restrict__ x,
 // of 1280 8.4 and 8.6, of 2560 15.2 and 17.9; 16384 rows of 768 18.1 and 14.4, of
 // 1024 19.6 and 17.9, of 1152 26.7 and 26.7, of 1280 28.4 and 29.4, of 2048 40.7
 // and 42.5; 65536 rows of 1152 to 2560 0.95 to 1.01 of the wave's time, 131072
-// 0.99 to 1.02; of 4096 always below 0.99.
-static bool norm_row_block(int n_rows, int H) {
-  return n_rows <= 8 || (H > 512 && n_rows <= 2048) ||
-         (H > 1024 && n_rows <= 65536) || H >= 3072;
+// 0.99 to 1.02; of 4096 always below 0.99. Without a residual 65536 rows of 1152 and
+// 1280 70.8 and 64.6, 78.4 and 75.1. With a sum to write 2500 rows of 768 5.7 and 6.1,
+// of 1024 6.7 and 7.3, 4096 of 1024 8.6 and 8.6.
+static bool norm_row_block(int n_rows, int H, bool has_res, bool write_sum) {
+  const int narrow = write_sum && H > 640 ? 3000 : 2048;
+  const int wide = has_res || H >= 1536 ? 65536 : 16384;
+  return n_rows <= 8 || (H > 512 && n_rows <= narrow) ||
+         (H > 1024 && n_rows <= wide) || H >= 3072;
 }
 
 extern "C" void launch_norm_fwd(const void* x, const void* res, const void* w,
@@ -257,8 +272,12 @@ extern "C" void launch_norm_fwd(const void* x, const void* res, const void* w,
                    cap != 0 ? cap : H > 512 ? 1 << 20 : 32768);
   bool has_res = res != nullptr;
   bool write_sum = sum_out != nullptr;
-  const bool small = norm_row_block(n_rows, H);
-  const bool ahead = n_rows <= 512 || n_rows >= 1500;
+  const bool small = norm_row_block(n_rows, H, has_res, write_sum);
+  // (2048 rows without a residual: of 640 and 768 columns 3.88 ahead and 3.70, of 8192
+  // 16.2 and 14.4)
+  const bool ahead =
+      n_rows <= 512 || n_rows > 2048 ||
+      (n_rows >= 1500 && H > 1024 && (has_res || H < 3072));
   int ncl = small ? (H / 8 + 255) / 256 : (H / 8 + WAVE - 1) / WAVE;
 
 #define DISPATCH4(KERNEL, BLOCKS)                                              \
