@@ -415,7 +415,8 @@ latent_values_kernel(const float* __restrict__ pacc,
   // of 8 rows a wave joins one, of 4 half of one
   constexpr int PARTS = (R + 255) / 256 * ROWS / LV_WAVES, AHEAD = 8;
   static_assert(PARTS * LV_WAVES == (R + 255) / 256 * ROWS, "whole parts");
-  const int mine = wid % ROWS, c0 = wid / ROWS * 256 + lane * 4;
+  const int mine = ROWS == LV_WAVES ? wid : wid % ROWS;
+  const int c0 = (ROWS == LV_WAVES ? 0 : wid / ROWS * 256) + lane * 4;
   const long rh = (long)min(m0 + mine, M - 1) * H + head;
   const float* state = pml + (rh * NS + min(lane, NS - 1)) * 2;
   float m = state[0], l = state[1];
