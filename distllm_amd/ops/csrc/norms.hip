@@ -45,12 +45,13 @@ norm_fwd_kernel(const unsigned short* __restrict__ x,
       xv[k] = *reinterpret_cast<const s16x8*>(xr + c);
       if (HAS_RES) rv[k] = *reinterpret_cast<const s16x8*>(rr + c);
     }
-    // The weights behind the row, not ahead of the loop and waited for there (up to
-    // 512 columns the compiler would); the bias, which an RMS norm seldom has, behind
-    // its sums: us without and with these two, RMS norms, 65536 rows of 128 17.9 and
-    // 16.3, with a residual and its sum 26 and 22, 8192 of 640 8.9 and 7.9.
+    // The weights behind the row, not ahead of the loop and waited for there, as the
+    // compiler would have it up to 512 columns (us then and so, RMS norms of 65536 rows
+    // of 128 17.9 and 16.3, with a residual and its sum 26 and 22). Of two and more
+    // chunks that is 3 to 5% faster with a sum to write and slower without. The bias,
+    // which an RMS norm seldom has, behind its sums: 8192 rows of 640 8.9 and 7.9.
     int behind = 0;
-    asm volatile("" : "+s"(behind));
+    if (NCL == 1 || WRITE_SUM) asm volatile("" : "+s"(behind));
     auto bias_at = [&](int k) {
       const int c = min(lane + k * WAVE, chunks - 1) * 8 + behind;
       if (b != nullptr) bv[k] = *reinterpret_cast<const s16x8*>(b + c);
