@@ -141,6 +141,7 @@ class HipFlatIndex:
         had it or replaced it, and will not write to it any more. Takes half of
         its memory again; nothing where they are of no use to the index."""
         self.narrow = None
+        self._without, self._without_next = 0, 1
         rows = self.__dict__.get("corpus")
         if (rows is not None and self.precision == "float32"
                 and self.search_algorithm != "ivf"):

@@ -124,6 +124,8 @@ def test_rows_that_leave_most_questions_are_spared(index, monkeypatch):
     assert all(search() for _ in range(3))
     left[0] = 3
     assert search() and not search() and search()
+    index.renew_narrow()
+    assert search()
 
 
 @pytest.mark.parametrize("Q, N, K, k, by", [
