@@ -402,24 +402,24 @@ class HipFlatIndex:
                 or getattr(self._topk_exact, "__func__", None)
                 is not HipFlatIndex._topk_exact):
             return None
-        if not narrow.holds(self._rows):
+        rows = self._rows
+        if not narrow.holds(rows):
             self.narrow = None
             return None
         if self._without > 0:
             self._without -= 1
             return None
-        left = 0
+        left = []
 
         def general(rest, k):
-            nonlocal left
-            left = len(rest)
+            left.append(len(rest))
             return self._topk_exact(rest, k)
 
-        lists = ops.found_narrow(q, self._rows, min(k, self.n), narrow, general)
-        if lists is not None and 5 * left > 2 * len(q):
+        lists = ops.found_narrow(q, rows, min(k, self.n), narrow, general)
+        if left and 5 * left[-1] > 2 * len(q):
             self._without = self._without_next
             self._without_next = min(2 * self._without_next, 64)
-        elif lists is not None:
+        elif lists is not None and self._without_next > 1:
             self._without_next = 1
         return lists
 
